@@ -344,6 +344,14 @@ __global__ __launch_bounds__(64 * NW) void window_decode_vec_kernel(bf16_t* __re
 // running maximum, rescaling or a cross-lane sum per tile (the lanes' parts of the denominator meet at the
 // end); only tiles at a row's first or last key are masked.
 constexpr float kMaxCapPlain = 60.f;
+// The LDS-staged kernel of window_flash.hip takes a step that has enough (row, head) pairs to fill the chip with its
+// 256 pairs per workgroup, or rows that may see enough keys for the shared tiles to pay with few workgroups.  Register
+// kernel at its better width -> staged kernel, us (128-wide heads): 13 prompts x 120, 8 heads (12480 pairs, 120 keys)
+// 9.2 -> 12.5; x 250 21.3 -> 16.6; x 500 52 -> 25; one prompt of 512, 8 heads 20.3 -> 21.7; 1024 38 -> 34; 64 rows
+// behind 2000 keys, 16 heads 70 -> 61.  mfma = kFlashForced asks for it at any size (tests, measurements).
+constexpr long kFlashPairs = 16 * 1024;
+constexpr long kFlashKeys = 1024;
+constexpr int kFlashForced = 256;
 template <int DK, int DV, int QT, int CAP>
 __global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv, long q_stride, const bf16_t* __restrict__ k_cache,
@@ -524,6 +532,11 @@ using namespace k8sllm;
 
 extern "C" {
 
+int k8sllm_hy_window_flash(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache, const int* cu,
+                           const int* ctx, const int* block_tables, int bt_stride, int S, long T, int Hq, int G, int dk, int dv,
+                           float scale, int window, int chunked, int keep, float cap, int plain_cap, int sink,
+                           const float* sinks, const void* gate, long g_stride, hipStream_t s);
+
 int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float* kw, float eps, long T, int nq,
                             int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s) {
   if (T <= 0) return 0;
@@ -546,9 +559,16 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
   if (dk > kGenDK || dv > 64 * kGenVC || G < 1 || Hq % G) return -1;
   // bf16 with matrix-core head sizes and 16-byte aligned rows: the MFMA kernel
   if (!f32 && mfma && bs == 16 && q_stride % 8 == 0 && (dk == 64 || dk == 128) && (dv == 64 || dv == 128)) {
+    const long keys = window > 0 && window < 16l * bt_stride ? window : 16l * bt_stride;  // at most, per row
+    if (mfma == kFlashForced || (mfma < 16 && (T * Hq >= kFlashPairs || keys >= kFlashKeys))) {
+      const int rc = k8sllm_hy_window_flash(out, qkv, q_stride, k_cache, v_cache, cu, ctx, block_tables, bt_stride, S, T, Hq, G,
+                                            dk, dv, scale, window, chunked, keep, cap, cap <= kMaxCapPlain && !sink, sink,
+                                            sinks, gate, g_stride, s);
+      if (rc != 1) return rc;
+    }
     // query rows per wave: 32 once the step is large enough to fill the chip that way (two row tiles
     // share every K / V^T fragment), else 16; mfma = 16 / 32 / 64 forces one (tests, measurements)
-    const int qrows = mfma >= 16 ? mfma : (T * Hq >= 64 * 1024 ? 32 : 16);
+    const int qrows = mfma >= 16 && mfma != kFlashForced ? mfma : (T * Hq >= 64 * 1024 ? 32 : 16);
     const dim3 grid((unsigned)(T / qrows + S), (unsigned)Hq);
 #define K8SLLM_WPC(DK, DV, QT, CAP)                                                                                    \
   hipLaunchKernelGGL((window_prefill_mfma_kernel<DK, DV, QT, CAP>), grid, dim3(64), 0, s, (bf16_t*)out,                 \
@@ -562,7 +582,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
   if (qrows == 64) { K8SLLM_WP(DK, DV, 4); }                     \
   else if (qrows == 32) { K8SLLM_WP(DK, DV, 2); }                \
   else { K8SLLM_WP(DK, DV, 1); }
-    if (mfma >= 16 && mfma != 16 && mfma != 32 && mfma != 64) return -1;
+    if (mfma >= 16 && mfma != 16 && mfma != 32 && mfma != 64 && mfma != kFlashForced) return -1;
     if (dk == 64 && dv == 64) { K8SLLM_WPQ(64, 64); }
     else if (dk == 64) { K8SLLM_WPQ(64, 128); }
     else if (dv == 64) { K8SLLM_WPQ(128, 64); }

@@ -524,8 +524,9 @@ def window_attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: 
     ``cap * tanh(s / cap)``.  ``sink``: the softmax denominator has one more term that carries
     no value - exp(0), or exp(sinks[h]) for head h where ``sinks`` [Hq] fp32 is given (a learned,
     unscaled logit).  Scores and weights are fp32.  Returns [T, Hq*dv].  GPU, bf16, head sizes
-    64 / 128: the matrix-core kernel, 16 query rows per wave or 32 in large steps (``mfma`` 0: the
-    any-size wave-per-row kernel; 16 / 32 / 64: that many rows per wave)."""
+    64 / 128: the matrix-core kernels - tiles staged in LDS for large steps and long contexts, else 16
+    query rows per wave (``mfma`` 0: the any-size wave-per-row kernel; 16 / 32 / 64: the register kernel with
+    that many rows per wave; 256: the staged kernel)."""
     T = qkv.shape[0]
     if not qkv.is_cuda:
         out = torch.empty(T, Hq * dv, dtype=qkv.dtype)
