@@ -214,26 +214,6 @@ def _rows8(ws: list, pad: bool = True) -> torch.Tensor:
     return torch.cat(ws).contiguous()
 
 
-def _fresh_pages(meta: AttnMeta, T: int, device) -> tuple:
-    """Temporary pages for a step of whole prompts: (slot of every row, block tables [S, W], blocks),
-    every segment starting on a page of its own.  Computed once per step (cached on ``meta``), on the
-    device, from the segment offsets."""
-    got = getattr(meta, "_fresh_pages", None)
-    if got is None:
-        cu = meta.cu_seqlens.long()
-        S = cu.numel() - 1
-        nblk = (cu[1:] - cu[:-1] + BLOCK - 1) // BLOCK
-        first = torch.cumsum(nblk, 0) - nblk  # a segment's first temporary block
-        rows = torch.arange(T, device=device)
-        seg = torch.bucketize(rows, cu[1:], right=True).clamp(max=S - 1)
-        slots = (first[seg] * BLOCK + rows - cu[:-1][seg]).to(torch.int32)
-        nb = T // BLOCK + S
-        W = meta.block_tables.shape[1]
-        bt = (first[:, None] + torch.arange(W, device=device)[None, :]).clamp(max=nb - 1).to(torch.int32)
-        got = meta._fresh_pages = (slots, bt.contiguous(), nb)
-    return got
-
-
 class LatentAttention:
     """Attention over a compressed key/value stream (one normed latent of ``kv_rank`` and one
     rotated key part of ``rot_dim`` per token, shared by all heads), rotary positions on the
@@ -247,14 +227,17 @@ class LatentAttention:
     (a [T, n] view) - the block's residual gate rides in the mixer's first GEMM.
 
     Two forms of the same attention.  Over the cache the per-head expansions are moved to the query
-    side (module docstring): every step can take it.  A step of whole prompts (every chunk starts at
-    position 0, no decode rows beside them; bf16, head sizes of the matrix-core kernel) of at least
-    ``EXPAND_MIN_ROWS`` rows instead expands this step's keys ``[W_uk c | shared part]`` and values
-    ``W_uv c`` per head into temporary pages and runs windowed attention's kernel over them:
-    ``dim + rot_dim + vdim`` multiply-adds per (query, key, head) instead of ``2 kv_rank + rot_dim``."""
+    side (module docstring): every step can take it.  The prompt rows of a step with at least ``EXPAND_MIN_ROWS`` of them
+    (bf16, head sizes of the matrix-core kernels) instead expand the keys ``[W_uk c | shared part]`` and values
+    ``W_uv c`` of all positions they see per head into temporary pages and run windowed attention's kernel over
+    them: ``dim + rot_dim + vdim`` multiply-adds per (query, key, head) instead of ``2 kv_rank + rot_dim``.  With
+    more than ``EXPAND_KEYS`` positions per row the expansion costs more than it saves (16 heads, kv_rank 256, one layer, cache
+    form -> expanded, us: 1 x 64 rows 151 -> 85; 1 x 128 behind 4000 tokens 171 -> 155; 16 x 128 behind 4000 1466 -> 569;
+    2 x 2000 behind 2816 1740 -> 200; 16 x 64 behind 4000, 64 positions per row, 428 -> 513)."""
 
     kind = "latent_attention"
-    EXPAND_MIN_ROWS = 1024
+    EXPAND_MIN_ROWS = 64
+    EXPAND_KEYS = 32
 
     def __init__(self, spec: LayerSpec, d: int, eps: float, p: _Params, prefix: str, traits: Optional[dict] = None,
                  tail: Optional[torch.Tensor] = None):
@@ -322,8 +305,21 @@ class LatentAttention:
         hops.latent_prep(down, Q, R, dr, self.qn, self.kn, self.eps, meta.positions, self.freq,
                          kc if own else None, vc if own else None, meta.slot_mapping if own else None, pairs=self.pairs)
         q = F.linear(down[:, :Q], self.w_uq)
-        if self._expand_ok(h, meta):
-            return self._forward_expanded(q, down, meta, kc, gate)
+        ex = self._expand_ok(h, meta)
+        nd = meta.num_decode if meta.is_prefill else T  # single-token rows in front
+        parts = []
+        if nd or not ex:
+            n = nd if ex else T
+            parts.append(self._forward_latent(q[:n], meta, kc, vc, gate[:n] if gate is not None else None, not ex))
+        if ex:
+            parts.append(self._forward_expanded(q[nd:], down[nd:], meta, kc, gate[nd:] if gate is not None else None))
+        return F.linear(parts[0] if len(parts) == 1 else torch.cat(parts), self.wo)
+
+    def _forward_latent(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
+                        chunks: bool) -> torch.Tensor:
+        """Attention over the latent pages: the step's single-token rows and, with ``chunks``, its prompt rows."""
+        H, dn, dr, dv, R = self.H, self.dn, self.dr, self.dv, self.R
+        T = q.shape[0]
         # the per-head key expansion moved to the query: q_lat[h] = q_unrotated[h] @ W_uk[h]  ([H, T, R])
         q_lat = torch.bmm(q.view(T, H, dn + dr)[:, :, :dn].transpose(0, 1), self.w_uk.view(H, dn, R))
         qa = hops.latent_queries(q, q_lat, H, dn, dr, meta.positions, self.freq, self.pitch, pairs=self.pairs)
@@ -334,48 +330,37 @@ class LatentAttention:
         else:
             nd = meta.num_decode
             gc, gd = (gate[nd:], gate[:nd]) if gate is not None else (None, None)
-            o = hops.latent_attention(qa[nd:], kc, vc, meta.block_tables, *args, cu=meta.cu_seqlens, ctx=meta.ctx_start, gate=gc,
-                                      **kw)
+            parts = []
             if nd:
-                od = hops.latent_attention(qa[:nd], kc, vc, meta.dec_block_tables, *args, seq_lens=meta.dec_seq_lens, gate=gd,
-                                           **kw)
-                o = torch.cat([od, o])
+                parts.append(hops.latent_attention(qa[:nd], kc, vc, meta.dec_block_tables, *args, seq_lens=meta.dec_seq_lens,
+                                                   gate=gd, **kw))
+            if chunks:
+                parts.append(hops.latent_attention(qa[nd:], kc, vc, meta.block_tables, *args, cu=meta.cu_seqlens,
+                                                   ctx=meta.ctx_start, gate=gc, **kw))
+            o = parts[0] if len(parts) == 1 else torch.cat(parts)
         # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T, written head by head
         # into the rows the out-projection reads
-        v = torch.empty(T, H, dv, dtype=h.dtype, device=h.device)
+        v = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
         torch.bmm(o.view(T, H, R).transpose(0, 1), self.w_uv.view(H, dv, R).transpose(1, 2), out=v.transpose(0, 1))
-        return F.linear(v.view(T, H * dv), self.wo)
+        return v.view(T, H * dv)
 
     def _expand_ok(self, h: torch.Tensor, meta: AttnMeta) -> bool:
-        return (meta.is_prefill and meta.all_fresh and not meta.num_decode and h.is_cuda and h.dtype == torch.bfloat16
-                and bool(self.fast) and h.shape[0] >= self.EXPAND_MIN_ROWS
+        rows = h.shape[0] - meta.num_decode
+        return (meta.is_prefill and meta.page_list is not None and h.is_cuda and h.dtype == torch.bfloat16
+                and bool(self.fast) and rows >= self.EXPAND_MIN_ROWS
+                and (meta.all_fresh or meta.page_list.numel() * BLOCK <= self.EXPAND_KEYS * rows)
                 and (self.dn + self.dr) in (64, 128) and self.dv in (64, 128))
 
     def _forward_expanded(self, q: torch.Tensor, down: torch.Tensor, meta: AttnMeta, kc: torch.Tensor,
                           gate: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """Whole prompts: per-head keys and values of this step's rows in temporary pages, windowed
-        attention's matrix-core kernel over them.  ``q`` [T, H * (dim + rot_dim)] still unturned."""
-        H, dn, dr, dv, Q, R = self.H, self.dn, self.dr, self.dv, self.Q, self.R
-        T, D = q.shape[0], self.dn + self.dr
-        if self.kv_from is None:  # latent_prep left the normed latent and the turned shared part in place
-            c, kr = down[:, Q:Q + R], down[:, Q + R:Q + R + dr]
-        else:  # the other layer's, as its pages hold them
-            rows = kc.view(-1, kc.shape[2]).index_select(0, meta.slot_mapping[:T].long())
-            c, kr = rows[:, :R], rows[:, R:R + dr]
-        fused = torch.empty(T, 2 * H * D + H * dv, dtype=q.dtype, device=q.device)  # [q | k | v], head by head
-        fused[:, :H * D] = q
-        kx = fused[:, H * D:2 * H * D].view(T, H, D)
-        kx[:, :, :dn] = F.linear(c, self.w_uk).view(T, H, dn)
-        kx[:, :, dn:] = kr.unsqueeze(1)
-        fused[:, 2 * H * D:] = F.linear(c, self.w_uv)
-        slots, bt, nb = _fresh_pages(meta, T, q.device)
-        kt = torch.zeros(nb, BLOCK, H * D, dtype=q.dtype, device=q.device)
-        vt = torch.zeros(nb, H, dv, BLOCK, dtype=q.dtype, device=q.device)
-        # the queries' rotated parts turn here; the shared key part was turned by latent_prep
-        hops.rotary_cache(fused, H, H, D, dv, meta.positions, self.freq, self.pairs, None, kt, vt, slots, rot_off=dn, rot_k=False)
-        o = hops.window_attention_prefill(fused, kt, vt, meta.cu_seqlens, meta.ctx_start, bt, H, H, D, dv, self.scale,
-                                          self.window, self.sink, mfma=self.fast, sinks=self.sinks, gate=gate)
-        return F.linear(o, self.wo)
+        """Prompt rows: per-head keys and values of every position they see in temporary pages, windowed
+        attention's matrix-core kernel over them.  ``q`` [rows, H * (dim + rot_dim)] still unturned."""
+        H, dn, dr, dv = self.H, self.dn, self.dr, self.dv
+        nd = meta.num_decode
+        kt, vt = hops.latent_expand(kc, meta.page_list, self.w_uk, self.w_uv, H, self.R, dr)
+        hops.rotate_heads(q, H, dn + dr, meta.positions[nd:], self.freq, self.pairs, dn)
+        return hops.window_attention_prefill(q, kt, vt, meta.cu_seqlens, meta.ctx_start, meta.page_bt, H, H, dn + dr, dv, self.scale,
+                                             self.window, self.sink, mfma=self.fast, sinks=self.sinks, gate=gate)
 
 
 class RotaryAttention:

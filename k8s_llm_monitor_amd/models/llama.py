@@ -82,6 +82,10 @@ class AttnMeta:
     seg_slot: Optional[torch.Tensor] = None
     # prefill: every chunk of this step starts at position 0 (whole prompts, nothing cached before)
     all_fresh: bool = False
+    # layer-list prefill: the pages of every chunk's sequence up to its last token of this step, sequence after
+    # sequence [n], and per chunk the numbers of its pages in that list [S, W] (latent attention's expanded form)
+    page_list: Optional[torch.Tensor] = None
+    page_bt: Optional[torch.Tensor] = None
 
 
 def _seed_for(name: str, seed: int) -> int:

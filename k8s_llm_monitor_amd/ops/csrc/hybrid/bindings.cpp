@@ -101,6 +101,10 @@ int k8sllm_hy_latent_attention(void* out, const void* q, long q_stride, const vo
                                const int* cu, const int* ctx, const int* seq_lens, const int* block_tables,
                                int bt_stride, int S, long T, int H, int dkp, int dv, int bs, float scale, int window,
                                const float* sinks, const void* gate, long g_stride, int split, hipStream_t s);
+int k8sllm_hy_latent_expand(void* kt, void* vt, const void* k_cache, int pitch, const int* page_list, int npages, const void* wk,
+                            const void* wv, int H, int R, int dn, int dr, int dv, hipStream_t s);
+int k8sllm_hy_rotate_heads(void* x, long stride, long T, int heads, int D, const int* positions, const float* freq, int nf,
+                           int pairs, int rot_off, int f32, hipStream_t s);
 int k8sllm_moe_align(const int* topk_ids, long n, int E, int* expert_offsets, int* sorted_idx, int* inv_idx,
                      hipStream_t s);
 }
@@ -525,6 +529,33 @@ void rotary_cache(Tensor qkv, int64_t Hq, int64_t G, int64_t dk, int64_t dv, Ten
                                freq.data_ptr<float>(), (int)freq.numel(), pairs, (int)rot_off, rot_k, qs, kc, vc, sp,
                                k_cache.has_value() ? (int)k_cache->size(1) : 16, f, cur()),
         "rotary_cache");
+}
+
+void rotate_heads(Tensor x, int64_t heads, int64_t D, Tensor positions, Tensor freq, bool pairs, int64_t rot_off) {
+  const int f = act(x, "x");
+  f32c(freq, "freq");
+  i32c(positions, "positions");
+  const int64_t T = x.size(0), nf = freq.numel();
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && heads >= 1 && x.size(1) >= heads * D && positions.numel() >= T && rot_off >= 0 &&
+                  rot_off + 2 * nf <= D,
+              "rotate_heads: x [T, heads*D], positions [T], freq");
+  check(k8sllm_hy_rotate_heads(x.data_ptr(), x.stride(0), T, (int)heads, (int)D, positions.data_ptr<int>(), freq.data_ptr<float>(),
+                               (int)nf, pairs, (int)rot_off, f, cur()),
+        "rotate_heads");
+}
+
+void latent_expand(Tensor kt, Tensor vt, Tensor k_cache, Tensor page_list, Tensor wk, Tensor wv, int64_t H, int64_t dr) {
+  for (const Tensor* t : {&kt, &vt, &k_cache, &wk, &wv})
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == torch::kBFloat16 && t->is_contiguous(), "latent_expand: contiguous bf16");
+  i32c(page_list, "page_list");
+  TORCH_CHECK(k_cache.dim() == 3 && k_cache.size(1) == 16 && wk.dim() == 2 && wv.dim() == 2 && wk.size(1) == wv.size(1) && H >= 1 &&
+                  wk.size(0) % H == 0 && wv.size(0) % H == 0,
+              "latent_expand: latent pages [blocks, 16, pitch], weights [H*dn, R], [H*dv, R]");
+  const int64_t R = wk.size(1), dn = wk.size(0) / H, dv = wv.size(0) / H, n = page_list.numel();
+  TORCH_CHECK(kt.numel() == n * 16 * H * (dn + dr) && vt.numel() == n * H * dv * 16, "latent_expand: temporary pages");
+  check(k8sllm_hy_latent_expand(kt.data_ptr(), vt.data_ptr(), k_cache.data_ptr(), (int)k_cache.size(2), page_list.data_ptr<int>(),
+                                (int)n, wk.data_ptr(), wv.data_ptr(), (int)H, (int)R, (int)dn, (int)dr, (int)dv, cur()),
+        "latent_expand");
 }
 
 void moe_router(Tensor ids, Tensor wts, OptT gate, Tensor h, Tensor wr, OptT bias, int64_t E, int64_t K,
@@ -1067,6 +1098,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sigmoid_gate", &sigmoid_gate);
   m.def("softcap", &softcap);
   m.def("rotary_cache", &rotary_cache);
+  m.def("rotate_heads", &rotate_heads);
+  m.def("latent_expand", &latent_expand);
   m.def("linear_attention_chunked", &linear_attention_chunked);
   m.def("qk_norm_cache", &qk_norm_cache);
   m.def("window_attention_prefill", &window_attention_prefill);

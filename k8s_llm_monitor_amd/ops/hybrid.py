@@ -674,6 +674,44 @@ def latent_queries(q: torch.Tensor, q_lat: torch.Tensor, H: int, dim: int, rot_d
     return out
 
 
+def rotate_heads(x: torch.Tensor, heads: int, dim: int, positions: torch.Tensor, freq: torch.Tensor, pairs: bool,
+                 rot_off: int = 0) -> None:
+    """In place on rows [T, heads * dim]: entries ``rot_off .. rot_off + 2 len(freq)`` of every head turn by the
+    row's position, as in rotary_cache."""
+    if not x.is_cuda:
+        T = x.shape[0]
+        v = x[:, :heads * dim].float().view(T, heads, dim)
+        turned = _rotate(v[..., rot_off:], positions, freq, pairs)
+        x[:, :heads * dim] = torch.cat([v[..., :rot_off], turned], -1).reshape(T, heads * dim).to(x.dtype)
+        return
+    native().rotate_heads(x, int(heads), int(dim), positions, freq, bool(pairs), int(rot_off))
+
+
+def latent_expand(k_cache: torch.Tensor, page_list: torch.Tensor, w_uk: torch.Tensor, w_uv: torch.Tensor, H: int, kv_rank: int,
+                  rot_dim: int) -> tuple:
+    """Per-head keys and values of the latent pages ``page_list`` names, as temporary pages of the windowed
+    attention kernels in the list's order: ([n, 16, H * (dim + rot_dim)], [n, H, vdim, 16]).  A key is ``[W_uk[h] c |
+    shared part]``, a value ``W_uv[h] c``, rounded once.  GPU, bf16, kv_rank 128 / 256, dim and vdim multiples of 32,
+    rot_dim of 8: one kernel; else matrix products over the gathered pages."""
+    n, R = page_list.numel(), kv_rank
+    dn, dv = w_uk.shape[0] // H, w_uv.shape[0] // H
+    D = dn + rot_dim
+    if k_cache.is_cuda and k_cache.dtype == torch.bfloat16 and R in (128, 256) and dn % 32 == 0 and dv % 32 == 0 and \
+            rot_dim % 8 == 0 and k_cache.shape[2] % 8 == 0:
+        kt = torch.empty(n, 16, H * D, dtype=k_cache.dtype, device=k_cache.device)
+        vt = torch.empty(n, H, dv, 16, dtype=k_cache.dtype, device=k_cache.device)
+        native().latent_expand(kt, vt, k_cache, page_list, w_uk, w_uv, int(H), int(rot_dim))
+        return kt, vt
+    rows = k_cache.index_select(0, page_list.long())
+    bs = rows.shape[1]
+    c = rows[..., :R].reshape(n * bs, R)
+    kt = torch.empty(n, bs, H, D, dtype=k_cache.dtype, device=k_cache.device)
+    kt[..., :dn] = F.linear(c, w_uk).view(n, bs, H, dn)
+    kt[..., dn:] = rows[..., R:R + rot_dim].unsqueeze(2)
+    vt = F.linear(c, w_uv).view(n, bs, H, dv).permute(0, 2, 3, 1).contiguous()
+    return kt.view(n, bs, H * D), vt
+
+
 _NO_SINK: dict = {}
 
 

@@ -5,7 +5,7 @@ import math
 import pytest
 import torch
 
-from k8s_llm_monitor_amd.ops import hybrid as H
+from k8s_llm_monitor_amd.ops import hybrid as hops
 
 from test_hybrid_ops_gpu import _g, _i32, _paged, _r
 
@@ -36,8 +36,61 @@ def test_window_flash(dk, dv, Hq, G, new, ctx, window, kw):
     sinks = _r(g, Hq) if kw.pop("sinks", False) else None
     gate = _r(g, sum(new), Hq + 8, dt=BF) if kw.pop("gate", False) else None
     a = (Hq, G, dk, dv, 1.0 / math.sqrt(dk), window, kw.pop("sink", False) or sinks is not None)
-    want = H.window_attention_prefill(qkv, kc, vc, cu, _i32(ctx), bt, *a, sinks=sinks, gate=gate, g_col=8 if gate is not None else 0, **kw)
+    want = hops.window_attention_prefill(qkv, kc, vc, cu, _i32(ctx), bt, *a, sinks=sinks, gate=gate, g_col=8 if gate is not None else 0, **kw)
     dev = [x.cuda() for x in (qkv, kc, vc, cu, _i32(ctx), bt)]
-    got = H.window_attention_prefill(*dev, *a, mfma=256, sinks=sinks.cuda() if sinks is not None else None,
+    got = hops.window_attention_prefill(*dev, *a, mfma=256, sinks=sinks.cuda() if sinks is not None else None,
                                      gate=gate.cuda() if gate is not None else None, g_col=8 if gate is not None else 0, **kw)
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("H,R,dn,dr,dv,pages", [(4, 128, 96, 32, 128, 1), (3, 256, 32, 32, 64, 9), (2, 256, 96, 32, 128, 17), (2, 48, 12, 4, 20, 5)])
+def test_latent_expand_and_rotate_heads(H, R, dn, dr, dv, pages):
+    """Temporary pages from listed latent pages (in and out of order, a list that does not fill the last workgroup; the
+    last case: matrix products).  Sums of R bf16 products in fp32, one rounding: 2^-8 of the value."""
+    g = _g(62)
+    pitch = (R + dr + 31) // 32 * 32
+    kc = torch.cat([_r(g, 40, 16, R + dr, dt=BF), torch.zeros(40, 16, pitch - R - dr, dtype=BF)], -1)
+    wk, wv = _r(g, H * dn, R, s=R ** -0.5, dt=BF), _r(g, H * dv, R, s=R ** -0.5, dt=BF)
+    pl = torch.randperm(40, generator=g)[:pages].to(torch.int32)
+    kt, vt = hops.latent_expand(kc, pl, wk, wv, H, R, dr)
+    kg, vg = hops.latent_expand(kc.cuda(), pl.cuda(), wk.cuda(), wv.cuda(), H, R, dr)
+    torch.testing.assert_close(kg.cpu().float(), kt.float(), rtol=1e-2, atol=1e-2)
+    torch.testing.assert_close(vg.cpu().float(), vt.float(), rtol=1e-2, atol=1e-2)
+    for pairs in (False, True):
+        x, pos = _r(g, 7, H * (dn + dr) + 8, dt=BF), torch.randint(0, 3000, (7,), generator=g, dtype=torch.int32)
+        freq = hops.rotary_freq(1e4, dr, "cpu")
+        a, b = x.clone(), x.clone().cuda()
+        hops.rotate_heads(a, H, dn + dr, pos, freq, pairs, dn)
+        hops.rotate_heads(b, H, dn + dr, pos.cuda(), freq.cuda(), pairs, dn)
+        torch.testing.assert_close(b.cpu().float(), a.float(), rtol=1e-2, atol=1e-2)
+
+
+def test_latent_portions_in_the_expanded_form(monkeypatch):
+    """Portions of prompts beside a decode row, their keys expanded from cached and new latents, a layer that reads
+    another's pages; against whole-sequence float64 results and the form over the latent cache."""
+    import bitonex_oracle as O
+    import test_bitonex_model as B
+    from k8s_llm_monitor_amd.models.hybrid import LatentAttention
+
+    cfg = B.make_cfg([B.lat(4, 32, 32, 64, 48, 128, 0.12, 1e4, mlp=B.dense(64)), B.lat(2, 96, 32, 128, 40, 128, 0.09, 1e4, kv_from=0)],
+                     width=128, vocab=211, mult=0.35)
+    w = O.random_weights(cfg, 9)
+    t, u = B.toks(200, cfg["vocab"], 4), B.toks(120, cfg["vocab"], 5)
+    calls = []
+    real = LatentAttention._forward_expanded
+    monkeypatch.setattr(LatentAttention, "_forward_expanded", lambda self, *a: calls.append(1) or real(self, *a))
+
+    def run(min_rows):
+        monkeypatch.setattr(LatentAttention, "EXPAND_MIN_ROWS", min_rows)
+        rig = B.rig_for(cfg, w=w, device="cuda", dtype=BF, num_blocks=48)
+        a = rig.step([("a", t[:90]), ("b", u[:119])])
+        b = rig.step([("a", t[90:161]), ("b", u[119:])], end=["b"])  # a portion behind 90 cached tokens, a decode row
+        c = rig.step([("a", t[161:])], end=["a"])
+        return torch.cat([a["a"], b["a"], c["a"]]), torch.cat([a["b"], b["b"]])
+
+    ga, gb = run(32)
+    assert len(calls) == 6
+    ha, hb = run(1 << 30)
+    for got, form, ref in ((ga, ha, O.forward(cfg, w, t)), (gb, hb, O.forward(cfg, w, u))):
+        B.close_most(got, ref, 0.05, frac=1.0)
+        B.close_most(got, form.double(), 0.02, frac=1.0)
