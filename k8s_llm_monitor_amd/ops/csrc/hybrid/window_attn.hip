@@ -348,7 +348,8 @@ constexpr float kMaxCapPlain = 60.f;
 // 256 pairs per workgroup, or rows that may see enough keys for the shared tiles to pay with few workgroups.  Register
 // kernel at its better width -> staged kernel, us (128-wide heads): 13 prompts x 120, 8 heads (12480 pairs, 120 keys)
 // 9.2 -> 12.5; x 250 21.3 -> 16.6; x 500 52 -> 25; one prompt of 512, 8 heads 20.3 -> 21.7; 1024 38 -> 34; 64 rows
-// behind 2000 keys, 16 heads 70 -> 61.  mfma = kFlashForced asks for it at any size (tests, measurements).
+// behind 2000 keys, 16 heads 70 -> 61.  mfma = kFlashForced asks for it at any size (tests, measurements), 2 for the
+// register kernel whatever the size.
 constexpr long kFlashPairs = 16 * 1024;
 constexpr long kFlashKeys = 1024;
 constexpr int kFlashForced = 256;
@@ -560,7 +561,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
   // bf16 with matrix-core head sizes and 16-byte aligned rows: the MFMA kernel
   if (!f32 && mfma && bs == 16 && q_stride % 8 == 0 && (dk == 64 || dk == 128) && (dv == 64 || dv == 128)) {
     const long keys = window > 0 && window < 16l * bt_stride ? window : 16l * bt_stride;  // at most, per row
-    if (mfma == kFlashForced || (mfma < 16 && (T * Hq >= kFlashPairs || keys >= kFlashKeys))) {
+    if (mfma == kFlashForced || (mfma == 1 && (T * Hq >= kFlashPairs || keys >= kFlashKeys))) {
       const int rc = k8sllm_hy_window_flash(out, qkv, q_stride, k_cache, v_cache, cu, ctx, block_tables, bt_stride, S, T, Hq, G,
                                             dk, dv, scale, window, chunked, keep, cap, cap <= kMaxCapPlain && !sink, sink,
                                             sinks, gate, g_stride, s);
