@@ -75,8 +75,8 @@ int k8sllm_hy_join_norm(void* out, float* residual, const void* y0, int t0, cons
                         long rows, int d, float eps, int f32, hipStream_t s);
 int k8sllm_hy_token_mix(void* out, const float* h, const float* mu, int n, float* state, const int* cu, const int* ctx,
                         const int* slot, int S, long rows, int d, int f32, hipStream_t s);
-int k8sllm_hy_linear_attn_chunk(float* y, const void* vkq, const float* decay, float* state, const int* cu,
-                                const int* ctx, const int* slot, int S, int H, int dk, int dv, int nt, hipStream_t s);
+int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* state, const int* cu, const int* ctx,
+                         const int* slot, int S, int H, int dk, int dv, int nt, hipStream_t s);
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
                      const float* bias, int E, int K, int rows_w, int over_all, int f32, hipStream_t s);
 int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* offsets, const int* sorted_idx, int div,
@@ -433,9 +433,12 @@ void conv_silu(Tensor out, Tensor proj, int64_t col0, Tensor cw, OptT cb, Tensor
 }
 
 // decay given: the fixed-decay recurrence (dt = 1, no skip term); proj, dt_bias, a_log, d_skip are then not read
+// mode 0: with a decay table and G == nh, the chunked matrix-core kernel for bf16 steps with a mean of 32 rows per segment
+// and more whose sizes are its own, else a scan; 1 / 2: a scan in the decode / prompt mapping; 3: the chunked kernel (nt: its
+// value-column tiles per workgroup, 0: its choice), or the scan where it does not apply
 void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, OptT a_log, OptT d_skip, OptT decay,
               Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t nh, int64_t P, int64_t N, int64_t G,
-              int64_t mode) {
+              int64_t mode, int64_t nt) {
   const int f = act(xbc, "xbc");
   f32c(y, "y");
   f32c(state, "ssm_state");
@@ -467,32 +470,17 @@ void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, Opt
   TORCH_CHECK(y.numel() == T * nh * P, "ssm: y [T, nh*P]");
   TORCH_CHECK(state.dim() == 4 && state.size(1) == nh && state.size(2) == N && state.size(3) == P, "ssm_state [slots, nh, N, P]");
   TORCH_CHECK(G >= 1 && nh % G == 0 && N <= 256, "ssm: groups / state size (<= 256)");
+  if (cp != nullptr && !f && G == nh && (mode == 3 || (mode == 0 && T >= 32 * ctx.numel())) &&
+      reinterpret_cast<uintptr_t>(xbc.data_ptr()) % 16 == 0) {
+    const int rc = k8sllm_hy_chunk_scan(y.data_ptr<float>(), xbc.data_ptr(), cp, state.data_ptr<float>(), cu.data_ptr<int>(),
+                                        ctx.data_ptr<int>(), slot.data_ptr<int>(), (int)ctx.numel(), (int)nh, (int)N, (int)P, (int)nt, cur());
+    if (rc != 1) return check(rc, "ssm_scan (chunked)");
+  }
+  if (mode == 3) mode = 0;
   check(k8sllm_hy_ssm_scan(y.data_ptr<float>(), xbc.data_ptr(), pp, pstride, (int)dt_col, bp, ap, dp, cp,
                            state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
                            (int)ctx.numel(), T, (int)nh, (int)P, (int)N, (int)G, f, (int)mode, cur()),
         "ssm_scan");
-}
-
-// The matrix-core (chunked) linear attention for bf16 prompts; false: these sizes or dtype are not the
-// kernel's, nothing was launched.
-bool linear_attention_chunked(Tensor y, Tensor vkq, Tensor decay, Tensor state, Tensor cu, Tensor ctx, Tensor slot,
-                              int64_t H, int64_t dk, int64_t dv, int64_t nt) {
-  if (act(vkq, "vkq") != 0) return false;
-  f32c(y, "y");
-  f32c(decay, "decay");
-  f32c(state, "state");
-  segs(cu, ctx, slot);
-  const int64_t T = vkq.size(0);
-  TORCH_CHECK(vkq.dim() == 2 && vkq.is_contiguous() && vkq.size(1) == H * dv + 2 * H * dk, "vkq [T, H*dv + 2*H*dk]");
-  TORCH_CHECK(y.numel() == T * H * dv && decay.numel() == H, "linear attention: y [T, H*dv], decay [H]");
-  TORCH_CHECK(state.dim() == 4 && state.size(1) == H && state.size(2) == dk && state.size(3) == dv,
-              "state [slots, H, dk, dv]");
-  const int rc = k8sllm_hy_linear_attn_chunk(y.data_ptr<float>(), vkq.data_ptr(), decay.data_ptr<float>(),
-                                             state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(),
-                                             slot.data_ptr<int>(), (int)ctx.numel(), (int)H, (int)dk, (int)dv, (int)nt, cur());
-  if (rc == 1) return false;
-  check(rc, "linear_attention_chunked");
-  return true;
 }
 
 // In place on the fused rows [T, Hq*dk | G*dk | G*dv | ...]: rotary positions on the first 2 * len(freq)
@@ -1100,7 +1088,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rotary_cache", &rotary_cache);
   m.def("rotate_heads", &rotate_heads);
   m.def("latent_expand", &latent_expand);
-  m.def("linear_attention_chunked", &linear_attention_chunked);
   m.def("qk_norm_cache", &qk_norm_cache);
   m.def("window_attention_prefill", &window_attention_prefill);
   m.def("window_attention_decode", &window_attention_decode);

@@ -525,7 +525,7 @@ def window_attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: 
     no value - exp(0), or exp(sinks[h]) for head h where ``sinks`` [Hq] fp32 is given (a learned,
     unscaled logit).  Scores and weights are fp32.  Returns [T, Hq*dv].  GPU, bf16, head sizes
     64 / 128: the matrix-core kernels - tiles staged in LDS for large steps and long contexts, else 16
-    query rows per wave (``mfma`` 0: the any-size wave-per-row kernel; 16 / 32 / 64: the register kernel with
+    query rows per wave (``mfma`` 0: the any-size wave-per-row kernel; 2: the register kernel; 16 / 32 / 64: with
     that many rows per wave; 256: the staged kernel)."""
     T = qkv.shape[0]
     if not qkv.is_cuda:
@@ -796,7 +796,7 @@ def conv_silu(proj: torch.Tensor, col0: int, C: int, conv_w: torch.Tensor, conv_
 def ssm_scan(xbc: torch.Tensor, proj: Optional[torch.Tensor], dt_col: int, dt_bias: Optional[torch.Tensor],
              a_log: Optional[torch.Tensor], d_skip: Optional[torch.Tensor], state: torch.Tensor, seg_cu: torch.Tensor,
              seg_ctx: torch.Tensor, seg_slot: torch.Tensor, nh: int, P: int, N: int, G: int, mode: int = 0,
-             decay: Optional[torch.Tensor] = None) -> torch.Tensor:
+             decay: Optional[torch.Tensor] = None, col_tiles: int = 0) -> torch.Tensor:
     """The selective state-space recurrence, fp32, token by token within each segment:
 
         dt = softplus(proj[t, dt_col + h] + dt_bias[h]);  S <- exp(-exp(a_log[h]) dt) S + dt B_t x_t^T
@@ -804,8 +804,10 @@ def ssm_scan(xbc: torch.Tensor, proj: Optional[torch.Tensor], dt_col: int, dt_bi
 
     ``xbc`` [T, nh*P | G*N | G*N] holds x, B, C (head h reads group h // (nh / G)); ``state``
     [slots, nh, N, P] fp32 is read at the segment's start (zero where seg_ctx is 0) and written
-    back at its end.  Returns y [T, nh*P] fp32.  GPU: two lane mappings of the same arithmetic,
-    chosen by the step's mean segment length (``mode`` 1 / 2 forces the decode / the prompt one).
+    back at its end.  Returns y [T, nh*P] fp32.
+
+    GPU: two lane mappings of the same arithmetic, chosen by the step's mean segment length (``mode`` 1 / 2 forces the
+    decode / the prompt one).
 
     ``decay`` [nh] fp32 (then ``proj``, ``dt_bias``, ``a_log``, ``d_skip`` are not read): the
     recurrence with a fixed decay per head, step size 1 and no skip term,
@@ -840,7 +842,7 @@ def ssm_scan(xbc: torch.Tensor, proj: Optional[torch.Tensor], dt_col: int, dt_bi
         return y
     y = torch.empty(T, nh * P, dtype=torch.float32, device=xbc.device)
     native().ssm_scan(y, xbc, proj, int(dt_col), dt_bias, a_log, d_skip, decay, state, seg_cu, seg_ctx, seg_slot, nh, P,
-                      N, G, int(mode))
+                      N, G, int(mode), int(col_tiles))
     return y
 
 
@@ -855,18 +857,14 @@ def linear_attention(vkq: torch.Tensor, decay: torch.Tensor, state: torch.Tensor
     dv] fp32 is read at a segment's start (zero where seg_ctx is 0) and written back at its end.
     Returns o [T, H*dv] fp32.  State, products and sums are fp32.
 
-    GPU: the sequential scan (``ssm_scan`` with the decay table; ``mode`` 1 / 2 force its decode /
-    prompt lane mapping), or - bf16 prompts (a mean of 32 rows per segment and more), ``dim`` a multiple
-    of 32 up to 128, ``vdim`` a multiple of 16; ``mode`` 3 forces it, ``col_tiles`` 1 / 2 its value
-    columns per workgroup (16 / 32; 0: 16) - chunks of 64 tokens on the matrix
-    cores: q.k on the bf16 instruction, everything that holds scores or state on the fp32 one, only the
-    state crossing chunks (the order of the fp32 sums then follows the chunk grid, which starts at the
-    segment's first row)."""
-    if vkq.is_cuda and vkq.dtype == torch.bfloat16 and (mode == 3 or (mode == 0 and vkq.shape[0] >= 32 * seg_ctx.numel())):
-        y = torch.empty(vkq.shape[0], H * dv, dtype=torch.float32, device=vkq.device)
-        if native().linear_attention_chunked(y, vkq, decay, state, seg_cu, seg_ctx, seg_slot, H, dk, dv, int(col_tiles)):
-            return y
-    return ssm_scan(vkq, None, 0, None, None, None, state, seg_cu, seg_ctx, seg_slot, H, dv, dk, H, mode if mode < 3 else 0, decay=decay)
+    GPU: bf16 prompts (a mean of 32 rows per segment and more), ``dim`` a multiple of 32 up to 128, ``vdim`` of 16
+    (``mode`` 3 forces it, ``col_tiles`` 1 / 2 / 4 its value columns per workgroup, 16 / 32 / 64; 0: its choice): chunks of 64
+    tokens on the matrix cores, only the state crossing chunks - fp32 scores, decays and state enter the products as three
+    bf16 parts that add up to them, so only the order of the fp32 sums differs, which follows the chunk grid from the
+    segment's first row on.  Else the sequential scan (``ssm_scan`` with the decay table; ``mode`` 1 / 2 force its decode /
+    prompt lane mapping)."""
+    return ssm_scan(vkq, None, 0, None, None, None, state, seg_cu, seg_ctx, seg_slot, H, dv, dk, H, mode, decay=decay,
+                    col_tiles=col_tiles)
 
 
 def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.Tensor, z_bias: torch.Tensor,

@@ -94,3 +94,18 @@ def test_latent_portions_in_the_expanded_form(monkeypatch):
     for got, form, ref in ((ga, ha, O.forward(cfg, w, t)), (gb, hb, O.forward(cfg, w, u))):
         B.close_most(got, ref, 0.05, frac=1.0)
         B.close_most(got, form.double(), 0.02, frac=1.0)
+
+
+def _segments(lens, ctx, slot):
+    return _i32([0] + torch.tensor(lens).cumsum(0).tolist()), _i32(ctx), _i32(slot)
+
+
+def test_chunked_linear_attention_negative_decay():
+    g = _g(64)
+    cu, ctx, slot = _segments([70, 129], [0, 2], [1, 0])
+    vkq, decay, state = _r(g, 199, 2 * (32 + 64), s=0.7, dt=BF), torch.tensor([-0.9, -1.0]), _r(g, 2, 2, 32, 32)
+    want_s, got_s = state.clone(), state.cuda()
+    want = hops.linear_attention(vkq, decay, want_s, cu, ctx, slot, 2, 32, 32)
+    got = hops.linear_attention(vkq.cuda(), decay.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), 2, 32, 32, mode=3)
+    for a, b in ((got.cpu(), want), (got_s.cpu(), want_s)):
+        torch.testing.assert_close(a, b, rtol=2e-5, atol=2e-5 * float(b.abs().max()))
