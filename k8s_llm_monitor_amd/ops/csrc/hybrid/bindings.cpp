@@ -75,6 +75,11 @@ int k8sllm_hy_join_norm(void* out, float* residual, const void* y0, int t0, cons
                         long rows, int d, float eps, int f32, hipStream_t s);
 int k8sllm_hy_token_mix(void* out, const float* h, const float* mu, int n, float* state, const int* cu, const int* ctx,
                         const int* slot, int S, long rows, int d, int f32, hipStream_t s);
+long k8sllm_hy_delta_chunk_ws(long T, int S, int H, int dk, int dv);
+int k8sllm_hy_delta_chunk(float* o, const void* qkv, long stride, int q_col, int k_col, int v_col, const void* z, long z_stride,
+                          const float* z_bias, const float* a_log, float inv_tau, int dkind, const void* beta, long b_stride,
+                          float* state, const int* cu, const int* ctx, const int* slot, int S, int H, int Gk, int dk, int dv,
+                          float q_scale, int unit, void* ws, long T, hipStream_t s);
 int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* state, const int* cu, const int* ctx,
                          const int* slot, int S, int H, int dk, int dv, int nt, hipStream_t s);
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
@@ -669,9 +674,11 @@ void rotary_norm_cache(Tensor qkv, int64_t Hq, int64_t G, int64_t dk, int64_t dv
 // (beta given) or with a bonus for the current token (bonus given); see decay_scan.hip.  dkind: how a decay
 // comes from its logit.  z_col: first column of the decay logits in z
 // ws: fp32 workspace of decay_scan_ws(T, ...) floats - given, the two-launch form for prompts runs
+// mode 0: by the step's mean segment length - prompts in chunks on the matrix cores where the form, sizes and alignment
+// are those kernels', else the two-launch scan; 1: the one-launch scan; 2: the two-launch scan; 3: the chunks
 void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_col, Tensor z, Tensor z_bias, OptT a_log,
                 double tau, OptT beta, int64_t beta_col, Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t H,
-                int64_t Gk, int64_t dk, int64_t dv, double q_scale, bool unit, OptT ws, int64_t z_col, int64_t dkind,
+                int64_t Gk, int64_t dk, int64_t dv, double q_scale, bool unit, int64_t mode, int64_t z_col, int64_t dkind,
                 OptT bonus) {
   const int f = act(qkv, "qkv");
   same(z, f, "z");
@@ -714,15 +721,34 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
     bp = (const char*)beta->data_ptr() + beta_col * beta->element_size();
     bstride = beta->stride(0);
   }
+  const int S = (int)ctx.numel();
+  const bool prompts = T >= 32l * S;
+  const void* zp = (const char*)z.data_ptr() + z_col * z.element_size();
+  if (!f && (mode == 3 || (mode == 0 && prompts)) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 &&
+      qkv.stride(0) % 8 == 0 && q_col % 8 == 0 && k_col % 8 == 0 && v_col % 8 == 0) {
+    // a chunk costs the same whatever it holds (us, 16 heads of 128 x 128, scan -> chunks: 40 segments of 33 rows 99 -> 101;
+    // 16 of 64 73 -> 51; one of 64 21 -> 28; 4 of 2048 542 -> 209)
+    if (per_head && (mode == 3 || (T >= 64l * S && T >= 128))) {
+      const long nb = k8sllm_hy_delta_chunk_ws(T, S, (int)H, (int)dk, (int)dv);
+      if (nb > 0) {
+        Tensor ws = torch::empty({nb}, o.options().dtype(torch::kUInt8));
+        return check(k8sllm_hy_delta_chunk(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
+                                           zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, bp,
+                                           bstride, state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(),
+                                           slot.data_ptr<int>(), S, (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale, unit,
+                                           ws.data_ptr(), (long)T, cur()),
+                     "decay_scan (chunks)");
+      }
+    }
+  }
+  Tensor ws;
   float* wp = nullptr;
-  if (ws.has_value()) {
-    f32c(*ws, "workspace");
-    TORCH_CHECK(ws->numel() >= k8sllm_hy_decay_scan_ws(T, (int)H, (int)Gk, (int)dk), "decay_scan: workspace too small");
-    wp = ws->data_ptr<float>();
+  if (mode == 2 || (mode != 1 && prompts)) {
+    ws = torch::empty({k8sllm_hy_decay_scan_ws(T, (int)H, (int)Gk, (int)dk)}, o.options());
+    wp = ws.data_ptr<float>();
   }
   check(k8sllm_hy_decay_scan(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
-                             (const char*)z.data_ptr() + z_col * z.element_size(), z.stride(0), z_bias.data_ptr<float>(), ap,
-                             (float)(1.0 / tau), (int)dkind, per_head, bp, bstride, wp_bonus, state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
+                             zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, per_head, bp, bstride, wp_bonus, state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
                              (int)ctx.numel(), (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale, unit, f, wp, (long)T, cur()),
         "decay_scan");
 }

@@ -896,9 +896,11 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     sums are fp32.
 
     GPU: steps of prompts (a mean segment length of 32 rows or more) run as two launches - everything
-    that does not depend on the state (decays, unit norms, k . q, beta) for all rows at once into an fp32
-    workspace, then the recurrence over it; decode steps run as one launch.  ``mode`` 1 / 2 force the
-    one-launch / two-launch form (tests)."""
+    that does not depend on the state (decays, unit norms, k . q, beta) for all rows at once into a
+    workspace, then the recurrence over it; decode steps run as one launch.  bf16 prompts of the delta rule with one decay
+    per head (``dk`` a multiple of 32 up to 128, ``dv`` of 16) go in chunks of 64 tokens on the matrix cores, fp32 operands as
+    three bf16 parts that add up to them; else token by token.  ``mode`` 1 / 2 force the one-launch / two-launch
+    scan, 3 the chunks (tests)."""
     T = qkv.shape[0]
     nz = z_bias.numel()
     dkind = 0 if a_log is not None else 2 if decay == "exp_exp" else 1
@@ -944,11 +946,8 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
             state[slot] = S
         return o
     o = torch.empty(T, H * dv, dtype=torch.float32, device=qkv.device)
-    ws = None
-    if mode == 2 or (mode == 0 and T >= 32 * seg_slot.numel()):
-        ws = torch.empty(T * (2 * Gk * dk + H * dk + Gk + H), dtype=torch.float32, device=qkv.device)
     native().decay_scan(o, qkv, int(q_col), int(k_col), int(v_col), z, z_bias, a_log, float(tau), beta, int(beta_col),
-                        state, seg_cu, seg_ctx, seg_slot, int(H), int(Gk), int(dk), int(dv), float(q_scale), bool(unit), ws, int(z_col), dkind,
+                        state, seg_cu, seg_ctx, seg_slot, int(H), int(Gk), int(dk), int(dv), float(q_scale), bool(unit), int(mode), int(z_col), dkind,
                         bonus)
     return o
 

@@ -109,3 +109,33 @@ def test_chunked_linear_attention_negative_decay():
     got = hops.linear_attention(vkq.cuda(), decay.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), 2, 32, 32, mode=3)
     for a, b in ((got.cpu(), want), (got_s.cpu(), want_s)):
         torch.testing.assert_close(a, b, rtol=2e-5, atol=2e-5 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("H,Gk,dk,dv", [(4, 2, 128, 128), (2, 2, 32, 16), (3, 1, 64, 48), (2, 1, 96, 32)])
+@pytest.mark.parametrize("kind", ["slow", "fast", "root", "plain_keys"])
+def test_chunked_delta_rule(H, Gk, dk, dv, kind):
+    """The delta rule with one decay per head in chunks of 64 tokens: segments around the chunk size, continued ones, a padding
+    one, decays near one and down to zero, keys that repeat (the triangular solve's worst case) and keys that are no unit
+    vectors.  fp32 sums in another order through a recurrence of a few hundred tokens: 5e-5 of the result's scale."""
+    g = _g(65)
+    lens = [1, 63, 64, 65, 200, 7, 130, 128]
+    cu, ctx, slot = _segments(lens, [0, 5, 0, 64, 0, 3, 9, 1], [0, 1, 2, 3, 4, -1, 5, 6])
+    T = sum(lens)
+    qkv = _r(g, T, 2 * Gk * dk + H * dv, dt=BF)
+    qkv[100:160, Gk * dk:2 * Gk * dk] = qkv[100, Gk * dk:2 * Gk * dk]  # equal keys in a row
+    kw = dict(unit=True, a_log=_r(g, H, s=0.5))
+    if kind == "plain_keys":
+        kw["unit"] = False
+        qkv[:, :2 * Gk * dk] *= 0.7 * dk ** -0.5
+    if kind == "root":
+        kw = dict(unit=True, tau=4.0)
+    z, zb = _r(g, T, H + 3, s=4.0 if kind == "fast" else 1.0, dt=BF), _r(g, H) - (4.0 if kind != "fast" else -1.0) * (1 if kind != "root" else -1)
+    beta, state = _r(g, T, H + 2, dt=BF), _r(g, 7, H, dv, dk)
+    want_s, got_s = state.clone(), state.cuda()
+    a = (0, Gk * dk, 2 * Gk * dk)
+    want = hops.decay_scan(qkv, *a, z, zb, want_s, cu, ctx, slot, H, Gk, dk, dv, dk ** -0.5, beta=beta, beta_col=2, z_col=3, **kw)
+    dev = {k: v.cuda() if isinstance(v, torch.Tensor) else v for k, v in kw.items()}
+    got = hops.decay_scan(qkv.cuda(), *a, z.cuda(), zb.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), H, Gk, dk, dv, dk ** -0.5,
+                          beta=beta.cuda(), beta_col=2, z_col=3, mode=3, **dev)
+    for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
+        torch.testing.assert_close(x, y, rtol=5e-5, atol=5e-5 * float(y.abs().max()))
