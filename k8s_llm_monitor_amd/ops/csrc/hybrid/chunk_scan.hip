@@ -103,7 +103,7 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
   fetch(t0, min(kCsChunk, t1 - t0));
   for (int tb = t0; tb < t1; tb += kCsChunk) {
     const int n = min(kCsChunk, t1 - tb);
-    __syncthreads();  // the previous chunk's reads of Kl, Vl, Sl are done (and lam is written)
+    lds_barrier();  // the previous chunk's reads of Kl, Vl, Sl are done (and lam is written)
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       const int idx = tid + 512 * u, row = idx / (DK / 8), c8 = idx - row * (DK / 8);
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
     bf16x8 qf[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = qn[ks];
-    __syncthreads();
+    lds_barrier();
     if (tb + kCsChunk < t1) {  // in flight during the products
       fetch(tb + kCsChunk, min(kCsChunk, t1 - tb - kCsChunk));
     }

@@ -363,7 +363,7 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
     }
     dl = dn;
     if (tb + kChunk < t1) fetch(tb + kChunk);
-    __syncthreads();  // Sl is written, Rl has been read
+    lds_barrier();  // Sl is written, Rl has been read
     // outs: (S^T Q^T)[column 16 ct + 4 quad + i][query c16]; else (K S)[token 4 quad + i][column c16]
     f32x4 acc[NT];
 #pragma unroll
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
           *reinterpret_cast<uint2*>(&Rl[k][(16 * ct + c16) * kDcP + 16 * w + 4 * quad]) = make_uint2(p[k][0], p[k][1]);
       }
     }
-    __syncthreads();  // Rl is written, Sl has been read
+    lds_barrier();  // Rl is written, Sl has been read
     if (outs) {
       if (16 * w < n) {
 #pragma unroll

@@ -36,6 +36,10 @@ __device__ __forceinline__ bf16x8 frag(const uint32_t* w) {
   return __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
 }
 
+// A workgroup barrier for data that passes through LDS: unlike __syncthreads() it leaves global loads in flight (a
+// prefetch across the barrier) instead of waiting for them.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // An operand fragment whose k index runs down the rows of a row-major LDS matrix (row pitch in elements): this lane's
 // column c0 + (lane & 15), rows r0 .. r0 + 3 and r1 .. r1 + 3.  The transposing read takes, for 16 lanes, four rows of 16
 // columns and gives each lane one column's four rows.

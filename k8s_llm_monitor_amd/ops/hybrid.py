@@ -898,8 +898,9 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     GPU: steps of prompts (a mean segment length of 32 rows or more) run as two launches - everything
     that does not depend on the state (decays, unit norms, k . q, beta) for all rows at once into a
     workspace, then the recurrence over it; decode steps run as one launch.  bf16 prompts of the delta rule with one decay
-    per head (``dk`` a multiple of 32 up to 128, ``dv`` of 16) go in chunks of 64 tokens on the matrix cores, fp32 operands as
-    three bf16 parts that add up to them; else token by token.  ``mode`` 1 / 2 force the one-launch / two-launch
+    per head, and without the delta rule and unit norms of decays per channel (``dk`` a multiple of 32 up to 128, ``dv`` of
+    16), go in chunks of 64 tokens on the matrix cores, fp32 operands as three bf16 parts that add up to them; else token by
+    token.  ``mode`` 1 / 2 force the one-launch / two-launch
     scan, 3 the chunks (tests)."""
     T = qkv.shape[0]
     nz = z_bias.numel()

@@ -139,3 +139,28 @@ def test_chunked_delta_rule(H, Gk, dk, dv, kind):
                           beta=beta.cuda(), beta_col=2, z_col=3, mode=3, **dev)
     for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
         torch.testing.assert_close(x, y, rtol=5e-5, atol=5e-5 * float(y.abs().max()))
+
+
+@pytest.mark.parametrize("H,Gk,dk,dv", [(4, 4, 64, 64), (2, 2, 32, 16), (3, 3, 128, 48), (2, 2, 96, 32), (4, 2, 64, 128)])
+@pytest.mark.parametrize("kind", ["bonus", "bonus_fast", "root", "softplus_fast"])
+def test_chunked_channel_decays(H, Gk, dk, dv, kind):
+    """Decays per key channel in chunks of 64 tokens, plain and with a bonus: segments around the chunk size and its sub-blocks
+    of 16, continued ones, a padding one, channels that keep hundreds of tokens beside channels that forget at once (their
+    sums leave the fp32 range of 2^x).  fp32 sums of a few hundred terms in another order: 2e-5 of the result's scale."""
+    if kind.startswith("bonus") and Gk != H:
+        pytest.skip("a bonus goes with a key head per head")
+    g = _g(66)
+    lens = [1, 63, 64, 65, 200, 7, 130, 128, 16, 17, 48]
+    cu, ctx, slot = _segments(lens, [0, 5, 0, 64, 0, 3, 9, 1, 0, 2, 0], [0, 1, 2, 3, 4, -1, 5, 6, 7, 8, 9])
+    T = sum(lens)
+    qkv = _r(g, T, 2 * Gk * dk + H * dv, dt=BF)
+    z, zb, state = _r(g, T, H * dk, s=2.0, dt=BF), _r(g, H * dk, s=2.0), _r(g, 10, H, dv, dk)
+    kw = dict(decay="exp_exp", bonus=_r(g, H, dk)) if kind.startswith("bonus") else dict(tau=3.0) if kind == "root" else dict(a_log=_r(g, H) + 2.0)
+    zb += {"bonus": -3.0, "bonus_fast": 2.0, "root": 3.0, "softplus_fast": 1.0}[kind]
+    want_s, got_s = state.clone(), state.cuda()
+    a = (0, Gk * dk, 2 * Gk * dk)
+    want = hops.decay_scan(qkv, *a, z, zb, want_s, cu, ctx, slot, H, Gk, dk, dv, dk ** -0.5, **kw)
+    dev = {k: v.cuda() if isinstance(v, torch.Tensor) else v for k, v in kw.items()}
+    got = hops.decay_scan(qkv.cuda(), *a, z.cuda(), zb.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), H, Gk, dk, dv, dk ** -0.5, mode=3, **dev)
+    for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
+        torch.testing.assert_close(x, y, rtol=2e-5, atol=2e-5 * float(y.abs().max()))
