@@ -285,6 +285,7 @@ class ModelRunner:
             meta.block_tables = dv["bt"].view(len(seqs), W)
         if hy:
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = dv["gcu"], dv["gctx"], dv["gslot"]
+            meta.seg_max = max([1] * (nd > 0) + lens)
             if seqs:
                 meta.page_list, meta.page_bt = dv["pgl"], dv["pgb"].view(len(seqs), W)
         if kA:
@@ -340,6 +341,7 @@ class ModelRunner:
                         dec_src=self.d_src[:b], dec_prev=self.d_out)
         if self.hybrid:  # one-token segments: the tokens before this one are its position
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = self.d_rows[:b + 1], self.d_pos[:b], self.d_state[:b]
+            meta.seg_max = 1
         logits = self.model.forward(self.d_ids[:b], meta, self.kv)
         if self.cfg.keep_logits:
             if self.d_logits is None:

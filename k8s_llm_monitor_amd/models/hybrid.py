@@ -729,7 +729,8 @@ class Mamba1Mixer:
         x = hops.conv_silu(proj, 0, C, self.conv_w, self.conv_b, cache["conv"], *seg)
         q = F.linear(x, self.w_x)
         dt = F.linear(q[:, :r], self.w_dt)
-        y = hops.selective_scan(x, q, r, r + N, dt, self.dt_bias, self.a_log, self.d_skip, proj, C, cache["state"], *seg)
+        y = hops.selective_scan(x, q, r, r + N, dt, self.dt_bias, self.a_log, self.d_skip, proj, C, cache["state"], *seg,
+                                meta.seg_max)
         return F.linear(y, self.wo)
 
     def export(self, p: str) -> dict:

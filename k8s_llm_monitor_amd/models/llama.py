@@ -80,6 +80,7 @@ class AttnMeta:
     seg_cu: Optional[torch.Tensor] = None
     seg_ctx: Optional[torch.Tensor] = None
     seg_slot: Optional[torch.Tensor] = None
+    seg_max: int = 0  # rows of the longest segment (0: not known)
     # prefill: every chunk of this step starts at position 0 (whole prompts, nothing cached before)
     all_fresh: bool = False
     # layer-list prefill: the pages of every chunk's sequence up to its last token of this step, sequence after

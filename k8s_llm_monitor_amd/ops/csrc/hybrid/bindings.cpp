@@ -69,7 +69,8 @@ int k8sllm_hy_ssm_scan(float* y, const void* xbc, const void* proj, long p_strid
 int k8sllm_hy_selective_scan(void* out, const void* xc, const void* q, long q_stride, int b_col, int c_col,
                              const void* dt, long dt_stride, const float* dt_bias, const float* a_log, const float* d_skip,
                              const void* z, long z_stride, float* state, const int* cu, const int* ctx, const int* slot,
-                             int S, long T, int C, int N, int f32, hipStream_t s);
+                             int S, long T, int C, int N, int f32, float* ws, hipStream_t s);
+long k8sllm_hy_selective_scan_ws(long T, int S, int longest, int C, int N, int mode);
 int k8sllm_hy_join_norm(void* out, float* residual, const void* y0, int t0, const void* y1, int t1, const float* w0,
                         const float* w1, float mix, const float* pw, const float* pb, const float* nw, const float* nb,
                         long rows, int d, float eps, int f32, hipStream_t s);
@@ -772,9 +773,10 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
 }
 
 // The selective state-space recurrence with a decay per channel and state; see selective_scan.hip.  q holds
-// the state inputs B and read-outs C from columns b_col, c_col on; proj's columns z_col .. are the output gate
+// the state inputs B and read-outs C from columns b_col, c_col on; proj's columns z_col .. are the output gate.
+// longest: rows of the longest segment (0: not known); mode: 0 chosen by the sizes, 1 whole segments, 2 cut into spans
 void selective_scan(Tensor out, Tensor xc, Tensor q, int64_t b_col, int64_t c_col, Tensor dt, Tensor dt_bias, Tensor a_log,
-                    Tensor d_skip, Tensor proj, int64_t z_col, Tensor state, Tensor cu, Tensor ctx, Tensor slot) {
+                    Tensor d_skip, Tensor proj, int64_t z_col, Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t longest, int64_t mode) {
   const int f = act(xc, "xc");
   same(out, f, "out");
   same(q, f, "q");
@@ -797,11 +799,13 @@ void selective_scan(Tensor out, Tensor xc, Tensor q, int64_t b_col, int64_t c_co
   TORCH_CHECK(proj.dim() == 2 && proj.stride(1) == 1 && proj.size(0) == T && z_col >= 0 && z_col + C <= proj.size(1),
               "selective_scan: gate columns");
   TORCH_CHECK(state.dim() == 3 && state.size(1) == C && state.size(2) == N, "state [slots, C, N]");
+  const long n_ws = k8sllm_hy_selective_scan_ws((long)T, (int)ctx.numel(), (int)longest, (int)C, (int)N, (int)mode);
+  Tensor ws = n_ws > 0 ? at::empty({n_ws}, state.options()) : Tensor();
   check(k8sllm_hy_selective_scan(out.data_ptr(), xc.data_ptr(), q.data_ptr(), q.stride(0), (int)b_col, (int)c_col, dt.data_ptr(),
                                  dt.stride(0), dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), d_skip.data_ptr<float>(),
                                  (const char*)proj.data_ptr() + z_col * proj.element_size(), proj.stride(0),
                                  state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
-                                 (int)ctx.numel(), T, (int)C, (int)N, f, cur()),
+                                 (int)ctx.numel(), T, (int)C, (int)N, f, n_ws > 0 ? ws.data_ptr<float>() : nullptr, cur()),
         "selective_scan");
 }
 

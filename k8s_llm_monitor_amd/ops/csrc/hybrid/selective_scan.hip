@@ -15,8 +15,15 @@
 // workgroup adds the skip term, applies the gate and stores rows.  Loads are not predicated: a token past
 // the segment reads the segment's last row, a channel past the end the last channel, and what they must
 // not contribute is zeroed when it is staged - a branch around a load would wait for it there.
-// One exponential per state and token (v_exp_f32 in base 2, log2 e folded into the factor) is what bounds it.
-#include "hy_common.h"
+// One exponential per state and token (v_exp_f32 in base 2, log2 e folded into the factor) bounds a wave, and the chain of
+// tokens a launch with few sequences: there long segments are cut into spans of 128 or 256 tokens that run side by side (MODE
+// kSpanEnds, then kSpanRun).  The first launch runs every span but a segment's last from a zero state and keeps its end E and
+// its sum of step sizes s; since a span's decays multiply to exp(-exp(a_log) s), the state before span k is
+//     I;  then for j = 0 .. k - 1:  S <- exp(-exp(a_log) s_j) S + E_j
+// which the second launch folds in front of its own tokens (I, the state the segment starts from, is kept in the last span's
+// place, so that no workgroup reads the slot that another one writes).  One prompt of 8192 tokens, 4096 channels x 16 states:
+// 1072 us whole, 290 in spans, each launch at the rate of its exponentials and multiply-adds; 2048 tokens 265 -> 86.
+#include "chunk_seg.h"
 
 namespace k8sllm {
 
@@ -31,12 +38,15 @@ __device__ __forceinline__ float softplus_fast(float x) {
   return fmaxf(x, 0.f) + (e < 0.03125f ? series : lg);
 }
 
-template <typename T, int LPC, int NPL>
+constexpr int kWhole = 0, kSpanEnds = 1, kSpanRun = 2;
+
+template <typename T, int LPC, int NPL, int MODE>
 __global__ __launch_bounds__(256) void selective_scan_kernel(
     T* __restrict__ out, const T* __restrict__ xc, const T* __restrict__ q, long q_stride, int b_col, int c_col,
     const T* __restrict__ dt, long dt_stride, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
     const float* __restrict__ d_skip, const T* __restrict__ z, long z_stride, float* __restrict__ state,
-    const int* __restrict__ cu, const int* __restrict__ ctx, const int* __restrict__ slot, int C, int N) {
+    const int* __restrict__ cu, const int* __restrict__ ctx, const int* __restrict__ slot, int n_seg, int span, int C, int N,
+    float* __restrict__ ends, float* __restrict__ sums) {
   constexpr int TB = 16, PB = 256 / LPC, NS = LPC * NPL;
   constexpr int NV = TB * PB / 256;           // (token, channel) pairs a thread stages and finishes
   constexpr int NB = (TB * NS + 255) / 256;   // B / C elements a thread stages
@@ -44,9 +54,14 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   __shared__ __attribute__((aligned(16))) float Cs[TB][NS];
   __shared__ float dts[TB][PB], us[TB][PB];
   __shared__ float ys[TB][PB + 64 / LPC];  // padded: the lanes of a channel write neighbouring rows to different banks
-  const int s = blockIdx.x;
+  ChunkAt at = {(int)blockIdx.x, 0, 0, 0, 1};
+  if (MODE != kWhole) {
+    at = chunk_at(cu, n_seg, blockIdx.x, span);
+    if (at.seg < 0 || (MODE == kSpanEnds && (at.k == at.count - 1 || slot[at.seg] < 0))) return;
+  }
+  const int s = at.seg;
   const int sl = slot[s];
-  const int t0 = cu[s], t1 = cu[s + 1];
+  const int t0 = MODE == kWhole ? cu[s] : at.row, t1 = MODE == kWhole ? cu[s + 1] : at.row + at.n;
   const int pc = threadIdx.x % PB, tt0 = threadIdx.x / PB;  // staging: channel pc, tokens tt0 + LPC u
   const int cs = blockIdx.y * PB + pc;
   const bool slive = cs < C;
@@ -61,7 +76,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   const int c = blockIdx.y * PB + pl, n0 = chunk * NPL;
   const bool live = c < C;
   const bool vec = (N & 3) == 0 && n0 + NPL <= N;
-  const bool carried = ctx[s] > 0;
+  const bool carried = ctx[s] > 0 && (MODE == kWhole || at.count == 1 || (MODE == kSpanEnds && at.k == 0));
   float S[NPL], A[NPL];
   float* sp = state + ((long)sl * C + c) * N + n0;
   const float* ap = a_log + (long)c * N + n0;
@@ -84,6 +99,43 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
       S[i] = (in && carried) ? sp[i] : 0.f;
     }
   }
+  // span j's end state of this channel; the state that a segment of several spans starts from goes to the last one's place
+  auto end_of = [&](int j) { return ends + (((long)blockIdx.x - at.k + j) * C + min(c, C - 1)) * N; };
+  auto read = [&](float (&v)[NPL], const float* p) {
+#pragma unroll
+    for (int i = 0; i < NPL; i += 4) {
+      if (vec) {
+        const float4 f = *reinterpret_cast<const float4*>(p + n0 + i);
+        v[i] = f.x; v[i + 1] = f.y; v[i + 2] = f.z; v[i + 3] = f.w;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[i + j] = p[min(n0 + i + j, N - 1)];
+      }
+    }
+  };
+  if (MODE == kSpanEnds && at.k == 0) {
+    float* ip = end_of(at.count - 1);
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) {
+      if (live && n0 + i < N) ip[n0 + i] = S[i];
+      S[i] = 0.f;
+    }
+  }
+  if (MODE == kSpanRun && at.count > 1) {
+    read(S, end_of(at.count - 1));
+#pragma unroll 4
+    for (int j = 0; j < at.k; ++j) {
+      float E[NPL];
+      read(E, end_of(j));
+      const float d = sums[((long)blockIdx.x - at.k + j) * C + min(c, C - 1)];
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) S[i] = __builtin_amdgcn_exp2f(d * A[i]) * S[i] + E[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NPL; ++i)
+      if (n0 + i >= N) S[i] = 0.f;
+  }
+  float dsum = 0.f;
   const float bias = slive ? dt_bias[cs] : 0.f, D = slive ? d_skip[cs] : 0.f;
   T rd[NV], rx[NV], rz[NV], rB[NB], rC[NB];
   const int cl = min(cs, C - 1);
@@ -93,14 +145,14 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
       const long t = min(tb + tt0 + LPC * u, t1 - 1);
       rd[u] = dt[t * dt_stride + cl];
       rx[u] = xc[t * C + cl];
-      rz[u] = z[t * z_stride + cl];
+      if (MODE != kSpanEnds) rz[u] = z[t * z_stride + cl];
     }
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
       const int i = threadIdx.x + 256 * u;
       const T* row = q + (long)min(tb + i / NS, t1 - 1) * q_stride + min(i % NS, N - 1);
       rB[u] = row[b_col];
-      rC[u] = row[c_col];
+      if (MODE != kSpanEnds) rC[u] = row[c_col];
     }
   };
   auto token = [&](int tt) -> float {  // the recurrence for one staged token; the channel's read-out on all its lanes
@@ -109,12 +161,17 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
 #pragma unroll
     for (int i = 0; i < NPL; i += 4) {
       const float4 b = *reinterpret_cast<const float4*>(&Bs[tt][n0 + i]);
-      const float4 g = *reinterpret_cast<const float4*>(&Cs[tt][n0 + i]);
+      float4 g;
+      if (MODE != kSpanEnds) g = *reinterpret_cast<const float4*>(&Cs[tt][n0 + i]);
       S[i] = __builtin_amdgcn_exp2f(d * A[i]) * S[i] + u * b.x;
       S[i + 1] = __builtin_amdgcn_exp2f(d * A[i + 1]) * S[i + 1] + u * b.y;
       S[i + 2] = __builtin_amdgcn_exp2f(d * A[i + 2]) * S[i + 2] + u * b.z;
       S[i + 3] = __builtin_amdgcn_exp2f(d * A[i + 3]) * S[i + 3] + u * b.w;
-      acc += S[i] * g.x + S[i + 1] * g.y + S[i + 2] * g.z + S[i + 3] * g.w;
+      if (MODE != kSpanEnds) acc += S[i] * g.x + S[i + 1] * g.y + S[i + 2] * g.z + S[i + 3] * g.w;
+    }
+    if (MODE == kSpanEnds) {
+      dsum += d;
+      return 0.f;
     }
     return lanes_sum<LPC>(acc);
   };
@@ -127,7 +184,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
       const int tt = tt0 + LPC * u;
       const float d = softplus_fast(ldf(&rd[u]) + bias);
       ex[u] = ldf(&rx[u]);
-      ez[u] = ldf(&rz[u]);
+      if (MODE != kSpanEnds) ez[u] = ldf(&rz[u]);
       dts[tt][pc] = d;
       us[tt][pc] = d * ex[u];
     }
@@ -137,11 +194,17 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
       const bool in = i % NS < N;  // states beyond N stay zero
       if (NB * 256 == TB * NS || i < TB * NS) {
         (&Bs[0][0])[i] = in ? ldf(&rB[u]) : 0.f;
-        (&Cs[0][0])[i] = in ? ldf(&rC[u]) : 0.f;
+        if (MODE != kSpanEnds) (&Cs[0][0])[i] = in ? ldf(&rC[u]) : 0.f;
       }
     }
     __syncthreads();
     if (tb + TB < t1) fetch(tb + TB);
+    if (MODE == kSpanEnds) {  // whole tiles: a span that is not its segment's last holds `span` tokens
+#pragma unroll
+      for (int tt = 0; tt < TB; ++tt) token(tt);
+      __syncthreads();
+      continue;
+    }
     if (nt == TB) {
 #pragma unroll
       for (int t4 = 0; t4 < TB; t4 += LPC) {
@@ -166,7 +229,11 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
       if (slive && tt < nt) stf(out + (long)(tb + tt) * C + cs, (ys[tt][pc] + D * ex[u]) * silu_f(ez[u]));
     }
   }
-  if (live) {
+  if (MODE == kSpanEnds) {
+    sp = end_of(at.k) + n0;
+    if (live && chunk == 0) sums[(long)blockIdx.x * C + c] = dsum;
+  }
+  if (live && (MODE != kSpanRun || at.k == at.count - 1)) {
     if (vec) {
 #pragma unroll
       for (int i = 0; i < NPL; i += 4) *reinterpret_cast<float4*>(sp + i) = make_float4(S[i], S[i + 1], S[i + 2], S[i + 3]);
@@ -182,37 +249,72 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
 
 using namespace k8sllm;
 
+static long channel_groups(int C, int N) {  // workgroups per segment or span
+  const int lpc = N <= 8 ? 2 : N <= 16 ? 4 : N <= 64 ? 8 : 16;
+  return (C + 256 / lpc - 1) / (256 / lpc);
+}
+
+// A span of 128 costs a workgroup 17 us and its longest fold grows with their number; from where spans of 256 give every
+// compute unit four workgroups, these are faster (one prompt of 8192, 4096 channels x 16: 300 us against 321; of 2048: 111
+// against 88).
+static int span_tokens(long T, int C, int N) { return T * channel_groups(C, N) >= 256l * 1024 ? 256 : 128; }
+
 template <typename T>
 static int launch_selective(void* out, const void* xc, const void* q, long q_stride, int b_col, int c_col, const void* dt,
                             long dt_stride, const float* dt_bias, const float* a_log, const float* d_skip, const void* z,
                             long z_stride, float* state, const int* cu, const int* ctx, const int* slot, int S, int C,
-                            int N, hipStream_t s) {
-#define K8SLLM_SS(LPC, NPL)                                                                                          \
-  hipLaunchKernelGGL((selective_scan_kernel<T, LPC, NPL>), dim3((unsigned)S, (unsigned)((C + 256 / LPC - 1) / (256 / LPC))), \
-                     dim3(256), 0, s, (T*)out, (const T*)xc, (const T*)q, q_stride, b_col, c_col, (const T*)dt, dt_stride,   \
-                     dt_bias, a_log, d_skip, (const T*)z, z_stride, state, cu, ctx, slot, C, N)
-  if (N <= 8) K8SLLM_SS(2, 4);
-  else if (N <= 16) K8SLLM_SS(4, 4);
-  else if (N <= 32) K8SLLM_SS(8, 4);
-  else if (N <= 64) K8SLLM_SS(8, 8);
-  else if (N <= 128) K8SLLM_SS(16, 8);
-  else if (N <= 256) K8SLLM_SS(16, 16);
+                            int N, long T_, float* ws, hipStream_t s) {
+  const int span = span_tokens(T_, C, N);
+  const long spans = T_ / span + S;
+  float* sums = ws + spans * C * N;
+#define K8SLLM_SSM(LPC, NPL, MODE)                                                                                           \
+  hipLaunchKernelGGL((selective_scan_kernel<T, LPC, NPL, MODE>),                                                               \
+                     dim3((unsigned)(MODE == kWhole ? S : spans), (unsigned)((C + 256 / LPC - 1) / (256 / LPC))), dim3(256), 0, s, \
+                     (T*)out, (const T*)xc, (const T*)q, q_stride, b_col, c_col, (const T*)dt, dt_stride, dt_bias, a_log,       \
+                     d_skip, (const T*)z, z_stride, state, cu, ctx, slot, S, span, C, N, ws, sums)
+#define K8SLLM_SS(LPC, NPL)                  \
+  if (ws != nullptr) {                       \
+    K8SLLM_SSM(LPC, NPL, kSpanEnds);         \
+    K8SLLM_SSM(LPC, NPL, kSpanRun);          \
+  } else {                                   \
+    K8SLLM_SSM(LPC, NPL, kWhole);            \
+  }
+  if (N <= 8) { K8SLLM_SS(2, 4); }
+  else if (N <= 16) { K8SLLM_SS(4, 4); }
+  else if (N <= 32) { K8SLLM_SS(8, 4); }
+  else if (N <= 64) { K8SLLM_SS(8, 8); }
+  else if (N <= 128) { K8SLLM_SS(16, 8); }
+  else if (N <= 256) { K8SLLM_SS(16, 16); }
   else return -1;
 #undef K8SLLM_SS
+#undef K8SLLM_SSM
   return (int)hipGetLastError();
 }
 
 extern "C" {
 
-// xc, out [T][C] contiguous; q's rows hold B from b_col on and C from c_col on (N each)
+// floats of workspace for a step of T rows in S segments, the longest of `longest` rows (0: not known, the mean is taken), that
+// is to be cut into spans; 0: it runs whole (mode 1 / 2: whole / cut whatever the sizes).  Whole, a step takes as long as its
+// longest segment's chain, 0.13 us a token, or as all its workgroups' tokens, 467 at a time; cut, twice the latter and what the
+// spans' own chains and the folds come to, about 200 tokens' time.  Measured (4096 channels x 16, whole against cut): one
+// prompt of 384 53 / 38 us, of 8192 1072 / 300; two of 4096 547 / 286; four of 2048 274 / 275; eight of 1024 211 / 287; one of
+// 2048 beside 24 single tokens 322 / 115.
+long k8sllm_hy_selective_scan_ws(long T, int S, int longest, int C, int N, int mode) {
+  const long n = longest > 0 ? longest : S > 0 ? T / S : 0;
+  const bool cut = mode == 2 || (mode == 0 && n >= 200 + T * channel_groups(C, N) / 233);
+  return cut ? (T / span_tokens(T, C, N) + S) * C * (N + 1) : 0;
+}
+
+// xc, out [T][C] contiguous; q's rows hold B from b_col on and C from c_col on (N each); ws: nullptr, or the workspace of a
+// step cut into spans
 int k8sllm_hy_selective_scan(void* out, const void* xc, const void* q, long q_stride, int b_col, int c_col,
                              const void* dt, long dt_stride, const float* dt_bias, const float* a_log, const float* d_skip,
                              const void* z, long z_stride, float* state, const int* cu, const int* ctx, const int* slot,
-                             int S, long T, int C, int N, int f32, hipStream_t s) {
+                             int S, long T, int C, int N, int f32, float* ws, hipStream_t s) {
   if (S <= 0 || T <= 0) return 0;
   if (C < 1 || N < 1) return -1;
 #define K8SLLM_ARGS \
-  out, xc, q, q_stride, b_col, c_col, dt, dt_stride, dt_bias, a_log, d_skip, z, z_stride, state, cu, ctx, slot, S, C, N, s
+  out, xc, q, q_stride, b_col, c_col, dt, dt_stride, dt_bias, a_log, d_skip, z, z_stride, state, cu, ctx, slot, S, C, N, T, ws, s
   return f32 ? launch_selective<float>(K8SLLM_ARGS) : launch_selective<bf16_t>(K8SLLM_ARGS);
 #undef K8SLLM_ARGS
 }

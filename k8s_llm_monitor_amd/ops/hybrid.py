@@ -955,7 +955,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
 
 def selective_scan(xc: torch.Tensor, q: torch.Tensor, b_col: int, c_col: int, dt: torch.Tensor, dt_bias: torch.Tensor,
                    a_log: torch.Tensor, d_skip: torch.Tensor, proj: torch.Tensor, z_col: int, state: torch.Tensor,
-                   seg_cu: torch.Tensor, seg_ctx: torch.Tensor, seg_slot: torch.Tensor) -> torch.Tensor:
+                   seg_cu: torch.Tensor, seg_ctx: torch.Tensor, seg_slot: torch.Tensor, longest: int = 0, mode: int = 0) -> torch.Tensor:
     """The selective state-space recurrence with a decay per channel and state, fp32, token by token within
     each segment, and its output gate.  Per channel c and state n:
 
@@ -964,7 +964,8 @@ def selective_scan(xc: torch.Tensor, q: torch.Tensor, b_col: int, c_col: int, dt
 
     ``xc`` [T, C] (contiguous), ``dt`` [T, C] (a projection), B and C: columns ``b_col`` / ``c_col`` .. of ``q``
     (N each); ``state`` [slots, C, N] fp32 is read at the segment's start (zero where seg_ctx is 0) and
-    written back at its end.  Returns out [T, C] in the activation dtype."""
+    written back at its end.  ``longest``: rows of the longest segment (0: not known); ``mode``
+    (device only): 0 whole segments or spans of tokens side by side, by the sizes, 1 whole, 2 spans.  Returns out [T, C] in the activation dtype."""
     T, C = xc.shape
     N = a_log.shape[1]
     if not xc.is_cuda:
@@ -988,7 +989,7 @@ def selective_scan(xc: torch.Tensor, q: torch.Tensor, b_col: int, c_col: int, dt
         return out
     out = torch.empty(T, C, dtype=xc.dtype, device=xc.device)
     native().selective_scan(out, xc, q, int(b_col), int(c_col), dt, dt_bias, a_log, d_skip, proj, int(z_col), state, seg_cu,
-                            seg_ctx, seg_slot)
+                            seg_ctx, seg_slot, int(longest), int(mode))
     return out
 
 

@@ -164,3 +164,22 @@ def test_chunked_channel_decays(H, Gk, dk, dv, kind):
     got = hops.decay_scan(qkv.cuda(), *a, z.cuda(), zb.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), H, Gk, dk, dv, dk ** -0.5, mode=3, **dev)
     for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
         torch.testing.assert_close(x, y, rtol=2e-5, atol=2e-5 * float(y.abs().max()))
+
+
+@pytest.mark.parametrize("C,N,long", [(40, 3, 700), (70, 16, 513), (33, 20, 300), (129, 64, 260), (20, 7, 384), (17, 130, 257), (1030, 66, 3700)])
+def test_selective_scan_in_spans(C, N, long):
+    """The selective recurrence with long segments cut into spans: segments around the spans' lengths (128; in the last case 256),
+    continued ones, a padding one, a long one, odd channel and state counts, steps from near zero to such that forget at once.
+    The CPU form rounds every product of decays as well: fp32 noise of a recurrence of hundreds of tokens, 2e-5 of the scale."""
+    g = _g(67)
+    lens = [1, 127, 128, 129, long, 7, 256, 255, 257]
+    cu, ctx, slot = _segments(lens, [0, 5, 0, 64, 9, 3, 0, 1, 2], [0, 1, 2, 3, 4, -1, 5, 6, 7])
+    T = sum(lens)
+    xc, q, dt, pr = _r(g, T, C), _r(g, T, 2 * N + 3), _r(g, T, C, s=3.0), _r(g, T, C + 5)
+    db, al, D, state = _r(g, C) - 2.0, _r(g, C, N), _r(g, C), _r(g, 8, C, N)
+    want_s, got_s = state.clone(), state.cuda()
+    want = hops.selective_scan(xc, q, 3, 3 + N, dt, db, al, D, pr, 5, want_s, cu, ctx, slot)
+    dev = [v.cuda() for v in (xc, q, dt, db, al, D, pr, cu, ctx, slot)]
+    got = hops.selective_scan(dev[0], dev[1], 3, 3 + N, *dev[2:7], 5, got_s, *dev[7:], longest=max(lens), mode=2)
+    for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
+        torch.testing.assert_close(x, y, rtol=2e-5, atol=2e-5 * float(y.abs().max()))
