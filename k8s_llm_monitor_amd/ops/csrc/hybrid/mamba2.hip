@@ -256,12 +256,32 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(float* __restrict__ y, co
   }
 }
 
-// Long segments (prompts): the same recurrence with the state spread thinner - 8 states per lane,
-// CH = N / 8 lanes per value of p (reduced by xor-shuffles over neighbouring lanes), 64 / CH values
-// of p per wave.  Per token a lane then issues a quarter of the instructions of the mapping above
-// (at N = 128) and four times as many waves share the work, which is what bounds a prompt's scan:
-// the token loop is sequential per (sequence, head, p).  State rows are read and written with a
-// stride here, which is why single-token segments (decode) keep the mapping above.
+// Long segments (prompts): the same recurrence with the state spread thinner - 8 states per lane, CH = N / 8 lanes per value of p
+// (their partial sums meet in DPP adds over neighbouring lanes), 64 / CH values of p per wave.  The token loop is sequential per
+// (sequence, head, p), so a prompt's scan takes what a token costs a wave: three VALU instructions per state, the DPP adds and
+// the LDS reads of B and C.  Everything else is kept out of that loop: a tile of 16 tokens is fetched into registers (16 bytes a load where `vec` says so) while the one
+// before it runs, step sizes and decays are computed for 256 tokens at a time, one per thread, and a tile's read-outs meet in LDS
+// (lane k of a group keeps token k's) and leave as rows.  State rows are read and written with a stride here, which is why
+// single-token segments (decode) keep the mapping above.
+// 4 prompts of 2048 tokens, 64 heads of 64 x 128 bf16: 850 us when every tile waited for its loads and computed its own step
+// sizes and every token stored its own read-outs, 625 now, the vector unit busy throughout; the mapping below takes the shapes
+// that it can (464).  The products and sums are spelled out: both mappings give the same bits.
+template <typename T>
+struct Raw8 {  // eight values as they lie in memory
+  uint4 q[sizeof(T) / 2];
+  __device__ __forceinline__ void from(const T* p) {  // 16-byte aligned
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 2); ++i) q[i] = reinterpret_cast<const uint4*>(p)[i];
+  }
+  __device__ __forceinline__ void from(const T* p, int n, int last) {  // p[n .. n + 7], past `last` that one
+    T v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = p[min(n + k, last)];
+    __builtin_memcpy(q, v, sizeof(v));
+  }
+  __device__ __forceinline__ void to(float* f) const { load8(reinterpret_cast<const T*>(q), f); }
+};
+
 template <typename T, int CH>
 __global__ __launch_bounds__(256) void ssm_scan_wide_kernel(float* __restrict__ y, const T* __restrict__ xbc,
                                                             const T* __restrict__ proj, long p_stride, int dt_col,
@@ -271,111 +291,337 @@ __global__ __launch_bounds__(256) void ssm_scan_wide_kernel(float* __restrict__ 
                                                             const float* __restrict__ decay,
                                                             float* __restrict__ state, const int* __restrict__ cu,
                                                             const int* __restrict__ ctx, const int* __restrict__ slot,
-                                                            int nh, int P, int N, int G) {
-  constexpr int TB = 16, PW = 64 / CH, PB = 4 * PW;
+                                                            int nh, int P, int N, int G, int vec) {
+  constexpr int TB = 16, PW = 64 / CH, PB = 4 * PW, LB = 256;
   constexpr int ROW = 8 * CH + (CH / 8) * 4 + 4;  // state n sits at n + 4 (n / 64): 64-float halves 4 banks apart
+  constexpr int GR = CH < TB ? CH : TB;           // tokens whose read-outs the lanes of a group keep
+  constexpr int NB = (TB * CH + 255) / 256, NX = (TB * PB + 255) / 256;
   __shared__ __attribute__((aligned(16))) float Bs[TB][ROW];
   __shared__ __attribute__((aligned(16))) float Cs[TB][ROW];
-  __shared__ float xs[TB][PB];
-  __shared__ float dts[TB], dAs[TB];
+  __shared__ __attribute__((aligned(16))) float dx[TB][PB];
+  __shared__ __attribute__((aligned(16))) float ys[TB][PB + 1];  // padded: neighbouring lanes write neighbouring rows
+  __shared__ float dts[LB], dAs[LB];
   const int s = blockIdx.x, h = blockIdx.y;
   const int sl = slot[s];
   const int t0 = cu[s], t1 = cu[s + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int chunk = lane % CH, pl = wave * PW + lane / CH;
-  const int p = blockIdx.z * PB + pl;
-  const bool live = p < P;
+  const int p0 = blockIdx.z * PB;
   const int inner = nh * P, C = inner + 2 * G * N;
   if (sl < 0) {  // padding rows: defined output, no state
-    if (live && chunk == 0)
-      for (int t = t0; t < t1; ++t) y[(long)t * inner + (long)h * P + p] = 0.f;
+    for (int i = threadIdx.x; i < (t1 - t0) * PB; i += 256)
+      if (p0 + i % PB < P) y[(long)(t0 + i / PB) * inner + (long)h * P + p0 + i % PB] = 0.f;
     return;
   }
   if (t1 <= t0) return;
   const int n0 = chunk * 8;
   const int g = h / (nh / G);
-  for (int i = threadIdx.x; i < TB * ROW; i += 256) {  // entries beyond N stay zero
-    (&Bs[0][0])[i] = 0.f;
-    (&Cs[0][0])[i] = 0.f;
-  }
   float S[8];
-  float* sp = state + (((long)sl * nh + h) * N) * P + p;
+  float* sp = state + (((long)sl * nh + h) * N) * P + p0 + pl;
   const bool carried = ctx[s] > 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) S[i] = (carried && live && n0 + i < N) ? sp[(long)(n0 + i) * P] : 0.f;
+  for (int i = 0; i < 8; ++i) S[i] = (carried && p0 + pl < P && n0 + i < N) ? sp[(long)(n0 + i) * P] : 0.f;
   const bool fixed = decay != nullptr;  // fixed decay per head: dt = 1, no skip term
   const float A = fixed ? 0.f : expf(a_log[h]), Dh = fixed ? 0.f : d_skip[h], bias = fixed ? 0.f : dt_bias[h];
   const float dfix = fixed ? decay[h] : 0.f;
   const int boff = n0 + (n0 >> 6) * 4;
-  // a thread stages the same elements of every tile: their token, LDS offset and offset from the
-  // tile's first row are computed once (the division by N is ~40 instructions)
-  constexpr int NB = (TB * 8 * CH + 255) / 256;
-  int st_tt[NB], st_lds[NB], st_glb[NB];
+  Raw8<T> rb[NB], rc[NB];
+  T rx[NX];
+  auto fetch = [&](int tb) {  // tokens past the segment read its last row, states past N the last ones
 #pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    const int i = threadIdx.x + 256 * u;
-    const int tt = i / N, n = i - tt * N;
-    st_tt[u] = tt;  // >= TB: beyond the tile
-    st_lds[u] = tt * ROW + n + (n >> 6) * 4;
-    st_glb[u] = tt * C + inner + g * N + n;
-  }
-  const int cgap = G * N;
-  float* yp = y + (long)t0 * inner + (long)h * P + p;  // this lane's output column, advanced per tile
-  for (int tb = t0; tb < t1; tb += TB) {
-    const int nt = min(TB, t1 - tb);
-    __syncthreads();  // the previous tile is consumed (and the zero fill is done)
-    const T* tile = xbc + (long)tb * C;
-#pragma unroll
-    for (int u = 0; u < NB; ++u)  // unrolled: the independent loads go out together
-      if (st_tt[u] < nt) {
-        (&Bs[0][0])[st_lds[u]] = ldf(tile + st_glb[u]);
-        (&Cs[0][0])[st_lds[u]] = ldf(tile + st_glb[u] + cgap);
-      }
-    for (int i = threadIdx.x; i < nt * PB; i += 256) {
-      const int tt = i / PB, pp = i % PB;
-      const int pg = blockIdx.z * PB + pp;
-      xs[tt][pp] = pg < P ? ldf(xbc + (long)(tb + tt) * C + (long)h * P + pg) : 0.f;
-    }
-    if (threadIdx.x < nt) {
-      if (fixed) {
-        dts[threadIdx.x] = 1.f;
-        dAs[threadIdx.x] = dfix;
+    for (int u = 0; u < NB; ++u) {
+      const int i = threadIdx.x + 256 * u, n = i % CH * 8;
+      const T* row = xbc + (long)min(tb + min(i / CH, TB - 1), t1 - 1) * C + inner + g * N;
+      if (vec) {
+        rb[u].from(row + min(n, N - 8));
+        rc[u].from(row + G * N + min(n, N - 8));
       } else {
-        const float raw = ldf(proj + (long)(tb + threadIdx.x) * p_stride + dt_col + h) + bias;
-        const float dt = raw > 20.f ? raw : log1pf(expf(raw));
-        dts[threadIdx.x] = dt;
-        dAs[threadIdx.x] = expf(-A * dt);
+        rb[u].from(row, n, N - 1);
+        rc[u].from(row + G * N, n, N - 1);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int i = threadIdx.x + 256 * u;
+      rx[u] = xbc[(long)min(tb + min(i / PB, TB - 1), t1 - 1) * C + (long)h * P + min(p0 + i % PB, P - 1)];
+    }
+  };
+  struct Token {
+    float b[8], c[8], d, dA;
+  };
+  auto stage = [&](Token& k, int tt, int lb) {  // one staged token into registers
+    load8(&Bs[tt][boff], k.b);
+    load8(&Cs[tt][boff], k.c);
+    k.dA = dAs[lb + tt];
+    k.d = dx[tt][pl];
+  };
+  auto token = [&](const Token& k) -> float {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) S[i] = fmaf(S[i], k.dA, k.d * k.b[i]);
+    float a = fmaf(S[0], k.c[0], S[1] * k.c[1]);
+#pragma unroll
+    for (int i = 2; i < 8; ++i) a = fmaf(S[i], k.c[i], a);
+    return group_sum<CH>(a);
+  };
+  fetch(t0);
+  for (int tb = t0; tb < t1; tb += TB) {
+    const int nt = min(TB, t1 - tb), lb = (tb - t0) % LB;
+    if (lb == 0) {  // the step sizes and decays of the next 256 tokens (all have left the loop over the last ones)
+      const int t = min(tb + (int)threadIdx.x, t1 - 1);
+      float dt = 1.f, dA = dfix;
+      if (!fixed) {
+        const float raw = ldf(proj + (long)t * p_stride + dt_col + h) + bias;
+        dt = raw > 20.f ? raw : log1pf(expf(raw));
+        dA = expf(-A * dt);
+      }
+      dts[threadIdx.x] = dt;
+      dAs[threadIdx.x] = dA;
+      __syncthreads();
+    }
+    float ex[NX];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int i = threadIdx.x + 256 * u, tt = i / CH, n = i % CH * 8;
+      if (NB * 256 == TB * CH || i < TB * CH) {
+        float fb[8], fc[8];
+        rb[u].to(fb);
+        rc[u].to(fc);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {  // states beyond N stay zero
+          fb[k] = n + k < N ? fb[k] : 0.f;
+          fc[k] = n + k < N ? fc[k] : 0.f;
+        }
+        store8(&Bs[tt][n + (n >> 6) * 4], fb);
+        store8(&Cs[tt][n + (n >> 6) * 4], fc);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int i = threadIdx.x + 256 * u, tt = min(i / PB, TB - 1);
+      ex[u] = ldf(&rx[u]);
+      if (NX * 256 == TB * PB || i < TB * PB) dx[tt][i % PB] = dts[lb + tt] * ex[u];
+    }
+    __syncthreads();
+    if (tb + TB < t1) fetch(tb + TB);
+    if (nt == TB) {
+      Token k[2];  // the next one is read while one is processed
+      stage(k[0], 0, lb);
+#pragma unroll
+      for (int t4 = 0; t4 < TB; t4 += GR) {
+        float keep = 0.f;
+#pragma unroll
+        for (int j = 0; j < GR; ++j) {
+          if (t4 + j + 1 < TB) stage(k[(t4 + j + 1) & 1], t4 + j + 1, lb);
+          __builtin_amdgcn_sched_barrier(0);  // (the reads would be moved down to their uses)
+          const float acc = token(k[(t4 + j) & 1]);
+          keep = chunk == j ? acc : keep;
+        }
+        if (CH <= TB || chunk < TB) ys[t4 + chunk][pl] = keep;
+      }
+    } else {
+      for (int tt = 0; tt < nt; ++tt) {
+        Token k;
+        stage(k, tt, lb);
+        const float acc = token(k);
+        if (chunk == 0) ys[tt][pl] = acc;
+      }
+    }
+    __syncthreads();  // the tile's inputs are consumed and its read-outs complete
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int i = threadIdx.x + 256 * u, tt = i / PB, p = p0 + i % PB;
+      if (tt < nt && p < P) y[(long)(tb + tt) * inner + (long)h * P + p] = fmaf(Dh, ex[u], ys[tt][i % PB]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (p0 + pl < P && n0 + i < N) sp[(long)(n0 + i) * P] = S[i];
+}
+
+// The same with the products dt x (x) B taken off the vector unit, which the mapping above keeps busy all the time, and the sums the
+// same bit for bit: a wave holds 64 states of 16 values of p, and v_mfma_f32_16x16x1 (four blocks, no sum: each of its results is
+// one rounded product) writes the products of a token.  Row r of block k is the wave's state 16 (r / 4) + 4 k + r % 4, so that
+// quarter q of the wave holds states 16 q .. 16 q + 15, each eight of which in neighbouring registers, and the sums over eight meet
+// in the order of the mapping above: inside a lane, between the quarters, then between the NW = N / 64 waves that share a p, whose
+// read-outs meet in LDS.  Per token a lane is left with two instructions per state; the products of a token are formed while the
+// one before runs, its B and dt x read one token earlier still.  Rows past the segment's end are staged as zeros with decay 1,
+// which leave the state as it is.  A wave alone on a SIMD issues every eighth cycle here, two of them every fifth, hence no more
+// than 64 states to a wave: with 128 of them four prompts of 2048 tokens (64 heads of 64 x 128) took 585 us, so 464; one prompt
+// 294 (758 before either mapping was reworked).
+template <typename T, int NW>
+__global__ __launch_bounds__(256, 2) void ssm_scan_tile_kernel(float* __restrict__ y, const T* __restrict__ xbc,
+                                                               const T* __restrict__ proj, long p_stride, int dt_col,
+                                                               const float* __restrict__ dt_bias,
+                                                               const float* __restrict__ a_log,
+                                                               const float* __restrict__ d_skip,
+                                                               const float* __restrict__ decay,
+                                                               float* __restrict__ state, const int* __restrict__ cu,
+                                                               const int* __restrict__ ctx, const int* __restrict__ slot,
+                                                               int nh, int P, int N, int G) {
+  typedef float floatx16 __attribute__((ext_vector_type(16)));
+  constexpr int TB = NW < 4 ? 32 : 16, PB = 64 / NW, LB = 256, NS = 64 * NW, CR = NS / 8, XR = PB / 4;
+  constexpr int ROW = NS / 16 * 20;  // state n sits at n + 4 (n / 16): the quarters' reads 20 banks apart
+  constexpr int NB = TB * CR / 256, NX = (TB * XR + 255) / 256;
+  __shared__ __attribute__((aligned(16))) float Bs[TB][ROW];
+  __shared__ __attribute__((aligned(16))) float Cs[TB][ROW];
+  __shared__ __attribute__((aligned(16))) float dx[TB][PB];
+  __shared__ __attribute__((aligned(16))) float ys[NW][TB][PB + 16];
+  __shared__ float dts[LB], dAs[LB];
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int sl = slot[s];
+  const int t0 = cu[s], t1 = cu[s + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, wn = wave % NW;
+  const int pl = wave / NW * 16 + (lane & 15), p0 = blockIdx.z * PB, p = p0 + pl;
+  const int inner = nh * P, C = inner + 2 * G * N;
+  const int xp = threadIdx.x % XR * 4, xt0 = threadIdx.x / XR;  // staging, finishing: values xp .. xp + 3 of tokens xt0 + 256 / XR u
+  if (sl < 0) {  // padding rows: defined output, no state
+    if (p0 + xp < P)
+      for (int t = t0 + xt0; t < t1; t += 256 / XR)
+        *reinterpret_cast<float4*>(y + (long)t * inner + (long)h * P + p0 + xp) = make_float4(0.f, 0.f, 0.f, 0.f);
+    return;
+  }
+  if (t1 <= t0) return;
+  const int g = h / (nh / G);
+  float S[16];
+  float* sp = state + (((long)sl * nh + h) * N) * P + p;
+  const bool carried = ctx[s] > 0 && p < P;
+  const int n0 = 64 * wn + 16 * q;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) S[i] = carried && n0 + i < N ? sp[(long)(n0 + i) * P] : 0.f;
+  const bool fixed = decay != nullptr;  // fixed decay per head: dt = 1, no skip term
+  const float A = fixed ? 0.f : expf(a_log[h]), Dh = fixed ? 0.f : d_skip[h], bias = fixed ? 0.f : dt_bias[h];
+  const float dfix = fixed ? decay[h] : 0.f;
+  const int coff = 80 * wn + 20 * q;                                          // this quarter's states
+  const int aoff = 80 * wn + 20 * ((lane & 15) >> 2) + 4 * q + (lane & 3);    // this lane's row of the product
+  Raw8<T> rb[NB], rc[NB];
+  T rx[NX][4];
+  auto fetch = [&](int tb) {
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int i = threadIdx.x + 256 * u, n = min(i % CR * 8, N - 8);
+      const T* row = xbc + (long)min(tb + i / CR, t1 - 1) * C + inner + g * N + n;
+      rb[u].from(row);
+      rc[u].from(row + G * N);
+    }
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const T* row = xbc + (long)min(tb + xt0 + 256 / XR * u, t1 - 1) * C + (long)h * P + min(p0 + xp, P - 4);
+      __builtin_memcpy(rx[u], __builtin_assume_aligned(row, 4 * sizeof(T)), 4 * sizeof(T));
+    }
+  };
+  struct Ab {
+    float a, d, dA;
+  };
+  auto read_ab = [&](Ab& k, int tt, int lb) {
+    k.a = Bs[tt][aoff];
+    k.d = dx[tt][pl];
+    k.dA = dAs[lb + tt];
+  };
+  auto read_c = [&](float (&c)[16], int tt) {
+    load8(&Cs[tt][coff], &c[0]);
+    load8(&Cs[tt][coff + 8], &c[8]);
+  };
+  auto products = [&](const Ab& k) {
+    const floatx16 zero = {};
+    return __builtin_amdgcn_mfma_f32_16x16x1f32(k.a, k.d, zero, 0, 0, 0);
+  };
+  fetch(t0);
+  for (int tb = t0; tb < t1; tb += TB) {
+    const int nt = min(TB, t1 - tb), lb = (tb - t0) % LB;
+    if (lb == 0) {  // the step sizes and decays of the next 256 tokens (all have left the loop over the last ones)
+      const int t = tb + (int)threadIdx.x;
+      float dt = 1.f, dA = dfix;
+      if (!fixed) {
+        const float raw = ldf(proj + (long)min(t, t1 - 1) * p_stride + dt_col + h) + bias;
+        dt = raw > 20.f ? raw : log1pf(expf(raw));
+        dA = expf(-A * dt);
+      }
+      dts[threadIdx.x] = dt;
+      dAs[threadIdx.x] = t < t1 ? dA : 1.f;
+      __syncthreads();
+    }
+    float ex[NX][4];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int i = threadIdx.x + 256 * u, tt = i / CR, n = i % CR * 8;
+      float fb[8], fc[8];
+      rb[u].to(fb);
+      rc[u].to(fc);
+      const bool in = n < N && tt < nt;  // (N is a multiple of 8)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        fb[k] = in ? fb[k] : 0.f;
+        fc[k] = in ? fc[k] : 0.f;
+      }
+      store8(&Bs[tt][n + 4 * (n / 16)], fb);
+      store8(&Cs[tt][n + 4 * (n / 16)], fc);
+    }
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int xt = xt0 + 256 / XR * u;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) ex[u][v] = ldf(&rx[u][v]);
+      if (256 / XR * NX == TB || xt < TB) {
+        const float dt = dts[lb + xt];
+        *reinterpret_cast<float4*>(&dx[xt][xp]) = xt < nt ? make_float4(dt * ex[u][0], dt * ex[u][1], dt * ex[u][2], dt * ex[u][3])
+                                                          : make_float4(0.f, 0.f, 0.f, 0.f);
       }
     }
     __syncthreads();
-#pragma unroll 2
-    for (int tt = 0; tt < nt; ++tt) {
-      const float dA = dAs[tt], x = xs[tt][pl];
-      const float dtx = dts[tt] * x;
-      const float4 b0 = *reinterpret_cast<const float4*>(&Bs[tt][boff]);
-      const float4 b1 = *reinterpret_cast<const float4*>(&Bs[tt][boff + 4]);
-      const float4 c0 = *reinterpret_cast<const float4*>(&Cs[tt][boff]);
-      const float4 c1 = *reinterpret_cast<const float4*>(&Cs[tt][boff + 4]);
-      S[0] = dA * S[0] + dtx * b0.x;
-      S[1] = dA * S[1] + dtx * b0.y;
-      S[2] = dA * S[2] + dtx * b0.z;
-      S[3] = dA * S[3] + dtx * b0.w;
-      S[4] = dA * S[4] + dtx * b1.x;
-      S[5] = dA * S[5] + dtx * b1.y;
-      S[6] = dA * S[6] + dtx * b1.z;
-      S[7] = dA * S[7] + dtx * b1.w;
-      float acc = S[0] * c0.x + S[1] * c0.y + S[2] * c0.z + S[3] * c0.w + S[4] * c1.x + S[5] * c1.y + S[6] * c1.z +
-                  S[7] * c1.w;
-      acc = group_sum<CH>(acc);
-      if (live && chunk == 0) yp[(long)tt * inner] = acc + Dh * x;
-    }
-    yp += (long)TB * inner;
-  }
-  if (live) {
+    if (tb + TB < t1) fetch(tb + TB);
+    Ab ab[2];
+    float c[2][16];
+    floatx16 t[2];
+    read_ab(ab[0], 0, lb);
+    read_ab(ab[1], 1, lb);
+    read_c(c[0], 0);
+    t[0] = products(ab[0]);
+    float dA[2] = {ab[0].dA, 0.f}, r[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (n0 + i < N) sp[(long)(n0 + i) * P] = S[i];
+    for (int tt = 0; tt < TB; ++tt) {
+      if (tt + 1 < TB) {
+        read_c(c[(tt + 1) & 1], tt + 1);
+        t[(tt + 1) & 1] = products(ab[(tt + 1) & 1]);
+        dA[(tt + 1) & 1] = ab[(tt + 1) & 1].dA;
+      }
+      if (tt + 2 < TB) read_ab(ab[tt & 1], tt + 2, lb);
+      __builtin_amdgcn_sched_barrier(0);  // (the reads would be moved down to their uses)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S[i] = fmaf(S[i], dA[tt & 1], t[tt & 1][i]);
+      float a[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const float* cv = &c[tt & 1][8 * m];
+        a[m] = fmaf(S[8 * m], cv[0], S[8 * m + 1] * cv[1]);
+#pragma unroll
+        for (int i = 2; i < 8; ++i) a[m] = fmaf(S[8 * m + i], cv[i], a[m]);
+      }
+      r[tt & 3] = a[0] + a[1];
+      if ((tt & 3) == 3) {  // four tokens' sums over the quarters in three exchanges: quarter k ends with token k's
+        const float r01 = swap16_sum(r[0], r[1]), r23 = swap16_sum(r[2], r[3]);
+        ys[wn][tt - 3 + q][pl] = swap32_sum(r01, r23);
+      }
+    }
+    __syncthreads();  // the tile's inputs are consumed and its read-outs complete
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int xt = xt0 + 256 / XR * u;
+      if (xt >= nt || p0 + xp >= P) continue;
+      float o[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        o[v] = ys[0][xt][xp + v];
+        if (NW == 2) o[v] += ys[NW - 1][xt][xp + v];
+        if (NW == 4) o[v] = (o[v] + ys[1 % NW][xt][xp + v]) + (ys[2 % NW][xt][xp + v] + ys[3 % NW][xt][xp + v]);
+        o[v] = fmaf(Dh, ex[u][v], o[v]);
+      }
+      *reinterpret_cast<float4*>(y + (long)(tb + xt) * inner + (long)h * P + p0 + xp) = make_float4(o[0], o[1], o[2], o[3]);
+    }
   }
+  if (p < P)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (n0 + i < N) sp[(long)(n0 + i) * P] = S[i];
 }
 
 }  // namespace k8sllm
@@ -387,10 +633,25 @@ static int launch_scan(float* y, const void* xbc, const void* proj, long p_strid
                        const float* a_log, const float* d_skip, const float* decay, float* state, const int* cu, const int* ctx,
                        const int* slot, int S, int nh, int P, int N, int G, int wide, hipStream_t s) {
   if (wide && N > 8) {  // long segments: 8 states per lane
+    const int vec = N % 8 == 0 && (nh * P) % 8 == 0 && reinterpret_cast<uintptr_t>(xbc) % 16 == 0;
+    // the tile form wants 16-byte rows of B and C and 4 values of p at a time; below 33 states half its products would be padding
+    if (N > 32 && vec && P % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
+#define K8SLLM_TILE(NW)                                                                                              \
+  hipLaunchKernelGGL((ssm_scan_tile_kernel<T, NW>),                                                                   \
+                     dim3((unsigned)S, (unsigned)nh, (unsigned)((P + 64 / NW - 1) / (64 / NW))), dim3(256), 0, s, y,   \
+                     (const T*)xbc, (const T*)proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot, nh, \
+                     P, N, G)
+      if (N <= 64) K8SLLM_TILE(1);
+      else if (N <= 128) K8SLLM_TILE(2);
+      else if (N <= 256) K8SLLM_TILE(4);
+      else return -1;
+#undef K8SLLM_TILE
+      return (int)hipGetLastError();
+    }
 #define K8SLLM_WIDE(CH)                                                                                              \
   hipLaunchKernelGGL((ssm_scan_wide_kernel<T, CH>), dim3((unsigned)S, (unsigned)nh, (unsigned)((P + 256 / CH - 1) / (256 / CH))), \
                      dim3(256), 0, s, y, (const T*)xbc, (const T*)proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, \
-                     cu, ctx, slot, nh, P, N, G)
+                     cu, ctx, slot, nh, P, N, G, vec)
     if (N <= 16) K8SLLM_WIDE(2);
     else if (N <= 32) K8SLLM_WIDE(4);
     else if (N <= 64) K8SLLM_WIDE(8);

@@ -183,3 +183,33 @@ def test_selective_scan_in_spans(C, N, long):
     got = hops.selective_scan(dev[0], dev[1], 3, 3 + N, *dev[2:7], 5, got_s, *dev[7:], longest=max(lens), mode=2)
     for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
         torch.testing.assert_close(x, y, rtol=2e-5, atol=2e-5 * float(y.abs().max()))
+
+
+@pytest.mark.parametrize("nh,P,N,G", [(4, 64, 128, 1), (3, 24, 40, 1), (2, 20, 64, 2), (2, 64, 256, 2), (2, 40, 136, 1), (8, 32, 72, 4)])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+@pytest.mark.parametrize("fixed", [False, True])
+def test_state_scan_products_on_the_matrix_cores(nh, P, N, G, dt, fixed):
+    """The long-segment scan with its products on the matrix cores gives the bits of the other long-segment mapping (which an
+    input that is not 16-byte aligned takes), and the oracle's values within fp32 noise: segments around the tile of 32 tokens
+    and the 256 tokens whose step sizes are computed at once, continued ones, a padding one."""
+    g = _g(68)
+    lens = [1, 31, 32, 33, 300, 7, 257, 64]
+    cu, ctx, slot = _segments(lens, [0, 5, 0, 64, 9, 3, 0, 1], [0, 1, 2, 3, 4, -1, 5, 6])
+    T, W = sum(lens), nh * P + 2 * G * N
+    xbc, proj, state = _r(g, T, W, dt=dt), _r(g, T, nh + 3, dt=dt), _r(g, 7, nh, N, P)
+    db, al, D = _r(g, nh) - 2.0, _r(g, nh, s=0.5), _r(g, nh)
+    decay = torch.sigmoid(_r(g, nh) + 3.0) if fixed else None
+    par = (None, 0, None, None, None) if fixed else (proj, 3, db, al, D)
+    want_s = state.clone()
+    want = hops.ssm_scan(xbc, *par, want_s, cu, ctx, slot, nh, P, N, G, decay=decay)
+    dev = [v.cuda() if isinstance(v, torch.Tensor) else v for v in par]
+    odd = torch.empty(T * W + 2, dtype=dt, device="cuda")[2:].view(T, W).copy_(xbc)
+    assert odd.data_ptr() % 16 != 0
+    res = []
+    for x in (xbc.cuda(), odd):
+        st = state.cuda()
+        y = hops.ssm_scan(x, *dev, st, cu.cuda(), ctx.cuda(), slot.cuda(), nh, P, N, G, mode=2, decay=None if decay is None else decay.cuda())
+        res.append((y.cpu(), st.cpu()))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    for a, b in zip(res[0], (want, want_s)):
+        torch.testing.assert_close(a, b.view_as(a), rtol=2e-5, atol=2e-5 * float(b.abs().max()))
