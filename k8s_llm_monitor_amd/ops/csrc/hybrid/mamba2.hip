@@ -61,67 +61,119 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(T* __restrict__ out, con
   stf(out + (long)row * C + c, silu_f(acc));
 }
 
-// The same with 8 channels per thread (16 / 32-byte accesses): channel count, column offset and
-// row strides multiples of 8.
 template <typename T>
+struct Raw8 {  // eight values as they lie in memory
+  uint4 q[sizeof(T) / 2];
+  __device__ __forceinline__ void from(const T* p) {  // 16-byte aligned
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 2); ++i) q[i] = reinterpret_cast<const uint4*>(p)[i];
+  }
+  __device__ __forceinline__ void from(const T* p, int n, int last) {  // p[n .. n + 7], past `last` that one
+    T v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = p[min(n + k, last)];
+    __builtin_memcpy(q, v, sizeof(v));
+  }
+  __device__ __forceinline__ void to(float* f) const { load8(reinterpret_cast<const T*>(q), f); }
+};
+
+// The same with 8 channels and R rows per thread (16 / 32-byte accesses): channel count, column offset and row strides multiples
+// of 8.  A row's weights are 128 bytes to its 16 of input at the usual 4 taps, so a thread that takes one row (R = 1: the few rows of
+// a decode step) mostly reads weights; R rows share them, and inside a segment each row's input is read once for its four taps,
+// all of them in flight together.  8000 rows of 4096 channels bf16: 89 -> 38 us, 3.5 TB/s.
+template <typename T, int R>
 __global__ __launch_bounds__(256) void conv_silu_vec8_kernel(T* __restrict__ out, const T* __restrict__ proj,
                                                              long stride, int col0, int C, const float* __restrict__ cw,
                                                              const float* __restrict__ cb, int taps,
                                                              const T* __restrict__ state, const int* __restrict__ cu,
                                                              const int* __restrict__ ctx, const int* __restrict__ slot,
-                                                             int S) {
-  const int row = blockIdx.x;
+                                                             int S, int rows) {
   const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
   if (c >= C) return;
-  const int s = find_segment(cu, S, row);
-  const int sl = slot[s];
-  float acc[8], x[8];
-  if (sl < 0) {  // padding row: defined output, no state
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-    store8(out + (long)row * C + c, acc);
-    return;
-  }
-  const int r = row - cu[s];
-  const bool carried = ctx[s] > 0;
-  if (cb != nullptr) {
-    load8(cb + c, acc);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-  }
-  if (taps == 4) {  // the usual width: a thread's 8 x 4 weights are 128 contiguous bytes, read as 16-byte loads
-    float4 wv[8];
+  const int row0 = blockIdx.x * R;
+  float4 wv[8];
+  if (taps == 4) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) wv[k] = *reinterpret_cast<const float4*>(cw + (long)(c + k) * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = r - 3 + j;
-      if (i >= 0)
-        load8(proj + (long)(row - 3 + j) * stride + col0 + c, x);
-      else if (carried)
-        load8(state + ((long)sl * 3 + (3 + i)) * C + c, x);
-      else
-        continue;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) acc[k] += (j == 0 ? wv[k].x : j == 1 ? wv[k].y : j == 2 ? wv[k].z : wv[k].w) * x[k];
-    }
-  } else {
-    for (int j = 0; j < taps; ++j) {
-      const int i = r - (taps - 1) + j;
-      if (i >= 0)
-        load8(proj + (long)(row - (taps - 1) + j) * stride + col0 + c, x);
-      else if (carried)
-        load8(state + ((long)sl * (taps - 1) + (taps - 1 + i)) * C + c, x);
-      else
-        continue;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) acc[k] += cw[(long)(c + k) * taps + j] * x[k];
-    }
   }
+  float bias[8];
+  if (cb != nullptr) {
+    load8(cb + c, bias);
+  } else {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = silu_f(acc[k]);
-  store8(out + (long)row * C + c, acc);
+    for (int i = 0; i < 8; ++i) bias[i] = 0.f;
+  }
+  int s = find_segment(cu, S, row0);
+  if (R > 1 && taps == 4 && row0 + R <= cu[s + 1] && row0 - 3 >= cu[s] && slot[s] >= 0) {  // all inputs lie in one segment
+    Raw8<T> in[R + 3];
+    const T* px = proj + (long)(row0 - 3) * stride + col0 + c;
+#pragma unroll
+    for (int i = 0; i < R + 3; ++i) in[i].from(px + i * stride);
+    float x[4][8];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) in[i].to(x[i]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      in[r + 3].to(x[(r + 3) & 3]);
+      float acc[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        float v = bias[k];
+        v += wv[k].x * x[r & 3][k];
+        v += wv[k].y * x[(r + 1) & 3][k];
+        v += wv[k].z * x[(r + 2) & 3][k];
+        v += wv[k].w * x[(r + 3) & 3][k];
+        acc[k] = silu_f(v);
+      }
+      store8(out + (long)(row0 + r) * C + c, acc);
+    }
+    return;
+  }
+  for (int row = row0; row < min(row0 + R, rows); ++row) {
+    if (R > 1)
+      while (s < S - 1 && row >= cu[s + 1]) ++s;
+    const int sl = slot[s];
+    float acc[8], x[8];
+    if (sl < 0) {  // padding row: defined output, no state
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+      store8(out + (long)row * C + c, acc);
+      continue;
+    }
+    const int r = row - cu[s];
+    const bool carried = ctx[s] > 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = bias[i];
+    if (taps == 4) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = r - 3 + j;
+        if (i >= 0)
+          load8(proj + (long)(row - 3 + j) * stride + col0 + c, x);
+        else if (carried)
+          load8(state + ((long)sl * 3 + (3 + i)) * C + c, x);
+        else
+          continue;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] += (j == 0 ? wv[k].x : j == 1 ? wv[k].y : j == 2 ? wv[k].z : wv[k].w) * x[k];
+      }
+    } else {
+      for (int j = 0; j < taps; ++j) {
+        const int i = r - (taps - 1) + j;
+        if (i >= 0)
+          load8(proj + (long)(row - (taps - 1) + j) * stride + col0 + c, x);
+        else if (carried)
+          load8(state + ((long)sl * (taps - 1) + (taps - 1 + i)) * C + c, x);
+        else
+          continue;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] += cw[(long)(c + k) * taps + j] * x[k];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[k] = silu_f(acc[k]);
+    store8(out + (long)row * C + c, acc);
+  }
 }
 
 template <typename T>
@@ -266,22 +318,6 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(float* __restrict__ y, co
 // 4 prompts of 2048 tokens, 64 heads of 64 x 128 bf16: 850 us when every tile waited for its loads and computed its own step
 // sizes and every token stored its own read-outs, 625 now, the vector unit busy throughout; the mapping below takes the shapes
 // that it can (464).  The products and sums are spelled out: both mappings give the same bits.
-template <typename T>
-struct Raw8 {  // eight values as they lie in memory
-  uint4 q[sizeof(T) / 2];
-  __device__ __forceinline__ void from(const T* p) {  // 16-byte aligned
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(T) / 2); ++i) q[i] = reinterpret_cast<const uint4*>(p)[i];
-  }
-  __device__ __forceinline__ void from(const T* p, int n, int last) {  // p[n .. n + 7], past `last` that one
-    T v[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = p[min(n + k, last)];
-    __builtin_memcpy(q, v, sizeof(v));
-  }
-  __device__ __forceinline__ void to(float* f) const { load8(reinterpret_cast<const T*>(q), f); }
-};
-
 template <typename T, int CH>
 __global__ __launch_bounds__(256) void ssm_scan_wide_kernel(float* __restrict__ y, const T* __restrict__ xbc,
                                                             const T* __restrict__ proj, long p_stride, int dt_col,
@@ -675,6 +711,30 @@ static int launch_scan(float* y, const void* xbc, const void* proj, long p_strid
   return (int)hipGetLastError();
 }
 
+template <typename T>
+static int launch_conv(void* out, const void* proj, long stride, int col0, int C, const float* cw, const float* cb, int taps,
+                       void* state, const int* cu, const int* ctx, const int* slot, int S, long rows, hipStream_t s) {
+  const int gy = (C + 255) / 256, gy8 = (C / 8 + 255) / 256;
+  if (C % 8 == 0 && col0 % 8 == 0 && stride % 8 == 0) {
+#define K8SLLM_CONV(R)                                                                                                 \
+  hipLaunchKernelGGL((conv_silu_vec8_kernel<T, R>), dim3((unsigned)((rows + R - 1) / R), (unsigned)gy8), dim3(256), 0, s, (T*)out, \
+                     (const T*)proj, stride, col0, C, cw, cb, taps, (const T*)state, cu, ctx, slot, S, (int)rows)
+    // four rows a thread from 512 rows on (773 of 4096 channels: 15.9 us one row a thread, 12.9 four), below them it lacks threads
+    // (256: 9.6 / 10.6); eight or sixteen rows are no faster at 8000 and slower where segments start (13 prompts of 300: 43 us with
+    // one row, 25 with four, 28 with eight)
+    if (taps == 4 && rows >= 512) K8SLLM_CONV(4);
+    else K8SLLM_CONV(1);
+#undef K8SLLM_CONV
+  } else {
+    hipLaunchKernelGGL(conv_silu_kernel<T>, dim3((unsigned)rows, (unsigned)gy), dim3(256), 0, s, (T*)out, (const T*)proj, stride, col0,
+                       C, cw, cb, taps, (const T*)state, cu, ctx, slot, S);
+  }
+  if (taps > 1)
+    hipLaunchKernelGGL(conv_state_step_kernel<T>, dim3((unsigned)S, (unsigned)gy), dim3(256), 0, s, (T*)state, (const T*)proj, stride,
+                       col0, C, taps, cu, ctx, slot);
+  return (int)hipGetLastError();
+}
+
 extern "C" {
 
 int k8sllm_hy_conv_silu(void* out, const void* proj, long stride, int col0, int C, const float* cw, const float* cb,
@@ -682,31 +742,8 @@ int k8sllm_hy_conv_silu(void* out, const void* proj, long stride, int col0, int 
                         hipStream_t s) {
   if (T <= 0 || S <= 0) return 0;
   if (taps < 1 || taps > kMaxTaps) return -1;
-  const dim3 g1((unsigned)T, (unsigned)((C + 255) / 256)), g2((unsigned)S, (unsigned)((C + 255) / 256));
-  const bool v8 = C % 8 == 0 && col0 % 8 == 0 && stride % 8 == 0;
-  const dim3 g8((unsigned)T, (unsigned)((C / 8 + 255) / 256));
-  if (f32) {
-    if (v8)
-      hipLaunchKernelGGL(conv_silu_vec8_kernel<float>, g8, dim3(256), 0, s, (float*)out, (const float*)proj, stride, col0,
-                         C, cw, cb, taps, (const float*)state, cu, ctx, slot, S);
-    else
-      hipLaunchKernelGGL(conv_silu_kernel<float>, g1, dim3(256), 0, s, (float*)out, (const float*)proj, stride, col0, C,
-                         cw, cb, taps, (const float*)state, cu, ctx, slot, S);
-    if (taps > 1)
-      hipLaunchKernelGGL(conv_state_step_kernel<float>, g2, dim3(256), 0, s, (float*)state, (const float*)proj, stride,
-                         col0, C, taps, cu, ctx, slot);
-  } else {
-    if (v8)
-      hipLaunchKernelGGL(conv_silu_vec8_kernel<bf16_t>, g8, dim3(256), 0, s, (bf16_t*)out, (const bf16_t*)proj, stride,
-                         col0, C, cw, cb, taps, (const bf16_t*)state, cu, ctx, slot, S);
-    else
-      hipLaunchKernelGGL(conv_silu_kernel<bf16_t>, g1, dim3(256), 0, s, (bf16_t*)out, (const bf16_t*)proj, stride, col0,
-                         C, cw, cb, taps, (const bf16_t*)state, cu, ctx, slot, S);
-    if (taps > 1)
-      hipLaunchKernelGGL(conv_state_step_kernel<bf16_t>, g2, dim3(256), 0, s, (bf16_t*)state, (const bf16_t*)proj,
-                         stride, col0, C, taps, cu, ctx, slot);
-  }
-  return (int)hipGetLastError();
+  return f32 ? launch_conv<float>(out, proj, stride, col0, C, cw, cb, taps, state, cu, ctx, slot, S, T, s)
+             : launch_conv<bf16_t>(out, proj, stride, col0, C, cw, cb, taps, state, cu, ctx, slot, S, T, s);
 }
 
 int k8sllm_hy_ssm_scan(float* y, const void* xbc, const void* proj, long p_stride, int dt_col, const float* dt_bias,

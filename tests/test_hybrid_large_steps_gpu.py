@@ -213,3 +213,24 @@ def test_state_scan_products_on_the_matrix_cores(nh, P, N, G, dt, fixed):
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
     for a, b in zip(res[0], (want, want_s)):
         torch.testing.assert_close(a, b.view_as(a), rtol=2e-5, atol=2e-5 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("C,col0,pad", [(2056, 8, 16), (64, 0, 0)])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_conv_rows_of_large_steps(C, col0, pad, dt):
+    """The convolution of a step whose threads take four rows each: segments that start anywhere in a group of four, of one row and of
+    many, continued ones and a padding one, gives the bits of the same segments in steps too small for it."""
+    g = _g(69)
+    lens = [1, 2, 3, 4, 5, 130, 7, 200, 1, 1, 203]
+    ctxs, slots = [0, 5, 0, 64, 9, 3, 0, 1, 0, 8, 2], [0, 1, 2, 3, 4, -1, 5, 6, 7, 8, 9]
+    T = sum(lens)
+    assert T >= 512
+    proj, cw, cb, state = _r(g, T, col0 + C + pad, dt=dt).cuda(), _r(g, C, 4).cuda(), _r(g, C).cuda(), _r(g, 10, 3, C, dt=dt)
+    sa, sb = state.cuda(), state.cuda()
+    got = hops.conv_silu(proj, col0, C, cw, cb, sa, *(v.cuda() for v in _segments(lens, ctxs, slots)))
+    r = 0
+    for n, c, sl in zip(lens, ctxs, slots):
+        want = hops.conv_silu(proj[r:r + n], col0, C, cw, cb, sb, *(v.cuda() for v in _segments([n], [c], [sl])))
+        assert torch.equal(got[r:r + n], want)
+        r += n
+    assert torch.equal(sa, sb)
