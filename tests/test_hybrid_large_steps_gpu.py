@@ -234,3 +234,29 @@ def test_conv_rows_of_large_steps(C, col0, pad, dt):
         assert torch.equal(got[r:r + n], want)
         r += n
     assert torch.equal(sa, sb)
+
+
+@pytest.mark.parametrize("rows,N,Kd", [(1, 64, 32), (63, 65, 64), (64, 128, 1024), (300, 200, 96), (65, 1, 160)])
+@pytest.mark.parametrize("act", [0, 1, 2, 3, 4])
+def test_fp32_grouped_gemm(rows, N, Kd, act):
+    """Grouped fp32 products on the matrix cores: rows and columns around the 64 x 64 tile, an expert without rows, every activation,
+    gathered and plain rows.  fp32 sums of Kd products of unit variance: 1e-6 sqrt(Kd) before the activation, which at most
+    doubles it times the other factor."""
+    g = _g(70)
+    E, gated = 4, act in (1, 3)
+    off = [0, rows // 3, rows // 3, rows - rows // 4, rows]
+    a, w = _r(g, rows, Kd), _r(g, E, N * (2 if gated else 1), Kd)
+    idx = torch.randperm(rows, generator=g).int()
+    ext = hops.native()
+    for sorted_idx in (None, idx):
+        y = torch.empty(rows, N, device="cuda")
+        ext.grouped_gemm(y, a.cuda(), w.cuda(), _i32(off).cuda(), None if sorted_idx is None else sorted_idx.cuda(), 1, act, False, True,
+                         7.0 if act == 3 else 0.0)
+        x = (a if sorted_idx is None else a[sorted_idx.long()]).double()
+        z = torch.cat([x[off[e]:off[e + 1]] @ w[e].double().t() for e in range(E)])
+        u, z = (z[:, N:], z[:, :N]) if gated else (z, z)
+        lim = 7.0
+        want = {0: lambda: z, 1: lambda: z * torch.sigmoid(z) * u, 2: lambda: torch.nn.functional.gelu(z), 4: lambda: z.clamp(min=0) ** 2,
+                3: lambda: z.clamp(max=lim) * torch.sigmoid(1.702 * z.clamp(max=lim)) * (u.clamp(-lim, lim) + 1)}[act]()
+        tol = 1e-6 * Kd ** 0.5 * 4 * (1 + z.abs().max() + u.abs().max())
+        assert float((y.cpu().double() - want).abs().max()) <= float(tol)
