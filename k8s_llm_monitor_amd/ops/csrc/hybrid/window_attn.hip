@@ -537,6 +537,10 @@ int k8sllm_hy_window_flash(void* out, const void* qkv, long q_stride, const void
                            const int* ctx, const int* block_tables, int bt_stride, int S, long T, int Hq, int G, int dk, int dv,
                            float scale, int window, int chunked, int keep, float cap, int plain_cap, int sink,
                            const float* sinks, const void* gate, long g_stride, hipStream_t s);
+int k8sllm_hy_window_f32(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache, const int* cu,
+                         const int* ctx, const int* block_tables, int bt_stride, int S, long T, int Hq, int G, int dk, int dv,
+                         int bs, float scale, int window, int chunked, int keep, float cap, int sink, const float* sinks,
+                         const void* gate, long g_stride, int decode, hipStream_t s);
 
 int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float* kw, float eps, long T, int nq,
                             int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s) {
@@ -593,6 +597,11 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
 #undef K8SLLM_WPC
     return (int)hipGetLastError();
   }
+  if (f32 && mfma) {  // head sizes of 64 and 128: window_f32.hip, faster at every size measured there
+    const int rc = k8sllm_hy_window_f32(out, qkv, q_stride, k_cache, v_cache, cu, ctx, block_tables, bt_stride, S, T, Hq, G, dk, dv,
+                                        bs, scale, window, chunked, keep, cap, sink, sinks, gate, g_stride, 0, s);
+    if (rc != 1) return rc;
+  }
   if (f32)
     hipLaunchKernelGGL(window_prefill_kernel<float>, dim3(T, Hq), dim3(64), 0, s, (float*)out, (const float*)qkv,
                        q_stride, (const float*)k_cache, (const float*)v_cache, cu, ctx, block_tables, bt_stride, S, Hq,
@@ -625,6 +634,11 @@ int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const voi
     else K8SLLM_WD(8);
 #undef K8SLLM_WD
     return (int)hipGetLastError();
+  }
+  if (f32 && vec) {
+    const int rc = k8sllm_hy_window_f32(out, qkv, q_stride, k_cache, v_cache, nullptr, seq_lens, block_tables, bt_stride, B, B, Hq, G,
+                                        dk, dv, bs, scale, window, chunked, keep, cap, sink, sinks, gate, g_stride, 1, s);
+    if (rc != 1) return rc;
   }
   if (f32)
     hipLaunchKernelGGL(window_decode_kernel<float>, dim3(B, Hq), dim3(64), 0, s, (float*)out, (const float*)qkv,

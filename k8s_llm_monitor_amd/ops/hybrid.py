@@ -526,7 +526,8 @@ def window_attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: 
     unscaled logit).  Scores and weights are fp32.  Returns [T, Hq*dv].  GPU, bf16, head sizes
     64 / 128: the matrix-core kernels - tiles staged in LDS for large steps and long contexts, else 16
     query rows per wave (``mfma`` 0: the any-size wave-per-row kernel; 2: the register kernel; 16 / 32 / 64: with
-    that many rows per wave; 256: the staged kernel)."""
+    that many rows per wave; 256: the staged kernel); fp32, the same sizes: 16 rows per wave on the fp32
+    matrix instruction."""
     T = qkv.shape[0]
     if not qkv.is_cuda:
         out = torch.empty(T, Hq * dv, dtype=qkv.dtype)

@@ -260,3 +260,32 @@ def test_fp32_grouped_gemm(rows, N, Kd, act):
                 3: lambda: z.clamp(max=lim) * torch.sigmoid(1.702 * z.clamp(max=lim)) * (u.clamp(-lim, lim) + 1)}[act]()
         tol = 1e-6 * Kd ** 0.5 * 4 * (1 + z.abs().max() + u.abs().max())
         assert float((y.cpu().double() - want).abs().max()) <= float(tol)
+
+
+@pytest.mark.parametrize("dk,dv,Hq,G", [(128, 128, 8, 2), (64, 128, 3, 1), (128, 64, 2, 2), (64, 64, 16, 2)])
+@pytest.mark.parametrize("kw", [dict(window=0, sink=False), dict(window=5, sink=True), dict(window=40, sink=False, keep=3),
+                                dict(window=33, sink=True, keep=20, cap=2.0), dict(window=32, sink=False, chunked=True)])
+def test_fp32_window_attention(dk, dv, Hq, G, kw):
+    """fp32 windowed attention on the matrix cores: chunks around the 16-row tile with and without a past, kept tokens before, inside
+    and past the window, caps, sinks, gates, a padding row; the pages' unused ends hold NaN.  fp32 softmax sums: 2e-5."""
+    g = _g(71)
+    kw = dict(kw)
+    new, ctx = [1, 15, 16, 17, 50, 3], [0, 37, 0, 130, 16, 250]
+    lens = [a + b for a, b in zip(ctx, new)]
+    W = max((n + 15) // 16 for n in lens)
+    bt = torch.randperm(len(lens) * W, generator=g).int().view(-1, W)
+    kc, vc = _r(g, bt.numel(), 16, G * dk), _r(g, bt.numel(), G, dv, 16)
+    for row, n in zip(bt, lens):
+        for j in range(n, W * 16):
+            vc[row[j // 16].item(), :, :, j % 16] = float("nan")
+            kc[row[j // 16].item(), j % 16] = float("nan")
+    cu = _i32([0] + torch.tensor(new).cumsum(0).tolist())
+    qkv, gate = _r(g, sum(new), Hq * dk + G * (dk + dv)), _r(g, sum(new), Hq)
+    a = (Hq, G, dk, dv, dk ** -0.5, kw.pop("window"), kw.pop("sink"))
+    want = hops.window_attention_prefill(qkv, kc, vc, cu, _i32(ctx), bt, *a, gate=gate, **kw)
+    got = hops.window_attention_prefill(qkv.cuda(), kc.cuda(), vc.cuda(), cu.cuda(), _i32(ctx).cuda(), bt.cuda(), *a, gate=gate.cuda(), **kw)
+    torch.testing.assert_close(got.cpu(), want, rtol=2e-5, atol=2e-5)
+    q1, bt1, sl = qkv[:7], torch.cat([bt, bt[:1]]), _i32(lens + [0])
+    want = hops.window_attention_decode(q1, kc, vc, bt1, sl, *a, gate=gate[:7], **kw)
+    got = hops.window_attention_decode(q1.cuda(), kc.cuda(), vc.cuda(), bt1.cuda(), sl.cuda(), *a, gate=gate[:7].cuda(), **kw)
+    torch.testing.assert_close(got.cpu(), want, rtol=2e-5, atol=2e-5)
