@@ -545,15 +545,18 @@ __global__ __launch_bounds__(256, 2) void hy_grouped_gemm_f32_kernel(float* __re
   }
 }
 
-// bf16 on the matrix cores (K a multiple of 32): one wave = 16 sorted rows x 16 NT output columns
-// (NT = 4; NT = 1 with a deeper unroll when there are few rows, so that a decode step's weight
-// stream is spread over four times as many waves),
-// v_mfma_f32_16x16x32_bf16 with both operands loaded straight from global memory as 16-byte
-// fragments (A = the gathered activation rows, B = weight rows, 8 consecutive k per lane).  Few
-// rows per expert (decode) make this a weight-streaming kernel: many small workgroups, no LDS.
+// bf16 on the matrix cores (K a multiple of 32): one wave = 16 MT sorted rows of one expert x 16 NT output columns,
+// v_mfma_f32_16x16x32_bf16 with both operands loaded straight from global memory as 16-byte fragments (A = the gathered
+// activation rows, B = weight rows, 8 consecutive k per lane), batches of them in flight while the last is multiplied.  Few rows
+// per expert (decode) make this a weight-streaming kernel: many small workgroups, no LDS, NT = 1 so that the stream is spread over
+// as many waves as there are columns, and MT so that the rows of an expert share one pass over its weights (a second row
+// tile lands on another XCD and reads them again).  With more rows NT = 4, MT = 1.  Every output is one chain of products in the
+// order of k, whatever the tile.
+// 128 rows over 8 experts, K = N = 2048, gated / plain: 54.5 / 34.3 us with 16 rows a wave and a wait per batch, 36.1 / 20.3 now
+// (3.7 and 3.3 TB/s of weights); widths 4096 x 3584: 194 / 101 and 110 / 68.
 // ``il``: the gate / up rows are interleaved per 128 rows as [64 gate | 64 up] (the prefill tile
 // GEMM's pairing), else [all gate rows ; all up rows].
-template <int ACT, int NT>
+template <int ACT, int NT, int MT>
 __global__ __launch_bounds__(64) void hy_grouped_gemm_mfma_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ A,
                                                                   const bf16_t* __restrict__ W,
                                                                   const int* __restrict__ offsets,
@@ -564,18 +567,21 @@ __global__ __launch_bounds__(64) void hy_grouped_gemm_mfma_kernel(bf16_t* __rest
   for (; e < E; ++e) {
     r0 = offsets[e];
     r1 = offsets[e + 1];
-    const int nt = (r1 - r0 + 15) >> 4;
+    const int nt = (r1 - r0 + 16 * MT - 1) / (16 * MT);
     if (tile < nt) break;
     tile -= nt;
   }
   if (e >= E) return;
-  r0 += tile * 16;
+  r0 += tile * (16 * MT);
   const int lane = threadIdx.x, c16 = lane & 15, quad = lane >> 4;
   const int n0 = blockIdx.y * (16 * NT);
   const bf16_t* We = W + (long)e * w_es;
-  const int arow = min(r0 + c16, r1 - 1);
-  const long asrc = sorted_idx != nullptr ? sorted_idx[arow] / div : arow;
-  const bf16_t* ap = A + asrc * Kd + 8 * quad;
+  const bf16_t* ap[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int arow = min(r0 + 16 * m + c16, r1 - 1);
+    ap[m] = A + (long)(sorted_idx != nullptr ? sorted_idx[arow] / div : arow) * Kd + 8 * quad;
+  }
   const bf16_t* wg[NT];
   const bf16_t* wu[NT];
 #pragma unroll
@@ -585,35 +591,70 @@ __global__ __launch_bounds__(64) void hy_grouped_gemm_mfma_kernel(bf16_t* __rest
     wg[t] = We + g * Kd + 8 * quad;
     wu[t] = We + (SWIGLU ? (il ? g + 64 : (long)N + n) : 0) * Kd + 8 * quad;
   }
-  f32x4 acc[NT], accu[NT];
+  f32x4 acc[MT][NT], accu[MT][NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = accu[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll(NT == 1 ? 8 : 2)
-  for (int k0 = 0; k0 < Kd; k0 += 32) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(ap + k0);
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[m][t] = accu[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](const bf16x8 (&a)[MT], const bf16x8 (&w)[NT], const bf16x8 (&u)[NT]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], w[t], acc[m][t], 0, 0, 0);
+        if (SWIGLU) accu[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], u[t], accu[m][t], 0, 0, 0);
+      }
+  };
+  auto load = [&](bf16x8 (&a)[MT], bf16x8 (&w)[NT], bf16x8 (&u)[NT], int k0) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const bf16x8*>(ap[m] + k0);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, *reinterpret_cast<const bf16x8*>(wg[t] + k0), acc[t], 0, 0, 0);
-      if (SWIGLU)
-        accu[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, *reinterpret_cast<const bf16x8*>(wu[t] + k0), accu[t], 0, 0, 0);
+      w[t] = *reinterpret_cast<const bf16x8*>(wg[t] + k0);
+      if (SWIGLU) u[t] = *reinterpret_cast<const bf16x8*>(wu[t] + k0);
+    }
+  };
+  // batches of U steps of 32 k: the next one is fetched while one is multiplied
+  constexpr int U = NT > 1 ? 2 : SWIGLU || MT > 2 ? 4 : 8;
+  bf16x8 a[2][U][MT], w[2][U][NT], u[2][U][NT];
+  const int nb = Kd / (32 * U);
+  if (nb > 0)
+#pragma unroll
+    for (int i = 0; i < U; ++i) load(a[0][i], w[0][i], u[0][i], 32 * i);
+  for (int k = 0; k < nb; k += 2) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (k + h >= nb) break;
+      if (k + h + 1 < nb)
+#pragma unroll
+        for (int i = 0; i < U; ++i) load(a[h ^ 1][i], w[h ^ 1][i], u[h ^ 1][i], 32 * ((k + h + 1) * U + i));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < U; ++i) step(a[h][i], w[h][i], u[h][i]);
     }
   }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {  // acc[t][i]: row r0 + 4 quad + i, column n0 + 16 t + c16
-    const int n = n0 + 16 * t + c16;
-    if (n >= N) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = r0 + 4 * quad + i;
-      if (r >= r1) continue;
-      float v = acc[t][i];
-      if (ACT == 3) v = clamped_unit_f(bf2f(f2bf(v)), bf2f(f2bf(accu[t][i])), limit);
-      else if (SWIGLU) v = silu_f(bf2f(f2bf(v))) * bf2f(f2bf(accu[t][i]));
-      else if (ACT == 2) v = gelu_erf_f(bf2f(f2bf(v)));
-      else if (ACT == 4) v = relu_sq_f(bf2f(f2bf(v)));
-      Y[(long)r * N + n] = f2bf(v);
-    }
+  for (int k0 = nb * 32 * U; k0 < Kd; k0 += 32) {
+    load(a[0][0], w[0][0], u[0][0], k0);
+    step(a[0][0], w[0][0], u[0][0]);
   }
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {  // acc[m][t][i]: row r0 + 16 m + 4 quad + i, column n0 + 16 t + c16
+      const int n = n0 + 16 * t + c16;
+      if (n >= N) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = r0 + 16 * m + 4 * quad + i;
+        if (r >= r1) continue;
+        float v = acc[m][t][i];
+        if (ACT == 3) v = clamped_unit_f(bf2f(f2bf(v)), bf2f(f2bf(accu[m][t][i])), limit);
+        else if (SWIGLU) v = silu_f(bf2f(f2bf(v))) * bf2f(f2bf(accu[m][t][i]));
+        else if (ACT == 2) v = gelu_erf_f(bf2f(f2bf(v)));
+        else if (ACT == 4) v = relu_sq_f(bf2f(f2bf(v)));
+        Y[(long)r * N + n] = f2bf(v);
+      }
+    }
 }
 
 template <typename T, bool V8>
@@ -717,21 +758,25 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
   if (il && (!swiglu || N % 64)) return -1;
   if (!f32 && mfma && Kd % 32 == 0) {
     const bool few = rows <= 512;  // a decode-sized step: one n-tile per wave
-    const dim3 g16((unsigned)(rows / 16 + E), (unsigned)(few ? (N + 15) / 16 : (N + 63) / 64));
-#define K8SLLM_GM(SW, NT)                                                                                        \
-  hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<SW, NT>), g16, dim3(64), 0, s, (bf16_t*)Y, (const bf16_t*)A,      \
+    // a wave takes 16, 32 or 64 rows of an expert, so that its weights are mostly read once: by the mean number of rows an expert
+    // gets (K = N = 2048, 8 experts, gated + plain: mean 6 55 / 53 us with 16 / 32 rows, 16 81 / 56, 32 113 / 105 and 64 rows 80;
+    // 64 experts, mean 8: 175 / 178)
+    const int mt = !few || rows <= 8l * E ? 1 : rows <= 24l * E ? 2 : 4;
+    const dim3 g16((unsigned)(rows / (16 * mt) + E), (unsigned)(few ? (N + 15) / 16 : (N + 63) / 64));
+#define K8SLLM_GM(SW, NT, MT)                                                                                        \
+  hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<SW, NT, MT>), g16, dim3(64), 0, s, (bf16_t*)Y, (const bf16_t*)A,      \
                      (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)
-    if (swiglu) {
-      if (few) K8SLLM_GM(1, 1); else K8SLLM_GM(1, 4);
-    } else if (act == 3) {
-      if (few) K8SLLM_GM(3, 1); else K8SLLM_GM(3, 4);
-    } else if (act == 2) {
-      if (few) K8SLLM_GM(2, 1); else K8SLLM_GM(2, 4);
-    } else if (act == 4) {
-      if (few) K8SLLM_GM(4, 1); else K8SLLM_GM(4, 4);
-    } else {
-      if (few) K8SLLM_GM(0, 1); else K8SLLM_GM(0, 4);
-    }
+#define K8SLLM_GMS(SW)                  \
+  if (!few) K8SLLM_GM(SW, 4, 1);        \
+  else if (mt == 1) K8SLLM_GM(SW, 1, 1); \
+  else if (mt == 2) K8SLLM_GM(SW, 1, 2); \
+  else K8SLLM_GM(SW, 1, 4)
+    if (swiglu) { K8SLLM_GMS(1); }
+    else if (act == 3) { K8SLLM_GMS(3); }
+    else if (act == 2) { K8SLLM_GMS(2); }
+    else if (act == 4) { K8SLLM_GMS(4); }
+    else { K8SLLM_GMS(0); }
+#undef K8SLLM_GMS
 #undef K8SLLM_GM
     return (int)hipGetLastError();
   }

@@ -289,3 +289,28 @@ def test_fp32_window_attention(dk, dv, Hq, G, kw):
     want = hops.window_attention_decode(q1, kc, vc, bt1, sl, *a, gate=gate[:7], **kw)
     got = hops.window_attention_decode(q1.cuda(), kc.cuda(), vc.cuda(), bt1.cuda(), sl.cuda(), *a, gate=gate[:7].cuda(), **kw)
     torch.testing.assert_close(got.cpu(), want, rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("rows", [17, 40, 90])  # a mean of 8.5, 20, 45 rows an expert: 32, 32 and 64 rows a wave
+@pytest.mark.parametrize("N,Kd", [(40, 32), (64, 288), (16, 1024)])
+@pytest.mark.parametrize("act", [0, 1, 3])
+def test_grouped_gemm_rows_per_wave(rows, N, Kd, act):
+    """The bf16 weight-streaming products give the same bits however many rows of an expert a wave takes (experts without rows lower
+    the mean that decides it), at K of less than one batch of loads, of a batch and a rest, and of several batches; and the
+    oracle's values within the rounding of the bf16 result."""
+    g = _g(72)
+    gated = act in (1, 3)
+    a, w = _r(g, rows, Kd, dt=BF), _r(g, 2, N * (2 if gated else 1), Kd, s=Kd ** -0.5, dt=BF)
+    off = [0, rows // 3, rows]
+    ext, res = hops.native(), []
+    for E in (2, rows):
+        y = torch.empty(rows, N, dtype=BF, device="cuda")
+        wide = torch.cat([w, torch.zeros(E - 2, *w.shape[1:], dtype=BF)])
+        ext.grouped_gemm(y, a.cuda(), wide.cuda(), _i32(off + [rows] * (E - 2)).cuda(), None, 1, act, False, True, 7.0 if act == 3 else 0.0)
+        res.append(y.cpu())
+    assert torch.equal(res[0], res[1])
+    z = torch.cat([a[off[e]:off[e + 1]].float() @ w[e].float().t() for e in range(2)]).to(BF).float()
+    u, z = (z[:, N:], z[:, :N]) if gated else (z, z)
+    want = {0: lambda: z, 1: lambda: z * torch.sigmoid(z) * u,
+            3: lambda: z.clamp(max=7) * torch.sigmoid(1.702 * z.clamp(max=7)) * (u.clamp(-7, 7) + 1)}[act]()
+    torch.testing.assert_close(res[0].float(), want, rtol=2e-2, atol=2e-2)
