@@ -56,7 +56,9 @@ State: an attention run owns paged K ``[blocks, 16, heads*dim]`` and V ``[blocks
 Mamba-2 run owns per-sequence slots - the fp32 state ``[slots, heads, N, P]`` and the last
 taps-1 convolution inputs.  Every RUN (a looped layer counts once per pass) has its own.
 
-Dense projections go to the BLAS library (``F.linear``); everything else is ops.hybrid.
+Dense projections go to ops.hybrid.linear (the BLAS library, its own kernel for a few rows) or, in the layers of the
+window-and-Mamba-2 decoder, straight to the library (``F.linear``): its routers pick other experts with the last bit of
+their input, so those layers' sums stay what they are; everything else is ops.hybrid.
 """
 from __future__ import annotations
 
@@ -297,7 +299,7 @@ class LatentAttention:
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
         H, dn, dr, dv, Q, R = self.H, self.dn, self.dr, self.dv, self.Q, self.R
         T = h.shape[0]
-        proj = down = F.linear(h, self.w_down)
+        proj = down = hops.linear(h, self.w_down)
         if self.n_tail:
             self.tail_out = (proj, self.n_in)
         if proj.shape[1] > self.n_down:
@@ -307,7 +309,7 @@ class LatentAttention:
         own = self.kv_from is None
         hops.latent_prep(down, Q, R, dr, self.qn, self.kn, self.eps, meta.positions, self.freq,
                          kc if own else None, vc if own else None, meta.slot_mapping if own else None, pairs=self.pairs)
-        q = F.linear(down[:, :Q], self.w_uq)
+        q = hops.linear(down[:, :Q], self.w_uq)
         ex = self._expand_ok(h, meta)
         nd = meta.num_decode if meta.is_prefill else T  # single-token rows in front
         parts = []
@@ -316,7 +318,7 @@ class LatentAttention:
             parts.append(self._forward_latent(q[:n], meta, kc, vc, gate[:n] if gate is not None else None, not ex))
         if ex:
             parts.append(self._forward_expanded(q[nd:], down[nd:], meta, kc, gate[nd:] if gate is not None else None))
-        return F.linear(parts[0] if len(parts) == 1 else torch.cat(parts), self.wo)
+        return hops.linear(parts[0] if len(parts) == 1 else torch.cat(parts), self.wo)
 
     def _forward_latent(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
                         chunks: bool) -> torch.Tensor:
@@ -452,7 +454,7 @@ class RotaryAttention:
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
         H, G, dk, dv = self.H, self.G, self.dk, self.dv
         if proj is None:
-            proj = F.linear(h, self.w_in)
+            proj = hops.linear(h, self.w_in)
         if self.n_tail:
             self.tail_out = (proj, self.n_in)
         kc, vc = cache["k"], cache["v"]
@@ -474,7 +476,7 @@ class RotaryAttention:
                 o = torch.cat([od, o])
         if self.has_gate and not hg:
             o = hops.sigmoid_gate(o, proj, self.g_col)
-        return F.linear(o, self.wo)
+        return hops.linear(o, self.wo)
 
     def export(self, p: str) -> dict:
         nq, nk = self.H * self.dk, self.G * self.dk
@@ -532,14 +534,14 @@ class LightningMixer:
         return 0, self.H * self.dk * self.dv * 4
 
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
-        proj = F.linear(h, self.w_in)
+        proj = hops.linear(h, self.w_in)
         if self.n_tail:
             self.tail_out = (proj, self.n_in)
         vkq = hops.activation_cols(proj, 0, self.n_act, "silu")
         o = hops.linear_attention(vkq, self.decay, cache["state"], meta.seg_cu, meta.seg_ctx, meta.seg_slot,
                                   self.H, self.dk, self.dv)
         g = hops.gated_group_norm(o, proj, self.n_act, self.norm_w, self.eps, 1, h.dtype, after=True)
-        return F.linear(g, self.wo)
+        return hops.linear(g, self.wo)
 
 
 def _low_rank(p: _Params, prefix: str, name1: str, name2: str, n_out: int, d: int, default: int) -> tuple:
@@ -612,18 +614,18 @@ class GatedDeltaMixer:
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
         H, Gk, dk, dv = self.H, self.Gk, self.dk, self.dv
         if proj is None:
-            proj = F.linear(h, self.w_in)
+            proj = hops.linear(h, self.w_in)
         seg = (meta.seg_cu, meta.seg_ctx, meta.seg_slot)
         qkv = hops.conv_silu(proj, 0, self.C, self.conv_w, None, cache["conv"], *seg)
-        z, z_col = (proj, self.a_col) if self.per_head else (F.linear(proj[:, self.a_col:self.a_col + self.ra], self.wa2), 0)
+        z, z_col = (proj, self.a_col) if self.per_head else (hops.linear(proj[:, self.a_col:self.a_col + self.ra], self.wa2), 0)
         o = hops.decay_scan(qkv, 0, Gk * dk, 2 * Gk * dk, z, self.dt_bias, cache["state"], *seg, H, Gk, dk, dv,
                             dk ** -0.5, a_log=self.a_log, beta=proj, beta_col=self.b_col, unit=True, z_col=z_col)
         if self.low_rank_gate:
-            gate = F.linear(proj[:, self.g_col:self.g_col + self.rg], self.wg2)
+            gate = hops.linear(proj[:, self.g_col:self.g_col + self.rg], self.wg2)
             g = hops.gated_group_norm(o, gate, 0, self.norm_all, self.eps, H, h.dtype, after=True)
         else:
             g = hops.gated_group_norm(o, proj, self.g_col, self.norm_all, self.eps, H, h.dtype, after=True, gate="silu")
-        return F.linear(g, self.wo)
+        return hops.linear(g, self.wo)
 
     def export(self, p: str) -> dict:
         n = self.Gk * self.dk
@@ -674,12 +676,12 @@ class GatedLinearMixer:
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
         H, dk, dv = self.H, self.dk, self.dv
         if proj is None:
-            proj = F.linear(h, self.w_in)
-        z = F.linear(proj[:, self.a_col:self.a_col + self.ra], self.wa2)
+            proj = hops.linear(h, self.w_in)
+        z = hops.linear(proj[:, self.a_col:self.a_col + self.ra], self.wa2)
         o = hops.decay_scan(proj, 0, H * dk, 2 * H * dk, z, self.a_bias, cache["state"], meta.seg_cu, meta.seg_ctx,
                             meta.seg_slot, H, H, dk, dv, dk ** -0.5, tau=self.tau)
         g = hops.gated_group_norm(o, proj, self.g_col, self.norm_all, self.eps, H, h.dtype, after=True, gate="silu")
-        return F.linear(g, self.wo)
+        return hops.linear(g, self.wo)
 
     def export(self, p: str) -> dict:
         n, w = self.H * self.dk, self.w_in
@@ -725,13 +727,13 @@ class Mamba1Mixer:
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
         C, N, r = self.inner, self.N, self.rank
         seg = (meta.seg_cu, meta.seg_ctx, meta.seg_slot)
-        proj = F.linear(h, self.w_in)
+        proj = hops.linear(h, self.w_in)
         x = hops.conv_silu(proj, 0, C, self.conv_w, self.conv_b, cache["conv"], *seg)
-        q = F.linear(x, self.w_x)
-        dt = F.linear(q[:, :r], self.w_dt)
+        q = hops.linear(x, self.w_x)
+        dt = hops.linear(q[:, :r], self.w_dt)
         y = hops.selective_scan(x, q, r, r + N, dt, self.dt_bias, self.a_log, self.d_skip, proj, C, cache["state"], *seg,
                                 meta.seg_max)
-        return F.linear(y, self.wo)
+        return hops.linear(y, self.wo)
 
     def export(self, p: str) -> dict:
         return {p + "in": self.w_in, p + "conv": self.conv_w, p + "conv.b": self.conv_b, p + "x": self.w_x, p + "dt": self.w_dt,
@@ -783,10 +785,10 @@ class WkvMixer:
         mix = hops.token_mix(h, self.mu, cache["prev"], *seg, dtype)
         rkvg = torch.empty(T, 4 * n, dtype=dtype, device=h.device)
         torch.bmm(mix[:, :4].transpose(0, 1), self.w_rkvg, out=rkvg.view(T, 4, n).transpose(0, 1))
-        z = F.linear(hops.activation(F.linear(mix[:, 4], self.w1), "tanh"), self.w2)
+        z = hops.linear(hops.activation(hops.linear(mix[:, 4], self.w1), "tanh"), self.w2)
         o = hops.decay_scan(rkvg, 0, n, 2 * n, z, self.w0, cache["state"], *seg, H, H, dk, dk, 1.0, decay="exp_exp", bonus=self.u)
         g = hops.gated_group_norm(o, rkvg, 3 * n, self.norm_w, self.eps, H, dtype, after=True, gate="silu")
-        return F.linear(g, self.wo)
+        return hops.linear(g, self.wo)
 
     def export(self, p: str) -> dict:
         out = {p + "mu." + k: self.mu[i] for i, k in enumerate("rkvgw")}
@@ -857,7 +859,7 @@ class SideBySide:
         return a[0] + b[0], a[1] + b[1]
 
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> tuple:
-        proj = F.linear(h, self.w_in)
+        proj = hops.linear(h, self.w_in)
         yl, yr = (x.forward(h, meta, cache[side], proj=proj[:, a:b])
                   for x, side, (a, b) in zip(self.subs, ("left", "right"), self.cols))
         if self.out_w is not None:
@@ -929,7 +931,7 @@ class DenseFFN:
         self.a_pos, self.a_neg = _softplus(a[0]), 0.5 + _softplus(a[1])
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(hops.activation(F.linear(h, self.w_up), "xielu", self.a_pos, self.a_neg), self.w_down)
+        return hops.linear(hops.activation(hops.linear(h, self.w_up), "xielu", self.a_pos, self.a_neg), self.w_down)
 
 
 class UngatedDenseFFN:
@@ -941,7 +943,7 @@ class UngatedDenseFFN:
         self.w_down = p.get(prefix + "down", (d, self.ff), 1.0 / math.sqrt(self.ff))
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(hops.activation(F.linear(h, self.w_up), self.act), self.w_down)
+        return hops.linear(hops.activation(hops.linear(h, self.w_up), self.act), self.w_down)
 
 
 class GatedDenseFFN:
@@ -962,10 +964,10 @@ class GatedDenseFFN:
         self.w_down = p.get(prefix + "down", (d, self.ff), 1.0 / math.sqrt(self.ff))
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        proj = F.linear(h, self.w_in)
+        proj = hops.linear(h, self.w_in)
         if self.n_tail:
             self.tail_out = (proj, 2 * self.ff)
-        return F.linear(hops.glu(proj, 0, self.ff, self.act), self.w_down)
+        return hops.linear(hops.glu(proj, 0, self.ff, self.act), self.w_down)
 
 
 class PlainRoutedFFN:
@@ -993,7 +995,7 @@ class PlainRoutedFFN:
         ids, wts, _ = hops.moe_router(h, self.wr, None, self.E, self.K, over_all=True)
         shared = None
         if self.fs:
-            shared = F.linear(hops.activation(F.linear(h, self.ws1), "gelu"), self.ws2)
+            shared = hops.linear(hops.activation(hops.linear(h, self.ws1), "gelu"), self.ws2)
         return hops.moe_experts(h, ids, wts, self.w1, self.w2, shared, None, act="gelu")
 
 
@@ -1061,7 +1063,7 @@ class CorrectedRoutedFFN:
                                            corr=self.corr, best2=False, renorm=False)
         shared = None
         if self.fs:
-            shared = F.linear(hops.activation(F.linear(h, self.ws1), "relu_sq"), self.ws2)
+            shared = hops.linear(hops.activation(hops.linear(h, self.ws1), "relu_sq"), self.ws2)
         return hops.moe_experts(h, ids, wts, self.w1, self.w2, shared, None, act="relu_sq", identity=self.ident)
 
 

@@ -90,6 +90,7 @@ int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* s
                          const int* slot, int S, int H, int dk, int dv, int nt, hipStream_t s);
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
                      const float* bias, int E, int K, int rows_w, int over_all, int f32, hipStream_t s);
+int k8sllm_hy_few_rows(void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, hipStream_t s);
 int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* offsets, const int* sorted_idx, int div,
                            int E, long rows, int N, int Kd, long w_es, int act, int il, int f32, int mfma, float limit,
                            hipStream_t s);
@@ -898,6 +899,19 @@ void moe_align(Tensor ids, int64_t E, Tensor offsets, Tensor sorted_idx, Tensor 
 // y [rows, N] = W[e] a over expert-sorted rows; sorted_idx given: a's row of sorted row r is sorted_idx[r] / div
 // act_code: 0 none, 1 SwiGLU (w = [gate rows ; up rows]), 2 erf GELU
 // 3 the clamped gated unit (w = [gate rows ; up rows], limit), 4 squared ReLU
+// y [M, N] = x [M, K] w [N, K]^T, bf16, few rows; see few_rows.hip
+void few_rows(Tensor y, Tensor x, Tensor w) {
+  TORCH_CHECK(act(x, "x") == 0, "few_rows: bf16");
+  same(w, 0, "w");
+  same(y, 0, "y");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && w.dim() == 2 && w.is_contiguous() && y.dim() == 2 && y.is_contiguous() &&
+                  y.size(0) == x.size(0) && y.size(1) == w.size(0) && x.size(1) == w.size(1),
+              "few_rows: layouts");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0, "few_rows: alignment");
+  check(k8sllm_hy_few_rows(y.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), (int)x.size(0), (int)w.size(0), (int)x.size(1), cur()),
+        "few_rows");
+}
+
 void grouped_gemm(Tensor y, Tensor a, Tensor w, Tensor offsets, OptT sorted_idx, int64_t div, int64_t act_code, bool il,
                   bool mfma, double limit) {
   TORCH_CHECK(act_code >= 0 && act_code <= 4 && (act_code != 3 || limit > 0), "grouped_gemm: activation code");
@@ -1143,6 +1157,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ssm_scan", &ssm_scan);
   m.def("moe_router", &moe_router);
   m.def("moe_align", &moe_align);
+  m.def("few_rows", &few_rows);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("moe_combine", &moe_combine);
   m.def("norm_shift", &norm_shift);

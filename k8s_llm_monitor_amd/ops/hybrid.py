@@ -1158,6 +1158,23 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
     return out
 
 
+FEW_ROWS, FEW_ROWS_K, FEW_ROWS_WEIGHTS = 16, 4096, 1 << 24
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``x`` [T, K] times ``w`` [N, K] transposed.  The BLAS library's product, but for the few rows of a small decode step in
+    bf16 on the device: up to FEW_ROWS rows against weights of up to 16 M elements, K up to 4096 (and a multiple of 32, rows
+    16-byte aligned), where a call takes what it takes to get enough loads in flight (few_rows.hip has both sides' times)."""
+    if (x.shape[0] <= FEW_ROWS and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+            and w.shape[1] % 32 == 0 and w.shape[1] <= FEW_ROWS_K and w.numel() <= FEW_ROWS_WEIGHTS and x.shape[0] > 0
+            and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        native().few_rows(y, x, w)
+        return y
+    return F.linear(x, w)
+
+
 def swiglu(gu: torch.Tensor) -> torch.Tensor:
     """silu(gu[:, :f]) * gu[:, f:] for [T, 2f] rows ([gate | up])."""
     f = gu.shape[1] // 2

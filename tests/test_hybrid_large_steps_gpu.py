@@ -314,3 +314,16 @@ def test_grouped_gemm_rows_per_wave(rows, N, Kd, act):
     want = {0: lambda: z, 1: lambda: z * torch.sigmoid(z) * u,
             3: lambda: z.clamp(max=7) * torch.sigmoid(1.702 * z.clamp(max=7)) * (u.clamp(-7, 7) + 1)}[act]()
     torch.testing.assert_close(res[0].float(), want, rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17])
+@pytest.mark.parametrize("N,K", [(16, 32), (1, 96), (200, 512), (72, 2080), (1024, 4096), (24, 4128)])
+def test_linear_of_few_rows(M, N, K):
+    """Projections of a few rows against 64 bits: fewer steps of 32 k than waves, a rest, whole batches, columns around the tile of
+    16, a slice of wider rows, and one row or 32 k past the kernel's limits.  fp32 sums, one bf16 rounding: 2^-8 of the value
+    and 1e-6 sqrt(K) of what cancels."""
+    g = _g(73)
+    x, w = _r(g, M, K + 24, dt=BF).cuda()[:, 16:16 + K], _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
+    got, want = hops.linear(x, w).double(), x.double() @ w.double().t()
+    assert got.shape == want.shape
+    assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 1e-6 * K ** 0.5).all())
