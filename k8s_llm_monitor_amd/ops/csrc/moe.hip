@@ -137,6 +137,49 @@ __device__ __forceinline__ int block_exscan(int v, int* wsum, int& total) {
   return pre + x - v;
 }
 
+// Up to 1024 items and 64 experts (a decode step's), an item per thread: ranks among a wave's items of the same expert come from
+// ballots, one lane per expert then sums the waves' counts.  Two barriers where the counters below take two per expert: 128
+// items of 8 experts 8.5 -> 2.3 us, 512 of 64 25.8 -> 5.4.
+__global__ __launch_bounds__(1024) void moe_align_small_kernel(const int* __restrict__ ids, int n, int E,
+                                                               int* __restrict__ offsets, int* __restrict__ sorted_idx,
+                                                               int* __restrict__ inv_idx) {
+  __shared__ int cnt[16][64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = (blockDim.x + 63) >> 6;
+  const int e = t < n ? ids[t] : -1;
+  int rank = 0, mine = 0;
+  for (int i = 0; i < E; ++i) {
+    const unsigned long long mask = __ballot(e == i);
+    if (e == i) rank = __popcll(mask & ((1ull << lane) - 1));
+    if (lane == i) mine = __popcll(mask);
+  }
+  cnt[wave][lane] = mine;
+  __syncthreads();
+  if (wave == 0) {
+    int tot = 0;
+    for (int w = 0; w < nw; ++w) tot += cnt[w][lane];
+    int x = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    int at = x - tot;  // lanes past E hold no items
+    if (lane < E) offsets[lane] = at;
+    if (lane == E - 1) offsets[E] = x;
+    for (int w = 0; w < nw; ++w) {
+      const int c = cnt[w][lane];
+      cnt[w][lane] = at;
+      at += c;
+    }
+  }
+  __syncthreads();
+  if (t < n) {
+    const int pos = cnt[wave][e] + rank;
+    sorted_idx[pos] = t;
+    inv_idx[t] = pos;
+  }
+}
+
 // NT threads x ME experts of per-thread counters fill the 64 KiB of LDS: 1024 x 16 (Mixtral),
 // 256 x 64, 64 x 256.
 template <int NT, int ME>
@@ -247,7 +290,10 @@ int k8sllm_moe_router(const void* x, const void* wr, long T, int d, int E, int K
 int k8sllm_moe_align(const int* topk_ids, long n, int E, int* expert_offsets, int* sorted_idx, int* inv_idx,
                      hipStream_t s) {
   if (E > kAlignMaxE) return -1;
-  if (E <= kMaxE)
+  if (n > 0 && n <= 1024 && E <= 64)
+    hipLaunchKernelGGL(moe_align_small_kernel, dim3(1), dim3((unsigned)((n + 63) / 64 * 64)), 0, s, topk_ids, (int)n, E, expert_offsets,
+                       sorted_idx, inv_idx);
+  else if (E <= kMaxE)
     hipLaunchKernelGGL((moe_align_kernel<kAT, kMaxE>), dim3(1), dim3(kAT), 0, s, topk_ids, n, E, expert_offsets,
                        sorted_idx, inv_idx);
   else if (E <= 64)

@@ -327,3 +327,36 @@ def test_linear_of_few_rows(M, N, K):
     got, want = hops.linear(x, w).double(), x.double() @ w.double().t()
     assert got.shape == want.shape
     assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 1e-6 * K ** 0.5).all())
+
+
+@pytest.mark.parametrize("T", [1, 5, 4099])  # one token a workgroup, two with a rest
+@pytest.mark.parametrize("E,K,shared", [(8, 2, 0), (7, 3, 1), (16, 4, 1), (70, 16, 0)])
+def test_router_ranks(T, E, K, shared):
+    """Routers: the K largest logits in order, the lower number first among equal ones (whole rows of ties), weights and the shared
+    expert's gate.  Logits are fp32 sums: 1e-5."""
+    g = _g(74)
+    d = 136
+    h, wr, bias = _r(g, T, d, dt=BF), _r(g, E + shared, d, s=d ** -0.5), _r(g, E)
+    h[::3] = 0  # the bias alone decides there
+    bias[1:4] = bias.max() + 1
+    got = hops.moe_router(h.cuda(), wr.cuda(), bias.cuda(), E, K)
+    want = torch.sort(bias, descending=True, stable=True).indices[:K]
+    assert want[:3].tolist() == [1, 2, 3][:min(K, 3)] and bool((got[0][::3].cpu() == want).all())
+    lg = h.float() @ wr[:E].t() + bias
+    chosen = lg.gather(1, got[0].cpu().long())
+    assert bool((chosen[:, :-1] >= chosen[:, 1:] - 1e-5).all()) and all(len(set(r)) == K for r in got[0].tolist())
+    torch.testing.assert_close(chosen, lg.sort(1, descending=True).values[:, :K], rtol=0, atol=1e-5)
+    torch.testing.assert_close(got[1].cpu(), chosen.softmax(1), rtol=1e-5, atol=1e-5)
+    if shared:
+        torch.testing.assert_close(got[2].cpu().view(-1), torch.sigmoid(h.float() @ wr[E]), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("n,E", [(1, 1), (63, 8), (128, 8), (1000, 64), (1024, 5), (1025, 8), (700, 65)])
+def test_expert_sort(n, E):
+    """The counting sort of (token, expert) pairs around the limits of its one-pass form: stable, every pair once."""
+    ids = torch.randint(0, E, (n, 1), generator=_g(75)).int()
+    off, srt, inv = (torch.full((k,), -1, dtype=torch.int32, device="cuda") for k in (E + 1, n, n))
+    hops.native().moe_align(ids.cuda(), E, off, srt, inv)
+    want = torch.sort(ids.view(-1), stable=True).indices
+    assert torch.equal(srt.cpu().long(), want) and torch.equal(inv.cpu().long(), torch.sort(want).indices)
+    assert off.tolist() == [0] + torch.bincount(ids.view(-1).long(), minlength=E).cumsum(0).tolist()
