@@ -87,7 +87,7 @@ int k8sllm_hy_decay_chunk(float* o, const void* qkv, long stride, int q_col, int
                           const int* cu, const int* ctx, const int* slot, int S, int H, int Gk, int dk, int dv, float q_scale,
                           void* ws, long T, hipStream_t s);
 int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* state, const int* cu, const int* ctx,
-                         const int* slot, int S, int H, int dk, int dv, int nt, hipStream_t s);
+                         const int* slot, int S, long T, int longest, int H, int dk, int dv, int nt, hipStream_t s);
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
                      const float* bias, int E, int K, int rows_w, int over_all, int f32, hipStream_t s);
 int k8sllm_hy_few_rows(void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, hipStream_t s);
@@ -450,7 +450,7 @@ void conv_silu(Tensor out, Tensor proj, int64_t col0, Tensor cw, OptT cb, Tensor
 // value-column tiles per workgroup, 0: its choice), or the scan where it does not apply
 void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, OptT a_log, OptT d_skip, OptT decay,
               Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t nh, int64_t P, int64_t N, int64_t G,
-              int64_t mode, int64_t nt) {
+              int64_t mode, int64_t nt, int64_t longest) {
   const int f = act(xbc, "xbc");
   f32c(y, "y");
   f32c(state, "ssm_state");
@@ -482,10 +482,11 @@ void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, Opt
   TORCH_CHECK(y.numel() == T * nh * P, "ssm: y [T, nh*P]");
   TORCH_CHECK(state.dim() == 4 && state.size(1) == nh && state.size(2) == N && state.size(3) == P, "ssm_state [slots, nh, N, P]");
   TORCH_CHECK(G >= 1 && nh % G == 0 && N <= 256, "ssm: groups / state size (<= 256)");
-  if (cp != nullptr && !f && G == nh && (mode == 3 || (mode == 0 && T >= 32 * ctx.numel())) &&
+  if (cp != nullptr && !f && G == nh && (mode == 3 || (mode == 0 && (T >= 32 * ctx.numel() || longest >= 256))) &&
       reinterpret_cast<uintptr_t>(xbc.data_ptr()) % 16 == 0) {
     const int rc = k8sllm_hy_chunk_scan(y.data_ptr<float>(), xbc.data_ptr(), cp, state.data_ptr<float>(), cu.data_ptr<int>(),
-                                        ctx.data_ptr<int>(), slot.data_ptr<int>(), (int)ctx.numel(), (int)nh, (int)N, (int)P, (int)nt, cur());
+                                        ctx.data_ptr<int>(), slot.data_ptr<int>(), (int)ctx.numel(), (long)T, (int)longest, (int)nh, (int)N, (int)P,
+                                        (int)nt, cur());
     if (rc != 1) return check(rc, "ssm_scan (chunked)");
   }
   if (mode == 3) mode = 0;
@@ -686,7 +687,7 @@ void rotary_norm_cache(Tensor qkv, int64_t Hq, int64_t G, int64_t dk, int64_t dv
 void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_col, Tensor z, Tensor z_bias, OptT a_log,
                 double tau, OptT beta, int64_t beta_col, Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t H,
                 int64_t Gk, int64_t dk, int64_t dv, double q_scale, bool unit, int64_t mode, int64_t z_col, int64_t dkind,
-                OptT bonus) {
+                OptT bonus, int64_t longest) {
   const int f = act(qkv, "qkv");
   same(z, f, "z");
   f32c(o, "o");
@@ -729,13 +730,15 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
     bstride = beta->stride(0);
   }
   const int S = (int)ctx.numel();
-  const bool prompts = T >= 32l * S;
+  // prompts, or a long one beside single tokens (us, token by token -> chunks, delta rule / 32 heads of
+  // 64 x 64: one of 2000 rows beside 60 575 -> 186, 399 -> 181; one of 256 beside 60 142 -> 139, 125 -> 107)
+  const bool prompts = T >= 32l * S || longest >= 256;
   const void* zp = (const char*)z.data_ptr() + z_col * z.element_size();
   if (!f && (mode == 3 || (mode == 0 && prompts)) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 &&
       qkv.stride(0) % 8 == 0 && q_col % 8 == 0 && k_col % 8 == 0 && v_col % 8 == 0) {
     // a chunk costs the same whatever it holds (us, 16 heads of 128 x 128, scan -> chunks: 40 segments of 33 rows 99 -> 101;
     // 16 of 64 73 -> 51; one of 64 21 -> 28; 4 of 2048 542 -> 209)
-    if (per_head && (mode == 3 || (T >= 64l * S && T >= 128))) {
+    if (per_head && (mode == 3 || longest >= 256 || (T >= 64l * S && T >= 128))) {
       const long nb = k8sllm_hy_delta_chunk_ws(T, S, (int)H, (int)dk, (int)dv);
       if (nb > 0) {
         Tensor ws = torch::empty({nb}, o.options().dtype(torch::kUInt8));
@@ -746,7 +749,7 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
                                            ws.data_ptr(), (long)T, cur()),
                      "decay_scan (chunks)");
       }
-    } else if (bp == nullptr && !unit && (mode == 3 || T >= 128l * S)) {
+    } else if (bp == nullptr && !unit && (mode == 3 || longest >= 256 || T >= 128l * S)) {
       // (us, 32 heads of 64 x 64, scan -> chunks: 16 segments of 64 rows 45 -> 52; one of 128, 16 heads, 29 -> 21; 13 of 500 140 ->
       // 104; 4 of 2048 428 -> 235)
       const long nb = k8sllm_hy_decay_chunk_ws(T, S, (int)H, (int)dk, (int)dv);

@@ -47,7 +47,8 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
   // common keys and queries
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
   if (pair >= S_ * H) return;
-  const int s = pair % S_, h = pair / S_, dvb = zb * NV;
+  // from the last segment on: a step's prompts come after its running sequences, and their chains take longest
+  const int s = S_ - 1 - pair / H, h = pair % H, dvb = zb * NV;
   const int sl = slot[s], t0 = cu[s], t1 = cu[s + 1];
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
@@ -266,16 +267,18 @@ using namespace k8sllm;
 // (nothing launched) for sizes that are not this kernel's: dk a multiple of 32 up to 128, dv of 16, rows 16-byte
 // aligned.  nt: value-column tiles per workgroup, 1, 2 or 4 (0: chosen here).
 extern "C" int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* state, const int* cu, const int* ctx,
-                                    const int* slot, int S, int H, int dk, int dv, int nt, hipStream_t s) {
+                                    const int* slot, int S, long T, int longest, int H, int dk, int dv, int nt, hipStream_t s) {
   if (S <= 0) return 0;
   if (dk % 32 || dk < 32 || dk > 128 || dv % 16 || dv < 16 || H < 1) return 1;
   if (nt != 0 && nt != 1 && nt != 2 && nt != 4) return -1;
   if (nt > 1 && dv % (16 * nt)) return 1;
-  // column blocks repeat the scores' products, so wide ones once they give enough workgroups to fill the chip (us for 16 / 32 /
-  // 64 columns, heads of 128 x 128: 5 x 1600 rows, 16 heads 182 / 134 / 125; 1 x 8000 rows 403 / 474 / 560)
-  const long pairs = (long)S * H;
-  if (nt == 0) nt = dv % 64 == 0 && pairs * (dv / 64) >= 144 ? 4 : dv % 32 == 0 && pairs * (dv / 32) >= 192 ? 2 : 1;
-  const dim3 grid((unsigned)((pairs + 7) / 8 * 8 * (dv / (16 * nt))));
+  // column blocks repeat the scores' products, so wide ones once they give enough workgroups to fill the chip; those of 32 columns
+  // only where 64 do not divide (us for 16 / 32 / 64 columns, 16 heads of 128 x 128: 5 x 1637 rows 179 / 153 / 121; 1 x 8000
+  // 382 / 567 / 526; 1000, 900, 800, 300 and three short 62 / 90 / 82; 2 x 2048 beside 32 single tokens 113 / 169 / 149).
+  // Segments count by the longest one's length (0: not known): single tokens beside it are a chunk each
+  const long pairs = (longest > 0 ? min((long)S, (T + longest - 1) / longest) : S) * H;
+  if (nt == 0) nt = dv % 64 == 0 ? (pairs * (dv / 64) >= 144 ? 4 : 1) : dv % 32 == 0 && pairs * (dv / 32) >= 192 ? 2 : 1;
+  const dim3 grid((unsigned)(((long)S * H + 7) / 8 * 8 * (dv / (16 * nt))));
 #define K8SLLM_CS(KS, NT)                                                                                           \
   hipLaunchKernelGGL((chunk_scan_kernel<KS, NT>), grid, dim3(512), 0, s, y, (const bf16_t*)vkq, decay, state, cu, ctx, \
                      slot, S, H, dv)

@@ -263,7 +263,8 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
   __shared__ __attribute__((aligned(16))) bf16_t Vl[2][kChunk * PV];
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
   if (pair >= S_ * H) return;
-  const int s = pair % S_, h = pair / S_, dvb = zb * NV;
+  // from the last segment on: a step's prompts come after its running sequences, and their chains take longest
+  const int s = S_ - 1 - pair / H, h = pair % H, dvb = zb * NV;
   const int sl = slot[s], t0 = cu[s], t1 = cu[s + 1];
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;

@@ -360,3 +360,29 @@ def test_expert_sort(n, E):
     want = torch.sort(ids.view(-1), stable=True).indices
     assert torch.equal(srt.cpu().long(), want) and torch.equal(inv.cpu().long(), torch.sort(want).indices)
     assert off.tolist() == [0] + torch.bincount(ids.view(-1).long(), minlength=E).cumsum(0).tolist()
+
+
+@pytest.mark.parametrize("longest", [0, 300])
+def test_scans_of_a_long_prompt_beside_single_tokens(longest):
+    """One prompt of 300 rows after 40 single tokens, where a known longest segment brings the chunks to linear attention, the delta
+    rule and decays per channel: both routes against the oracle.  Tolerances as for the chunks above: 2e-5, the delta rule 5e-5."""
+    g = _g(76)
+    lens = [1] * 40 + [300]
+    cu, ctx, slot = _segments(lens, [3 + i for i in range(40)] + [0], list(range(41)))
+    T, H, d = sum(lens), 2, 32
+    dev = [v.cuda() for v in (cu, ctx, slot)]
+
+    def check(f, state, tol):
+        a, b = state.clone(), state.cuda()
+        want, got = f(lambda v: v, a, cu, ctx, slot), f(lambda v: v.cuda(), b, *dev)
+        for x, y in ((got.cpu(), want), (b.cpu(), a)):
+            torch.testing.assert_close(x, y, rtol=tol, atol=tol * float(y.abs().max()))
+
+    qkv, z, zb, beta, bonus = _r(g, T, 3 * H * d, dt=BF), _r(g, T, H * d, dt=BF), _r(g, H * d) - 3.0, _r(g, T, H, dt=BF), _r(g, H, d)
+    lam, al = torch.sigmoid(_r(g, H) + 3.0), _r(g, H)
+    check(lambda c, s, *seg: hops.linear_attention(c(qkv), c(lam), s, *seg, H, d, d, longest=longest), _r(g, 41, H, d, d), 2e-5)
+    a = (0, H * d, 2 * H * d)
+    check(lambda c, s, *seg: hops.decay_scan(c(qkv), *a, c(z[:, :H].contiguous()), c(zb[:H]), s, *seg, H, H, d, d, d ** -0.5, a_log=c(al), beta=c(beta),
+                                             unit=True, longest=longest), _r(g, 41, H, d, d), 5e-5)
+    check(lambda c, s, *seg: hops.decay_scan(c(qkv), *a, c(z), c(zb), s, *seg, H, H, d, d, 1.0, decay="exp_exp", bonus=c(bonus),
+                                             longest=longest), _r(g, 41, H, d, d), 2e-5)
