@@ -12,6 +12,9 @@
 // sigmoid(gate[row][head]) before its one rounding.
 // The sink is one more softmax term with no value and a fixed score - 0, or a learned unscaled logit
 // per query head (sinks[h]): the running maximum starts at that score and the running denominator at 1.  Scores, weights and the output accumulation are fp32.
+#include <type_traits>
+#include <utility>
+
 #include "hy_common.h"
 
 namespace k8sllm {
@@ -329,6 +332,250 @@ __global__ __launch_bounds__(64 * NW) void window_decode_vec_kernel(bf16_t* __re
   }
 }
 
+// t = sum of 8 (4) products v[k] x[N + k], x's elements those of this 16-lane row (DPP row_newbcast), for one or two x at a time; the
+// second product first, then the first, the third, ..  The s_nop keeps the two wait states between a vector write and a DPP
+// read of the same register, whatever stands in front.
+template <int N>
+__device__ __forceinline__ void row_dot8(float xa, float xb, const float* v, float& ta, float& tb) {
+  asm("s_nop 1\n\t"
+      "v_mul_f32_dpp %[ta], %[xa], %[v1] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_mul_f32_dpp %[tb], %[xb], %[v1] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v0] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v0] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v2] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v2] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v3] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v3] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v4] row_newbcast:%[n4] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v4] row_newbcast:%[n4] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v5] row_newbcast:%[n5] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v5] row_newbcast:%[n5] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v6] row_newbcast:%[n6] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v6] row_newbcast:%[n6] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v7] row_newbcast:%[n7] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v7] row_newbcast:%[n7] row_mask:0xf bank_mask:0xf\n\t"
+      : [ta] "=&v"(ta), [tb] "=&v"(tb)
+      : [xa] "v"(xa), [xb] "v"(xb), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]), [v4] "v"(v[4]), [v5] "v"(v[5]), [v6] "v"(v[6]), [v7] "v"(v[7]), [n0] "n"(N + 0), [n1] "n"(N + 1), [n2] "n"(N + 2), [n3] "n"(N + 3), [n4] "n"(N + 4), [n5] "n"(N + 5), [n6] "n"(N + 6), [n7] "n"(N + 7));
+}
+template <int N>
+__device__ __forceinline__ void row_dot8(float xa, const float* v, float& ta) {
+  asm("s_nop 1\n\t"
+      "v_mul_f32_dpp %[ta], %[xa], %[v1] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v0] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v2] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v3] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v4] row_newbcast:%[n4] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v5] row_newbcast:%[n5] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v6] row_newbcast:%[n6] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v7] row_newbcast:%[n7] row_mask:0xf bank_mask:0xf\n\t"
+      : [ta] "=&v"(ta)
+      : [xa] "v"(xa), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]), [v4] "v"(v[4]), [v5] "v"(v[5]), [v6] "v"(v[6]), [v7] "v"(v[7]), [n0] "n"(N + 0), [n1] "n"(N + 1), [n2] "n"(N + 2), [n3] "n"(N + 3), [n4] "n"(N + 4), [n5] "n"(N + 5), [n6] "n"(N + 6), [n7] "n"(N + 7));
+}
+template <int N>
+__device__ __forceinline__ void row_dot4(float xa, float xb, const float* v, float& ta, float& tb) {
+  asm("s_nop 1\n\t"
+      "v_mul_f32_dpp %[ta], %[xa], %[v1] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_mul_f32_dpp %[tb], %[xb], %[v1] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v0] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v0] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v2] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v2] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v3] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[tb], %[xb], %[v3] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+      : [ta] "=&v"(ta), [tb] "=&v"(tb)
+      : [xa] "v"(xa), [xb] "v"(xb), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]), [n0] "n"(N + 0), [n1] "n"(N + 1), [n2] "n"(N + 2), [n3] "n"(N + 3));
+}
+template <int N>
+__device__ __forceinline__ void row_dot4(float xa, const float* v, float& ta) {
+  asm("s_nop 1\n\t"
+      "v_mul_f32_dpp %[ta], %[xa], %[v1] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v0] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v2] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %[ta], %[xa], %[v3] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+      : [ta] "=&v"(ta)
+      : [xa] "v"(xa), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]), [n0] "n"(N + 0), [n1] "n"(N + 1), [n2] "n"(N + 2), [n3] "n"(N + 3));
+}
+template <int N, typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
+}
+
+// The same for head sizes of 64 and 128, without the LDS reads that bound it (a tile of 64 keys took a wave 256 16-byte reads of
+// queries and weights that all lanes share): each 16-lane row holds all dims of the queries, 16 to a register, and a page's 16
+// weights in one, and the multiply-adds pick the element by their DPP row broadcast.  Keys and values of a tile are in flight
+// together.  Sums in the same order: the same bits.
+// 64 sequences, 1024 visible keys, 16 heads on 4 of 128: 40.8 -> 34.3 us (3.9 TB/s); 24 of ~1200, 32 on 8: 28.1 -> 25.5; 5 of 700, 8
+// heads on one of 128 / 64: 37 -> 27.  What is left of a tile is its ~1500 vector instructions.
+template <int R, int NW, int DKC, int VC>
+__global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv,
+                                                                long q_stride, const bf16_t* __restrict__ k_cache,
+                                                                const bf16_t* __restrict__ v_cache,
+                                                                const int* __restrict__ block_tables, int bt_stride,
+                                                                const int* __restrict__ seq_lens, int Hq, int G, float scale, int window, int chunked, int keep,
+                                                                float cap, int sink, const float* __restrict__ sinks,
+                                                                const bf16_t* __restrict__ gate, long g_stride) {
+  constexpr int bs = 16;
+  __shared__ __attribute__((aligned(16))) float p_s[NW][R][64];
+  __shared__ float ml_s[NW][R][2];
+  __shared__ float acc_s[NW][R][64 * VC];
+  constexpr int dk = 64 * DKC, dv = 64 * VC;
+  const int b = blockIdx.x, g = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = seq_lens[b];
+  bf16_t* o = out + (long)b * Hq * dv + (long)g * R * dv;
+  if (n <= 0) {  // padding row of a decode bucket
+    for (int c = threadIdx.x; c < R * dv; c += 64 * NW) o[c] = 0;
+    return;
+  }
+  const bf16_t* q = qkv + (long)b * q_stride + (long)g * R * dk;
+  // base-2 scores; lane l of every 16-lane row holds the queries' dims 16 i + l % 16
+  float qr[R][4 * DKC];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int i = 0; i < 4 * DKC; ++i) qr[r][i] = bf2f(q[r * dk + 16 * i + (lane & 15)]) * (scale * 1.44269504088896341f);
+  const int* bt = block_tables + (long)b * bt_stride;
+  const int lo = first_key(n - 1, window, chunked);
+  const float cap2 = cap * 1.44269504088896341f, icap2 = cap > 0.f ? 1.f / cap2 : 0.f;  // base-2 scores
+  const bool first = sink && wave == 0;
+  float m[R], l[R], acc[R][VC];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    // the sink's logit is not scaled; scores live in the base-2 domain
+    m[r] = first ? (sinks != nullptr ? sinks[g * R + r] * 1.44269504088896341f : 0.f) : -INFINITY;
+    l[r] = first ? 1.f : 0.f;
+#pragma unroll
+    for (int c = 0; c < VC; ++c) acc[r][c] = 0.f;
+  }
+  const long krs = (long)G * dk;
+  // the tiles that hold kept keys (kt of them, from position 0), then the window's from w0 on
+  const int kf = min(keep, n), kt = (kf + 63) >> 6, w0 = max(kt, lo >> 6);
+  for (int it = wave;; it += NW) {
+    const int j0 = 64 * (it < kt ? it : w0 + it - kt);
+    if (j0 >= n) break;
+    const int j = j0 + lane;
+    const bool valid = (j >= lo || j < keep) && j < n;
+    float sc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) sc[r] = 0.f;
+    // the lane's key row (of a key that is not seen: the newest one's)
+    uint4 kr[8 * DKC];
+    const int jc = valid ? j : n - 1;
+    const bf16_t* kp = k_cache + ((long)bt[jc / bs] * bs + jc % bs) * krs + (long)g * dk;
+#pragma unroll
+    for (int u = 0; u < 8 * DKC; ++u) kr[u] = *reinterpret_cast<const uint4*>(kp + 8 * u);
+    // value loads of the tile's pages go out before the arithmetic: 2 x 16 bytes per page and
+    // 64 dims (pages at or past the sequence's end are not touched: their weights are zero)
+    const int jend = j0 + 64 > lo ? n : kf;  // a tile of kept keys alone: the pages behind them are not needed
+    const int npg = min(4, (jend - j0 + bs - 1) / bs);
+    uint4 vq[4][VC][2];
+#pragma unroll
+    for (int pg = 0; pg < 4; ++pg)
+      if (pg < npg) {
+        const long base = ((long)bt[j0 / bs + pg] * G + g) * dv;
+#pragma unroll
+        for (int c = 0; c < VC; ++c)
+        {
+          const uint4* vp = reinterpret_cast<const uint4*>(v_cache + (base + lane + 64 * c) * bs);
+          vq[pg][c][0] = vp[0];
+          vq[pg][c][1] = vp[1];
+        }
+      }
+    static_for<8 * DKC>([&](auto uc) {
+      constexpr int u = decltype(uc)::value;
+      float kv[8];
+      unpack8(kr[u], kv);
+      constexpr int h = 8 * (u & 1);
+      if constexpr (R == 1) {
+        float t;
+        row_dot8<h>(qr[0][u / 2], kv, t);
+        sc[0] += t;
+      } else {
+#pragma unroll
+        for (int r = 0; r < R; r += 2) {
+          float t0, t1;
+          row_dot8<h>(qr[r][u / 2], qr[r + 1][u / 2], kv, t0, t1);
+          sc[r] += t0;
+          sc[r + 1] += t1;
+        }
+      }
+    });
+    __builtin_amdgcn_wave_barrier();  // this wave's previous reads of its p_s rows come first
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (cap > 0.f) sc[r] = cap2 * tanh_exp2(sc[r] * icap2);
+      const float sv = valid ? sc[r] : -INFINITY;
+      const float mt = fmaxf(m[r], wave_max_dpp(sv));  // the tile holds at least one live key, or m is the sink's
+      const float pw = (valid && mt != -INFINITY) ? __builtin_amdgcn_exp2f(sv - mt) : 0.f;
+      const float alpha = (m[r] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[r] - mt);
+      l[r] = l[r] * alpha + wave_sum_dpp(pw);
+      m[r] = mt;
+      p_s[wave][r][lane] = pw;
+#pragma unroll
+      for (int c = 0; c < VC; ++c) acc[r][c] *= alpha;
+    }
+    __builtin_amdgcn_wave_barrier();  // a wave's LDS instructions execute in issue order
+#pragma unroll
+    for (int pg = 0; pg < 4; ++pg)
+      if (pg < npg) {
+        float pr[R];  // every row of lanes: the page's 16 weights
+#pragma unroll
+        for (int r = 0; r < R; ++r) pr[r] = p_s[wave][r][16 * pg + (lane & 15)];
+#pragma unroll
+        for (int c = 0; c < VC; ++c) {
+          float vv[16];
+          unpack8(vq[pg][c][0], vv);
+          unpack8(vq[pg][c][1], vv + 8);
+          static_for<4>([&](auto tc) {
+            constexpr int t4 = 4 * decltype(tc)::value;
+            if constexpr (R == 1) {
+              float t;
+              row_dot4<t4>(pr[0], vv + t4, t);
+              acc[0][c] += t;
+            } else {
+#pragma unroll
+              for (int r = 0; r < R; r += 2) {
+                float t0, t1;
+                row_dot4<t4>(pr[r], pr[r + 1], vv + t4, t0, t1);
+                acc[r][c] += t0;
+                acc[r + 1][c] += t1;
+              }
+            }
+          });
+        }
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (int c = 0; c < VC; ++c)
+      acc_s[wave][r][lane + 64 * c] = acc[r][c];
+    if (lane == 0) {
+      ml_s[wave][r][0] = m[r];
+      ml_s[wave][r][1] = l[r];
+    }
+  }
+  __syncthreads();
+  for (int c = threadIdx.x; c < R * dv; c += 64 * NW) {
+    const int r = c / dv, dcol = c - r * dv;
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_s[w][r][0]);
+    float L = 0.f, val = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = ml_s[w][r][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml_s[w][r][0] - M);
+      L += ml_s[w][r][1] * f;
+      val += acc_s[w][r][dcol] * f;
+    }
+    const float gt = gate != nullptr ? sigmoid_f(bf2f(gate[(long)b * g_stride + g * R + r])) : 1.f;
+    o[c] = f2bf(L > 0.f ? val / L * gt : 0.f);
+  }
+}
+
 // bf16 prefill on the matrix cores, head sizes that are multiples of 32 (keys) / 16 (values).
 // One wave = 16 consecutive chunk rows of one sequence x one query head; key tiles of 16.
 //   S^T[key][q]  = K Q^T      v_mfma_f32_16x16x32_bf16: A = K rows (16-byte loads straight from the
@@ -623,6 +870,24 @@ int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const voi
   const int R = Hq / G;
   if (!f32 && vec && bs == 16 && dk % 8 == 0 && q_stride % 8 == 0 && dk <= kMaxDK && dv <= 64 * kMaxVC &&
       (R == 1 || R == 2 || R == 4 || R == 8)) {
+#define K8SLLM_WDR(RR, DKC, VC)                                                                                        \
+  hipLaunchKernelGGL((window_decode_row_kernel<RR, (RR == 8 ? 4 : 8), DKC, VC>), dim3(B, G), dim3(RR == 8 ? 256 : 512), 0, s, \
+                     (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, \
+                     bt_stride, seq_lens, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
+#define K8SLLM_WDD(DKC, VC)             \
+  if (R == 1) K8SLLM_WDR(1, DKC, VC);   \
+  else if (R == 2) K8SLLM_WDR(2, DKC, VC); \
+  else if (R == 4) K8SLLM_WDR(4, DKC, VC); \
+  else K8SLLM_WDR(8, DKC, VC)
+    if ((dk == 64 || dk == 128) && (dv == 64 || dv == 128)) {
+      if (dk == 64 && dv == 64) { K8SLLM_WDD(1, 1); }
+      else if (dk == 64) { K8SLLM_WDD(1, 2); }
+      else if (dv == 64) { K8SLLM_WDD(2, 1); }
+      else { K8SLLM_WDD(2, 2); }
+      return (int)hipGetLastError();
+    }
+#undef K8SLLM_WDD
+#undef K8SLLM_WDR
 #define K8SLLM_WD(RR)                                                                                                  \
   hipLaunchKernelGGL((window_decode_vec_kernel<RR, (RR == 8 ? 4 : 8)>), dim3(B, G), dim3(RR == 8 ? 256 : 512), 0, s,     \
                      (bf16_t*)out, (const bf16_t*)qkv,                                                                  \

@@ -386,3 +386,22 @@ def test_scans_of_a_long_prompt_beside_single_tokens(longest):
                                              unit=True, longest=longest), _r(g, 41, H, d, d), 5e-5)
     check(lambda c, s, *seg: hops.decay_scan(c(qkv), *a, c(z), c(zb), s, *seg, H, H, d, d, 1.0, decay="exp_exp", bonus=c(bonus),
                                              longest=longest), _r(g, 41, H, d, d), 2e-5)
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("Hq,G", [(3, 3), (4, 2), (4, 1), (16, 2)])  # 1, 2, 4, 8 heads per kv head
+def test_decode_attention_row_broadcasts(dk, dv, Hq, G):
+    """bf16 decode attention whose multiply-adds pick queries and weights from their 16-lane row: lengths around pages, tiles of 64 and
+    a round of all waves, windows, kept tokens, caps, sinks.  bf16 rounding of the result: 2e-2; fp32 inside, so against the
+    oracle on the same bf16 values half a unit in the last place and a few more."""
+    g = _g(77)
+    lens = [1, 15, 16, 17, 63, 64, 65, 500, 600, 0]
+    W = max((n + 15) // 16 for n in lens)
+    bt = torch.randperm(len(lens) * W, generator=g).int().view(-1, W)
+    kc, vc = _r(g, bt.numel(), 16, G * dk, dt=BF), _r(g, bt.numel(), G, dv, 16, dt=BF)
+    q, gate, sl = _r(g, len(lens), Hq * dk + G * (dk + dv), dt=BF), _r(g, len(lens), Hq, dt=BF), _i32(lens)
+    for window, sink, kw in ((0, False, {}), (70, True, dict(keep=20)), (64, False, dict(chunked=True, cap=2.0))):
+        a = (Hq, G, dk, dv, dk ** -0.5, window, sink)
+        want = hops.window_attention_decode(q, kc, vc, bt, sl, *a, gate=gate, **kw)
+        got = hops.window_attention_decode(q.cuda(), kc.cuda(), vc.cuda(), bt.cuda(), sl.cuda(), *a, gate=gate.cuda(), **kw)
+        torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1e-2, atol=2e-3)
