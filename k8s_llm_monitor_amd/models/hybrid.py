@@ -966,10 +966,10 @@ class GatedDenseFFN:
         self.w_down = p.get(prefix + "down", (d, self.ff), 1.0 / math.sqrt(self.ff))
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        proj = hops.linear(h, self.w_in)
+        a, rest, col = hops.linear_glu(h, self.w_in, self.ff, self.act)
         if self.n_tail:
-            self.tail_out = (proj, 2 * self.ff)
-        return hops.linear(hops.glu(proj, 0, self.ff, self.act), self.w_down)
+            self.tail_out = (rest, col)
+        return hops.linear(a, self.w_down)
 
 
 class PlainRoutedFFN:

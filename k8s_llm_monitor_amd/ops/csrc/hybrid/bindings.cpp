@@ -91,6 +91,8 @@ int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* s
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
                      const float* bias, int E, int K, int rows_w, int over_all, int f32, hipStream_t s);
 int k8sllm_hy_few_rows(void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, hipStream_t s);
+int k8sllm_hy_few_rows_glu(void* yg, void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, int f, int kind,
+                           hipStream_t s);
 int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* offsets, const int* sorted_idx, int div,
                            int E, long rows, int N, int Kd, long w_es, int act, int il, int f32, int mfma, float limit,
                            hipStream_t s);
@@ -915,6 +917,23 @@ void few_rows(Tensor y, Tensor x, Tensor w) {
         "few_rows");
 }
 
+// yg [M, f]: the gated unit of w's rows [f gate | f up | ..]; y [M, N - 2 f]: the other rows' products; see few_rows.hip
+void few_rows_glu(Tensor yg, Tensor y, Tensor x, Tensor w, int64_t kind) {
+  TORCH_CHECK(act(x, "x") == 0, "few_rows_glu: bf16");
+  same(w, 0, "w");
+  same(y, 0, "y");
+  same(yg, 0, "yg");
+  const int64_t f = yg.size(1);
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && w.dim() == 2 && w.is_contiguous() && y.dim() == 2 && y.is_contiguous() &&
+                  yg.dim() == 2 && yg.is_contiguous() && yg.size(0) == x.size(0) && y.size(0) == x.size(0) &&
+                  2 * f + y.size(1) == w.size(0) && x.size(1) == w.size(1),
+              "few_rows_glu: layouts");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0, "few_rows_glu: alignment");
+  check(k8sllm_hy_few_rows_glu(yg.data_ptr(), y.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), (int)x.size(0), (int)w.size(0),
+                               (int)x.size(1), (int)f, (int)kind, cur()),
+        "few_rows_glu");
+}
+
 void grouped_gemm(Tensor y, Tensor a, Tensor w, Tensor offsets, OptT sorted_idx, int64_t div, int64_t act_code, bool il,
                   bool mfma, double limit) {
   TORCH_CHECK(act_code >= 0 && act_code <= 4 && (act_code != 3 || limit > 0), "grouped_gemm: activation code");
@@ -1161,6 +1180,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_router", &moe_router);
   m.def("moe_align", &moe_align);
   m.def("few_rows", &few_rows);
+  m.def("few_rows_glu", &few_rows_glu);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("moe_combine", &moe_combine);
   m.def("norm_shift", &norm_shift);

@@ -88,6 +88,31 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
 __device__ __forceinline__ float silu_f(float z) { return z / (1.f + __expf(-z)); }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
 
+// KIND 0: erf GELU, 1: tanh GELU, 2: xIELU (a z^2 + z/2 above zero, b (exp(z) - 1 - z) + z/2 below), 3: SiLU,
+// 4: ReLU, 6: squared ReLU, 7: tanh (5 is a gated unit, glu_unit)
+template <int KIND>
+__device__ __forceinline__ float act_f(float z, float a, float b) {
+  if (KIND == 6) return z > 0.f ? z * z : 0.f;
+  if (KIND == 7) return tanhf(z);
+  if (KIND == 4) return fmaxf(z, 0.f);
+  if (KIND == 0) return 0.5f * z * (1.f + erff(z * 0.70710678118654752f));
+  if (KIND == 1) return 0.5f * z * (1.f + tanhf(0.79788456080286536f * (z + 0.044715f * z * z * z)));
+  if (KIND == 3) return z / (1.f + expf(-z));
+  return z > 0.f ? a * z * z + 0.5f * z : b * (expm1f(z) - z) + 0.5f * z;
+}
+
+// KIND 5: the clamped unit g sigmoid(1.702 g) (u + 1) with g = min(gate, limit), u = clamp(up, -limit, limit);
+// others: act(gate) * up
+template <int KIND>
+__device__ __forceinline__ float glu_unit(float g, float u, float limit) {
+  if (KIND == 5) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g * sigmoid_f(1.702f * g) * (u + 1.f);
+  }
+  return act_f<KIND>(g, 0.f, 0.f) * u;
+}
+
 // sum over groups of CH neighbouring lanes (CH a power of two <= 32, groups aligned); every lane of a group
 // ends with its total
 template <int CH>

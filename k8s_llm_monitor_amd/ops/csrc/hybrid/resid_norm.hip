@@ -337,19 +337,6 @@ __global__ __launch_bounds__(256) void depth_mix_scalar_kernel(float* __restrict
   stack[(long)(n + 1) * plane + i] = acc + coef[n] * top;
 }
 
-// KIND 0: erf GELU, 1: tanh GELU, 2: xIELU (a z^2 + z/2 above zero, b (exp(z) - 1 - z) + z/2 below), 3: SiLU,
-// 4: ReLU, 6: squared ReLU, 7: tanh (5 is a gated unit, glu_unit)
-template <int KIND>
-__device__ __forceinline__ float act_f(float z, float a, float b) {
-  if (KIND == 6) return z > 0.f ? z * z : 0.f;
-  if (KIND == 7) return tanhf(z);
-  if (KIND == 4) return fmaxf(z, 0.f);
-  if (KIND == 0) return 0.5f * z * (1.f + erff(z * 0.70710678118654752f));
-  if (KIND == 1) return 0.5f * z * (1.f + tanhf(0.79788456080286536f * (z + 0.044715f * z * z * z)));
-  if (KIND == 3) return z / (1.f + expf(-z));
-  return z > 0.f ? a * z * z + 0.5f * z : b * (expm1f(z) - z) + 0.5f * z;
-}
-
 // out [rows, n] (contiguous) = act(x[:, 0:n]) where x's rows are x_stride apart; 8 columns per thread
 // where n, the stride and the column offset are multiples of 8 (vec)
 template <typename T, int KIND>
@@ -369,18 +356,6 @@ __global__ __launch_bounds__(256) void activation_cols_kernel(T* __restrict__ ou
     return;
   }
   stf(out + r * n + c, act_f<KIND>(ldf(x + r * x_stride + c), 0.f, 0.f));
-}
-
-// KIND 5: the clamped unit g sigmoid(1.702 g) (u + 1) with g = min(gate, limit), u = clamp(up, -limit, limit);
-// others: act(gate) * up
-template <int KIND>
-__device__ __forceinline__ float glu_unit(float g, float u, float limit) {
-  if (KIND == 5) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-    return g * sigmoid_f(1.702f * g) * (u + 1.f);
-  }
-  return act_f<KIND>(g, 0.f, 0.f) * u;
 }
 
 // out [rows, f] = act(gu[:, 0:f]) * gu[:, f:2f], gu's rows g_stride apart

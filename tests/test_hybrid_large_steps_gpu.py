@@ -405,3 +405,15 @@ def test_decode_attention_row_broadcasts(dk, dv, Hq, G):
         want = hops.window_attention_decode(q, kc, vc, bt, sl, *a, gate=gate, **kw)
         got = hops.window_attention_decode(q.cuda(), kc.cuda(), vc.cuda(), bt.cuda(), sl.cuda(), *a, gate=gate.cuda(), **kw)
         torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1e-2, atol=2e-3)
+
+
+@pytest.mark.parametrize("M,f,rest,K", [(1, 16, 0, 32), (3, 48, 40, 1024), (16, 176, 16, 160), (17, 32, 8, 64), (2, 24, 8, 64)])
+@pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
+def test_gated_unit_in_the_projection(M, f, rest, K, kind):
+    """The gated unit at the end of a few rows' projection gives the bits of the projection and the unit as two launches, and so do
+    the rows of the weights behind the unit's (one row, or an f that is no multiple of 16, past its limits: two launches)."""
+    g = _g(78)
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, 2 * f + rest, K, s=K ** -0.5, dt=BF).cuda()
+    a, y, col = hops.linear_glu(x, w, f, kind)
+    proj = hops.linear(x, w)
+    assert torch.equal(a, hops.glu(proj, 0, f, kind)) and torch.equal(y[:, col:col + rest], proj[:, 2 * f:])
