@@ -202,14 +202,15 @@ class ModelRunner:
         # layout of the staging buffer (int32 words; the float sampling parameters bit-cast)
         nl = sum(len(x) for x in logit_rows) if logit_rows is not None else R
         hy = R if self.hybrid else 0
-        # layer-list models: the chunks' pages in one list, and where each chunk's begin in it
-        npg = [(c + n + BLOCK_SIZE - 1) // BLOCK_SIZE for c, n in zip(starts, lens)] if hy else []
+        # latent attention: the chunks' pages in one list, and where each chunk's begin in it
+        npg = [(c + n + BLOCK_SIZE - 1) // BLOCK_SIZE for c, n in zip(starts, lens)] if hy and self.model.lists_pages else []
         sizes = dict(ids=T, pos=T, slots=T, cu=len(seqs) + 1, qs=nq, st=nq, lidx=nl, temp=R, topk=R, topp=R,
                      gcu=hy + 1 if hy else 0, gctx=hy, gslot=hy,
-                     pgl=sum(npg), pgb=len(npg) * W,
                      cst=len(seqs) if paged else 0, bt=len(seqs) * W, dbt=nd * Wd, dlen=nd,
                      mcu=len(seqs) + 2 if kA else 0, mqs=nq if kA else 0, mst=nq if kA else 0,
                      mlidx=len(seqs) if kA else 0)
+        if npg:
+            sizes.update(pgl=sum(npg), pgb=len(npg) * W)
         off, o = {}, 0
         for k, n in sizes.items():
             off[k] = o
@@ -256,11 +257,10 @@ class ModelRunner:
             bt2[:] = 0
             for i, s in enumerate(seqs):
                 bt2[i, : len(s.block_table)] = s.block_table
-            o = 0
-            for i, k in enumerate(npg):
-                v["pgl"][o:o + k] = bt2[i, :k]
-                v["pgb"][i * W:(i + 1) * W] = np.minimum(np.arange(o, o + W), o + k - 1)
-                o += k
+            if npg:
+                k, end = np.asarray(npg), np.cumsum(npg)
+                v["pgl"][:] = bt2[np.arange(W) < k[:, None]]
+                v["pgb"][:] = np.minimum((end - k)[:, None] + np.arange(W), end[:, None] - 1).ravel()
         if nd:
             dbt = v["dbt"].reshape(nd, Wd)
             dbt[:] = 0
@@ -286,7 +286,7 @@ class ModelRunner:
         if hy:
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = dv["gcu"], dv["gctx"], dv["gslot"]
             meta.seg_max = max([1] * (nd > 0) + lens)
-            if seqs:
+            if npg:
                 meta.page_list, meta.page_bt = dv["pgl"], dv["pgb"].view(len(seqs), W)
         if kA:
             TA, S_ = int(cu[kA]), len(seqs)

@@ -241,6 +241,7 @@ class LatentAttention:
     2 x 2000 behind 2816 1740 -> 200; 16 x 64 behind 4000, 64 positions per row, 428 -> 513)."""
 
     kind = "latent_attention"
+    lists_pages = True  # its expanded form reads a step's pages as one list (AttnMeta.page_list)
     EXPAND_MIN_ROWS = 64
     EXPAND_KEYS = 32
 
@@ -829,6 +830,7 @@ class SideBySide:
         self.out_w = None if self.mix is None else tuple(p.get(f"{prefix}{side}.out", (d,), 0.1, 1.0, small=True)
                                                          for side in ("left", "right"))
         self.stateful = any(getattr(x, "stateful", False) for x in self.subs)
+        self.lists_pages = any(getattr(x, "lists_pages", False) for x in self.subs)
         # each mixer's rows padded with zeros to a multiple of 8: the kernels' 16-byte accesses need aligned
         # row strides and first columns
         parts, self.cols = [], []
@@ -1231,6 +1233,7 @@ class HybridLM:
             self.kv_run.append(prev[-1])
         self.unused = sorted(set(weights.keys()) - p.used) if weights is not None else []
         self.has_state = self.shifted or any(getattr(m, "stateful", False) for m in self.mixers)
+        self.lists_pages = any(getattr(m, "lists_pages", False) for m in self.mixers)
         # large steps of such layers run on the Mixtral path's tile GEMM (extension _k8sllm_ops)
         self.uses_tile_gemm = any(f is not None and (getattr(f, "il", False) or getattr(f, "tile", False))
                                   for f in self.ffns)
