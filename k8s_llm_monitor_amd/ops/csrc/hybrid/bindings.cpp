@@ -81,11 +81,11 @@ int k8sllm_hy_delta_chunk(float* o, const void* qkv, long stride, int q_col, int
                           const float* z_bias, const float* a_log, float inv_tau, int dkind, const void* beta, long b_stride,
                           float* state, const int* cu, const int* ctx, const int* slot, int S, int H, int Gk, int dk, int dv,
                           float q_scale, int unit, void* ws, long T, hipStream_t s);
-long k8sllm_hy_decay_chunk_ws(long T, int S, int H, int dk, int dv);
+long k8sllm_hy_decay_chunk_ws(long T, int S, int longest, int H, int dk, int dv, int mode);
 int k8sllm_hy_decay_chunk(float* o, const void* qkv, long stride, int q_col, int k_col, int v_col, const void* z, long z_stride,
                           const float* z_bias, const float* a_log, float inv_tau, int dkind, const float* bonus, float* state,
                           const int* cu, const int* ctx, const int* slot, int S, int H, int Gk, int dk, int dv, float q_scale,
-                          void* ws, long T, hipStream_t s);
+                          void* ws, long T, int longest, int mode, hipStream_t s);
 int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* state, const int* cu, const int* ctx,
                          const int* slot, int S, long T, int longest, int H, int dk, int dv, int nt, hipStream_t s);
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
@@ -736,7 +736,7 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
   // 64 x 64: one of 2000 rows beside 60 575 -> 186, 399 -> 181; one of 256 beside 60 142 -> 139, 125 -> 107)
   const bool prompts = T >= 32l * S || longest >= 256;
   const void* zp = (const char*)z.data_ptr() + z_col * z.element_size();
-  if (!f && (mode == 3 || (mode == 0 && prompts)) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 &&
+  if (!f && (mode >= 3 || (mode == 0 && prompts)) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 &&
       qkv.stride(0) % 8 == 0 && q_col % 8 == 0 && k_col % 8 == 0 && v_col % 8 == 0) {
     // a chunk costs the same whatever it holds (us, 16 heads of 128 x 128, scan -> chunks: 40 segments of 33 rows 99 -> 101;
     // 16 of 64 73 -> 51; one of 64 21 -> 28; 4 of 2048 542 -> 209)
@@ -751,17 +751,18 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
                                            ws.data_ptr(), (long)T, cur()),
                      "decay_scan (chunks)");
       }
-    } else if (bp == nullptr && !unit && (mode == 3 || longest >= 256 || T >= 128l * S)) {
+    } else if (bp == nullptr && !unit && (mode >= 3 || longest >= 256 || T >= 128l * S)) {
       // (us, 32 heads of 64 x 64, scan -> chunks: 16 segments of 64 rows 45 -> 52; one of 128, 16 heads, 29 -> 21; 13 of 500 140 ->
       // 104; 4 of 2048 428 -> 235)
-      const long nb = k8sllm_hy_decay_chunk_ws(T, S, (int)H, (int)dk, (int)dv);
+      const int cut = mode == 4 ? 2 : mode == 3 ? 1 : 0;  // spans of chunks: forced, not, by the sizes
+      const long nb = k8sllm_hy_decay_chunk_ws(T, S, (int)longest, (int)H, (int)dk, (int)dv, cut);
       if (nb > 0) {
         Tensor ws = torch::empty({nb}, o.options().dtype(torch::kUInt8));
         return check(k8sllm_hy_decay_chunk(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
                                            zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind,
                                            wp_bonus, state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(),
                                            slot.data_ptr<int>(), S, (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale,
-                                           ws.data_ptr(), (long)T, cur()),
+                                           ws.data_ptr(), (long)T, (int)longest, cut, cur()),
                      "decay_scan (chunks)");
       }
     }

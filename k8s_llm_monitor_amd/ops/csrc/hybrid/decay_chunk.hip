@@ -14,11 +14,12 @@
 //  * decay_chunk_scan: eight waves per (segment, head, 16 NT value columns) walk the chunks, four for O, four for S; S is
 //    published in LDS as three parts, double-buffered: one barrier per chunk.  Values are bf16 activations (exact), so
 //    their products take three instructions, Q' S the six that matter at 2^-24.
+//    Long segments that leave the chip idle are cut into spans of chunks: a launch for their ends, one for the outputs.
 // What bounds it: the scan by the workspace's operands (72 KiB per chunk and head at 64 channels, read by every column block:
 // 1.2 us a chunk at the 25 bytes per clock that a CU draws from L2, where the products and the trip through LDS take 0.3);
 // the preparation by vector instructions.
-// Measured, both launches (us; the staged scan with its preparation), 32 heads of 64 x 64 with a bonus: 1 x 8000 rows 384
-// (1347), 4 x 2048 235 (428); plain, 16 heads of 128 x 128: 1 x 8000 591 (1548), 4 x 2048 407 (567).  Error against 64 bits, 2048
+// Measured, both launches (us; the staged scan with its preparation), 32 heads of 64 x 64 with a bonus: 1 x 8000 rows 254
+// (1347), 4 x 2048 235 (428); plain, 16 heads of 128 x 128: 1 x 8000 436 (1548), 4 x 2048 407 (567).  Error against 64 bits, 2048
 // rows, bonus: outputs 1.3e-7 (scan 2.7e-7), state 7.9e-8 (3.0e-7); plain: 2.3e-7 (1.5e-6), 2.1e-7 (2.0e-6).
 #include "chunk_seg.h"
 #include "split_bf16.h"
@@ -252,20 +253,33 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
   }
 }
 
-template <int KS, int NT>
+constexpr int kWhole = 0, kSpanEnds = 1, kSpanRun = 2;
+
+// MODE kWhole: workgroups own whole segments.  Else a segment is cut into spans of `span` chunks that run side by side: kSpanEnds
+// leaves the end state of every span but a segment's last from a zero state in spans_s [span][head][dv][channels], its decays'
+// products in spans_d [span][head][channels], and the state that the segment starts from in its last span's place; kSpanRun
+// folds those in front of its own span, S <- diag(d_j) S + E_j.
+template <int KS, int NT, int MODE>
 __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restrict__ o, const bf16_t* __restrict__ qkv,
                                                                   long stride, int v_col, const bf16_t* __restrict__ mats,
                                                                   const float* __restrict__ ends, float* __restrict__ state,
                                                                   const int* __restrict__ cu, const int* __restrict__ ctx,
-                                                                  const int* __restrict__ slot, int S_, int H, int dv) {
+                                                                  const int* __restrict__ slot, int S_, int H, int dv, int span, int n_span,
+                                                                  float* __restrict__ spans_s, float* __restrict__ spans_d) {
   constexpr int DK = 32 * KS, PK = DK + 8, NV = 16 * NT, PV = NV + 8, RTW = (2 * KS + 3) / 4;
   __shared__ __attribute__((aligned(16))) bf16_t Sl[2][3][NV * PK];  // the state before a chunk, [column][channel]
   __shared__ __attribute__((aligned(16))) bf16_t Vl[2][kChunk * PV];
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
-  if (pair >= S_ * H) return;
+  if (pair >= (MODE == kWhole ? S_ : n_span) * H) return;
   // from the last segment on: a step's prompts come after its running sequences, and their chains take longest
-  const int s = S_ - 1 - pair / H, h = pair % H, dvb = zb * NV;
-  const int sl = slot[s], t0 = cu[s], t1 = cu[s + 1];
+  const int h = pair % H, dvb = zb * NV, sp_i = n_span - 1 - pair / H;
+  ChunkAt at = {S_ - 1 - pair / H, 0, 0, 0, 1};
+  if (MODE != kWhole) {
+    at = chunk_at(cu, S_, sp_i, span * kChunk);
+    if (at.seg < 0 || (MODE == kSpanEnds && (at.k == at.count - 1 || slot[at.seg] < 0))) return;
+  }
+  const int s = at.seg;
+  const int sl = slot[s], t0 = MODE == kWhole ? cu[s] : at.row, t1 = MODE == kWhole ? cu[s + 1] : at.row + at.n;
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const bool outs = wave < 4;  // wave-uniform
@@ -275,10 +289,10 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
     return;
   }
   if (t1 <= t0) return;
-  const int c0 = first_chunk(cu, s);
+  const int c0 = first_chunk(cu, s) + (MODE == kWhole ? 0 : at.k * span);
   f32x4 S[RTW][NT];  // S[16 (w RTW + r) + 4 quad + i][16 ct + c16]
   float* sp = state + (((long)sl * H + h) * dv + dvb) * DK;
-  const bool carried = ctx[s] > 0, mine = !outs && w * RTW < 2 * KS;
+  const bool carried = ctx[s] > 0 && (MODE == kWhole || at.count == 1 || (MODE == kSpanEnds && at.k == 0)), mine = !outs && w * RTW < 2 * KS;
 #pragma unroll
   for (int r = 0; r < RTW; ++r)
 #pragma unroll
@@ -290,7 +304,40 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
         S[r][ct] = f32x4{v.x, v.y, v.z, v.w};
       }
     }
+  // the place of span j of this segment; this thread's part of a state there
+  auto end_of = [&](int j) { return spans_s + (((long)(sp_i - at.k + j) * H + h) * dv + dvb) * DK; };
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int r = 0; r < RTW; ++r)
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct) {
+        const int row = 16 * (w * RTW + r) + 4 * quad;
+        if (mine && row < DK) f(S[r][ct], (long)(16 * ct + c16) * DK + row, r, row);
+      }
+  };
+  float4 prod[RTW];
+#pragma unroll
+  for (int r = 0; r < RTW; ++r) prod[r] = make_float4(1.f, 1.f, 1.f, 1.f);
+  if (MODE == kSpanEnds && at.k == 0) {
+    float* p = end_of(at.count - 1);
+    each([&](f32x4& v, long o, int, int) {
+      *reinterpret_cast<f32x4*>(p + o) = v;
+      v = f32x4{0.f, 0.f, 0.f, 0.f};
+    });
+  }
+  if (MODE == kSpanRun && at.count > 1) {
+    const float* p = end_of(at.count - 1);
+    each([&](f32x4& v, long o, int, int) { v = *reinterpret_cast<const f32x4*>(p + o); });
+    for (int j = 0; j < at.k; ++j) {
+      const float* e = end_of(j);
+      const float* d = spans_d + ((long)(sp_i - at.k + j) * H + h) * DK;
+      each([&](f32x4& v, long o, int, int row) {
+        v = v * *reinterpret_cast<const f32x4*>(d + row) + *reinterpret_cast<const f32x4*>(e + o);
+      });
+    }
+  }
   auto publish = [&](int buf) {
+    if (MODE == kSpanEnds) return;  // nobody reads it
 #pragma unroll
     for (int r = 0; r < RTW; ++r) {
       const int rt = w * RTW + r;
@@ -320,6 +367,7 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
     const long ch = (long)(c0 + (tb - t0) / kChunk) * H + h;
     const bf16_t* m = mats + ch * kc_mats(DK) + lane * 8;
     if (outs) {
+      if (MODE == kSpanEnds) return;
 #pragma unroll
       for (int i = 0; i < 3 * KS; ++i) mn[i] = *reinterpret_cast<const bf16x8*>(m + (long)(3 * KS * w + i) * 512);
       m += 3 * 64 * DK;
@@ -370,7 +418,7 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
       if (tb + 2 * kChunk < t1) fetch_v(tb + 2 * kChunk);
     }
     if (outs) {
-      if (16 * w < n) {
+      if (MODE != kSpanEnds && 16 * w < n) {
 #pragma unroll
         for (int ct = 0; ct < NT; ++ct) {  // (column 16 ct + 4 quad + i, query c16)
           f32x4 d[3] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
@@ -396,6 +444,10 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
         }
       }
     } else if (mine) {
+      if (MODE == kSpanEnds)
+#pragma unroll
+        for (int r = 0; r < RTW; ++r)
+          prod[r] = make_float4(prod[r].x * ef[r].x, prod[r].y * ef[r].y, prod[r].z * ef[r].z, prod[r].w * ef[r].w);
 #pragma unroll
       for (int r = 0; r < RTW; ++r)
 #pragma unroll
@@ -419,17 +471,19 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
       publish(buf ^ 1);
     }
   }
-  if (mine) {
+  if (MODE == kSpanEnds) {
+    sp = end_of(at.k);
+    if (zb == 0 && c16 == 0) {
+      float* d = spans_d + ((long)sp_i * H + h) * DK;
 #pragma unroll
-    for (int r = 0; r < RTW; ++r)
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct) {
+      for (int r = 0; r < RTW; ++r) {
         const int row = 16 * (w * RTW + r) + 4 * quad;
-        if (row < DK)
-          *reinterpret_cast<float4*>(sp + (long)(16 * ct + c16) * DK + row) =
-              make_float4(S[r][ct][0], S[r][ct][1], S[r][ct][2], S[r][ct][3]);
+        if (mine && row < DK) *reinterpret_cast<float4*>(d + row) = prod[r];
       }
+    }
   }
+  if (MODE != kSpanRun || at.k == at.count - 1)
+    each([&](f32x4& v, long o, int, int) { *reinterpret_cast<f32x4*>(sp + o) = v; });
 }
 
 }  // namespace k8sllm
@@ -438,33 +492,60 @@ using namespace k8sllm;
 
 extern "C" {
 
-// bytes of workspace for T rows in S segments; 0: not a case for these kernels (dk a multiple of 32 up to 128, dv of 16)
-long k8sllm_hy_decay_chunk_ws(long T, int S, int H, int dk, int dv) {
+// Chunks per span of a step cut into spans, 0: whole segments.  Cut where long chains leave the chip idle - spans then take 64 columns
+// at once, a quarter of the operand traffic, and twice the state's products (us, whole / spans, 32 heads of 64 x 64: 1 x 8000 rows
+// 384 / 254, 1 x 2048 79 / 69, 2 x 4000 291 / 259, 4 x 2048, not cut, 239 / 241; 16 heads 1 x 8000 217 / 133; plain, 16 heads of
+// 128 x 128, 1 x 8000 605 / 436) - about 256 workgroups of them.
+static int span_chunks(long T, int S, int longest, int H, int dv, int mode) {
+  const long n = longest > 0 ? longest : S > 0 ? T / S : 0;
+  const int cols = dv % 64 == 0 ? dv / 64 : dv % 32 == 0 ? dv / 32 : dv / 16;
+  if (n <= 0 || mode == 1 || (mode == 0 && (n < 1536 || H * ((T + n - 1) / n) * (dv / 16) > 256))) return 0;
+  const long want = T / kChunk * H * cols / 256;
+  return (int)(want < 4 ? 4 : want > 32 ? 32 : want);
+}
+
+// bytes of workspace for T rows in S segments, the longest of `longest` rows (0: not known, the mean is taken); 0: not a case for
+// these kernels (dk a multiple of 32 up to 128, dv of 16).  mode 1 / 2: whole segments / spans whatever the sizes
+long k8sllm_hy_decay_chunk_ws(long T, int S, int longest, int H, int dk, int dv, int mode) {
   if (dk % 32 || dk < 32 || dk > 128 || dv % 16 || dv < 16) return 0;
-  return (T / kChunk + S) * H * (kc_mats(dk) * 2 + dk * 4);
+  const int span = span_chunks(T, S, longest, H, dv, mode);
+  return (T / kChunk + S) * H * (kc_mats(dk) * 2 + dk * 4) + (span > 0 ? (T / (span * kChunk) + S) * H * (long)dk * (dv + 1) * 4 : 0);
 }
 
 // as k8sllm_hy_decay_scan's plain form (bonus nullptr) or bonus form, without unit norms
 int k8sllm_hy_decay_chunk(float* o, const void* qkv, long stride, int q_col, int k_col, int v_col, const void* z, long z_stride,
                           const float* z_bias, const float* a_log, float inv_tau, int dkind, const float* bonus, float* state,
                           const int* cu, const int* ctx, const int* slot, int S, int H, int Gk, int dk, int dv, float q_scale,
-                          void* ws, long T, hipStream_t s) {
+                          void* ws, long T, int longest, int mode, hipStream_t s) {
   if (S <= 0 || T <= 0) return 0;
-  if (k8sllm_hy_decay_chunk_ws(T, S, H, dk, dv) == 0 || Gk < 1 || H % Gk || dkind < 0 || dkind > 2 || (dkind == 0 && a_log == nullptr))
+  if (k8sllm_hy_decay_chunk_ws(T, S, longest, H, dk, dv, mode) == 0 || Gk < 1 || H % Gk || dkind < 0 || dkind > 2 || (dkind == 0 && a_log == nullptr))
     return -1;
   const long nch = T / kChunk + S;
   bf16_t* mats = (bf16_t*)ws;
   float* ends = (float*)(mats + nch * H * kc_mats(dk));
   const long pairs = (long)S * H;
   // narrow column blocks until they fill the chip: the chain of chunks bounds a block
-  const int nt = dv % 64 == 0 && pairs * (dv / 16) >= 1024 ? 4 : dv % 32 == 0 && pairs * (dv / 16) >= 512 ? 2 : 1;
-  const dim3 grid((unsigned)((pairs + 7) / 8 * 8 * (dv / (16 * nt)))), pgrid((unsigned)nch, (unsigned)H);
+  const int span = span_chunks(T, S, longest, H, dv, mode);
+  const long n_span = span > 0 ? T / (span * kChunk) + S : S, units = n_span * H;
+  float* spans_s = ends + nch * H * dk;
+  float* spans_d = spans_s + units * dk * dv;
+  const int nt = dv % 64 == 0 && (span > 0 || pairs * (dv / 16) >= 1024) ? 4 : dv % 32 == 0 && (span > 0 || pairs * (dv / 16) >= 512) ? 2 : 1;
+  const dim3 grid((unsigned)((units + 7) / 8 * 8 * (dv / (16 * nt)))), pgrid((unsigned)nch, (unsigned)H);
 #define K8SLLM_KCP(KS, B)                                                                                                    \
   hipLaunchKernelGGL((decay_chunk_prep_kernel<KS, B>), pgrid, dim3(256), 0, s, mats, ends, (const bf16_t*)qkv, stride, q_col, \
                      k_col, (const bf16_t*)z, z_stride, z_bias, a_log, inv_tau, dkind, bonus, cu, slot, S, H, Gk, q_scale)
-#define K8SLLM_KCS(KS, NT)                                                                                                   \
-  hipLaunchKernelGGL((decay_chunk_scan_kernel<KS, NT>), grid, dim3(512), 0, s, o, (const bf16_t*)qkv, stride, v_col, mats, ends, \
-                     state, cu, ctx, slot, S, H, dv)
+#define K8SLLM_KCM(KS, NT, MODE)                                                                                             \
+  hipLaunchKernelGGL((decay_chunk_scan_kernel<KS, NT, MODE>), grid, dim3(512), 0, s, o, (const bf16_t*)qkv, stride, v_col, mats, \
+                     ends, state, cu, ctx, slot, S, H, dv, span, (int)n_span, spans_s, spans_d)
+#define K8SLLM_KCS(KS, NT)                       \
+  do {                                           \
+    if (span > 0) {                              \
+      K8SLLM_KCM(KS, NT, kSpanEnds);             \
+      K8SLLM_KCM(KS, NT, kSpanRun);              \
+    } else {                                     \
+      K8SLLM_KCM(KS, NT, kWhole);                \
+    }                                            \
+  } while (0)
 #define K8SLLM_KC(KS)                        \
   if (bonus != nullptr) K8SLLM_KCP(KS, true); \
   else K8SLLM_KCP(KS, false);                \
@@ -478,6 +559,7 @@ int k8sllm_hy_decay_chunk(float* o, const void* qkv, long stride, int q_col, int
     default: K8SLLM_KC(4); break;
   }
 #undef K8SLLM_KC
+#undef K8SLLM_KCM
 #undef K8SLLM_KCS
 #undef K8SLLM_KCP
   return (int)hipGetLastError();

@@ -902,7 +902,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     per head, and without the delta rule and unit norms of decays per channel (``dk`` a multiple of 32 up to 128, ``dv`` of
     16), go in chunks of 64 tokens on the matrix cores, fp32 operands as three bf16 parts that add up to them; else token by
     token.  ``mode`` 1 / 2 force the one-launch / two-launch
-    scan, 3 the chunks (tests)."""
+    scan, 3 the chunks, 4 the chunks in spans where decays are per channel (tests)."""
     T = qkv.shape[0]
     nz = z_bias.numel()
     dkind = 0 if a_log is not None else 2 if decay == "exp_exp" else 1

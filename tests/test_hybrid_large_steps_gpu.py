@@ -417,3 +417,24 @@ def test_gated_unit_in_the_projection(M, f, rest, K, kind):
     a, y, col = hops.linear_glu(x, w, f, kind)
     proj = hops.linear(x, w)
     assert torch.equal(a, hops.glu(proj, 0, f, kind)) and torch.equal(y[:, col:col + rest], proj[:, 2 * f:])
+
+
+@pytest.mark.parametrize("H,dk,dv", [(4, 64, 64), (2, 32, 48), (2, 128, 32)])
+@pytest.mark.parametrize("kind", ["bonus", "root"])
+def test_chunked_channel_decays_in_spans(H, dk, dv, kind):
+    """Decays per key channel with segments cut into spans of chunks (256 tokens here): segments around the span and the chunk,
+    continued ones, a padding one, one of several spans beside single rows.  Tolerance as for whole segments: 2e-5."""
+    g = _g(79)
+    lens = [1, 256, 257, 700, 300, 64, 512, 1]
+    cu, ctx, slot = _segments(lens, [4, 5, 0, 64, 3, 0, 9, 1], [0, 1, 2, 3, -1, 4, 5, 6])
+    T = sum(lens)
+    qkv, z, zb, state = _r(g, T, 2 * H * dk + H * dv, dt=BF), _r(g, T, H * dk, s=2.0, dt=BF), _r(g, H * dk, s=2.0), _r(g, 7, H, dv, dk)
+    kw = dict(decay="exp_exp", bonus=_r(g, H, dk)) if kind == "bonus" else dict(tau=3.0)
+    zb += -3.0 if kind == "bonus" else 3.0
+    want_s, got_s = state.clone(), state.cuda()
+    a = (0, H * dk, 2 * H * dk)
+    want = hops.decay_scan(qkv, *a, z, zb, want_s, cu, ctx, slot, H, H, dk, dv, dk ** -0.5, **kw)
+    dev = {k: v.cuda() if isinstance(v, torch.Tensor) else v for k, v in kw.items()}
+    got = hops.decay_scan(qkv.cuda(), *a, z.cuda(), zb.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), H, H, dk, dv, dk ** -0.5, mode=4, **dev)
+    for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
+        torch.testing.assert_close(x, y, rtol=2e-5, atol=2e-5 * float(y.abs().max()))
