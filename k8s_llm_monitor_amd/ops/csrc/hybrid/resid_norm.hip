@@ -104,7 +104,10 @@ __global__ __launch_bounds__(256) void add_norm_kernel(T* __restrict__ out, floa
   }
 }
 
-template <typename T>
+// NV > 0: groups of up to 256 NV, kept in registers between the sum and the norm with all loads in flight at once; 0: any size, read
+// twice.  A thread's elements and the order of its sum are the same.  8192 rows of one group of 4096, bf16: 76 -> 41
+// us (6.5 TB/s), 64 rows 8.0 -> 4.8; 7600 of 2048 34 -> 24.
+template <typename T, int NV>
 __global__ __launch_bounds__(256) void gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y,
                                                                const T* __restrict__ z, long z_stride,
                                                                const float* __restrict__ w, int n, int groups,
@@ -114,14 +117,43 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(T* __restrict__ o
   const int g = blockIdx.y, gs = n / groups;
   const float* yr = y + row * n + (long)g * gs;
   const T* zr = z + row * z_stride + (long)g * gs;
+  const float* wr = w + (long)g * gs;
+  T* o = out + row * n + (long)g * gs;
   float ss = 0.f;
+  if (NV > 0) {
+    float v[NV > 0 ? NV : 1], t[NV > 0 ? NV : 1];
+    T zq[NV > 0 ? NV : 1];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = min((int)threadIdx.x + 256 * i, gs - 1);
+      v[i] = yr[c];
+      zq[i] = zr[c];
+      t[i] = wr[c];
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if ((int)threadIdx.x + 256 * i < gs) {
+        if (!after) v[i] = v[i] * silu_f(ldf(&zq[i]));
+        ss += v[i] * v[i];
+      }
+    ss = block_sum<256>(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float)gs + eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      if (c < gs) {
+        const float x = v[i] * inv * t[i];
+        stf(o + c, !after ? x : x * (after == 2 ? silu_f(ldf(&zq[i])) : sigmoid_f(ldf(&zq[i]))));
+      }
+    }
+    return;
+  }
   if (after) {  // the norm first, then a sigmoid gate
     for (int c = threadIdx.x; c < gs; c += 256) ss += yr[c] * yr[c];
     ss = block_sum<256>(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float)gs + eps);
     for (int c = threadIdx.x; c < gs; c += 256)
-      stf(out + row * n + (long)g * gs + c,
-          yr[c] * inv * w[(long)g * gs + c] * (after == 2 ? silu_f(ldf(zr + c)) : sigmoid_f(ldf(zr + c))));
+      stf(o + c, yr[c] * inv * wr[c] * (after == 2 ? silu_f(ldf(zr + c)) : sigmoid_f(ldf(zr + c))));
     return;
   }
   for (int c = threadIdx.x; c < gs; c += 256) {
@@ -132,7 +164,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(T* __restrict__ o
   const float inv = 1.0f / sqrtf(ss / (float)gs + eps);
   for (int c = threadIdx.x; c < gs; c += 256) {
     const float v = yr[c] * silu_f(ldf(zr + c));
-    stf(out + row * n + (long)g * gs + c, v * inv * w[(long)g * gs + c]);
+    stf(o + c, v * inv * wr[c]);
   }
 }
 
@@ -797,12 +829,17 @@ int k8sllm_hy_gated_group_norm(void* out, const float* y, const void* z, long z_
 #undef K8SLLM_GW
     return (int)hipGetLastError();
   }
-  if (f32)
-    hipLaunchKernelGGL(gated_group_norm_kernel<float>, dim3(rows, groups), dim3(256), 0, s, (float*)out, y,
-                       (const float*)z, z_stride, w, n, groups, eps, after);
-  else
-    hipLaunchKernelGGL(gated_group_norm_kernel<bf16_t>, dim3(rows, groups), dim3(256), 0, s, (bf16_t*)out, y,
-                       (const bf16_t*)z, z_stride, w, n, groups, eps, after);
+#define K8SLLM_GN(T_, NV)                                                                                            \
+  hipLaunchKernelGGL((gated_group_norm_kernel<T_, NV>), dim3(rows, groups), dim3(256), 0, s, (T_*)out, y, (const T_*)z, z_stride, w, \
+                     n, groups, eps, after)
+#define K8SLLM_GNT(T_)                      \
+  if (gs <= 1024) K8SLLM_GN(T_, 4);         \
+  else if (gs <= 2048) K8SLLM_GN(T_, 8);    \
+  else if (gs <= 4096) K8SLLM_GN(T_, 16);   \
+  else K8SLLM_GN(T_, 0)
+  if (f32) { K8SLLM_GNT(float); } else { K8SLLM_GNT(bf16_t); }
+#undef K8SLLM_GNT
+#undef K8SLLM_GN
   return (int)hipGetLastError();
 }
 

@@ -438,3 +438,16 @@ def test_chunked_channel_decays_in_spans(H, dk, dv, kind):
     got = hops.decay_scan(qkv.cuda(), *a, z.cuda(), zb.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), H, H, dk, dv, dk ** -0.5, mode=4, **dev)
     for x, y in ((got.cpu(), want), (got_s.cpu(), want_s)):
         torch.testing.assert_close(x, y, rtol=2e-5, atol=2e-5 * float(y.abs().max()))
+
+
+@pytest.mark.parametrize("n,groups", [(1, 1), (255, 1), (257, 1), (1024, 1), (1025, 1), (2048, 1), (4096, 2), (4097, 1), (3072, 3)])
+@pytest.mark.parametrize("after,gate", [(False, "silu"), (True, "sigmoid"), (True, "silu")])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_gated_group_norm_sizes(n, groups, after, gate, dt):
+    """Groups around what the kernel keeps in registers (4, 8 and 16 values a thread, more than that from memory).  fp32 inside: 1e-5 of
+    the value, and the rounding of a bf16 result."""
+    g = _g(80)
+    y, z, w = _r(g, 3, n), _r(g, 3, n + 5, dt=dt), _r(g, n)
+    want = hops.gated_group_norm(y, z, 5, w, 1e-5, groups, dt, after=after, gate=gate)
+    got = hops.gated_group_norm(y.cuda(), z.cuda(), 5, w.cuda(), 1e-5, groups, dt, after=after, gate=gate)
+    torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
