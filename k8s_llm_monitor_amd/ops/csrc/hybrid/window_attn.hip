@@ -35,7 +35,10 @@ __device__ __forceinline__ float tanh_exp2(float x) {
   return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * 2.88539008177792681f));
 }
 
-template <typename T>
+// NV > 0: up to 256 NV columns of q and of k, kept in registers between the sums and the norms with all loads in flight at once; 0: any
+// size, read twice.  The order of the sums is the same.  8192 rows of 2048 + 512 + 512 columns, bf16:
+// 44.8 -> 32.2 us, 64 rows 5.8 -> 4.4; 2048 rows of 4096 + 1024 + 1024 25 -> 21.
+template <typename T, int NV>
 __global__ __launch_bounds__(256) void qk_norm_cache_kernel(T* __restrict__ qkv, long stride,
                                                             const float* __restrict__ qw,
                                                             const float* __restrict__ kw, float eps, int nq, int nk,
@@ -44,7 +47,41 @@ __global__ __launch_bounds__(256) void qk_norm_cache_kernel(T* __restrict__ qkv,
   __shared__ float red[4];
   const long t = blockIdx.x;
   T* row = qkv + t * stride;
+  const long slot = (slots != nullptr && k_cache != nullptr) ? slots[t] : -1;
   float sq = 0.f, sk = 0.f;
+  if (NV > 0) {
+    float q[NV > 0 ? NV : 1], kk[NV > 0 ? NV : 1], wq[NV > 0 ? NV : 1], wk[NV > 0 ? NV : 1];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + 256 * i, cq = min(c, nq - 1), ck = min(c, nk - 1);
+      q[i] = ldf(row + cq);
+      wq[i] = qw[cq];
+      if (256 * i < nk) {
+        kk[i] = ldf(row + nq + ck);
+        wk[i] = kw[ck];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      if (c < nq) sq += q[i] * q[i];
+      if (c < nk) sk += kk[i] * kk[i];
+    }
+    sq = block_sum<256>(sq, red);
+    sk = block_sum<256>(sk, red);
+    const float iq = 1.0f / sqrtf(sq / (float)nq + eps), ik = 1.0f / sqrtf(sk / (float)nk + eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      if (c < nq) stf(row + c, q[i] * iq * wq[i]);
+      if (c < nk) {
+        T kr;
+        stf(&kr, kk[i] * ik * wk[i]);
+        row[nq + c] = kr;
+        if (slot >= 0) k_cache[slot * nk + c] = kr;
+      }
+    }
+  } else {
   for (int c = threadIdx.x; c < nq; c += 256) {
     const float x = ldf(row + c);
     sq += x * x;
@@ -56,11 +93,11 @@ __global__ __launch_bounds__(256) void qk_norm_cache_kernel(T* __restrict__ qkv,
   sq = block_sum<256>(sq, red);
   sk = block_sum<256>(sk, red);
   const float iq = 1.0f / sqrtf(sq / (float)nq + eps), ik = 1.0f / sqrtf(sk / (float)nk + eps);
-  const long slot = (slots != nullptr && k_cache != nullptr) ? slots[t] : -1;
   for (int c = threadIdx.x; c < nq; c += 256) stf(row + c, ldf(row + c) * iq * qw[c]);
   for (int c = threadIdx.x; c < nk; c += 256) {
     stf(row + nq + c, ldf(row + nq + c) * ik * kw[c]);
     if (slot >= 0) k_cache[slot * nk + c] = row[nq + c];
+  }
   }
   if (slot >= 0)
     for (int c = threadIdx.x; c < nv; c += 256) v_cache[((slot / bs) * nv + c) * bs + slot % bs] = row[nq + nk + c];
@@ -792,12 +829,16 @@ int k8sllm_hy_window_f32(void* out, const void* qkv, long q_stride, const void* 
 int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float* kw, float eps, long T, int nq,
                             int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s) {
   if (T <= 0) return 0;
-  if (f32)
-    hipLaunchKernelGGL(qk_norm_cache_kernel<float>, dim3(T), dim3(256), 0, s, (float*)qkv, stride, qw, kw, eps, nq, nk,
-                       nv, (float*)k_cache, (float*)v_cache, slots, bs);
-  else
-    hipLaunchKernelGGL(qk_norm_cache_kernel<bf16_t>, dim3(T), dim3(256), 0, s, (bf16_t*)qkv, stride, qw, kw, eps, nq,
-                       nk, nv, (bf16_t*)k_cache, (bf16_t*)v_cache, slots, bs);
+#define K8SLLM_QK(T_, NV)                                                                                             \
+  hipLaunchKernelGGL((qk_norm_cache_kernel<T_, NV>), dim3(T), dim3(256), 0, s, (T_*)qkv, stride, qw, kw, eps, nq, nk, nv, \
+                     (T_*)k_cache, (T_*)v_cache, slots, bs)
+#define K8SLLM_QKT(T_)                                          \
+  if (nq <= 2048 && nk <= 2048) K8SLLM_QK(T_, 8);               \
+  else if (nq <= 4096 && nk <= 4096) K8SLLM_QK(T_, 16);         \
+  else K8SLLM_QK(T_, 0)
+  if (f32) { K8SLLM_QKT(float); } else { K8SLLM_QKT(bf16_t); }
+#undef K8SLLM_QKT
+#undef K8SLLM_QK
   return (int)hipGetLastError();
 }
 

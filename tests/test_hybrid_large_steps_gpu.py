@@ -451,3 +451,18 @@ def test_gated_group_norm_sizes(n, groups, after, gate, dt):
     want = hops.gated_group_norm(y, z, 5, w, 1e-5, groups, dt, after=after, gate=gate)
     got = hops.gated_group_norm(y.cuda(), z.cuda(), 5, w.cuda(), 1e-5, groups, dt, after=after, gate=gate)
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("Hq,G,dk,dv", [(1, 1, 1, 1), (2, 1, 128, 64), (16, 4, 128, 128), (17, 1, 128, 8), (32, 8, 128, 16), (33, 3, 128, 8)])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_qk_norm_sizes(Hq, G, dk, dv, dt):
+    """Whole-projection norms around what the kernel keeps in registers (8 and 16 columns a thread, more from memory), rows without a
+    slot.  fp32 inside: 1e-5 of the value, and the rounding of bf16 results."""
+    g = _g(81)
+    qkv, qw, kw = _r(g, 5, Hq * dk + G * (dk + dv), dt=dt), _r(g, Hq * dk), _r(g, G * dk)
+    kc, vc, slots = torch.zeros(3, 16, G * dk, dtype=dt), torch.zeros(3, G, dv, 16, dtype=dt), _i32([17, -1, 3, 40, 0])
+    dev = [v.cuda() for v in (qkv, qw, kw, kc, vc, slots)]
+    hops.qk_norm_cache(qkv, qw, kw, 1e-5, Hq, G, dk, dv, kc, vc, slots)
+    hops.qk_norm_cache(dev[0], dev[1], dev[2], 1e-5, Hq, G, dk, dv, dev[3], dev[4], dev[5])
+    for a, b in zip((dev[0], dev[3], dev[4]), (qkv, kc, vc)):
+        torch.testing.assert_close(a.cpu().float(), b.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
