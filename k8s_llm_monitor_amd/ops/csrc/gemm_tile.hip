@@ -41,11 +41,10 @@
 //     `(2t + i) % 5` written inline hipcc emitted ~25 mul-hi / per-read address instructions in
 //     front of every k-tile's first MFMA; removing them made the kernel 4-5 % faster on every
 //     shape (profiles/r03/gemm_ring_addressing.jsonl).
-// Measured against hipBLASLt's own gfx950 256x256x64 kernel (profiles/r06/README.md): the same
-// instruction mix per k-tile (128 MFMA, 32 ds_read_b128, 16 LDS-DMA pieces); ported its schedule
-// (two whole-k-tile buffers, three barriers per k-tile, reads one per two MFMAs, its operand
-// order) and four other row swizzles - all within +-1 % of this kernel, bit-identical, removed;
-// the 5-7 % gap to it is per-tile and independent of the tile-wave count (1, 4, 16).
+// What bounds it: the matrix cores, busy 74.5 % of the time (counters, 16384 x 4096 x 4096), and the issue of 32
+// fragment reads and 16 LDS-DMA pieces beside a k-tile's 128 MFMAs.  The library's product of that shape takes 5 to 7 %
+// less per tile at any number of tiles per CU (1, 4, 16).  Four other row swizzles: 1.6 %
+// faster to 18 % slower, the faster one not at 14336 x 4096; DMA sources in lane order (timing only): the same.
 // Measured and removed (profiles/r03, r05): an 8-wave 128 x 64-per-wave kernel (0.375 reads per MFMA;
 // the round-5 ping-pong form of it, bit-identical, 5-6 % slower), non-temporal residual-epilogue
 // stores (-1.9 % on o in isolation, below what an end-to-end A/B resolves),
