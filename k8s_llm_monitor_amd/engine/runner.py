@@ -21,7 +21,7 @@ import numpy as np
 import torch
 
 from .. import ops
-from ..models.llama import AttnMeta, CausalLM
+from ..models.llama import AttnMeta, CausalLM, PageList
 from .sequence import Sequence
 
 BLOCK_SIZE = 16
@@ -202,15 +202,16 @@ class ModelRunner:
         # layout of the staging buffer (int32 words; the float sampling parameters bit-cast)
         nl = sum(len(x) for x in logit_rows) if logit_rows is not None else R
         hy = R if self.hybrid else 0
-        # latent attention: the chunks' pages in one list, and where each chunk's begin in it
-        npg = [(c + n + BLOCK_SIZE - 1) // BLOCK_SIZE for c, n in zip(starts, lens)] if hy and self.model.lists_pages else []
+        # latent attention: for every window of those layers the pages that the chunks see through it, [first, end) of each
+        seen = {w: [(max(0, c - w + 1) // BLOCK_SIZE if w else 0, (c + n + BLOCK_SIZE - 1) // BLOCK_SIZE) for c, n in zip(starts, lens)]
+                for w in (self.model.page_windows if hy and seqs else ())}
         sizes = dict(ids=T, pos=T, slots=T, cu=len(seqs) + 1, qs=nq, st=nq, lidx=nl, temp=R, topk=R, topp=R,
                      gcu=hy + 1 if hy else 0, gctx=hy, gslot=hy,
                      cst=len(seqs) if paged else 0, bt=len(seqs) * W, dbt=nd * Wd, dlen=nd,
                      mcu=len(seqs) + 2 if kA else 0, mqs=nq if kA else 0, mst=nq if kA else 0,
                      mlidx=len(seqs) if kA else 0)
-        if npg:
-            sizes.update(pgl=sum(npg), pgb=len(npg) * W)
+        for w, ab in seen.items():
+            sizes.update({f"pgl{w}": sum(b - a for a, b in ab), f"pgb{w}": len(ab) * W})
         off, o = {}, 0
         for k, n in sizes.items():
             off[k] = o
@@ -257,10 +258,12 @@ class ModelRunner:
             bt2[:] = 0
             for i, s in enumerate(seqs):
                 bt2[i, : len(s.block_table)] = s.block_table
-            if npg:
-                k, end = np.asarray(npg), np.cumsum(npg)
-                v["pgl"][:] = bt2[np.arange(W) < k[:, None]]
-                v["pgb"][:] = np.minimum((end - k)[:, None] + np.arange(W), end[:, None] - 1).ravel()
+            for w, ab in seen.items():
+                a, b = np.asarray(ab).T[:, :, None]
+                end, col = np.cumsum(b - a)[:, None], np.arange(W)
+                v[f"pgl{w}"][:] = bt2[(col >= a) & (col < b)]
+                # (pages that are not seen get the number of one that is)
+                v[f"pgb{w}"][:] = np.clip(end - b + col, end - b + a, end - 1).ravel()
         if nd:
             dbt = v["dbt"].reshape(nd, Wd)
             dbt[:] = 0
@@ -286,8 +289,8 @@ class ModelRunner:
         if hy:
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = dv["gcu"], dv["gctx"], dv["gslot"]
             meta.seg_max = max([1] * (nd > 0) + lens)
-            if npg:
-                meta.page_list, meta.page_bt = dv["pgl"], dv["pgb"].view(len(seqs), W)
+            meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W),
+                                           np.cumsum([b - a for a, b in ab]).tolist()) for w, ab in seen.items()}
         if kA:
             TA, S_ = int(cu[kA]), len(seqs)
             parts = []

@@ -234,14 +234,14 @@ class LatentAttention:
     Two forms of the same attention.  Over the cache the per-head expansions are moved to the query
     side (module docstring): every step can take it.  The prompt rows of a step with at least ``EXPAND_MIN_ROWS`` of them
     (bf16, head sizes of the matrix-core kernels) instead expand the keys ``[W_uk c | shared part]`` and values
-    ``W_uv c`` of all positions they see per head into temporary pages and run windowed attention's kernel over
+    ``W_uv c`` of all positions they see (the window's) per head into temporary pages and run windowed attention's kernel over
     them: ``dim + rot_dim + vdim`` multiply-adds per (query, key, head) instead of ``2 kv_rank + rot_dim``.  With
     more than ``EXPAND_KEYS`` positions per row the expansion costs more than it saves (16 heads, kv_rank 256, one layer, cache
     form -> expanded, us: 1 x 64 rows 151 -> 85; 1 x 128 behind 4000 tokens 171 -> 155; 16 x 128 behind 4000 1466 -> 569;
-    2 x 2000 behind 2816 1740 -> 200; 16 x 64 behind 4000, 64 positions per row, 428 -> 513)."""
+    2 x 2000 behind 2816 1740 -> 200; 16 x 64 behind 4000, 64 positions per row, 428 -> 513; with a window of 512: 1 x 256 behind 7900
+    155 -> 86, 16 x 64 behind 4000 175 -> 133, 16 x 16 behind 4000, 33 positions per row, 131 -> 112)."""
 
     kind = "latent_attention"
-    lists_pages = True  # its expanded form reads a step's pages as one list (AttnMeta.page_list)
     EXPAND_MIN_ROWS = 64
     EXPAND_KEYS = 32
 
@@ -256,6 +256,7 @@ class LatentAttention:
         self.Q, self.R = int(m["q_rank"]), int(m["kv_rank"])
         self.scale = float(m.get("scale", 1.0 / math.sqrt(self.dn + self.dr)))
         self.window = int(m.get("mask.size", 0) or 0)
+        self.page_windows = (self.window,)  # its expanded form reads the pages that a step sees as one list (AttnMeta.page_lists)
         self.base, self.rdims = float(m.get("rot.base", 10000.0)), int(m.get("rot.dims", self.dr))
         if self.rdims % 2 or self.rdims > self.dr:
             raise ValueError(f"{prefix}: rot.dims {self.rdims} must be even and at most rot_dim {self.dr}")
@@ -318,7 +319,7 @@ class LatentAttention:
             n = nd if ex else T
             parts.append(self._forward_latent(q[:n], meta, kc, vc, gate[:n] if gate is not None else None, not ex))
         if ex:
-            parts.append(self._forward_expanded(q[nd:], down[nd:], meta, kc, gate[nd:] if gate is not None else None))
+            parts.append(self._forward_expanded(q[nd:], meta, kc, gate[nd:] if gate is not None else None))
         return hops.linear(parts[0] if len(parts) == 1 else torch.cat(parts), self.wo)
 
     def _forward_latent(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
@@ -352,20 +353,20 @@ class LatentAttention:
 
     def _expand_ok(self, h: torch.Tensor, meta: AttnMeta) -> bool:
         rows = h.shape[0] - meta.num_decode
-        return (meta.is_prefill and meta.page_list is not None and h.is_cuda and h.dtype == torch.bfloat16
+        return (meta.is_prefill and meta.page_lists is not None and h.is_cuda and h.dtype == torch.bfloat16
                 and bool(self.fast) and rows >= self.EXPAND_MIN_ROWS
-                and (meta.all_fresh or meta.page_list.numel() * BLOCK <= self.EXPAND_KEYS * rows)
+                and (meta.all_fresh or meta.page_lists[self.window].ends[-1] * BLOCK <= self.EXPAND_KEYS * rows)
                 and (self.dn + self.dr) in (64, 128) and self.dv in (64, 128))
 
-    def _forward_expanded(self, q: torch.Tensor, down: torch.Tensor, meta: AttnMeta, kc: torch.Tensor,
-                          gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def _forward_expanded(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Prompt rows: per-head keys and values of every position they see in temporary pages, windowed
         attention's matrix-core kernel over them.  ``q`` [rows, H * (dim + rot_dim)] still unturned."""
         H, dn, dr, dv = self.H, self.dn, self.dr, self.dv
         nd = meta.num_decode
-        kt, vt = hops.latent_expand(kc, meta.page_list, self.w_uk, self.w_uv, H, self.R, dr)
+        seen = meta.page_lists[self.window]
+        kt, vt = hops.latent_expand(kc, seen.pages, self.w_uk, self.w_uv, H, self.R, dr)
         hops.rotate_heads(q, H, dn + dr, meta.positions[nd:], self.freq, self.pairs, dn)
-        return hops.window_attention_prefill(q, kt, vt, meta.cu_seqlens, meta.ctx_start, meta.page_bt, H, H, dn + dr, dv, self.scale,
+        return hops.window_attention_prefill(q, kt, vt, meta.cu_seqlens, meta.ctx_start, seen.tables, H, H, dn + dr, dv, self.scale,
                                              self.window, self.sink, mfma=self.fast, sinks=self.sinks, gate=gate)
 
 
@@ -830,7 +831,7 @@ class SideBySide:
         self.out_w = None if self.mix is None else tuple(p.get(f"{prefix}{side}.out", (d,), 0.1, 1.0, small=True)
                                                          for side in ("left", "right"))
         self.stateful = any(getattr(x, "stateful", False) for x in self.subs)
-        self.lists_pages = any(getattr(x, "lists_pages", False) for x in self.subs)
+        self.page_windows = tuple(w for x in self.subs for w in getattr(x, "page_windows", ()))
         # each mixer's rows padded with zeros to a multiple of 8: the kernels' 16-byte accesses need aligned
         # row strides and first columns
         parts, self.cols = [], []
@@ -1233,7 +1234,7 @@ class HybridLM:
             self.kv_run.append(prev[-1])
         self.unused = sorted(set(weights.keys()) - p.used) if weights is not None else []
         self.has_state = self.shifted or any(getattr(m, "stateful", False) for m in self.mixers)
-        self.lists_pages = any(getattr(m, "lists_pages", False) for m in self.mixers)
+        self.page_windows = sorted({w for m in self.mixers for w in getattr(m, "page_windows", ())})
         # large steps of such layers run on the Mixtral path's tile GEMM (extension _k8sllm_ops)
         self.uses_tile_gemm = any(f is not None and (getattr(f, "il", False) or getattr(f, "tile", False))
                                   for f in self.ffns)

@@ -32,7 +32,7 @@ import hashlib
 import math
 import os
 from dataclasses import dataclass
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 import torch.nn.functional as F
@@ -43,6 +43,14 @@ from ..parallel.comm import (kv_head_range, shard_range, tp_all_gather_last, tp_
                              tp_all_reduce_async, tp_all_to_all)
 from ..parallel.state import ParallelState, get_state
 from .config import ModelConfig
+
+
+class PageList(NamedTuple):
+    """The cache pages that the chunks of a prefill step see through one attention window, chunk after chunk."""
+
+    pages: torch.Tensor  # [n] int32
+    tables: torch.Tensor  # [S, W] int32: a chunk's page of each position as its number in the list
+    ends: list  # [S]: pages up to and with each chunk's
 
 
 @dataclass
@@ -83,10 +91,8 @@ class AttnMeta:
     seg_max: int = 0  # rows of the longest segment (0: not known)
     # prefill: every chunk of this step starts at position 0 (whole prompts, nothing cached before)
     all_fresh: bool = False
-    # layer-list prefill: the pages of every chunk's sequence up to its last token of this step, sequence after
-    # sequence [n], and per chunk the numbers of its pages in that list [S, W] (latent attention's expanded form)
-    page_list: Optional[torch.Tensor] = None
-    page_bt: Optional[torch.Tensor] = None
+    # layer-list prefill, latent attention's expanded form: a PageList for each attention window of those layers (0: none)
+    page_lists: Optional[dict] = None
 
 
 def _seed_for(name: str, seed: int) -> int:

@@ -206,6 +206,32 @@ def test_whole_prompts_in_the_expanded_form(monkeypatch):
     close(torch.cat([a["b"], b["b"]]), wu)
 
 
+def test_expanded_portions_see_no_more_pages_than_their_windows(monkeypatch):
+    """Portions far into two prompts in the expanded form, beside a decode row: each layer expands the pages that its window
+    leaves visible (rows + window - 1 positions, at most one page more than they fill) and no others."""
+    from k8s_llm_monitor_amd.models.hybrid import LatentAttention
+
+    pages = []
+    real = hops.latent_expand
+    monkeypatch.setattr(hops, "latent_expand", lambda kc, pl, *a: pages.append(pl.numel()) or real(kc, pl, *a))
+    monkeypatch.setattr(LatentAttention, "_expand_ok", lambda self, h, meta: meta.is_prefill)
+    rig = rig_for(FULL, 6)
+    V = FULL["vocab"]
+    t, u, v = toks(230, V, 4), toks(150, V, 5), toks(9, V, 6)
+    wt, wu, wv = (O.forward(FULL, rig.w, x) for x in (t, u, v))
+    a = rig.step([("a", t[:200]), ("b", u[:3]), ("c", v[:8])])
+    pages.clear()
+    b = rig.step([("c", v[8:]), ("a", t[200:]), ("b", u[3:20])], end=["c"])
+    windows = [l["mixer"]["mask"]["size"] for l in FULL["layers"]]
+    assert len(pages) == len(windows)
+    for n, w in zip(pages, windows):
+        assert n == -(-230 // 16) - (200 - w + 1) // 16 + 2
+    c = rig.step([("b", u[20:])], end=["b"])
+    close(torch.cat([a["a"], b["a"]]), wt)
+    close(torch.cat([a["b"], b["b"], c["b"]]), wu)
+    close(torch.cat([a["c"], b["c"]]), wv)
+
+
 def test_first_tokens_and_single_token_prompt():
     rig = rig_for(FULL, 7)
     for n in (1, 2, 3):
