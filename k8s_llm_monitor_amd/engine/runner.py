@@ -290,7 +290,8 @@ class ModelRunner:
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = dv["gcu"], dv["gctx"], dv["gslot"]
             meta.seg_max = max([1] * (nd > 0) + lens)
             meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W),
-                                           np.cumsum([b - a for a, b in ab]).tolist()) for w, ab in seen.items()}
+                                           np.cumsum([b - a for a, b in ab]).tolist(), max(b - a for a, b in ab))
+                               for w, ab in seen.items()}
         if kA:
             TA, S_ = int(cu[kA]), len(seqs)
             parts = []

@@ -73,7 +73,7 @@ from .. import ops as _ops
 from ..ops import hybrid as hops
 from ..parallel.state import ParallelState, get_state
 from .config import DenseSpec, HybridConfig, LayerSpec, MoESpec
-from .llama import AttnMeta
+from .llama import AttnMeta, PageList
 
 BLOCK = 16  # tokens per cache page (engine/runner.BLOCK_SIZE)
 
@@ -239,7 +239,11 @@ class LatentAttention:
     more than ``EXPAND_KEYS`` positions per row the expansion costs more than it saves (16 heads, kv_rank 256, one layer, cache
     form -> expanded, us: 1 x 64 rows 151 -> 85; 1 x 128 behind 4000 tokens 171 -> 155; 16 x 128 behind 4000 1466 -> 569;
     2 x 2000 behind 2816 1740 -> 200; 16 x 64 behind 4000, 64 positions per row, 428 -> 513; with a window of 512: 1 x 256 behind 7900
-    155 -> 86, 16 x 64 behind 4000 175 -> 133, 16 x 16 behind 4000, 33 positions per row, 131 -> 112)."""
+    155 -> 86, 16 x 64 behind 4000 175 -> 133, 16 x 16 behind 4000, 33 positions per row, 131 -> 112).  With few rows and heads the
+    expanded form's time is its longest sequence's, walked by a workgroup a head, and the other form's that of its launches: more than
+    128 rows take the expanded form up to ``1024 + 1.5 rows heads`` positions (8 heads: 1 x 256 behind 4000 157 / 166, behind 7600
+    168 / 256; 1 x 512 behind 7600 241 / 263, behind 4000 183 / 173; 4 x 256 behind 7600 395 / 295; 16 heads: 1 x 256 behind 7600
+    248 / 284; 1 x 512 392 / 296)."""
 
     kind = "latent_attention"
     EXPAND_MIN_ROWS = 64
@@ -355,8 +359,12 @@ class LatentAttention:
         rows = h.shape[0] - meta.num_decode
         return (meta.is_prefill and meta.page_lists is not None and h.is_cuda and h.dtype == torch.bfloat16
                 and bool(self.fast) and rows >= self.EXPAND_MIN_ROWS
-                and (meta.all_fresh or meta.page_lists[self.window].ends[-1] * BLOCK <= self.EXPAND_KEYS * rows)
-                and (self.dn + self.dr) in (64, 128) and self.dv in (64, 128))
+                and (self.dn + self.dr) in (64, 128) and self.dv in (64, 128)
+                and (meta.all_fresh or self._expand_pays(rows, meta.page_lists[self.window])))
+
+    def _expand_pays(self, rows: int, seen: PageList) -> bool:
+        return seen.ends[-1] * BLOCK <= self.EXPAND_KEYS * rows and (rows <= 128 or
+                                                                      seen.longest * BLOCK <= 1024 + 1.5 * rows * self.H)
 
     def _forward_expanded(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Prompt rows: per-head keys and values of every position they see in temporary pages, windowed

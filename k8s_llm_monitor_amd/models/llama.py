@@ -51,6 +51,7 @@ class PageList(NamedTuple):
     pages: torch.Tensor  # [n] int32
     tables: torch.Tensor  # [S, W] int32: a chunk's page of each position as its number in the list
     ends: list  # [S]: pages up to and with each chunk's
+    longest: int  # most pages of a chunk
 
 
 @dataclass

@@ -232,6 +232,22 @@ def test_expanded_portions_see_no_more_pages_than_their_windows(monkeypatch):
     close(torch.cat([a["c"], b["c"]]), wv)
 
 
+@pytest.mark.parametrize("heads,chunks,want", [
+    (16, [(64, 2064)], True), (16, [(64, 4064)], False), (8, [(128, 4128)], True), (8, [(256, 4256)], False), (8, [(256, 7856)], False),
+    (16, [(256, 4256)], True), (16, [(256, 7856)], False), (8, [(512, 8112)], False), (8, [(512, 4512)], True), (16, [(512, 8112)], True),
+    (8, [(256, 7856)] * 2, False), (8, [(256, 7856)] * 4, True), (16, [(64, 4064)] * 16, False)])
+def test_form_of_latent_portions_by_sizes(heads, chunks, want):
+    """Portions (rows, positions seen) take the expanded form exactly where it was the faster one."""
+    from k8s_llm_monitor_amd.models.hybrid import LatentAttention
+    from k8s_llm_monitor_amd.models.llama import PageList
+
+    m = LatentAttention.__new__(LatentAttention)
+    m.H = heads
+    pages = torch.tensor([(p + 15) // 16 for _, p in chunks])
+    seen = PageList(None, None, pages.cumsum(0).tolist(), int(pages.max()))
+    assert m._expand_pays(sum(n for n, _ in chunks), seen) is want
+
+
 def test_first_tokens_and_single_token_prompt():
     rig = rig_for(FULL, 7)
     for n in (1, 2, 3):
