@@ -233,7 +233,7 @@ def test_expanded_portions_see_no_more_pages_than_their_windows(monkeypatch):
 
 
 @pytest.mark.parametrize("heads,chunks,want", [
-    (16, [(64, 2064)], True), (16, [(64, 4064)], False), (8, [(128, 4128)], True), (8, [(256, 4256)], False), (8, [(256, 7856)], False),
+    (16, [(64, 2048)], True), (16, [(64, 4064)], False), (8, [(128, 4096)], True), (8, [(256, 4256)], False), (8, [(256, 7856)], False),
     (16, [(256, 4256)], True), (16, [(256, 7856)], False), (8, [(512, 8112)], False), (8, [(512, 4512)], True), (16, [(512, 8112)], True),
     (8, [(256, 7856)] * 2, False), (8, [(256, 7856)] * 4, True), (16, [(64, 4064)] * 16, False)])
 def test_form_of_latent_portions_by_sizes(heads, chunks, want):
