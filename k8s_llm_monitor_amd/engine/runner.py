@@ -292,6 +292,7 @@ class ModelRunner:
             meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W),
                                            np.cumsum([b - a for a, b in ab]).tolist(), max(b - a for a, b in ab))
                                for w, ab in seen.items()}
+            meta.row_ends = cu[1:].tolist()
         if kA:
             TA, S_ = int(cu[kA]), len(seqs)
             parts = []

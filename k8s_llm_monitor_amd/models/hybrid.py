@@ -243,11 +243,14 @@ class LatentAttention:
     expanded form's time is its longest sequence's, walked by a workgroup a head, and the other form's that of its launches: more than
     128 rows take the expanded form up to ``1024 + 1.5 rows heads`` positions (8 heads: 1 x 256 behind 4000 157 / 166, behind 7600
     168 / 256; 1 x 512 behind 7600 241 / 263, behind 4000 183 / 173; 4 x 256 behind 7600 395 / 295; 16 heads: 1 x 256 behind 7600
-    248 / 284; 1 x 512 392 / 296)."""
+    248 / 284; 1 x 512 392 / 296).  The temporary pages of a layer take at most ``EXPAND_BYTES``: a step's sequences go in groups of
+    that size, and where one cached sequence alone is larger the step stays on the form over the cache.  (A whole prompt's own
+    rows are expanded whatever they take, as each projection of the step holds them too.)"""
 
     kind = "latent_attention"
     EXPAND_MIN_ROWS = 64
     EXPAND_KEYS = 32
+    EXPAND_BYTES = 1 << 30
 
     def __init__(self, spec: LayerSpec, d: int, eps: float, p: _Params, prefix: str, traits: Optional[dict] = None,
                  tail: Optional[torch.Tensor] = None):
@@ -362,9 +365,21 @@ class LatentAttention:
                 and (self.dn + self.dr) in (64, 128) and self.dv in (64, 128)
                 and (meta.all_fresh or self._expand_pays(rows, meta.page_lists[self.window])))
 
+    def _page_bytes(self) -> int:
+        return 2 * BLOCK * self.H * (self.dn + self.dr + self.dv)  # a temporary page's keys and values
+
     def _expand_pays(self, rows: int, seen: PageList) -> bool:
-        return seen.ends[-1] * BLOCK <= self.EXPAND_KEYS * rows and (rows <= 128 or
-                                                                      seen.longest * BLOCK <= 1024 + 1.5 * rows * self.H)
+        return (seen.ends[-1] * BLOCK <= self.EXPAND_KEYS * rows and seen.longest * self._page_bytes() <= self.EXPAND_BYTES
+                and (rows <= 128 or seen.longest * BLOCK <= 1024 + 1.5 * rows * self.H))
+
+    def _expand_groups(self, seen: PageList) -> list:
+        """[first, end) of consecutive chunks whose temporary pages are made together."""
+        most, cuts, held = self.EXPAND_BYTES // self._page_bytes(), [0], 0
+        for i, end in enumerate(seen.ends):
+            if end - held > most and i > cuts[-1]:
+                held = seen.ends[i - 1]
+                cuts.append(i)
+        return list(zip(cuts, cuts[1:] + [len(seen.ends)]))
 
     def _forward_expanded(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Prompt rows: per-head keys and values of every position they see in temporary pages, windowed
@@ -372,10 +387,22 @@ class LatentAttention:
         H, dn, dr, dv = self.H, self.dn, self.dr, self.dv
         nd = meta.num_decode
         seen = meta.page_lists[self.window]
-        kt, vt = hops.latent_expand(kc, seen.pages, self.w_uk, self.w_uv, H, self.R, dr)
         hops.rotate_heads(q, H, dn + dr, meta.positions[nd:], self.freq, self.pairs, dn)
-        return hops.window_attention_prefill(q, kt, vt, meta.cu_seqlens, meta.ctx_start, seen.tables, H, H, dn + dr, dv, self.scale,
-                                             self.window, self.sink, mfma=self.fast, sinks=self.sinks, gate=gate)
+
+        def attend(pages, q, cu, ctx, tables, gate):
+            kt, vt = hops.latent_expand(kc, pages, self.w_uk, self.w_uv, H, self.R, dr)
+            return hops.window_attention_prefill(q, kt, vt, cu, ctx, tables, H, H, dn + dr, dv, self.scale, self.window, self.sink,
+                                                 mfma=self.fast, sinks=self.sinks, gate=gate)
+
+        groups = self._expand_groups(seen)
+        if len(groups) == 1:
+            return attend(seen.pages, q, meta.cu_seqlens, meta.ctx_start, seen.tables, gate)
+        out = []
+        for a, b in groups:  # (one group's pages are given back before the next one's are made)
+            r, p = ([0] + meta.row_ends)[a:b + 1:b - a], ([0] + seen.ends)[a:b + 1:b - a]
+            out.append(attend(seen.pages[p[0]:p[1]], q[r[0]:r[1]], meta.cu_seqlens[a:b + 1] - r[0], meta.ctx_start[a:b],
+                              seen.tables[a:b] - p[0], gate[r[0]:r[1]] if gate is not None else None))
+        return torch.cat(out)
 
 
 class RotaryAttention:

@@ -92,8 +92,10 @@ class AttnMeta:
     seg_max: int = 0  # rows of the longest segment (0: not known)
     # prefill: every chunk of this step starts at position 0 (whole prompts, nothing cached before)
     all_fresh: bool = False
-    # layer-list prefill, latent attention's expanded form: a PageList for each attention window of those layers (0: none)
+    # layer-list prefill, latent attention's expanded form: a PageList for each attention window of those layers (0: none),
+    # and the chunks' ends in rows (cu_seqlens from 1 on) for the host
     page_lists: Optional[dict] = None
+    row_ends: Optional[list] = None
 
 
 def _seed_for(name: str, seed: int) -> int:

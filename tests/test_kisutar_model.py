@@ -242,10 +242,39 @@ def test_form_of_latent_portions_by_sizes(heads, chunks, want):
     from k8s_llm_monitor_amd.models.llama import PageList
 
     m = LatentAttention.__new__(LatentAttention)
-    m.H = heads
+    m.H, m.dn, m.dr, m.dv = heads, 96, 32, 128
     pages = torch.tensor([(p + 15) // 16 for _, p in chunks])
     seen = PageList(None, None, pages.cumsum(0).tolist(), int(pages.max()))
     assert m._expand_pays(sum(n for n, _ in chunks), seen) is want
+
+
+@pytest.mark.parametrize("most", [1, 5, 8, 1000])
+def test_expanded_steps_in_groups_of_bounded_pages(monkeypatch, most):
+    """However few temporary pages a layer may hold at once, a step in the expanded form gives the same results, group by group;
+    only a sequence that is larger alone takes more, and where it is a cached one the step's form is the other one."""
+    from k8s_llm_monitor_amd.models.hybrid import LatentAttention
+
+    made = []
+    real = hops.latent_expand
+    monkeypatch.setattr(hops, "latent_expand", lambda kc, pl, *a: made.append(pl.numel()) or real(kc, pl, *a))
+    monkeypatch.setattr(LatentAttention, "_expand_ok", lambda self, h, meta: meta.is_prefill)
+    cfg = make_cfg([lat(window=500), lat(2, 8, 4, 6, 12, 16, 190, 0.3, mlp=moe())])
+    rig = rig_for(cfg, 6)
+    for m in rig.model.mixers:
+        monkeypatch.setattr(m, "EXPAND_BYTES", most * m._page_bytes() + 1, raising=False)
+    seqs = {n: toks(k, cfg["vocab"], k) for n, k in (("a", 50), ("b", 33), ("c", 70), ("d", 9))}
+    a = rig.step([("a", seqs["a"][:20]), ("b", seqs["b"][:33]), ("c", seqs["c"][:65]), ("d", seqs["d"][:8])], end=["b"])
+    first = list(made)
+    b = rig.step([("d", seqs["d"][8:]), ("c", seqs["c"][65:68]), ("a", seqs["a"][20:])], end=["a", "d"])
+    c = rig.step([("c", seqs["c"][68:])], end=["c"])
+    pages = {1: [2, 3, 5, 1], 5: [5, 5, 1], 8: [5, 6], 1000: [11]}[most]  # of 20, 33, 65 and 8 tokens
+    assert first[:len(pages)] == pages and first[len(pages):] == pages
+    for n, t in seqs.items():
+        close(torch.cat([x[n] for x in (a, b, c) if n in x]), O.forward(cfg, rig.w, t))
+    m = rig.model.mixers[0]
+    from k8s_llm_monitor_amd.models.llama import PageList
+    assert m._expand_pays(64, PageList(None, None, [most], most)) is (most * 16 <= 32 * 64)
+    assert not m._expand_pays(10 ** 6, PageList(None, None, [most + 1], most + 1))
 
 
 def test_first_tokens_and_single_token_prompt():
