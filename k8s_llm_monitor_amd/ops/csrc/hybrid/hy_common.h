@@ -41,6 +41,13 @@ __device__ __forceinline__ void load8_any(const void* p, int dt, long i, float* 
   else load8(reinterpret_cast<const bf16_t*>(p) + i, f);
 }
 
+// Eight 16-bit values of tokens j .. j + 7, zero where not (j < end): what lies behind a sequence's last token in its last page is
+// another sequence's, and a weight of zero does not take away a NaN
+__device__ __forceinline__ uint32_t pair_below(int j, int end) { return j + 1 < end ? ~0u : j < end ? 0xffffu : 0u; }
+__device__ __forceinline__ uint4 tokens_below(uint4 v, int j, int end) {
+  return make_uint4(v.x & pair_below(j, end), v.y & pair_below(j + 2, end), v.z & pair_below(j + 4, end), v.w & pair_below(j + 6, end));
+}
+
 // Wave-wide butterflies without the LDS crossbar: quads and rows by DPP (quad_perm, the row's mirror
 // controls pair equal partial results), rows 0/1 and 2/3 by v_permlane16_swap, the halves by
 // v_permlane32_swap.  Every lane ends with the result.

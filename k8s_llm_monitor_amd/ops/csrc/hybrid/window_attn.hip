@@ -325,6 +325,10 @@ __global__ __launch_bounds__(64 * NW) void window_decode_vec_kernel(bf16_t* __re
 #pragma unroll
         for (int c = 0; c < kMaxVC; ++c)
           if (lane + 64 * c < dv) {
+            if (j0 + 16 * pg + 16 > n) {  // the last page's unused end (uniform)
+              vq[pg][c][0] = tokens_below(vq[pg][c][0], j0 + 16 * pg, n);
+              vq[pg][c][1] = tokens_below(vq[pg][c][1], j0 + 16 * pg + 8, n);
+            }
             float vv[16];
             unpack8(vq[pg][c][0], vv);
             unpack8(vq[pg][c][1], vv + 8);
@@ -563,6 +567,10 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
         for (int r = 0; r < R; ++r) pr[r] = p_s[wave][r][16 * pg + (lane & 15)];
 #pragma unroll
         for (int c = 0; c < VC; ++c) {
+          if (j0 + 16 * pg + 16 > n) {  // the last page's unused end (uniform)
+            vq[pg][c][0] = tokens_below(vq[pg][c][0], j0 + 16 * pg, n);
+            vq[pg][c][1] = tokens_below(vq[pg][c][1], j0 + 16 * pg + 8, n);
+          }
           float vv[16];
           unpack8(vq[pg][c][0], vv);
           unpack8(vq[pg][c][1], vv + 8);
@@ -723,6 +731,15 @@ __global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
     if (j1 < hi) {
       issue(j1);
       pg_n = bt[min(next_tile(j1), hi - 1) >> 4];
+    }
+    if (j0 + 16 > hi) {  // the last page's unused end (wave-uniform)
+      const int j = j0 + 4 * quad;
+      const uint32_t ma = pair_below(j, hi), mb = pair_below(j + 2, hi);
+#pragma unroll
+      for (int dt = 0; dt < DV / 16; ++dt) {
+        const uint2 v = __builtin_bit_cast(uint2, vf[dt]);
+        vf[dt] = __builtin_bit_cast(s16x4, make_uint2(v.x & ma, v.y & mb));
+      }
     }
     s16x4 pb[QT];
     float alpha[QT];

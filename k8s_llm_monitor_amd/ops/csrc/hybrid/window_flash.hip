@@ -16,7 +16,9 @@
 //    lane order): K piece ^ row, V piece ^ bit 3 of the dim, so that a read's 16 lanes touch 16 different bank quads;
 //  * the running maximum moves only when a tile's exceeds it by 2^8: weights stay <= 256, exact in fp32 and in their
 //    bf16 rounding; the accumulator is rescaled on such a jump only.  Tiles inside every row's range are not masked,
-//    tiles outside all rows' are not visited, and a wave skips the tiles that none of its rows sees.
+//    tiles outside all rows' are not visited, and a wave skips the tiles that none of its rows sees.  Where a wave's rows see a
+//    tile in part, the 8-token pieces of V^T that none of them sees are read from zeros, and what lies behind the workgroup's last
+//    token (the last page's unused end) is cleared in LDS: a masked weight of zero would not take away a NaN.
 // Measured (us, 128-wide heads, register kernel -> this one): 4 x 2048 rows, 16 query heads on 4 kv heads, window 1024:
 // 201 -> 87 (596 TFLOP/s); 2 x 2000 rows behind 2816 cached ones: 403 -> 145 (861 TFLOP/s); one prompt of 8000: 982 -> 274
 // (957 TFLOP/s); the same in capped chunks of 1024: 122 -> 89 (three transcendental instructions per score bound it).
@@ -46,7 +48,8 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
   constexpr int WPH = 8 / HW, QR = 32 * WPH;
   constexpr int KB = 64 * DK * 2, TILE = KB + 64 * DV * 2;
   constexpr int NP = (DK + DV) / 64;  // 1 KiB copies per wave and tile
-  __shared__ __attribute__((aligned(16))) char smem[kFlashRing * TILE + kFlashIds * 4];
+  constexpr int ZEROS = kFlashRing * TILE + kFlashIds * 4, ZB = (DT - 1) * 1024 + 16;
+  __shared__ __attribute__((aligned(16))) char smem[ZEROS + ZB];
   int* s_blk = reinterpret_cast<int*>(smem + kFlashRing * TILE);
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -103,6 +106,7 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
 
   const int* bt = block_tables + (long)seq * bt_stride;
   const int last_page = (hi - 1) >> 4;
+  for (int i = tid; i < ZB / 4; i += 512) *reinterpret_cast<int*>(smem + ZEROS + 4 * i) = 0;
   for (int i = tid; i < nu * 4; i += 512) s_blk[i] = bt[min(4 * tile_of(i >> 2) + (i & 3), last_page)];
   bf16x8 qf[KS];
   {
@@ -163,9 +167,33 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
     __builtin_amdgcn_s_barrier();  // every wave's pieces of tile u are there, and tile u - 1 has been read
     if (u + 3 < nu) issue(u + 3, (u + 3) % kFlashRing);
     const int k0 = tile_of(u) * 64;
+    if (k0 + 64 > hi) {  // workgroup-uniform: the last tile
+      for (int i = tid; i < 8 * DV; i += 512) {  // pieces of 8 tokens: page i / (2 DV), dim, half
+        const int d = (i >> 1) % DV, half = (i & 1) ^ ((d >> 3) & 1);
+        uint4* p = reinterpret_cast<uint4*>(smem + (u % kFlashRing) * TILE + KB + 16 * i);
+        const int j = k0 + 16 * (i / (2 * DV)) + 8 * half;
+        if (j + 8 > hi) *p = tokens_below(*p, j, hi);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+    }
     if (!any || k0 > pw1 || (k0 + 63 < lo_w && k0 >= keep)) continue;
     const char* kb = smem + (u % kFlashRing) * TILE;
-    const char* vb = kb + KB;
+    int vo[2][2];  // this lane's V^T pieces of a page (dims r32, r32 + 32, ..)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        vo[i][s] = (u % kFlashRing) * TILE + KB + (2 * i + s) * (DV * 32) + (r32 * 2 + (hh ^ ((r32 >> 3) & 1))) * 16;
+    if (k0 + 63 > pw1 || (k0 < lo_w && k0 + 63 >= keep)) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int t0 = k0 + 32 * i + 16 * s + 8 * hh;
+          if (t0 > pw1 || (t0 + 7 < lo_w && t0 >= keep)) vo[i][s] = ZEROS;
+        }
+    }
     f32x16 sa[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -210,10 +238,7 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const int d = 32 * dt + r32;
-          vf[i][s][dt] = *reinterpret_cast<const bf16x8*>(vb + (2 * i + s) * (DV * 32) + (d * 2 + (hh ^ ((d >> 3) & 1))) * 16);
-        }
+        for (int dt = 0; dt < DT; ++dt) vf[i][s][dt] = *reinterpret_cast<const bf16x8*>(smem + vo[i][s] + 1024 * dt);
     __builtin_amdgcn_sched_barrier(0);
     if (CAP != 2) {
       float mq[4];

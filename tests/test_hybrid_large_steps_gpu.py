@@ -466,3 +466,28 @@ def test_qk_norm_sizes(Hq, G, dk, dv, dt):
     hops.qk_norm_cache(dev[0], dev[1], dev[2], 1e-5, Hq, G, dk, dv, dev[3], dev[4], dev[5])
     for a, b in zip((dev[0], dev[3], dev[4]), (qkv, kc, vc)):
         torch.testing.assert_close(a.cpu().float(), b.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dk,dv,Hq,G", [(128, 128, 4, 1), (64, 128, 3, 3), (128, 64, 2, 1), (128, 8, 2, 1)])
+def test_page_ends_that_hold_no_numbers(dk, dv, Hq, G):
+    """NaN behind the last token in a sequence's last page - what an earlier owner of the page may leave - reaches no result of the
+    bf16 kernels: staged and register prefill, decode by row broadcasts and (the last case) by LDS broadcasts."""
+    g = _g(82)
+    new, ctx = [1, 40, 130, 16], [0, 9, 60, 0]
+    lens = [a + b for a, b in zip(ctx, new)]
+    kc, vc, bt = _paged(g, BF, lens, Hq, G, dk, dv)
+    for row, n in zip(bt, lens):
+        for j in range(n, (n + 15) // 16 * 16):
+            vc[row[j // 16].item(), :, :, j % 16] = float("nan")
+            kc[row[j // 16].item(), j % 16] = float("nan")
+    cu = _i32([0] + torch.tensor(new).cumsum(0).tolist())
+    qkv = _r(g, sum(new), Hq * dk + 8, dt=BF)
+    for window, sink, kw in ((0, False, {}), (37, True, dict(keep=3)), (32, False, dict(chunked=True, cap=5.0))):
+        a = (Hq, G, dk, dv, dk ** -0.5, window, sink)
+        want = hops.window_attention_prefill(qkv, kc, vc, cu, _i32(ctx), bt, *a, **kw)
+        for mfma in (256, 16, 32) if dv >= 64 else ():
+            got = hops.window_attention_prefill(*(x.cuda() for x in (qkv, kc, vc, cu, _i32(ctx), bt)), *a, mfma=mfma, **kw)
+            torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2e-2, atol=2e-2)
+        want = hops.window_attention_decode(qkv[:4], kc, vc, bt, _i32(lens), *a, **kw)
+        got = hops.window_attention_decode(*(x.cuda() for x in (qkv[:4].contiguous(), kc, vc, bt, _i32(lens))), *a, **kw)
+        torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2e-2, atol=2e-2)
