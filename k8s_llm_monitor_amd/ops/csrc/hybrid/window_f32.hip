@@ -8,7 +8,9 @@
 //  * The next page's K and V are in flight while one is processed; nothing goes through LDS but the decode merge.
 //  * Decode: 8 waves take every eighth visible page and meet in LDS.
 // Everything is fp32 with the any-size kernel's expf / tanhf.  A key that a query does not see is selected away before the
-// softmax, and value columns past the last visible token (a page's unused end) count as zero.
+// softmax, and value columns past the last visible token (a page's unused end) count as zero.  An infinity or NaN among the
+// values reaches the queries that see its token and no others, as there: a page that only some of a wave's queries see whole is
+// looked through for one, and such values are added one by one (the matrix instruction would multiply them by the others' zeros).
 // Prompts of 2 x 2048 tokens, 16 heads on 4 of 128: 13.9 -> 0.44 ms; 3 prompts of 250 to 400, 8 heads on 2: 490 -> 74 us (host
 // work of the call included); decode of 2 sequences at 2048: 350 -> 30 us, of 8 at 301: 106 -> 14.  Distance to 64 bits 6.3e-7 ->
 // 4.5e-7 (decode 7.1e-7 -> 3.2e-7).
@@ -63,6 +65,7 @@ __global__ __launch_bounds__(DECODE ? 512 : 64, DECODE ? 1 : 2) void window_f32_
   }
   const int g = h / R, hi = DECODE ? p + 1 : p0 + n;  // no column sees a position from hi on
   const int lo = first_key_f32(p, window, chunked);
+  const int lo_last = DECODE ? lo : first_key_f32(p0 + n - 1, window, chunked);  // from here to p0: keys that every column sees
   // pages: the kept ones, then those from the first column's window on
   const int w_first = first_key_f32(p0, window, chunked) >> 4, k_end = (keep + 15) >> 4;
   const int t_end = (hi + 15) >> 4, gap_from = keep > 0 ? k_end : 0, gap_to = max(w_first, gap_from);
@@ -134,6 +137,35 @@ __global__ __launch_bounds__(DECODE ? 512 : 64, DECODE ? 1 : 2) void window_f32_
     }
 #pragma unroll
     for (int u = 0; u < VG; ++u) o[u] *= alpha;
+    const int k0 = page_of(i) * 16;
+    if (k0 + 15 > p0 || (k0 < lo_last && k0 + 15 >= keep)) {  // wave-uniform
+      float z = 0.f;  // NaN if any value is no number
+#pragma unroll
+      for (int u = 0; u < VG; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) z = fmaf(v[u][j], 0.f, z);
+      if (__any(z != z)) {
+#pragma unroll 1
+        for (int a = 0; a < 4; ++a)  // tokens k0 + 4 a + j
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int kk = k0 + 4 * a + j;
+            const float w = __shfl(s[j], 16 * a + col);
+            const bool seen = kk <= p && (kk >= lo || kk < keep);
+#pragma unroll
+            for (int u = 0; u < VG; ++u)
+#pragma unroll
+              for (int d = 0; d < 4; ++d) {
+                const float x = __shfl(v[u][j], 16 * a + 4 * qt + d);
+                if (seen && !isfinite(x)) o[u][d] = fmaf(w, x, o[u][d]);
+              }
+          }
+#pragma unroll
+        for (int u = 0; u < VG; ++u)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[u][j] = isfinite(v[u][j]) ? v[u][j] : 0.f;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll

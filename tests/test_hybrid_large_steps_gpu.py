@@ -491,3 +491,34 @@ def test_page_ends_that_hold_no_numbers(dk, dv, Hq, G):
         want = hops.window_attention_decode(qkv[:4], kc, vc, bt, _i32(lens), *a, **kw)
         got = hops.window_attention_decode(*(x.cuda() for x in (qkv[:4].contiguous(), kc, vc, bt, _i32(lens))), *a, **kw)
         torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("t", [20, 35, 36, 59])
+@pytest.mark.parametrize("kw", [dict(window=0, sink=False), dict(window=9, sink=True), dict(window=10, sink=False, keep=24),
+                                dict(window=16, sink=False, chunked=True)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_fp32_values_that_are_no_numbers(t, kw, bad):
+    """fp32 attention: a value of one head that is no number reaches the rows that see its token, in its column, and no others; all
+    other results are those of the same step without it, bit for bit."""
+    g = _g(83)
+    kw = dict(kw)
+    G, dk, dv, n, ctx = 2, 64, 64, 40, 20
+    kc, vc, bt = _paged(g, torch.float32, [n + ctx], 4, G, dk, dv)
+    a = (4, G, dk, dv, dk ** -0.5, kw.pop("window"), kw.pop("sink"))
+    q = _r(g, n, 4 * dk).cuda()
+    dev = (_i32([0, n]).cuda(), _i32([ctx]).cuda(), bt.cuda())
+    v2 = vc.clone()
+    v2[bt[0, t // 16].item(), 1, 5, t % 16] = bad
+    p = torch.arange(ctx, ctx + n)
+    lo = p - p % a[5] if kw.get("chunked") else (p - a[5] + 1 if a[5] else 0 * p)
+    seen = (t <= p) & ((t >= lo) | (t < kw.get("keep", 0)))
+    hit = torch.zeros(n, 4, dv, dtype=torch.bool)
+    hit[seen, 2:, 5] = True
+    want = hops.window_attention_prefill(q, kc.cuda(), vc.cuda(), *dev, *a, **kw).cpu().view(n, 4, dv)
+    got = hops.window_attention_prefill(q, kc.cuda(), v2.cuda(), *dev, *a, **kw).cpu().view(n, 4, dv)
+    assert torch.equal(got[~hit], want[~hit]) and not bool(torch.isfinite(got[hit]).any())
+    for i in (0, 15, 16, 39):  # each row as a decode step
+        sl = _i32([ctx + i + 1]).cuda()
+        want = hops.window_attention_decode(q[i:i + 1], kc.cuda(), vc.cuda(), dev[2], sl, *a, **kw).cpu().view(4, dv)
+        got = hops.window_attention_decode(q[i:i + 1], kc.cuda(), v2.cuda(), dev[2], sl, *a, **kw).cpu().view(4, dv)
+        assert torch.equal(got[~hit[i]], want[~hit[i]]) and not bool(torch.isfinite(got[hit[i]]).any())
