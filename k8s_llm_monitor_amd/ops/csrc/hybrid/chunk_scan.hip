@@ -23,11 +23,12 @@
 // Measured, bf16, 16 heads of 128 x 128: 5 x 1600 rows 125 us (the sequential scan 569; chunks whose fp32 products ran on the
 // fp32 matrix instruction 296), 1 x 8000 rows 403 us (2680; 1400).  Error against 64 bits, 1600 rows: outputs 1.4e-7 (scan
 // 2.2e-7), state 1.3e-7 (2.2e-7).
+#include "chunk_seg.h"
 #include "split_bf16.h"
 
 namespace k8sllm {
 
-constexpr int kCsChunk = 64;
+constexpr int kCsChunk = kChunk;
 
 template <int KS, int NT>  // key dim / 32, value columns / 16 per workgroup
 __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ y, const bf16_t* __restrict__ vkq,
@@ -43,6 +44,7 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
   __shared__ __attribute__((aligned(16))) bf16_t Vl[4][kCsChunk * PV];  // values, then the decayed values' three parts
   __shared__ __attribute__((aligned(16))) bf16_t Sl[3][NV * PK];        // the state before the chunk, [column][key dim]
   __shared__ float lam[kCsChunk + 1];                                   // the decay's powers
+  __shared__ __attribute__((aligned(16))) int first[NV];                // chunk_seg.h: rows from which a column is no number
   // workgroups go round the eight XCDs: all column blocks of a (segment, head) pair on one, whose L2 then serves their
   // common keys and queries
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
@@ -62,6 +64,7 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
   const bf16_t* vcol = vkq + (long)h * dv + dvb;
   const bf16_t* kcol = vkq + inner + (long)h * DK;
   const bf16_t* qcol = kcol + (long)H * DK;
+  if (tid < NV) first[tid] = kNone;
   if (tid <= kCsChunk) lam[tid] = tid == 0 ? 1.f : powf(decay[h], (float)tid);
   // state tile (r, ct): S[16 (w RTW + r) + 4 quad + i][16 ct + c16]
   f32x4 S[RTW][NT];
@@ -126,6 +129,7 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
         else if constexpr (VPT == 4) *reinterpret_cast<uint2*>(d) = make_uint2(x[0], x[1]);
         else *reinterpret_cast<uint4*>(d) = make_uint4(x[0], x[1], x[2], x[3]);
       };
+      keep_finite<VPT>(rv, vr, n, first + vc);  // (the state takes its values as they are)
       put(&Vl[0][o], rv);
 #pragma unroll
       for (int k = 0; k < 3; ++k) put(&Vl[k + 1][o], p[k]);
@@ -213,6 +217,14 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
             for (int k = 2; k >= 0; --k) o[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, frag(pw[k]), o[ct], 0, 0, 0);
           }
         }
+      }
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct) {
+        const int4 f = *reinterpret_cast<const int4*>(&first[16 * ct + 4 * quad]);
+        if (qi >= f.x) o[ct][0] = NAN;
+        if (qi >= f.y) o[ct][1] = NAN;
+        if (qi >= f.z) o[ct][2] = NAN;
+        if (qi >= f.w) o[ct][3] = NAN;
       }
       if (qi < n) {
         float* yr = y + (long)(tb + qi) * inner + (long)h * dv + dvb + 4 * quad;

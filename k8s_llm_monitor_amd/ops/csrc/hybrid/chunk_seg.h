@@ -7,6 +7,34 @@ namespace k8sllm {
 
 constexpr int kChunk = 64;
 
+// The chunked recurrences multiply the values of a chunk by weights that are zero for the tokens in front of them.  So that an
+// infinity or NaN reaches no earlier token, as token by token, such a value is staged as zero, the first row at which it stood in a
+// column is kept (kNone: there was none), and the column's results are NaN from that row on, its state with them.
+constexpr int kNone = kChunk;
+__device__ __forceinline__ bool odd_bf16(uint32_t x) { return (x & 0x7f80u) == 0x7f80u; }  // infinity or NaN
+__device__ __forceinline__ bool odd_pair(uint32_t w) { return odd_bf16(w) || odd_bf16(w >> 16); }
+// stages VW bf16 values of row `row` of n (words w) as above; first: their columns' first rows
+template <int VW>
+__device__ __forceinline__ void keep_finite(uint32_t (&w)[VW / 2], int row, int n, int* first) {
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < VW / 2; ++i) any |= odd_pair(w[i]);
+  if (!any) return;
+#pragma unroll
+  for (int i = 0; i < VW; ++i)
+    if (odd_bf16(w[i / 2] >> (16 * (i & 1)))) {
+      w[i / 2] &= i & 1 ? 0x0000ffffu : 0xffff0000u;
+      if (row < n) atomicMin(first + i, row);
+    }
+}
+
+// log2 of a decay from its logit (kinds of decay_scan.hip); 2^-4096 is zero in fp32, and a NaN stays one
+__device__ __forceinline__ float log2_decay(float x, int kind, float A, float inv_tau) {
+  const float e = kind == 0 ? A * softplus_f(x) : kind == 1 ? softplus_f(-x) * inv_tau : expf(x);
+  const float l = -1.44269504088896341f * e;
+  return l < -4096.f ? -4096.f : l;
+}
+
 struct ChunkAt {
   int seg, row, n;  // segment (-1: no such chunk), first row of the step, rows
   int k, count;     // the chunk's number within its segment, the segment's chunks

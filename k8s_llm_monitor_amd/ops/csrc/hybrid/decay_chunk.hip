@@ -29,11 +29,6 @@ namespace k8sllm {
 // bf16 elements of Q', M and N of one (chunk, head) in the workspace
 __host__ __device__ constexpr long kc_mats(int dk) { return 3L * 64 * (64 + 2 * dk); }
 
-__device__ __forceinline__ float log2_channel_decay(float x, int kind, float A, float inv_tau) {
-  const float e = kind == 0 ? A * softplus_f(x) : kind == 1 ? softplus_f(-x) * inv_tau : expf(x);
-  return fmaxf(-1.44269504088896341f * e, -4096.f);  // 2^-4096 is zero in fp32
-}
-
 template <int KS, bool BONUS>
 __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restrict__ mats, float* __restrict__ ends,
                                                                const bf16_t* __restrict__ qkv, long stride, int q_col,
@@ -82,7 +77,7 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
       const int t = QT * tq + i;
-      x[i] = t < n ? log2_channel_decay(bf2f(zr[i]) + zb, dkind, A, inv_tau) : 0.f;
+      x[i] = t < n ? log2_decay(bf2f(zr[i]) + zb, dkind, A, inv_tau) : 0.f;
       Gl[t * DK + c] = __builtin_amdgcn_exp2f(x[i]);
       run += (double)x[i];
     }
@@ -269,6 +264,7 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
   constexpr int DK = 32 * KS, PK = DK + 8, NV = 16 * NT, PV = NV + 8, RTW = (2 * KS + 3) / 4;
   __shared__ __attribute__((aligned(16))) bf16_t Sl[2][3][NV * PK];  // the state before a chunk, [column][channel]
   __shared__ __attribute__((aligned(16))) bf16_t Vl[2][kChunk * PV];
+  __shared__ __attribute__((aligned(16))) int first[2][NV];  // chunk_seg.h: rows from which a column is no number
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
   if (pair >= (MODE == kWhole ? S_ : n_span) * H) return;
   // from the last segment on: a step's prompts come after its running sequences, and their chains take longest
@@ -395,14 +391,17 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
       rv[0] = t.x, rv[1] = t.y, rv[2] = t.z, rv[3] = t.w;
     }
   };
-  auto stage_v = [&](int buf) {
+  auto stage_v = [&](int buf, int n) {
+    keep_finite<VW>(rv, vr, n, first[buf] + vc);
 #pragma unroll
     for (int i = 0; i < VW / 2; ++i) *reinterpret_cast<uint32_t*>(&Vl[buf][vr * PV + vc + 2 * i]) = rv[i];
   };
   fetch_v(t0);
   fetch(t0);
+  if (tid < 2 * NV) first[tid / NV][tid % NV] = kNone;
+  lds_barrier();
   publish(0);
-  stage_v(0);
+  stage_v(0, min(kChunk, t1 - t0));
   if (t0 + kChunk < t1) fetch_v(t0 + kChunk);
   int buf = 0;
   for (int tb = t0; tb < t1; tb += kChunk, buf ^= 1) {
@@ -414,7 +413,7 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
     if (tb + kChunk < t1) fetch(tb + kChunk);
     lds_barrier();  // this chunk's state and values are written; the other buffers have been read
     if (tb + kChunk < t1) {
-      stage_v(buf ^ 1);
+      stage_v(buf ^ 1, min(kChunk, t1 - tb - kChunk));
       if (tb + 2 * kChunk < t1) fetch_v(tb + 2 * kChunk);
     }
     if (outs) {
@@ -437,10 +436,12 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
 #pragma unroll
             for (int m = 2; m >= 0; --m) d[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, mf[3 * KS + 3 * ks + m], d[m], 0, 0, 0);
           }
-          if (16 * w + c16 < n)
-            *reinterpret_cast<float4*>(o + (long)(tb + 16 * w + c16) * inner + (long)h * dv + dvb + 16 * ct + 4 * quad) =
-                make_float4((d[2][0] + d[1][0]) + d[0][0], (d[2][1] + d[1][1]) + d[0][1], (d[2][2] + d[1][2]) + d[0][2],
-                            (d[2][3] + d[1][3]) + d[0][3]);
+          const int4 f = *reinterpret_cast<const int4*>(&first[buf][16 * ct + 4 * quad]);
+          const int q = 16 * w + c16;
+          if (q < n)
+            *reinterpret_cast<float4*>(o + (long)(tb + q) * inner + (long)h * dv + dvb + 16 * ct + 4 * quad) =
+                make_float4(q < f.x ? (d[2][0] + d[1][0]) + d[0][0] : NAN, q < f.y ? (d[2][1] + d[1][1]) + d[0][1] : NAN,
+                            q < f.z ? (d[2][2] + d[1][2]) + d[0][2] : NAN, q < f.w ? (d[2][3] + d[1][3]) + d[0][3] : NAN);
         }
       }
     } else if (mine) {
@@ -467,6 +468,12 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
 #pragma unroll
             for (int r = 0; r < RTW; ++r)
               S[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf[6 * r + 3 * ks + m], x, S[r][ct], 0, 0, 0);
+        }
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct)
+        if (first[buf][16 * ct + c16] < kNone) {
+#pragma unroll
+          for (int r = 0; r < RTW; ++r) S[r][ct] = f32x4{NAN, NAN, NAN, NAN};
         }
       publish(buf ^ 1);
     }

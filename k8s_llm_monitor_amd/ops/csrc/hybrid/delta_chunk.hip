@@ -34,12 +34,6 @@ constexpr int kDcP = kChunk + 8;  // LDS pitch of [.][token] rows
 __host__ __device__ constexpr long dc_mats(int dk) { return 3L * 64 * (64 + dk); }
 constexpr long kDcFac = 132;
 
-// log2 of a decay from its logit (kinds of decay_scan.hip); 2^-4096 is zero in fp32
-__device__ __forceinline__ float log2_decay(float x, int kind, float A, float inv_tau) {
-  const float e = kind == 0 ? A * softplus_f(x) : kind == 1 ? softplus_f(-x) * inv_tau : expf(x);
-  return fmaxf(-1.44269504088896341f * e, -4096.f);
-}
-
 template <int KS>
 __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__ mats, float* __restrict__ fac,
                                                             const bf16_t* __restrict__ qkv, long stride, int q_col, int k_col,
@@ -55,6 +49,7 @@ __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__
   __shared__ __attribute__((aligned(16))) bf16_t Pl[3][64 * kDcP];  // first A as fp32 [64][PA], then P [query][token]
   __shared__ double Ll[64];
   __shared__ float nk[64], nq[64], bl[64];
+  __shared__ int odd_row;  // the first token whose key, decay or beta is no number: M is NaN from there on (kNone: there is none)
   float* Al = reinterpret_cast<float*>(&Pl[0][0]);
   static_assert(64 * PA * 4 <= 3 * 64 * kDcP * 2, "A fits where P will be");
   const ChunkAt at = chunk_at(cu, S, blockIdx.x);
@@ -70,7 +65,7 @@ __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__
     const int r = tid >> 2, c0 = (tid & 3) * (DK / 4);
     const bf16_t* kr = kb + (long)min(r, n - 1) * stride + c0;
     const bf16_t* qr = qb + (long)min(r, n - 1) * stride + c0;
-    float sk = 0.f, sq = 0.f;
+    float sk = 0.f, sq = 0.f, odd = 0.f;  // odd: NaN if the key has an infinity or a NaN
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
       const uint4 kv = *reinterpret_cast<const uint4*>(kr + 8 * u), qv = *reinterpret_cast<const uint4*>(qr + 8 * u);
@@ -82,12 +77,14 @@ __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__
       for (int i = 0; i < 8; ++i) {
         sk += a[i] * a[i];
         sq += b[i] * b[i];
+        odd = fmaf(a[i], 0.f, odd);
       }
     }
     sk = lanes_sum<4>(sk);
     sq = lanes_sum<4>(sq);
+    odd = lanes_sum<4>(odd);
     if ((tid & 3) == 0) {
-      nk[r] = unit ? 1.0f / sqrtf(sk + 1e-6f) : 1.f;
+      nk[r] = (unit ? 1.0f / sqrtf(sk + 1e-6f) : 1.f) + odd;
       nq[r] = unit ? q_scale / sqrtf(sq + 1e-6f) : q_scale;
     }
   }
@@ -141,6 +138,9 @@ __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__
   __syncthreads();
   float t[64];  // wave 0: column `lane` of T
   if (w == 0) {
+    const float num = nk[lane] + (float)Ll[lane] + bl[lane];
+    const unsigned long long odd = __ballot(lane < n && num != num);
+    if (lane == 0) odd_row = odd != 0 ? (int)__builtin_ctzll(odd) : kNone;
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       float s0 = lane == i ? 1.f : 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
@@ -163,6 +163,12 @@ __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__
       split_pairs<4>(t + i, x[0], x[1], x[2]);
 #pragma unroll
       for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(&Wl[k][lane * kDcP + i]) = make_uint4(x[k][0], x[k][1], x[k][2], x[k][3]);
+    }
+    if (odd_row < kNone) {  // M's rows in front of that one do not see what it and its beta make of later ones and of its column
+#pragma unroll 1
+      for (int i = 0; i < 64; ++i)
+        if (i >= odd_row || i < lane)
+          for (int k = 0; k < 3; ++k) Wl[k][lane * kDcP + i] = 0;
     }
   }
   __syncthreads();  // A has been read
@@ -215,6 +221,7 @@ __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__
           for (int m = 2 - k; m >= 0; --m) d[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b[m], d[a], 0, 0, 0);
         }
     }
+    if (qi >= odd_row) d[0] = d[1] = f32x4{NAN, NAN, NAN, NAN};
     put(Mo, 2 * w + ks, d[0], d[1]);
   }
   __syncthreads();
@@ -263,6 +270,7 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
   constexpr int DK = 32 * KS, PK = DK + 8, NV = 16 * NT, RTW = (2 * KS + 3) / 4;
   __shared__ __attribute__((aligned(16))) bf16_t Sl[3][NV * PK];    // the state before the chunk, [column][key dim]
   __shared__ __attribute__((aligned(16))) bf16_t Rl[3][NV * kDcP];  // R, [column][token]
+  __shared__ __attribute__((aligned(16))) int first[NV];            // chunk_seg.h: rows from which a column is no number
   // all column blocks of a (segment, head) pair on one XCD: its L2 then serves their common operands
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
   if (pair >= S_ * H) return;
@@ -350,6 +358,7 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
   };
   fetch(t0);
   publish();
+  if (tid < NV) first[tid] = kNone;
   for (int tb = t0; tb < t1; tb += kChunk) {
     const int n = min(kChunk, t1 - tb);
 #pragma unroll
@@ -386,7 +395,14 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
       for (int ct = 0; ct < NT; ++ct) {
         float x[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = bf2f(vf[i][ct]) - gf[i] * acc[ct][i];
+        for (int i = 0; i < 4; ++i) {
+          x[i] = bf2f(vf[i][ct]) - gf[i] * acc[ct][i];
+          if (!isfinite(x[i])) {
+            const int row = 16 * w + 4 * quad + i;
+            if (row < n) atomicMin(&first[16 * ct + c16], row);
+            x[i] = 0.f;
+          }
+        }
         uint32_t p[3][2];
         split_pairs<2>(x, p[0], p[1], p[2]);
 #pragma unroll
@@ -412,9 +428,12 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
               for (int m = 2 - k; m >= 0; --m) d[m & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, mf[3 * ks + m], d[m & 1], 0, 0, 0);
             }
           }
-          if (16 * w + c16 < n)
-            *reinterpret_cast<float4*>(o + (long)(tb + 16 * w + c16) * inner + (long)h * dv + dvb + 16 * ct + 4 * quad) =
-                make_float4(d[0][0] + d[1][0], d[0][1] + d[1][1], d[0][2] + d[1][2], d[0][3] + d[1][3]);
+          const int4 f = *reinterpret_cast<const int4*>(&first[16 * ct + 4 * quad]);
+          const int q = 16 * w + c16;
+          if (q < n)
+            *reinterpret_cast<float4*>(o + (long)(tb + q) * inner + (long)h * dv + dvb + 16 * ct + 4 * quad) =
+                make_float4(q < f.x ? d[0][0] + d[1][0] : NAN, q < f.y ? d[0][1] + d[1][1] : NAN, q < f.z ? d[0][2] + d[1][2] : NAN,
+                            q < f.w ? d[0][3] + d[1][3] : NAN);
         }
       }
     } else if (mine) {
@@ -437,6 +456,12 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
               for (int r = 0; r < RTW; ++r)
                 S[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf[6 * r + 3 * ks + m], x, S[r][ct], 0, 0, 0);
           }
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct)
+        if (first[16 * ct + c16] < kNone) {
+#pragma unroll
+          for (int r = 0; r < RTW; ++r) S[r][ct] = f32x4{NAN, NAN, NAN, NAN};
+        }
       publish();
     }
   }

@@ -522,3 +522,50 @@ def test_fp32_values_that_are_no_numbers(t, kw, bad):
         want = hops.window_attention_decode(q[i:i + 1], kc.cuda(), vc.cuda(), dev[2], sl, *a, **kw).cpu().view(4, dv)
         got = hops.window_attention_decode(q[i:i + 1], kc.cuda(), v2.cuda(), dev[2], sl, *a, **kw).cpu().view(4, dv)
         assert torch.equal(got[~hit[i]], want[~hit[i]]) and not bool(torch.isfinite(got[hit[i]]).any())
+
+
+@pytest.mark.parametrize("where", ["v", "k", "q", "z", "beta"])
+@pytest.mark.parametrize("t", [0, 63, 70, 149, 402])
+@pytest.mark.parametrize("kind", ["linear", "delta", "delta_plain", "bonus", "root", "root_spans"])
+def test_chunks_keep_later_tokens_out_of_earlier_ones(kind, where, t):
+    """A NaN or an infinity in a token's value, key, query, decay or beta leaves the outputs in front of it as they are, and the same
+    outputs and states are no numbers as token by token (the scan): at the first and last token of a segment and of a chunk, and
+    inside one.  Tolerances as for the chunks above."""
+    if where == "z" and kind == "linear" or where == "beta" and not kind.startswith("delta"):
+        pytest.skip("not an input of this form")
+    g = _g(84)
+    H, d = 2, 32
+    cu, ctx, slot = _segments([150, 300, 40], [0, 7, 3], [1, 0, 2])
+    T = 490
+    qkv, beta, state = _r(g, T, 3 * H * d, s=0.5, dt=BF), _r(g, T, H, dt=BF), _r(g, 3, H, d, d)
+    per_head = kind.startswith("delta")
+    z, zb = _r(g, T, H if per_head else H * d, dt=BF), _r(g, H if per_head else H * d) + (3.0 if kind.startswith("root") else -3.0)
+    cols = {"q": 0, "k": H * d, "v": 2 * H * d}
+    if kind == "linear":  # rows are [v | k | q] there
+        cols = {"v": 0, "k": H * d, "q": 2 * H * d}
+    for bad in (float("nan"),) if where in ("z", "beta") else (float("nan"), float("inf")):
+        a = [qkv.clone(), z.clone(), beta.clone()]
+        if where in cols:
+            a[0][t, cols[where] + d + 3] = bad
+        else:
+            a[1 if where == "z" else 2][t, -1] = bad
+        dev = [x.cuda() for x in a]
+
+        def run(chunks):
+            s = state.cuda()
+            seg = (s, cu.cuda(), ctx.cuda(), slot.cuda())
+            if kind == "linear":
+                o = hops.linear_attention(dev[0], torch.tensor([0.9, 0.99]).cuda(), *seg, H, d, d, mode=3 if chunks else 2)
+            else:
+                kw = dict(a_log=_r(_g(85), H).cuda(), beta=dev[2], unit=kind == "delta") if per_head else \
+                    dict(decay="exp_exp", bonus=_r(_g(85), H, d).cuda()) if kind == "bonus" else dict(tau=3.0)
+                o = hops.decay_scan(dev[0], 0, H * d, 2 * H * d, dev[1], zb.cuda(), *seg, H, H, d, d, 0.2,
+                                    mode=(4 if kind == "root_spans" else 3) if chunks else 2, **kw)
+            return o.cpu(), s.cpu()
+
+        for x, y in zip(run(True), run(False)):
+            fin = torch.isfinite(y)
+            assert torch.equal(torch.isfinite(x), fin)
+            if x.shape[0] == T:
+                assert bool(fin[:t].all()) and (kind == "bonus" and where == "z" or not bool(fin[t].all()))  # (a bonus token reads the state before its own decay)
+            torch.testing.assert_close(x[fin], y[fin], rtol=5e-5, atol=5e-5 * float(y[fin].abs().max()))
