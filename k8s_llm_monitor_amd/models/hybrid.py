@@ -576,7 +576,7 @@ class LightningMixer:
             self.tail_out = (proj, self.n_in)
         vkq = hops.activation_cols(proj, 0, self.n_act, "silu")
         o = hops.linear_attention(vkq, self.decay, cache["state"], meta.seg_cu, meta.seg_ctx, meta.seg_slot,
-                                  self.H, self.dk, self.dv, longest=meta.seg_max)
+                                  self.H, self.dk, self.dv, longest=meta.seg_max, singles=meta.num_decode)
         g = hops.gated_group_norm(o, proj, self.n_act, self.norm_w, self.eps, 1, h.dtype, after=True)
         return hops.linear(g, self.wo)
 
@@ -657,7 +657,7 @@ class GatedDeltaMixer:
         z, z_col = (proj, self.a_col) if self.per_head else (hops.linear(proj[:, self.a_col:self.a_col + self.ra], self.wa2), 0)
         o = hops.decay_scan(qkv, 0, Gk * dk, 2 * Gk * dk, z, self.dt_bias, cache["state"], *seg, H, Gk, dk, dv,
                             dk ** -0.5, a_log=self.a_log, beta=proj, beta_col=self.b_col, unit=True, z_col=z_col,
-                            longest=meta.seg_max)
+                            longest=meta.seg_max, singles=meta.num_decode)
         if self.low_rank_gate:
             gate = hops.linear(proj[:, self.g_col:self.g_col + self.rg], self.wg2)
             g = hops.gated_group_norm(o, gate, 0, self.norm_all, self.eps, H, h.dtype, after=True)
@@ -717,7 +717,7 @@ class GatedLinearMixer:
             proj = hops.linear(h, self.w_in)
         z = hops.linear(proj[:, self.a_col:self.a_col + self.ra], self.wa2)
         o = hops.decay_scan(proj, 0, H * dk, 2 * H * dk, z, self.a_bias, cache["state"], meta.seg_cu, meta.seg_ctx,
-                            meta.seg_slot, H, H, dk, dv, dk ** -0.5, tau=self.tau, longest=meta.seg_max)
+                            meta.seg_slot, H, H, dk, dv, dk ** -0.5, tau=self.tau, longest=meta.seg_max, singles=meta.num_decode)
         g = hops.gated_group_norm(o, proj, self.g_col, self.norm_all, self.eps, H, h.dtype, after=True, gate="silu")
         return hops.linear(g, self.wo)
 
@@ -825,7 +825,7 @@ class WkvMixer:
         torch.bmm(mix[:, :4].transpose(0, 1), self.w_rkvg, out=rkvg.view(T, 4, n).transpose(0, 1))
         z = hops.linear(hops.activation(hops.linear(mix[:, 4], self.w1), "tanh"), self.w2)
         o = hops.decay_scan(rkvg, 0, n, 2 * n, z, self.w0, cache["state"], *seg, H, H, dk, dk, 1.0, decay="exp_exp", bonus=self.u,
-                            longest=meta.seg_max)
+                            longest=meta.seg_max, singles=meta.num_decode)
         g = hops.gated_group_norm(o, rkvg, 3 * n, self.norm_w, self.eps, H, dtype, after=True, gate="silu")
         return hops.linear(g, self.wo)
 

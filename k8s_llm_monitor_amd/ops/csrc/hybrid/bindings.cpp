@@ -449,10 +449,13 @@ void conv_silu(Tensor out, Tensor proj, int64_t col0, Tensor cw, OptT cb, Tensor
 // decay given: the fixed-decay recurrence (dt = 1, no skip term); proj, dt_bias, a_log, d_skip are then not read
 // mode 0: with a decay table and G == nh, the chunked matrix-core kernel for bf16 steps with a mean of 32 rows per segment
 // and more whose sizes are its own, else a scan; 1 / 2: a scan in the decode / prompt mapping; 3: the chunked kernel (nt: its
-// value-column tiles per workgroup, 0: its choice), or the scan where it does not apply
+// value-column tiles per workgroup, 0: its choice), or the scan where it does not apply.  singles: so many segments in front are
+// running sequences' next tokens; where only the longest segment brings the chunks they stay on the decode mapping beside them (us,
+// in the chunked kernel -> beside it: 200 and 2 x 1000 236 -> 137, 60 and one of 256 68 -> 45; with a mean of 32 rows they run in the
+// shadow of the long chains: 60 and one of 2000 115 / 133, 32 and 2 x 2048 110 / 120)
 void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, OptT a_log, OptT d_skip, OptT decay,
               Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t nh, int64_t P, int64_t N, int64_t G,
-              int64_t mode, int64_t nt, int64_t longest) {
+              int64_t mode, int64_t nt, int64_t longest, int64_t singles) {
   const int f = act(xbc, "xbc");
   f32c(y, "y");
   f32c(state, "ssm_state");
@@ -484,18 +487,26 @@ void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, Opt
   TORCH_CHECK(y.numel() == T * nh * P, "ssm: y [T, nh*P]");
   TORCH_CHECK(state.dim() == 4 && state.size(1) == nh && state.size(2) == N && state.size(3) == P, "ssm_state [slots, nh, N, P]");
   TORCH_CHECK(G >= 1 && nh % G == 0 && N <= 256, "ssm: groups / state size (<= 256)");
-  if (cp != nullptr && !f && G == nh && (mode == 3 || (mode == 0 && (T >= 32 * ctx.numel() || longest >= 256))) &&
+  const int64_t S = ctx.numel();
+  TORCH_CHECK(singles >= 0 && singles <= S && singles <= T, "ssm_scan: single tokens in front");
+  auto scan = [&](int64_t segments, int64_t rows, int64_t m) {
+    check(k8sllm_hy_ssm_scan(y.data_ptr<float>(), xbc.data_ptr(), pp, pstride, (int)dt_col, bp, ap, dp, cp,
+                             state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
+                             (int)segments, rows, (int)nh, (int)P, (int)N, (int)G, f, (int)m, cur()),
+          "ssm_scan");
+  };
+  if (T >= 32 * S) singles = 0;
+  if (cp != nullptr && !f && G == nh && singles < S && (mode == 3 || (mode == 0 && (T >= 32 * S || longest >= 256))) &&
       reinterpret_cast<uintptr_t>(xbc.data_ptr()) % 16 == 0) {
-    const int rc = k8sllm_hy_chunk_scan(y.data_ptr<float>(), xbc.data_ptr(), cp, state.data_ptr<float>(), cu.data_ptr<int>(),
-                                        ctx.data_ptr<int>(), slot.data_ptr<int>(), (int)ctx.numel(), (long)T, (int)longest, (int)nh, (int)N, (int)P,
-                                        (int)nt, cur());
-    if (rc != 1) return check(rc, "ssm_scan (chunked)");
+    const int rc = k8sllm_hy_chunk_scan(y.data_ptr<float>(), xbc.data_ptr(), cp, state.data_ptr<float>(), cu.data_ptr<int>() + singles,
+                                        ctx.data_ptr<int>() + singles, slot.data_ptr<int>() + singles, (int)(S - singles),
+                                        (long)(T - singles), (int)longest, (int)nh, (int)N, (int)P, (int)nt, cur());
+    if (rc != 1) {
+      check(rc, "ssm_scan (chunked)");
+      return scan(singles, singles, 1);
+    }
   }
-  if (mode == 3) mode = 0;
-  check(k8sllm_hy_ssm_scan(y.data_ptr<float>(), xbc.data_ptr(), pp, pstride, (int)dt_col, bp, ap, dp, cp,
-                           state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
-                           (int)ctx.numel(), T, (int)nh, (int)P, (int)N, (int)G, f, (int)mode, cur()),
-        "ssm_scan");
+  scan(S, T, mode == 3 ? 0 : mode);
 }
 
 // In place on the fused rows [T, Hq*dk | G*dk | G*dv | ...]: rotary positions on the first 2 * len(freq)
@@ -683,13 +694,16 @@ void rotary_norm_cache(Tensor qkv, int64_t Hq, int64_t G, int64_t dk, int64_t dv
 // Linear attention with decays per head and key channel, or per head (z_bias [H]); plain, with the delta rule
 // (beta given) or with a bonus for the current token (bonus given); see decay_scan.hip.  dkind: how a decay
 // comes from its logit.  z_col: first column of the decay logits in z
-// ws: fp32 workspace of decay_scan_ws(T, ...) floats - given, the two-launch form for prompts runs
-// mode 0: by the step's mean segment length - prompts in chunks on the matrix cores where the form, sizes and alignment
-// are those kernels', else the two-launch scan; 1: the one-launch scan; 2: the two-launch scan; 3: the chunks
+// mode 0: prompts (by the step's mean segment length or a longest segment of 256 rows) in chunks on the matrix cores where the
+// form, sizes and alignment are those kernels', else the two-launch scan; other steps the one-launch scan; 1: the one-launch
+// scan; 2: the two-launch scan; 3: the chunks; 4: the chunks in spans where decays are per channel.  longest: rows of the
+// longest segment (0: not known).  singles: so many segments in front are running sequences' next tokens, which stay on the
+// one-launch scan of a decode step beside the chunks (us, in chunks of their own -> beside them, delta rule / 32 heads of 64 x 64:
+// 60 and one of 2000 192 -> 147, 175 -> 91; 32 and 2 x 2048 181 -> 157, 200 -> 137; 1 and one of 4000 206 -> 215, 132 -> 134)
 void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_col, Tensor z, Tensor z_bias, OptT a_log,
                 double tau, OptT beta, int64_t beta_col, Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t H,
                 int64_t Gk, int64_t dk, int64_t dv, double q_scale, bool unit, int64_t mode, int64_t z_col, int64_t dkind,
-                OptT bonus, int64_t longest) {
+                OptT bonus, int64_t longest, int64_t singles) {
   const int f = act(qkv, "qkv");
   same(z, f, "z");
   f32c(o, "o");
@@ -736,34 +750,46 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
   // 64 x 64: one of 2000 rows beside 60 575 -> 186, 399 -> 181; one of 256 beside 60 142 -> 139, 125 -> 107)
   const bool prompts = T >= 32l * S || longest >= 256;
   const void* zp = (const char*)z.data_ptr() + z_col * z.element_size();
-  if (!f && (mode >= 3 || (mode == 0 && prompts)) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 &&
+  TORCH_CHECK(singles >= 0 && singles <= S && singles <= T, "decay_scan: single tokens in front");
+  auto scan = [&](int64_t segments, int64_t rows, float* wp) {
+    check(k8sllm_hy_decay_scan(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col, zp, z.stride(0),
+                               z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, per_head, bp, bstride, wp_bonus,
+                               state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(), (int)segments,
+                               (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale, unit, f, wp, (long)rows, cur()),
+          "decay_scan");
+  };
+  const int* cu1 = cu.data_ptr<int>() + singles;
+  const int *ctx1 = ctx.data_ptr<int>() + singles, *slot1 = slot.data_ptr<int>() + singles;
+  const int S1 = S - (int)singles;
+  const long T1 = (long)(T - singles);
+  if (!f && S1 > 0 && (mode >= 3 || (mode == 0 && prompts)) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 &&
       qkv.stride(0) % 8 == 0 && q_col % 8 == 0 && k_col % 8 == 0 && v_col % 8 == 0) {
     // a chunk costs the same whatever it holds (us, 16 heads of 128 x 128, scan -> chunks: 40 segments of 33 rows 99 -> 101;
     // 16 of 64 73 -> 51; one of 64 21 -> 28; 4 of 2048 542 -> 209)
     if (per_head && (mode == 3 || longest >= 256 || (T >= 64l * S && T >= 128))) {
-      const long nb = k8sllm_hy_delta_chunk_ws(T, S, (int)H, (int)dk, (int)dv);
+      const long nb = k8sllm_hy_delta_chunk_ws(T1, S1, (int)H, (int)dk, (int)dv);
       if (nb > 0) {
         Tensor ws = torch::empty({nb}, o.options().dtype(torch::kUInt8));
-        return check(k8sllm_hy_delta_chunk(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
-                                           zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, bp,
-                                           bstride, state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(),
-                                           slot.data_ptr<int>(), S, (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale, unit,
-                                           ws.data_ptr(), (long)T, cur()),
-                     "decay_scan (chunks)");
+        check(k8sllm_hy_delta_chunk(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
+                                    zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, bp,
+                                    bstride, state.data_ptr<float>(), cu1, ctx1, slot1, S1, (int)H, (int)Gk, (int)dk, (int)dv,
+                                    (float)q_scale, unit, ws.data_ptr(), T1, cur()),
+              "decay_scan (chunks)");
+        return scan(singles, singles, nullptr);
       }
     } else if (bp == nullptr && !unit && (mode >= 3 || longest >= 256 || T >= 128l * S)) {
       // (us, 32 heads of 64 x 64, scan -> chunks: 16 segments of 64 rows 45 -> 52; one of 128, 16 heads, 29 -> 21; 13 of 500 140 ->
       // 104; 4 of 2048 428 -> 235)
       const int cut = mode == 4 ? 2 : mode == 3 ? 1 : 0;  // spans of chunks: forced, not, by the sizes
-      const long nb = k8sllm_hy_decay_chunk_ws(T, S, (int)longest, (int)H, (int)dk, (int)dv, cut);
+      const long nb = k8sllm_hy_decay_chunk_ws(T1, S1, (int)longest, (int)H, (int)dk, (int)dv, cut);
       if (nb > 0) {
         Tensor ws = torch::empty({nb}, o.options().dtype(torch::kUInt8));
-        return check(k8sllm_hy_decay_chunk(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
-                                           zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind,
-                                           wp_bonus, state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(),
-                                           slot.data_ptr<int>(), S, (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale,
-                                           ws.data_ptr(), (long)T, (int)longest, cut, cur()),
-                     "decay_scan (chunks)");
+        check(k8sllm_hy_decay_chunk(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
+                                    zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, wp_bonus,
+                                    state.data_ptr<float>(), cu1, ctx1, slot1, S1, (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale,
+                                    ws.data_ptr(), T1, (int)longest, cut, cur()),
+              "decay_scan (chunks)");
+        return scan(singles, singles, nullptr);
       }
     }
   }
@@ -773,10 +799,7 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
     ws = torch::empty({k8sllm_hy_decay_scan_ws(T, (int)H, (int)Gk, (int)dk)}, o.options());
     wp = ws.data_ptr<float>();
   }
-  check(k8sllm_hy_decay_scan(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col,
-                             zp, z.stride(0), z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, per_head, bp, bstride, wp_bonus, state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
-                             (int)ctx.numel(), (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale, unit, f, wp, (long)T, cur()),
-        "decay_scan");
+  scan(S, T, wp);
 }
 
 // The selective state-space recurrence with a decay per channel and state; see selective_scan.hip.  q holds

@@ -797,7 +797,7 @@ def conv_silu(proj: torch.Tensor, col0: int, C: int, conv_w: torch.Tensor, conv_
 def ssm_scan(xbc: torch.Tensor, proj: Optional[torch.Tensor], dt_col: int, dt_bias: Optional[torch.Tensor],
              a_log: Optional[torch.Tensor], d_skip: Optional[torch.Tensor], state: torch.Tensor, seg_cu: torch.Tensor,
              seg_ctx: torch.Tensor, seg_slot: torch.Tensor, nh: int, P: int, N: int, G: int, mode: int = 0,
-             decay: Optional[torch.Tensor] = None, col_tiles: int = 0, longest: int = 0) -> torch.Tensor:
+             decay: Optional[torch.Tensor] = None, col_tiles: int = 0, longest: int = 0, singles: int = 0) -> torch.Tensor:
     """The selective state-space recurrence, fp32, token by token within each segment:
 
         dt = softplus(proj[t, dt_col + h] + dt_bias[h]);  S <- exp(-exp(a_log[h]) dt) S + dt B_t x_t^T
@@ -843,13 +843,13 @@ def ssm_scan(xbc: torch.Tensor, proj: Optional[torch.Tensor], dt_col: int, dt_bi
         return y
     y = torch.empty(T, nh * P, dtype=torch.float32, device=xbc.device)
     native().ssm_scan(y, xbc, proj, int(dt_col), dt_bias, a_log, d_skip, decay, state, seg_cu, seg_ctx, seg_slot, nh, P,
-                      N, G, int(mode), int(col_tiles), int(longest))
+                      N, G, int(mode), int(col_tiles), int(longest), int(singles))
     return y
 
 
 def linear_attention(vkq: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, seg_cu: torch.Tensor,
                      seg_ctx: torch.Tensor, seg_slot: torch.Tensor, H: int, dk: int, dv: int, mode: int = 0,
-                     col_tiles: int = 0, longest: int = 0) -> torch.Tensor:
+                     col_tiles: int = 0, longest: int = 0, singles: int = 0) -> torch.Tensor:
     """Linear attention with a fixed decay per head, as a recurrence over each segment:
 
         S_t = decay[h] S_(t-1) + k_t v_t^T;   o_t = S_t^T q_t
@@ -858,21 +858,22 @@ def linear_attention(vkq: torch.Tensor, decay: torch.Tensor, state: torch.Tensor
     dv] fp32 is read at a segment's start (zero where seg_ctx is 0) and written back at its end.
     Returns o [T, H*dv] fp32.  State, products and sums are fp32.
 
-    GPU: bf16 prompts (a mean of 32 rows per segment and more, or a ``longest`` segment of 256 if that is given), ``dim`` a multiple of 32 up to 128, ``vdim`` of 16
-    (``mode`` 3 forces it, ``col_tiles`` 1 / 2 / 4 its value columns per workgroup, 16 / 32 / 64; 0: its choice): chunks of 64
+    GPU: bf16 prompts (a mean of 32 rows per segment and more, or a ``longest`` segment of 256 if that is given), ``dim`` a
+    multiple of 32 up to 128, ``vdim`` of 16 (``mode`` 3 forces it, ``col_tiles`` 1 / 2 / 4 its value columns per workgroup, 16 / 32 / 64; 0: its choice): chunks of 64
     tokens on the matrix cores, only the state crossing chunks - fp32 scores, decays and state enter the products as three
     bf16 parts that add up to them, so only the order of the fp32 sums differs, which follows the chunk grid from the
-    segment's first row on.  Else the sequential scan (``ssm_scan`` with the decay table; ``mode`` 1 / 2 force its decode /
-    prompt lane mapping)."""
+    segment's first row on.  Where it is the longest segment that brings the chunks, the first ``singles`` segments, running
+    sequences' next tokens, stay on the scan of a decode step.  Else the sequential scan (``ssm_scan`` with the decay
+    table; ``mode`` 1 / 2 force its decode / prompt lane mapping)."""
     return ssm_scan(vkq, None, 0, None, None, None, state, seg_cu, seg_ctx, seg_slot, H, dv, dk, H, mode, decay=decay,
-                    col_tiles=col_tiles, longest=longest)
+                    col_tiles=col_tiles, longest=longest, singles=singles)
 
 
 def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.Tensor, z_bias: torch.Tensor,
                state: torch.Tensor, seg_cu: torch.Tensor, seg_ctx: torch.Tensor, seg_slot: torch.Tensor, H: int, Gk: int,
                dk: int, dv: int, q_scale: float, a_log: Optional[torch.Tensor] = None, tau: float = 1.0,
                beta: Optional[torch.Tensor] = None, beta_col: int = 0, unit: bool = False, mode: int = 0, z_col: int = 0,
-               decay: Optional[str] = None, bonus: Optional[torch.Tensor] = None, longest: int = 0) -> torch.Tensor:
+               decay: Optional[str] = None, bonus: Optional[torch.Tensor] = None, longest: int = 0, singles: int = 0) -> torch.Tensor:
     """Linear attention with a decay per head and key channel (or per head), optionally with the delta rule
     or a bonus for the current token, as an fp32 recurrence over each segment.  Per head h (reading query / key head ``h // (H / Gk)``) and token:
 
@@ -900,8 +901,9 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     that does not depend on the state (decays, unit norms, k . q, beta) for all rows at once into a
     workspace, then the recurrence over it; decode steps run as one launch.  bf16 prompts of the delta rule with one decay
     per head, and without the delta rule and unit norms of decays per channel (``dk`` a multiple of 32 up to 128, ``dv`` of
-    16), go in chunks of 64 tokens on the matrix cores, fp32 operands as three bf16 parts that add up to them; else token by
-    token.  ``mode`` 1 / 2 force the one-launch / two-launch
+    16), go in chunks of 64 tokens on the matrix cores, fp32 operands as three bf16 parts that add up to them, and the first
+    ``singles`` segments, running sequences' next tokens, beside them as in a decode step: their bits do not depend on what else
+    is in the step.  Else token by token.  ``mode`` 1 / 2 force the one-launch / two-launch
     scan, 3 the chunks, 4 the chunks in spans where decays are per channel (tests)."""
     T = qkv.shape[0]
     nz = z_bias.numel()
@@ -950,7 +952,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     o = torch.empty(T, H * dv, dtype=torch.float32, device=qkv.device)
     native().decay_scan(o, qkv, int(q_col), int(k_col), int(v_col), z, z_bias, a_log, float(tau), beta, int(beta_col),
                         state, seg_cu, seg_ctx, seg_slot, int(H), int(Gk), int(dk), int(dv), float(q_scale), bool(unit), int(mode), int(z_col), dkind,
-                        bonus, int(longest))
+                        bonus, int(longest), int(singles))
     return o
 
 

@@ -569,3 +569,35 @@ def test_chunks_keep_later_tokens_out_of_earlier_ones(kind, where, t):
             if x.shape[0] == T:
                 assert bool(fin[:t].all()) and (kind == "bonus" and where == "z" or not bool(fin[t].all()))  # (a bonus token reads the state before its own decay)
             torch.testing.assert_close(x[fin], y[fin], rtol=5e-5, atol=5e-5 * float(y[fin].abs().max()))
+
+
+@pytest.mark.parametrize("kind", ["linear", "delta", "bonus", "root"])
+@pytest.mark.parametrize("prompts", [[300], [290, 1, 70], [256, 513]])
+def test_single_tokens_beside_prompts_keep_their_bits(kind, prompts):
+    """Running sequences' next tokens in front of prompts that go in chunks: outputs and states have the bits of the same tokens in a
+    step of their own, and the prompts' those of a step without them."""
+    g = _g(86)
+    H, d, nd = 2, 32, 40
+    lens = [1] * nd + prompts
+    S, T = len(lens), nd + sum(prompts)
+    cu, ctx, slot = (v.cuda() for v in _segments(lens, [9] * nd + [0, 3, 0][:len(prompts)], list(range(S))))
+    qkv, state = _r(g, T, 3 * H * d, s=0.5, dt=BF).cuda(), _r(g, S, H, d, d).cuda()
+    per_head = kind == "delta"
+    z, zb = _r(g, T, H if per_head else H * d, dt=BF).cuda(), (_r(g, H if per_head else H * d) - 1.0).cuda()
+    beta, al, bonus, lam = _r(g, T, H, dt=BF).cuda(), _r(g, H).cuda(), _r(g, H, d).cuda(), torch.tensor([0.9, 0.99]).cuda()
+    longest = max(prompts)
+    assert T < 32 * S  # (linear attention takes steps of longer segments in chunks as a whole)
+
+    def run(a, b, s0, s1, **kw):  # rows [a, b), segments [s0, s1)
+        s = state.clone()
+        seg = (s, cu[s0:s1 + 1] - cu[s0], ctx[s0:s1], slot[s0:s1])
+        if kind == "linear":
+            return hops.linear_attention(qkv[a:b], lam, *seg, H, d, d, **kw), s
+        form = dict(a_log=al, beta=beta[a:b], unit=True) if per_head else dict(decay="exp_exp", bonus=bonus) if kind == "bonus" else dict(tau=3.0)
+        return hops.decay_scan(qkv[a:b], 0, H * d, 2 * H * d, z[a:b], zb, *seg, H, H, d, d, 0.2, **form, **kw), s
+
+    o, s = run(0, T, 0, S, longest=longest, singles=nd)
+    od, sd = run(0, nd, 0, nd, longest=1)
+    assert torch.equal(o[:nd], od) and torch.equal(s[:nd], sd[:nd])
+    op, sp = run(nd, T, nd, S, longest=longest)
+    assert torch.equal(o[nd:], op) and torch.equal(s[nd:], sp[nd:])
