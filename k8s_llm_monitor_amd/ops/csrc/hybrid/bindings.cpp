@@ -793,6 +793,7 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
       }
     }
   }
+  TORCH_CHECK(mode < 3, "decay_scan: not a form, size or alignment of the chunks that were asked for");
   Tensor ws;
   float* wp = nullptr;
   if (mode == 2 || (mode != 1 && prompts)) {

@@ -874,11 +874,11 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
       const int rc = k8sllm_hy_window_flash(out, qkv, q_stride, k_cache, v_cache, cu, ctx, block_tables, bt_stride, S, T, Hq, G,
                                             dk, dv, scale, window, chunked, keep, cap, cap <= kMaxCapPlain && !sink, sink,
                                             sinks, gate, g_stride, s);
-      if (rc != 1) return rc;
+      if (rc != 1 || mfma == kFlashForced) return rc;
     }
     // query rows per wave: 32 once the step is large enough to fill the chip that way (two row tiles
     // share every K / V^T fragment), else 16; mfma = 16 / 32 / 64 forces one (tests, measurements)
-    const int qrows = mfma >= 16 && mfma != kFlashForced ? mfma : (T * Hq >= 64 * 1024 ? 32 : 16);
+    const int qrows = mfma >= 16 ? mfma : (T * Hq >= 64 * 1024 ? 32 : 16);
     const dim3 grid((unsigned)(T / qrows + S), (unsigned)Hq);
 #define K8SLLM_WPC(DK, DV, QT, CAP)                                                                                    \
   hipLaunchKernelGGL((window_prefill_mfma_kernel<DK, DV, QT, CAP>), grid, dim3(64), 0, s, (bf16_t*)out,                 \
@@ -892,7 +892,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
   if (qrows == 64) { K8SLLM_WP(DK, DV, 4); }                     \
   else if (qrows == 32) { K8SLLM_WP(DK, DV, 2); }                \
   else { K8SLLM_WP(DK, DV, 1); }
-    if (mfma >= 16 && mfma != 16 && mfma != 32 && mfma != 64 && mfma != kFlashForced) return -1;
+    if (mfma >= 16 && mfma != 16 && mfma != 32 && mfma != 64) return -1;
     if (dk == 64 && dv == 64) { K8SLLM_WPQ(64, 64); }
     else if (dk == 64) { K8SLLM_WPQ(64, 128); }
     else if (dv == 64) { K8SLLM_WPQ(128, 64); }
@@ -902,6 +902,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
 #undef K8SLLM_WPC
     return (int)hipGetLastError();
   }
+  if (mfma == kFlashForced) return 1;
   if (f32 && mfma) {  // head sizes of 64 and 128: window_f32.hip, faster at every size measured there
     const int rc = k8sllm_hy_window_f32(out, qkv, q_stride, k_cache, v_cache, cu, ctx, block_tables, bt_stride, S, T, Hq, G, dk, dv,
                                         bs, scale, window, chunked, keep, cap, sink, sinks, gate, g_stride, 0, s);

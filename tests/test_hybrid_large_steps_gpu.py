@@ -109,6 +109,34 @@ def test_chunked_linear_attention_negative_decay():
     got = hops.linear_attention(vkq.cuda(), decay.cuda(), got_s, cu.cuda(), ctx.cuda(), slot.cuda(), 2, 32, 32, mode=3)
     for a, b in ((got.cpu(), want), (got_s.cpu(), want_s)):
         torch.testing.assert_close(a, b, rtol=2e-5, atol=2e-5 * float(b.abs().max()))
+    scan = hops.linear_attention(vkq.cuda(), decay.cuda(), state.cuda(), cu.cuda(), ctx.cuda(), slot.cuda(), 2, 32, 32, mode=2)
+    assert not torch.equal(got, scan)  # it was the chunked kernel
+
+
+def test_forms_that_are_asked_for_run_or_raise():
+    """A forced kernel that is not one for the call's sizes, form or alignment raises instead of leaving the call to another one."""
+    g = _g(87)
+    cu, ctx, slot = (v.cuda() for v in _segments([70], [0], [0]))
+
+    def decay(mode, dk=32, per_head=True, shift=0, **kw):
+        qkv, z = _r(g, 70, 3 * dk + shift, dt=BF).cuda()[:, shift:], _r(g, 70, 1 if per_head else dk, dt=BF).cuda()
+        zb, st = _r(g, z.shape[1]).cuda(), torch.zeros(1, 1, dk, dk).cuda()
+        if per_head:
+            kw = dict(kw, beta=_r(g, 70, 1, dt=BF).cuda())
+        return hops.decay_scan(qkv, 0, dk, 2 * dk, z, zb, st, cu, ctx, slot, 1, 1, dk, dk, 1.0, tau=2.0, mode=mode, **kw)
+
+    for kw in (dict(mode=3), dict(mode=3, per_head=False), dict(mode=4, per_head=False)):
+        decay(**kw)
+    for kw in (dict(mode=4), dict(mode=3, dk=24), dict(mode=3, shift=1), dict(mode=3, per_head=False, unit=True), dict(mode=4, per_head=False, dk=160)):
+        with pytest.raises(RuntimeError):
+            decay(**kw)
+    kc, vc, bt = (v.cuda() for v in _paged(g, BF, [20], 2, 1, 96, 64))
+    q = _r(g, 20, 2 * 96, dt=BF).cuda()
+    a = (_i32([0, 20]).cuda(), _i32([0]).cuda(), bt, 2, 1, 96, 64, 0.1, 0, False)
+    hops.window_attention_prefill(q, kc, vc, *a)
+    for x in ((q, kc, vc), (q.float(), kc.float(), vc.float())):
+        with pytest.raises(RuntimeError):
+            hops.window_attention_prefill(*x, *a, mfma=256)
 
 
 @pytest.mark.parametrize("H,Gk,dk,dv", [(4, 2, 128, 128), (2, 2, 32, 16), (3, 1, 64, 48), (2, 1, 96, 32)])
