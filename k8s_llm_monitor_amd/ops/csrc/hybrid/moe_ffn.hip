@@ -23,10 +23,10 @@ namespace k8sllm {
 constexpr int kMaxE = 256;
 constexpr int kMaxK = 16;
 
-// A strict order of logits: larger first, equal ones by number (-0 equals 0), NaN last
+// A strict order of logits: NaN first (its weights then show it, as torch's topk does), larger ones, equal ones by number (-0 equals 0)
 __device__ __forceinline__ bool goes_before(float a, int ia, float b, int ib) {
   const bool na = a != a, nb = b != b;
-  if (na || nb) return na && nb ? ia < ib : nb;
+  if (na || nb) return na && nb ? ia < ib : na;
   return a > b || (a == b && ia < ib);
 }
 

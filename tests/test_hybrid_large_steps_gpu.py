@@ -379,6 +379,21 @@ def test_router_ranks(T, E, K, shared):
         torch.testing.assert_close(got[2].cpu().view(-1), torch.sigmoid(h.float() @ wr[E]), rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("over_all", [False, True])
+def test_router_logits_that_are_no_numbers(over_all):
+    """An expert whose logit is NaN is chosen first and the token's weights are NaN, as in the torch form: a fault in a router's weights
+    does not pass unseen.  Infinite logits keep their place."""
+    g = _g(88)
+    E, K = 9, 2
+    h, wr = _r(g, 5, 64, dt=BF), _r(g, E, 64, s=0.1)
+    for e, bad in ((0, float("nan")), (4, float("nan")), (8, float("nan")), (4, float("-inf"))):
+        bias = _r(g, E)
+        bias[e] = bad
+        want = hops.moe_router(h, wr, bias, E, K, over_all)
+        got = hops.moe_router(h.cuda(), wr.cuda(), bias.cuda(), E, K, over_all)
+        assert torch.equal(got[0].cpu(), want[0]) and torch.equal(got[1].cpu().isnan(), want[1].isnan())
+
+
 @pytest.mark.parametrize("n,E", [(1, 1), (63, 8), (128, 8), (1000, 64), (1024, 5), (1025, 8), (700, 65)])
 def test_expert_sort(n, E):
     """The counting sort of (token, expert) pairs around the limits of its one-pass form: stable, every pair once."""
