@@ -1165,7 +1165,7 @@ FEW_ROWS, FEW_ROWS_K, FEW_ROWS_WEIGHTS = 16, 4096, 1 << 24
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-            and w.shape[1] % 32 == 0 and w.shape[1] <= FEW_ROWS_K and w.numel() <= FEW_ROWS_WEIGHTS and x.shape[0] > 0
+            and w.shape[1] % 32 == 0 and 32 <= w.shape[1] <= FEW_ROWS_K and w.numel() <= FEW_ROWS_WEIGHTS and x.shape[0] > 0
             and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
@@ -1184,7 +1184,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def linear_glu(x: torch.Tensor, w: torch.Tensor, f: int, kind: str) -> tuple:
     """The gated unit ``act(gate x) * (up x)`` [T, f] of ``w``'s rows [f gate | f up | the rest], and a projection with the column
     at which the rest's outputs begin in it.  ``linear`` and ``glu``, in one launch for the rows that ``linear`` takes itself."""
-    if len(x) <= FEW_ROWS and f % 16 == 0 and _few_rows(x, w):
+    if len(x) <= FEW_ROWS and f > 0 and f % 16 == 0 and _few_rows(x, w):
         a = torch.empty(x.shape[0], f, dtype=x.dtype, device=x.device)
         y = torch.empty(x.shape[0], w.shape[0] - 2 * f, dtype=x.dtype, device=x.device)
         native().few_rows_glu(a, y, x, w, ACTS[kind])

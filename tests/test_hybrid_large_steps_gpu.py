@@ -450,6 +450,17 @@ def test_decode_attention_row_broadcasts(dk, dv, Hq, G):
         torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1e-2, atol=2e-3)
 
 
+def test_linear_of_nothing():
+    """Empty sums, no columns, no rows and no gated unit are what the library makes of them."""
+    g = _g(89)
+    for M, N, K in ((3, 8, 0), (3, 0, 64), (0, 8, 64)):
+        x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, dt=BF).cuda()
+        assert torch.equal(hops.linear(x, w), torch.nn.functional.linear(x, w))
+    x, w = _r(g, 2, 64, dt=BF).cuda(), _r(g, 24, 64, dt=BF).cuda()
+    a, y, col = hops.linear_glu(x, w, 0, "silu")
+    assert a.shape == (2, 0) and torch.equal(y[:, col:], hops.linear(x, w))
+
+
 @pytest.mark.parametrize("M,f,rest,K", [(1, 16, 0, 32), (3, 48, 40, 1024), (16, 176, 16, 160), (17, 32, 8, 64), (2, 24, 8, 64)])
 @pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
 def test_gated_unit_in_the_projection(M, f, rest, K, kind):
