@@ -35,6 +35,10 @@ __device__ __forceinline__ float log2_decay(float x, int kind, float A, float in
   return l < -4096.f ? -4096.f : l;
 }
 
+// what a workgroup of a scan owns: a whole segment, or one of the spans that a long one is cut into - the launch that leaves the
+// spans' end states, and the one that folds those in front of its own
+constexpr int kWhole = 0, kSpanEnds = 1, kSpanRun = 2;
+
 struct ChunkAt {
   int seg, row, n;  // segment (-1: no such chunk), first row of the step, rows
   int k, count;     // the chunk's number within its segment, the segment's chunks

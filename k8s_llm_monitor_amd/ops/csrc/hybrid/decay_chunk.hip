@@ -248,8 +248,6 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
   }
 }
 
-constexpr int kWhole = 0, kSpanEnds = 1, kSpanRun = 2;
-
 // MODE kWhole: workgroups own whole segments.  Else a segment is cut into spans of `span` chunks that run side by side: kSpanEnds
 // leaves the end state of every span but a segment's last from a zero state in spans_s [span][head][dv][channels], its decays'
 // products in spans_d [span][head][channels], and the state that the segment starts from in its last span's place; kSpanRun

@@ -134,6 +134,12 @@ __device__ __forceinline__ float lanes_sum(float v) {
 
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
+// windowed attention: the first position that a row at position p sees
+__device__ __forceinline__ int first_key(int p, int window, int chunked) {
+  if (window <= 0) return 0;
+  return chunked ? p - p % window : max(0, p - window + 1);
+}
+
 // the segment that holds row r: largest s with cu[s] <= r (cu has S + 1 entries, cu[0] = 0)
 __device__ __forceinline__ int find_segment(const int* __restrict__ cu, int S, int r) {
   int lo = 0, hi = S - 1;

@@ -38,8 +38,6 @@ __device__ __forceinline__ float softplus_fast(float x) {
   return fmaxf(x, 0.f) + (e < 0.03125f ? series : lg);
 }
 
-constexpr int kWhole = 0, kSpanEnds = 1, kSpanRun = 2;
-
 template <typename T, int LPC, int NPL, int MODE>
 __global__ __launch_bounds__(256) void selective_scan_kernel(
     T* __restrict__ out, const T* __restrict__ xc, const T* __restrict__ q, long q_stride, int b_col, int c_col,

@@ -24,11 +24,6 @@ constexpr int kMaxDK = 512;
 constexpr int kGenVC = 8;  // the any-size kernels: dv <= 64 * kGenVC, dk <= kGenDK
 constexpr int kGenDK = 1024;
 
-// the first position that a row at position p sees
-__device__ __forceinline__ int first_key(int p, int window, int chunked) {
-  if (window <= 0) return 0;
-  return chunked ? p - p % window : max(0, p - window + 1);
-}
 // tanh from one exponential and one reciprocal: absolute error about 1e-7 (the bf16 kernels' scores; the
 // any-size kernels call tanhf)
 __device__ __forceinline__ float tanh_exp2(float x) {

@@ -20,11 +20,6 @@ namespace k8sllm {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ int first_key_f32(int p, int window, int chunked) {
-  if (window <= 0) return 0;
-  return chunked ? p - p % window : max(0, p - window + 1);
-}
-
 // max over the lanes of a query column (its four quarters)
 __device__ __forceinline__ float quarters_max(float x) {
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -64,10 +59,10 @@ __global__ __launch_bounds__(DECODE ? 512 : 64, DECODE ? 1 : 2) void window_f32_
     row = at.row + min(col, n - 1);
   }
   const int g = h / R, hi = DECODE ? p + 1 : p0 + n;  // no column sees a position from hi on
-  const int lo = first_key_f32(p, window, chunked);
-  const int lo_last = DECODE ? lo : first_key_f32(p0 + n - 1, window, chunked);  // from here to p0: keys that every column sees
+  const int lo = first_key(p, window, chunked);
+  const int lo_last = DECODE ? lo : first_key(p0 + n - 1, window, chunked);  // from here to p0: keys that every column sees
   // pages: the kept ones, then those from the first column's window on
-  const int w_first = first_key_f32(p0, window, chunked) >> 4, k_end = (keep + 15) >> 4;
+  const int w_first = first_key(p0, window, chunked) >> 4, k_end = (keep + 15) >> 4;
   const int t_end = (hi + 15) >> 4, gap_from = keep > 0 ? k_end : 0, gap_to = max(w_first, gap_from);
   const int tiles = min(gap_from, t_end) + max(t_end - gap_to, 0);
   auto page_of = [&](int i) { return i < gap_from ? i : i - gap_from + gap_to; };

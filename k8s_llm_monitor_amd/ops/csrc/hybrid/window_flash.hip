@@ -32,11 +32,6 @@ typedef __attribute__((address_space(1))) void gbl_void_t;
 constexpr int kFlashRing = 4;
 constexpr int kFlashIds = 4096;  // page ids that a workgroup keeps in LDS
 
-__device__ __forceinline__ int flash_first(int p, int window, int chunked) {
-  if (window <= 0) return 0;
-  return chunked ? p - p % window : max(0, p - window + 1);
-}
-
 // CAP 0: plain scores; 1: capped; 2: capped with a small cap and no sink, softmax without a running maximum
 template <int DK, int DV, int HW, int CAP>
 __global__ __launch_bounds__(512, 2) void window_flash_kernel(
@@ -94,13 +89,13 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
   const int wq = qs + (wave % WPH) * 32;  // the wave's first row within the segment
   const bool any = wq < L;
   const int myq = wq + r32;
-  const int my_p = cst + min(myq, L - 1), my_lo = flash_first(my_p, window, chunked);
+  const int my_p = cst + min(myq, L - 1), my_lo = first_key(my_p, window, chunked);
   const int pw0 = cst + min(wq, L - 1), pw1 = cst + min(wq + 31, L - 1);  // the wave's positions
-  const int lo_w = flash_first(pw0, window, chunked), lo_in = flash_first(pw1, window, chunked);
+  const int lo_w = first_key(pw0, window, chunked), lo_in = first_key(pw1, window, chunked);
   const int hi = cst + min(qs + QR, L);  // one past the workgroup's last position
   // tiles: those that hold kept keys, then from the first one that the workgroup's first row sees
   const int kt = (min(keep, hi) + 63) >> 6;
-  const int w0 = max(kt, flash_first(cst + qs, window, chunked) >> 6);
+  const int w0 = max(kt, first_key(cst + qs, window, chunked) >> 6);
   const int nu = kt + max(0, ((hi - 1) >> 6) - w0 + 1);
   auto tile_of = [&](int u) { return u < kt ? u : w0 + u - kt; };
 

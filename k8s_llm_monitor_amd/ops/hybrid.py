@@ -420,17 +420,15 @@ def qk_norm_cache(qkv: torch.Tensor, qw: torch.Tensor, kw: torch.Tensor, eps: fl
 
 def rotary_cache(qkv: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int, positions: torch.Tensor, freq: torch.Tensor,
                  pairs: bool, q_scale: Optional[torch.Tensor], k_cache: Optional[torch.Tensor],
-                 v_cache: Optional[torch.Tensor], slot_mapping: Optional[torch.Tensor], rot_off: int = 0,
-                 rot_k: bool = True, norm: int = 0, qw: Optional[torch.Tensor] = None, kw: Optional[torch.Tensor] = None,
+                 v_cache: Optional[torch.Tensor], slot_mapping: Optional[torch.Tensor], norm: int = 0,
+                 qw: Optional[torch.Tensor] = None, kw: Optional[torch.Tensor] = None,
                  eps: float = 0.0, v_from_k: bool = False) -> None:
     """In place on the fused rows [T, Hq*dk | Hkv*dk | Hkv*dv | ...]: the first ``2 len(freq)`` entries
     of every query and key head turn by the angle ``position * freq[i]`` (fp32; ``pairs``: entry 2i
     with 2i + 1, else entry i with i + len(freq); rotary_freq); the rest of a head passes.  ``q_scale``
     [Hq] fp32 (optional): every query head is multiplied by its number in the same pass (a per-head
     temperature folded into the query).  Keys (turned) and values go to the paged cache at
-    ``slot_mapping`` (< 0: not written).  ``rot_off``: the turning entries are ``rot_off .. rot_off +
-    2 len(freq)`` of every head instead of the first; ``rot_k`` False: the keys are taken as they are
-    (turned already) and only written to the pages.
+    ``slot_mapping`` (< 0: not written).
 
     ``norm``: every query and key head is also RMS-normed over its ``dk`` entries (fp32, ``eps`` inside
     the root) - 1: BEFORE the turn, times ``qw`` / ``kw`` ([dk] fp32, shared by the heads); 2: AFTER the
@@ -447,7 +445,7 @@ def rotary_cache(qkv: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int, positio
             x = x.clone()
             if norm == 1:
                 x = rms(x) * w.float()
-            x[..., rot_off:] = _rotate(x[..., rot_off:], positions, freq, pairs)
+            x = _rotate(x, positions, freq, pairs)
             return rms(x) if norm == 2 else x
 
         q = turn(qkv[:, :nq].float().view(T, Hq, dk), qw)
@@ -455,7 +453,7 @@ def rotary_cache(qkv: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int, positio
             q = q * q_scale.float().view(1, Hq, 1)
         k_raw = qkv[:, nq:nq + nk].clone()
         k = qkv[:, nq:nq + nk].float().view(T, Hkv, dk)
-        k = turn(k, kw) if rot_k else k
+        k = turn(k, kw)
         qkv[:, :nq] = q.reshape(T, nq).to(qkv.dtype)
         qkv[:, nq:nq + nk] = k.reshape(T, nk).to(qkv.dtype)
         if k_cache is not None:
@@ -469,8 +467,7 @@ def rotary_cache(qkv: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int, positio
         native().rotary_norm_cache(qkv, Hq, Hkv, dk, dv, positions, freq, bool(pairs), int(norm), qw, kw, float(eps), q_scale,
                                    k_cache, v_cache, slot_mapping, bool(v_from_k))
         return
-    native().rotary_cache(qkv, Hq, Hkv, dk, dv, positions, freq, bool(pairs), q_scale, k_cache, v_cache, slot_mapping,
-                          int(rot_off), bool(rot_k))
+    native().rotary_cache(qkv, Hq, Hkv, dk, dv, positions, freq, bool(pairs), q_scale, k_cache, v_cache, slot_mapping)
 
 
 def _attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float, sink: bool,
@@ -1094,10 +1091,11 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
 
     GPU: the (token, slot) pairs are counting-sorted by expert on the device and both projections
     run as ONE grouped launch each over the sorted rows (SwiGLU in the first epilogue); no host
-    synchronisation.  bf16: matrix-core kernels - 16-row tiles with the rows gathered on load
+    synchronisation.  bf16: matrix-core kernels - tiles of 16, 32 or 64 rows by the mean rows of an expert, gathered on load
     (decode, small steps), or from TILE_MIN_ROWS sorted rows of an ``il`` layer the prefill tile
     GEMM of the Mixtral path (ungated experts whose widths are multiples of 256 take it too, with
-    the GELU as a launch between); fp32 (and K not a multiple of 32): the 64 x 64 fp32 tile kernel."""
+    the GELU as a launch between); fp32: 64 x 64 tiles on the fp32 matrix instruction.  K that is no multiple of 32 and
+    unaligned fp32 rows: 64 x 64 tiles on the vector unit."""
     T, d = h.shape
     E, K = w13.shape[0], ids.shape[1]
     ff = w2.shape[2]
