@@ -202,16 +202,22 @@ class ModelRunner:
         # layout of the staging buffer (int32 words; the float sampling parameters bit-cast)
         nl = sum(len(x) for x in logit_rows) if logit_rows is not None else R
         hy = R if self.hybrid else 0
-        # latent attention: for every window of those layers the pages that the chunks see through it, [first, end) of each
-        seen = {w: [(max(0, c - w + 1) // BLOCK_SIZE if w else 0, (c + n + BLOCK_SIZE - 1) // BLOCK_SIZE) for c, n in zip(starts, lens)]
-                for w in (self.model.page_windows if hy and seqs else ())}
+        # latent attention: for every window of those layers the first page that each chunk sees through it and the pages up to its
+        # last token, one chunk after the other
+        seen = {}
+        if hy and seqs and self.model.page_windows:
+            c0 = np.asarray(starts)
+            pages = (c0 + lens + BLOCK_SIZE - 1) // BLOCK_SIZE
+            for w in self.model.page_windows:
+                first = np.maximum(c0 - (w - 1), 0) // BLOCK_SIZE if w else np.zeros_like(c0)
+                seen[w] = first, np.cumsum(pages - first)
         sizes = dict(ids=T, pos=T, slots=T, cu=len(seqs) + 1, qs=nq, st=nq, lidx=nl, temp=R, topk=R, topp=R,
                      gcu=hy + 1 if hy else 0, gctx=hy, gslot=hy,
                      cst=len(seqs) if paged else 0, bt=len(seqs) * W, dbt=nd * Wd, dlen=nd,
                      mcu=len(seqs) + 2 if kA else 0, mqs=nq if kA else 0, mst=nq if kA else 0,
                      mlidx=len(seqs) if kA else 0)
-        for w, ab in seen.items():
-            sizes.update({f"pgl{w}": sum(b - a for a, b in ab), f"pgb{w}": len(ab) * W})
+        for w, (_, end) in seen.items():
+            sizes[f"pgl{w}"], sizes[f"pgb{w}"] = int(end[-1]), len(seqs) * W
         off, o = {}, 0
         for k, n in sizes.items():
             off[k] = o
@@ -258,12 +264,11 @@ class ModelRunner:
             bt2[:] = 0
             for i, s in enumerate(seqs):
                 bt2[i, : len(s.block_table)] = s.block_table
-            for w, ab in seen.items():
-                a, b = np.asarray(ab).T[:, :, None]
-                end, col = np.cumsum(b - a)[:, None], np.arange(W)
-                v[f"pgl{w}"][:] = bt2[(col >= a) & (col < b)]
-                # (pages that are not seen get the number of one that is)
-                v[f"pgb{w}"][:] = np.clip(end - b + col, end - b + a, end - 1).ravel()
+            for w, (first, end) in seen.items():
+                a, b, e, col = first[:, None], pages[:, None], end[:, None], np.arange(W)
+                v[f"pgl{w}"][:] = bt2[(col >= a) & (col < b) if w else col < b]
+                at = np.minimum(col + (e - b), e - 1)  # (pages that are not seen get the number of one that is)
+                v[f"pgb{w}"].reshape(at.shape)[:] = np.maximum(at, e - b + a) if w else at
         if nd:
             dbt = v["dbt"].reshape(nd, Wd)
             dbt[:] = 0
@@ -289,10 +294,10 @@ class ModelRunner:
         if hy:
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = dv["gcu"], dv["gctx"], dv["gslot"]
             meta.seg_max = max([1] * (nd > 0) + lens)
-            meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W),
-                                           np.cumsum([b - a for a, b in ab]).tolist(), max(b - a for a, b in ab))
-                               for w, ab in seen.items()}
-            meta.row_ends = cu[1:].tolist()
+            if seen:
+                meta.row_ends = cu[1:].tolist()
+                meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W), end.tolist(), int((pages - first).max()))
+                                   for w, (first, end) in seen.items()}
         if kA:
             TA, S_ = int(cu[kA]), len(seqs)
             parts = []
