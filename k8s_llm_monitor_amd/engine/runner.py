@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass
+from itertools import accumulate
 from typing import Optional
 
 import numpy as np
@@ -202,22 +203,20 @@ class ModelRunner:
         # layout of the staging buffer (int32 words; the float sampling parameters bit-cast)
         nl = sum(len(x) for x in logit_rows) if logit_rows is not None else R
         hy = R if self.hybrid else 0
-        # latent attention: for every window of those layers the first page that each chunk sees through it and the pages up to its
-        # last token, one chunk after the other
+        # latent attention: for every window of those layers the first page that each chunk sees through it, how many it sees, and
+        # their sums chunk after chunk
         seen = {}
-        if hy and seqs and self.model.page_windows:
-            c0 = np.asarray(starts)
-            pages = (c0 + lens + BLOCK_SIZE - 1) // BLOCK_SIZE
-            for w in self.model.page_windows:
-                first = np.maximum(c0 - (w - 1), 0) // BLOCK_SIZE if w else np.zeros_like(c0)
-                seen[w] = first, np.cumsum(pages - first)
+        for w in self.model.page_windows if hy and seqs else ():
+            first = [max(0, c - w + 1) // BLOCK_SIZE if w else 0 for c in starts]
+            n = [(c + n + BLOCK_SIZE - 1) // BLOCK_SIZE - a for c, n, a in zip(starts, lens, first)]
+            seen[w] = first, n, list(accumulate(n))
         sizes = dict(ids=T, pos=T, slots=T, cu=len(seqs) + 1, qs=nq, st=nq, lidx=nl, temp=R, topk=R, topp=R,
                      gcu=hy + 1 if hy else 0, gctx=hy, gslot=hy,
                      cst=len(seqs) if paged else 0, bt=len(seqs) * W, dbt=nd * Wd, dlen=nd,
                      mcu=len(seqs) + 2 if kA else 0, mqs=nq if kA else 0, mst=nq if kA else 0,
                      mlidx=len(seqs) if kA else 0)
-        for w, (_, end) in seen.items():
-            sizes[f"pgl{w}"], sizes[f"pgb{w}"] = int(end[-1]), len(seqs) * W
+        for w, (_, _, ends) in seen.items():
+            sizes[f"pgl{w}"], sizes[f"pgb{w}"] = ends[-1], len(seqs) * W
         off, o = {}, 0
         for k, n in sizes.items():
             off[k] = o
@@ -264,11 +263,15 @@ class ModelRunner:
             bt2[:] = 0
             for i, s in enumerate(seqs):
                 bt2[i, : len(s.block_table)] = s.block_table
-            for w, (first, end) in seen.items():
-                a, b, e, col = first[:, None], pages[:, None], end[:, None], np.arange(W)
-                v[f"pgl{w}"][:] = bt2[(col >= a) & (col < b) if w else col < b]
-                at = np.minimum(col + (e - b), e - 1)  # (pages that are not seen get the number of one that is)
-                v[f"pgb{w}"].reshape(at.shape)[:] = np.maximum(at, e - b + a) if w else at
+            for w, (first, n, ends) in seen.items():
+                k, end, col = np.asarray(n)[:, None], np.asarray(ends)[:, None], np.arange(W)
+                if w:  # (pages that are not seen get the number of one that is)
+                    col = col - np.asarray(first)[:, None]
+                    v[f"pgl{w}"][:] = bt2[(col >= 0) & (col < k)]
+                    col = np.maximum(col, 0)
+                else:
+                    v[f"pgl{w}"][:] = bt2[col < k]
+                v[f"pgb{w}"].reshape(len(seqs), W)[:] = np.minimum(col + (end - k), end - 1)
         if nd:
             dbt = v["dbt"].reshape(nd, Wd)
             dbt[:] = 0
@@ -295,9 +298,9 @@ class ModelRunner:
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = dv["gcu"], dv["gctx"], dv["gslot"]
             meta.seg_max = max([1] * (nd > 0) + lens)
             if seen:
-                meta.row_ends = cu[1:].tolist()
-                meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W), end.tolist(), int((pages - first).max()))
-                                   for w, (first, end) in seen.items()}
+                meta.chunk_rows = cu
+                meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W), ends, max(n))
+                                   for w, (_, n, ends) in seen.items()}
         if kA:
             TA, S_ = int(cu[kA]), len(seqs)
             parts = []

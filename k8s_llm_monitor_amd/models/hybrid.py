@@ -273,6 +273,7 @@ class LatentAttention:
         self.fast = 1
         self.pitch = (self.R + self.dr + 31) // 32 * 32
         H, dn, dr, dv, Q, R = self.H, self.dn, self.dr, self.dv, self.Q, self.R
+        self.most_pages = self.EXPAND_BYTES // (2 * BLOCK * H * (dn + dr + dv))  # temporary pages (bf16 keys and values) at once
         wd = [p.get(prefix + "dq", (Q, d), 1.0 / math.sqrt(d))]
         self.kn = None
         if self.kv_from is None:
@@ -365,18 +366,15 @@ class LatentAttention:
                 and (self.dn + self.dr) in (64, 128) and self.dv in (64, 128)
                 and (meta.all_fresh or self._expand_pays(rows, meta.page_lists[self.window])))
 
-    def _page_bytes(self) -> int:
-        return 2 * BLOCK * self.H * (self.dn + self.dr + self.dv)  # a temporary page's keys and values
-
     def _expand_pays(self, rows: int, seen: PageList) -> bool:
-        return (seen.ends[-1] * BLOCK <= self.EXPAND_KEYS * rows and seen.longest * self._page_bytes() <= self.EXPAND_BYTES
+        return (seen.ends[-1] * BLOCK <= self.EXPAND_KEYS * rows and seen.longest <= self.most_pages
                 and (rows <= 128 or seen.longest * BLOCK <= 1024 + 1.5 * rows * self.H))
 
     def _expand_groups(self, seen: PageList) -> list:
         """[first, end) of consecutive chunks whose temporary pages are made together."""
-        most, cuts, held = self.EXPAND_BYTES // self._page_bytes(), [0], 0
+        cuts, held = [0], 0
         for i, end in enumerate(seen.ends):
-            if end - held > most and i > cuts[-1]:
+            if end - held > self.most_pages and i > cuts[-1]:
                 held = seen.ends[i - 1]
                 cuts.append(i)
         return list(zip(cuts, cuts[1:] + [len(seen.ends)]))
@@ -394,12 +392,11 @@ class LatentAttention:
             return hops.window_attention_prefill(q, kt, vt, cu, ctx, tables, H, H, dn + dr, dv, self.scale, self.window, self.sink,
                                                  mfma=self.fast, sinks=self.sinks, gate=gate)
 
-        groups = self._expand_groups(seen)
-        if len(groups) == 1:
+        if seen.ends[-1] <= self.most_pages:
             return attend(seen.pages, q, meta.cu_seqlens, meta.ctx_start, seen.tables, gate)
         out = []
-        for a, b in groups:  # (one group's pages are given back before the next one's are made)
-            r, p = ([0] + meta.row_ends)[a:b + 1:b - a], ([0] + seen.ends)[a:b + 1:b - a]
+        for a, b in self._expand_groups(seen):  # (one group's pages are given back before the next one's are made)
+            r, p = meta.chunk_rows[a:b + 1:b - a].tolist(), ([0] + seen.ends)[a:b + 1:b - a]
             out.append(attend(seen.pages[p[0]:p[1]], q[r[0]:r[1]], meta.cu_seqlens[a:b + 1] - r[0], meta.ctx_start[a:b],
                               seen.tables[a:b] - p[0], gate[r[0]:r[1]] if gate is not None else None))
         return torch.cat(out)

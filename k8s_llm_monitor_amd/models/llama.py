@@ -34,6 +34,7 @@ import os
 from dataclasses import dataclass
 from typing import NamedTuple, Optional
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
@@ -93,9 +94,9 @@ class AttnMeta:
     # prefill: every chunk of this step starts at position 0 (whole prompts, nothing cached before)
     all_fresh: bool = False
     # layer-list prefill, latent attention's expanded form: a PageList for each attention window of those layers (0: none),
-    # and the chunks' ends in rows (cu_seqlens from 1 on) for the host
+    # and cu_seqlens on the host
     page_lists: Optional[dict] = None
-    row_ends: Optional[list] = None
+    chunk_rows: Optional[np.ndarray] = None
 
 
 def _seed_for(name: str, seed: int) -> int:

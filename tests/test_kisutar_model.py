@@ -242,7 +242,7 @@ def test_form_of_latent_portions_by_sizes(heads, chunks, want):
     from k8s_llm_monitor_amd.models.llama import PageList
 
     m = LatentAttention.__new__(LatentAttention)
-    m.H, m.dn, m.dr, m.dv = heads, 96, 32, 128
+    m.H, m.most_pages = heads, (1 << 30) // (32 * heads * 256)
     pages = torch.tensor([(p + 15) // 16 for _, p in chunks])
     seen = PageList(None, None, pages.cumsum(0).tolist(), int(pages.max()))
     assert m._expand_pays(sum(n for n, _ in chunks), seen) is want
@@ -261,7 +261,8 @@ def test_expanded_steps_in_groups_of_bounded_pages(monkeypatch, most):
     cfg = make_cfg([lat(window=500), lat(2, 8, 4, 6, 12, 16, 190, 0.3, mlp=moe())])
     rig = rig_for(cfg, 6)
     for m in rig.model.mixers:
-        monkeypatch.setattr(m, "EXPAND_BYTES", most * m._page_bytes() + 1, raising=False)
+        assert m.most_pages * 32 * m.H * (m.dn + m.dr + m.dv) <= 1 << 30
+        m.most_pages = most
     seqs = {n: toks(k, cfg["vocab"], k) for n, k in (("a", 50), ("b", 33), ("c", 70), ("d", 9))}
     a = rig.step([("a", seqs["a"][:20]), ("b", seqs["b"][:33]), ("c", seqs["c"][:65]), ("d", seqs["d"][:8])], end=["b"])
     first = list(made)
