@@ -154,7 +154,7 @@ class WindowAttention:
             o = hops.window_attention_decode(qkv, kc, vc, meta.block_tables, meta.seq_lens, *args, vec=bool(self.fast))
         else:
             nd = meta.num_decode
-            # mfma 2: the register kernel.  The staged one (201 -> 87 us at 4 x 2048 rows, 16 heads) rounds the weights against
+            # mfma 2: the register kernel.  The staged one (201 -> 88 us at 4 x 2048 rows, 16 heads) rounds the weights against
             # another running maximum, and this design's routers - the softmax over the two best of near-equal logits - turn such
             # differences into other experts: recurrent states behind them moved by more than their root mean square.
             o = hops.window_attention_prefill(qkv[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,

@@ -746,7 +746,7 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
   }
   const int S = (int)ctx.numel();
   // prompts, or a long one beside single tokens (us, token by token -> chunks, delta rule / 32 heads of
-  // 64 x 64: one of 2000 rows beside 60 575 -> 186, 399 -> 181; one of 256 beside 60 142 -> 139, 125 -> 107)
+  // 64 x 64: one of 2000 rows beside 60 575 -> 147, 399 -> 91; one of 256 beside 60 142 -> 68, 125 -> 44)
   const bool prompts = T >= 32l * S || longest >= 256;
   const void* zp = (const char*)z.data_ptr() + z_col * z.element_size();
   TORCH_CHECK(singles >= 0 && singles <= S && singles <= T, "decay_scan: single tokens in front");
@@ -763,8 +763,8 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
   const long T1 = (long)(T - singles);
   if (!f && S1 > 0 && (mode >= 3 || (mode == 0 && prompts)) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 &&
       qkv.stride(0) % 8 == 0 && q_col % 8 == 0 && k_col % 8 == 0 && v_col % 8 == 0) {
-    // a chunk costs the same whatever it holds (us, 16 heads of 128 x 128, scan -> chunks: 40 segments of 33 rows 99 -> 101;
-    // 16 of 64 73 -> 51; one of 64 21 -> 28; 4 of 2048 542 -> 209)
+    // a chunk costs the same whatever it holds (us, 16 heads of 128 x 128, scan -> chunks: 40 segments of 33 rows 99 -> 105;
+    // 16 of 64 75 -> 55; one of 64 21 -> 27; 4 of 2048 544 -> 212)
     if (per_head && (mode == 3 || longest >= 256 || (T >= 64l * S && T >= 128))) {
       const long nb = k8sllm_hy_delta_chunk_ws(T1, S1, (int)H, (int)dk, (int)dv);
       if (nb > 0) {

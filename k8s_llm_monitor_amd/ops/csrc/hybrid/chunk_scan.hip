@@ -20,8 +20,8 @@
 // products run.
 // What bounds it: the chain of LDS round trips and two barriers per chunk (3.2 to 4.6 us a chunk and workgroup; the vector
 // instructions of the splits would take 1 us, the matrix instructions half of that).
-// Measured, bf16, 16 heads of 128 x 128: 5 x 1600 rows 125 us (the sequential scan 569; chunks whose fp32 products ran on the
-// fp32 matrix instruction 296), 1 x 8000 rows 403 us (2680; 1400).  Error against 64 bits, 1600 rows: outputs 1.4e-7 (scan
+// Measured, bf16, 16 heads of 128 x 128: 5 x 1600 rows 129 us (the sequential scan 314; chunks whose fp32 products ran on the
+// fp32 matrix instruction 296), 1 x 8000 rows 403 us (1068; 1400).  Error against 64 bits, 1600 rows: outputs 1.4e-7 (scan
 // 2.2e-7), state 1.3e-7 (2.2e-7).
 #include "chunk_seg.h"
 #include "split_bf16.h"
@@ -285,8 +285,8 @@ extern "C" int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* deca
   if (nt != 0 && nt != 1 && nt != 2 && nt != 4) return -1;
   if (nt > 1 && dv % (16 * nt)) return 1;
   // column blocks repeat the scores' products, so wide ones once they give enough workgroups to fill the chip; those of 32 columns
-  // only where 64 do not divide (us for 16 / 32 / 64 columns, 16 heads of 128 x 128: 5 x 1637 rows 179 / 153 / 121; 1 x 8000
-  // 382 / 567 / 526; 1000, 900, 800, 300 and three short 62 / 90 / 82; 2 x 2048 beside 32 single tokens 113 / 169 / 149).
+  // only where 64 do not divide (us for 16 / 32 / 64 columns, 16 heads of 128 x 128: 5 x 1600 rows 184 / 161 / 129; 1 x 8000
+  // 403 / 617 / 574; 1000, 900, 800, 300 and three short 62 / 90 / 82; 2 x 2048 beside 32 single tokens 113 / 169 / 149).
   // Segments count by the longest one's length (0: not known): single tokens beside it are a chunk each
   const long pairs = (longest > 0 ? min((long)S, (T + longest - 1) / longest) : S) * H;
   if (nt == 0) nt = dv % 64 == 0 ? (pairs * (dv / 64) >= 144 ? 4 : 1) : dv % 32 == 0 && pairs * (dv / 32) >= 192 ? 2 : 1;

@@ -18,8 +18,8 @@
 // What bounds it: the scan by the workspace's operands (72 KiB per chunk and head at 64 channels, read by every column block:
 // 1.2 us a chunk at the 25 bytes per clock that a CU draws from L2, where the products and the trip through LDS take 0.3);
 // the preparation by vector instructions.
-// Measured, both launches (us; the staged scan with its preparation), 32 heads of 64 x 64 with a bonus: 1 x 8000 rows 254
-// (1347), 4 x 2048 235 (428); plain, 16 heads of 128 x 128: 1 x 8000 436 (1548), 4 x 2048 407 (567).  Error against 64 bits, 2048
+// Measured, both launches (us; the staged scan with its preparation), 32 heads of 64 x 64 with a bonus: 1 x 8000 rows 259
+// (1347), 4 x 2048 240 (428); plain, 16 heads of 128 x 128: 1 x 8000 449 (1548), 4 x 2048 407 (567).  Error against 64 bits, 2048
 // rows, bonus: outputs 1.3e-7 (scan 2.7e-7), state 7.9e-8 (3.0e-7); plain: 2.3e-7 (1.5e-6), 2.1e-7 (2.0e-6).
 #include "chunk_seg.h"
 #include "split_bf16.h"
@@ -499,8 +499,8 @@ extern "C" {
 
 // Chunks per span of a step cut into spans, 0: whole segments.  Cut where long chains leave the chip idle - spans then take 64 columns
 // at once, a quarter of the operand traffic, and twice the state's products (us, whole / spans, 32 heads of 64 x 64: 1 x 8000 rows
-// 384 / 254, 1 x 2048 79 / 69, 2 x 4000 291 / 259, 4 x 2048, not cut, 239 / 241; 16 heads 1 x 8000 217 / 133; plain, 16 heads of
-// 128 x 128, 1 x 8000 605 / 436) - about 256 workgroups of them.
+// 420 / 259, 1 x 2048 86 / 72, 2 x 4000 305 / 259, 4 x 2048, not cut, 241 / 244; 16 heads 1 x 8000 242 / 133; plain, 16 heads of
+// 128 x 128, 1 x 8000 599 / 451) - about 256 workgroups of them.
 static int span_chunks(long T, int S, int longest, int H, int dv, int mode) {
   const long n = longest > 0 ? longest : S > 0 ? T / S : 0;
   const int cols = dv % 64 == 0 ? dv / 64 : dv % 32 == 0 ? dv / 32 : dv / 16;

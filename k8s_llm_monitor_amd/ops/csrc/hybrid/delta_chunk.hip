@@ -20,8 +20,8 @@
 // Sums of log2 g are kept in 64 bits: differences of large sums lose nothing.  Everything else is fp32.
 // What bounds it: the chain K S -> R -> N R -> S per chunk, two barriers long; the workspace's traffic (72 KiB per chunk and
 // head, read by every column block, at dk 128).
-// Measured, 16 heads of 128 x 128 on 8 key heads, both launches (us; the staged scan with its preparation): 1 x 8000 rows 399
-// (1604), 4 x 2048 209 (542), 8 heads, 13 x 500 110 (268).  Error against 64 bits at 4 x 2048: outputs 1.9e-7 (scan 3.0e-7),
+// Measured, 16 heads of 128 x 128 on 8 key heads, both launches (us; the staged scan with its preparation): 1 x 8000 rows 412
+// (1599), 4 x 2048 212 (544), 8 heads, 13 x 500 114 (267).  Error against 64 bits at 4 x 2048: outputs 1.9e-7 (scan 3.0e-7),
 // state 1.7e-7 (3.1e-7).
 #include "chunk_seg.h"
 #include "split_bf16.h"

@@ -634,8 +634,8 @@ constexpr float kMaxCapPlain = 60.f;
 // The LDS-staged kernel of window_flash.hip takes a step that has enough (row, head) pairs to fill the chip with its
 // 256 pairs per workgroup, or rows that may see enough keys for the shared tiles to pay with few workgroups.  Register
 // kernel at its better width -> staged kernel, us (128-wide heads): 13 prompts x 120, 8 heads (12480 pairs, 120 keys)
-// 9.2 -> 12.5; x 250 21.3 -> 16.6; x 500 52 -> 25; one prompt of 512, 8 heads 20.3 -> 21.7; 1024 38 -> 34; 64 rows
-// behind 2000 keys, 16 heads 70 -> 61.  mfma = kFlashForced asks for it at any size (tests, measurements), 2 for the
+// 9.5 -> 13.4; x 250 22.4 -> 17.7; x 500 52 -> 26; one prompt of 512, 8 heads 20.9 -> 22.2; 1024 39 -> 35; 64 rows
+// behind 2000 keys, 16 heads 72 -> 64.  mfma = kFlashForced asks for it at any size (tests, measurements), 2 for the
 // register kernel whatever the size.
 constexpr long kFlashPairs = 16 * 1024;
 constexpr long kFlashKeys = 1024;

@@ -11,8 +11,8 @@
 // softmax, and value columns past the last visible token (a page's unused end) count as zero.  An infinity or NaN among the
 // values reaches the queries that see its token and no others, as there: a page that only some of a wave's queries see whole is
 // looked through for one, and such values are added one by one (the matrix instruction would multiply them by the others' zeros).
-// Prompts of 2 x 2048 tokens, 16 heads on 4 of 128: 13.9 -> 0.44 ms; 3 prompts of 250 to 400, 8 heads on 2: 490 -> 74 us (host
-// work of the call included); decode of 2 sequences at 2048: 350 -> 30 us, of 8 at 301: 106 -> 14.  Distance to 64 bits 6.3e-7 ->
+// Prompts of 2 x 2048 tokens, 16 heads on 4 of 128: 13.9 -> 0.45 ms; 3 prompts of 250 to 400, 8 heads on 2: 488 -> 80 us (host
+// work of the call included); decode of 2 sequences at 2048: 351 -> 31 us, of 8 at 301: 107 -> 15.  Distance to 64 bits 6.3e-7 ->
 // 4.5e-7 (decode 7.1e-7 -> 3.2e-7).
 #include "chunk_seg.h"
 

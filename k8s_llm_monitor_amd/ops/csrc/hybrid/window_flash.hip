@@ -20,8 +20,9 @@
 //    tile in part, the 8-token pieces of V^T that none of them sees are read from zeros, and what lies behind the workgroup's last
 //    token (the last page's unused end) is cleared in LDS: a masked weight of zero would not take away a NaN.
 // Measured (us, 128-wide heads, register kernel -> this one): 4 x 2048 rows, 16 query heads on 4 kv heads, window 1024:
-// 201 -> 87 (596 TFLOP/s); 2 x 2000 rows behind 2816 cached ones: 403 -> 145 (861 TFLOP/s); one prompt of 8000: 982 -> 274
-// (957 TFLOP/s); the same in capped chunks of 1024: 122 -> 89 (three transcendental instructions per score bound it).
+// 201 -> 88 (586 TFLOP/s); 2 x 2000 rows behind 2816 cached ones: 399 -> 148 (843 TFLOP/s); one prompt of 8000: 977 -> 272
+// (962 TFLOP/s); the same in capped chunks of 1024: 122 -> 93 (three transcendental instructions per score bound it).  The zeros for
+// pieces that are not seen and the cleared page end are 1 to 3 of these us.
 #include "hy_common.h"
 
 namespace k8sllm {
