@@ -80,9 +80,11 @@ def test_latent_portions_in_the_expanded_form(monkeypatch):
     real = LatentAttention._forward_expanded
     monkeypatch.setattr(LatentAttention, "_forward_expanded", lambda self, *a: calls.append(1) or real(self, *a))
 
-    def run(min_rows):
+    def run(min_rows, most=None):
         monkeypatch.setattr(LatentAttention, "EXPAND_MIN_ROWS", min_rows)
         rig = B.rig_for(cfg, w=w, device="cuda", dtype=BF, num_blocks=48)
+        for m in rig.model.mixers:
+            m.most_pages = most or m.most_pages
         a = rig.step([("a", t[:90]), ("b", u[:119])])
         b = rig.step([("a", t[90:161]), ("b", u[119:])], end=["b"])  # a portion behind 90 cached tokens, a decode row
         c = rig.step([("a", t[161:])], end=["a"])
@@ -90,6 +92,9 @@ def test_latent_portions_in_the_expanded_form(monkeypatch):
 
     ga, gb = run(32)
     assert len(calls) == 6
+    ca, cb = run(32, 13)  # the first step's 6 and 8 pages in two groups; the cached sequence has 11, then 13
+    assert len(calls) == 12
+    assert torch.equal(ca, ga) and torch.equal(cb, gb)
     ha, hb = run(1 << 30)
     for got, form, ref in ((ga, ha, O.forward(cfg, w, t)), (gb, hb, O.forward(cfg, w, u))):
         B.close_most(got, ref, 0.05, frac=1.0)
