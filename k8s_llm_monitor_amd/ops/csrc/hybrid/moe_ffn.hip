@@ -16,7 +16,9 @@
 //                 relu(W A)^2.  64 x 64 tiles, fp32 accumulation.
 //   moe_combine   out[t] = sum_k w[t][k] Y[inv[t*K + k]] + gate[t] * shared[t]   (fp32; no gate: 1); a chosen id
 //                 >= n_real is an identity expert, its Y is the layer's input h[t]
-#include "hy_common.h"
+#include "stream_rows.h"
+
+#include <algorithm>
 
 namespace k8sllm {
 
@@ -556,78 +558,73 @@ __global__ __launch_bounds__(256, 2) void hy_grouped_gemm_f32_kernel(float* __re
   }
 }
 
-// bf16 on the matrix cores (K a multiple of 32): one wave = 16 MT sorted rows of one expert x 16 NT output columns,
+// What an activation makes of a row's product (and, gated, of the up projection's), both rounded to bf16 first
+template <int ACT>
+__device__ __forceinline__ bf16_t expert_unit(float v, float u, float limit) {
+  if (ACT == 3) v = clamped_unit_f(bf2f(f2bf(v)), bf2f(f2bf(u)), limit);
+  else if (ACT == 1) v = silu_f(bf2f(f2bf(v))) * bf2f(f2bf(u));
+  else if (ACT == 2) v = gelu_erf_f(bf2f(f2bf(v)));
+  else if (ACT == 4) v = relu_sq_f(bf2f(f2bf(v)));
+  return f2bf(v);
+}
+
+// bf16, many rows (K a multiple of 32): one wave = 16 sorted rows of one expert x 64 output columns,
 // v_mfma_f32_16x16x32_bf16 with both operands loaded straight from global memory as 16-byte fragments (A = the gathered
-// activation rows, B = weight rows, 8 consecutive k per lane), batches of them in flight while the last is multiplied.  Few rows
-// per expert (decode) make this a weight-streaming kernel: many small workgroups, no LDS, NT = 1 so that the stream is spread over
-// as many waves as there are columns, and MT so that the rows of an expert share one pass over its weights (a second row
-// tile lands on another XCD and reads them again).  With more rows NT = 4, MT = 1.  Every output is one chain of products in the
-// order of k, whatever the tile.
-// 128 rows over 8 experts, K = N = 2048, gated / plain: 54.5 / 34.3 us with 16 rows a wave and a wait per batch, 36.1 / 20.3 now
-// (3.7 and 3.3 TB/s of weights); widths 4096 x 3584: 194 / 101 and 110 / 68.
+// activation rows, B = weight rows, 8 consecutive k per lane), a batch of them in flight while the last is multiplied.  Every
+// output is one chain of products in the order of k.
 // ``il``: the gate / up rows are interleaved per 128 rows as [64 gate | 64 up] (the prefill tile
 // GEMM's pairing), else [all gate rows ; all up rows].
-template <int ACT, int NT, int MT>
+template <int ACT>
 __global__ __launch_bounds__(64) void hy_grouped_gemm_mfma_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ A,
                                                                   const bf16_t* __restrict__ W,
                                                                   const int* __restrict__ offsets,
                                                                   const int* __restrict__ sorted_idx, int div, int E,
                                                                   int N, int Kd, long w_es, int il, float limit) {
-  constexpr bool SWIGLU = ACT == 1 || ACT == 3;  // gated: gate rows and up rows
+  constexpr bool GATED = ACT == 1 || ACT == 3;  // gate rows and up rows
+  constexpr int NT = 4;
   int e = 0, tile = blockIdx.x, r0 = 0, r1 = 0;
   for (; e < E; ++e) {
     r0 = offsets[e];
     r1 = offsets[e + 1];
-    const int nt = (r1 - r0 + 16 * MT - 1) / (16 * MT);
+    const int nt = (r1 - r0 + 15) / 16;
     if (tile < nt) break;
     tile -= nt;
   }
   if (e >= E) return;
-  r0 += tile * (16 * MT);
+  r0 += tile * 16;
   const int lane = threadIdx.x, c16 = lane & 15, quad = lane >> 4;
   const int n0 = blockIdx.y * (16 * NT);
   const bf16_t* We = W + (long)e * w_es;
-  const bf16_t* ap[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int arow = min(r0 + 16 * m + c16, r1 - 1);
-    ap[m] = A + (long)(sorted_idx != nullptr ? sorted_idx[arow] / div : arow) * Kd + 8 * quad;
-  }
+  const int arow = min(r0 + c16, r1 - 1);
+  const bf16_t* ap = A + (long)(sorted_idx != nullptr ? sorted_idx[arow] / div : arow) * Kd + 8 * quad;
   const bf16_t* wg[NT];
   const bf16_t* wu[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int n = min(n0 + 16 * t + c16, N - 1);
-    const long g = SWIGLU && il ? (long)(n >> 6) * 128 + (n & 63) : n;
+    const long g = GATED && il ? (long)(n >> 6) * 128 + (n & 63) : n;
     wg[t] = We + g * Kd + 8 * quad;
-    wu[t] = We + (SWIGLU ? (il ? g + 64 : (long)N + n) : 0) * Kd + 8 * quad;
+    wu[t] = We + (GATED ? (il ? g + 64 : (long)N + n) : 0) * Kd + 8 * quad;
   }
-  f32x4 acc[MT][NT], accu[MT][NT];
+  f32x4 acc[NT] = {}, accu[NT] = {};
+  auto step = [&](const bf16x8& a, const bf16x8 (&w)[NT], const bf16x8 (&u)[NT]) {
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[m][t] = accu[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](const bf16x8 (&a)[MT], const bf16x8 (&w)[NT], const bf16x8 (&u)[NT]) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], w[t], acc[m][t], 0, 0, 0);
-        if (SWIGLU) accu[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], u[t], accu[m][t], 0, 0, 0);
-      }
+    for (int t = 0; t < NT; ++t) {
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[t], acc[t], 0, 0, 0);
+      if (GATED) accu[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, u[t], accu[t], 0, 0, 0);
+    }
   };
-  auto load = [&](bf16x8 (&a)[MT], bf16x8 (&w)[NT], bf16x8 (&u)[NT], int k0) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const bf16x8*>(ap[m] + k0);
+  auto load = [&](bf16x8& a, bf16x8 (&w)[NT], bf16x8 (&u)[NT], int k0) {
+    a = *reinterpret_cast<const bf16x8*>(ap + k0);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       w[t] = *reinterpret_cast<const bf16x8*>(wg[t] + k0);
-      if (SWIGLU) u[t] = *reinterpret_cast<const bf16x8*>(wu[t] + k0);
+      if (GATED) u[t] = *reinterpret_cast<const bf16x8*>(wu[t] + k0);
     }
   };
   // batches of U steps of 32 k: the next one is fetched while one is multiplied
-  constexpr int U = NT > 1 ? 2 : SWIGLU || MT > 2 ? 4 : 8;
-  bf16x8 a[2][U][MT], w[2][U][NT], u[2][U][NT];
+  constexpr int U = 2;
+  bf16x8 a[2][U], w[2][U][NT], u[2][U][NT];
   const int nb = Kd / (32 * U);
   if (nb > 0)
 #pragma unroll
@@ -649,22 +646,61 @@ __global__ __launch_bounds__(64) void hy_grouped_gemm_mfma_kernel(bf16_t* __rest
     step(a[0][0], w[0][0], u[0][0]);
   }
 #pragma unroll
+  for (int t = 0; t < NT; ++t) {  // acc[t][i]: row r0 + 4 quad + i, column n0 + 16 t + c16
+    const int n = n0 + 16 * t + c16;
+    if (n >= N) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = r0 + 4 * quad + i;
+      if (r < r1) Y[(long)r * N + n] = expert_unit<ACT>(acc[t][i], accu[t][i], limit);
+    }
+  }
+}
+
+// The same for the few rows of a decode step (A and W 16-byte aligned): a pass over the chosen experts' weights, bound by how much
+// of them is in flight.  A workgroup takes 16 MT rows of one expert and 16 columns a wave; rows and weights come through LDS
+// (stream_rows.h has why).  The same chains of products, so the same bits.
+// us, gated / plain, 8 experts, with register loads and here: 2048 x 2048, 128 rows 39.9 / 24.0, 33.5 / 16.8 (4.0 TB/s); 2 rows 21.6 /
+// 11.5, 10.3 / 7.9; 512 rows 92.6 / 73.8, 44.9 / 25.5; 4096 x 3584, 128 rows 132 / 77, 96 / 44 (4.9 and 5.3 TB/s).
+template <int ACT, int MT, int NW>
+__global__ __launch_bounds__(64 * NW) void hy_grouped_gemm_few_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ A,
+                                                                      const bf16_t* __restrict__ W,
+                                                                      const int* __restrict__ offsets,
+                                                                      const int* __restrict__ sorted_idx, int div, int E,
+                                                                      int N, int Kd, long w_es, int il, float limit) {
+  constexpr bool GATED = ACT == 1 || ACT == 3;
+  constexpr int NS = GATED ? 2 : 1;
+  using S = SharedRows<MT, NS, NW>;
+  __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
+  int e = 0, tile = blockIdx.y, r0 = 0, r1 = 0;
+  for (; e < E; ++e) {
+    r0 = offsets[e];
+    r1 = offsets[e + 1];
+    const int nt = (r1 - r0 + 16 * MT - 1) / (16 * MT);
+    if (tile < nt) break;
+    tile -= nt;
+  }
+  if (e >= E) return;
+  r0 += tile * (16 * MT);
+  const int n0 = (blockIdx.x * NW + (threadIdx.x >> 6)) * 16, nw = min(n0 + piece_row(), N - 1);
+  const bf16_t* We = W + (long)e * w_es + piece_k();
+  const long gate = GATED && il ? (long)(nw >> 6) * 128 + (nw & 63) : nw;
+  const bf16_t* w[NS];
+  w[0] = We + gate * Kd;
+  if (GATED) w[NS - 1] = We + (il ? gate + 64 : (long)N + nw) * Kd;
+  f32x4 acc[MT][NS] = {};
+  S::run(smem, [&](int m) {
+    const int r = min(r0 + 16 * m + piece_row(), r1 - 1);
+    return A + (long)(sorted_idx != nullptr ? sorted_idx[r] / div : r) * Kd + piece_k();
+  }, w, Kd / 32, acc);
+  const int n = n0 + (threadIdx.x & 15), quad = (threadIdx.x & 63) >> 4;
+  if (n >= N) return;
+#pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {  // acc[m][t][i]: row r0 + 16 m + 4 quad + i, column n0 + 16 t + c16
-      const int n = n0 + 16 * t + c16;
-      if (n >= N) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = r0 + 16 * m + 4 * quad + i;
-        if (r >= r1) continue;
-        float v = acc[m][t][i];
-        if (ACT == 3) v = clamped_unit_f(bf2f(f2bf(v)), bf2f(f2bf(accu[m][t][i])), limit);
-        else if (SWIGLU) v = silu_f(bf2f(f2bf(v))) * bf2f(f2bf(accu[m][t][i]));
-        else if (ACT == 2) v = gelu_erf_f(bf2f(f2bf(v)));
-        else if (ACT == 4) v = relu_sq_f(bf2f(f2bf(v)));
-        Y[(long)r * N + n] = f2bf(v);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int r = r0 + 16 * m + 4 * quad + i;
+      if (r < r1) Y[(long)r * N + n] = expert_unit<ACT>(acc[m][0][i], acc[m][NS - 1][i], limit);
     }
 }
 
@@ -773,26 +809,42 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
   const bool swiglu = act == 1;
   if (il && (!swiglu || N % 64)) return -1;
   if (!f32 && mfma && Kd % 32 == 0) {
-    const bool few = rows <= 512;  // a decode-sized step: one n-tile per wave
-    // a wave takes 16, 32 or 64 rows of an expert, so that its weights are mostly read once: by the mean number of rows an expert
-    // gets (K = N = 2048, 8 experts, gated + plain: mean 6 55 / 53 us with 16 / 32 rows, 16 81 / 56, 32 113 / 105 and 64 rows 80;
-    // 64 experts, mean 8: 175 / 178)
-    const int mt = !few || rows <= 8l * E ? 1 : rows <= 24l * E ? 2 : 4;
-    const dim3 g16((unsigned)(rows / (16 * mt) + E), (unsigned)(few ? (N + 15) / 16 : (N + 63) / 64));
-#define K8SLLM_GM(SW, NT, MT)                                                                                        \
-  hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<SW, NT, MT>), g16, dim3(64), 0, s, (bf16_t*)Y, (const bf16_t*)A,      \
+    const bool few = rows <= 512 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;  // a decode-sized step
+    if (few) {
+      // a workgroup takes 16, 32 or 64 rows of an expert, so that its weights are mostly read once, by the mean number of rows an
+      // expert gets (8 experts, 2048 x 2048, gated + plain: mean 16 60.0 / 50.3 / 51.9 us with 16 / 32 / 64 rows, 32 68.6 / 64.1 / 52.4;
+      // 32 experts, mean 8: 156.8 / 177.4), and four waves where that leaves every CU a workgroup (1024 x 1024, 8 experts: 14.8 / 18.0
+      // with one / four waves at 16 rows each, 16.4 / 19.9 with two / four at 32; 2048 x 2048 47.5 / 48.5, 51.3 / 50.3)
+      const int mt = rows <= 8l * E ? 1 : rows <= 24l * E ? 2 : 4;
+      const bool wide = std::min<long>(rows, E) * ((N + 63) / 64) >= 256;
+      const int nw = wide || mt == 4 ? 4 : mt;
+      const dim3 g((unsigned)((N + 16 * nw - 1) / (16 * nw)), (unsigned)(rows / (16 * mt) + E));
+#define K8SLLM_GX(ACT, MT, NW)                                                                                            \
+  hipLaunchKernelGGL((hy_grouped_gemm_few_kernel<ACT, MT, NW>), g, dim3(64 * NW), 0, s, (bf16_t*)Y, (const bf16_t*)A,        \
                      (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)
-#define K8SLLM_GMS(SW)                  \
-  if (!few) K8SLLM_GM(SW, 4, 1);        \
-  else if (mt == 1) K8SLLM_GM(SW, 1, 1); \
-  else if (mt == 2) K8SLLM_GM(SW, 1, 2); \
-  else K8SLLM_GM(SW, 1, 4)
-    if (swiglu) { K8SLLM_GMS(1); }
-    else if (act == 3) { K8SLLM_GMS(3); }
-    else if (act == 2) { K8SLLM_GMS(2); }
-    else if (act == 4) { K8SLLM_GMS(4); }
-    else { K8SLLM_GMS(0); }
-#undef K8SLLM_GMS
+#define K8SLLM_GXS(ACT)                                                          \
+  if (mt == 4) K8SLLM_GX(ACT, 4, 4);                                             \
+  else if (mt == 2) { if (nw == 4) K8SLLM_GX(ACT, 2, 4); else K8SLLM_GX(ACT, 2, 2); } \
+  else if (nw == 4) K8SLLM_GX(ACT, 1, 4);                                        \
+  else K8SLLM_GX(ACT, 1, 1)
+      if (act == 1) { K8SLLM_GXS(1); }
+      else if (act == 3) { K8SLLM_GXS(3); }
+      else if (act == 2) { K8SLLM_GXS(2); }
+      else if (act == 4) { K8SLLM_GXS(4); }
+      else { K8SLLM_GXS(0); }
+#undef K8SLLM_GXS
+#undef K8SLLM_GX
+      return (int)hipGetLastError();
+    }
+    const dim3 g16((unsigned)(rows / 16 + E), (unsigned)((N + 63) / 64));
+#define K8SLLM_GM(ACT)                                                                                               \
+  hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<ACT>), g16, dim3(64), 0, s, (bf16_t*)Y, (const bf16_t*)A,             \
+                     (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)
+    if (act == 1) K8SLLM_GM(1);
+    else if (act == 3) K8SLLM_GM(3);
+    else if (act == 2) K8SLLM_GM(2);
+    else if (act == 4) K8SLLM_GM(4);
+    else K8SLLM_GM(0);
 #undef K8SLLM_GM
     return (int)hipGetLastError();
   }

@@ -349,6 +349,26 @@ def test_grouped_gemm_rows_per_wave(rows, N, Kd, act):
     torch.testing.assert_close(res[0].float(), want, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("rows,N", [(3, 40), (3, 8200), (33, 72), (33, 8200), (130, 136)])  # 16 rows by 1 and 4 waves, 32 by 2 and 4, 64 by 4
+@pytest.mark.parametrize("Kd", [32, 256, 288, 1056])  # one step, a whole chunk of 8, a chunk and a rest, four chunks and a rest
+@pytest.mark.parametrize("act,il", [(0, False), (1, False), (1, True)])
+def test_grouped_gemm_few_rows_keeps_the_bits(rows, N, Kd, act, il):
+    """Experts' products of a decode step (rows gathered by index) against the register kernel that takes over above 512 rows: both are
+    one chain of products in the order of k."""
+    if il:
+        N = N // 64 * 64 or 64
+    g = _g(75)
+    more = 520
+    a = _r(g, rows + more, Kd, dt=BF).cuda()
+    w = _r(g, 3, N * (2 if act else 1), Kd, s=Kd ** -0.5, dt=BF).cuda()
+    perm = torch.cat([torch.randperm(rows, generator=g), torch.arange(rows, rows + more)]).int().cuda()
+    ext, off = hops.native(), [0, rows // 3, rows]
+    few, many = (torch.empty(n, N, dtype=BF, device="cuda") for n in (rows, rows + more))
+    ext.grouped_gemm(few, a[:rows], w[:2].contiguous(), _i32(off).cuda(), perm[:rows].contiguous(), 1, act, il, True, 0.0)
+    ext.grouped_gemm(many, a, w, _i32(off + [rows + more]).cuda(), perm, 1, act, il, True, 0.0)
+    assert torch.equal(few, many[:rows])
+
+
 @pytest.mark.parametrize("M", [1, 2, 15, 16, 17])
 @pytest.mark.parametrize("N,K", [(16, 32), (1, 96), (200, 512), (72, 2080), (1024, 4096), (24, 4128)])
 def test_linear_of_few_rows(M, N, K):
