@@ -568,102 +568,17 @@ __device__ __forceinline__ bf16_t expert_unit(float v, float u, float limit) {
   return f2bf(v);
 }
 
-// bf16, many rows (K a multiple of 32): one wave = 16 sorted rows of one expert x 64 output columns,
-// v_mfma_f32_16x16x32_bf16 with both operands loaded straight from global memory as 16-byte fragments (A = the gathered
-// activation rows, B = weight rows, 8 consecutive k per lane), a batch of them in flight while the last is multiplied.  Every
-// output is one chain of products in the order of k.
+// bf16 on the matrix cores (K a multiple of 32, A and W 16-byte aligned).  Few rows per expert (decode) make this a pass over the
+// chosen experts' weights, bound by how much of them is in flight.  A workgroup takes 16 MT sorted rows of one expert, gathered on
+// load, and 16 columns a wave; rows and weights come through LDS (stream_rows.h has why).  Every output is one chain of products in the
+// order of k, whatever the tile.
+// us, gated / plain, 8 experts, with both operands loaded into registers and here: 2048 x 2048, 128 rows 35.8 / 21.4, 34.5 / 17.2
+// (3.9 TB/s); 2 rows 19.9 / 12.6, 9.4 / 7.2; 800 rows 144 / 77, 47 / 28; 2000 rows 258 / 144, 87 / 57; 4096 x 3584, 128 rows 111 / 69,
+// 105 / 44 (4.5 and 5.4 TB/s); 2000 rows 951 / 521, 240 / 158.
 // ``il``: the gate / up rows are interleaved per 128 rows as [64 gate | 64 up] (the prefill tile
 // GEMM's pairing), else [all gate rows ; all up rows].
-template <int ACT>
-__global__ __launch_bounds__(64) void hy_grouped_gemm_mfma_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ A,
-                                                                  const bf16_t* __restrict__ W,
-                                                                  const int* __restrict__ offsets,
-                                                                  const int* __restrict__ sorted_idx, int div, int E,
-                                                                  int N, int Kd, long w_es, int il, float limit) {
-  constexpr bool GATED = ACT == 1 || ACT == 3;  // gate rows and up rows
-  constexpr int NT = 4;
-  int e = 0, tile = blockIdx.x, r0 = 0, r1 = 0;
-  for (; e < E; ++e) {
-    r0 = offsets[e];
-    r1 = offsets[e + 1];
-    const int nt = (r1 - r0 + 15) / 16;
-    if (tile < nt) break;
-    tile -= nt;
-  }
-  if (e >= E) return;
-  r0 += tile * 16;
-  const int lane = threadIdx.x, c16 = lane & 15, quad = lane >> 4;
-  const int n0 = blockIdx.y * (16 * NT);
-  const bf16_t* We = W + (long)e * w_es;
-  const int arow = min(r0 + c16, r1 - 1);
-  const bf16_t* ap = A + (long)(sorted_idx != nullptr ? sorted_idx[arow] / div : arow) * Kd + 8 * quad;
-  const bf16_t* wg[NT];
-  const bf16_t* wu[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int n = min(n0 + 16 * t + c16, N - 1);
-    const long g = GATED && il ? (long)(n >> 6) * 128 + (n & 63) : n;
-    wg[t] = We + g * Kd + 8 * quad;
-    wu[t] = We + (GATED ? (il ? g + 64 : (long)N + n) : 0) * Kd + 8 * quad;
-  }
-  f32x4 acc[NT] = {}, accu[NT] = {};
-  auto step = [&](const bf16x8& a, const bf16x8 (&w)[NT], const bf16x8 (&u)[NT]) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[t], acc[t], 0, 0, 0);
-      if (GATED) accu[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, u[t], accu[t], 0, 0, 0);
-    }
-  };
-  auto load = [&](bf16x8& a, bf16x8 (&w)[NT], bf16x8 (&u)[NT], int k0) {
-    a = *reinterpret_cast<const bf16x8*>(ap + k0);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      w[t] = *reinterpret_cast<const bf16x8*>(wg[t] + k0);
-      if (GATED) u[t] = *reinterpret_cast<const bf16x8*>(wu[t] + k0);
-    }
-  };
-  // batches of U steps of 32 k: the next one is fetched while one is multiplied
-  constexpr int U = 2;
-  bf16x8 a[2][U], w[2][U][NT], u[2][U][NT];
-  const int nb = Kd / (32 * U);
-  if (nb > 0)
-#pragma unroll
-    for (int i = 0; i < U; ++i) load(a[0][i], w[0][i], u[0][i], 32 * i);
-  for (int k = 0; k < nb; k += 2) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (k + h >= nb) break;
-      if (k + h + 1 < nb)
-#pragma unroll
-        for (int i = 0; i < U; ++i) load(a[h ^ 1][i], w[h ^ 1][i], u[h ^ 1][i], 32 * ((k + h + 1) * U + i));
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < U; ++i) step(a[h][i], w[h][i], u[h][i]);
-    }
-  }
-  for (int k0 = nb * 32 * U; k0 < Kd; k0 += 32) {
-    load(a[0][0], w[0][0], u[0][0], k0);
-    step(a[0][0], w[0][0], u[0][0]);
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {  // acc[t][i]: row r0 + 4 quad + i, column n0 + 16 t + c16
-    const int n = n0 + 16 * t + c16;
-    if (n >= N) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = r0 + 4 * quad + i;
-      if (r < r1) Y[(long)r * N + n] = expert_unit<ACT>(acc[t][i], accu[t][i], limit);
-    }
-  }
-}
-
-// The same for the few rows of a decode step (A and W 16-byte aligned): a pass over the chosen experts' weights, bound by how much
-// of them is in flight.  A workgroup takes 16 MT rows of one expert and 16 columns a wave; rows and weights come through LDS
-// (stream_rows.h has why).  The same chains of products, so the same bits.
-// us, gated / plain, 8 experts, with register loads and here: 2048 x 2048, 128 rows 39.9 / 24.0, 33.5 / 16.8 (4.0 TB/s); 2 rows 21.6 /
-// 11.5, 10.3 / 7.9; 512 rows 92.6 / 73.8, 44.9 / 25.5; 4096 x 3584, 128 rows 132 / 77, 96 / 44 (4.9 and 5.3 TB/s).
 template <int ACT, int MT, int NW>
-__global__ __launch_bounds__(64 * NW) void hy_grouped_gemm_few_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ A,
+__global__ __launch_bounds__(64 * NW) void hy_grouped_gemm_mfma_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ A,
                                                                       const bf16_t* __restrict__ W,
                                                                       const int* __restrict__ offsets,
                                                                       const int* __restrict__ sorted_idx, int div, int E,
@@ -808,49 +723,42 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
   if (act < 0 || act > 4) return -1;
   const bool swiglu = act == 1;
   if (il && (!swiglu || N % 64)) return -1;
-  if (!f32 && mfma && Kd % 32 == 0) {
-    const bool few = rows <= 512 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;  // a decode-sized step
-    if (few) {
-      // a workgroup takes 16, 32 or 64 rows of an expert, so that its weights are mostly read once, by the mean number of rows an
-      // expert gets (8 experts, 2048 x 2048, gated + plain: mean 16 60.0 / 50.3 / 51.9 us with 16 / 32 / 64 rows, 32 68.6 / 64.1 / 52.4;
-      // 32 experts, mean 8: 156.8 / 177.4), and four waves where that leaves every CU a workgroup (1024 x 1024, 8 experts: 14.8 / 18.0
-      // with one / four waves at 16 rows each, 16.4 / 19.9 with two / four at 32; 2048 x 2048 47.5 / 48.5, 51.3 / 50.3)
-      const int mt = rows <= 8l * E ? 1 : rows <= 24l * E ? 2 : 4;
-      const bool wide = std::min<long>(rows, E) * ((N + 63) / 64) >= 256;
-      const int nw = wide || mt == 4 ? 4 : mt;
-      const dim3 g((unsigned)((N + 16 * nw - 1) / (16 * nw)), (unsigned)(rows / (16 * mt) + E));
-#define K8SLLM_GX(ACT, MT, NW)                                                                                            \
-  hipLaunchKernelGGL((hy_grouped_gemm_few_kernel<ACT, MT, NW>), g, dim3(64 * NW), 0, s, (bf16_t*)Y, (const bf16_t*)A,        \
+  const bool aligned = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
+  if (!f32 && mfma && Kd % 32 == 0 && aligned) {
+    // a workgroup takes 16, 32 or 64 rows of an expert, so that its weights are mostly read once, by the mean number of rows an
+    // expert gets (8 experts, 2048 x 2048, gated + plain: mean 16 60 / 50 / 52 us with 16 / 32 / 64 rows, 32 69 / 64 / 52; 32 experts,
+    // mean 8: 157 / 177).  Two waves or, for 64 rows and where plain columns fill the chip, four (gated, two / four: 4096 x 3584, 8
+    // rows 70 / 93, 32 rows 91 / 96, 128 rows 105 / 109; plain, 128 rows 50 / 44; 2048 x 2048, 512 rows 48 + 32 / 47 + 27).
+    const bool gated = act == 1 || act == 3;
+    const int mt = rows <= 8l * E ? 1 : rows <= 24l * E ? 2 : 4;
+    const int nw = mt == 4 || (!gated && std::min<long>(rows, E) * ((N + 63) / 64) >= 256) ? 4 : 2;
+    const dim3 g((unsigned)((N + 16 * nw - 1) / (16 * nw)), (unsigned)(rows / (16 * mt) + E));
+#define K8SLLM_GM(ACT, MT, NW)                                                                                       \
+  hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<ACT, MT, NW>), g, dim3(64 * NW), 0, s, (bf16_t*)Y, (const bf16_t*)A,  \
                      (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)
-#define K8SLLM_GXS(ACT)                                                          \
-  if (mt == 4) K8SLLM_GX(ACT, 4, 4);                                             \
-  else if (mt == 2) { if (nw == 4) K8SLLM_GX(ACT, 2, 4); else K8SLLM_GX(ACT, 2, 2); } \
-  else if (nw == 4) K8SLLM_GX(ACT, 1, 4);                                        \
-  else K8SLLM_GX(ACT, 1, 1)
-      if (act == 1) { K8SLLM_GXS(1); }
-      else if (act == 3) { K8SLLM_GXS(3); }
-      else if (act == 2) { K8SLLM_GXS(2); }
-      else if (act == 4) { K8SLLM_GXS(4); }
-      else { K8SLLM_GXS(0); }
-#undef K8SLLM_GXS
-#undef K8SLLM_GX
-      return (int)hipGetLastError();
-    }
-    const dim3 g16((unsigned)(rows / 16 + E), (unsigned)((N + 63) / 64));
-#define K8SLLM_GM(ACT)                                                                                               \
-  hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<ACT>), g16, dim3(64), 0, s, (bf16_t*)Y, (const bf16_t*)A,             \
-                     (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)
-    if (act == 1) K8SLLM_GM(1);
-    else if (act == 3) K8SLLM_GM(3);
-    else if (act == 2) K8SLLM_GM(2);
-    else if (act == 4) K8SLLM_GM(4);
-    else K8SLLM_GM(0);
+#define K8SLLM_GMP(ACT)                                 \
+  if (mt == 4) K8SLLM_GM(ACT, 4, 4);                    \
+  else if (mt == 2 && nw == 4) K8SLLM_GM(ACT, 2, 4);    \
+  else if (mt == 2) K8SLLM_GM(ACT, 2, 2);               \
+  else if (nw == 4) K8SLLM_GM(ACT, 1, 4);               \
+  else K8SLLM_GM(ACT, 1, 2)
+#define K8SLLM_GMG(ACT)                \
+  if (mt == 4) K8SLLM_GM(ACT, 4, 4);   \
+  else if (mt == 2) K8SLLM_GM(ACT, 2, 2); \
+  else K8SLLM_GM(ACT, 1, 2)
+    if (act == 1) { K8SLLM_GMG(1); }
+    else if (act == 3) { K8SLLM_GMG(3); }
+    else if (act == 2) { K8SLLM_GMP(2); }
+    else if (act == 4) { K8SLLM_GMP(4); }
+    else { K8SLLM_GMP(0); }
+#undef K8SLLM_GMG
+#undef K8SLLM_GMP
 #undef K8SLLM_GM
     return (int)hipGetLastError();
   }
   const dim3 grid((unsigned)(rows / TM + E), (unsigned)((N + TN - 1) / TN));
-  // other K and alignments (and bf16 whose K is no multiple of 32) stay on the vector unit
-  if (f32 && Kd % 32 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0) {
+  // other K and alignments stay on the vector unit
+  if (f32 && Kd % 32 == 0 && aligned) {
 #define K8SLLM_GF(ACT)                                                                                             \
   hipLaunchKernelGGL((hy_grouped_gemm_f32_kernel<ACT>), dim3(grid.y, grid.x), dim3(256), 0, s, (float*)Y, (const float*)A, \
                      (const float*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)

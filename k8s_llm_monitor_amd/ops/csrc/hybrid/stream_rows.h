@@ -32,25 +32,22 @@ __device__ __forceinline__ void loads_left() {  // waits until at most N of this
 template <int MT, int NS, int NW>
 struct SharedRows {
   static constexpr int D = 8;  // steps of a chunk, and of the weights' ring
-  // pieces of a chunk that a wave brings: all of one row tile (MT <= NW), or of every NW-th one
   static constexpr int SLOT = D * MT * 1024, RING = D * NS * 1024, BYTES = 2 * SLOT + NW * RING;
-  static constexpr int TPW = MT > NW ? MT / NW : 1, KSTEP = MT > NW ? 1 : NW / MT, PER = D * MT / NW;
-  static_assert(MT > NW ? MT % NW == 0 : NW % MT == 0, "");
+  static constexpr int PER = D * MT / NW;  // pieces of a chunk that a wave brings, all of one row tile
+  static_assert(NW % MT == 0, "");
 
   // x(m): this lane's source in row tile m of the rows; w[t]: in weight tile t; nk: steps
   template <class X>
   static __device__ __forceinline__ void run(char* lds, X x, const bf16_t* const (&w)[NS], int nk, f32x4 (&acc)[MT][NS]) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rd = piece_frag();
-    const int m0 = wave % MT, k0 = MT > NW ? 0 : wave / MT;
+    const int m0 = wave % MT, k0 = wave / MT;
+    const bf16_t* xs = x(m0);
     char* ring = lds + 2 * SLOT + wave * RING;
-    const bf16_t* xs[TPW];
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) xs[i] = x(m0 + i * NW);
     auto stage = [&](int c) {  // steps past the last repeat it; nothing multiplies them
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
-        const int ks = k0 + (i / TPW) * KSTEP, m = m0 + (i % TPW) * NW;
-        load_piece(lds + (c & 1) * SLOT + (ks * MT + m) * 1024, xs[i % TPW] + 32 * min(c * D + ks, nk - 1));
+        const int ks = k0 + i * (NW / MT);
+        load_piece(lds + (c & 1) * SLOT + (ks * MT + m0) * 1024, xs + 32 * min(c * D + ks, nk - 1));
       }
     };
     auto refill = [&](int d, int k) {

@@ -4,6 +4,7 @@ import math
 
 import pytest
 import torch
+import torch.nn.functional as F
 
 from k8s_llm_monitor_amd.ops import hybrid as hops
 
@@ -349,12 +350,13 @@ def test_grouped_gemm_rows_per_wave(rows, N, Kd, act):
     torch.testing.assert_close(res[0].float(), want, rtol=2e-2, atol=2e-2)
 
 
-@pytest.mark.parametrize("rows,N", [(3, 40), (3, 8200), (33, 72), (33, 8200), (130, 136)])  # 16 rows by 1 and 4 waves, 32 by 2 and 4, 64 by 4
+@pytest.mark.parametrize("rows,N", [(3, 40), (3, 8200), (33, 72), (33, 8200), (130, 136)])  # 16 rows by 2 and 4 waves, 32 by 2 and 4, 64 by 4
 @pytest.mark.parametrize("Kd", [32, 256, 288, 1056])  # one step, a whole chunk of 8, a chunk and a rest, four chunks and a rest
 @pytest.mark.parametrize("act,il", [(0, False), (1, False), (1, True)])
-def test_grouped_gemm_few_rows_keeps_the_bits(rows, N, Kd, act, il):
-    """Experts' products of a decode step (rows gathered by index) against the register kernel that takes over above 512 rows: both are
-    one chain of products in the order of k."""
+def test_grouped_gemm_tiles_keep_the_bits(rows, N, Kd, act, il):
+    """Experts' products, rows gathered by index, give the same bits by every tile (one chain of products in the order of k): against the
+    same rows beside an expert of 520 more, which brings the mean to 64 rows a tile; and the values of fp64 products within the
+    roundings of gate, up and result."""
     if il:
         N = N // 64 * 64 or 64
     g = _g(75)
@@ -367,6 +369,12 @@ def test_grouped_gemm_few_rows_keeps_the_bits(rows, N, Kd, act, il):
     ext.grouped_gemm(few, a[:rows], w[:2].contiguous(), _i32(off).cuda(), perm[:rows].contiguous(), 1, act, il, True, 0.0)
     ext.grouped_gemm(many, a, w, _i32(off + [rows + more]).cuda(), perm, 1, act, il, True, 0.0)
     assert torch.equal(few, many[:rows])
+    z = torch.cat([a[perm[off[e]:off[e + 1]].long()].double() @ w[e].double().t() for e in range(2)])
+    if act:
+        z = z.view(rows, -1, 2, 64) if il else z.view(rows, 2, N)
+        p, u = (z[:, :, i].reshape(rows, N) if il else z[:, i] for i in (0, 1))
+        z = F.silu(p) * u
+    torch.testing.assert_close(few.double(), z, rtol=2e-2, atol=1e-2)  # three roundings of 2^-9, gate and up of up to 4
 
 
 @pytest.mark.parametrize("M", [1, 2, 15, 16, 17])
