@@ -820,7 +820,7 @@ class WkvMixer:
         mix = hops.token_mix(h, self.mu, cache["prev"], *seg, dtype)
         rkvg = torch.empty(T, 4 * n, dtype=dtype, device=h.device)
         torch.bmm(mix[:, :4].transpose(0, 1), self.w_rkvg, out=rkvg.view(T, 4, n).transpose(0, 1))
-        z = hops.linear(hops.activation(hops.linear(mix[:, 4], self.w1), "tanh"), self.w2)
+        z = hops.linear(hops.linear_act(mix[:, 4], self.w1, "tanh"), self.w2)
         o = hops.decay_scan(rkvg, 0, n, 2 * n, z, self.w0, cache["state"], *seg, H, H, dk, dk, 1.0, decay="exp_exp", bonus=self.u,
                             longest=meta.seg_max, singles=meta.num_decode)
         g = hops.gated_group_norm(o, rkvg, 3 * n, self.norm_w, self.eps, H, dtype, after=True, gate="silu")
@@ -980,7 +980,7 @@ class UngatedDenseFFN:
         self.w_down = p.get(prefix + "down", (d, self.ff), 1.0 / math.sqrt(self.ff))
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return hops.linear(hops.activation(hops.linear(h, self.w_up), self.act), self.w_down)
+        return hops.linear(hops.linear_act(h, self.w_up, self.act), self.w_down)
 
 
 class GatedDenseFFN:
@@ -1100,7 +1100,7 @@ class CorrectedRoutedFFN:
                                            corr=self.corr, best2=False, renorm=False)
         shared = None
         if self.fs:
-            shared = hops.linear(hops.activation(hops.linear(h, self.ws1), "relu_sq"), self.ws2)
+            shared = hops.linear(hops.linear_act(h, self.ws1, "relu_sq"), self.ws2)
         return hops.moe_experts(h, ids, wts, self.w1, self.w2, shared, None, act="relu_sq", identity=self.ident)
 
 
@@ -1507,12 +1507,7 @@ class HybridLM:
 
     def _logits(self, hf: torch.Tensor) -> torch.Tensor:
         c = self.cfg
-        z = F.linear(hf, self.head).float()
-        if c.logit_scale != 1.0:
-            z = z * c.logit_scale
-        if c.logit_softcap > 0:
-            z = hops.softcap(z.contiguous(), c.logit_softcap)
-        return z
+        return hops.logits(hf, self.head, c.logit_scale, c.logit_softcap)
 
     def _gate_of(self, sub, g: dict, h: torch.Tensor) -> tuple:
         """(projection, first column) holding a sublayer's residual-gate logits for this step."""

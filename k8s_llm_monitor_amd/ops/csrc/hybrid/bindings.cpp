@@ -90,9 +90,8 @@ int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* decay, float* s
                          const int* slot, int S, long T, int longest, int H, int dk, int dv, int nt, hipStream_t s);
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
                      const float* bias, int E, int K, int rows_w, int over_all, int f32, hipStream_t s);
-int k8sllm_hy_few_rows(void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, hipStream_t s);
-int k8sllm_hy_few_rows_glu(void* yg, void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, int f, int kind,
-                           hipStream_t s);
+int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const void* w, int M, int N, int Kd, int f, int kind, int f32,
+                       float cap, int shared, hipStream_t s);
 int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* offsets, const int* sorted_idx, int div,
                            int E, long rows, int N, int Kd, long w_es, int act, int il, int f32, int mfma, float limit,
                            hipStream_t s);
@@ -925,34 +924,27 @@ void moe_align(Tensor ids, int64_t E, Tensor offsets, Tensor sorted_idx, Tensor 
         "moe_align");
 }
 
-// y [M, N] = x [M, K] w [N, K]^T, bf16, few rows; see few_rows.hip
-void few_rows(Tensor y, Tensor x, Tensor w) {
+// y [M, N - 2 f] = x [M, K] w [N, K]^T, bf16, M <= 64; kinds, f, yg [M, f], an fp32 y and cap: see few_rows.hip
+void few_rows(Tensor y, OptT yg, Tensor x, Tensor w, int64_t kind, double cap, bool shared) {
   TORCH_CHECK(act(x, "x") == 0, "few_rows: bf16");
   same(w, 0, "w");
-  same(y, 0, "y");
+  const int f32 = act(y, "y");
+  int64_t f = 0;
+  void* yp = nullptr;
+  TORCH_CHECK(yg.has_value() == (kind >= 0 && kind < 16), "few_rows: a gated unit's output");
+  if (yg.has_value()) {
+    same(*yg, 0, "yg");
+    TORCH_CHECK(yg->dim() == 2 && yg->is_contiguous() && yg->size(0) == x.size(0), "few_rows: yg [M, f]");
+    f = yg->size(1);
+    yp = yg->data_ptr();
+  }
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && w.dim() == 2 && w.is_contiguous() && y.dim() == 2 && y.is_contiguous() &&
-                  y.size(0) == x.size(0) && y.size(1) == w.size(0) && x.size(1) == w.size(1),
+                  y.size(0) == x.size(0) && 2 * f + y.size(1) == w.size(0) && x.size(1) == w.size(1),
               "few_rows: layouts");
   TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0, "few_rows: alignment");
-  check(k8sllm_hy_few_rows(y.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), (int)x.size(0), (int)w.size(0), (int)x.size(1), cur()),
+  check(k8sllm_hy_few_rows(y.data_ptr(), yp, x.data_ptr(), x.stride(0), w.data_ptr(), (int)x.size(0), (int)w.size(0), (int)x.size(1), (int)f,
+                           (int)kind, f32, (float)cap, shared, cur()),
         "few_rows");
-}
-
-// yg [M, f]: the gated unit of w's rows [f gate | f up | ..]; y [M, N - 2 f]: the other rows' products; see few_rows.hip
-void few_rows_glu(Tensor yg, Tensor y, Tensor x, Tensor w, int64_t kind) {
-  TORCH_CHECK(act(x, "x") == 0, "few_rows_glu: bf16");
-  same(w, 0, "w");
-  same(y, 0, "y");
-  same(yg, 0, "yg");
-  const int64_t f = yg.size(1);
-  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && w.dim() == 2 && w.is_contiguous() && y.dim() == 2 && y.is_contiguous() &&
-                  yg.dim() == 2 && yg.is_contiguous() && yg.size(0) == x.size(0) && y.size(0) == x.size(0) &&
-                  2 * f + y.size(1) == w.size(0) && x.size(1) == w.size(1),
-              "few_rows_glu: layouts");
-  TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0, "few_rows_glu: alignment");
-  check(k8sllm_hy_few_rows_glu(yg.data_ptr(), y.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), (int)x.size(0), (int)w.size(0),
-                               (int)x.size(1), (int)f, (int)kind, cur()),
-        "few_rows_glu");
 }
 
 // y [rows, N] = W[e] a over expert-sorted rows; sorted_idx given: a's row of sorted row r is sorted_idx[r] / div
@@ -1204,7 +1196,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_router", &moe_router);
   m.def("moe_align", &moe_align);
   m.def("few_rows", &few_rows);
-  m.def("few_rows_glu", &few_rows_glu);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("moe_combine", &moe_combine);
   m.def("norm_shift", &norm_shift);

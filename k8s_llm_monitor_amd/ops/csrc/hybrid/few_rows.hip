@@ -1,82 +1,129 @@
-// Y[M][N] = X[M][K] W[N][K]^T for the few rows of a decode step (bf16, fp32 sums, M up to 16, K a multiple of 32).
-// A projection of one or a few rows is a pass over its weights: at the widths of a small model that is 1 to 3 us of memory traffic,
-// and what a call takes is set by how soon enough loads are in flight.  A workgroup takes 16 output columns and its 16 waves a
-// slice of K each, both operands as 16-byte fragments of v_mfma_f32_16x16x32_bf16 straight from global memory, a batch of loads
-// in flight while the last is multiplied; the waves' sums meet in LDS in the order of K.
-// us, the BLAS library's call against this one, 1 and 16 rows (N x K): 1024 x 1024 5.6 / 4.1, 5.7 / 5.4; 4096 x 1024 7.5 / 4.7, 7.6 /
-// 6.0; 1024 x 4096 14.4 / 7.1, 14.5 / 9.6; 2048 x 2048 11.0 / 4.8, 11.2 / 6.3; 4096 x 4096 15.5 / 9.3, 15.6 / 10.7.  Eight waves:
-// up to 0.9 more.  Past the caller's limits the library is faster: 2048 x 5632 10.3 / 10.3, 11.2 / 15.2 (too few workgroups);
-// 32000 x 1024 18.7 / 25.5; 16384 x 4096 at 16 rows 33.4 / 39.0.
-#include "hy_common.h"
+// Y[M][N] = X[M][K] W[N][K]^T for the few rows of a decode step (bf16, fp32 sums, M up to 64, K a multiple of 32).
+// A projection of a few rows is a pass over its weights; what a call takes is set by how soon enough loads are in flight, and by how
+// often the rows are fetched beside the weights.  Two forms (stream_rows.h has the streams):
+//   own     a workgroup takes 16 columns, its four waves a quarter of K each with their own copies of the rows; the waves' sums meet in
+//           LDS in the order of K.  As many workgroups as there are column tiles.
+//   shared  a workgroup takes 64 columns and all of K, its four waves share the rows.
+#include "stream_rows.h"
 
 namespace k8sllm {
 
-constexpr int NWV = 16;
+// What becomes of a product: KIND -1 nothing; 1, 3, 4: W's first 2 f rows are a gated unit's gate and up rows, Yg [M][f] = act(gate) * up of
+// the products rounded to bf16 (as the separate launch finds them), Y gets the products of the rest; 16 + a: act_f<a> of the rounded
+// product.  One launch less each.  F32: Y is fp32, the rounded products capped at +-cap if cap > 0 (logits).
+struct RowsOut {
+  void* y;
+  bf16_t* yg;
+  int M, N, f, f32;
+  float cap;
+};
 
-// KIND >= 0: W's first 2 f rows are a gated unit's gate and up rows, Yg [M][f] = act(gate) * up of the products rounded to bf16 (as
-// the separate launch finds them), each workgroup below f / 16 taking 16 columns of both; Y gets the products of the rest.  One launch less a gated
-// feed-forward: a step with six of them (one row, width 1024, f 2816) 422 -> 404 us.
 template <int KIND>
-__global__ __launch_bounds__(64 * NWV) void few_rows_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ X, long x_stride,
-                                                             const bf16_t* __restrict__ W, int M, int N, int Kd,
-                                                             bf16_t* __restrict__ Yg, int f) {
-  constexpr int U = 4;
-  constexpr bool GLU = KIND >= 0;
-  __shared__ __attribute__((aligned(16))) float red[GLU ? 2 : 1][NWV][64][4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, quad = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  const bool pair = GLU && n0 < f;  // uniform
-  const int m0 = GLU && !pair ? n0 + f : n0;  // first row of W
+__device__ __forceinline__ void rows_store(const RowsOut& o, int r, int n, float v) {  // n: row of W
+  if (r >= o.M || n >= o.N) return;
+  const int first = KIND >= 0 && KIND < 16 ? 2 * o.f : 0;
+  const long i = (long)r * (o.N - first) + n - first;
+  const bf16_t b = f2bf(v);
+  if (KIND >= 16) {
+    reinterpret_cast<bf16_t*>(o.y)[i] = f2bf(act_f<KIND >= 16 ? KIND - 16 : 3>(bf2f(b), 0.f, 0.f));
+  } else if (o.f32) {
+    const float z = bf2f(b);
+    reinterpret_cast<float*>(o.y)[i] = o.cap > 0.f ? o.cap * tanhf(z / o.cap) : z;
+  } else {
+    reinterpret_cast<bf16_t*>(o.y)[i] = b;
+  }
+}
+template <int KIND>
+__device__ __forceinline__ void rows_store_unit(const RowsOut& o, int r, int n, float g, float u) {
+  if (r < o.M) o.yg[(long)r * o.f + n] = f2bf(glu_unit<KIND >= 0 && KIND < 16 ? KIND : 3>(bf2f(f2bf(g)), bf2f(f2bf(u)), 0.f));
+}
+
+// Column tile ``j`` of a launch: gated kinds take two tiles of W's rows, a unit's gate and up or two neighbours of the rest
+template <int KIND>
+__device__ __forceinline__ bool rows_tiles(int j, int f, int (&n)[KIND >= 0 && KIND < 16 ? 2 : 1]) {
+  if constexpr (KIND >= 0 && KIND < 16) {
+    const bool pair = j < f / 16;
+    n[0] = pair ? 16 * j : 2 * f + 32 * (j - f / 16);
+    n[1] = pair ? n[0] + f : n[0] + 16;
+    return pair;
+  } else {
+    n[0] = 16 * j;
+    return false;
+  }
+}
+
+template <int KIND, int MT>
+__global__ __launch_bounds__(256) void few_rows_own_kernel(RowsOut o, const bf16_t* __restrict__ X, long x_stride,
+                                                           const bf16_t* __restrict__ W, int Kd) {
+  constexpr int NWV = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1, D = MT <= 2 ? 8 : 4, NT = MT * NS;
+  using S = OwnRows<MT, NS, D>;
+  static_assert(NT <= S::BYTES / 1024, "");
+  __shared__ __attribute__((aligned(1024))) char smem[NWV * S::BYTES];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int n[NS];
+  const bool pair = rows_tiles<KIND>(blockIdx.x, o.f, n);
   const int per = (Kd / 32 + NWV - 1) / NWV, s0 = min(wave * per, Kd / 32), ns = min(per, Kd / 32 - s0);
-  const bf16_t* wp = W + (long)min(m0 + c16, N - 1) * Kd + 32 * s0 + 8 * quad;
-  const bf16_t* up = wp + (pair ? (long)f * Kd : 0);
-  const bf16_t* xp = X + (long)min(c16, M - 1) * x_stride + 32 * s0 + 8 * quad;
-  f32x4 acc = {}, accu = {};
-  bf16x8 a[2][U], w[2][U], u[2][U];
-  auto load = [&](int h, int i, int k) {
-    w[h][i] = *reinterpret_cast<const bf16x8*>(wp + 32 * k);
-    if (GLU) u[h][i] = *reinterpret_cast<const bf16x8*>(up + 32 * k);
-    a[h][i] = *reinterpret_cast<const bf16x8*>(xp + 32 * k);
-  };
-  const int nb = (ns + U - 1) / U;  // the last batch repeats its last step's loads and leaves their products out
-  if (ns > 0)
+  const bf16_t* src[NS + MT];
 #pragma unroll
-    for (int i = 0; i < U; ++i) load(0, i, min(i, ns - 1));
-  for (int k = 0; k < nb; k += 2) {
+  for (int t = 0; t < NS; ++t) src[t] = W + (long)min(n[t] + piece_row(), o.N - 1) * Kd + 32 * s0 + piece_k();
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (k + h >= nb) break;
-      if (k + h + 1 < nb)
+  for (int m = 0; m < MT; ++m) src[NS + m] = X + (long)min(16 * m + piece_row(), o.M - 1) * x_stride + 32 * s0 + piece_k();
+  f32x4 acc[MT][NS] = {};
+  S::run(smem + wave * S::BYTES, src, ns, acc);
+  __syncthreads();  // the rings have been read
+  f32x4* red = reinterpret_cast<f32x4*>(smem);
 #pragma unroll
-        for (int i = 0; i < U; ++i) load(h ^ 1, i, min((k + h + 1) * U + i, ns - 1));
-      __builtin_amdgcn_sched_barrier(0);
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int i = 0; i < U; ++i)
-        if ((k + h) * U + i < ns) {
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i], w[h][i], acc, 0, 0, 0);
-          if (GLU) accu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i], u[h][i], accu, 0, 0, 0);
-        }
-    }
-  }
-  *reinterpret_cast<f32x4*>(red[0][wave][lane]) = acc;
-  if (GLU) *reinterpret_cast<f32x4*>(red[GLU][wave][lane]) = accu;
+    for (int t = 0; t < NS; ++t) red[(wave * NT + m * NS + t) * 64 + lane] = acc[m][t];
   __syncthreads();
-  if (threadIdx.x < 256) {  // element i of lane l: row 4 (l / 16) + i, column l % 16
-    const int r = threadIdx.x >> 4, l = (r >> 2) * 16 + c16, i = r & 3;
-    if (r >= M || m0 + c16 >= N) return;
-    float v = red[0][0][l][i];
+  // element i of lane l: row 4 (l / 16) + i, column l % 16
+  auto sum = [&](int m, int t, int l) {
+    f32x4 v = red[(m * NS + t) * 64 + l];
 #pragma unroll
-    for (int g = 1; g < NWV; ++g) v += red[0][g][l][i];
+    for (int g = 1; g < NWV; ++g) v += red[(g * NT + m * NS + t) * 64 + l];
+    return v;
+  };
+  for (int i = threadIdx.x; i < (pair ? MT : NT) * 64; i += 64 * NWV) {
+    const int l = i & 63, q = i >> 6, m = pair ? q : q / NS, t = pair ? 0 : q % NS, c = l & 15, r = 16 * m + 4 * (l >> 4);
+    const f32x4 v = sum(m, t, l);
     if (pair) {
-      float t = red[GLU][0][l][i];
+      const f32x4 u = sum(m, NS - 1, l);
 #pragma unroll
-      for (int g = 1; g < NWV; ++g) t += red[GLU][g][l][i];
-      Yg[(long)r * f + n0 + c16] = f2bf(glu_unit<GLU ? KIND : 3>(bf2f(f2bf(v)), bf2f(f2bf(t)), 0.f));
+      for (int j = 0; j < 4; ++j) rows_store_unit<KIND>(o, r + j, n[0] + c, v[j], u[j]);
     } else {
-      const int o = GLU ? 2 * f : 0;
-      Y[(long)r * (N - o) + m0 + c16 - o] = f2bf(v);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) rows_store<KIND>(o, r + j, n[NS > 1 ? t : 0] + c, v[j]);
     }
   }
+}
+
+template <int KIND, int MT>
+__global__ __launch_bounds__(256) void few_rows_shared_kernel(RowsOut o, const bf16_t* __restrict__ X, long x_stride,
+                                                              const bf16_t* __restrict__ W, int Kd) {
+  constexpr int NW = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1;
+  using S = SharedRows<MT, NS, NW>;
+  __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
+  int n[NS];
+  const bool pair = rows_tiles<KIND>(blockIdx.x * NW + (threadIdx.x >> 6), o.f, n);
+  const bf16_t* w[NS];
+#pragma unroll
+  for (int t = 0; t < NS; ++t) w[t] = W + (long)min(n[t] + piece_row(), o.N - 1) * Kd + piece_k();
+  f32x4 acc[MT][NS] = {};
+  S::run(smem, [&](int m) { return X + (long)min(16 * m + piece_row(), o.M - 1) * x_stride + piece_k(); }, w, Kd / 32, acc);
+  const int c = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * m + 4 * quad + i;
+      if (pair) {
+        rows_store_unit<KIND>(o, r, n[0] + c, acc[m][0][i], acc[m][NS - 1][i]);
+      } else {
+#pragma unroll
+        for (int t = 0; t < NS; ++t) rows_store<KIND>(o, r, n[t] + c, acc[m][t][i]);
+      }
+    }
 }
 
 }  // namespace k8sllm
@@ -85,28 +132,34 @@ using namespace k8sllm;
 
 extern "C" {
 
-int k8sllm_hy_few_rows(void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, hipStream_t s) {
+// kind: see RowsOut (gated: yg [M][f], y [M][N - 2 f]); f32: y is fp32, capped if cap > 0 (kind -1); shared: the form
+int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const void* w, int M, int N, int Kd, int f, int kind, int f32,
+                       float cap, int shared, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 16 || Kd < 32 || Kd % 32 || x_stride % 8) return -1;
-  hipLaunchKernelGGL((few_rows_kernel<-1>), dim3((unsigned)((N + 15) / 16)), dim3(64 * NWV), 0, s, (bf16_t*)y, (const bf16_t*)x, x_stride,
-                     (const bf16_t*)w, M, N, Kd, (bf16_t*)nullptr, 0);
-  return (int)hipGetLastError();
-}
-
-// yg [M][f]: the gated unit (kind 1 tanh GELU, 3 SiLU, 4 ReLU) of w's first 2 f rows; y [M][N - 2 f]: the other rows' products
-int k8sllm_hy_few_rows_glu(void* yg, void* y, const void* x, long x_stride, const void* w, int M, int N, int Kd, int f, int kind,
-                           hipStream_t s) {
-  if (M <= 0 || f <= 0) return 0;
-  if (M > 16 || Kd < 32 || Kd % 32 || x_stride % 8 || f % 16 || N < 2 * f) return -1;
-  const dim3 grid((unsigned)(f / 16 + (N - 2 * f + 15) / 16));
-#define K8SLLM_FRG(K)                                                                                                   \
-  hipLaunchKernelGGL((few_rows_kernel<K>), grid, dim3(64 * NWV), 0, s, (bf16_t*)y, (const bf16_t*)x, x_stride, (const bf16_t*)w, M, N, \
-                     Kd, (bf16_t*)yg, f)
-  if (kind == 1) K8SLLM_FRG(1);
-  else if (kind == 3) K8SLLM_FRG(3);
-  else if (kind == 4) K8SLLM_FRG(4);
+  const bool gated = kind >= 0 && kind < 16;
+  if (M > 64 || Kd < 32 || Kd % 32 || x_stride % 8 || (f32 && kind != -1)) return -1;
+  if (gated ? f <= 0 || f % 16 || N < 2 * f || yg == nullptr : f != 0) return -1;
+  const RowsOut o{y, (bf16_t*)yg, M, N, f, f32, cap};
+  const unsigned tiles = (unsigned)(gated ? f / 16 + (N - 2 * f + 31) / 32 : (N + 15) / 16);
+#define K8SLLM_FR(KIND, MT)                                                                                                  \
+  if (shared)                                                                                                                \
+    hipLaunchKernelGGL((few_rows_shared_kernel<KIND, MT>), dim3((tiles + 3) / 4), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, \
+                       (const bf16_t*)w, Kd);                                                                                \
+  else                                                                                                                       \
+    hipLaunchKernelGGL((few_rows_own_kernel<KIND, MT>), dim3(tiles), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, (const bf16_t*)w, Kd)
+#define K8SLLM_FRM(KIND)              \
+  if (M <= 16) { K8SLLM_FR(KIND, 1); } \
+  else if (M <= 32) { K8SLLM_FR(KIND, 2); } \
+  else { K8SLLM_FR(KIND, 4); }
+  if (kind == -1) { K8SLLM_FRM(-1) }
+  else if (kind == 1) { K8SLLM_FRM(1) }
+  else if (kind == 3) { K8SLLM_FRM(3) }
+  else if (kind == 4) { K8SLLM_FRM(4) }
+  else if (kind == 16 + 6) { K8SLLM_FRM(16 + 6) }
+  else if (kind == 16 + 7) { K8SLLM_FRM(16 + 7) }
   else return -1;
-#undef K8SLLM_FRG
+#undef K8SLLM_FRM
+#undef K8SLLM_FR
   return (int)hipGetLastError();
 }
 }

@@ -94,4 +94,51 @@ struct SharedRows {
   }
 };
 
+// One wave streams 16 MT rows and NS weight tiles, its own part of K, through a private ring D steps deep: no barrier.
+template <int MT, int NS, int D>
+struct OwnRows {
+  static constexpr int L = MT + NS, BYTES = D * L * 1024;
+
+  // src: this lane's sources, weight tiles first; ns: steps
+  static __device__ __forceinline__ void run(char* lds, const bf16_t* const (&src)[L], int ns, f32x4 (&acc)[MT][NS]) {
+    if (ns <= 0) return;
+    const int rd = piece_frag();
+    auto issue = [&](int slot, int k) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) load_piece(lds + (slot * L + i) * 1024, src[i] + 32 * k);
+    };
+    auto consume = [&](int slot) {
+      bf16x8 f[L];
+#pragma unroll
+      for (int i = 0; i < L; ++i) f[i] = *reinterpret_cast<const bf16x8*>(lds + (slot * L + i) * 1024 + rd);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot may be refilled
+#pragma unroll
+      for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[NS + m], f[t], acc[m][t], 0, 0, 0);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) issue(d, min(d, ns - 1));
+    int slot = 0, k = 0;
+    for (; k + D < ns; ++k) {
+      loads_left<(D - 1) * L>();
+      consume(slot);
+      issue(slot, k + D);
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    auto rest = [&](auto self, auto dc) {
+      constexpr int d = decltype(dc)::value;
+      if constexpr (d < D) {
+        loads_left<(D - 1 - d) * L>();
+        if (k + d < ns) {
+          consume(slot);
+          slot = slot + 1 == D ? 0 : slot + 1;
+        }
+        self(self, std::integral_constant<int, d + 1>{});
+      }
+    };
+    rest(rest, std::integral_constant<int, 0>{});
+  }
+};
+
 }  // namespace k8sllm

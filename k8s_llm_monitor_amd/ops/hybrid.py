@@ -1158,37 +1158,77 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
     return out
 
 
-FEW_ROWS, FEW_ROWS_K, FEW_ROWS_WEIGHTS = 16, 4096, 1 << 24
+def _rows_form(M: int, N: int, K: int, fused: bool) -> Optional[str]:
+    """Which kernel of few_rows.hip takes a bf16 product of M rows with weights [N, K], ``fused`` where it also saves the launch behind it;
+    None: the BLAS library.  us, library / own / shared, in a graph over weights from memory: 2048 x 2048, 1 row 10.9 / 4.4 / 8.2,
+    64 rows 11.6 / 10.1 / 13.5; 4096 x 4096, 16 rows 15.6 / 9.5 / 17.0, 32 rows 13.2 / 12.6 / 18.7, 48 rows 13.8 / 17.0 / 21.8; 16384 x
+    4096, 1 row 34.0 / 25.4 / 31.6, 16 rows 33.8 / 36.5 / 30.5, 32 rows 33.8 / 44.4 / 31.2, 64 rows 33.5 / 67.3 / 36.4 (a launch behind
+    it takes 4 to 6); 8192 x 1024, 64 rows 11.9 / 10.5 / 9.5; 4096 x 8192, 1 row 16.6 / 17.1 / 27.7."""
+    if M > 64 or K > 6144 or (M > 4 and K > 4096):
+        return None
+    if M <= 4 or (M <= 32 and N * K <= 1 << 24 and N < 8192) or (M <= 16 and N * K <= 1 << 24) or (N * K <= 1 << 22 and K <= 2048):
+        return "own"
+    if 8192 <= N and (M <= 16 or (M <= 32 and N * K <= 1 << 26) or fused or (K <= 1024 and N <= 16384)):
+        return "shared"
+    return None
 
 
-def _few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
-    return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-            and w.shape[1] % 32 == 0 and 32 <= w.shape[1] <= FEW_ROWS_K and w.numel() <= FEW_ROWS_WEIGHTS and x.shape[0] > 0
+def _few_rows(x: torch.Tensor, w: torch.Tensor, fused: bool = False) -> Optional[str]:
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+            and w.shape[1] % 32 == 0 and w.shape[1] >= 32 and x.shape[0] > 0
             and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        return None
+    return _rows_form(x.shape[0], w.shape[0], w.shape[1], fused)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x`` [T, K] times ``w`` [N, K] transposed.  The BLAS library's product, but for the few rows of a small decode step in
-    bf16 on the device: up to FEW_ROWS rows against weights of up to 16 M elements, K up to 4096 (and a multiple of 32, rows
-    16-byte aligned), where a call takes what it takes to get enough loads in flight (few_rows.hip has both sides' times)."""
-    if len(x) <= FEW_ROWS and _few_rows(x, w):
+    """``x`` [T, K] times ``w`` [N, K] transposed.  The BLAS library's product, but for the few rows of a decode step in bf16 on the
+    device, K a multiple of 32 and rows 16-byte aligned, where a call takes what it takes to get enough loads in flight
+    (few_rows.hip, by the rule of ``_rows_form``)."""
+    form = _few_rows(x, w)
+    if form is not None:
         y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
-        native().few_rows(y, x, w)
+        native().few_rows(y, None, x, w, -1, 0.0, form == "shared")
         return y
     return F.linear(x, w)
 
 
+def linear_act(x: torch.Tensor, w: torch.Tensor, kind: str) -> torch.Tensor:
+    """``activation(linear(x, w), kind)``, in one launch for the rows that few_rows.hip takes (``relu_sq`` and ``tanh``)."""
+    form = _few_rows(x, w, True) if kind in ("relu_sq", "tanh") else None
+    if form is not None:
+        y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        native().few_rows(y, None, x, w, 16 + ACTS[kind], 0.0, form == "shared")
+        return y
+    return activation(linear(x, w), kind)
+
+
 def linear_glu(x: torch.Tensor, w: torch.Tensor, f: int, kind: str) -> tuple:
     """The gated unit ``act(gate x) * (up x)`` [T, f] of ``w``'s rows [f gate | f up | the rest], and a projection with the column
-    at which the rest's outputs begin in it.  ``linear`` and ``glu``, in one launch for the rows that ``linear`` takes itself."""
-    if len(x) <= FEW_ROWS and f > 0 and f % 16 == 0 and _few_rows(x, w):
+    at which the rest's outputs begin in it.  ``linear`` and ``glu``, in one launch for the rows that few_rows.hip takes."""
+    form = _few_rows(x, w, True) if f > 0 and f % 16 == 0 else None
+    if form is not None:
         a = torch.empty(x.shape[0], f, dtype=x.dtype, device=x.device)
         y = torch.empty(x.shape[0], w.shape[0] - 2 * f, dtype=x.dtype, device=x.device)
-        native().few_rows_glu(a, y, x, w, ACTS[kind])
+        native().few_rows(y, a, x, w, ACTS[kind], 0.0, form == "shared")
         return a, y, 0
     proj = linear(x, w)
     return glu(proj, 0, f, kind), proj, 2 * f
+
+
+def logits(x: torch.Tensor, w: torch.Tensor, scale: float = 1.0, cap: float = 0.0) -> torch.Tensor:
+    """fp32 ``scale * (x w^T)`` of the product rounded to x's dtype, through ``cap * tanh(. / cap)`` if cap > 0.  In one launch for the
+    few rows of a decode step (no scale)."""
+    form = _few_rows(x, w) if scale == 1.0 else None
+    if form is not None:
+        z = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
+        native().few_rows(z, None, x, w, -1, float(cap), form == "shared")
+        return z
+    z = F.linear(x, w).float()
+    if scale != 1.0:
+        z = z * scale
+    return softcap(z.contiguous(), cap) if cap > 0 else z
 
 
 def swiglu(gu: torch.Tensor) -> torch.Tensor:

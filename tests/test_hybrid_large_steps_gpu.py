@@ -483,6 +483,37 @@ def test_decode_attention_row_broadcasts(dk, dv, Hq, G):
         torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1e-2, atol=2e-3)
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])  # one, two and four row tiles
+@pytest.mark.parametrize("f,rest,K", [(16, 0, 32), (48, 40, 96), (112, 24, 288), (32, 200, 2080)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_few_rows_forms(M, f, rest, K, shared):
+    """Both forms of a few rows' projection, plain, with a unit at its end and as capped fp32 logits, against 64 bits: fewer steps
+    of 32 k than waves, a chunk of 8 and a rest, columns around the tile, a slice of wider rows.  fp32 sums, one bf16 rounding: 2^-8 of
+    the value and 1e-6 sqrt(K) of what cancels; what a unit makes of two rounded products of up to 4: 2e-2."""
+    g = _g(76)
+    x, w = _r(g, M, K + 24, dt=BF).cuda()[:, 16:16 + K], _r(g, 2 * f + rest, K, s=K ** -0.5, dt=BF).cuda()
+    N, z, ext = 2 * f + rest, x.double() @ w.double().t(), hops.native()
+
+    def out(n, dt=BF):
+        return torch.full((M, n), float("nan"), dtype=dt, device="cuda")
+
+    y = out(N)
+    ext.few_rows(y, None, x, w, -1, 0.0, shared)
+    assert bool(((y.double() - z).abs() <= 2 ** -8 * z.abs() + 1e-6 * K ** 0.5).all())
+    for cap in (0.0, 3.0):
+        q = out(N, torch.float32)
+        ext.few_rows(q, None, x, w, -1, cap, shared)
+        torch.testing.assert_close(q, cap * torch.tanh(y.float() / cap) if cap else y.float(), rtol=1e-6, atol=1e-6)
+    for kind in ("relu_sq", "tanh"):
+        q = out(N)
+        ext.few_rows(q, None, x, w, 16 + hops.ACTS[kind], 0.0, shared)
+        assert torch.equal(q, hops.activation(y, kind))
+    for kind in ("gelu_tanh", "silu", "relu"):
+        a, q = out(f), out(rest)
+        ext.few_rows(q, a, x, w, hops.ACTS[kind], 0.0, shared)
+        assert torch.equal(a, hops.glu(y, 0, f, kind)) and torch.equal(q, y[:, 2 * f:])
+
+
 def test_linear_of_nothing():
     """Empty sums, no columns, no rows and no gated unit are what the library makes of them."""
     g = _g(89)
