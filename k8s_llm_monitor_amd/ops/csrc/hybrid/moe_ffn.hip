@@ -463,101 +463,6 @@ __global__ __launch_bounds__(256) void hy_grouped_gemm_kernel(T* __restrict__ Y,
   }
 }
 
-// fp32 on the matrix cores (K a multiple of 32, rows 16-byte aligned): 64 x 64 tiles (gated: 64 gate and 64 up columns) of four
-// waves with 32 x 32 outputs (each of gate and up) on v_mfma_f32_32x32x2_f32, whose sums are fp32 like the vector unit's at twice
-// its rate.  32 k at a time are copied to LDS by global_load_lds, 16 bytes a lane, into a ring of two, while the tile before
-// runs; piece c of a row lies at c ^ (row % 8), so that the fragments' 16-byte reads (four k of a row; the upper half of a wave
-// takes the next four, and both operands agree on that) are spread over the banks.  Consecutive workgroups are consecutive
-// column tiles: the row tiles of an expert meet its weight columns in the same XCD's L2.  Rows past an expert's end and
-// columns past N read the last ones and are not stored.
-// 1996 rows over 8 experts, K = N = 1024, gated / not: 343 / 215 us on the vector unit (whose 64 x 64 tiles waited for their loads
-// every 16 k), 123 / 67 here; 16 rows 199 / 98 and 50 / 26.  Distance to 64 bits the same (8.8e-7, 5.7e-7).
-template <int ACT>
-__global__ __launch_bounds__(256, 2) void hy_grouped_gemm_f32_kernel(float* __restrict__ Y, const float* __restrict__ A,
-                                                                     const float* __restrict__ W,
-                                                                     const int* __restrict__ offsets,
-                                                                     const int* __restrict__ sorted_idx, int div, int E,
-                                                                     int N, int Kd, long w_es, int il, float limit) {
-  typedef float floatx16 __attribute__((ext_vector_type(16)));
-  using gbl_void_t = __attribute__((address_space(1))) const void;
-  using lds_void_t = __attribute__((address_space(3))) void;
-  constexpr bool GATED = ACT == 1 || ACT == 3;
-  constexpr int NB = GATED ? 2 : 1, PIECES = 8 + 8 * NB, NP = PIECES / 4, TKF = 32;  // a piece: 8 rows of 128 bytes
-  __shared__ __attribute__((aligned(1024))) char buf[2][PIECES * 1024];
-  int e = 0, tile = blockIdx.y, r0 = 0, r1 = 0;
-  for (; e < E; ++e) {
-    r0 = offsets[e];
-    r1 = offsets[e + 1];
-    const int nt = (r1 - r0 + TM - 1) / TM;
-    if (tile < nt) break;
-    tile -= nt;
-  }
-  if (e >= E) return;
-  r0 += tile * TM;
-  const int n0 = blockIdx.x * TN;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, l32 = lane & 31;
-  const int wm = wave & 1, wn = wave >> 1;
-  const float* src[NP];
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int piece = wave + 4 * i, row = (piece & 7) * 8 + (lane >> 3), ch = (lane & 7) ^ (lane >> 3);
-    if (piece < 8) {
-      const int r = min(r0 + row, r1 - 1);
-      src[i] = A + (long)(sorted_idx != nullptr ? sorted_idx[r] / div : r) * Kd + ch * 4;
-    } else {
-      const int n = min(n0 + row, N - 1);
-      const long gate = GATED && il ? (long)(n >> 6) * 128 + (n & 63) : n, up = il ? gate + 64 : (long)N + n;
-      src[i] = W + (long)e * w_es + (piece < 16 ? gate : up) * Kd + ch * 4;
-    }
-  }
-  auto issue = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      __builtin_amdgcn_global_load_lds((gbl_void_t*)src[i], (lds_void_t*)(buf[b] + (wave + 4 * i) * 1024), 16, 0, 0);
-      src[i] += TKF;
-    }
-  };
-  floatx16 acc[NB] = {};
-  issue(0);
-  for (int k0 = 0, b = 0; k0 < Kd; k0 += TKF, b ^= 1) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();  // every wave's pieces are there, and the other buffer has been read
-    if (k0 + TKF < Kd) issue(b ^ 1);
-    auto frag = [&](int row, int ch) {
-      return *reinterpret_cast<const float4*>(buf[b] + row * 128 + ((ch ^ (row & 7)) << 4));
-    };
-#pragma unroll
-    for (int g = 0; g < TKF / 8; ++g) {
-      const float4 a = frag(wm * 32 + l32, 2 * g + half);
-      float4 w[NB];
-#pragma unroll
-      for (int u = 0; u < NB; ++u) w[u] = frag(64 + 64 * u + wn * 32 + l32, 2 * g + half);
-#pragma unroll
-      for (int u = 0; u < NB; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, w[u].x, acc[u], 0, 0, 0);
-#pragma unroll
-      for (int u = 0; u < NB; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, w[u].y, acc[u], 0, 0, 0);
-#pragma unroll
-      for (int u = 0; u < NB; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, w[u].z, acc[u], 0, 0, 0);
-#pragma unroll
-      for (int u = 0; u < NB; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, w[u].w, acc[u], 0, 0, 0);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads are done before it meets the next barrier
-  }
-  const int n = n0 + wn * 32 + l32;
-  if (n >= N) return;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = r0 + wm * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-    if (r >= r1) continue;
-    float v = acc[0][i];
-    if (ACT == 1) v = silu_f(v) * acc[NB - 1][i];
-    if (ACT == 3) v = clamped_unit_f(v, acc[NB - 1][i], limit);
-    if (ACT == 2) v = gelu_erf_f(v);
-    if (ACT == 4) v = relu_sq_f(v);
-    Y[(long)r * N + n] = v;
-  }
-}
-
 // What an activation makes of a row's product (and, gated, of the up projection's), both rounded to bf16 first
 template <int ACT>
 __device__ __forceinline__ bf16_t expert_unit(float v, float u, float limit) {
@@ -663,6 +568,9 @@ using namespace k8sllm;
 
 extern "C" {
 
+int k8sllm_hy_experts_f32(float* y, const float* a, const float* w, const int* offsets, const int* sorted_idx, int div, int E, long rows,
+                          int N, int Kd, long w_es, int act, int il, float limit, hipStream_t s);  // experts_f32.hip
+
 int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, int d, const float* wr,
                      const float* bias, int E, int K, int rows_w, int over_all, int f32, hipStream_t s) {
   if (T <= 0) return 0;
@@ -756,20 +664,10 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
 #undef K8SLLM_GM
     return (int)hipGetLastError();
   }
+  if (f32 && Kd % 32 == 0 && aligned)
+    return k8sllm_hy_experts_f32((float*)Y, (const float*)A, (const float*)W, offsets, sorted_idx, div, E, rows, N, Kd, w_es, act, il, limit, s);
+  // other K and alignments: the vector unit
   const dim3 grid((unsigned)(rows / TM + E), (unsigned)((N + TN - 1) / TN));
-  // other K and alignments stay on the vector unit
-  if (f32 && Kd % 32 == 0 && aligned) {
-#define K8SLLM_GF(ACT)                                                                                             \
-  hipLaunchKernelGGL((hy_grouped_gemm_f32_kernel<ACT>), dim3(grid.y, grid.x), dim3(256), 0, s, (float*)Y, (const float*)A, \
-                     (const float*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)
-    if (swiglu) K8SLLM_GF(1);
-    else if (act == 2) K8SLLM_GF(2);
-    else if (act == 3) K8SLLM_GF(3);
-    else if (act == 4) K8SLLM_GF(4);
-    else K8SLLM_GF(0);
-#undef K8SLLM_GF
-    return (int)hipGetLastError();
-  }
 #define K8SLLM_GG(T, SW)                                                                                            \
   hipLaunchKernelGGL((hy_grouped_gemm_kernel<T, SW>), grid, dim3(256), 0, s, (T*)Y, (const T*)A, (const T*)W, offsets, \
                      sorted_idx, div, E, N, Kd, w_es, il, limit)

@@ -296,6 +296,28 @@ def test_fp32_grouped_gemm(rows, N, Kd, act):
         assert float((y.cpu().double() - want).abs().max()) <= float(tol)
 
 
+@pytest.mark.parametrize("rows,N", [(70, 72), (700, 3000)])  # 64 and 128 columns a workgroup
+def test_fp32_grouped_gemm_what_is_no_number(rows, N):
+    """Infinities, NaN, values that a bf16 rounding takes to infinity and sums that overflow come out of the fp32 products as the CPU's
+    fp32 has them, and nothing else is touched: within a unit in the last place of the largest sum for each of three steps of 32
+    products and the last addition."""
+    g, K, inf, nan = _g(90), 96, float("inf"), float("nan")
+    a, w = _r(g, rows, K), _r(g, 1, N, K)
+    a[0, 3], a[1, 40], a[2, 95], a[3, 7], a[4] = inf, nan, -inf, 3.4e38, 1e38
+    w[0, 5, 3], w[0, 6, 3], w[0, 7, 50], w[0, 8, 9] = 0.0, -1.0, inf, 3.39e38
+    w[0, 9] = 8.0
+    got = torch.empty(rows, N, device="cuda")
+    hops.native().grouped_gemm(got, a.cuda(), w.cuda(), _i32([0, rows]).cuda(), None, 1, 0, False, True, 0.0)
+    want, z = a @ w[0].t(), a.double() @ w[0].double().t()
+    got = got.cpu()
+    assert got[4, 9] == inf  # elsewhere in this row the order of the sums decides what overflows
+    got[4], want[4], z[4] = 0.0, 0.0, 0.0
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    plain = torch.ones(rows, N, dtype=torch.bool)
+    plain[:5], plain[:, 5:10] = False, False
+    assert float((got.double() - z)[plain].abs().max()) <= 4 * 2 ** -23 * float(z[plain].abs().max())
+
+
 @pytest.mark.parametrize("dk,dv,Hq,G", [(128, 128, 8, 2), (64, 128, 3, 1), (128, 64, 2, 2), (64, 64, 16, 2)])
 @pytest.mark.parametrize("kw", [dict(window=0, sink=False), dict(window=5, sink=True), dict(window=40, sink=False, keep=3),
                                 dict(window=33, sink=True, keep=20, cap=2.0), dict(window=32, sink=False, chunked=True)])
