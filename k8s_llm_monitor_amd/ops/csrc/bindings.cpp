@@ -43,6 +43,7 @@ int k8sllm_moe_align(const int* topk_ids, long n, int E, int* expert_offsets, in
 int k8sllm_moe_combine(void* out, const void* expert_out, const int* inv_idx, const float* topk_w, long T, int K,
                        int d, hipStream_t s);
 int k8sllm_gather_rows(void* out, const void* x, const int* idx, long n, int d, int div, hipStream_t s);
+int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void* Y2, int M, int N, int K, int f, int epi, hipStream_t s);
 int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, int N, int K, const int* offsets, int E, long w_es,
                      int epi, int algo, const int* rope_pos, const float* rope_cs, int rope_heads,
                      const float* rs_part, int rs_np, float rs_eps, void* resid, void* hw, const void* norm_w,
@@ -392,6 +393,31 @@ void moe_grouped_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, torch::
   check(k8sllm_moe_grouped_gemm(x.data_ptr(), w.data_ptr(), y.data_ptr(), offsets.data_ptr<int>(), E, x.size(0), N, K,
                                 (long)N * K, swiglu ? 1 : 0, cur()),
         "moe_grouped_gemm");
+}
+
+// y [M, f] = the unit ``epi`` (tile_epi.h) of x . w^T with w's rows [f gate | f up | rest], rest [M, N - 2 f] their products; the squared
+// ReLU: f 0, y [M, N], no rest
+void gemm_tile_unit(torch::Tensor y, c10::optional<torch::Tensor> rest, torch::Tensor x, torch::Tensor w, int64_t epi) {
+  dev_bf16(y, "y"); dev_bf16(x, "x"); dev_bf16(w, "w");
+  const bool glu = rest.has_value();
+  TORCH_CHECK(x.dim() == 2 && x.is_contiguous() && w.dim() == 2 && w.is_contiguous() && y.dim() == 2 && y.is_contiguous() &&
+                  x.size(1) == w.size(1) && y.size(0) == x.size(0),
+              "gemm_tile_unit: x [M, K], w [N, K], y [M, f]");
+  const int64_t f = glu ? y.size(1) : 0;
+  void* rp = nullptr;
+  if (glu) {
+    dev_bf16(*rest, "rest");
+    TORCH_CHECK(rest->dim() == 2 && rest->is_contiguous() && rest->size(0) == x.size(0) && 2 * f + rest->size(1) == w.size(0),
+                "gemm_tile_unit: rest [M, N - 2 f]");
+    rp = rest->data_ptr();
+  }
+  TORCH_CHECK(glu == (epi >= 5 && epi <= 7) && (glu || y.size(1) == w.size(0)), "gemm_tile_unit: unit");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr()) |
+               reinterpret_cast<uintptr_t>(y.data_ptr()) | reinterpret_cast<uintptr_t>(rp)) % 16 == 0,
+              "gemm_tile_unit: alignment");
+  check(k8sllm_gemm_tile_unit(x.data_ptr(), w.data_ptr(), y.data_ptr(), rp, (int)x.size(0), (int)w.size(0), (int)x.size(1), (int)f, (int)epi,
+                              cur()),
+        "gemm_tile_unit");
 }
 
 // 256 x 256 MFMA GEMM (gemm_tile.hip) for prefill-sized projections: y = x . w^T, x [M, K], w [N, K]
@@ -942,6 +968,7 @@ PYBIND11_MODULE(_k8sllm_ops, m) {
   m.def("layer_norm", &layer_norm);
   m.def("silu_mul", &silu_mul);
   m.def("moe_grouped_gemm", &moe_grouped_gemm);
+  m.def("gemm_tile_unit", &gemm_tile_unit);
   m.def("gemm_tile", &gemm_tile, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("offsets"), py::arg("swiglu"),
         py::arg("algo") = 1, py::arg("rope_pos") = py::none(), py::arg("rope_cs") = py::none(),
         py::arg("rope_heads") = 0, py::arg("rs_part") = py::none(), py::arg("rs_eps") = 1e-5,

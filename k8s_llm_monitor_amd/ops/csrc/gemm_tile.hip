@@ -112,8 +112,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     row0 = mt * 256;
     mrows = min(256, M - row0);
   }
-  const int n0 = nt * 256;
-  const int nrows = min(256, N - n0);
+  // GLU: the unit's tiles first, 128 features each, then the rest's
+  constexpr bool GLU = tile_epi_glu(EPI);
+  const int n_unit = GLU ? (ep.f + 127) >> 7 : 0;
+  const bool unit = GLU && nt < n_unit;
+  const int n0 = GLU ? (unit ? nt * 128 : 2 * ep.f + (nt - n_unit) * 256) : nt * 256;
+  const int nrows = unit ? 2 * min(128, ep.f - n0) : min(256, N - n0);
 
   // ---- DMA of one half-tile (256 rows x 128 B = 32 pieces of 1 KiB): piece p (0..7) of this
   // wave covers rows (p * 4 + wave) * 8 .. + 7; lane -> row + (lane >> 3), physical chunk lane & 7 ----
@@ -123,7 +127,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int rl = (p * 4 + wave) * 8 + (lane >> 3);
     const int cl = (lane & 7) ^ ((rl >> 1) & 7);
     soff[0][p] = (uint32_t)(((long)min(rl, mrows - 1) * K + cl * 8) * 2);  // rows past the end: clamped, never stored
-    soff[1][p] = (uint32_t)(((long)min(rl, nrows - 1) * K + cl * 8) * 2);
+    if constexpr (GLU) {  // rows [64 gate | 64 up] per 128, from the start of W
+      const int wrow = unit ? min(n0 + ((rl >> 7) << 6) + (rl & 63), ep.f - 1) + (rl & 64 ? ep.f : 0) : n0 + min(rl, nrows - 1);
+      soff[1][p] = (uint32_t)(((long)wrow * K + cl * 8) * 2);
+    } else {
+      soff[1][p] = (uint32_t)(((long)min(rl, nrows - 1) * K + cl * 8) * 2);
+    }
     if (wpk) {  // W fragment-packed [N/16][K/32][64][8]: piece = one contiguous 1-KiB block (n-tile, k-step)
       const int blk = p * 4 + wave, j = min(blk >> 1, (nrows >> 4) - 1);
       soff[1][p] = (uint32_t)(((long)j * (K >> 5) + (blk & 1)) * 1024 + lane * 16);
@@ -139,7 +148,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0, nb, 0x00020000);
   };
   const __amdgpu_buffer_rsrc_t xr = rsrc(reinterpret_cast<const char*>(X) + (long)row0 * K * 2, (long)mrows * K * 2);
-  const __amdgpu_buffer_rsrc_t wr = rsrc(reinterpret_cast<const char*>(Wt) + (long)n0 * K * 2, (long)nrows * K * 2);
+  const __amdgpu_buffer_rsrc_t wr = GLU ? rsrc(Wt, (long)N * K * 2)
+                                        : rsrc(reinterpret_cast<const char*>(Wt) + (long)n0 * K * 2, (long)nrows * K * 2);
   const int nk = K >> 6;
 
   // piece p of half-tile (operand o, k-tile kt) into half-slot `slot`; k-tiles past the end re-read
@@ -378,7 +388,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   // the accumulator layout directly, which is what bounds a store tail (T21). ----
   lgkm_wait0();
   __builtin_amdgcn_s_barrier();  // every wave is done with the ring (its last DMAs retired above)
-  constexpr bool SWG = EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8;
+  auto finish = [&](auto gated) {  // gated: a unit's tile
+  constexpr bool SWG = decltype(gated)::value;
   constexpr int OUTW = SWG ? 64 : 128;  // output columns of this wave's quarter
   constexpr int RS_ = OUTW * 2 + 16;                       // LDS row stride (16-B pad: 2-way writes)
   char* stage = smem + wave * (128 * RS_);
@@ -401,14 +412,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   for (int i = 0; i < 8; ++i) {
     __builtin_amdgcn_sched_barrier(0);  // one row block's accumulators at a time (no hoisted AGPR reads)
     char* srow = stage + (i * 16 + ml) * RS_ + nq * 2;
-    if constexpr (EPI == TILE_EPI_SWIGLU) {
+    if constexpr (EPI == TILE_EPI_SWIGLU || (GLU && SWG)) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         float o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float gt = bf2f(f2bf(acc[i][j][r] * sc[i])), up = bf2f(f2bf(acc[i][j + 4][r] * sc[i]));
-          o[r] = gt * up / (1.f + __expf(-gt));
+          o[r] = GLU ? tile_unit<EPI>(gt, up) : gt * up / (1.f + __expf(-gt));
         }
         *reinterpret_cast<uint2*>(srow + j * 32) = uint2{pack2(o[0], o[1]), pack2(o[2], o[3])};
       }
@@ -440,7 +451,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const f32x4 v = acc[i][j] * sc[i];
+        f32x4 v = acc[i][j] * sc[i];
+        if constexpr (EPI == TILE_EPI_RELU_SQ) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float z = bf2f(f2bf(v[r]));
+            v[r] = z > 0.f ? z * z : 0.f;
+          }
+        }
         *reinterpret_cast<uint2*>(srow + j * 32) = uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
       }
     }
@@ -515,13 +533,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   }
   constexpr int CPR = OUTW / 8;  // 16-B chunks per row
   constexpr int RPI = 64 / CPR;  // rows per wave instruction
-  const int ldy = SWG ? (N >> 1) : N;
-  const int col0 = SWG ? ((n0 + wn * 128) >> 1) : n0 + wn * 128;
+  const int ldy = GLU ? (SWG ? ep.f : N - 2 * ep.f) : SWG ? (N >> 1) : N;
+  const int col0 = GLU ? (SWG ? n0 + wn * 64 : n0 - 2 * ep.f + wn * 128) : SWG ? ((n0 + wn * 128) >> 1) : n0 + wn * 128;
   const int ncols = SWG ? (nrows >> 1) - wn * 64 : nrows - wn * 128;
+  bf16_t* const out = GLU && !SWG ? ep.y2 : Y;
   const int rr2 = lane / CPR, cc2 = lane % CPR;
   // branch-free masked stores: a buffer descriptor over this m-tile's rows drops every store past
   // row mrows (out of range), and a lane whose columns are past N gets an out-of-range offset
-  const __amdgpu_buffer_rsrc_t yr = rsrc(Y + (long)row0 * ldy, (long)mrows * ldy * 2);
+  const __amdgpu_buffer_rsrc_t yr = rsrc(out + (long)row0 * ldy, (long)mrows * ldy * 2);
   const uint32_t yo = cc2 * 8 < ncols ? (uint32_t)(((wm * 128 + rr2) * ldy + col0 + cc2 * 8) * 2) : 0x80000000u;
 #pragma unroll
   for (int b = 0; b < 128 / RPI; b += 8) {  // 8 row groups per batch: reads issued back to back
@@ -531,6 +550,13 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       __builtin_amdgcn_raw_buffer_store_b128(v[u], yr, yo + (uint32_t)((b + u) * RPI * ldy * 2), 0, 0);
+  }
+  };
+  if constexpr (GLU) {
+    if (unit) finish(std::true_type{});
+    else finish(std::false_type{});
+  } else {
+    finish(std::bool_constant<EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8>{});
   }
 }
 
@@ -568,7 +594,7 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
              (epi != TILE_EPI_ROPE && !swg)))
     return -1;
   const TileEpi ep{rope_pos, rope_cs, rope_heads, rs_part, rs_np, rs_eps, (bf16_t*)resid, (bf16_t*)hw,
-                   (const bf16_t*)norm_w, ss_out};
+                   (const bf16_t*)norm_w, ss_out, 0, nullptr};
   // 32-bit DMA offsets (X: relative to the tile's first row; W: within one expert / n-tile)
   if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31)) return -3;
   if (epi == TILE_EPI_RESID && 256L * N * 2 >= (1L << 31)) return -3;
@@ -603,5 +629,29 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   }
 #undef K8_TILE_SCH
 #undef K8_TILE_LAUNCH
+  return (int)hipGetLastError();
+}
+
+// Dense, row-major W, a unit at the end (TILE_EPI_*_GLU, TILE_EPI_RELU_SQ, see tile_epi.h).  f, N % 16 == 0, K % 64 == 0, K >= 192.
+// us, the library's product and the unit's launch against this: 7830 rows, 2 x 5632 + 2048 rows of W, K 2048, tanh GELU 388 + 47, 355; 3749
+// rows 236 + 25, 195; squared ReLU, 8000 x 8192 x 2048 200 + 41, 216; 6403 x 4096 x 1024 53 + 18, 58.
+extern "C" int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void* Y2, int M, int N, int K, int f, int epi, hipStream_t s) {
+  if (M <= 0) return 0;
+  const bool glu = tile_epi_glu(epi);
+  if (!glu && epi != TILE_EPI_RELU_SQ) return -1;
+  if (N <= 0 || N % 16 || K % 64 || K < 192 || (glu ? f <= 0 || f % 16 || N < 2 * f : f != 0)) return -1;
+  if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31) || 256L * N * 2 >= (1L << 31)) return -3;
+  const TileEpi ep{nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, f, (bf16_t*)Y2};
+  const int n_mt = (M + 255) / 256, n_nt = glu ? (f + 127) / 128 + (N - 2 * f + 255) / 256 : (N + 255) / 256;
+  const long nwg = (long)n_mt * n_nt;
+  if (nwg > (1L << 30)) return -2;
+#define K8_TILE_UNIT(EPI_)                                                                                             \
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false>), dim3((unsigned)nwg), dim3(256), 0, s, (const bf16_t*)X,    \
+                     (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0)
+  if (epi == TILE_EPI_GELU_GLU) K8_TILE_UNIT(TILE_EPI_GELU_GLU);
+  else if (epi == TILE_EPI_SILU_GLU) K8_TILE_UNIT(TILE_EPI_SILU_GLU);
+  else if (epi == TILE_EPI_RELU_GLU) K8_TILE_UNIT(TILE_EPI_RELU_GLU);
+  else K8_TILE_UNIT(TILE_EPI_RELU_SQ);
+#undef K8_TILE_UNIT
   return (int)hipGetLastError();
 }

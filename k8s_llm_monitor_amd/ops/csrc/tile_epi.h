@@ -5,7 +5,8 @@
 
 namespace k8sllm {
 
-enum { TILE_EPI_BF16 = 0, TILE_EPI_SWIGLU = 1, TILE_EPI_ROPE = 2, TILE_EPI_RESID = 3, TILE_EPI_SWIGLU8 = 4 };
+enum { TILE_EPI_BF16 = 0, TILE_EPI_SWIGLU = 1, TILE_EPI_ROPE = 2, TILE_EPI_RESID = 3, TILE_EPI_SWIGLU8 = 4,
+       TILE_EPI_GELU_GLU = 5, TILE_EPI_SILU_GLU = 6, TILE_EPI_RELU_GLU = 7, TILE_EPI_RELU_SQ = 8 };
 
 // Fused epilogues of the dense prefill projections.
 //
@@ -26,6 +27,10 @@ enum { TILE_EPI_BF16 = 0, TILE_EPI_SWIGLU = 1, TILE_EPI_ROPE = 2, TILE_EPI_RESID
 // RS (row scale, the consumers qkv / gate_up that read hw): every output row is multiplied by
 // rsqrt(sum_c rs_part[row][c] / K + rs_eps) before its epilogue - the deferred half of the RMSNorm
 // (a row scale commutes with the projection; SwiGLU and RoPE see the normalised values).
+//
+// TILE_EPI_*_GLU: W's rows are [f gate | f up | the rest]; a tile of the unit takes 128 features' gate and up rows, arranged while they
+// are loaded as SWIGLU finds them, and writes act(gate) * up (tanh GELU, SiLU, ReLU) of the rounded products to Y [M][f]; the tiles
+// behind write the other rows' products to y2 [M][N - 2 f].  TILE_EPI_RELU_SQ: the squared ReLU of the rounded products.
 struct TileEpi {
   const int* positions;  // ROPE: [M] absolute position of each row
   const float* cos_sin;  // ROPE: [max_pos][128]: cos (64) | sin (64)
@@ -37,7 +42,19 @@ struct TileEpi {
   bf16_t* hw;            // RESID: [M][N] resid * norm_w
   const bf16_t* norm_w;  // RESID: [N] the next RMSNorm's weight
   float* ss_out;         // RESID: [M][N / 128]
+  int f;                 // GLU: features of the unit
+  bf16_t* y2;            // GLU: [M][N - 2 f]
 };
+
+__host__ __device__ constexpr bool tile_epi_glu(int epi) { return epi >= TILE_EPI_GELU_GLU && epi <= TILE_EPI_RELU_GLU; }
+
+// The gated units.  tanh GELU as z / (1 + exp(-2 t)): the same function without the cancellation of 1 + tanh t.
+template <int EPI>
+__device__ __forceinline__ float tile_unit(float g, float u) {
+  if (EPI == TILE_EPI_RELU_GLU) return fmaxf(g, 0.f) * u;
+  const float t = EPI == TILE_EPI_GELU_GLU ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
+  return g * u / (1.f + __expf(-t));
+}
 
 // sum over the 16 lanes of a DPP row (lanes 16r .. 16r + 15), the total in every lane
 __device__ __forceinline__ float row16_sum(float v) {

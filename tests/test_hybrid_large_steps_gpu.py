@@ -536,6 +536,37 @@ def test_few_rows_forms(M, f, rest, K, shared):
         assert torch.equal(a, hops.glu(y, 0, f, kind)) and torch.equal(q, y[:, 2 * f:])
 
 
+@pytest.mark.parametrize("M", [1, 257, 600])
+@pytest.mark.parametrize("f,rest,K", [(128, 0, 192), (144, 48, 256), (400, 272, 320), (16, 256, 192)])  # tiles of 128 features and 256 columns
+@pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
+def test_gated_unit_in_the_tile_gemm(M, f, rest, K, kind):
+    """The tile GEMM's gated unit and the rows behind it against 64 bits: whole and partial tiles of both.  Two rounded factors and a
+    rounded product: 2^-7 of it, and 2^-8 of each factor's unit scale where the other is small."""
+    from k8s_llm_monitor_amd import ops
+
+    g = _g(91)
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, 2 * f + rest, K, s=K ** -0.5, dt=BF).cuda()
+    a, y = (torch.full((M, n), float("nan"), dtype=BF, device="cuda") for n in (f, rest))
+    ops.native().gemm_tile_unit(a, y, x, w, hops.TILE_UNITS[kind])
+    z = x.double() @ w.double().t()
+    p, u = z[:, :f], z[:, f:2 * f]
+    t = {"gelu_tanh": lambda v: F.gelu(v, approximate="tanh"), "silu": F.silu, "relu": F.relu}[kind](p)
+    assert bool(((a.double() - t * u).abs() <= 2 ** -7 * (t * u).abs() + 2 ** -8 * (t.abs() + 1.2 * p.abs() * u.abs()) + 1e-5).all())
+    assert bool(((y.double() - z[:, 2 * f:]).abs() <= 2 ** -8 * z[:, 2 * f:].abs() + 1e-6 * K ** 0.5).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 192), (300, 272, 256), (256, 512, 320)])
+def test_squared_relu_in_the_tile_gemm(M, N, K):
+    from k8s_llm_monitor_amd import ops
+
+    g = _g(92)
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
+    y = torch.empty(M, N, dtype=BF, device="cuda")
+    ops.native().gemm_tile_unit(y, None, x, w, hops.TILE_UNITS["relu_sq"])
+    z = torch.relu(x.double() @ w.double().t())
+    assert bool(((y.double() - z ** 2).abs() <= 3 * 2 ** -8 * z ** 2 + 1e-5).all())  # twice the rounding of z, once that of its square
+
+
 def test_linear_of_nothing():
     """Empty sums, no columns, no rows and no gated unit are what the library makes of them."""
     g = _g(89)
