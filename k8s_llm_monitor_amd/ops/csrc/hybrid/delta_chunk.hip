@@ -18,11 +18,14 @@
 //    take the six products of two three-part operands that matter at 2^-24.  R and S pass between the waves through
 //    LDS as three parts; all other operands are fetched straight into operand registers one chunk ahead.
 // Sums of log2 g are kept in 64 bits: differences of large sums lose nothing.  Everything else is fp32.
-// What bounds it: the chain K S -> R -> N R -> S per chunk, two barriers long; the workspace's traffic (72 KiB per chunk and
-// head, read by every column block, at dk 128).
-// Measured, 16 heads of 128 x 128 on 8 key heads, both launches (us; the staged scan with its preparation): 1 x 8000 rows 412
-// (1599), 4 x 2048 212 (544), 8 heads, 13 x 500 114 (267).  Error against 64 bits at 4 x 2048: outputs 1.9e-7 (scan 3.0e-7),
+// What bounds it: the chain K S -> R -> N R -> S per chunk, two barriers long, 1.3 us without its loads; the workspace's traffic (72 KiB
+// per chunk and head, read by every column block, at dk 128), 0.8 us of a workgroup's load path.  Loads at the head of a chunk delayed its
+// chain by all of that, branches around them made their first use wait for them: 2.5 us a chunk, 2.2 now.
+// Measured, 16 heads of 128 x 128 on 8 key heads, both launches (us; the staged scan with its preparation): 1 x 8000 rows 362
+// (1599), 4 x 2048 219 (544); 32 heads on 16, 4000 + 3000 + 1000 rows 472 (522 before).  Error against 64 bits at 4 x 2048: outputs 1.9e-7 (scan 3.0e-7),
 // state 1.7e-7 (3.1e-7).
+#include <type_traits>
+
 #include "chunk_seg.h"
 #include "split_bf16.h"
 
@@ -321,150 +324,175 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
       }
     }
   };
-  // operands of a chunk, fetched one chunk ahead: this wave's 16 rows of Q or K, their row factors, M's tiles or N's,
-  // the values that R starts from
+  // operands of a chunk, fetched one chunk ahead (two sets in turn): this wave's 16 rows of Q or K, their row factors, M's tiles or
+  // N's, the values that R starts from
   constexpr int NF = RTW > 1 ? 6 * RTW : 6;
-  bf16x8 rf[KS], mf[NF], rn[KS], mn[NF];
-  float gf[4], gn_[4], dl = 1.f, dn = 1.f;  // outs: gf[0] is this lane's query
-  bf16_t vf[4][NT], vn[4][NT];
+  struct Operands {
+    bf16x8 rows[KS], m[NF];
+    float f[4], dl;  // outs: f[0] is this lane's query
+    bf16_t v[4][NT];
+  } ops[2];
   const bf16_t* rb = qkv + (outs ? q_col : k_col) + (long)g * DK + 8 * quad;
-  auto fetch = [&](int tb) {
+  // The same number of loads for every chunk and wave of a kind, with no branch around them (past the last chunk they repeat it): only
+  // then does the use of one chunk's operands leave the next one's on their way.
+  auto fetch = [&](auto queries, int tb, Operands& x) {
+    tb = min(tb, t0 + (t1 - 1 - t0) / kChunk * kChunk);
     const int n = min(kChunk, t1 - tb);
     const long ch = (long)(c0 + (tb - t0) / kChunk) * H + h;
     const bf16_t* r = rb + (long)(tb + min(16 * w + c16, n - 1)) * stride;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) rn[ks] = *reinterpret_cast<const bf16x8*>(r + 32 * ks);
+    for (int ks = 0; ks < KS; ++ks) x.rows[ks] = *reinterpret_cast<const bf16x8*>(r + 32 * ks);
     const bf16_t* m = mats + ch * dc_mats(DK) + lane * 8;
     const float* f = fac + ch * kDcFac;
-    if (outs) {
+    if constexpr (decltype(queries)::value) {
 #pragma unroll
-      for (int i = 0; i < 6; ++i)
-        if (i < 3 || w >= 2) mn[i] = *reinterpret_cast<const bf16x8*>(m + (long)(6 * w + i) * 512);
-      gn_[0] = f[16 * w + c16];
+      for (int i = 0; i < 6; ++i) x.m[i] = *reinterpret_cast<const bf16x8*>(m + (long)(6 * w + i) * 512);
+      x.f[0] = f[16 * w + c16];
     } else {
       m += 3 * 64 * 64;
 #pragma unroll
-      for (int i = 0; i < 6 * RTW; ++i)
-        if (mine) mn[i] = *reinterpret_cast<const bf16x8*>(m + (long)min(6 * w * RTW + i, 12 * KS - 1) * 512);
-      dn = f[128];
+      for (int i = 0; i < 6 * RTW; ++i) x.m[i] = *reinterpret_cast<const bf16x8*>(m + (long)min(6 * w * RTW + i, 12 * KS - 1) * 512);
+      x.dl = f[128];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        gn_[i] = f[64 + 16 * w + 4 * quad + i];
+        x.f[i] = f[64 + 16 * w + 4 * quad + i];
         const bf16_t* v = qkv + (long)(tb + min(16 * w + 4 * quad + i, n - 1)) * stride + v_col + (long)h * dv + dvb + c16;
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) vn[i][ct] = v[16 * ct];
+        for (int ct = 0; ct < NT; ++ct) x.v[i][ct] = v[16 * ct];
       }
     }
   };
-  fetch(t0);
   publish();
   if (tid < NV) first[tid] = kNone;
-  for (int tb = t0; tb < t1; tb += kChunk) {
+  // three parts' products with this wave's rows; QUERIES: (S^T Q^T)[column 16 ct + 4 quad + i][query c16], else (K S)[token 4 quad +
+  // i][column c16].  All of the state's fragments are on their way before the first product.
+  auto dots = [&](auto queries, const bf16x8 (&rows)[KS], int ct) {
+    bf16x8 x[KS][3];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[ks][k] = *reinterpret_cast<const bf16x8*>(&Sl[k][(16 * ct + c16) * PK + 32 * ks + 8 * quad]);
+    f32x4 part[3] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}, sum;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        part[k] = decltype(queries)::value ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[ks][k], rows[ks], part[k], 0, 0, 0)
+                                           : __builtin_amdgcn_mfma_f32_16x16x32_bf16(rows[ks], x[ks][k], part[k], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = (part[2][i] + part[1][i]) + part[0][i];
+    return sum;
+  };
+  auto query_chunk = [&](int tb, const Operands& c, auto&& ahead) {
     const int n = min(kChunk, t1 - tb);
-#pragma unroll
-    for (int i = 0; i < KS; ++i) rf[i] = rn[i];
-#pragma unroll
-    for (int i = 0; i < NF; ++i) mf[i] = mn[i];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      gf[i] = gn_[i];
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct) vf[i][ct] = vn[i][ct];
-    }
-    dl = dn;
-    if (tb + kChunk < t1) fetch(tb + kChunk);
-    lds_barrier();  // Sl is written, Rl has been read
-    // outs: (S^T Q^T)[column 16 ct + 4 quad + i][query c16]; else (K S)[token 4 quad + i][column c16]
     f32x4 acc[NT];
 #pragma unroll
+    for (int ct = 0; ct < NT; ++ct) acc[ct] = dots(std::true_type{}, c.rows, ct);
+    ahead();
+    lds_barrier();  // Rl is written, Sl has been read
+    if (16 * w >= n) return;
+#pragma unroll
     for (int ct = 0; ct < NT; ++ct) {
-      f32x4 part[3] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+      f32x4 d[2];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
+      for (int i = 0; i < 4; ++i) d[0][i] = acc[ct][i] * c.f[0], d[1][i] = 0.f;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const bf16x8 x = *reinterpret_cast<const bf16x8*>(&Sl[k][(16 * ct + c16) * PK + 32 * ks + 8 * quad]);
-          part[k] = outs ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, rf[ks], part[k], 0, 0, 0)
-                         : __builtin_amdgcn_mfma_f32_16x16x32_bf16(rf[ks], x, part[k], 0, 0, 0);
-        }
+      for (int ks = 0; ks < 2; ++ks) {
+        if (ks == 1 && w < 2) continue;  // M is lower triangular
+        bf16x8 x[3];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[ct][i] = (part[2][i] + part[1][i]) + part[0][i];
-    }
-    if (!outs) {
+        for (int k = 2; k >= 0; --k) x[k] = *reinterpret_cast<const bf16x8*>(&Rl[k][(16 * ct + c16) * kDcP + 32 * ks + 8 * quad]);
 #pragma unroll
-      for (int ct = 0; ct < NT; ++ct) {
-        float x[4];
+        for (int k = 2; k >= 0; --k)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          x[i] = bf2f(vf[i][ct]) - gf[i] * acc[ct][i];
-          if (!isfinite(x[i])) {
-            const int row = 16 * w + 4 * quad + i;
-            if (row < n) atomicMin(&first[16 * ct + c16], row);
-            x[i] = 0.f;
-          }
-        }
-        uint32_t p[3][2];
-        split_pairs<2>(x, p[0], p[1], p[2]);
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          *reinterpret_cast<uint2*>(&Rl[k][(16 * ct + c16) * kDcP + 16 * w + 4 * quad]) = make_uint2(p[k][0], p[k][1]);
+          for (int m = 2 - k; m >= 0; --m) d[m & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[k], c.m[3 * ks + m], d[m & 1], 0, 0, 0);
       }
+      const int4 f = *reinterpret_cast<const int4*>(&first[16 * ct + 4 * quad]);
+      const int q = 16 * w + c16;
+      if (q < n)
+        *reinterpret_cast<float4*>(o + (long)(tb + q) * inner + (long)h * dv + dvb + 16 * ct + 4 * quad) =
+            make_float4(q < f.x ? d[0][0] + d[1][0] : NAN, q < f.y ? d[0][1] + d[1][1] : NAN, q < f.z ? d[0][2] + d[1][2] : NAN,
+                        q < f.w ? d[0][3] + d[1][3] : NAN);
+    }
+  };
+  auto key_chunk = [&](int tb, const Operands& c, auto&& ahead) {
+    const int n = min(kChunk, t1 - tb);
+    f32x4 acc[NT];
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct) acc[ct] = dots(std::false_type{}, c.rows, ct);
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct) {
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = bf2f(c.v[i][ct]) - c.f[i] * acc[ct][i];
+        if (!isfinite(x[i])) {
+          const int row = 16 * w + 4 * quad + i;
+          if (row < n) atomicMin(&first[16 * ct + c16], row);
+          x[i] = 0.f;
+        }
+      }
+      uint32_t p[3][2];
+      split_pairs<2>(x, p[0], p[1], p[2]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        *reinterpret_cast<uint2*>(&Rl[k][(16 * ct + c16) * kDcP + 16 * w + 4 * quad]) = make_uint2(p[k][0], p[k][1]);
     }
     lds_barrier();  // Rl is written, Sl has been read
-    if (outs) {
-      if (16 * w < n) {
+    if (!mine) return ahead();
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-          f32x4 d[2];
+    for (int ct = 0; ct < NT; ++ct)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) d[0][i] = acc[ct][i] * gf[0], d[1][i] = 0.f;
+      for (int r = 0; r < RTW; ++r)
 #pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            if (ks == 1 && w < 2) continue;  // M is lower triangular
+        for (int i = 0; i < 4; ++i) S[r][ct][i] *= c.dl;
+    bf16x8 x[2][NT][3];
 #pragma unroll
-            for (int k = 2; k >= 0; --k) {
-              const bf16x8 x = *reinterpret_cast<const bf16x8*>(&Rl[k][(16 * ct + c16) * kDcP + 32 * ks + 8 * quad]);
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-              for (int m = 2 - k; m >= 0; --m) d[m & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, mf[3 * ks + m], d[m & 1], 0, 0, 0);
-            }
-          }
-          const int4 f = *reinterpret_cast<const int4*>(&first[16 * ct + 4 * quad]);
-          const int q = 16 * w + c16;
-          if (q < n)
-            *reinterpret_cast<float4*>(o + (long)(tb + q) * inner + (long)h * dv + dvb + 16 * ct + 4 * quad) =
-                make_float4(q < f.x ? d[0][0] + d[1][0] : NAN, q < f.y ? d[0][1] + d[1][1] : NAN, q < f.z ? d[0][2] + d[1][2] : NAN,
-                            q < f.w ? d[0][3] + d[1][3] : NAN);
-        }
+      for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+        for (int k = 2; k >= 0; --k) x[ks][ct][k] = *reinterpret_cast<const bf16x8*>(&Rl[k][(16 * ct + c16) * kDcP + 32 * ks + 8 * quad]);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+        for (int k = 2; k >= 0; --k)
+#pragma unroll
+          for (int m = 2 - k; m >= 0; --m)
+#pragma unroll
+            for (int r = 0; r < RTW; ++r)
+              S[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.m[6 * r + 3 * ks + m], x[ks][ct][k], S[r][ct], 0, 0, 0);
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct)
+      if (first[16 * ct + c16] < kNone) {
+#pragma unroll
+        for (int r = 0; r < RTW; ++r) S[r][ct] = f32x4{NAN, NAN, NAN, NAN};
       }
-    } else if (mine) {
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-        for (int r = 0; r < RTW; ++r)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) S[r][ct][i] *= dl;
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-          for (int k = 2; k >= 0; --k) {
-            const bf16x8 x = *reinterpret_cast<const bf16x8*>(&Rl[k][(16 * ct + c16) * kDcP + 32 * ks + 8 * quad]);
-#pragma unroll
-            for (int m = 2 - k; m >= 0; --m)
-#pragma unroll
-              for (int r = 0; r < RTW; ++r)
-                S[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf[6 * r + 3 * ks + m], x, S[r][ct], 0, 0, 0);
-          }
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct)
-        if (first[16 * ct + c16] < kNone) {
-#pragma unroll
-          for (int r = 0; r < RTW; ++r) S[r][ct] = f32x4{NAN, NAN, NAN, NAN};
-        }
-      publish();
+    publish();
+    ahead();
+  };
+  // The two kinds of waves walk the chunks apart, meeting at two barriers each.  The next chunk's loads take a wave up to 0.8 us to
+  // issue (104 KB a chunk and workgroup): the keys' waves do that when their state is published, the queries' behind their first products.
+  auto walk = [&](auto queries, auto&& work) {
+    auto chunk = [&](int tb, const Operands& c, Operands& next) {
+      lds_barrier();  // Sl is written, Rl has been read
+      work(tb, c, [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(queries, tb + kChunk, next);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    fetch(queries, t0, ops[0]);
+    for (int tb = t0; tb < t1; tb += 2 * kChunk) {
+      chunk(tb, ops[0], ops[1]);
+      if (tb + kChunk >= t1) break;
+      chunk(tb + kChunk, ops[1], ops[0]);
     }
-  }
+  };
+  if (outs) walk(std::true_type{}, query_chunk);
+  else walk(std::false_type{}, key_chunk);
   if (mine) {
 #pragma unroll
     for (int r = 0; r < RTW; ++r)
