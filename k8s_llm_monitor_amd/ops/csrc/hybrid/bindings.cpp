@@ -449,9 +449,8 @@ void conv_silu(Tensor out, Tensor proj, int64_t col0, Tensor cw, OptT cb, Tensor
 // mode 0: with a decay table and G == nh, the chunked matrix-core kernel for bf16 steps with a mean of 32 rows per segment
 // and more whose sizes are its own, else a scan; 1 / 2: a scan in the decode / prompt mapping; 3: the chunked kernel (nt: its
 // value-column tiles per workgroup, 0: its choice), or the scan where it does not apply.  singles: so many segments in front are
-// running sequences' next tokens; where only the longest segment brings the chunks they stay on the decode mapping beside them (us,
-// in the chunked kernel -> beside it: 200 and 2 x 1000 236 -> 137, 60 and one of 256 68 -> 45; with a mean of 32 rows they run in the
-// shadow of the long chains: 60 and one of 2000 115 / 133, 32 and 2 x 2048 110 / 120)
+// running sequences' next tokens, which stay on the decode mapping beside the chunks (us, in the chunked kernel -> beside it: 200 and 2 x
+// 1000 236 -> 137, 60 and one of 256 68 -> 45, 32 and 2048 + 1500 104 -> 78)
 void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, OptT a_log, OptT d_skip, OptT decay,
               Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t nh, int64_t P, int64_t N, int64_t G,
               int64_t mode, int64_t nt, int64_t longest, int64_t singles) {
@@ -494,7 +493,6 @@ void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, Opt
                              (int)segments, rows, (int)nh, (int)P, (int)N, (int)G, f, (int)m, cur()),
           "ssm_scan");
   };
-  if (T >= 32 * S) singles = 0;
   if (cp != nullptr && !f && G == nh && singles < S && (mode == 3 || (mode == 0 && (T >= 32 * S || longest >= 256))) &&
       reinterpret_cast<uintptr_t>(xbc.data_ptr()) % 16 == 0) {
     const int rc = k8sllm_hy_chunk_scan(y.data_ptr<float>(), xbc.data_ptr(), cp, state.data_ptr<float>(), cu.data_ptr<int>() + singles,

@@ -18,10 +18,11 @@
 // are row-major in LDS and read down the columns by the transposing LDS read; the state is republished there once per
 // chunk as three bf16 parts, [column][key dim].  The next chunk's rows are fetched into registers while this chunk's
 // products run.
-// What bounds it: the chain of LDS round trips and two barriers per chunk (3.2 to 4.6 us a chunk and workgroup; the vector
-// instructions of the splits would take 1 us, the matrix instructions half of that).
-// Measured, bf16, 16 heads of 128 x 128: 5 x 1600 rows 129 us (the sequential scan 314; chunks whose fp32 products ran on the
-// fp32 matrix instruction 296), 1 x 8000 rows 403 us (1068; 1400).  Error against 64 bits, 1600 rows: outputs 1.4e-7 (scan
+// What bounds it: the chain of LDS round trips and two barriers per chunk, 1.7 us (16 columns) to 4.4 us (64) a chunk and workgroup.
+// Its fragments are on their way before the first product that takes one, and no LDS read or prefetched row stands behind a
+// branch or goes through scratch: with one wait for every read and product it was 3.2 to 5.4 us.
+// Measured, bf16, 16 heads of 128 x 128: 5 of 1500 to 1637 rows 113 us (the sequential scan 314; before 138), 1 x 8000 rows 216 us (1068;
+// before 402).  Error against 64 bits, 1600 rows: outputs 1.4e-7 (scan
 // 2.2e-7), state 1.3e-7 (2.2e-7).
 #include "chunk_seg.h"
 #include "split_bf16.h"
@@ -31,7 +32,7 @@ namespace k8sllm {
 constexpr int kCsChunk = kChunk;
 
 template <int KS, int NT>  // key dim / 32, value columns / 16 per workgroup
-__global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ y, const bf16_t* __restrict__ vkq,
+__global__ __launch_bounds__(512, 2) void chunk_scan_kernel(float* __restrict__ y, const bf16_t* __restrict__ vkq,
                                                          const float* __restrict__ decay,
                                                          float* __restrict__ state, const int* __restrict__ cu,
                                                          const int* __restrict__ ctx, const int* __restrict__ slot, int S_,
@@ -79,7 +80,8 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
         const int row = 16 * (w * RTW + r) + 4 * quad + i;
         S[r][ct][i] = carried && !outs && row < DK ? sp[(long)row * dv + 16 * ct + c16] : 0.f;
       }
-  uint4 rk[KU];
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // (an array of uint4 went through scratch or LDS behind its loads)
+  u32x4 rk[KU];
   uint32_t rv[VPT / 2];
   bf16x8 qn[KS];
   const int vr = tid / (NV / VPT), vc = VPT * (tid % (NV / VPT));  // the value row and columns this thread stages
@@ -87,7 +89,7 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       const int idx = min(tid + 512 * u, kCsChunk * DK / 8 - 1), row = idx / (DK / 8), c8 = idx - row * (DK / 8);
-      rk[u] = *reinterpret_cast<const uint4*>(kcol + (long)(tb + min(row, n - 1)) * C + 8 * c8);
+      rk[u] = *reinterpret_cast<const u32x4*>(kcol + (long)(tb + min(row, n - 1)) * C + 8 * c8);
     }
     const bf16_t* v = vcol + (long)(tb + min(vr, n - 1)) * C + vc;
     if constexpr (VPT == 2) {
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       const int idx = tid + 512 * u, row = idx / (DK / 8), c8 = idx - row * (DK / 8);
-      if (KS % 2 == 0 || idx < kCsChunk * DK / 8) *reinterpret_cast<uint4*>(&Kl[row * PK + 8 * c8]) = rk[u];
+      if (KS % 2 == 0 || idx < kCsChunk * DK / 8) *reinterpret_cast<u32x4*>(&Kl[row * PK + 8 * c8]) = rk[u];
     }
     {
       const float f = vr < n ? lam[n - 1 - vr] : 0.f;
@@ -161,24 +163,24 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
     if (outs && 16 * w < n) {
       const int qi = 16 * w + c16;
       // o[ct][i]: query 16 w + c16, value column 16 ct + 4 quad + i; the three parts in chains of their own
-      f32x4 o[NT], part[3][NT];
+      // (each block's fragments are on their way before its first product)
+      f32x4 o[NT];
 #pragma unroll
-      for (int ct = 0; ct < NT; ++ct)
+      for (int ct = 0; ct < NT; ++ct) {
+        bf16x8 x[KS][3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) part[k][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
+          for (int k = 0; k < 3; ++k) x[ks][k] = *reinterpret_cast<const bf16x8*>(&Sl[k][(16 * ct + c16) * PK + 32 * ks + 8 * quad]);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 part[3] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct)
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&Sl[k][(16 * ct + c16) * PK + 32 * ks + 8 * quad]);
-            part[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], part[k][ct], 0, 0, 0);
-          }
+          for (int k = 0; k < 3; ++k) part[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[ks][k], qf[ks], part[k], 0, 0, 0);
 #pragma unroll
-      for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[ct][i] = (part[2][ct][i] + part[1][ct][i]) + part[0][ct][i];
+        for (int i = 0; i < 4; ++i) o[ct][i] = (part[2][i] + part[1][i]) + part[0][i];
+      }
       const float gq = lam[qi + 1];
 #pragma unroll
       for (int ct = 0; ct < NT; ++ct)
@@ -187,35 +189,34 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
 #pragma unroll
       for (int kp = 0; kp < 2; ++kp) {  // pairs of 16-key tiles
         if (2 * kp <= w) {
-          float p[8];
+          float p[8], decays[8];  // read for every key: a read behind a condition is a branch and a wait each
+          bf16x8 a[2][KS], v[NT];
 #pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int kt = 2 * kp + u;
-            if (kt <= w) {
-              f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int u = 0; u < 2; ++u)
 #pragma unroll
-              for (int ks = 0; ks < KS; ++ks) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(&Kl[(16 * kt + c16) * PK + 32 * ks + 8 * quad]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], acc, 0, 0, 0);
-              }
+            for (int ks = 0; ks < KS; ++ks)
+              a[u][ks] = *reinterpret_cast<const bf16x8*>(&Kl[(32 * kp + 16 * u + c16) * PK + 32 * ks + 8 * quad]);
 #pragma unroll
-              for (int i = 0; i < 4; ++i) {  // acc[i]: key 16 kt + 4 quad + i
-                const int j = 16 * kt + 4 * quad + i;
-                p[4 * u + i] = j <= qi ? acc[i] * lam[qi - j] : 0.f;
-              }
-            } else {
+          for (int i = 0; i < 8; ++i) decays[i] = lam[max(qi - (32 * kp + 16 * (i >> 2) + 4 * quad + (i & 3)), 0)];
 #pragma unroll
-              for (int i = 0; i < 4; ++i) p[4 * u + i] = 0.f;
-            }
+          for (int ct = 0; ct < NT; ++ct) v[ct] = frag_down(Vl[0], PV, 32 * kp + 4 * quad, 32 * kp + 16 + 4 * quad, 16 * ct);
+          __builtin_amdgcn_sched_barrier(0);
+          f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][ks], qf[ks], acc[u], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {  // acc[i / 4][i % 4]: key 32 kp + 16 (i / 4) + 4 quad + i % 4
+            const int j = 32 * kp + 16 * (i >> 2) + 4 * quad + (i & 3);
+            p[i] = j <= qi ? acc[i >> 2][i & 3] * decays[i] : 0.f;
           }
           uint32_t pw[3][4];
           split_pairs<4>(p, pw[0], pw[1], pw[2]);
 #pragma unroll
-          for (int ct = 0; ct < NT; ++ct) {
-            const bf16x8 a = frag_down(Vl[0], PV, 32 * kp + 4 * quad, 32 * kp + 16 + 4 * quad, 16 * ct);
+          for (int k = 2; k >= 0; --k)
 #pragma unroll
-            for (int k = 2; k >= 0; --k) o[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, frag(pw[k]), o[ct], 0, 0, 0);
-          }
+            for (int ct = 0; ct < NT; ++ct) o[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[ct], frag(pw[k]), o[ct], 0, 0, 0);
         }
       }
 #pragma unroll
@@ -249,13 +250,15 @@ __global__ __launch_bounds__(512, 4) void chunk_scan_kernel(float* __restrict__ 
 #pragma unroll
           for (int r = 0; r < RTW; ++r) a[r] = frag_down(Kl, PK, r0, r0 + 4, 16 * min(w * RTW + r, 2 * KS - 1));
 #pragma unroll
-          for (int k = 2; k >= 0; --k)
+          for (int k = 2; k >= 0; --k) {
+            bf16x8 b[NT];
 #pragma unroll
-            for (int ct = 0; ct < NT; ++ct) {
-              const bf16x8 b = frag_down(Vl[k + 1], PV, r0, r0 + 4, 16 * ct);
+            for (int ct = 0; ct < NT; ++ct) b[ct] = frag_down(Vl[k + 1], PV, r0, r0 + 4, 16 * ct);
 #pragma unroll
-              for (int r = 0; r < RTW; ++r) S[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b, S[r][ct], 0, 0, 0);
-            }
+            for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+              for (int r = 0; r < RTW; ++r) S[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b[ct], S[r][ct], 0, 0, 0);
+          }
         }
       }
     }
@@ -284,12 +287,13 @@ extern "C" int k8sllm_hy_chunk_scan(float* y, const void* vkq, const float* deca
   if (dk % 32 || dk < 32 || dk > 128 || dv % 16 || dv < 16 || H < 1) return 1;
   if (nt != 0 && nt != 1 && nt != 2 && nt != 4) return -1;
   if (nt > 1 && dv % (16 * nt)) return 1;
-  // column blocks repeat the scores' products, so wide ones once they give enough workgroups to fill the chip; those of 32 columns
-  // only where 64 do not divide (us for 16 / 32 / 64 columns, 16 heads of 128 x 128: 5 x 1600 rows 184 / 161 / 129; 1 x 8000
-  // 403 / 617 / 574; 1000, 900, 800, 300 and three short 62 / 90 / 82; 2 x 2048 beside 32 single tokens 113 / 169 / 149).
-  // Segments count by the longest one's length (0: not known): single tokens beside it are a chunk each
+  // column blocks repeat the scores' products, and a CU holds one: the narrowest that give it no second one (us for 16 / 32 / 64 columns,
+  // 128 x 128: 16 heads, 1 x 8000 rows 216 / 340 / 500; 2 x 4000 118 / 177 / 251; 3 x 2700 154 / 124 / 174; 4 x 2048 118 / 95 / 131; 5 of
+  // 1500 to 1637 143 / 149 / 113; 16 x 500 125 / 100 / 76).  Segments count by the longest one's length (0: not known): short ones beside it
+  // are a chunk or two each
   const long pairs = (longest > 0 ? min((long)S, (T + longest - 1) / longest) : S) * H;
-  if (nt == 0) nt = dv % 64 == 0 ? (pairs * (dv / 64) >= 144 ? 4 : 1) : dv % 32 == 0 && pairs * (dv / 32) >= 192 ? 2 : 1;
+  if (nt == 0)
+    for (nt = 1; nt < 4 && dv % (32 * nt) == 0 && pairs * (dv / (16 * nt)) > 256;) nt *= 2;
   const dim3 grid((unsigned)(((long)S * H + 7) / 8 * 8 * (dv / (16 * nt))));
 #define K8SLLM_CS(KS, NT)                                                                                           \
   hipLaunchKernelGGL((chunk_scan_kernel<KS, NT>), grid, dim3(512), 0, s, y, (const bf16_t*)vkq, decay, state, cu, ctx, \

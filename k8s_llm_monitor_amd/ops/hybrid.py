@@ -859,8 +859,8 @@ def linear_attention(vkq: torch.Tensor, decay: torch.Tensor, state: torch.Tensor
     multiple of 32 up to 128, ``vdim`` of 16 (``mode`` 3 forces it, ``col_tiles`` 1 / 2 / 4 its value columns per workgroup, 16 / 32 / 64; 0: its choice): chunks of 64
     tokens on the matrix cores, only the state crossing chunks - fp32 scores, decays and state enter the products as three
     bf16 parts that add up to them, so only the order of the fp32 sums differs, which follows the chunk grid from the
-    segment's first row on.  Where it is the longest segment that brings the chunks, the first ``singles`` segments, running
-    sequences' next tokens, stay on the scan of a decode step.  Else the sequential scan (``ssm_scan`` with the decay
+    segment's first row on.  The first ``singles`` segments, running sequences' next tokens, stay on the scan of a decode step
+    beside them.  Else the sequential scan (``ssm_scan`` with the decay
     table; ``mode`` 1 / 2 force its decode / prompt lane mapping)."""
     return ssm_scan(vkq, None, 0, None, None, None, state, seg_cu, seg_ctx, seg_slot, H, dv, dk, H, mode, decay=decay,
                     col_tiles=col_tiles, longest=longest, singles=singles)
