@@ -15,7 +15,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "hy_common.h"
+#include "stream_rows.h"
 
 namespace k8sllm {
 
@@ -640,8 +640,13 @@ constexpr float kMaxCapPlain = 60.f;
 constexpr long kFlashPairs = 16 * 1024;
 constexpr long kFlashKeys = 1024;
 constexpr int kFlashForced = 256;
-template <int DK, int DV, int QT, int CAP>
-__global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
+// WH = 4: four waves, each with its own query head of one kv head, share that head's keys and values.  Register loads of K
+// in fragment order touch 16 rows per 16 lanes, which the load path takes at about a quarter of its rate, and every head
+// fetched every key for itself: 4 x 2048 rows, 16 heads over 4, window 1024: 218 us; through LDS 154.  4 x 1024, 32 heads over
+// 8: 164 -> 122.  The products and their order are the same, so are the bits.  Smaller steps keep one wave per workgroup:
+// there a wave's chain bounds, and the barriers lengthen it (3 x 64 rows: 9.9 us, shared 12.6).
+template <int DK, int DV, int QT, int CAP, int WH>
+__global__ __launch_bounds__(WH ? 64 * WH : 64, WH == 0 || QT == 4 ? 1 : 3) void window_prefill_mfma_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv, long q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ cu, const int* __restrict__ ctx,
     const int* __restrict__ block_tables, int bt_stride, int S, int Hq, int G, float scale, int window,
@@ -661,8 +666,10 @@ __global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
   }
   if (s >= S) return;
   const int q0 = tile * QB, nq = min(QB, n - q0);
-  const int h = blockIdx.y, g = h / (Hq / G);
-  const int lane = threadIdx.x, c16 = lane & 15, quad = lane >> 4;
+  constexpr bool SHARED = WH > 0;
+  const int wave = SHARED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int h = SHARED ? blockIdx.y * WH + wave : blockIdx.y, g = h / (Hq / G);
+  const int lane = threadIdx.x & 63, c16 = lane & 15, quad = lane >> 4;
   const int* bt = block_tables + (long)s * bt_stride;
   const int row0 = cu[s] + q0, p0 = ctx[s] + q0;
   int my_p[QT], my_lo[QT];
@@ -681,20 +688,13 @@ __global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
     for (int ks = 0; ks < DK / 32; ++ks) qf[t][ks] = *reinterpret_cast<const bf16x8*>(qrow + 32 * ks + 8 * quad);
 #pragma unroll
     for (int dt = 0; dt < DV / 16; ++dt) oacc[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    m[t] = sink ? (sinks != nullptr ? sinks[blockIdx.y] * 1.44269504088896341f : 0.f) : -INFINITY;
+    m[t] = sink ? (sinks != nullptr ? sinks[h] * 1.44269504088896341f : 0.f) : -INFINITY;
     l[t] = sink ? 1.f : 0.f;
   }
   const int lo_max = first_key(p0 + nq - 1, window, chunked);  // from here to p0: keys that every row of the tile sees
   const float k1 = CAP ? icap * 2.88539008177792681f : 0.f;
   const int lo_t = first_key(p0, window, chunked), hi = p0 + nq;
   const long krs = (long)G * DK, vrs = (long)G * DV;
-  // Register double buffer: while tile j0 is computed, the K and V^T fragments of tile j0 + 16 are
-  // in flight, and the page id of tile j0 + 32 behind them (no load waits on a load issued in the
-  // same iteration).  A key tile is one 16-token page: its V^T fragments (4 consecutive tokens of
-  // one value dim per lane) are 8-byte loads straight from the d-major page, 512 contiguous bytes
-  // per 16 dims - no LDS, no barrier.
-  const bf16_t* kbase = k_cache + (long)g * DK + 8 * quad;
-  const bf16_t* vbase = v_cache + ((long)g * DV + c16) * 16 + 4 * quad;
   // key tiles: those that hold kept keys (up to kend), then the window's from wfirst on
   const int kend = (min(keep, hi) + 15) & ~15, wfirst = max(kend, lo_t & ~15);
   const int jfirst = kend > 0 ? 0 : wfirst;
@@ -702,30 +702,96 @@ __global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
     j += 16;
     return j >= kend && j < wfirst ? wfirst : j;
   };
-  int pg_n = bt[jfirst >> 4];
-  bf16x8 kf_n[DK / 32];
-  s16x4 vf_n[DV / 16];
-  auto issue = [&](int j0) {  // loads of tile j0 from the page id in pg_n
-    const bf16_t* krow = kbase + (((long)pg_n << 4) + (min(j0 + c16, hi - 1) & 15)) * krs;
+  // SHARED: two tiles at a time come to LDS for all waves (stream_rows.h: K in pieces of 16 keys x 32 dims, V^T as the page has it), a
+  // ring of three such stages with one barrier each; two are on their way while one is computed, the next one's page ids behind them.
+  // Else registers: while a tile is computed, the K and V^T fragments of the next are in flight, and the page id of the one after it.
+  constexpr int KP = DK / 32, VP = DV / 32, W = SHARED ? WH : 1, PK = 2 * KP / W, PV = 2 * VP / W, STAGE = 2 * (KP + VP) * 1024;
+  __shared__ __attribute__((aligned(1024))) char ring[SHARED ? 3 * STAGE : 16];
+  const bf16_t* kbase = k_cache + (long)g * DK + (SHARED ? piece_k() : 8 * quad);
+  const bf16_t* vbase = v_cache + (long)g * DV * 16 + (SHARED ? 8 * lane : 16 * c16 + 4 * quad);
+  constexpr int AHEAD = SHARED ? 2 : 1;
+  int ji = jfirst, jn[AHEAD], pg[AHEAD];  // the tiles that are loaded next and their pages
+  auto pages = [&]() {
 #pragma unroll
-    for (int ks = 0; ks < DK / 32; ++ks) kf_n[ks] = *reinterpret_cast<const bf16x8*>(krow + 32 * ks);
-    const bf16_t* vpg = vbase + (long)pg_n * vrs * 16;
-#pragma unroll
-    for (int dt = 0; dt < DV / 16; ++dt) vf_n[dt] = *reinterpret_cast<const s16x4*>(vpg + dt * 256);
+    for (int u = 0; u < AHEAD; ++u) {
+      jn[u] = ji;
+      pg[u] = bt[min(ji, hi - 1) >> 4];
+      ji = next_tile(ji);
+    }
   };
-  issue(jfirst);
-  int j1 = next_tile(jfirst);
-  pg_n = bt[min(j1, hi - 1) >> 4];
-  for (int j0 = jfirst; j0 < hi; j0 = j1, j1 = next_tile(j1)) {
+  bf16x8 kn[DK / 32];
+  s16x4 vn[DV / 16];
+  auto issue = [&](int slot) {  // (a tile past the last key: the last page once more)
+    if constexpr (SHARED) {
+      char* dst = ring + slot * STAGE;
+#pragma unroll
+      for (int q = 0; q < PK; ++q) {
+        const int i = wave + W * q, u = i / KP, ks = i % KP;
+        const int j = u ? jn[AHEAD - 1] : jn[0];
+        const long row = ((long)(u ? pg[AHEAD - 1] : pg[0]) << 4) + (min(j + piece_row(), hi - 1) & 15);
+        load_piece(dst + i * 1024, kbase + row * krs + 32 * ks);
+      }
+#pragma unroll
+      for (int q = 0; q < PV; ++q) {
+        const int i = wave + W * q, u = i / VP, dp = i % VP;
+        load_piece(dst + (2 * KP + i) * 1024, vbase + (long)(u ? pg[AHEAD - 1] : pg[0]) * vrs * 16 + 512 * dp);
+      }
+    } else {
+      const bf16_t* krow = kbase + (((long)pg[0] << 4) + (min(jn[0] + c16, hi - 1) & 15)) * krs;
+#pragma unroll
+      for (int ks = 0; ks < DK / 32; ++ks) kn[ks] = *reinterpret_cast<const bf16x8*>(krow + 32 * ks);
+      const bf16_t* vpg = vbase + (long)pg[0] * vrs * 16;
+#pragma unroll
+      for (int dt = 0; dt < DV / 16; ++dt) vn[dt] = *reinterpret_cast<const s16x4*>(vpg + dt * 256);
+    }
+  };
+  const int kfrag = piece_frag(), vfrag = c16 * 32 + quad * 8;
+  pages();
+  issue(0);
+  pages();
+  if (SHARED) {
+    issue(1);
+    pages();
+  }
+  int slot = 0;
+  for (int j2 = jfirst; j2 < hi;) {
+   const char* src = ring;
+   if (SHARED) {
+    loads_left<PK + PV>();  // this stage's, of this wave
+    __builtin_amdgcn_s_barrier();  // of all waves; and the slot filled next has been read
+    issue(slot == 0 ? 2 : slot - 1);
+    pages();
+    src = ring + slot * STAGE;
+    slot = slot == 2 ? 0 : slot + 1;
+   }
+#pragma unroll 1
+   for (int u = 0; u < AHEAD; ++u) {
+    const int j0 = j2;
+    j2 = next_tile(j2);
+    if (j0 >= hi) break;
     bf16x8 kf[DK / 32];
     s16x4 vf[DV / 16];
 #pragma unroll
-    for (int ks = 0; ks < DK / 32; ++ks) kf[ks] = kf_n[ks];
+    for (int ks = 0; ks < DK / 32; ++ks) kf[ks] = SHARED ? *reinterpret_cast<const bf16x8*>(src + (u * KP + ks) * 1024 + kfrag) : kn[ks];
+    if constexpr (!SHARED) {
 #pragma unroll
-    for (int dt = 0; dt < DV / 16; ++dt) vf[dt] = vf_n[dt];
-    if (j1 < hi) {
-      issue(j1);
-      pg_n = bt[min(next_tile(j1), hi - 1) >> 4];
+      for (int dt = 0; dt < DV / 16; ++dt) vf[dt] = vn[dt];
+      if (j2 < hi) {
+        issue(0);
+        pages();
+      }
+    }
+    f32x4 scores[QT];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) scores[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < DK / 32; ++ks)
+#pragma unroll
+      for (int t = 0; t < QT; ++t) scores[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[t][ks], scores[t], 0, 0, 0);
+    if constexpr (SHARED) {  // (behind the scores' products, which need the keys only)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int dt = 0; dt < DV / 16; ++dt) vf[dt] = *reinterpret_cast<const s16x4*>(src + (2 * KP + u * VP) * 1024 + dt * 512 + vfrag);
     }
     if (j0 + 16 > hi) {  // the last page's unused end (wave-uniform)
       const int j = j0 + 4 * quad;
@@ -742,9 +808,7 @@ __global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
     const bool inner = (j0 >= lo_max || j0 + 15 < keep) && j0 + 15 <= p0;  // wave-uniform: every row sees every key
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-      f32x4 sacc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < DK / 32; ++ks) sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[t][ks], sacc, 0, 0, 0);
+      const f32x4 sacc = scores[t];
       if constexpr (CAP == 2) {
         float pv[4];
 #pragma unroll
@@ -805,7 +869,9 @@ __global__ __launch_bounds__(64) void window_prefill_mfma_kernel(
 #pragma unroll
       for (int t = 0; t < QT; ++t) oacc[t][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, pb[t], oacc[t][dt], 0, 0, 0);
     }
+   }
   }
+  if (SHARED) loads_left<0>();  // none may land after the workgroup's end
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
     if (CAP == 2) l[t] = xor32_sum_f(xor16_sum(l[t]));
@@ -871,18 +937,26 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
                                             sinks, gate, g_stride, s);
       if (rc != 1 || mfma == kFlashForced) return rc;
     }
-    // query rows per wave: 32 once the step is large enough to fill the chip that way (two row tiles
-    // share every K / V^T fragment), else 16; mfma = 16 / 32 / 64 forces one (tests, measurements)
-    const int qrows = mfma >= 16 ? mfma : (T * Hq >= 64 * 1024 ? 32 : 16);
-    const dim3 grid((unsigned)(T / qrows + S), (unsigned)Hq);
-#define K8SLLM_WPC(DK, DV, QT, CAP)                                                                                    \
-  hipLaunchKernelGGL((window_prefill_mfma_kernel<DK, DV, QT, CAP>), grid, dim3(64), 0, s, (bf16_t*)out,                 \
+    // query rows per wave: 32 once the step is large enough to fill the chip that way (two row tiles share every K / V^T
+    // fragment), else 16; mfma = 16 / 32 / 64 forces one (tests, measurements).  With 32 rows four heads of one kv head,
+    // where it has them, share the keys and values through LDS, and that pays from fewer (row, head) pairs.  16 rows -> 32
+    // rows shared, us, 8 heads over 2 kv heads: 16384 pairs 45 -> 57 and 28 -> 33; 26000 (13 x 250) 22.0 -> 20.4; 32768
+    // 75 -> 61; 52000 (13 x 500) 64 -> 40; 64000 behind 2800 keys 199 -> 90.
+    const bool share = Hq / G % 4 == 0;
+    const int qrows = mfma >= 16 ? mfma : (T * Hq >= (share ? 24 : 64) * 1024 ? 32 : 16);
+    const int wh = share && qrows == 32 ? 4 : 0;
+    const dim3 grid((unsigned)(T / qrows + S), (unsigned)(wh ? Hq / wh : Hq));
+#define K8SLLM_WPC(DK, DV, QT, CAP)                            \
+  if (wh && QT == 2) K8SLLM_WPW(DK, DV, 2, CAP, 4);            \
+  else K8SLLM_WPW(DK, DV, QT, CAP, 0)
+#define K8SLLM_WPW(DK, DV, QT, CAP, WH)                                                                                \
+  hipLaunchKernelGGL((window_prefill_mfma_kernel<DK, DV, QT, CAP, WH>), grid, dim3(WH ? 64 * WH : 64), 0, s, (bf16_t*)out, \
                      (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu, ctx,             \
                      block_tables, bt_stride, S, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
 #define K8SLLM_WP(DK, DV, QT) \
-  if (cap > 0.f && cap <= kMaxCapPlain && !sink) K8SLLM_WPC(DK, DV, QT, 2); \
-  else if (cap > 0.f) K8SLLM_WPC(DK, DV, QT, 1); \
-  else K8SLLM_WPC(DK, DV, QT, 0)
+  if (cap > 0.f && cap <= kMaxCapPlain && !sink) { K8SLLM_WPC(DK, DV, QT, 2); } \
+  else if (cap > 0.f) { K8SLLM_WPC(DK, DV, QT, 1); } \
+  else { K8SLLM_WPC(DK, DV, QT, 0); }
 #define K8SLLM_WPQ(DK, DV)                                       \
   if (qrows == 64) { K8SLLM_WP(DK, DV, 4); }                     \
   else if (qrows == 32) { K8SLLM_WP(DK, DV, 2); }                \
@@ -895,6 +969,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
 #undef K8SLLM_WPQ
 #undef K8SLLM_WP
 #undef K8SLLM_WPC
+#undef K8SLLM_WPW
     return (int)hipGetLastError();
   }
   if (mfma == kFlashForced) return 1;

@@ -772,3 +772,23 @@ def test_single_tokens_beside_prompts_keep_their_bits(kind, prompts):
     assert torch.equal(o[:nd], od) and torch.equal(s[:nd], sd[:nd])
     op, sp = run(nd, T, nd, S, longest=longest)
     assert torch.equal(o[nd:], op) and torch.equal(s[nd:], sp[nd:])
+
+
+@pytest.mark.parametrize("Hq,G", [(8, 2), (8, 1), (4, 4)])  # four heads that share their keys, twice; none
+@pytest.mark.parametrize("dk,dv", [(128, 128), (64, 128), (128, 64)])
+@pytest.mark.parametrize("window,kw", [(0, {}), (40, dict(keep=5)), (64, dict(chunked=True)), (33, dict(cap=20.0)), (0, dict(cap=80.0, sink=True))])
+def test_window_prefill_heads_that_share_their_keys(Hq, G, dk, dv, window, kw):
+    """Query rows 32 at a time, with the keys through LDS where four heads share them, have the bits of 16 at a time with keys of
+    their own: segments of one row and of whole and broken tiles, an odd and an even number of key tiles, ends inside a page."""
+    g = _g(91)
+    kw = dict(kw)
+    sink = kw.pop("sink", False)
+    lens, ctx = [1, 16, 32, 33, 47, 100], [0, 5, 16, 96, 31, 0]
+    T, S = sum(lens), len(lens)
+    W = max((a + b + 15) // 16 for a, b in zip(lens, ctx))
+    bt = torch.randperm(S * W, generator=g).int().view(S, W).cuda()
+    qkv = _r(g, T, Hq * dk + G * (dk + dv), dt=BF).cuda()
+    kc, vc = _r(g, S * W, 16, G * dk, dt=BF).cuda(), _r(g, S * W, G, dv, 16, dt=BF).cuda()
+    cu = _i32([0] + torch.tensor(lens).cumsum(0).tolist()).cuda()
+    run = lambda rows: hops.window_attention_prefill(qkv, kc, vc, cu, _i32(ctx).cuda(), bt, Hq, G, dk, dv, dk ** -0.5, window, sink, mfma=rows, **kw)
+    assert torch.equal(run(32), run(16))
