@@ -30,7 +30,11 @@ __device__ __forceinline__ void keep_finite(uint32_t (&w)[VW / 2], int row, int 
 
 // log2 of a decay from its logit (kinds of decay_scan.hip); 2^-4096 is zero in fp32, and a NaN stays one
 __device__ __forceinline__ float log2_decay(float x, int kind, float A, float inv_tau) {
-  const float e = kind == 0 ? A * softplus_f(x) : kind == 1 ? softplus_f(-x) * inv_tau : expf(x);
+  auto softplus = [](float v) {  // softplus_f without a branch, so that a run of tokens is evaluated side by side
+    const float r = log1pf(expf(v > 20.f ? 20.f : v));
+    return v > 20.f ? v : r;
+  };
+  const float e = kind == 0 ? A * softplus(x) : kind == 1 ? softplus(-x) * inv_tau : expf(x);
   const float l = -1.44269504088896341f * e;
   return l < -4096.f ? -4096.f : l;
 }

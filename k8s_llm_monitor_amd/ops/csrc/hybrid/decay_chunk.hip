@@ -9,28 +9,33 @@
 // No exponent is positive, so nothing overflows however fast a channel forgets: between sub-blocks of 16 tokens the
 // exponent of M is split at the query block's first token, 2^(E_i - ref) 2^(ref - L_j), and inside a sub-block M is summed
 // with running products of the decays, as the token-by-token form has them.
-//  * decay_chunk_prep: a workgroup per (chunk, head), all in parallel, leaves Q', M and N as three bf16 parts each
-//    (split_bf16.h) in operand order and 2^L_n in a workspace.  Sums of log2 g are kept in 64 bits.
+//  * decay_chunk_prep: a workgroup per (chunk, head), all in parallel, leaves Q', M and N as fp32 in operand order and 2^L_n in a
+//    workspace.  Sums of log2 g are kept in 64 bits.
 //  * decay_chunk_scan: eight waves per (segment, head, 16 NT value columns) walk the chunks, four for O, four for S; S is
-//    published in LDS as three parts, double-buffered: one barrier per chunk.  Values are bf16 activations (exact), so
-//    their products take three instructions, Q' S the six that matter at 2^-24.
+//    published in LDS as three bf16 parts (split_bf16.h), double-buffered: one barrier per chunk.  The operands are split into
+//    parts as they arrive.  Values are bf16 activations (exact), so their products take three instructions, Q' S the six that
+//    matter at 2^-24.
 //    Long segments that leave the chip idle are cut into spans of chunks: a launch for their ends, one for the outputs.
-// What bounds it: the scan by the workspace's operands (72 KiB per chunk and head at 64 channels, read by every column block:
-// 1.2 us a chunk at the 25 bytes per clock that a CU draws from L2, where the products and the trip through LDS take 0.3);
-// the preparation by vector instructions.
-// Measured, both launches (us; the staged scan with its preparation), 32 heads of 64 x 64 with a bonus: 1 x 8000 rows 259
-// (1347), 4 x 2048 240 (428); plain, 16 heads of 128 x 128: 1 x 8000 449 (1548), 4 x 2048 407 (567).  Error against 64 bits, 2048
-// rows, bonus: outputs 1.3e-7 (scan 2.7e-7), state 7.9e-8 (3.0e-7); plain: 2.3e-7 (1.5e-6), 2.1e-7 (2.0e-6).
+// What bounds it: the workspace's operands, 48 KiB per chunk and head at 64 channels, written once and read by every column
+// block (as three bf16 parts they were 72 KiB, and the spans' second launch went at the rate of memory: 1 x 8000 rows, 32 heads of
+// 64, both launches and the preparation 239 us, as fp32 221); the preparation also by vector instructions: it has no LDS read
+// behind a branch, no branch per token, and reads the rows of a diagonal's next product ahead of this one's (268 -> 239 us).
+// Measured, all launches (us, before these two changes; the staged scan with its preparation), 32 heads of 64 x 64 with a
+// bonus: 1 x 8000 rows 221 (268; 1347), 4 x 2048 201 (250; 428); plain, 16 heads of 128 x 128: 1 x 8000 342 (457; 1548).  Error
+// against 64 bits, 2048 rows, bonus: outputs 1.3e-7 (scan 2.7e-7), state 7.9e-8 (3.0e-7); plain: 2.3e-7 (1.5e-6), 2.1e-7 (2.0e-6).
 #include "chunk_seg.h"
 #include "split_bf16.h"
+#include <type_traits>
 
 namespace k8sllm {
 
-// bf16 elements of Q', M and N of one (chunk, head) in the workspace
-__host__ __device__ constexpr long kc_mats(int dk) { return 3L * 64 * (64 + 2 * dk); }
+// elements of Q', M and N of one (chunk, head) in the workspace
+__host__ __device__ constexpr long kc_mats(int dk) { return 64L * (64 + 2 * dk); }
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <int KS, bool BONUS>
-__global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restrict__ mats, float* __restrict__ ends,
+__global__ __launch_bounds__(256) void decay_chunk_prep_kernel(float* __restrict__ mats, float* __restrict__ ends,
                                                                const bf16_t* __restrict__ qkv, long stride, int q_col,
                                                                int k_col, const bf16_t* __restrict__ z, long z_stride,
                                                                const float* __restrict__ z_bias,
@@ -38,10 +43,10 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
                                                                const float* __restrict__ bonus, const int* __restrict__ cu,
                                                                const int* __restrict__ slot, int S, int H, int Gk,
                                                                float q_scale) {
-  constexpr int DK = 32 * KS, PK = DK + 8, PL = DK + 1, PM = 68;
+  constexpr int DK = 32 * KS, PK = DK + 8, PL = DK + 1, PG = DK + 4, PM = 68;  // (pitches under which sixteen rows lie in different banks)
   __shared__ __attribute__((aligned(16))) double Ll[64 * PL];  // L; later M as fp32 [64][PM]
   __shared__ __attribute__((aligned(16))) bf16_t Ql[64 * PK], Kl[64 * PK];
-  __shared__ __attribute__((aligned(16))) float Gl[64 * DK];  // the decays
+  __shared__ __attribute__((aligned(16))) float Gl[64 * PG];  // the decays
   float* Ml = reinterpret_cast<float*>(Ll);
   static_assert(64 * PM * 4 <= 64 * PL * 8 || KS == 1, "M fits where L was");
   __shared__ float Mx[KS == 1 ? 64 * PM : 1];
@@ -74,19 +79,28 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
     const float zb = z_bias[(long)h * DK + c];
     float x[QT];
     double run = 0.0;
+    auto decays = [&](auto kind) {  // (the kind's branch around the run, not around each token)
+#pragma unroll
+      for (int i = 0; i < QT; ++i) x[i] = log2_decay(bf2f(zr[i]) + zb, kind, A, inv_tau);
+    };
+    if (dkind == 0) decays(std::integral_constant<int, 0>{});
+    else if (dkind == 1) decays(std::integral_constant<int, 1>{});
+    else decays(std::integral_constant<int, 2>{});
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
       const int t = QT * tq + i;
-      x[i] = t < n ? log2_decay(bf2f(zr[i]) + zb, dkind, A, inv_tau) : 0.f;
-      Gl[t * DK + c] = __builtin_amdgcn_exp2f(x[i]);
+      x[i] = t < n ? x[i] : 0.f;
+      Gl[t * PG + c] = __builtin_amdgcn_exp2f(x[i]);
       run += (double)x[i];
     }
     Tl[tq * CT + cq] = run;
     __syncthreads();
     double at_t = 0.0;
 #pragma unroll
-    for (int u = 0; u < NQ - 1; ++u)
-      if (u < tq) at_t += Tl[u * CT + cq];
+    for (int u = 0; u < NQ - 1; ++u) {
+      const double v = Tl[u * CT + cq];
+      at_t += u < tq ? v : 0.0;
+    }
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
       at_t += (double)x[i];
@@ -95,29 +109,31 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
     __syncthreads();
   }
   const long ch = (long)blockIdx.x * H + h;
-  bf16_t* Qo = mats + ch * kc_mats(DK);
-  bf16_t* Mo = Qo + 3 * 64 * DK;
-  bf16_t* No = Mo + 3 * 64 * 64;
-  auto put = [&](bf16_t* o, int tile, const float* v) {
-    uint32_t x[3][4];
-    split_pairs<4>(v, x[0], x[1], x[2]);
+  float* Qo = mats + ch * kc_mats(DK);
+  float* Mo = Qo + 64 * DK;
+  float* No = Mo + 64 * 64;
+  auto put = [&](float* o, int tile, const float* v) {  // a lane's eight values of a fragment, in two rows of 16 bytes a lane
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      *reinterpret_cast<uint4*>(o + ((tile * 3 + k) * 64 + lane) * 8) = make_uint4(x[k][0], x[k][1], x[k][2], x[k][3]);
+    for (int k = 0; k < 2; ++k)
+      *reinterpret_cast<float4*>(o + ((tile * 2 + k) * 64 + lane) * 4) = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
   };
   const int qi = 16 * w + c16, ei = qi - (BONUS ? 1 : 0);  // this lane's query; the token whose sum its reads carry
   // eight channels of a row: sums (zero before the first token) and activations
   auto sums8 = [&](int row, int c, double* d) {
+    const double* l = Ll + max(row, 0) * PL + c;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) d[i] = row < 0 ? 0.0 : Ll[row * PL + c + i];
+    for (int i = 0; i < 8; ++i) d[i] = l[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) d[i] = row < 0 ? 0.0 : d[i];
   };
   auto acts8 = [&](const bf16_t* m, int row, int c, float* f) { unpack8(*reinterpret_cast<const uint4*>(&m[row * PK + c]), f); };
   // Q', and this query block's operand against earlier blocks, relative to the block's first token
   bf16x8 qf[KS][3];
+  double ref[KS][8];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int c = 32 * ks + 8 * quad;
-    double e[8], r[8];
+    double e[8], (&r)[8] = ref[ks];
     float q[8], a[8], b[8];
     sums8(ei, c, e);
     sums8(16 * w - 1, c, r);
@@ -143,10 +159,10 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const int c = 32 * ks + 8 * quad;
-        double l[8], r[8];
+        const double (&r)[8] = ref[ks];
+        double l[8];
         float k[8];
         sums8(16 * kt + c16, c, l);
-        sums8(16 * w - 1, c, r);
         acts8(Kl, 16 * kt + c16, c, k);
 #pragma unroll
         for (int i = 0; i < 8; ++i) k[i] *= __builtin_amdgcn_exp2f((float)(r[i] - l[i]));
@@ -168,8 +184,9 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
       float v[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int t = 32 * ks + 8 * quad + i;
-        v[i] = t < n ? bf2f(Kl[t * PK + c]) * __builtin_amdgcn_exp2f((float)(Ln - Ll[t * PL + c])) : 0.f;
+        const int t = 32 * ks + 8 * quad + i;  // (the decay behind a token past the chunk is one)
+        const uint32_t k = (uint32_t)Kl[t * PK + c] << 16;
+        v[i] = __builtin_bit_cast(float, t < n ? k : 0u) * __builtin_amdgcn_exp2f((float)(Ln - Ll[t * PL + c]));
       }
       put(No, 2 * rt + ks, v);
     }
@@ -195,33 +212,36 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
       own = xor32_sum_f(xor16_sum(own));
     }
     // query j + d for d = 1 .. 15 (past the block's end: clamped, not stored).  Plain: the decays behind key j up to the
-    // query's own; bonus: up to the token before it
-    auto decay = [&](int t) {
+    // query's own; bonus: up to the token before it.  The rows of the next d are read ahead of this one's products.
+    f32x4 gn[NC / 4], gv[NC / 4];
+    u32x4 qn[NC / 8], qv[NC / 8];
+    auto next = [&](int d) {
+      const int t = min(j + d, 16 * w + 15), tg = BONUS ? min(j + d - 1, 16 * w + 15) : t;
 #pragma unroll
-      for (int u = 0; u < NC; u += 4) {
-        const float4 gv = *reinterpret_cast<const float4*>(&Gl[t * DK + c0 + u]);
-        ke[u] *= gv.x;
-        ke[u + 1] *= gv.y;
-        ke[u + 2] *= gv.z;
-        ke[u + 3] *= gv.w;
-      }
+      for (int u = 0; u < NC / 4; ++u) gn[u] = *reinterpret_cast<const f32x4*>(&Gl[tg * PG + c0 + 4 * u]);
+#pragma unroll
+      for (int u = 0; u < NC / 8; ++u) qn[u] = *reinterpret_cast<const u32x4*>(&Ql[t * PK + c0 + 8 * u]);
     };
+    next(1);
     dg[0] = q_scale * own;
 #pragma unroll
     for (int d = 1; d < 16; ++d) {
-      const int t = min(j + d, 16 * w + 15);
-      if (!BONUS) decay(t);
-      else if (d > 1) decay(min(j + d - 1, 16 * w + 15));
+#pragma unroll
+      for (int u = 0; u < NC / 4; ++u) gv[u] = gn[u];
+#pragma unroll
+      for (int u = 0; u < NC / 8; ++u) qv[u] = qn[u];
+      if (d < 15) next(d + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!BONUS || d > 1) {
+#pragma unroll
+        for (int u = 0; u < NC; ++u) ke[u] *= gv[u / 4][u & 3];
+      }
       float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-      for (int u = 0; u < NC / 8; ++u) {
-        float q[8];
-        acts8(Ql, t, c0 + 8 * u, q);
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          s0 += q[e] * ke[8 * u + e];
-          s1 += q[e + 1] * ke[8 * u + e + 1];
-        }
+      for (int u = 0; u < NC; u += 2) {
+        const uint32_t x = qv[u / 8][(u & 7) >> 1];
+        s0 += __builtin_bit_cast(float, x << 16) * ke[u];
+        s1 += __builtin_bit_cast(float, x & 0xffff0000u) * ke[u + 1];
       }
       dg[d] = q_scale * xor32_sum_f(xor16_sum(s0 + s1));
     }
@@ -254,7 +274,7 @@ __global__ __launch_bounds__(256) void decay_chunk_prep_kernel(bf16_t* __restric
 // folds those in front of its own span, S <- diag(d_j) S + E_j.
 template <int KS, int NT, int MODE>
 __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restrict__ o, const bf16_t* __restrict__ qkv,
-                                                                  long stride, int v_col, const bf16_t* __restrict__ mats,
+                                                                  long stride, int v_col, const float* __restrict__ mats,
                                                                   const float* __restrict__ ends, float* __restrict__ state,
                                                                   const int* __restrict__ cu, const int* __restrict__ ctx,
                                                                   const int* __restrict__ slot, int S_, int H, int dv, int span, int n_span,
@@ -350,31 +370,45 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
       }
     }
   };
-  // operands, fetched one chunk ahead: outs: Q' (3 KS) and M (6); else N (6 RTW) and the ends of its rows
-  constexpr int NF = 3 * KS + 6 > 6 * RTW ? 3 * KS + 6 : 6 * RTW;
-  bf16x8 mf[NF], mn[NF];
+  // operands, fetched one chunk ahead as fp32 and split when their chunk begins: outs: fragments of Q' (KS) and M (2); else
+  // N (2 RTW) and the ends of its rows
+  constexpr int NF = KS + 2 > 2 * RTW ? KS + 2 : 2 * RTW;
+  bf16x8 mf[3 * NF];
+  f32x4 mn[2 * NF];
   float4 ef[RTW], en[RTW];
   constexpr int VW = NV * 64 / 512;  // values a thread stages: 2 NT
   uint32_t rv[VW / 2];
   const int vr = tid / (NV / VW), vc = VW * (tid % (NV / VW));
   auto fetch = [&](int tb) {
     const long ch = (long)(c0 + (tb - t0) / kChunk) * H + h;
-    const bf16_t* m = mats + ch * kc_mats(DK) + lane * 8;
+    const float* m = mats + ch * kc_mats(DK) + lane * 4;
     if (outs) {
       if (MODE == kSpanEnds) return;
 #pragma unroll
-      for (int i = 0; i < 3 * KS; ++i) mn[i] = *reinterpret_cast<const bf16x8*>(m + (long)(3 * KS * w + i) * 512);
-      m += 3 * 64 * DK;
+      for (int i = 0; i < 2 * KS; ++i) mn[i] = *reinterpret_cast<const f32x4*>(m + (long)(2 * KS * w + i) * 256);
+      m += 64 * DK;
 #pragma unroll
-      for (int i = 0; i < 6; ++i)
-        if (i < 3 || w >= 2) mn[3 * KS + i] = *reinterpret_cast<const bf16x8*>(m + (long)(6 * w + i) * 512);
+      for (int i = 0; i < 4; ++i)
+        if (i < 2 || w >= 2) mn[2 * KS + i] = *reinterpret_cast<const f32x4*>(m + (long)(4 * w + i) * 256);
     } else if (mine) {
-      m += 3 * 64 * DK + 3 * 64 * 64;
+      m += 64 * DK + 64 * 64;
 #pragma unroll
-      for (int i = 0; i < 6 * RTW; ++i) mn[i] = *reinterpret_cast<const bf16x8*>(m + (long)min(6 * w * RTW + i, 12 * KS - 1) * 512);
+      for (int i = 0; i < 4 * RTW; ++i) mn[i] = *reinterpret_cast<const f32x4*>(m + (long)min(4 * w * RTW + i, 8 * KS - 1) * 256);
 #pragma unroll
       for (int r = 0; r < RTW; ++r)
         en[r] = *reinterpret_cast<const float4*>(ends + ch * DK + min(16 * (w * RTW + r) + 4 * quad, DK - 4));
+    }
+  };
+  auto split = [&](auto frags) {
+#pragma unroll
+    for (int i = 0; i < decltype(frags)::value; ++i) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = mn[2 * i + (e >> 2)][e & 3];
+      uint32_t x[3][4];
+      split_pairs<4>(v, x[0], x[1], x[2]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) mf[3 * i + k] = frag(x[k]);
     }
   };
   auto fetch_v = [&](int tb) {
@@ -404,8 +438,8 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
   int buf = 0;
   for (int tb = t0; tb < t1; tb += kChunk, buf ^= 1) {
     const int n = min(kChunk, t1 - tb);
-#pragma unroll
-    for (int i = 0; i < NF; ++i) mf[i] = mn[i];
+    if (!outs) split(std::integral_constant<int, 2 * RTW>{});
+    else if (MODE != kSpanEnds) split(std::integral_constant<int, KS + 2>{});
 #pragma unroll
     for (int r = 0; r < RTW; ++r) ef[r] = en[r];
     if (tb + kChunk < t1) fetch(tb + kChunk);
@@ -514,7 +548,7 @@ static int span_chunks(long T, int S, int longest, int H, int dv, int mode) {
 long k8sllm_hy_decay_chunk_ws(long T, int S, int longest, int H, int dk, int dv, int mode) {
   if (dk % 32 || dk < 32 || dk > 128 || dv % 16 || dv < 16) return 0;
   const int span = span_chunks(T, S, longest, H, dv, mode);
-  return (T / kChunk + S) * H * (kc_mats(dk) * 2 + dk * 4) + (span > 0 ? (T / (span * kChunk) + S) * H * (long)dk * (dv + 1) * 4 : 0);
+  return (T / kChunk + S) * H * (kc_mats(dk) + dk) * 4 + (span > 0 ? (T / (span * kChunk) + S) * H * (long)dk * (dv + 1) * 4 : 0);
 }
 
 // as k8sllm_hy_decay_scan's plain form (bonus nullptr) or bonus form, without unit norms
@@ -526,8 +560,8 @@ int k8sllm_hy_decay_chunk(float* o, const void* qkv, long stride, int q_col, int
   if (k8sllm_hy_decay_chunk_ws(T, S, longest, H, dk, dv, mode) == 0 || Gk < 1 || H % Gk || dkind < 0 || dkind > 2 || (dkind == 0 && a_log == nullptr))
     return -1;
   const long nch = T / kChunk + S;
-  bf16_t* mats = (bf16_t*)ws;
-  float* ends = (float*)(mats + nch * H * kc_mats(dk));
+  float* mats = (float*)ws;
+  float* ends = mats + nch * H * kc_mats(dk);
   const long pairs = (long)S * H;
   // narrow column blocks until they fill the chip: the chain of chunks bounds a block
   const int span = span_chunks(T, S, longest, H, dv, mode);
