@@ -144,16 +144,30 @@ __global__ __launch_bounds__(256, 2) void delta_prep_kernel(bf16_t* __restrict__
     const float num = nk[lane] + (float)Ll[lane] + bl[lane];
     const unsigned long long odd = __ballot(lane < n && num != num);
     if (lane == 0) odd_row = odd != 0 ? (int)__builtin_ctzll(odd) : kNone;
+    // A's rows come four values at a time, the same for every lane, twelve reads ahead of their products (one or two ahead the
+    // wave spent three quarters of its time on the reads' latency)
+    constexpr int AHEAD = 12;
+    f32x4 ring[AHEAD];
+    int li = 1, lj = 0, at_k = 0;
+    auto load = [&](int k) {
+      if (li < 64) ring[k % AHEAD] = *reinterpret_cast<const f32x4*>(&Al[li * PA + lj]);
+      if ((lj += 4) >= li) ++li, lj = 0;
+    };
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) load(k);
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       float s0 = lane == i ? 1.f : 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
 #pragma unroll
       for (int j = 0; j < i; j += 4) {
-        const float4 a = *reinterpret_cast<const float4*>(&Al[i * PA + j]);
-        s0 -= a.x * t[j];
-        if (j + 1 < i) s1 -= a.y * t[j + 1];
-        if (j + 2 < i) s2 -= a.z * t[j + 2];
-        if (j + 3 < i) s3 -= a.w * t[j + 3];
+        const f32x4 a = ring[at_k % AHEAD];
+        s0 -= a[0] * t[j];
+        if (j + 1 < i) s1 -= a[1] * t[j + 1];
+        if (j + 2 < i) s2 -= a[2] * t[j + 2];
+        if (j + 3 < i) s3 -= a[3] * t[j + 3];
+        load(at_k + AHEAD);
+        ++at_k;
+        __builtin_amdgcn_sched_barrier(0);
       }
       t[i] = (s0 + s1) + (s2 + s3);
     }
