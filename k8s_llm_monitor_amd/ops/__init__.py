@@ -914,14 +914,26 @@ def gather_rows(x: torch.Tensor, idx: torch.Tensor, div: int = 1) -> torch.Tenso
 
 
 def moe_grouped_gemm(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, swiglu: bool = False,
-                     out: Optional[torch.Tensor] = None, zero_fill: bool = True) -> torch.Tensor:
+                     out: Optional[torch.Tensor] = None, zero_fill: bool = True, rows: Optional[torch.Tensor] = None,
+                     div: int = 1) -> torch.Tensor:
     """All experts' GEMMs in one launch over expert-sorted rows: ``x`` [rows, K], ``w`` [E, N, K],
     ``offsets`` [E + 1] int32 absolute row offsets of the experts' rows in ``x`` (moe_align, may be
     a slice for this rank's experts).  ``swiglu``: ``w`` is gate/up-interleaved and the result is
     silu(gate) * up [rows, N / 2].  Rows of other experts are left as in ``out`` (zeros when
     allocated here).  GPU: no host synchronisation (gemm_tile.hip 256 x 256 tiles where N % 256 == 0,
     else moe_gemm.hip).  A fragment-packed ``w`` [E, N/16, K/32, 64, 8] (ONE_LAYOUT; ``swiglu=8``:
-    the per-16 gate/up pairing) always takes the tile kernel."""
+    the per-16 gate/up pairing) always takes the tile kernel.  ``rows`` int32: ``x`` holds the rows in their own order,
+    and sorted row r is its row rows[r] / div (gather_rows); the tile kernel reads them from there."""
+    if rows is not None:
+        if not (_gpu(x) and w.dim() == 3 and w.shape[1] % 256 == 0 and w.shape[2] % 64 == 0 and w.shape[1] * w.shape[2] < 1 << 30
+                and x.numel() < 1 << 30):
+            x = gather_rows(x, rows, div)
+        else:
+            if out is None:
+                alloc = torch.zeros if zero_fill else torch.empty
+                out = alloc(rows.numel(), w.shape[1] // 2 if swiglu else w.shape[1], dtype=x.dtype, device=x.device)
+            native().gemm_tile_rows(out, x.contiguous(), w, offsets.contiguous(), rows, div, bool(swiglu), TILE_ALGO)
+            return out
     if w.dim() == 5:
         if out is None:
             alloc = torch.zeros if zero_fill else torch.empty

@@ -47,7 +47,7 @@ int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void* Y2, int M
 int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, int N, int K, const int* offsets, int E, long w_es,
                      int epi, int algo, const int* rope_pos, const float* rope_cs, int rope_heads,
                      const float* rs_part, int rs_np, float rs_eps, void* resid, void* hw, const void* norm_w,
-                     float* ss_out, int wpk, hipStream_t s);
+                     float* ss_out, int wpk, const int* src, int src_div, long src_rows, hipStream_t s);
 int k8sllm_moe_grouped_gemm(const void* X, const void* W, void* Y, const int* offsets, int E, long rows, int N, int K,
                             long w_es, int epi, hipStream_t s);
 int k8sllm_gemm_skinny(const void* A, long lda, const void* Wp, float* partial, void* Y, long ldy, int M, int N, int K,
@@ -498,8 +498,26 @@ void gemm_tile(torch::Tensor y, torch::Tensor x, torch::Tensor w, c10::optional<
                          (long)N * K, epi, (int)algo, rp, rc, (int)rope_heads, rsp, rs_np, (float)rs_eps,
                          rsd ? resid->data_ptr() : nullptr, rsd ? hw->data_ptr() : nullptr,
                          rsd ? norm_w->data_ptr() : nullptr, rsd ? ss_out->data_ptr<float>() : nullptr, wpk ? 1 : 0,
-                         cur()),
+                         nullptr, 1, 0, cur()),
         "gemm_tile");
+}
+
+// the grouped form over rows in their own order: sorted row r is row rows[r] / div of x (gather_rows' meaning), w [E, N, K]
+void gemm_tile_rows(torch::Tensor y, torch::Tensor x, torch::Tensor w, torch::Tensor offsets, torch::Tensor rows, int64_t div, bool swiglu,
+                    int64_t algo) {
+  dev_bf16(y, "y"); dev_bf16(x, "x"); dev_bf16(w, "w"); dev_i32(offsets, "offsets"); dev_i32(rows, "rows");
+  TORCH_CHECK(x.dim() == 2 && x.is_contiguous() && w.dim() == 3 && w.is_contiguous() && y.is_contiguous() && offsets.is_contiguous() &&
+                  rows.is_contiguous(), "gemm_tile_rows: x [T, K], w [E, N, K], contiguous");
+  const int E = (int)w.size(0), N = (int)w.size(1), K = (int)w.size(2);
+  const long M = rows.numel();
+  TORCH_CHECK(x.size(1) == K && offsets.numel() == E + 1 && algo >= 0 && algo <= 1, "gemm_tile_rows: K, offsets [E + 1], algo 0 or 1");
+  TORCH_CHECK(div >= 1 && M <= x.size(0) * div, "gemm_tile_rows: at most div sorted rows for each of x");
+  TORCH_CHECK(N % 16 == 0 && K % 64 == 0 && K >= 64 && (!swiglu || N % 256 == 0), "gemm_tile_rows: N % 16 == 0 (SwiGLU: % 256), K % 64 == 0");
+  TORCH_CHECK(y.dim() == 2 && y.size(0) == M && y.size(1) == (swiglu ? N / 2 : N), "gemm_tile_rows: y shape");
+  check(k8sllm_gemm_tile(x.data_ptr(), w.data_ptr(), y.data_ptr(), (int)M, N, K, offsets.data_ptr<int>(), E, (long)N * K, swiglu ? 1 : 0,
+                         (int)algo, nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, 0, rows.data_ptr<int>(),
+                         (int)div, x.size(0), cur()),
+        "gemm_tile_rows");
 }
 
 void gather_rows(torch::Tensor out, torch::Tensor x, torch::Tensor idx, int64_t div) {
@@ -968,6 +986,7 @@ PYBIND11_MODULE(_k8sllm_ops, m) {
   m.def("layer_norm", &layer_norm);
   m.def("silu_mul", &silu_mul);
   m.def("moe_grouped_gemm", &moe_grouped_gemm);
+  m.def("gemm_tile_rows", &gemm_tile_rows);
   m.def("gemm_tile_unit", &gemm_tile_unit);
   m.def("gemm_tile", &gemm_tile, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("offsets"), py::arg("swiglu"),
         py::arg("algo") = 1, py::arg("rope_pos") = py::none(), py::arg("rope_cs") = py::none(),

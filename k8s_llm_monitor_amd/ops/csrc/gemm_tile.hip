@@ -126,7 +126,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   for (int p = 0; p < 8; ++p) {
     const int rl = (p * 4 + wave) * 8 + (lane >> 3);
     const int cl = (lane & 7) ^ ((rl >> 1) & 7);
-    soff[0][p] = (uint32_t)(((long)min(rl, mrows - 1) * K + cl * 8) * 2);  // rows past the end: clamped, never stored
+    int xrow = min(rl, mrows - 1);  // rows past the end: clamped, never stored
+    if (GROUPED && ep.src != nullptr) xrow = ep.src[row0 + xrow] / ep.src_div;  // the rows are sorted as they are read
+    soff[0][p] = (uint32_t)(((long)xrow * K + cl * 8) * 2);
     if constexpr (GLU) {  // rows [64 gate | 64 up] per 128, from the start of W
       const int wrow = unit ? min(n0 + ((rl >> 7) << 6) + (rl & 63), ep.f - 1) + (rl & 64 ? ep.f : 0) : n0 + min(rl, nrows - 1);
       soff[1][p] = (uint32_t)(((long)wrow * K + cl * 8) * 2);
@@ -147,7 +149,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int nb = __builtin_amdgcn_readfirstlane((int)bytes);
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0, nb, 0x00020000);
   };
-  const __amdgpu_buffer_rsrc_t xr = rsrc(reinterpret_cast<const char*>(X) + (long)row0 * K * 2, (long)mrows * K * 2);
+  const bool sorts = GROUPED && ep.src != nullptr;
+  const __amdgpu_buffer_rsrc_t xr = rsrc(reinterpret_cast<const char*>(X) + (sorts ? 0 : (long)row0 * K * 2),
+                                         sorts ? ep.src_bytes : (long)mrows * K * 2);
   const __amdgpu_buffer_rsrc_t wr = GLU ? rsrc(Wt, (long)N * K * 2)
                                         : rsrc(reinterpret_cast<const char*>(Wt) + (long)n0 * K * 2, (long)nrows * K * 2);
   const int nk = K >> 6;
@@ -567,15 +571,19 @@ using namespace k8sllm;
 // Dense (offsets == nullptr): Y [M][N] (SwiGLU: [M][N / 2]) = X [M][K] . W[N][K]^T.
 // Grouped: W [E][N][K] with expert stride w_es elements; M = total expert-sorted rows (the grid
 // bound: ceil(M / 256) + E m-tiles); expert e's rows are offsets[e] .. offsets[e + 1] - 1.
+// src (grouped): X holds src_rows rows in their own order, sorted row r is row src[r] / src_div; only a lane's first address knows
+// (16384 sorted rows of 2048, 8 experts: the launch that sorted them took 20.6 us, the product the same time either way).
 // Shapes: N % 16 == 0 (SwiGLU: N % 256 == 0), K % 64 == 0.  algo: the refill schedule (0 or 1).
 // wpk: W is fragment-packed ([E][N/16][K/32][64][8], ops.pack_skinny - the decode GEMMs' layout)
 // instead of row-major: every W DMA piece is one contiguous 1-KiB block, read lane-linear from LDS.
 extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, int N, int K, const int* offsets, int E,
                                 long w_es, int epi, int algo, const int* rope_pos, const float* rope_cs,
                                 int rope_heads, const float* rs_part, int rs_np, float rs_eps, void* resid, void* hw,
-                                const void* norm_w, float* ss_out, int wpk, hipStream_t s) {
+                                const void* norm_w, float* ss_out, int wpk, const int* src, int src_div, long src_rows, hipStream_t s) {
   if (M <= 0) return 0;
   const bool grouped = offsets != nullptr;
+  if (src != nullptr && (!grouped || src_div < 1 || src_rows < 1)) return -1;
+  if (src != nullptr && src_rows * K * 2 >= (1L << 31)) return -3;
   const bool rs = rs_part != nullptr;
   if (grouped && (E < 1 || E > 256)) return -1;
   if (algo < 0 || algo > 1) return -1;
@@ -594,7 +602,7 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
              (epi != TILE_EPI_ROPE && !swg)))
     return -1;
   const TileEpi ep{rope_pos, rope_cs, rope_heads, rs_part, rs_np, rs_eps, (bf16_t*)resid, (bf16_t*)hw,
-                   (const bf16_t*)norm_w, ss_out, 0, nullptr};
+                   (const bf16_t*)norm_w, ss_out, 0, nullptr, src, src_div, src_rows * K * 2};
   // 32-bit DMA offsets (X: relative to the tile's first row; W: within one expert / n-tile)
   if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31)) return -3;
   if (epi == TILE_EPI_RESID && 256L * N * 2 >= (1L << 31)) return -3;
@@ -641,7 +649,7 @@ extern "C" int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void
   if (!glu && epi != TILE_EPI_RELU_SQ) return -1;
   if (N <= 0 || N % 16 || K % 64 || K < 192 || (glu ? f <= 0 || f % 16 || N < 2 * f : f != 0)) return -1;
   if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31) || 256L * N * 2 >= (1L << 31)) return -3;
-  const TileEpi ep{nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, f, (bf16_t*)Y2};
+  const TileEpi ep{nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, f, (bf16_t*)Y2, nullptr, 1, 0};
   const int n_mt = (M + 255) / 256, n_nt = glu ? (f + 127) / 128 + (N - 2 * f + 255) / 256 : (N + 255) / 256;
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;

@@ -44,6 +44,9 @@ struct TileEpi {
   float* ss_out;         // RESID: [M][N / 128]
   int f;                 // GLU: features of the unit
   bf16_t* y2;            // GLU: [M][N - 2 f]
+  const int* src;        // grouped: row r of the sorted rows is row src[r] / src_div of X (nullptr: row r)
+  int src_div;
+  long src_bytes;        // of X
 };
 
 __host__ __device__ constexpr bool tile_epi_glu(int epi) { return epi >= TILE_EPI_GELU_GLU && epi <= TILE_EPI_RELU_GLU; }

@@ -1093,7 +1093,7 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
     run as ONE grouped launch each over the sorted rows (SwiGLU in the first epilogue); no host
     synchronisation.  bf16: matrix-core kernels - tiles of 16, 32 or 64 rows by the mean rows of an expert, gathered on load
     (decode, small steps), or from TILE_MIN_ROWS sorted rows of an ``il`` layer the prefill tile
-    GEMM of the Mixtral path (ungated experts whose widths are multiples of 256 take it too, with
+    GEMM of the Mixtral path, which reads the rows in sorted order from where they are (ungated experts whose widths are multiples of 256 take it too, with
     the GELU as a launch between); fp32: 64 x 64 tiles on the fp32 matrix instruction.  K that is no multiple of 32 and
     unaligned fp32 rows: 64 x 64 tiles on the vector unit."""
     T, d = h.shape
@@ -1133,20 +1133,17 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
     if act in ("gelu", "relu_sq") and n >= TILE_MIN_ROWS and h.dtype == torch.bfloat16 and ff % 256 == 0 and d % 256 == 0:
         from .. import ops  # large steps of plain experts: the prefill tile GEMM twice, the activation between
 
-        xs = ops.gather_rows(h, sorted_idx, K)
-        a = activation(ops.moe_grouped_gemm(xs, w13, offsets, zero_fill=False), act)
+        a = activation(ops.moe_grouped_gemm(h, w13, offsets, zero_fill=False, rows=sorted_idx, div=K), act)
         ys = ops.moe_grouped_gemm(a, w2, offsets, zero_fill=False)
     elif act == "clamped_swish" and tile and n >= TILE_MIN_ROWS and h.dtype == torch.bfloat16:
         from .. import ops  # large steps: the prefill tile GEMM twice, the clamped unit as a launch between
 
-        xs = ops.gather_rows(h, sorted_idx, K)
-        a = glu(ops.moe_grouped_gemm(xs, w13, offsets, zero_fill=False), 0, ff, "clamped_swish", limit)
+        a = glu(ops.moe_grouped_gemm(h, w13, offsets, zero_fill=False, rows=sorted_idx, div=K), 0, ff, "clamped_swish", limit)
         ys = ops.moe_grouped_gemm(a, w2, offsets, zero_fill=False)
     elif il and n >= TILE_MIN_ROWS and h.dtype == torch.bfloat16:
         from .. import ops  # the Mixtral path's kernels (_k8sllm_ops)
 
-        xs = ops.gather_rows(h, sorted_idx, K)
-        a = ops.moe_grouped_gemm(xs, w13, offsets, swiglu=True, zero_fill=False)
+        a = ops.moe_grouped_gemm(h, w13, offsets, swiglu=True, zero_fill=False, rows=sorted_idx, div=K)
         ys = ops.moe_grouped_gemm(a, w2, offsets, zero_fill=False)
     else:
         a = torch.empty(n, ff, dtype=h.dtype, device=h.device)

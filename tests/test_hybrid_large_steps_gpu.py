@@ -792,3 +792,20 @@ def test_window_prefill_heads_that_share_their_keys(Hq, G, dk, dv, window, kw):
     cu = _i32([0] + torch.tensor(lens).cumsum(0).tolist()).cuda()
     run = lambda rows: hops.window_attention_prefill(qkv, kc, vc, cu, _i32(ctx).cuda(), bt, Hq, G, dk, dv, dk ** -0.5, window, sink, mfma=rows, **kw)
     assert torch.equal(run(32), run(16))
+
+
+@pytest.mark.parametrize("T,K,E", [(1, 1, 1), (300, 2, 3), (517, 3, 5)])
+@pytest.mark.parametrize("d,swiglu", [(64, False), (192, True), (320, False)])
+def test_grouped_tiles_sort_their_rows_as_they_read(T, K, E, d, swiglu):
+    """The grouped tile GEMM over rows in their own order has the bits of the sorted copy's: an expert without rows, tiles that end
+    inside an expert, every k-tile count of the ring's head."""
+    from k8s_llm_monitor_amd import ops
+
+    g = _g(92)
+    ids = torch.randint(0, max(E - 1, 1), (T, K), generator=g, dtype=torch.int32).cuda()
+    off, idx, _ = ops.moe_align(ids, E)
+    x, w = _r(g, T, d, dt=BF).cuda(), _r(g, E, 256, d, s=0.1, dt=BF).cuda()
+    want = ops.moe_grouped_gemm(ops.gather_rows(x, idx, K), w, off, swiglu=swiglu)
+    assert torch.equal(ops.moe_grouped_gemm(x, w, off, swiglu=swiglu, rows=idx, div=K), want)
+    cpu = ops.moe_grouped_gemm(x.cpu(), w.cpu(), off.cpu(), swiglu=swiglu, rows=idx.cpu(), div=K)
+    torch.testing.assert_close(want.cpu().float(), cpu.float(), rtol=2e-2, atol=2e-2 * float(cpu.float().abs().max()))
