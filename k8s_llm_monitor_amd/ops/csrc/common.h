@@ -68,16 +68,44 @@ __device__ __forceinline__ long act_index(int row, int col, long stride) {
 // LDS-DMA.  Paged decode reads 4-token groups, which v_perm keeps contiguous.
 __device__ __forceinline__ int v_perm(int t) { return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1); }
 
+// Wave-wide butterflies without the LDS crossbar: quads and rows by DPP (quad_perm, the row's mirror
+// controls pair equal partial results), rows 0/1 and 2/3 by v_permlane16_swap, the halves by
+// v_permlane32_swap.  Every lane ends with the result.
+#define K8SLLM_DPP(v, ctrl) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true))
+__device__ __forceinline__ float xor16_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float xor16_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float xor32_sum_f(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float xor32_max_f(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// Sum (maximum) over the wave in every lane: lanes 32, 16, 8, 4, 2 and 1 apart meet in turn (rotating a row by four is that, its
+// halves being equal by then).  All lanes take part.  __shfl_xor, which gives the same
+// bits, is a trip through the LDS crossbar each time: a step of one token through 32 layers took 3128 us with it, 3095 so, a decode step of 24
+// sequences through layer-list decoders 704 and 696.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+  v = xor16_sum(xor32_sum_f(v));
+  v += K8SLLM_DPP(v, 0x128);
+  v += K8SLLM_DPP(v, 0x124);
+  v += K8SLLM_DPP(v, 0x4E);
+  return v + K8SLLM_DPP(v, 0xB1);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
+  v = xor16_max(xor32_max_f(v));
+  v = fmaxf(v, K8SLLM_DPP(v, 0x128));
+  v = fmaxf(v, K8SLLM_DPP(v, 0x124));
+  v = fmaxf(v, K8SLLM_DPP(v, 0x4E));
+  return fmaxf(v, K8SLLM_DPP(v, 0xB1));
 }
 
 // Workgroup sum for blockDim.x == NT (multiple of 64). `red` must hold NT/64 floats.

@@ -30,18 +30,6 @@ __device__ __forceinline__ void wait_vmcnt_fp() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// x combined with its lane ^ 32 partner by one v_permlane32_swap (VALU, no LDS round trip; a
-// __shfl_xor(x, 32) is a ds_bpermute): the swap leaves (own, partner) in lanes 0-31 and
-// (partner, own) in lanes 32-63, so an order-free op of the pair is the same on every lane.
-__device__ __forceinline__ float xor32_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float xor32_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 template <int D, bool PAGED>
 __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(bf16_t* __restrict__ out, long out_stride,
                                                                const bf16_t* __restrict__ qkv, long qkv_stride,
@@ -194,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(bf16_t* __restric
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[i][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = xor32_max_f(mx);
     const float mnew = fmaxf(m, mx * scale_log2);
     const float alpha = __builtin_amdgcn_exp2f(m - mnew);
     float rs = 0.f;
@@ -206,7 +194,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(bf16_t* __restric
         sacc[i][r] = p;
         rs += p;
       }
-    rs += __shfl_xor(rs, 32, 64);
+    rs = xor32_sum_f(rs);
     l = l * alpha + rs;
     const bool grew = __builtin_amdgcn_ballot_w64(mnew > m) != 0;  // lazy rescale: O only when a max moved
     m = mnew;
@@ -422,7 +410,7 @@ __global__ __launch_bounds__(512, 2) void flash_prefill_paged_v2_kernel(
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int r = 2; r < 8; ++r) mq[c] = fmaxf(mq[c], sa[c >> 1][8 * (c & 1) + r]);
-    const float mx = xor32_max(fmaxf(fmaxf(mq[0], mq[1]), fmaxf(mq[2], mq[3])));
+    const float mx = xor32_max_f(fmaxf(fmaxf(mq[0], mq[1]), fmaxf(mq[2], mq[3])));
     // Lazy max with headroom: the reference max m moves only when the tile's max exceeds it by
     // more than 2^8 in probability (then to the exact max), so probabilities stay <= 256 - exact in
     // fp32 and in their bf16 rounding - and O is rescaled only on such a jump, which after a row's
@@ -455,7 +443,7 @@ __global__ __launch_bounds__(512, 2) void flash_prefill_paged_v2_kernel(
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[i][s][dt], pb, o[dt], 0, 0, 0);
       }
-    l = l * alpha + xor32_sum((rq[0] + rq[1]) + (rq[2] + rq[3]));
+    l = l * alpha + xor32_sum_f((rq[0] + rq[1]) + (rq[2] + rq[3]));
   };
 
   // Main loop: ONE barrier per tile; tiles t + 1 and t + 2 are in flight while tile t is

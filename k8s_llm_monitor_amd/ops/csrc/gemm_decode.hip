@@ -171,8 +171,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gemm_dec_kernel(
       const int row = min(rl, M - 1);
       for (int c = part; c < rn_nc; c += 4) ss += rn_ss[row * rn_nc + c];
     }
-    ss += __shfl_xor(ss, 1, kWave);
-    ss += __shfl_xor(ss, 2, kWave);
+    ss += K8SLLM_DPP(ss, 0xB1);
+    ss += K8SLLM_DPP(ss, 0x4E);
     if (part == 0) s_inv[rl] = rsqrtf(ss * rn_inv_d + rn_eps);
   }
 
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gemm_dec_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float v = acc[m][t][r] * rs[r];
-          const float o = __shfl_xor(v, 8, kWave);
+          const float o = K8SLLM_DPP(v, 0x128);
           const int row = m * 16 + (lane >> 4) * 4 + r;
           if ((lane & 8) == 0) {
             // gate and up rounded to bf16 first, as the unfused GEMM -> silu_mul does
@@ -361,8 +361,10 @@ __global__ __launch_bounds__(512, 1) void gemm_dec_rc_kernel(const bf16_t* __res
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     float v = ssr[r];
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, kWave);  // the 16 columns of the row
+    v += K8SLLM_DPP(v, 0xB1);  // the 16 columns of the row
+    v += K8SLLM_DPP(v, 0x4E);
+    v += K8SLLM_DPP(v, 0x141);
+    v += K8SLLM_DPP(v, 0x140);
     const int row = m * 16 + (lane >> 4) * 4 + r;
     if ((lane & 15) == 0 && row < M) ss_out[(long)row * (N >> 4) + tile] = v;
   }

@@ -194,8 +194,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_skinny_kernel(const bf16_t
     const int row = min(rl, M - 1);
     float ss = 0.f;
     for (int c = part; c < rn_nc; c += 4) ss += rn_ss[row * rn_nc + c];
-    ss += __shfl_xor(ss, 1, kWave);
-    ss += __shfl_xor(ss, 2, kWave);
+    ss += K8SLLM_DPP(ss, 0xB1);
+    ss += K8SLLM_DPP(ss, 0x4E);
     if (part == 0) s_inv[rl] = rsqrtf(ss * rn_inv_d + rn_eps);
   }
 
@@ -486,8 +486,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gemm_skinny_rm_kernel(
     const int t = threadIdx.x + p * 64 * WAVES;
     if (rn_ss != nullptr && t < MT * 64) {  // published by the epilogue's first barrier
       float v = ss[p];
-      v += __shfl_xor(v, 1, kWave);
-      v += __shfl_xor(v, 2, kWave);
+      v += K8SLLM_DPP(v, 0xB1);
+      v += K8SLLM_DPP(v, 0x4E);
       if ((t & 3) == 0) s_inv[t >> 2] = rsqrtf(v * rn_inv_d + rn_eps);
     }
   }

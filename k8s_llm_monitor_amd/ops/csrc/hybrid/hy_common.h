@@ -48,18 +48,6 @@ __device__ __forceinline__ uint4 tokens_below(uint4 v, int j, int end) {
   return make_uint4(v.x & pair_below(j, end), v.y & pair_below(j + 2, end), v.z & pair_below(j + 4, end), v.w & pair_below(j + 6, end));
 }
 
-// Wave-wide butterflies without the LDS crossbar: quads and rows by DPP (quad_perm, the row's mirror
-// controls pair equal partial results), rows 0/1 and 2/3 by v_permlane16_swap, the halves by
-// v_permlane32_swap.  Every lane ends with the result.
-#define K8SLLM_DPP(v, ctrl) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true))
-__device__ __forceinline__ float xor16_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float xor16_max(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 // Two values' sums at once: even rows (the lower half) end with a's sum over the two rows (halves), odd ones (the upper) with b's
 __device__ __forceinline__ float swap16_sum(float a, float b) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
@@ -69,14 +57,7 @@ __device__ __forceinline__ float swap32_sum(float a, float b) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-__device__ __forceinline__ float xor32_sum_f(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float xor32_max_f(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
+// as wave_sum and wave_max, nearest lanes first
 __device__ __forceinline__ float wave_sum_dpp(float v) {
   v += K8SLLM_DPP(v, 0xB1);
   v += K8SLLM_DPP(v, 0x4E);

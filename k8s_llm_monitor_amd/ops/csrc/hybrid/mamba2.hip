@@ -26,7 +26,7 @@ __device__ __forceinline__ float group_sum(float v) {
   if (CH >= 4) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));
   if (CH >= 8) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));
   if (CH >= 16) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xf, 0xf, true));
-  if (CH >= 32) v += __shfl_xor(v, 16, 64);
+  if (CH >= 32) v = xor16_sum(v);
   return v;
 }
 
@@ -296,8 +296,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(float* __restrict__ y, co
         S[4 * i + 3] = dA * S[4 * i + 3] + dtx * bv.w;
         acc += S[4 * i + 0] * cv.x + S[4 * i + 1] * cv.y + S[4 * i + 2] * cv.z + S[4 * i + 3] * cv.w;
       }
-      acc += __shfl_xor(acc, 16, 64);
-      acc += __shfl_xor(acc, 32, 64);
+      acc = xor32_sum_f(xor16_sum(acc));
       if (live && lane < 16) y[(long)(tb + tt) * inner + (long)h * P + p] = acc + Dh * x;
     }
   }

@@ -242,8 +242,7 @@ __global__ __launch_bounds__(256, TW == 32 ? 2 : 1) void paged_decode_kernel(bf1
         sacc[i][r] = v;
         mx = fmaxf(mx, v);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = xor32_max_f(xor16_max(mx));
     const float mnew = fmaxf(m, mx);
     const float alpha = exp2f(m - mnew);
     float ls = 0.f;
@@ -255,8 +254,7 @@ __global__ __launch_bounds__(256, TW == 32 ? 2 : 1) void paged_decode_kernel(bf1
         sacc[i][r] = p;
         ls += p;
       }
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
+    ls = xor32_sum_f(xor16_sum(ls));
     l = l * alpha + ls;
     m = mnew;
     // ---- P V  (oacc rows are dims, columns are heads: the rescale is per column = per lane)
@@ -303,8 +301,7 @@ __global__ __launch_bounds__(256, TW == 32 ? 2 : 1) void paged_decode_kernel(bf1
         const int d = kg * (D / 4) + j;
         sc += bf2f(s_q[hc][d]) * bf2f(s_kv[0][d]);
       }
-      sc += __shfl_xor(sc, 16, 64);
-      sc += __shfl_xor(sc, 32, 64);
+      sc = xor32_sum_f(xor16_sum(sc));
       sc *= scale_log2;
       const float mnew = fmaxf(m, sc);
       const float alpha = exp2f(m - mnew);
