@@ -624,6 +624,21 @@ def test_gated_group_norm_sizes(n, groups, after, gate, dt):
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("rows,groups,gs", [(1, 2, 64), (3, 3, 64), (5, 33, 64), (1, 2, 128), (7, 5, 128), (1, 2, 256), (3, 9, 256)])
+@pytest.mark.parametrize("col", [0, 8, 5])
+@pytest.mark.parametrize("gate", ["silu", "sigmoid"])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_head_norm_sizes(rows, groups, gs, col, gate, dt):
+    """Per-head norms of 64, 128 and 256 values, eight a lane, around whole workgroups (256 lanes), and a column where the gate's rows are not
+    aligned (a wave a group).  fp32 inside: 1e-5 of the value, and the rounding of a bf16 result."""
+    g = _g(81)
+    n = groups * gs
+    y, z, w = _r(g, rows, n), _r(g, rows, n + 8, dt=dt), _r(g, n)
+    want = hops.gated_group_norm(y, z, col, w, 1e-5, groups, dt, after=True, gate=gate)
+    got = hops.gated_group_norm(y.cuda(), z.cuda(), col, w.cuda(), 1e-5, groups, dt, after=True, gate=gate)
+    torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("Hq,G,dk,dv", [(1, 1, 1, 1), (2, 1, 128, 64), (16, 4, 128, 128), (17, 1, 128, 8), (32, 8, 128, 16), (33, 3, 128, 8)])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
 def test_qk_norm_sizes(Hq, G, dk, dv, dt):
