@@ -639,6 +639,23 @@ def test_head_norm_sizes(rows, groups, gs, col, gate, dt):
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("T,d,E,K,shared", [(1000, 2048, 8, 2, False), (1003, 8, 3, 1, True), (4100, 1000, 7, 7, True), (2049, 2056, 8, 8, False),
+                                            (2050, 4096, 5, 2, True)])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_router_long_steps(T, d, E, K, shared, dt):
+    """The router that keeps its weights in registers, around a round of four tokens and 2048 columns: the same bits as of short steps."""
+    g = _g(84)
+    h, wr, bias = _r(g, T, d, dt=dt).cuda(), _r(g, E + shared, d, s=0.3).cuda(), _r(g, E, s=0.3).cuda()
+    h[5, d // 2] = math.nan
+    h[T - 1] = 0.0  # ties, but for the bias
+    got = hops.moe_router(h, wr, bias, E, K)
+    parts = [hops.moe_router(h[i:i + 200], wr, bias, E, K) for i in range(0, T, 200)]
+    for x, *ys in zip(got, *parts):
+        if x is not None:
+            y = torch.cat(ys)
+            assert torch.equal(torch.nan_to_num(x, nan=-1.0) if x.is_floating_point() else x, torch.nan_to_num(y, nan=-1.0) if y.is_floating_point() else y)
+
+
 @pytest.mark.parametrize("Hq,G,dk,dv", [(1, 1, 1, 1), (2, 1, 128, 64), (16, 4, 128, 128), (17, 1, 128, 8), (32, 8, 128, 16), (33, 3, 128, 8)])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
 def test_qk_norm_sizes(Hq, G, dk, dv, dt):
