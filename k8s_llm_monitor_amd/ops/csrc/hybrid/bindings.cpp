@@ -58,7 +58,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
 int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                             const int* block_tables, int bt_stride, const int* seq_lens, int B, int Hq, int G, int dk,
                             int dv, int bs, float scale, int window, int chunked, int keep, float cap, int sink,
-                            const float* sinks, const void* gate, long g_stride, int f32, int vec, hipStream_t s);
+                            const float* sinks, const void* gate, long g_stride, int f32, int vec, int heads, hipStream_t s);
 int k8sllm_hy_conv_silu(void* out, const void* proj, long stride, int col0, int C, const float* cw, const float* cb,
                         int taps, void* state, const int* cu, const int* ctx, const int* slot, int S, long T, int f32,
                         hipStream_t s);
@@ -394,7 +394,7 @@ void window_attention_prefill(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_c
 void window_attention_decode(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_cache, Tensor block_tables,
                              Tensor seq_lens, int64_t Hq, int64_t G, int64_t dk, int64_t dv, double scale,
                              int64_t window, bool sink, OptT sinks, bool vec, bool chunked, double cap, int64_t keep,
-                             OptT gate, int64_t g_col) {
+                             OptT gate, int64_t g_col, int64_t heads) {
   const int f = act(qkv, "qkv");
   same(out, f, "out");
   pages(k_cache, f, G * dk, "k_cache");
@@ -414,7 +414,7 @@ void window_attention_decode(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_ca
                                 block_tables.data_ptr<int>(), (int)block_tables.stride(0), seq_lens.data_ptr<int>(),
                                 (int)B, (int)Hq, (int)G, (int)dk, (int)dv, (int)k_cache.size(1), (float)scale,
                                 (int)window, chunked, (int)keep, (float)cap, sink, sink_ptr(sinks, Hq), ga.p, ga.stride,
-                                f, vec, cur()),
+                                f, vec, (int)heads, cur()),
         "window_attention_decode");
 }
 

@@ -440,6 +440,16 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
 }
 
+// Query heads that a workgroup of the kernel below takes, R sharing a kv head: the fewest that leave each of 256 compute units at most one
+// workgroup, all that its registers let it run.  A wave's tile costs its instructions for every head, and its keys' loads once for each
+// workgroup.  us, all heads / half / one of four: 1 sequence of 333 keys, 8 heads on 2 14.1 / 11.2 / 9.7; 8 of 1500, 16 on 4 42.2 / 33.3 /
+// 29.2; 24 of 1500, 16 on 4 45.2 / 36.0 / 53.8; 64 of 1024 41.5 / 53.4 / 83.4; 16 of 1500, 8 heads on one, all / 2 / 1: 75.2 / 43.4 / 38.6.
+inline int decode_heads(long B, int Hq, int R) {
+  for (int heads : {1, 2})
+    if (heads < R && R % heads == 0 && B * Hq <= 256L * heads) return heads;
+  return R;
+}
+
 // The same for head sizes of 64 and 128, without the LDS reads that bound it (a tile of 64 keys took a wave 256 16-byte reads of
 // queries and weights that all lanes share): each 16-lane row holds all dims of the queries, 16 to a register, and a page's 16
 // weights in one, and the multiply-adds pick the element by their DPP row broadcast.  Keys and values of a tile are in flight
@@ -459,14 +469,14 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
   __shared__ float ml_s[NW][R][2];
   __shared__ float acc_s[NW][R][64 * VC];
   constexpr int dk = 64 * DKC, dv = 64 * VC;
-  const int b = blockIdx.x, g = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int b = blockIdx.x, h0 = blockIdx.y * R, g = h0 / (Hq / G), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = seq_lens[b];
-  bf16_t* o = out + (long)b * Hq * dv + (long)g * R * dv;
+  bf16_t* o = out + (long)b * Hq * dv + (long)h0 * dv;
   if (n <= 0) {  // padding row of a decode bucket
     for (int c = threadIdx.x; c < R * dv; c += 64 * NW) o[c] = 0;
     return;
   }
-  const bf16_t* q = qkv + (long)b * q_stride + (long)g * R * dk;
+  const bf16_t* q = qkv + (long)b * q_stride + (long)h0 * dk;
   // base-2 scores; lane l of every 16-lane row holds the queries' dims 16 i + l % 16
   float qr[R][4 * DKC];
 #pragma unroll
@@ -481,7 +491,7 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     // the sink's logit is not scaled; scores live in the base-2 domain
-    m[r] = first ? (sinks != nullptr ? sinks[g * R + r] * 1.44269504088896341f : 0.f) : -INFINITY;
+    m[r] = first ? (sinks != nullptr ? sinks[h0 + r] * 1.44269504088896341f : 0.f) : -INFINITY;
     l[r] = first ? 1.f : 0.f;
 #pragma unroll
     for (int c = 0; c < VC; ++c) acc[r][c] = 0.f;
@@ -611,7 +621,7 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
       L += ml_s[w][r][1] * f;
       val += acc_s[w][r][dcol] * f;
     }
-    const float gt = gate != nullptr ? sigmoid_f(bf2f(gate[(long)b * g_stride + g * R + r])) : 1.f;
+    const float gt = gate != nullptr ? sigmoid_f(bf2f(gate[(long)b * g_stride + h0 + r])) : 1.f;
     o[c] = f2bf(L > 0.f ? val / L * gt : 0.f);
   }
 }
@@ -992,22 +1002,26 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
 int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                             const int* block_tables, int bt_stride, const int* seq_lens, int B, int Hq, int G, int dk,
                             int dv, int bs, float scale, int window, int chunked, int keep, float cap, int sink,
-                            const float* sinks, const void* gate, long g_stride, int f32, int vec, hipStream_t s) {
+                            const float* sinks, const void* gate, long g_stride, int f32, int vec, int heads, hipStream_t s) {
   if (B <= 0) return 0;
   if (keep < 0 || (keep > 0 && (chunked || window <= 0))) return -1;
   if (dk > kGenDK || dv > 64 * kGenVC || G < 1 || Hq % G) return -1;
   const int R = Hq / G;
   if (!f32 && vec && bs == 16 && dk % 8 == 0 && q_stride % 8 == 0 && dk <= kMaxDK && dv <= 64 * kMaxVC &&
       (R == 1 || R == 2 || R == 4 || R == 8)) {
-#define K8SLLM_WDR(RR, DKC, VC)                                                                                        \
-  hipLaunchKernelGGL((window_decode_row_kernel<RR, (RR == 8 ? 4 : 8), DKC, VC>), dim3(B, G), dim3(RR == 8 ? 256 : 512), 0, s, \
-                     (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, \
-                     bt_stride, seq_lens, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
-#define K8SLLM_WDD(DKC, VC)             \
-  if (R == 1) K8SLLM_WDR(1, DKC, VC);   \
-  else if (R == 2) K8SLLM_WDR(2, DKC, VC); \
-  else if (R == 4) K8SLLM_WDR(4, DKC, VC); \
-  else K8SLLM_WDR(8, DKC, VC)
+#define K8SLLM_WDR(RR, NW, DKC, VC)                                                                                    \
+  hipLaunchKernelGGL((window_decode_row_kernel<RR, NW, DKC, VC>), dim3(B, Hq / RR), dim3(64 * NW), 0, s, (bf16_t*)out,   \
+                     (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, \
+                     seq_lens, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
+#define K8SLLM_WDD(DKC, VC)                                 \
+  if (R == 8 && heads == 8) K8SLLM_WDR(8, 4, DKC, VC);      \
+  else if (R == 8 && heads == 2) K8SLLM_WDR(2, 4, DKC, VC); \
+  else if (R == 8) K8SLLM_WDR(1, 4, DKC, VC);               \
+  else if (heads == 4) K8SLLM_WDR(4, 8, DKC, VC);           \
+  else if (heads == 2) K8SLLM_WDR(2, 8, DKC, VC);           \
+  else K8SLLM_WDR(1, 8, DKC, VC)
+    if (heads == 0) heads = decode_heads(B, Hq, R);
+    if (heads < 1 || R % heads || (R == 8 && heads == 4)) return -1;
     if ((dk == 64 || dk == 128) && (dv == 64 || dv == 128)) {
       if (dk == 64 && dv == 64) { K8SLLM_WDD(1, 1); }
       else if (dk == 64) { K8SLLM_WDD(1, 2); }

@@ -552,11 +552,12 @@ def window_attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: t
                             block_tables: torch.Tensor, seq_lens: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int,
                             scale: float, window: int, sink: bool, vec: bool = True,
                             sinks: Optional[torch.Tensor] = None, chunked: bool = False, cap: float = 0.0, keep: int = 0,
-                            gate: Optional[torch.Tensor] = None, g_col: int = 0) -> torch.Tensor:
+                            gate: Optional[torch.Tensor] = None, g_col: int = 0, heads: int = 0) -> torch.Tensor:
     """One query per sequence (its newest token, already in the cache) over the last ``window``
     cached positions (``chunked``: those of its own chunk; ``cap``, ``keep``, ``gate``: as in
     window_attention_prefill);
-    ``seq_lens`` count that token (0: a padding row, output zero)."""
+    ``seq_lens`` count that token (0: a padding row, output zero).  ``heads``: query heads of a kv
+    head that a workgroup takes (``vec``, head sizes of 64 and 128; 0: its choice)."""
     B = qkv.shape[0]
     if not qkv.is_cuda:
         out = torch.zeros(B, Hq * dv, dtype=qkv.dtype)
@@ -574,7 +575,7 @@ def window_attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     out = torch.empty(B, Hq * dv, dtype=qkv.dtype, device=qkv.device)
     native().window_attention_decode(out, qkv, k_cache, v_cache, block_tables, seq_lens, Hq, Hkv, dk, dv, float(scale),
                                      int(window), bool(sink), sinks, bool(vec), bool(chunked), float(cap), int(keep), gate,
-                                     int(g_col))
+                                     int(g_col), int(heads))
     return out
 
 

@@ -656,6 +656,25 @@ def test_router_long_steps(T, d, E, K, shared, dt):
             assert torch.equal(torch.nan_to_num(x, nan=-1.0) if x.is_floating_point() else x, torch.nan_to_num(y, nan=-1.0) if y.is_floating_point() else y)
 
 
+@pytest.mark.parametrize("Hq,G,dk,dv,window", [(4, 1, 64, 64, 0), (8, 1, 128, 128, 40), (8, 4, 128, 64, 0), (16, 2, 64, 128, 100), (4, 1, 128, 128, 64)])
+def test_window_decode_heads(Hq, G, dk, dv, window):
+    """Fewer query heads a workgroup than share a kv head: the same bits as all of them together, sinks and head gates included."""
+    g = _g(82)
+    lens = [1, 64, 65, 700, 17]
+    kc, vc, bt = _paged(g, BF, lens, Hq, G, dk, dv, nb=80)
+    q, gate, sinks = _r(g, len(lens) + 1, Hq * dk + 8, dt=BF), _r(g, len(lens) + 1, Hq + 8, dt=BF), _r(g, Hq)
+    bt = torch.cat([bt, torch.zeros(1, bt.shape[1], dtype=torch.int32)])
+    dev = [t.cuda() for t in (q, kc, vc, bt, _i32(lens + [0]))]
+    a = (Hq, G, dk, dv, 1.0 / math.sqrt(dk), window, True)
+    for kw in (dict(), dict(sinks=sinks.cuda(), gate=gate.cuda(), g_col=3, cap=9.0)):
+        want = hops.window_attention_decode(*dev, *a, **kw, heads=Hq // G)
+        for heads in (0, 2, 1):
+            if heads == 0 or (Hq // G) % heads == 0:
+                assert torch.equal(hops.window_attention_decode(*dev, *a, **kw, heads=heads), want)
+    with pytest.raises(RuntimeError):
+        hops.window_attention_decode(*dev, *a, heads=3)
+
+
 @pytest.mark.parametrize("Hq,G,dk,dv", [(1, 1, 1, 1), (2, 1, 128, 64), (16, 4, 128, 128), (17, 1, 128, 8), (32, 8, 128, 16), (33, 3, 128, 8)])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
 def test_qk_norm_sizes(Hq, G, dk, dv, dt):
