@@ -441,9 +441,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // Query heads that a workgroup of the kernel below takes, R sharing a kv head: the fewest that leave each of 256 compute units at most one
-// workgroup, all that its registers let it run.  A wave's tile costs its instructions for every head, and its keys' loads once for each
-// workgroup.  us, all heads / half / one of four: 1 sequence of 333 keys, 8 heads on 2 14.1 / 11.2 / 9.7; 8 of 1500, 16 on 4 42.2 / 33.3 /
-// 29.2; 24 of 1500, 16 on 4 45.2 / 36.0 / 53.8; 64 of 1024 41.5 / 53.4 / 83.4; 16 of 1500, 8 heads on one, all / 2 / 1: 75.2 / 43.4 / 38.6.
+// workgroup, all that its registers and LDS let it run.  A wave's tile costs its instructions for every head, and its keys' loads once for each
+// workgroup.  us, all heads / half / one of four: 1 sequence of 333 keys, 8 heads on 2 10.9 / 7.8 / 6.6; 8 of 1500, 16 on 4 30.6 / 22.6 /
+// 19.3; 24 of 1500, 16 on 4 35.6 / 27.5 / 36.3; 64 of 1024 35.0 / 39.9 / 58.8; 16 of 1500, 8 heads on one, all / 2 / 1: 58.2 / 28.6 / 25.5.
 inline int decode_heads(long B, int Hq, int R) {
   for (int heads : {1, 2})
     if (heads < R && R % heads == 0 && B * Hq <= 256L * heads) return heads;
@@ -455,7 +455,11 @@ inline int decode_heads(long B, int Hq, int R) {
 // weights in one, and the multiply-adds pick the element by their DPP row broadcast.  Keys and values of a tile are in flight
 // together.  Sums in the same order: the same bits.
 // 64 sequences, 1024 visible keys, 16 heads on 4 of 128: 40.8 -> 34.3 us (3.9 TB/s); 24 of ~1200, 32 on 8: 28.1 -> 25.5; 5 of 700, 8
-// heads on one of 128 / 64: 37 -> 27.  What is left of a tile is its ~1500 vector instructions.
+// heads on one of 128 / 64: 37 -> 27.
+// A tile's keys come to LDS by whole rows, 16 lanes a row, and the next tile's while this one is multiplied; a lane then reads its own.
+// Loads of a row a lane met 64 rows at a time, which is 64 cycles of the load path each, and a page's values, loaded behind a
+// branch, waited for the page before.  The same bits.  us, at decode_heads' choice: 1 sequence of 333 keys, 8 heads on 2 9.7 -> 6.6; of
+// 8000, 16 on 4 131 -> 74; 24 of 1500 36.0 -> 27.5; 64 of 1024 41.5 -> 35.0; 16 of 1500, 8 heads on one 38.6 -> 25.5.
 template <int R, int NW, int DKC, int VC>
 __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv,
                                                                 long q_stride, const bf16_t* __restrict__ k_cache,
@@ -465,17 +469,46 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
                                                                 float cap, int sink, const float* __restrict__ sinks,
                                                                 const bf16_t* __restrict__ gate, long g_stride) {
   constexpr int bs = 16;
-  __shared__ __attribute__((aligned(16))) float p_s[NW][R][64];
   __shared__ float ml_s[NW][R][2];
-  __shared__ float acc_s[NW][R][64 * VC];
   constexpr int dk = 64 * DKC, dv = 64 * VC;
-  const int b = blockIdx.x, h0 = blockIdx.y * R, g = h0 / (Hq / G), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  static_assert(4 * R * dv <= 128 * dk, "");
+  __shared__ __attribute__((aligned(1024))) char k_s[NW][128 * dk];  // a wave's tile of keys; its results when the keys are done
+  const int b = blockIdx.x, h0 = blockIdx.y * R, g = h0 / (Hq / G), lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = seq_lens[b];
   bf16_t* o = out + (long)b * Hq * dv + (long)h0 * dv;
   if (n <= 0) {  // padding row of a decode bucket
     for (int c = threadIdx.x; c < R * dv; c += 64 * NW) o[c] = 0;
     return;
   }
+  const int* bt = block_tables + (long)b * bt_stride;
+  const int lo = first_key(n - 1, window, chunked);
+  const long krs = (long)G * dk;
+  // the tiles that hold kept keys (kt of them, from position 0), then the window's from w0 on
+  const int kf = min(keep, n), kt = (kf + 63) >> 6, w0 = max(kt, lo >> 6);
+  auto tile = [&](int it) { return 64 * (it < kt ? it : w0 + it - kt); };
+  // keys j0 .. j0 + 63 to LDS, a row's 16-byte chunks turned by the row; pages without a key to be seen: the newest one's instead
+  constexpr int LPK = dk / 8, RPI = 64 / LPK;
+  auto turn = [](int r) { return DKC == 2 ? r & 15 : (r >> 1) & 7; };
+  auto stage = [&](int j0) {
+    long page[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int f = j0 + 16 * p;
+      page[p] = (long)bt[((f < n) & ((f + 15 >= lo) | (f < keep)) ? f : n - 1) / bs] * bs;
+    }
+#pragma unroll
+    for (int i = 0; i < LPK; ++i) {
+      const int r = i * RPI + lane / LPK;
+      load_piece(k_s[wave] + 1024 * i, k_cache + (page[i * RPI / bs] + r % bs) * krs + (long)g * dk + 8 * ((lane % LPK) ^ turn(r)));
+    }
+  };
+  int it = wave, j0 = tile(it);
+  if (j0 < n) stage(j0);
+  // loads from an argument may sink past a barrier into the branch of their use: an address of unknown origin
+  uint32_t vlo = (uint32_t)reinterpret_cast<uint64_t>(v_cache), vhi = (uint32_t)(reinterpret_cast<uint64_t>(v_cache) >> 32);
+  asm volatile("" : "+v"(vlo), "+v"(vhi));
+  const long values = (long)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(vhi) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane(vlo));
   const bf16_t* q = qkv + (long)b * q_stride + (long)h0 * dk;
   // base-2 scores; lane l of every 16-lane row holds the queries' dims 16 i + l % 16
   float qr[R][4 * DKC];
@@ -483,8 +516,6 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int i = 0; i < 4 * DKC; ++i) qr[r][i] = bf2f(q[r * dk + 16 * i + (lane & 15)]) * (scale * 1.44269504088896341f);
-  const int* bt = block_tables + (long)b * bt_stride;
-  const int lo = first_key(n - 1, window, chunked);
   const float cap2 = cap * 1.44269504088896341f, icap2 = cap > 0.f ? 1.f / cap2 : 0.f;  // base-2 scores
   const bool first = sink && wave == 0;
   float m[R], l[R], acc[R][VC];
@@ -496,40 +527,33 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
 #pragma unroll
     for (int c = 0; c < VC; ++c) acc[r][c] = 0.f;
   }
-  const long krs = (long)G * dk;
-  // the tiles that hold kept keys (kt of them, from position 0), then the window's from w0 on
-  const int kf = min(keep, n), kt = (kf + 63) >> 6, w0 = max(kt, lo >> 6);
-  for (int it = wave;; it += NW) {
-    const int j0 = 64 * (it < kt ? it : w0 + it - kt);
-    if (j0 >= n) break;
+  auto step = [&](int next, auto more) {  // no load behind a branch: the tile's values, then the next tile's keys, are on their way meanwhile
     const int j = j0 + lane;
     const bool valid = (j >= lo || j < keep) && j < n;
-    float sc[R];
+    float sc[R], p[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) sc[r] = 0.f;
-    // the lane's key row (of a key that is not seen: the newest one's)
-    uint4 kr[8 * DKC];
-    const int jc = valid ? j : n - 1;
-    const bf16_t* kp = k_cache + ((long)bt[jc / bs] * bs + jc % bs) * krs + (long)g * dk;
-#pragma unroll
-    for (int u = 0; u < 8 * DKC; ++u) kr[u] = *reinterpret_cast<const uint4*>(kp + 8 * u);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tile's keys are there
     // value loads of the tile's pages go out before the arithmetic: 2 x 16 bytes per page and
-    // 64 dims (pages at or past the sequence's end are not touched: their weights are zero)
+    // 64 dims (pages at or past the sequence's end are not touched: the last one is read again, and nothing multiplies it)
     const int jend = j0 + 64 > lo ? n : kf;  // a tile of kept keys alone: the pages behind them are not needed
     const int npg = min(4, (jend - j0 + bs - 1) / bs);
-    uint4 vq[4][VC][2];
+    uint4 vq[4][VC][2], kr[8 * DKC];
 #pragma unroll
-    for (int pg = 0; pg < 4; ++pg)
-      if (pg < npg) {
-        const long base = ((long)bt[j0 / bs + pg] * G + g) * dv;
+    for (int pg = 0; pg < 4; ++pg) {
+      const long base = ((long)bt[j0 / bs + min(pg, npg - 1)] * G + g) * dv;
 #pragma unroll
-        for (int c = 0; c < VC; ++c)
-        {
-          const uint4* vp = reinterpret_cast<const uint4*>(v_cache + (base + lane + 64 * c) * bs);
-          vq[pg][c][0] = vp[0];
-          vq[pg][c][1] = vp[1];
-        }
+      for (int c = 0; c < VC; ++c) {
+        using Raw = unsigned __attribute__((ext_vector_type(4)));
+        const auto vp = reinterpret_cast<__attribute__((address_space(1))) const Raw*>(values + 2 * (base + lane + 64 * c) * bs);
+        vq[pg][c][0] = __builtin_bit_cast(uint4, Raw(vp[0]));
+        vq[pg][c][1] = __builtin_bit_cast(uint4, Raw(vp[1]));
       }
+    }
+#pragma unroll
+    for (int u = 0; u < 8 * DKC; ++u) kr[u] = *reinterpret_cast<const uint4*>(k_s[wave] + 2 * dk * lane + 16 * (u ^ turn(lane)));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the keys have been read
+    if constexpr (decltype(more)::value) stage(next);
     static_for<8 * DKC>([&](auto uc) {
       constexpr int u = decltype(uc)::value;
       float kv[8];
@@ -549,7 +573,6 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
         }
       }
     });
-    __builtin_amdgcn_wave_barrier();  // this wave's previous reads of its p_s rows come first
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (cap > 0.f) sc[r] = cap2 * tanh_exp2(sc[r] * icap2);
@@ -559,17 +582,16 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
       const float alpha = (m[r] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[r] - mt);
       l[r] = l[r] * alpha + wave_sum_dpp(pw);
       m[r] = mt;
-      p_s[wave][r][lane] = pw;
+      p[r] = pw;
 #pragma unroll
       for (int c = 0; c < VC; ++c) acc[r][c] *= alpha;
     }
-    __builtin_amdgcn_wave_barrier();  // a wave's LDS instructions execute in issue order
 #pragma unroll
     for (int pg = 0; pg < 4; ++pg)
       if (pg < npg) {
         float pr[R];  // every row of lanes: the page's 16 weights
 #pragma unroll
-        for (int r = 0; r < R; ++r) pr[r] = p_s[wave][r][16 * pg + (lane & 15)];
+        for (int r = 0; r < R; ++r) pr[r] = __shfl(p[r], 16 * pg + (lane & 15), kWave);
 #pragma unroll
         for (int c = 0; c < VC; ++c) {
           if (j0 + 16 * pg + 16 > n) {  // the last page's unused end (uniform)
@@ -597,12 +619,16 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
           });
         }
       }
+  };
+  if (j0 < n) {
+    for (int next; (next = tile(it + NW)) < n; it += NW, j0 = next) step(next, std::true_type{});
+    step(0, std::false_type{});
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
 #pragma unroll
     for (int c = 0; c < VC; ++c)
-      acc_s[wave][r][lane + 64 * c] = acc[r][c];
+      reinterpret_cast<float*>(k_s[wave])[r * dv + lane + 64 * c] = acc[r][c];
     if (lane == 0) {
       ml_s[wave][r][0] = m[r];
       ml_s[wave][r][1] = l[r];
@@ -619,7 +645,7 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
     for (int w = 0; w < NW; ++w) {
       const float f = ml_s[w][r][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml_s[w][r][0] - M);
       L += ml_s[w][r][1] * f;
-      val += acc_s[w][r][dcol] * f;
+      val += reinterpret_cast<const float*>(k_s[w])[r * dv + dcol] * f;
     }
     const float gt = gate != nullptr ? sigmoid_f(bf2f(gate[(long)b * g_stride + h0 + r])) : 1.f;
     o[c] = f2bf(L > 0.f ? val / L * gt : 0.f);
