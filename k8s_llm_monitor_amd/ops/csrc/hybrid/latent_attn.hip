@@ -112,8 +112,9 @@ __global__ __launch_bounds__(256) void latent_queries_kernel(T* __restrict__ out
 //   O^T[d][head]  += V^T P^T   v_mfma_f32_16x16x16_bf16: B = the score accumulator itself, A = V^T,
 //                              8-byte loads from the dim-major latent page
 // The NW waves of a workgroup take the window's 16-key tiles in turn (decoding: the window is the
-// only parallel axis of a row) and merge their (maximum, denominator, output) through LDS: the common
-// maximum first, then the outputs summed wave after wave into one buffer.  Only wave 0 starts from
+// only parallel axis of a row) and merge their (maximum, denominator, output) through LDS, a copy each, in the order
+// of the waves behind one barrier (before, a wave at a time into one copy, a barrier each, us: 1 sequence of
+// 333 keys, 8 heads, 128 + 32 wide 11.6, now 8.0; 32 of 1500, 16 heads, 256 + 32 53.4, now 48.4).  Only wave 0 starts from
 // the sink.  Scores, weights and sums are fp32, base-2 exponentials (the scale carries log2 e).
 // QT consecutive tokens of a prompt chunk share a wave's key and value fragments (their windows
 // differ by one key at each end).  gate (optional): one logit per row and head; the head's output is
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
     int dv, float scale, int window, const float* __restrict__ sinks, const bf16_t* __restrict__ gate, long g_stride) {
   static_assert(NW == 1 || QT == 1, "the window is split over waves only for single tokens");
   constexpr int OP = DT_MAX * 16 + 4;  // LDS row pitch of the merge buffer (floats)
-  __shared__ __attribute__((aligned(16))) float o_s[NW > 1 ? 16 * OP : 4];
+  __shared__ __attribute__((aligned(16))) float o_s[NW][NW > 1 ? 16 * OP : 4];
   __shared__ float m_s[NW > 1 ? NW : 1][16];
   __shared__ float l_s[NW > 1 ? NW : 1][16];
   const float sc2 = scale * 1.44269504088896341f;
@@ -327,36 +328,29 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
     }
     return;
   }
-  if (quad == 0) m_s[wave][c16] = m[0];
-  __syncthreads();
-  float M = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) M = fmaxf(M, m_s[w][c16]);  // wave 0's is finite (the sink)
-  const float f = m[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[0] - M);
-  if (quad == 0) l_s[wave][c16] = l[0] * f;
-  for (int w = 0; w < NW; ++w) {
-    if (wave == w) {
-#pragma unroll
-      for (int dt = 0; dt < DT_MAX; ++dt)
-        if (dt < ndt) {
-          float4* dst = reinterpret_cast<float4*>(&o_s[c16 * OP + 16 * dt + 4 * quad]);
-          float4 v = make_float4(oacc[0][dt][0] * f, oacc[0][dt][1] * f, oacc[0][dt][2] * f, oacc[0][dt][3] * f);
-          if (w > 0) {
-            const float4 o = *dst;
-            v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
-          }
-          *dst = v;
-        }
-    }
-    __syncthreads();
+  if (quad == 0) {
+    m_s[wave][c16] = m[0];
+    l_s[wave][c16] = l[0];
   }
+#pragma unroll
+  for (int dt = 0; dt < DT_MAX; ++dt)
+    if (dt < ndt)
+      *reinterpret_cast<float4*>(&o_s[wave][c16 * OP + 16 * dt + 4 * quad]) =
+          make_float4(oacc[0][dt][0], oacc[0][dt][1], oacc[0][dt][2], oacc[0][dt][3]);
+  __syncthreads();
   for (int c = threadIdx.x; c < nh * dv; c += 64 * NW) {
     const int hh = c / dv, dd = c - hh * dv;
-    float L = 0.f;
+    float M = -INFINITY, L = 0.f, o = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) L += l_s[w][hh];
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, m_s[w][hh]);  // wave 0's is finite (the sink)
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = m_s[w][hh] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_s[w][hh] - M);
+      L = fmaf(l_s[w][hh], f, L);
+      o = fmaf(o_s[w][hh * OP + dd], f, o);
+    }
     const float gt = gate != nullptr ? sigmoid_f(bf2f(gate[(long)row0 * g_stride + hg * 16 + hh])) : 1.f;
-    obase[c] = f2bf(L > 0.f ? o_s[hh * OP + dd] / L * gt : 0.f);
+    obase[c] = f2bf(L > 0.f ? o / L * gt : 0.f);
   }
 }
 
