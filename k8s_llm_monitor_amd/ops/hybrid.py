@@ -1095,8 +1095,8 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
     synchronisation.  bf16: matrix-core kernels - tiles of 16, 32 or 64 rows by the mean rows of an expert, gathered on load
     (decode, small steps), or from TILE_MIN_ROWS sorted rows of an ``il`` layer the prefill tile
     GEMM of the Mixtral path, which reads the rows in sorted order from where they are (ungated experts whose widths are multiples of 256 take it too, with
-    the GELU as a launch between); fp32: 64 x 64 tiles on the fp32 matrix instruction.  K that is no multiple of 32 and
-    unaligned fp32 rows: 64 x 64 tiles on the vector unit."""
+    the GELU as a launch between); fp32: three-part operands on the bf16 matrix instruction (experts_f32.hip).  K that is no multiple of 32
+    and unaligned fp32 rows: 64 x 64 tiles on the vector unit."""
     T, d = h.shape
     E, K = w13.shape[0], ids.shape[1]
     ff = w2.shape[2]
