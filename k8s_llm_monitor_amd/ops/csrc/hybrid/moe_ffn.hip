@@ -722,8 +722,9 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
   if (act < 0 || act > 4) return -1;
   const bool swiglu = act == 1;
   if (il && (!swiglu || N % 64)) return -1;
-  const bool aligned = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  if (!f32 && mfma && Kd % 32 == 0 && aligned) {
+  // whole steps of 32 k, at least one: both matrix-core kernels load their first step before they look at how many there are
+  const bool steps = Kd >= 32 && Kd % 32 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
+  if (!f32 && mfma && steps) {
     // a workgroup takes 16, 32 or 64 rows of an expert, so that its weights are mostly read once, by the mean number of rows an
     // expert gets (8 experts, 2048 x 2048, gated + plain: mean 16 60 / 50 / 52 us with 16 / 32 / 64 rows, 32 69 / 64 / 52; 32 experts,
     // mean 8: 157 / 177).  Two waves or, for 64 rows and where plain columns fill the chip, four (gated, two / four: 4096 x 3584, 8
@@ -755,7 +756,7 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
 #undef K8SLLM_GM
     return (int)hipGetLastError();
   }
-  if (f32 && Kd % 32 == 0 && aligned)
+  if (f32 && steps)
     return k8sllm_hy_experts_f32((float*)Y, (const float*)A, (const float*)W, offsets, sorted_idx, div, E, rows, N, Kd, w_es, act, il, limit, s);
   // other K and alignments: the vector unit
   const dim3 grid((unsigned)(rows / TM + E), (unsigned)((N + TN - 1) / TN));

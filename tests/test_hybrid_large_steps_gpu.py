@@ -578,6 +578,17 @@ def test_linear_of_nothing():
     assert a.shape == (2, 0) and torch.equal(y[:, col:], hops.linear(x, w))
 
 
+@pytest.mark.parametrize("rows", [1, 40, 700])
+@pytest.mark.parametrize("act", [0, 1, 3, 4])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_experts_of_empty_sums(rows, act, dt):
+    """Products over no k are zero, and so is what every unit makes of them."""
+    a, w = torch.empty(rows, 0, dtype=dt, device="cuda"), torch.empty(2, 48, 0, dtype=dt, device="cuda")
+    y = torch.full((rows, 24 if act in (1, 3) else 48), float("nan"), dtype=dt, device="cuda")
+    hops.native().grouped_gemm(y, a, w, _i32([0, rows // 3, rows]).cuda(), None, 1, act, False, True, 7.0 if act == 3 else 0.0)
+    assert not bool(y.any()) and not bool(y.isnan().any())
+
+
 @pytest.mark.parametrize("M,f,rest,K", [(1, 16, 0, 32), (3, 48, 40, 1024), (16, 176, 16, 160), (17, 32, 8, 64), (2, 24, 8, 64)])
 @pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
 def test_gated_unit_in_the_projection(M, f, rest, K, kind):
