@@ -659,7 +659,8 @@ int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, i
 #define K8SLLM_RT(T_, NACC, TPW)                                                                                       \
   hipLaunchKernelGGL((hy_router_kernel<T_, NACC, TPW>), dim3((unsigned)((T + TPW - 1) / TPW)), dim3(256), 0, s, ids, wts, gate, \
                      (const T_*)h, (int)T, d, wr, bias, E, K, rows_w, over_all)
-  if (rows_w <= 8 && d % 8 == 0 && d <= 4096 && T >= kRouterWalkRows) {
+  // (d of at least 8: a lane behind the last column reads the last eight instead)
+  if (rows_w <= 8 && d >= 8 && d % 8 == 0 && d <= 4096 && T >= kRouterWalkRows) {
     const dim3 grid((unsigned)std::min((T + 3) / 4, 512L));
 #define K8SLLM_RK(T_, NC)                                                                                                  \
   hipLaunchKernelGGL((hy_router_walk_kernel<T_, NC>), grid, dim3(256), 0, s, ids, wts, gate, (const T_*)h, (int)T, d, wr, bias, E, K, \

@@ -667,6 +667,18 @@ def test_router_long_steps(T, d, E, K, shared, dt):
             assert torch.equal(torch.nan_to_num(x, nan=-1.0) if x.is_floating_point() else x, torch.nan_to_num(y, nan=-1.0) if y.is_floating_point() else y)
 
 
+@pytest.mark.parametrize("T", [300, 4100])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_router_of_empty_sums(T, dt):
+    """Rows of no columns leave the bias's choice: logits that are its values exactly, softmax to rounding."""
+    bias = _r(_g(85), 4)
+    h, wr = torch.empty(T, 0, dtype=dt), torch.empty(4, 0)
+    want = hops.moe_router(h, wr, bias, 4, 2)
+    ids, wts, _ = hops.moe_router(h.cuda(), wr.cuda(), bias.cuda(), 4, 2)
+    assert torch.equal(ids.cpu(), want[0])
+    torch.testing.assert_close(wts.cpu(), want[1], rtol=1e-6, atol=1e-6)
+
+
 @pytest.mark.parametrize("Hq,G,dk,dv,window", [(4, 1, 64, 64, 0), (8, 1, 128, 128, 40), (8, 4, 128, 64, 0), (16, 2, 64, 128, 100), (4, 1, 128, 128, 64)])
 def test_window_decode_heads(Hq, G, dk, dv, window):
     """Fewer query heads a workgroup than share a kv head: the same bits as all of them together, sinks and head gates included."""
