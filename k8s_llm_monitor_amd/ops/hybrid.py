@@ -1195,26 +1195,28 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 TILE_UNITS = {"gelu_tanh": 5, "silu": 6, "relu": 7, "relu_sq": 8}  # epilogues of ops.gemm_tile_unit
 
 
-def _tile_rounds_ok(tiles: int) -> bool:
-    """One 256 x 256 tile a compute unit at a time: a last round that is mostly empty takes as long as a full one."""
-    return tiles >= 200 and tiles >= 0.7 * 256 * -(-tiles // 256)
+def _tile_form(M: int, N: int, K: int, f: int) -> bool:
+    """Whether the tile GEMM takes a large product with a unit at its end (a gated one of f features, or f 0): its tiles take 5 % longer
+    than the BLAS library's, which leaves the unit a launch of its own that reads and writes the products once more.  us, library and
+    launch / tile GEMM: 7830 rows, 2 x 5632 + 2048 columns, K 2048 388 + 47 / 355; 3749 rows 236 + 25 / 195; 6403 x 4096 x 1024 (1.6
+    rounds of tiles) 53 + 18 / 58.  At least four fifths of the tiles' area must be products: 53248 columns, K 2048 1 row 48 / 62, 128
+    rows 59 / 64, 300 rows (two row tiles) 97 / 109, 256 rows 74 / 68, 1300 rows (six) 331 / 279."""
+    tiles = -(-M // 256) * (-(-f // 128) + -(-(N - 2 * f) // 256))
+    # one tile a compute unit at a time: a last round that is mostly empty takes as long as a full one
+    return (tiles >= 200 and tiles >= 0.7 * 256 * -(-tiles // 256) and M * N >= 0.8 * 256 * 256 * tiles
+            and K % 64 == 0 and K >= 192 and N % 16 == 0 and f % 16 == 0 and 2 * f <= N and max(N, 256) * max(K, 256) * 2 < 1 << 31
+            and 256 * N * 2 < 1 << 31)
 
 
 def _tile_unit(x: torch.Tensor, w: torch.Tensor, f: int) -> bool:
-    """Whether a large product with a unit at its end (a gated one of f features, or f 0) goes to the tile GEMM: its tiles take 5 % longer
-    than the BLAS library's, which leaves the unit a launch of its own that reads and writes the products once more.  us, library and
-    launch / tile GEMM: 7830 rows, 2 x 5632 + 2048 columns, K 2048 388 + 47 / 355; 3749 rows 236 + 25 / 195; 6403 x 4096 x 1024 (1.6
-    rounds of tiles) 53 + 18 / 58."""
-    M, (N, K) = x.shape[0], w.shape
+    """Whether ``gemm_tile_unit`` takes these operands, by the rule of ``_tile_form``."""
     return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and w.is_contiguous()
-            and K % 64 == 0 and K >= 192 and N % 16 == 0 and f % 16 == 0 and 2 * f <= N and max(N, 256) * max(K, 256) * 2 < 1 << 31
-            and 256 * N * 2 < 1 << 31 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and _tile_rounds_ok(-(-M // 256) * (-(-f // 128) + -(-(N - 2 * f) // 256))))
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _tile_form(x.shape[0], w.shape[0], w.shape[1], f))
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, kind: str) -> torch.Tensor:
     """``activation(linear(x, w), kind)``, in one launch for the rows that few_rows.hip takes (``relu_sq`` and ``tanh``) and for large
-    steps (``relu_sq``, by the rule of ``_tile_unit``)."""
+    steps (``relu_sq``, by the rule of ``_tile_form``)."""
     if kind == "relu_sq" and _tile_unit(x, w, 0):
         from .. import ops
 
@@ -1232,7 +1234,7 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, kind: str) -> torch.Tensor:
 def linear_glu(x: torch.Tensor, w: torch.Tensor, f: int, kind: str) -> tuple:
     """The gated unit ``act(gate x) * (up x)`` [T, f] of ``w``'s rows [f gate | f up | the rest], and a projection with the column
     at which the rest's outputs begin in it.  ``linear`` and ``glu``, in one launch for the rows that few_rows.hip takes and for large
-    steps (by the rule of ``_tile_unit``)."""
+    steps (by the rule of ``_tile_form``)."""
     if f > 0 and kind in TILE_UNITS and _tile_unit(x, w, f):
         from .. import ops
 
