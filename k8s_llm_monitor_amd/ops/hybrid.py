@@ -1156,28 +1156,51 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
     return out
 
 
-def _rows_form(M: int, N: int, K: int, fused: bool) -> Optional[str]:
-    """Which kernel of few_rows.hip takes a bf16 product of M rows with weights [N, K], ``fused`` where it also saves the launch behind it;
-    None: the BLAS library.  us, library / own / shared, in a graph over weights from memory: 2048 x 2048, 1 row 10.9 / 4.4 / 8.2,
-    64 rows 11.6 / 10.1 / 13.5; 4096 x 4096, 16 rows 15.6 / 9.5 / 17.0, 32 rows 13.2 / 12.6 / 18.7, 48 rows 13.8 / 17.0 / 21.8; 16384 x
-    4096, 1 row 34.0 / 25.4 / 31.6, 16 rows 33.8 / 36.5 / 30.5, 32 rows 33.8 / 44.4 / 31.2, 64 rows 33.5 / 67.3 / 36.4 (a launch behind
-    it takes 4 to 6); 8192 x 1024, 64 rows 11.9 / 10.5 / 9.5; 4096 x 8192, 1 row 16.6 / 17.1 / 27.7."""
-    if M > 64 or K > 6144 or (M > 4 and K > 4096):
+def _rows_form(M: int, N: int, K: int, end: str = "") -> Optional[str]:
+    """Which kernel of few_rows.hip takes a bf16 product of M rows with weights [N, K]; ``end``: what stands behind it and would be a launch
+    of its own, a gated unit of its first rows ("glu") or something elementwise ("act").  None: the BLAS library.  us, library (and launch)
+    / own / shared, in a graph over weights from memory:
+    plain     2048 x 2048, 1 row 8.5 / 3.6 / 6.0, 64 rows 9.2 / 7.8 / 11.5; 4096 x 4096, 16 rows 15.6 / 9.6 / 16.6, 48 rows 13.9 / 17.2 / 21.7;
+              8192 x 4096, 16 rows 17.2 / 19.1 / 19.8 (shared: 128 workgroups); 16384 x 4096, 1 row 34 / 26 / 32, 16 rows 34 / 35 / 30, 64
+              rows 36 / 70 / 37; 24576 x 2048, 32 rows 27 / 36 / 29; 65536 x 1024, 4 rows 28 / 30 / 26; 128256 x 4096, 4 rows 192 / 181 / -, 16
+              rows 191 / - / 205
+    act       8192 x 4096, 64 rows 23 / 38 / 26; 12288 x 4096, 64 rows 30 / 55 / 30; 24576 x 2048, 32 rows 30 / 35 / 28, 64 rows 32 / 52 / 36
+    glu       (a workgroup of either takes half as many columns) 8192 x 2048, 64 rows 17 / 15 / 22; 8192 x 4096, 16 rows 20 / 17 / 33; 16384 x
+              4096, 16 rows 37 / 33 / 39, 32 rows 36 / 39 / 41; 32768 x 4096, 4 rows 66 / 54 / 65, 64 rows 69 / 95 / 72; 10240 x 5632, 1 row 28 / 33 / 52"""
+    if M > 64 or K > 6144 or (N * K > 1 << 28 and (M > 4 or end == "glu")):
         return None
-    if M <= 4 or (M <= 32 and N * K <= 1 << 24 and N < 8192) or (M <= 16 and N * K <= 1 << 24) or (N * K <= 1 << 22 and K <= 2048):
+    if end == "glu":
+        if K > 4096:
+            return None
+        if M <= 4 and N * K <= 1 << 27 and (N < 32768 or K > 1024):
+            return "own"
+        if N >= 24576 and (K <= 2048 or M <= 16 or N >= 32768):
+            return "shared"
+        small = N <= 8192 or (N <= 16384 and K <= 2048)
+        if M <= 8 or (M <= 16 and (N <= 12288 or small)) or (M <= 24 and small) or (K <= 2048 and N * K <= 1 << 24):
+            return "own"
+        return None
+    if K > 4096:
+        return "own" if M <= 2 or (M <= 4 and (end or N <= 4096 or 8192 <= N <= 32768)) else None
+    if M <= 4:
+        return "shared" if N >= 32768 and K <= 1024 else "own"
+    if (M <= 16 and N * K <= 1 << 24) or (M <= 32 and N * K <= 1 << 24 and N < 8192) or (N * K <= 1 << 22 and K <= 2048):
         return "own"
-    if 8192 <= N and (M <= 16 or (M <= 32 and N * K <= 1 << 26) or fused or (K <= 1024 and N <= 16384)):
+    if N < 8192 or (N < 10240 and K > 3072):
+        return None
+    if M <= 16 or (N <= 16384 and (M <= 32 or end or K <= 1024)) or (
+            M <= 32 and ((K <= 1024 and N * K <= 1 << 26) or (end and (K <= 2048 or N >= 32768)))):
         return "shared"
     return None
 
 
-def _few_rows(x: torch.Tensor, w: torch.Tensor, fused: bool = False) -> Optional[str]:
+def _few_rows(x: torch.Tensor, w: torch.Tensor, end: str = "") -> Optional[str]:
     if not (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
             and w.shape[1] % 32 == 0 and w.shape[1] >= 32 and x.shape[0] > 0
             and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
         return None
-    return _rows_form(x.shape[0], w.shape[0], w.shape[1], fused)
+    return _rows_form(x.shape[0], w.shape[0], w.shape[1], end)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -1223,7 +1246,7 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, kind: str) -> torch.Tensor:
         y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
         ops.native().gemm_tile_unit(y, None, x, w, TILE_UNITS[kind])
         return y
-    form = _few_rows(x, w, True) if kind in ("relu_sq", "tanh") else None
+    form = _few_rows(x, w, "act") if kind in ("relu_sq", "tanh") else None
     if form is not None:
         y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
         native().few_rows(y, None, x, w, 16 + ACTS[kind], 0.0, form == "shared")
@@ -1242,7 +1265,7 @@ def linear_glu(x: torch.Tensor, w: torch.Tensor, f: int, kind: str) -> tuple:
         y = torch.empty(x.shape[0], w.shape[0] - 2 * f, dtype=x.dtype, device=x.device)
         ops.native().gemm_tile_unit(a, y, x, w, TILE_UNITS[kind])
         return a, y, 0
-    form = _few_rows(x, w, True) if f > 0 and f % 16 == 0 else None
+    form = _few_rows(x, w, "glu") if f > 0 and f % 16 == 0 else None
     if form is not None:
         a = torch.empty(x.shape[0], f, dtype=x.dtype, device=x.device)
         y = torch.empty(x.shape[0], w.shape[0] - 2 * f, dtype=x.dtype, device=x.device)
@@ -1255,7 +1278,7 @@ def linear_glu(x: torch.Tensor, w: torch.Tensor, f: int, kind: str) -> tuple:
 def logits(x: torch.Tensor, w: torch.Tensor, scale: float = 1.0, cap: float = 0.0) -> torch.Tensor:
     """fp32 ``scale * (x w^T)`` of the product rounded to x's dtype, through ``cap * tanh(. / cap)`` if cap > 0.  In one launch for the
     few rows of a decode step (no scale)."""
-    form = _few_rows(x, w) if scale == 1.0 else None
+    form = _few_rows(x, w, "act") if scale == 1.0 else None
     if form is not None:
         z = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
         native().few_rows(z, None, x, w, -1, float(cap), form == "shared")

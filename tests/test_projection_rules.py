@@ -13,3 +13,16 @@ from k8s_llm_monitor_amd.ops import hybrid as hops
 ])
 def test_tile_gemm_with_a_unit(M, N, K, f, takes):
     assert hops._tile_form(M, N, K, f) is takes
+
+
+@pytest.mark.parametrize("end,M,N,K,form", [
+    ("glu", 16, 8192, 4096, "own"), ("glu", 33, 8192, 4096, None), ("glu", 64, 8192, 2048, "own"), ("glu", 32, 13312, 2048, None),
+    ("glu", 64, 16384, 4096, None), ("glu", 4, 32768, 4096, "own"), ("glu", 16, 32768, 4096, "shared"), ("glu", 1, 10240, 5632, None),
+    ("", 16, 8192, 4096, None), ("", 16, 10240, 4096, "shared"), ("", 4, 8192, 4096, "own"), ("", 16, 2048, 2048, "own"),
+    ("", 64, 2048, 2048, "own"), ("", 64, 4096, 4096, None), ("", 4, 65536, 1024, "shared"), ("", 1, 128256, 4096, "own"),
+    ("", 16, 128256, 4096, None), ("", 3, 6144, 6144, None), ("", 4, 4096, 6144, "own"), ("", 1, 2048, 6176, None),
+    ("act", 64, 8192, 4096, None), ("act", 64, 12288, 4096, "shared"), ("act", 64, 24576, 2048, None), ("act", 32, 24576, 2048, "shared"),
+    ("act", 65, 2048, 2048, None),
+])
+def test_projections_of_few_rows(end, M, N, K, form):
+    assert hops._rows_form(M, N, K, end) == form
