@@ -1216,6 +1216,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 TILE_UNITS = {"gelu_tanh": 5, "silu": 6, "relu": 7, "relu_sq": 8}  # epilogues of ops.gemm_tile_unit
+GLU_ENDS = ("gelu_tanh", "silu", "relu")  # gated units that the projections' kernels have at their end; ``glu`` has others
 
 
 def _tile_form(M: int, N: int, K: int, f: int) -> bool:
@@ -1258,14 +1259,14 @@ def linear_glu(x: torch.Tensor, w: torch.Tensor, f: int, kind: str) -> tuple:
     """The gated unit ``act(gate x) * (up x)`` [T, f] of ``w``'s rows [f gate | f up | the rest], and a projection with the column
     at which the rest's outputs begin in it.  ``linear`` and ``glu``, in one launch for the rows that few_rows.hip takes and for large
     steps (by the rule of ``_tile_form``)."""
-    if f > 0 and kind in TILE_UNITS and _tile_unit(x, w, f):
+    if f > 0 and kind in GLU_ENDS and _tile_unit(x, w, f):
         from .. import ops
 
         a = torch.empty(x.shape[0], f, dtype=x.dtype, device=x.device)
         y = torch.empty(x.shape[0], w.shape[0] - 2 * f, dtype=x.dtype, device=x.device)
         ops.native().gemm_tile_unit(a, y, x, w, TILE_UNITS[kind])
         return a, y, 0
-    form = _few_rows(x, w, "glu") if f > 0 and f % 16 == 0 else None
+    form = _few_rows(x, w, "glu") if f > 0 and f % 16 == 0 and kind in GLU_ENDS else None
     if form is not None:
         a = torch.empty(x.shape[0], f, dtype=x.dtype, device=x.device)
         y = torch.empty(x.shape[0], w.shape[0] - 2 * f, dtype=x.dtype, device=x.device)

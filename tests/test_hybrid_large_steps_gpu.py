@@ -567,6 +567,17 @@ def test_squared_relu_in_the_tile_gemm(M, N, K):
     assert bool(((y.double() - z ** 2).abs() <= 3 * 2 ** -8 * z ** 2 + 1e-5).all())  # twice the rounding of z, once that of its square
 
 
+@pytest.mark.parametrize("M", [1, 17, 40, 65, 512])
+def test_gated_units_that_no_projection_ends_with(M):
+    """What is no gated unit of ``glu`` is refused as ``glu`` refuses it, whatever kernel the step's size would choose."""
+    g = _g(93)
+    f = 96 if M < 512 else 12800  # 512 rows: 200 tiles
+    x, w = _r(g, M, 192, dt=BF).cuda(), _r(g, 2 * f, 192, s=192 ** -0.5, dt=BF).cuda()
+    for kind in ("clamped_swish", "relu_sq", "tanh"):
+        with pytest.raises(RuntimeError, match="glu: columns / kind"):
+            hops.linear_glu(x, w, f, kind)
+
+
 def test_linear_of_nothing():
     """Empty sums, no columns, no rows and no gated unit are what the library makes of them."""
     g = _g(89)
