@@ -925,14 +925,16 @@ def moe_grouped_gemm(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, sw
     the per-16 gate/up pairing) always takes the tile kernel.  ``rows`` int32: ``x`` holds the rows in their own order,
     and sorted row r is its row rows[r] / div (gather_rows); the tile kernel reads them from there."""
     if rows is not None:
+        x = x.contiguous()
+        # the tile kernel's copies to LDS take 16 aligned bytes a lane; the sorted copy is aligned whatever x is
         if not (_gpu(x) and w.dim() == 3 and w.shape[1] % 256 == 0 and w.shape[2] % 64 == 0 and w.shape[1] * w.shape[2] < 1 << 30
-                and x.numel() < 1 << 30):
+                and x.numel() < 1 << 30 and x.data_ptr() % 16 == 0):
             x = gather_rows(x, rows, div)
         else:
             if out is None:
                 alloc = torch.zeros if zero_fill else torch.empty
                 out = alloc(rows.numel(), w.shape[1] // 2 if swiglu else w.shape[1], dtype=x.dtype, device=x.device)
-            native().gemm_tile_rows(out, x.contiguous(), w, offsets.contiguous(), rows, div, bool(swiglu), TILE_ALGO)
+            native().gemm_tile_rows(out, x, w, offsets.contiguous(), rows, div, bool(swiglu), TILE_ALGO)
             return out
     if w.dim() == 5:
         if out is None:

@@ -514,6 +514,7 @@ void gemm_tile_rows(torch::Tensor y, torch::Tensor x, torch::Tensor w, torch::Te
   TORCH_CHECK(div >= 1 && M <= x.size(0) * div, "gemm_tile_rows: at most div sorted rows for each of x");
   TORCH_CHECK(N % 16 == 0 && K % 64 == 0 && K >= 64 && (!swiglu || N % 256 == 0), "gemm_tile_rows: N % 16 == 0 (SwiGLU: % 256), K % 64 == 0");
   TORCH_CHECK(y.dim() == 2 && y.size(0) == M && y.size(1) == (swiglu ? N / 2 : N), "gemm_tile_rows: y shape");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "gemm_tile_rows: alignment of x");
   check(k8sllm_gemm_tile(x.data_ptr(), w.data_ptr(), y.data_ptr(), (int)M, N, K, offsets.data_ptr<int>(), E, (long)N * K, swiglu ? 1 : 0,
                          (int)algo, nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, 0, rows.data_ptr<int>(),
                          (int)div, x.size(0), cur()),

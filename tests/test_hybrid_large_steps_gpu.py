@@ -894,3 +894,20 @@ def test_grouped_tiles_sort_their_rows_as_they_read(T, K, E, d, swiglu):
     assert torch.equal(ops.moe_grouped_gemm(x, w, off, swiglu=swiglu, rows=idx, div=K), want)
     cpu = ops.moe_grouped_gemm(x.cpu(), w.cpu(), off.cpu(), swiglu=swiglu, rows=idx.cpu(), div=K)
     torch.testing.assert_close(want.cpu().float(), cpu.float(), rtol=2e-2, atol=2e-2 * float(cpu.float().abs().max()))
+
+
+@pytest.mark.parametrize("at", [1, 4, 8])
+def test_grouped_tiles_of_rows_at_any_address(at):
+    """Rows in their own order that do not start on 16 bytes (the first two) are sorted by a copy: the bits of an aligned clone.  The tile
+    kernel itself refuses them."""
+    from k8s_llm_monitor_amd import ops
+
+    g = _g(94)
+    T, K, E, d = 300, 2, 3, 192
+    off, idx, _ = ops.moe_align(torch.randint(0, E, (T, K), generator=g, dtype=torch.int32).cuda(), E)
+    x, w = _r(g, T * d + at, dt=BF).cuda()[at:].view(T, d), _r(g, E, 256, d, s=0.1, dt=BF).cuda()
+    want = ops.moe_grouped_gemm(x.clone(), w, off, rows=idx, div=K)
+    assert torch.equal(ops.moe_grouped_gemm(x, w, off, rows=idx, div=K), want)
+    if at != 8:
+        with pytest.raises(RuntimeError, match="alignment"):
+            ops.native().gemm_tile_rows(want, x, w, off, idx, K, False, 0)
