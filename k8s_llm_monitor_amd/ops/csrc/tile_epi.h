@@ -51,12 +51,13 @@ struct TileEpi {
 
 __host__ __device__ constexpr bool tile_epi_glu(int epi) { return epi >= TILE_EPI_GELU_GLU && epi <= TILE_EPI_RELU_GLU; }
 
-// The gated units.  tanh GELU as z / (1 + exp(-2 t)): the same function without the cancellation of 1 + tanh t.
+// The gated units, act(gate) before it meets up, which with a gate far below zero may be too large for their product.  tanh GELU as
+// z / (1 + exp(-2 t)): the same function without the cancellation of 1 + tanh t.
 template <int EPI>
 __device__ __forceinline__ float tile_unit(float g, float u) {
   if (EPI == TILE_EPI_RELU_GLU) return fmaxf(g, 0.f) * u;
   const float t = EPI == TILE_EPI_GELU_GLU ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
-  return g * u / (1.f + __expf(-t));
+  return g / (1.f + __expf(-t)) * u;
 }
 
 // sum over the 16 lanes of a DPP row (lanes 16r .. 16r + 15), the total in every lane

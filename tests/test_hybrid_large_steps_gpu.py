@@ -555,6 +555,25 @@ def test_gated_unit_in_the_tile_gemm(M, f, rest, K, kind):
     assert bool(((y.double() - z[:, 2 * f:]).abs() <= 2 ** -8 * z[:, 2 * f:].abs() + 1e-6 * K ** 0.5).all())
 
 
+@pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
+def test_tile_gemm_units_of_large_factors(kind):
+    """Gates far below zero beside ups whose product with them has no fp32, large gates, infinities and NaN: what the unit's own launch
+    makes of the same products (one nonzero term each, exact), to the rounding of the result."""
+    from k8s_llm_monitor_amd import ops
+
+    f, K, inf, nan = 16, 192, float("inf"), float("nan")
+    gate = torch.tensor([-1e20, -3e38, -100.0, -1e20, 1e20, 3e38, 0.0, -0.0, inf, -inf, nan, 2.0, -1e20, 50.0, -50.0, 1.0])
+    up = torch.tensor([1e20, 1e10, 1e38, -3e38, 1e10, 0.5, inf, 3e38, 2.0, 2.0, 1.0, nan, inf, -3e38, 3e38, 0.0])
+    w = torch.zeros(2 * f, K)
+    w[:, 0] = torch.cat([gate, up])
+    w, x = w.to(BF).cuda(), torch.zeros(3, K, dtype=BF, device="cuda")
+    x[:, 0] = 1.0
+    a, y = torch.empty(3, f, dtype=BF, device="cuda"), torch.empty(3, 0, dtype=BF, device="cuda")
+    ops.native().gemm_tile_unit(a, y, x, w, hops.TILE_UNITS[kind])
+    want = hops.glu((x.double() @ w.double().t()).to(BF), 0, f, kind)
+    torch.testing.assert_close(a, want, rtol=2 ** -7, atol=1e-30, equal_nan=True)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 192), (300, 272, 256), (256, 512, 320)])
 def test_squared_relu_in_the_tile_gemm(M, N, K):
     from k8s_llm_monitor_amd import ops
