@@ -1033,8 +1033,11 @@ int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const voi
   if (keep < 0 || (keep > 0 && (chunked || window <= 0))) return -1;
   if (dk > kGenDK || dv > 64 * kGenVC || G < 1 || Hq % G) return -1;
   const int R = Hq / G;
-  if (!f32 && vec && bs == 16 && dk % 8 == 0 && q_stride % 8 == 0 && dk <= kMaxDK && dv <= 64 * kMaxVC &&
-      (R == 1 || R == 2 || R == 4 || R == 8)) {
+  const bool lanes = !f32 && vec && bs == 16 && dk % 8 == 0 && q_stride % 8 == 0 && dk <= kMaxDK && dv <= 64 * kMaxVC &&
+                     (R == 1 || R == 2 || R == 4 || R == 8);
+  const bool rows = lanes && (dk == 64 || dk == 128) && (dv == 64 || dv == 128);
+  if (heads != 0 && (!rows || heads < 1 || R % heads || (R == 8 && heads == 4))) return -1;
+  if (lanes) {
 #define K8SLLM_WDR(RR, NW, DKC, VC)                                                                                    \
   hipLaunchKernelGGL((window_decode_row_kernel<RR, NW, DKC, VC>), dim3(B, Hq / RR), dim3(64 * NW), 0, s, (bf16_t*)out,   \
                      (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, \
@@ -1046,9 +1049,8 @@ int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const voi
   else if (heads == 4) K8SLLM_WDR(4, 8, DKC, VC);           \
   else if (heads == 2) K8SLLM_WDR(2, 8, DKC, VC);           \
   else K8SLLM_WDR(1, 8, DKC, VC)
-    if (heads == 0) heads = decode_heads(B, Hq, R);
-    if (heads < 1 || R % heads || (R == 8 && heads == 4)) return -1;
-    if ((dk == 64 || dk == 128) && (dv == 64 || dv == 128)) {
+    if (rows) {
+      if (heads == 0) heads = decode_heads(B, Hq, R);
       if (dk == 64 && dv == 64) { K8SLLM_WDD(1, 1); }
       else if (dk == 64) { K8SLLM_WDD(1, 2); }
       else if (dv == 64) { K8SLLM_WDD(2, 1); }

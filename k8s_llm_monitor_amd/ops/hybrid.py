@@ -557,7 +557,7 @@ def window_attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     cached positions (``chunked``: those of its own chunk; ``cap``, ``keep``, ``gate``: as in
     window_attention_prefill);
     ``seq_lens`` count that token (0: a padding row, output zero).  ``heads``: query heads of a kv
-    head that a workgroup takes (``vec``, head sizes of 64 and 128; 0: its choice)."""
+    head that a workgroup takes (GPU, ``vec``, bf16, head sizes of 64 and 128; 0: its choice, others are refused elsewhere)."""
     B = qkv.shape[0]
     if not qkv.is_cuda:
         out = torch.zeros(B, Hq * dv, dtype=qkv.dtype)

@@ -728,6 +728,19 @@ def test_window_decode_heads(Hq, G, dk, dv, window):
         hops.window_attention_decode(*dev, *a, heads=3)
 
 
+@pytest.mark.parametrize("Hq,G,dk,dv,vec,dt", [(8, 2, 96, 128, True, BF), (8, 2, 128, 96, True, BF), (8, 2, 128, 128, False, BF), (6, 2, 64, 64, True, BF),
+                                               (8, 2, 128, 128, True, torch.float32)])
+def test_window_decode_heads_elsewhere(Hq, G, dk, dv, vec, dt):
+    """A forced number of query heads raises where the kernels that take one do not apply; without one the call runs."""
+    g = _g(83)
+    lens = [1, 40]
+    kc, vc, bt = _paged(g, dt, lens, Hq, G, dk, dv, nb=8)
+    a = [t.cuda() for t in (_r(g, 2, Hq * dk, dt=dt), kc, vc, bt, _i32(lens))] + [Hq, G, dk, dv, 1.0 / math.sqrt(dk), 0, True]
+    assert bool(hops.window_attention_decode(*a, vec=vec).isfinite().all())
+    with pytest.raises(RuntimeError):
+        hops.window_attention_decode(*a, vec=vec, heads=1)
+
+
 @pytest.mark.parametrize("Hq,G,dk,dv", [(1, 1, 1, 1), (2, 1, 128, 64), (16, 4, 128, 128), (17, 1, 128, 8), (32, 8, 128, 16), (33, 3, 128, 8)])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
 def test_qk_norm_sizes(Hq, G, dk, dv, dt):
