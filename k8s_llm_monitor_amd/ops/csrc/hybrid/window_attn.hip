@@ -452,16 +452,18 @@ inline int decode_heads(long B, int Hq, int R) {
 
 // The same for head sizes of 64 and 128, without the LDS reads that bound it (a tile of 64 keys took a wave 256 16-byte reads of
 // queries and weights that all lanes share): each 16-lane row holds all dims of the queries, 16 to a register, and a page's 16
-// weights in one, and the multiply-adds pick the element by their DPP row broadcast.  Keys and values of a tile are in flight
-// together.  Sums in the same order: the same bits.
-// 64 sequences, 1024 visible keys, 16 heads on 4 of 128: 40.8 -> 34.3 us (3.9 TB/s); 24 of ~1200, 32 on 8: 28.1 -> 25.5; 5 of 700, 8
-// heads on one of 128 / 64: 37 -> 27.
+// weights in one, and the multiply-adds pick the element by their DPP row broadcast.  Sums in the same order: the same bits.
 // A tile's keys come to LDS by whole rows, 16 lanes a row, and the next tile's while this one is multiplied; a lane then reads its own.
 // Loads of a row a lane met 64 rows at a time, which is 64 cycles of the load path each, and a page's values, loaded behind a
-// branch, waited for the page before.  The same bits.  us, at decode_heads' choice: 1 sequence of 333 keys, 8 heads on 2 9.7 -> 6.6; of
-// 8000, 16 on 4 131 -> 74; 24 of 1500 36.0 -> 27.5; 64 of 1024 41.5 -> 35.0; 16 of 1500, 8 heads on one 38.6 -> 25.5.
-template <int R, int NW, int DKC, int VC>
-__global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv,
+// branch, waited for the page before.  The same bits.  us over pages from memory, keys by a row a lane and all heads a workgroup / now at
+// decode_heads' choice, heads of 128: 1 sequence of 333 keys, 8 heads on 2 13.7 / 6.6; of 4000, 16 on 4 84 / 36; 24 of 1500 45 / 28; 64 of 1000
+// 39 / 34 (3.9 TB/s); 256 of 300 66 / 52; 64 of 1000, 16 heads on 2 55 / 45.
+// A page's address is the wave's own, in scalar registers, and a lane adds one of a few offsets: an address a lane took up to 44 vector registers.
+// PER_CU: heads of 64, four a workgroup, in 128 registers (4 of 165 spilled), so that two share a compute unit once there is more than
+// one for each.  us, before the keys came through LDS / 165 registers / this, 32 heads on 8: 256 sequences of 64 keys 31 / 36 / 25, of 300 50 / 56 /
+// 44, of 1000 118 / 117 / 116; 16 on 4, 64 of 1000, one workgroup each, 23.0 / 18.9 / 20.0.
+template <int R, int NW, int DKC, int VC, int PER_CU = 1>
+__global__ __launch_bounds__(64 * NW, PER_CU * NW / 4) void window_decode_row_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv,
                                                                 long q_stride, const bf16_t* __restrict__ k_cache,
                                                                 const bf16_t* __restrict__ v_cache,
                                                                 const int* __restrict__ block_tables, int bt_stride,
@@ -487,20 +489,21 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
   // the tiles that hold kept keys (kt of them, from position 0), then the window's from w0 on
   const int kf = min(keep, n), kt = (kf + 63) >> 6, w0 = max(kt, lo >> 6);
   auto tile = [&](int it) { return 64 * (it < kt ? it : w0 + it - kt); };
-  // keys j0 .. j0 + 63 to LDS, a row's 16-byte chunks turned by the row; pages without a key to be seen: the newest one's instead
-  constexpr int LPK = dk / 8, RPI = 64 / LPK;
+  // keys j0 .. j0 + 63 to LDS, a row's 16-byte chunks turned by the row; pages without a key to be seen: the newest one's instead.
+  // A page's address is the wave's, a lane adds one of PER offsets.
+  constexpr int LPK = dk / 8, RPI = 64 / LPK, PER = bs / RPI;
   auto turn = [](int r) { return DKC == 2 ? r & 15 : (r >> 1) & 7; };
+  uint32_t koff[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) koff[i] = 2 * (uint32_t)((i * RPI + lane / LPK) * (int)krs + 8 * ((lane % LPK) ^ turn(i * RPI + lane / LPK)));
   auto stage = [&](int j0) {
-    long page[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const int f = j0 + 16 * p;
-      page[p] = (long)bt[((f < n) & ((f + 15 >= lo) | (f < keep)) ? f : n - 1) / bs] * bs;
-    }
+      const long page = (long)bt[((f < n) & ((f + 15 >= lo) | (f < keep)) ? f : n - 1) / bs] * bs;
+      const char* base = reinterpret_cast<const char*>(k_cache + page * krs + (long)g * dk);
 #pragma unroll
-    for (int i = 0; i < LPK; ++i) {
-      const int r = i * RPI + lane / LPK;
-      load_piece(k_s[wave] + 1024 * i, k_cache + (page[i * RPI / bs] + r % bs) * krs + (long)g * dk + 8 * ((lane % LPK) ^ turn(r)));
+      for (int i = 0; i < PER; ++i) load_piece(k_s[wave] + 1024 * (PER * p + i), reinterpret_cast<const bf16_t*>(base + koff[i]));
     }
   };
   int it = wave, j0 = tile(it);
@@ -541,11 +544,11 @@ __global__ __launch_bounds__(64 * NW) void window_decode_row_kernel(bf16_t* __re
     uint4 vq[4][VC][2], kr[8 * DKC];
 #pragma unroll
     for (int pg = 0; pg < 4; ++pg) {
-      const long base = ((long)bt[j0 / bs + min(pg, npg - 1)] * G + g) * dv;
+      const long base = values + 2 * bs * (((long)bt[j0 / bs + min(pg, npg - 1)] * G + g) * dv);
 #pragma unroll
       for (int c = 0; c < VC; ++c) {
         using Raw = unsigned __attribute__((ext_vector_type(4)));
-        const auto vp = reinterpret_cast<__attribute__((address_space(1))) const Raw*>(values + 2 * (base + lane + 64 * c) * bs);
+        const auto vp = reinterpret_cast<__attribute__((address_space(1))) const Raw*>(base + 2 * bs * 64 * c + (long)(2 * bs * (uint32_t)lane));
         vq[pg][c][0] = __builtin_bit_cast(uint4, Raw(vp[0]));
         vq[pg][c][1] = __builtin_bit_cast(uint4, Raw(vp[1]));
       }
@@ -1038,14 +1041,15 @@ int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const voi
   const bool rows = lanes && (dk == 64 || dk == 128) && (dv == 64 || dv == 128);
   if (heads != 0 && (!rows || heads < 1 || R % heads || (R == 8 && heads == 4))) return -1;
   if (lanes) {
-#define K8SLLM_WDR(RR, NW, DKC, VC)                                                                                    \
-  hipLaunchKernelGGL((window_decode_row_kernel<RR, NW, DKC, VC>), dim3(B, Hq / RR), dim3(64 * NW), 0, s, (bf16_t*)out,   \
+#define K8SLLM_WDR(RR, NW, ...)                                                                                        \
+  hipLaunchKernelGGL((window_decode_row_kernel<RR, NW, __VA_ARGS__>), dim3(B, Hq / RR), dim3(64 * NW), 0, s, (bf16_t*)out, \
                      (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, \
                      seq_lens, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
 #define K8SLLM_WDD(DKC, VC)                                 \
   if (R == 8 && heads == 8) K8SLLM_WDR(8, 4, DKC, VC);      \
   else if (R == 8 && heads == 2) K8SLLM_WDR(2, 4, DKC, VC); \
   else if (R == 8) K8SLLM_WDR(1, 4, DKC, VC);               \
+  else if (heads == 4 && DKC + VC == 2 && (long)B * Hq > 4 * 256) K8SLLM_WDR(4, 8, DKC, VC, (DKC + VC == 2 ? 2 : 1)); \
   else if (heads == 4) K8SLLM_WDR(4, 8, DKC, VC);           \
   else if (heads == 2) K8SLLM_WDR(2, 8, DKC, VC);           \
   else K8SLLM_WDR(1, 8, DKC, VC)

@@ -728,6 +728,25 @@ def test_window_decode_heads(Hq, G, dk, dv, window):
         hops.window_attention_decode(*dev, *a, heads=3)
 
 
+@pytest.mark.parametrize("B", [256, 257])  # one workgroup for each compute unit, and more
+@pytest.mark.parametrize("window", [0, 50])
+def test_window_decode_two_workgroups_a_unit(B, window):
+    """Heads of 64, four a workgroup: the form that leaves room for two gives the bits of two heads a workgroup, and the torch form's values
+    within the rounding of the bf16 weights and result."""
+    g = _g(95)
+    lens = [int(n) for n in torch.randint(1, 300, (B,), generator=g)]
+    lens[:4] = [1, 64, 65, 0]
+    kc, vc = _r(g, 40, 16, 64, dt=BF), _r(g, 40, 1, 64, 16, dt=BF)
+    bt = torch.randint(0, 40, (B, 19), generator=g, dtype=torch.int32)
+    q = _r(g, B, 4 * 64, dt=BF)
+    a = (4, 1, 64, 64, 0.125, window, True)
+    dev = [t.cuda() for t in (q, kc, vc, bt, _i32(lens))]
+    got = hops.window_attention_decode(*dev, *a)
+    assert torch.equal(got, hops.window_attention_decode(*dev, *a, heads=2)) and torch.equal(got, hops.window_attention_decode(*dev, *a, heads=4))
+    want = hops.window_attention_decode(q, kc, vc, bt, _i32(lens), *a)
+    torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1e-2, atol=2e-3)
+
+
 @pytest.mark.parametrize("Hq,G,dk,dv,vec,dt", [(8, 2, 96, 128, True, BF), (8, 2, 128, 96, True, BF), (8, 2, 128, 128, False, BF), (6, 2, 64, 64, True, BF),
                                                (8, 2, 128, 128, True, torch.float32)])
 def test_window_decode_heads_elsewhere(Hq, G, dk, dv, vec, dt):
