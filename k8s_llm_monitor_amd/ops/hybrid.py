@@ -1195,6 +1195,8 @@ def _rows_form(M: int, N: int, K: int, end: str = "") -> Optional[str]:
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, end: str = "") -> Optional[str]:
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):  # the library's product has a backward
+        return None
     if not (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
             and w.shape[1] % 32 == 0 and w.shape[1] >= 32 and x.shape[0] > 0
             and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0

@@ -586,6 +586,20 @@ def test_squared_relu_in_the_tile_gemm(M, N, K):
     assert bool(((y.double() - z ** 2).abs() <= 3 * 2 ** -8 * z ** 2 + 1e-5).all())  # twice the rounding of z, once that of its square
 
 
+@pytest.mark.parametrize("M", [4, 17, 64])
+def test_gradients_of_few_rows_products(M):
+    """A product or logits that a backward is wanted of stay the library's, which has one: gradients of a sum against the operands."""
+    g = _g(96)
+    x, w = _r(g, M, 64, dt=BF).cuda(), _r(g, 48, 64, dt=BF).cuda()
+    for f in (hops.linear, hops.logits):
+        xg, wg = x.clone().requires_grad_(), w.clone().requires_grad_()
+        f(xg, wg).float().sum().backward()
+        torch.testing.assert_close(xg.grad.float(), w.float().sum(0).expand(M, 64), rtol=1e-2, atol=1e-2)
+        torch.testing.assert_close(wg.grad.float(), x.float().sum(0).expand(48, 64), rtol=1e-2, atol=1e-2)
+        with torch.no_grad():
+            assert not f(xg, wg).requires_grad
+
+
 @pytest.mark.parametrize("M", [1, 17, 40, 65, 512])
 def test_gated_units_that_no_projection_ends_with(M):
     """What is no gated unit of ``glu`` is refused as ``glu`` refuses it, whatever kernel the step's size would choose."""
