@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void group_norm_gate_vec_kernel(T* __restrict_
   if constexpr (LPG >= 32) ss = xor16_sum(ss);
   const float inv = 1.0f / sqrtf(ss / (float)(8 * LPG) + eps);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) v[k] *= inv * wv[k] * (after == 2 ? silu_f(g[k]) : sigmoid_f(g[k]));
+  for (int k = 0; k < 8; ++k) v[k] = v[k] * inv * wv[k] * (after == 2 ? silu_f(g[k]) : sigmoid_f(g[k]));  // the norm first: it is of order one
   if (me < chunks) store8(out + 8L * me, v);
 }
 

@@ -694,6 +694,19 @@ def test_head_norm_sizes(rows, groups, gs, col, gate, dt):
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=2 ** -7 if dt == BF else 1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("gs", [64, 128, 256])
+@pytest.mark.parametrize("gate", ["silu", "sigmoid"])
+def test_head_norm_of_large_values_and_small_gates(gs, gate):
+    """Values of 1e18 with gates of e^-80: the norm, of order one, meets the gate, and nothing underflows on the way.  fp32 inside: 1e-5 of
+    the value, and e^-80 to its own 80 2^-24."""
+    g = _g(87)
+    y, z, w = _r(g, 3, 2 * gs, s=1e18), torch.full((3, 2 * gs), -80.0), _r(g, 2 * gs)
+    want = hops.gated_group_norm(y.double(), z.double(), 0, w.double(), 1e-5, 2, torch.float64, after=True, gate=gate)
+    got = hops.gated_group_norm(y.cuda(), z.cuda(), 0, w.cuda(), 1e-5, 2, torch.float32, after=True, gate=gate)
+    assert float(got.abs().max()) > 1e-35
+    torch.testing.assert_close(got.cpu().double(), want, rtol=2e-5, atol=1e-41)
+
+
 @pytest.mark.parametrize("T,d,E,K,shared", [(1000, 2048, 8, 2, False), (1003, 8, 3, 1, True), (4100, 1000, 7, 7, True), (2049, 2056, 8, 8, False),
                                             (2050, 4096, 5, 2, True)])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
