@@ -573,7 +573,7 @@ __global__ __launch_bounds__(64 * NW) void hy_grouped_gemm_mfma_kernel(bf16_t* _
   constexpr int NS = GATED ? 2 : 1;
   using S = SharedRows<MT, NS, NW>;
   __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
-  int e = 0, tile = blockIdx.y, r0 = 0, r1 = 0;
+  int e = 0, tile = blockIdx.y + blockIdx.z * gridDim.y, r0 = 0, r1 = 0;
   for (; e < E; ++e) {
     r0 = offsets[e];
     r1 = offsets[e + 1];
@@ -733,7 +733,8 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
     const bool gated = act == 1 || act == 3;
     const int mt = rows <= 8l * E ? 1 : rows <= 24l * E ? 2 : 4;
     const int nw = mt == 4 || (!gated && std::min<long>(rows, E) * ((N + 63) / 64) >= 256) ? 4 : 2;
-    const dim3 g((unsigned)((N + 16 * nw - 1) / (16 * nw)), (unsigned)(rows / (16 * mt) + E));
+    const unsigned tiles = (unsigned)(rows / (16 * mt) + E), gz = (tiles + 65534) / 65535;  // (a grid's y ends at 65535)
+    const dim3 g((unsigned)((N + 16 * nw - 1) / (16 * nw)), (tiles + gz - 1) / gz, gz);
 #define K8SLLM_GM(ACT, MT, NW)                                                                                       \
   hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<ACT, MT, NW>), g, dim3(64 * NW), 0, s, (bf16_t*)Y, (const bf16_t*)A,  \
                      (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)

@@ -622,6 +622,20 @@ def test_linear_of_nothing():
     assert a.shape == (2, 0) and torch.equal(y[:, col:], hops.linear(x, w))
 
 
+def test_experts_of_very_many_rows():
+    """More row tiles than a grid's second dimension holds (65535 of 64 rows): the bits of the same rows in smaller calls."""
+    g, rows, K, N = _g(97), 64 * 65600, 32, 32
+    a, w = _r(g, 4096, K, dt=BF).cuda(), _r(g, 2, N, K, dt=BF).cuda()
+    idx = torch.randint(0, 4096, (rows,), generator=g, dtype=torch.int32).cuda()
+    a = a[idx.long()]
+    y, few = torch.empty(rows, N, dtype=BF, device="cuda"), torch.empty(1000, N, dtype=BF, device="cuda")
+    off = [0, rows - 1000, rows]
+    hops.native().grouped_gemm(y, a, w, _i32(off).cuda(), None, 1, 0, False, True, 0.0)
+    for e, i in ((0, 0), (0, rows // 2), (0, rows - 2000), (1, rows - 1000)):
+        hops.native().grouped_gemm(few, a[i:i + 1000].contiguous(), w[e:e + 1].contiguous(), _i32([0, 1000]).cuda(), None, 1, 0, False, True, 0.0)
+        assert torch.equal(y[i:i + 1000], few)
+
+
 @pytest.mark.parametrize("rows", [1, 40, 700])
 @pytest.mark.parametrize("act", [0, 1, 3, 4])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
