@@ -61,15 +61,8 @@ __global__ __launch_bounds__(256, 3) void experts_f32_kernel(ExpertsF32 g) {
   static_assert(!GATED || NB == 2, "");
   constexpr int PLANE = (1 + NB) * 64 * 64, TK = 32;  // bytes of one part: the rows' 64, then the weights' 64 NB, of 64 bytes each
   __shared__ __attribute__((aligned(1024))) char buf[3 * PLANE];
-  int e = 0, tile = blockIdx.y, r0 = 0, r1 = 0;
-  for (; e < g.E; ++e) {
-    r0 = g.offsets[e];
-    r1 = g.offsets[e + 1];
-    const int nt = (r1 - r0 + 63) / 64;
-    if (tile < nt) break;
-    tile -= nt;
-  }
-  if (e >= g.E) return;
+  int e, tile = blockIdx.y, r0, r1;
+  if (!expert_tile<64>(g.offsets, g.E, tile, e, r0, r1)) return;
   r0 += tile * 64;
   const int n0 = blockIdx.x * (GATED ? 64 : 64 * NB);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, quad = lane >> 4, wm = wave & 1, wn = wave >> 1;

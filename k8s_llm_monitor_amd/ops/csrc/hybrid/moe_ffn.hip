@@ -573,15 +573,8 @@ __global__ __launch_bounds__(64 * NW) void hy_grouped_gemm_mfma_kernel(bf16_t* _
   constexpr int NS = GATED ? 2 : 1;
   using S = SharedRows<MT, NS, NW>;
   __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
-  int e = 0, tile = blockIdx.y + blockIdx.z * gridDim.y, r0 = 0, r1 = 0;
-  for (; e < E; ++e) {
-    r0 = offsets[e];
-    r1 = offsets[e + 1];
-    const int nt = (r1 - r0 + 16 * MT - 1) / (16 * MT);
-    if (tile < nt) break;
-    tile -= nt;
-  }
-  if (e >= E) return;
+  int e, tile = blockIdx.y + blockIdx.z * gridDim.y, r0, r1;
+  if (!expert_tile<16 * MT>(offsets, E, tile, e, r0, r1)) return;
   r0 += tile * (16 * MT);
   const int n0 = (blockIdx.x * NW + (threadIdx.x >> 6)) * 16, nw = min(n0 + piece_row(), N - 1);
   const bf16_t* We = W + (long)e * w_es + piece_k();

@@ -622,6 +622,24 @@ def test_linear_of_nothing():
     assert a.shape == (2, 0) and torch.equal(y[:, col:], hops.linear(x, w))
 
 
+@pytest.mark.parametrize("E", [64, 65, 128, 129, 200])  # one after another; 64 at a time, whole and broken
+@pytest.mark.parametrize("rows", [1, 70, 700, 4000])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_experts_by_their_number(E, rows, dt):
+    """Every row tile finds its expert, with none, one and many rows in the others, the last and the first: against the rows' own products in
+    64 bits, to the rounding of the result (bf16) or 2e-7 of sums of 32 products of order one (1e-5)."""
+    g = _g(98)
+    a, w = _r(g, rows, 32, dt=dt), _r(g, E, 16, 32, dt=dt)
+    for pick in (torch.randint(0, E, (rows,), generator=g), torch.full((rows,), E - 1), torch.zeros(rows, dtype=torch.int64),
+                 torch.where(torch.rand(rows, generator=g) < 0.9, E // 2, torch.randint(0, E, (rows,), generator=g))):
+        e = pick.sort().values
+        off = torch.cat([torch.zeros(1, dtype=torch.int64), torch.bincount(e, minlength=E).cumsum(0)]).int()
+        y = torch.full((rows, 16), float("nan"), dtype=dt, device="cuda")
+        hops.native().grouped_gemm(y, a.cuda(), w.cuda(), off.cuda(), None, 1, 0, False, True, 0.0)
+        want = torch.einsum("rk,rnk->rn", a.double(), w.double()[e])
+        torch.testing.assert_close(y.cpu().double(), want, rtol=2 ** -8, atol=1e-5) if dt == BF else torch.testing.assert_close(y.cpu().double(), want, rtol=0, atol=1e-5)
+
+
 def test_experts_of_very_many_rows():
     """More row tiles than a grid's second dimension holds (65535 of 64 rows): the bits of the same rows in smaller calls."""
     g, rows, K, N = _g(97), 64 * 65600, 32, 32
