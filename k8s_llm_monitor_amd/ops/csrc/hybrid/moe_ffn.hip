@@ -663,8 +663,8 @@ int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, i
 #undef K8SLLM_RK
     return (int)hipGetLastError();
   }
-  // two tokens a workgroup once that still leaves every compute unit several (8192 of 2048: 36.1 us with one, 28.8 with two, 30.7
-  // with four; 998 of 1024: 6.9 / 8.5 / 11.8)
+  // two tokens a workgroup once that still leaves every compute unit several, of what the kernel above does not take (us, one / two, 8 experts:
+  // 4096 tokens of 4104 39 / 20, 8192 of 8192 163 / 66; 4096 of 1003 13.3 / 10.7)
 #define K8SLLM_RTT(T_)                                \
   if (rows_w <= 8 && T >= 4096) K8SLLM_RT(T_, 8, 2);  \
   else if (rows_w <= 8) K8SLLM_RT(T_, 8, 1);          \

@@ -403,8 +403,8 @@ def test_grouped_gemm_tiles_keep_the_bits(rows, N, Kd, act, il):
 @pytest.mark.parametrize("N,K", [(16, 32), (1, 96), (200, 512), (72, 2080), (1024, 4096), (24, 4128)])
 def test_linear_of_few_rows(M, N, K):
     """Projections of a few rows against 64 bits: fewer steps of 32 k than waves, a rest, whole batches, columns around the tile of
-    16, a slice of wider rows, and one row or 32 k past the kernel's limits.  fp32 sums, one bf16 rounding: 2^-8 of the value
-    and 1e-6 sqrt(K) of what cancels."""
+    16, a slice of wider rows, and 32 k more than the kernel takes beside more than 4 rows.  fp32 sums, one bf16 rounding: 2^-8 of the
+    value and 1e-6 sqrt(K) of what cancels."""
     g = _g(73)
     x, w = _r(g, M, K + 24, dt=BF).cuda()[:, 16:16 + K], _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
     got, want = hops.linear(x, w).double(), x.double() @ w.double().t()
@@ -412,7 +412,7 @@ def test_linear_of_few_rows(M, N, K):
     assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 1e-6 * K ** 0.5).all())
 
 
-@pytest.mark.parametrize("T", [1, 5, 4099])  # one token a workgroup, two with a rest
+@pytest.mark.parametrize("T", [1, 5, 4099])  # one token a workgroup; up to 8 rows of weights in registers, four tokens a round with a rest
 @pytest.mark.parametrize("E,K,shared", [(8, 2, 0), (7, 3, 1), (16, 4, 1), (70, 16, 0)])
 def test_router_ranks(T, E, K, shared):
     """Routers: the K largest logits in order, the lower number first among equal ones (whole rows of ties), weights and the shared
@@ -600,6 +600,60 @@ def test_gradients_of_few_rows_products(M):
             assert not f(xg, wg).requires_grad
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 72, 6144), (5, 72, 6144), (2, 72, 6176), (3, 4096, 4128), (3, 4104, 4128), (16, 8200, 1056), (17, 8184, 1056),
+                                   (32, 72, 4096), (33, 72, 4096), (33, 2048, 2048), (33, 2064, 2048), (64, 1024, 96), (65, 1024, 96),
+                                   (16, 8192, 4096), (16, 10240, 4096), (64, 16384, 64), (64, 16400, 64)])
+def test_linear_at_the_limits_of_its_kernels(M, N, K):
+    """Products on both sides of each limit of the rule of few rows, against 64 bits, as above."""
+    g = _g(77)
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
+    got, want = hops.linear(x, w).double(), x.double() @ w.double().t()
+    assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 1e-6 * K ** 0.5).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 40, 96), (64, 8200, 288), (65, 8200, 288), (16, 40, 40), (512, 25616, 192), (511, 25616, 192), (300, 25616, 192)])
+@pytest.mark.parametrize("kind", ["relu_sq", "tanh"])
+def test_linear_act(M, N, K, kind):
+    """A product with an activation behind it, by a few-row kernel, the tile GEMM with partial tiles of rows and columns, and the library, against 64 bits:
+    the product's rounding through the activation, 2^-8 of its slope, and the result's."""
+    g = _g(79)
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
+    z = x.double() @ w.double().t()
+    want, slope = (torch.relu(z) ** 2, 2 * torch.relu(z)) if kind == "relu_sq" else (torch.tanh(z), 1 - torch.tanh(z) ** 2)
+    tol = 1.1 * 2 ** -8 * (want.abs() + slope * z.abs()) + 1e-4
+    assert bool(((hops.linear_act(x, w, kind).double() - want).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("M,f,rest", [(1, 4112, 24), (33, 4112, 24), (64, 208, 0), (65, 208, 24), (512, 12816, 48), (450, 12816, 48), (300, 12816, 48)])
+@pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
+def test_linear_glu_by_every_kernel(M, f, rest, kind):
+    """Gated units through ``linear_glu`` on both sides of its rules, the large ones with partial tiles of rows, features and the rest, against 64
+    bits: two rounded factors and a rounded product (as in test_gated_unit_in_the_tile_gemm)."""
+    g, K = _g(80), 192
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, 2 * f + rest, K, s=K ** -0.5, dt=BF).cuda()
+    a, y, col = hops.linear_glu(x, w, f, kind)
+    z = x.double() @ w.double().t()
+    p, u = z[:, :f], z[:, f:2 * f]
+    t = {"gelu_tanh": lambda v: F.gelu(v, approximate="tanh"), "silu": F.silu, "relu": F.relu}[kind](p)
+    assert bool(((a.double() - t * u).abs() <= 2 ** -7 * (t * u).abs() + 2 ** -8 * (t.abs() + 1.2 * p.abs() * u.abs()) + 1e-5).all())
+    r = z[:, 2 * f:]
+    assert bool(((y[:, col:col + rest].double() - r).abs() <= 2 ** -8 * r.abs() + 1e-6 * K ** 0.5).all())
+
+
+@pytest.mark.parametrize("M,N", [(1, 200), (3, 8200), (64, 8200), (65, 8200)])
+@pytest.mark.parametrize("scale,cap", [(1.0, 0.0), (1.0, 3.0), (0.25, 0.0), (0.25, 3.0)])
+def test_logits(M, N, scale, cap):
+    """fp32 logits of the rounded product, scaled and capped, in one launch and in several: exact but for the product's rounding, 2^-8 of it, and
+    1e-6 of the cap's tanh."""
+    g, K = _g(100), 288
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=2 * K ** -0.5, dt=BF).cuda()
+    z = scale * (x.double() @ w.double().t())
+    got = hops.logits(x, w, scale, cap)
+    assert got.dtype == torch.float32
+    want = cap * torch.tanh(z / cap) if cap else z
+    assert bool(((got.double() - want).abs() <= 2 ** -8 * z.abs() + 1e-5).all())
+
+
 @pytest.mark.parametrize("M", [1, 17, 40, 65, 512])
 def test_gated_units_that_no_projection_ends_with(M):
     """What is no gated unit of ``glu`` is refused as ``glu`` refuses it, whatever kernel the step's size would choose."""
@@ -669,7 +723,7 @@ def test_experts_of_empty_sums(rows, act, dt):
 @pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
 def test_gated_unit_in_the_projection(M, f, rest, K, kind):
     """The gated unit at the end of a few rows' projection gives the bits of the projection and the unit as two launches, and so do
-    the rows of the weights behind the unit's (one row, or an f that is no multiple of 16, past its limits: two launches)."""
+    the rows of the weights behind the unit's (an f that is no multiple of 16: two launches)."""
     g = _g(78)
     x, w = _r(g, M, K, dt=BF).cuda(), _r(g, 2 * f + rest, K, s=K ** -0.5, dt=BF).cuda()
     a, y, col = hops.linear_glu(x, w, f, kind)
@@ -754,6 +808,19 @@ def test_router_long_steps(T, d, E, K, shared, dt):
         if x is not None:
             y = torch.cat(ys)
             assert torch.equal(torch.nan_to_num(x, nan=-1.0) if x.is_floating_point() else x, torch.nan_to_num(y, nan=-1.0) if y.is_floating_point() else y)
+
+
+@pytest.mark.parametrize("d", [4104, 1003])  # wider than the registers hold; no multiple of 8
+@pytest.mark.parametrize("E,K,shared", [(8, 2, False), (7, 3, True)])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_router_two_tokens_a_workgroup(d, E, K, shared, dt):
+    """Long steps that the registers' router does not take, two tokens a workgroup and one left over: the bits of short steps."""
+    g, T = _g(101), 4099
+    h, wr, bias = _r(g, T, d, dt=dt).cuda(), _r(g, E + shared, d, s=d ** -0.5).cuda(), _r(g, E, s=0.3).cuda()
+    got = hops.moe_router(h, wr, bias, E, K)
+    parts = [hops.moe_router(h[i:i + 500], wr, bias, E, K) for i in range(0, T, 500)]
+    for x, *ys in zip(got, *parts):
+        assert x is None or torch.equal(x, torch.cat(ys))
 
 
 @pytest.mark.parametrize("T", [300, 4100])
@@ -952,7 +1019,7 @@ def test_single_tokens_beside_prompts_keep_their_bits(kind, prompts):
     z, zb = _r(g, T, H if per_head else H * d, dt=BF).cuda(), (_r(g, H if per_head else H * d) - 1.0).cuda()
     beta, al, bonus, lam = _r(g, T, H, dt=BF).cuda(), _r(g, H).cuda(), _r(g, H, d).cuda(), torch.tensor([0.9, 0.99]).cuda()
     longest = max(prompts)
-    assert T < 32 * S  # (linear attention takes steps of longer segments in chunks as a whole)
+    assert T < 32 * S  # (longer segments: test_single_tokens_beside_long_prompts)
 
     def run(a, b, s0, s1, **kw):  # rows [a, b), segments [s0, s1)
         s = state.clone()
@@ -966,6 +1033,27 @@ def test_single_tokens_beside_prompts_keep_their_bits(kind, prompts):
     od, sd = run(0, nd, 0, nd, longest=1)
     assert torch.equal(o[:nd], od) and torch.equal(s[:nd], sd[:nd])
     op, sp = run(nd, T, nd, S, longest=longest)
+    assert torch.equal(o[nd:], op) and torch.equal(s[nd:], sp[nd:])
+
+
+@pytest.mark.parametrize("prompts", [[1500, 700], [1100, 1, 64]])
+def test_single_tokens_beside_long_prompts(prompts):
+    """Linear attention with a mean of 32 rows a segment and more: running sequences' tokens in front have the bits of a step of their own, and
+    the prompts' those of a step without them."""
+    g, nd, H, d = _g(102), 20, 2, 32
+    lens = [1] * nd + prompts
+    S, T = len(lens), nd + sum(prompts)
+    assert T >= 32 * S
+    cu, ctx, slot = (v.cuda() for v in _segments(lens, [9] * nd + [0, 3, 0][:len(prompts)], list(range(S))))
+    vkq, state, lam = _r(g, T, 3 * H * d, s=0.5, dt=BF).cuda(), _r(g, S, H, d, d).cuda(), torch.tensor([0.9, 0.99]).cuda()
+
+    def run(a, b, s0, s1, **kw):
+        s = state.clone()
+        return hops.linear_attention(vkq[a:b], lam, s, cu[s0:s1 + 1] - cu[s0], ctx[s0:s1], slot[s0:s1], H, d, d, **kw), s
+
+    (o, s), (od, sd) = run(0, T, 0, S, longest=max(prompts), singles=nd), run(0, nd, 0, nd, longest=1)
+    op, sp = run(nd, T, nd, S, longest=max(prompts))
+    assert torch.equal(o[:nd], od) and torch.equal(s[:nd], sd[:nd])
     assert torch.equal(o[nd:], op) and torch.equal(s[nd:], sp[nd:])
 
 
