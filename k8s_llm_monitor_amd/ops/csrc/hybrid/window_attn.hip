@@ -458,6 +458,7 @@ inline int decode_heads(long B, int Hq, int R) {
 // branch, waited for the page before.  The same bits.  us over pages from memory, keys by a row a lane and all heads a workgroup / now at
 // decode_heads' choice, heads of 128: 1 sequence of 333 keys, 8 heads on 2 13.7 / 6.6; of 4000, 16 on 4 84 / 36; 24 of 1500 45 / 28; 64 of 1000
 // 39 / 34 (3.9 TB/s); 256 of 300 66 / 52; 64 of 1000, 16 heads on 2 55 / 45.
+// (In a step of 64 sequences behind 2048 tokens, window 1024, 46.8 / 44.3 a layer: 17 tiles of keys are three rounds of eight waves.)
 // A page's address is the wave's own, in scalar registers, and a lane adds one of a few offsets: an address a lane took up to 44 vector registers.
 // PER_CU: heads of 64, four a workgroup, in 128 registers (4 of 165 spilled), so that two share a compute unit once there is more than
 // one for each.  us, before the keys came through LDS / 165 registers / this, 32 heads on 8: 256 sequences of 64 keys 31 / 36 / 25, of 300 50 / 56 /
