@@ -561,8 +561,9 @@ __device__ __forceinline__ bf16_t expert_unit(float v, float u, float limit) {
 // us, gated / plain, 8 experts, with both operands loaded into registers and here: 2048 x 2048, 128 rows 35.8 / 21.4, 34.5 / 17.2
 // (3.9 TB/s); 2 rows 19.9 / 12.6, 9.4 / 7.2; 800 rows 144 / 77, 47 / 28; 2000 rows 258 / 144, 87 / 57; 4096 x 3584, 128 rows 111 / 69,
 // 105 / 44 (4.5 and 5.4 TB/s); 2000 rows 951 / 521, 240 / 158.
-// Not faster: 4096 x 3584, gated, 24 rows 91, 98 (one wave a workgroup 91, but 75 for 65 at 8 rows and up to 16 % more at most other widths);
-// the smallest calls, whose chain of chunks is longer: 2 experts, 1024 x 1024, plain, 2 rows 4.0, 4.4; 8 experts, 512 x 512, 8 rows 3.3, 3.9.
+// Not faster: gated, 4096 columns of K = 3584 (not 3584 of 4096), 24 to 64 rows 92, 98 (one wave a workgroup 93, but 75 for 65 at 8 rows and up
+// to 16 % more at most other widths); the smallest calls, whose chain of chunks is longer: 2 experts, 1024 x 1024, plain, 2 rows 4.0, 4.4;
+// 8 experts, 512 x 512, 8 rows 3.3, 3.9.
 // ``il``: the gate / up rows are interleaved per 128 rows as [64 gate | 64 up] (the prefill tile
 // GEMM's pairing), else [all gate rows ; all up rows].
 template <int ACT, int MT, int NW>
