@@ -52,24 +52,24 @@ __device__ __forceinline__ bool rows_tiles(int j, int f, int (&n)[KIND >= 0 && K
   }
 }
 
-template <int KIND, int MT>
+template <int KIND, int MT, bool ONCE>
 __global__ __launch_bounds__(256) void few_rows_own_kernel(RowsOut o, const bf16_t* __restrict__ X, long x_stride,
                                                            const bf16_t* __restrict__ W, int Kd) {
-  constexpr int NWV = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1, D = MT <= 2 ? 8 : 4, NT = MT * NS;
-  using S = OwnRows<MT, NS, D>;
+  constexpr int NWV = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1, D = MT <= 2 ? 4 : 2, NT = MT * NS;
+  using S = OwnRows<MT, NS, D, ONCE>;
   static_assert(NT <= S::BYTES / 1024, "");
   __shared__ __attribute__((aligned(1024))) char smem[NWV * S::BYTES];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int n[NS];
   const bool pair = rows_tiles<KIND>(blockIdx.x, o.f, n);
-  const int per = (Kd / 32 + NWV - 1) / NWV, s0 = min(wave * per, Kd / 32), ns = min(per, Kd / 32 - s0);
-  const bf16_t* src[NS + MT];
+  const int per = ((Kd + 63) / 64 + NWV - 1) / NWV * 64, k0 = min(wave * per, Kd);  // a wave's k begin at a line
+  LineSrc src[NS + MT];
 #pragma unroll
-  for (int t = 0; t < NS; ++t) src[t] = W + (long)min(n[t] + piece_row(), o.N - 1) * Kd + 32 * s0 + piece_k();
+  for (int t = 0; t < NS; ++t) src[t] = line_src([&](int r) { return W + (long)min(n[t] + r, o.N - 1) * Kd + k0; });
 #pragma unroll
-  for (int m = 0; m < MT; ++m) src[NS + m] = X + (long)min(16 * m + piece_row(), o.M - 1) * x_stride + 32 * s0 + piece_k();
+  for (int m = 0; m < MT; ++m) src[NS + m] = line_src([&](int r) { return X + (long)min(16 * m + r, o.M - 1) * x_stride + k0; });
   f32x4 acc[MT][NS] = {};
-  S::run(smem + wave * S::BYTES, src, ns, acc);
+  S::run(smem + wave * S::BYTES, src, min(per, Kd - k0), acc);
   __syncthreads();  // the rings have been read
   f32x4* red = reinterpret_cast<f32x4*>(smem);
 #pragma unroll
@@ -102,15 +102,17 @@ template <int KIND, int MT>
 __global__ __launch_bounds__(256) void few_rows_shared_kernel(RowsOut o, const bf16_t* __restrict__ X, long x_stride,
                                                               const bf16_t* __restrict__ W, int Kd) {
   constexpr int NW = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1;
-  using S = SharedRows<MT, NS, NW>;
+  using S = SharedRows<MT, NS, NW, true>;
   __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
   int n[NS];
   const bool pair = rows_tiles<KIND>(blockIdx.x * NW + (threadIdx.x >> 6), o.f, n);
-  const bf16_t* w[NS];
+  LineSrc w[NS];
 #pragma unroll
-  for (int t = 0; t < NS; ++t) w[t] = W + (long)min(n[t] + piece_row(), o.N - 1) * Kd + piece_k();
+  for (int t = 0; t < NS; ++t) w[t] = line_src([&](int r) { return W + (long)min(n[t] + r, o.N - 1) * Kd; });
   f32x4 acc[MT][NS] = {};
-  S::run(smem, [&](int m) { return X + (long)min(16 * m + piece_row(), o.M - 1) * x_stride + piece_k(); }, w, Kd / 32, acc);
+  S::run(smem, [&](int m) {
+    return line_src([&](int r) { return X + (long)min(16 * m + r, o.M - 1) * x_stride; });
+  }, w, Kd, acc);
   const int c = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int m = 0; m < MT; ++m)
@@ -141,12 +143,13 @@ int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const vo
   if (gated ? f <= 0 || f % 16 || N < 2 * f || yg == nullptr : f != 0) return -1;
   const RowsOut o{y, (bf16_t*)yg, M, N, f, f32, cap};
   const unsigned tiles = (unsigned)(gated ? f / 16 + (N - 2 * f + 31) / 32 : (N + 15) / 16);
-#define K8SLLM_FR(KIND, MT)                                                                                                  \
-  if (shared)                                                                                                                \
-    hipLaunchKernelGGL((few_rows_shared_kernel<KIND, MT>), dim3((tiles + 3) / 4), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, \
-                       (const bf16_t*)w, Kd);                                                                                \
-  else                                                                                                                       \
-    hipLaunchKernelGGL((few_rows_own_kernel<KIND, MT>), dim3(tiles), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, (const bf16_t*)w, Kd)
+  const bool once = 2l * N * Kd > kOnceBytes;  // (the shared form's calls are larger)
+#define K8SLLM_FRX(KERNEL, GRID) \
+  hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, (const bf16_t*)w, Kd)
+#define K8SLLM_FR(KIND, MT)                                                        \
+  if (shared) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT>), (tiles + 3) / 4);     \
+  else if (once) K8SLLM_FRX((few_rows_own_kernel<KIND, MT, true>), tiles);         \
+  else K8SLLM_FRX((few_rows_own_kernel<KIND, MT, false>), tiles)
 #define K8SLLM_FRM(KIND)              \
   if (M <= 16) { K8SLLM_FR(KIND, 1); } \
   else if (M <= 32) { K8SLLM_FR(KIND, 2); } \
@@ -160,6 +163,7 @@ int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const vo
   else return -1;
 #undef K8SLLM_FRM
 #undef K8SLLM_FR
+#undef K8SLLM_FRX
   return (int)hipGetLastError();
 }
 }

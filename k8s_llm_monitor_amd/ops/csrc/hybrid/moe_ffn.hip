@@ -558,15 +558,13 @@ __device__ __forceinline__ bf16_t expert_unit(float v, float u, float limit) {
 // chosen experts' weights, bound by how much of them is in flight.  A workgroup takes 16 MT sorted rows of one expert, gathered on
 // load, and 16 columns a wave; rows and weights come through LDS (stream_rows.h has why).  Every output is one chain of products in the
 // order of k, whatever the tile.
-// us, gated / plain, 8 experts, with both operands loaded into registers and here: 2048 x 2048, 128 rows 35.8 / 21.4, 34.5 / 17.2
-// (3.9 TB/s); 2 rows 19.9 / 12.6, 9.4 / 7.2; 800 rows 144 / 77, 47 / 28; 2000 rows 258 / 144, 87 / 57; 4096 x 3584, 128 rows 111 / 69,
-// 105 / 44 (4.5 and 5.4 TB/s); 2000 rows 951 / 521, 240 / 158.
-// Not faster: gated, 4096 columns of K = 3584 (not 3584 of 4096), 24 to 64 rows 92, 98 (one wave a workgroup 93, but 75 for 65 at 8 rows and up
-// to 16 % more at most other widths); the smallest calls, whose chain of chunks is longer: 2 experts, 1024 x 1024, plain, 2 rows 4.0, 4.4;
-// 8 experts, 512 x 512, 8 rows 3.3, 3.9.
+// us, gated / plain, 8 experts, lines of 32 k / of 64 with the weights non-temporal (stream_rows.h): 2048 x 2048, 16 rows 30.0 / 16.2, 26.8 /
+// 14.5; 128 rows 38.1 / 18.8, 32.9 / 16.6; 800 rows 49.8 / 28.8, 44.6 / 27.3; 2000 rows 92 / 61, 82 / 55; 4096 x 3584, 128 rows 96 / 50, 80 / 43
+// (5.9 and 5.5 TB/s); 2000 rows 284 / 171, 242 / 158; 1024 x 1024, 128 rows 10.7 / 7.1, 9.1 / 6.6; 64 experts of 512 x 2048, 128 rows 53 / 27,
+// 47 / 24, 4000 rows 87 / 56, 84 / 59.
 // ``il``: the gate / up rows are interleaved per 128 rows as [64 gate | 64 up] (the prefill tile
 // GEMM's pairing), else [all gate rows ; all up rows].
-template <int ACT, int MT, int NW>
+template <int ACT, int MT, int NW, bool ONCE>
 __global__ __launch_bounds__(64 * NW) void hy_grouped_gemm_mfma_kernel(bf16_t* __restrict__ Y, const bf16_t* __restrict__ A,
                                                                       const bf16_t* __restrict__ W,
                                                                       const int* __restrict__ offsets,
@@ -574,22 +572,28 @@ __global__ __launch_bounds__(64 * NW) void hy_grouped_gemm_mfma_kernel(bf16_t* _
                                                                       int N, int Kd, long w_es, int il, float limit) {
   constexpr bool GATED = ACT == 1 || ACT == 3;
   constexpr int NS = GATED ? 2 : 1;
-  using S = SharedRows<MT, NS, NW>;
+  using S = SharedRows<MT, NS, NW, ONCE>;
   __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
   int e, tile = blockIdx.y + blockIdx.z * gridDim.y, r0, r1;
   if (!expert_tile<16 * MT>(offsets, E, tile, e, r0, r1)) return;
   r0 += tile * (16 * MT);
-  const int n0 = (blockIdx.x * NW + (threadIdx.x >> 6)) * 16, nw = min(n0 + piece_row(), N - 1);
-  const bf16_t* We = W + (long)e * w_es + piece_k();
-  const long gate = GATED && il ? (long)(nw >> 6) * 128 + (nw & 63) : nw;
-  const bf16_t* w[NS];
-  w[0] = We + gate * Kd;
-  if (GATED) w[NS - 1] = We + (il ? gate + 64 : (long)N + nw) * Kd;
+  const int n0 = (blockIdx.x * NW + (threadIdx.x >> 6)) * 16;
+  const bf16_t* We = W + (long)e * w_es;
+  LineSrc w[NS];
+#pragma unroll
+  for (int t = 0; t < NS; ++t)
+    w[t] = line_src([&](int r) {
+      const int nw = min(n0 + r, N - 1);
+      const long gate = GATED && il ? (long)(nw >> 6) * 128 + (nw & 63) : nw;
+      return We + (t == 0 ? gate : il ? gate + 64 : (long)N + nw) * Kd;
+    });
   f32x4 acc[MT][NS] = {};
   S::run(smem, [&](int m) {
-    const int r = min(r0 + 16 * m + piece_row(), r1 - 1);
-    return A + (long)(sorted_idx != nullptr ? sorted_idx[r] / div : r) * Kd + piece_k();
-  }, w, Kd / 32, acc);
+    return line_src([&](int i) {
+      const int r = min(r0 + 16 * m + i, r1 - 1);
+      return A + (long)(sorted_idx != nullptr ? sorted_idx[r] / div : r) * Kd;
+    });
+  }, w, Kd, acc);
   const int n = n0 + (threadIdx.x & 15), quad = (threadIdx.x & 63) >> 4;
   if (n >= N) return;
 #pragma unroll
@@ -723,17 +727,22 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
   const bool steps = Kd >= 32 && Kd % 32 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
   if (!f32 && mfma && steps) {
     // a workgroup takes 16, 32 or 64 rows of an expert, so that its weights are mostly read once, by the mean number of rows an
-    // expert gets (8 experts, 2048 x 2048, gated + plain: mean 16 60 / 50 / 52 us with 16 / 32 / 64 rows, 32 69 / 64 / 52; 32 experts,
-    // mean 8: 157 / 177).  Two waves or, for 64 rows and where plain columns fill the chip, four (gated, two / four: 4096 x 3584, 8
+    // expert gets (8 experts, 2048 x 2048, gated + plain, in lines of 32 k: mean 16 60 / 50 / 52 us with 16 / 32 / 64 rows, 32 69 / 64 / 52; 32
+    // experts, mean 8: 157 / 177).  Two waves or, for 64 rows and where plain columns fill the chip, four (gated, two / four: 4096 x 3584, 8
     // rows 70 / 93, 32 rows 91 / 96, 128 rows 105 / 109; plain, 128 rows 50 / 44; 2048 x 2048, 512 rows 48 + 32 / 47 + 27).
     const bool gated = act == 1 || act == 3;
     const int mt = rows <= 8l * E ? 1 : rows <= 24l * E ? 2 : 4;
+    // Weights that several row tiles read stay in the caches, as those of small calls do (kOnceBytes, stream_rows.h); others are non-temporal (gated /
+    // plain us, as usual / non-temporal: 8 experts, 4096 x 3584, 128 rows 87 / 47, 80 / 43; 800 rows 123 / 77, 130 / 79; 2000 rows 242 / 158,
+    // 263 / 164).
+    const bool once = rows <= 64l * E && 2 * std::min<long>(rows, E) * (act == 1 || act == 3 ? 2 * N : N) * Kd > kOnceBytes;
     const int nw = mt == 4 || (!gated && std::min<long>(rows, E) * ((N + 63) / 64) >= 256) ? 4 : 2;
     const unsigned tiles = (unsigned)(rows / (16 * mt) + E), gz = (tiles + 65534) / 65535;  // (a grid's y ends at 65535)
     const dim3 g((unsigned)((N + 16 * nw - 1) / (16 * nw)), (tiles + gz - 1) / gz, gz);
-#define K8SLLM_GM(ACT, MT, NW)                                                                                       \
-  hipLaunchKernelGGL((hy_grouped_gemm_mfma_kernel<ACT, MT, NW>), g, dim3(64 * NW), 0, s, (bf16_t*)Y, (const bf16_t*)A,  \
-                     (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, il, limit)
+#define K8SLLM_GM(ACT, MT, NW)                                                                                             \
+  hipLaunchKernelGGL((once ? &hy_grouped_gemm_mfma_kernel<ACT, MT, NW, true> : &hy_grouped_gemm_mfma_kernel<ACT, MT, NW, false>), \
+                     g, dim3(64 * NW), 0, s, (bf16_t*)Y, (const bf16_t*)A, (const bf16_t*)W, offsets, sorted_idx, div, E, N, Kd, w_es, \
+                     il, limit)
 #define K8SLLM_GMP(ACT)                                 \
   if (mt == 4) K8SLLM_GM(ACT, 4, 4);                    \
   else if (mt == 2 && nw == 4) K8SLLM_GM(ACT, 2, 4);    \

@@ -1,8 +1,9 @@
-// Weight streams for a few rows: 16 output columns a wave, K in steps of 32, everything that v_mfma_f32_16x16x32_bf16 takes brought to
-// LDS by global_load_lds, 16 bytes a lane, 1 KB (16 rows x 32 k) a piece.
+// Weight streams for a few rows: 16 output columns a wave, everything that v_mfma_f32_16x16x32_bf16 takes brought to LDS by
+// global_load_lds, 16 bytes a lane, in lines of 16 rows x 64 k (windowed attention's keys in pieces of 16 rows x 32 k).
 // Why LDS and not registers: the instruction wants row lane % 16 in a lane, so a register load of row-major rows meets 16 cache lines in
 // every 16 lanes and takes about 60 cycles of the load path (512 KB from L2 by one CU: 13 us, 3.6 us in lane order), and activations take as
-// much of it as weights do.  A piece has four lanes a row; the chunk that lane l fetches is turned by the row, so that the
+// much of it as weights do.
+// A piece (1 KB) has four lanes a row; the chunk that lane l fetches is turned by the row, so that the
 // fragments' reads (row lane % 16, chunk lane / 16) are spread over the banks.
 #pragma once
 #include <type_traits>
@@ -22,116 +23,191 @@ __device__ __forceinline__ void load_piece(char* lds, const bf16_t* src) {
   __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) const void*)src, (__attribute__((address_space(3))) void*)lds, 16,
                                    0, 0);
 }
+// the same for what a step reads once: non-temporal, so that it does not push out what is read again
+__device__ __forceinline__ void load_piece_once(char* lds, const bf16_t* src) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) const void*)src, (__attribute__((address_space(3))) void*)lds, 16,
+                                   0, 2);
+}
 template <int N>
 __device__ __forceinline__ void loads_left() {  // waits until at most N of this wave's loads are on their way
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// NW waves of one workgroup share 16 MT rows, which come in chunks of 8 steps to a ring of two; each wave streams its own NS
-// weight tiles through a private ring, 8 steps ahead.  Every output is one chain of products in the order of k.
-template <int MT, int NS, int NW>
-struct SharedRows {
-  static constexpr int D = 8;  // steps of a chunk, and of the weights' ring
-  static constexpr int SLOT = D * MT * 1024, RING = D * NS * 1024, BYTES = 2 * SLOT + NW * RING;
-  static constexpr int PER = D * MT / NW;  // pieces of a chunk that a wave brings, all of one row tile
-  static_assert(NW % MT == 0, "");
-
-  // x(m): this lane's source in row tile m of the rows; w[t]: in weight tile t; nk: steps
-  template <class X>
-  static __device__ __forceinline__ void run(char* lds, X x, const bf16_t* const (&w)[NS], int nk, f32x4 (&acc)[MT][NS]) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rd = piece_frag();
-    const int m0 = wave % MT, k0 = wave / MT;
-    const bf16_t* xs = x(m0);
-    char* ring = lds + 2 * SLOT + wave * RING;
-    auto stage = [&](int c) {  // steps past the last repeat it; nothing multiplies them
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int ks = k0 + i * (NW / MT);
-        load_piece(lds + (c & 1) * SLOT + (ks * MT + m0) * 1024, xs + 32 * min(c * D + ks, nk - 1));
-      }
-    };
-    auto refill = [&](int d, int k) {
-#pragma unroll
-      for (int t = 0; t < NS; ++t) load_piece(ring + (d * NS + t) * 1024, w[t] + 32 * k);
-    };
-    auto chunk = [&](int c, auto whole) {
-      constexpr bool WHOLE = decltype(whole)::value;  // every step, the next chunk and every refill are inside K
-      if constexpr (WHOLE) loads_left<D * NS>();  // the chunk's pieces are older than the ring's
-      else loads_left<0>();
-      __builtin_amdgcn_s_barrier();  // every wave's pieces are there, and the other slot has been read
-      if (WHOLE || (c + 1) * D < nk) stage(c + 1);
-      auto step = [&](auto self, auto jc) {
-        constexpr int j = decltype(jc)::value;
-        if constexpr (j < D) {
-          if (WHOLE || c * D + j < nk) {
-            // younger than this step's weights: the D - 1 steps behind it and the chunk just begun
-            if constexpr (WHOLE) loads_left<(D - 1) * NS + PER>();
-            else if (j > 0) loads_left<0>();
-            bf16x8 a[MT], b[NS];
-#pragma unroll
-            for (int t = 0; t < NS; ++t) b[t] = *reinterpret_cast<const bf16x8*>(ring + (j * NS + t) * 1024 + rd);
-#pragma unroll
-            for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const bf16x8*>(lds + (c & 1) * SLOT + (j * MT + m) * 1024 + rd);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            if (WHOLE || (c + 1) * D + j < nk) refill(j, (c + 1) * D + j);
-#pragma unroll
-            for (int t = 0; t < NS; ++t)
-#pragma unroll
-              for (int m = 0; m < MT; ++m) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b[t], acc[m][t], 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          self(self, std::integral_constant<int, j + 1>{});
-        }
-      };
-      step(step, std::integral_constant<int, 0>{});
-    };
-    stage(0);
-#pragma unroll
-    for (int d = 0; d < D; ++d) refill(d, min(d, nk - 1));
-    int c = 0;
-    for (; (c + 2) * D <= nk; ++c) chunk(c, std::true_type{});
-    for (; c * D < nk; ++c) chunk(c, std::false_type{});
-  }
+// A line: 16 rows x 64 k, 2 KB, two loads of 8 rows in whole 128-byte cache lines (a piece's 64 bytes a row ask for every cache line
+// twice).  us over weights from memory, in pieces / in lines / in lines with the weights non-temporal, few_rows.hip: 4096 x 4096, 64 rows
+// 19.9 / 14.1 / 13.6; 16384 x 4096, 1 row 26.3 / 26.9 / 23.6, 64 rows 36.3 / 34.7 / 30.8; 128256 x 4096, 1 row 179 / 186 / 162 (6.5 TB/s);
+// 1024 x 1024, 1 row 2.9 / 3.0 / 3.1; 8 experts of 2048 x 2048, gated, 128 rows 36.9 / 35.1 / 31.9, 800 rows 47.7 / 42.9 / 41.7.  Twice the
+// lines in flight gain nothing anywhere.
+// The weights of a call of up to 8 MB are loaded as usual (kOnceBytes): a model of such calls has its place in the memory-side cache of 256 MB.
+// Steps of one sequence with 2 of 8 experts of 1024 x 1024 in four layers, us: never / always / above 8 MB non-temporal 245 / 250 / 244, of 64 424 /
+// 383 / 380.
+// Load i of lane l brings row 8 i + l / 8, and of its eight 16-byte chunks the one that is turned by row / 2: sixteen
+// rows' fragments of one k are then sixteen different chunks of 256 bytes.
+__device__ __forceinline__ int line_row(int i) { return 8 * i + ((threadIdx.x & 63) >> 3); }
+__device__ __forceinline__ int line_k(int i) { return 8 * ((threadIdx.x & 7) ^ (4 * i + ((threadIdx.x & 63) >> 4))); }
+__device__ __forceinline__ int line_frag() {  // of a line's first 32 k; the others' are at ^ 64
+  const int lane = threadIdx.x & 63, c16 = lane & 15;
+  return c16 * 128 + 16 * ((lane >> 4) ^ (c16 >> 1));
+}
+// Where this lane finds its chunks of a line's two loads, at k = 0.  K ends inside a line if it is an odd number of 32: the chunks behind
+// it, and lines behind the last, are read from the row's last chunk, and nothing multiplies them.
+constexpr long kOnceBytes = 8l << 20;
+struct LineSrc {
+  const bf16_t* p[2];
+  __device__ __forceinline__ int within(int i, int k, int kd) const { return min(k, kd - 8 - line_k(i)); }
+  __device__ __forceinline__ void load(char* lds, int i, int k) const { load_piece(lds + 1024 * i, p[i] + k); }
+  __device__ __forceinline__ void once(char* lds, int i, int k) const { load_piece_once(lds + 1024 * i, p[i] + k); }
 };
+// row(r): where row r (of 16) begins
+template <class R>
+__device__ __forceinline__ LineSrc line_src(R row) {
+  return {{row(line_row(0)) + line_k(0), row(line_row(1)) + line_k(1)}};
+}
 
-// One wave streams 16 MT rows and NS weight tiles, its own part of K, through a private ring D steps deep: no barrier.
-template <int MT, int NS, int D>
-struct OwnRows {
-  static constexpr int L = MT + NS, BYTES = D * L * 1024;
+// NW waves of one workgroup share 16 MT rows, which come in chunks of 4 lines to a ring of two; each wave streams its own NS
+// weight tiles through a private ring, 4 lines ahead.  Every output is one chain of products in the order of k.  ONCE: the
+// weights' loads are non-temporal.
+template <int MT, int NS, int NW, bool ONCE>
+struct SharedRows {
+  static constexpr int D = 4;  // lines of a chunk, and of the weights' ring
+  static constexpr int SLOT = D * MT * 2048, RING = D * NS * 2048, BYTES = 2 * SLOT + NW * RING;
+  // a wave brings one row tile's loads of a chunk: all, those of every line's half, or those of every other line's half
+  static constexpr int P = NW / MT, PER = 2 * D / P, HALVES = P == 1 ? 2 : 1, EVERY = P > 2 ? P / 2 : 1;
+  static_assert(NW % MT == 0 && P <= 4, "");
 
-  // src: this lane's sources, weight tiles first; ns: steps
-  static __device__ __forceinline__ void run(char* lds, const bf16_t* const (&src)[L], int ns, f32x4 (&acc)[MT][NS]) {
-    if (ns <= 0) return;
-    const int rd = piece_frag();
-    auto issue = [&](int slot, int k) {
+  // x(m): this lane's sources in row tile m of the rows; w[t]: in weight tile t; kd: a multiple of 32
+  template <class X>
+  static __device__ __forceinline__ void run(char* lds, X x, const LineSrc (&w)[NS], int kd, f32x4 (&acc)[MT][NS]) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rd = line_frag(), nl = (kd + 63) / 64;
+    const int m0 = wave % MT, h0 = (wave / MT) & (P > 1 ? 1 : 0), u0 = P > 2 ? wave / MT / 2 : 0;
+    const LineSrc xs = x(m0);
+    char* ring = lds + 2 * SLOT + wave * RING;
+    auto stage = [&](int c, auto whole) {
 #pragma unroll
-      for (int i = 0; i < L; ++i) load_piece(lds + (slot * L + i) * 1024, src[i] + 32 * k);
+      for (int i = 0; i < D / EVERY; ++i)
+#pragma unroll
+        for (int j = 0; j < HALVES; ++j) {
+          const int u = u0 + i * EVERY, h = HALVES == 1 ? h0 : j;
+          const int k = 64 * (c * D + u);
+          load_piece(lds + (c & 1) * SLOT + (u * MT + m0) * 2048 + 1024 * h,
+                     (h ? xs.p[1] : xs.p[0]) + (decltype(whole)::value ? k : xs.within(h, k, kd)));
+        }
     };
-    auto consume = [&](int slot) {
-      bf16x8 f[L];
-#pragma unroll
-      for (int i = 0; i < L; ++i) f[i] = *reinterpret_cast<const bf16x8*>(lds + (slot * L + i) * 1024 + rd);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot may be refilled
+    auto refill = [&](int u, int l, auto whole) {
 #pragma unroll
       for (int t = 0; t < NS; ++t)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[NS + m], f[t], acc[m][t], 0, 0, 0);
+        for (int i = 0; i < 2; ++i) {
+          const int k = decltype(whole)::value ? 64 * l : w[t].within(i, 64 * l, kd);
+          if constexpr (ONCE) w[t].once(ring + (u * NS + t) * 2048, i, k);
+          else w[t].load(ring + (u * NS + t) * 2048, i, k);
+        }
+    };
+    auto chunk = [&](int c, auto whole) {
+      constexpr bool WHOLE = decltype(whole)::value;  // every line, the next chunk and every refill are inside K
+      if constexpr (WHOLE) loads_left<2 * D * NS>();  // the chunk's loads are older than the ring's
+      else loads_left<0>();
+      __builtin_amdgcn_s_barrier();  // every wave's loads are there, and the other slot has been read
+      if (WHOLE || (c + 1) * D < nl) stage(c + 1, whole);
+      auto line = [&](auto self, auto uc) {
+        constexpr int u = decltype(uc)::value;
+        if constexpr (u < D) {
+          if (WHOLE || c * D + u < nl) {
+            // younger than this line's weights: the D - 1 lines behind it and the chunk just begun
+            if constexpr (WHOLE) loads_left<2 * (D - 1) * NS + PER>();
+            else if (u > 0) loads_left<0>();
+            bf16x8 a[2][MT], b[2][NS];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+              for (int t = 0; t < NS; ++t) b[j][t] = *reinterpret_cast<const bf16x8*>(ring + (u * NS + t) * 2048 + (rd ^ (64 * j)));
+#pragma unroll
+              for (int m = 0; m < MT; ++m)
+                a[j][m] = *reinterpret_cast<const bf16x8*>(lds + (c & 1) * SLOT + (u * MT + m) * 2048 + (rd ^ (64 * j)));
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (WHOLE || (c + 1) * D + u < nl) refill(u, (c + 1) * D + u, whole);
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              if (j == 0 || WHOLE || 64 * (c * D + u) + 32 < kd) {
+#pragma unroll
+                for (int t = 0; t < NS; ++t)
+#pragma unroll
+                  for (int m = 0; m < MT; ++m) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j][m], b[j][t], acc[m][t], 0, 0, 0);
+              }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          self(self, std::integral_constant<int, u + 1>{});
+        }
+      };
+      line(line, std::integral_constant<int, 0>{});
+    };
+    stage(0, std::false_type{});
+#pragma unroll
+    for (int u = 0; u < D; ++u) refill(u, u, std::false_type{});
+    int c = 0;
+    for (; 64 * (c + 2) * D <= kd; ++c) chunk(c, std::true_type{});
+    for (; c * D < nl; ++c) chunk(c, std::false_type{});
+  }
+};
+
+// One wave streams 16 MT rows and NS weight tiles, its own part of K, through a private ring D lines deep: no barrier.
+template <int MT, int NS, int D, bool ONCE>
+struct OwnRows {
+  static constexpr int L = MT + NS, BYTES = D * L * 2048;
+
+  // src: this lane's sources, weight tiles first; kd: k of this part, a multiple of 32
+  static __device__ __forceinline__ void run(char* lds, const LineSrc (&src)[L], int kd, f32x4 (&acc)[MT][NS]) {
+    if (kd <= 0) return;
+    const int rd = line_frag(), nl = (kd + 63) / 64;
+    auto issue = [&](int slot, int l, auto whole) {
+#pragma unroll
+      for (int i = 0; i < L; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int k = decltype(whole)::value ? 64 * l : src[i].within(j, 64 * l, kd);
+          if (ONCE && i < NS) src[i].once(lds + (slot * L + i) * 2048, j, k);
+          else src[i].load(lds + (slot * L + i) * 2048, j, k);
+        }
+    };
+    auto consume = [&](int slot, bool half) {
+      bf16x8 f[2][L];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < L; ++i) f[j][i] = *reinterpret_cast<const bf16x8*>(lds + (slot * L + i) * 2048 + (rd ^ (64 * j)));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot may be refilled
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (j == 0 || !half) {
+#pragma unroll
+          for (int t = 0; t < NS; ++t)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j][NS + m], f[j][t], acc[m][t], 0, 0, 0);
+        }
     };
 #pragma unroll
-    for (int d = 0; d < D; ++d) issue(d, min(d, ns - 1));
-    int slot = 0, k = 0;
-    for (; k + D < ns; ++k) {
-      loads_left<(D - 1) * L>();
-      consume(slot);
-      issue(slot, k + D);
+    for (int d = 0; d < D; ++d) issue(d, d, std::false_type{});
+    int slot = 0, l = 0;
+    for (; 64 * (l + D + 1) <= kd; ++l) {
+      loads_left<2 * (D - 1) * L>();
+      consume(slot, false);
+      issue(slot, l + D, std::true_type{});
       slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    if (l + D < nl) {  // the line that K ends in
+      loads_left<2 * (D - 1) * L>();
+      consume(slot, false);
+      issue(slot, l + D, std::false_type{});
+      slot = slot + 1 == D ? 0 : slot + 1;
+      ++l;
     }
     auto rest = [&](auto self, auto dc) {
       constexpr int d = decltype(dc)::value;
       if constexpr (d < D) {
-        loads_left<(D - 1 - d) * L>();
-        if (k + d < ns) {
-          consume(slot);
+        loads_left<2 * (D - 1 - d) * L>();
+        if (l + d < nl) {
+          consume(slot, 64 * (l + d) + 32 >= kd);
           slot = slot + 1 == D ? 0 : slot + 1;
         }
         self(self, std::integral_constant<int, d + 1>{});

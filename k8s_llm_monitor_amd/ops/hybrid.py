@@ -1160,38 +1160,45 @@ def _rows_form(M: int, N: int, K: int, end: str = "") -> Optional[str]:
     """Which kernel of few_rows.hip takes a bf16 product of M rows with weights [N, K]; ``end``: what stands behind it and would be a launch
     of its own, a gated unit of its first rows ("glu") or something elementwise ("act").  None: the BLAS library.  us, library (and launch)
     / own / shared, in a graph over weights from memory:
-    plain     2048 x 2048, 1 row 8.5 / 3.6 / 6.0, 64 rows 9.2 / 7.8 / 11.5; 4096 x 4096, 16 rows 15.6 / 9.6 / 16.6, 48 rows 13.9 / 17.2 / 21.7;
-              8192 x 4096, 16 rows 17.2 / 19.1 / 19.8 (shared: 128 workgroups); 16384 x 4096, 1 row 34 / 26 / 32, 16 rows 34 / 35 / 30, 64
-              rows 36 / 70 / 37; 24576 x 2048, 32 rows 27 / 36 / 29; 65536 x 1024, 4 rows 28 / 30 / 26; 128256 x 4096, 4 rows 192 / 181 / -, 16
-              rows 191 / - / 205
-    act       8192 x 4096, 64 rows 23 / 38 / 26; 12288 x 4096, 64 rows 30 / 55 / 30; 24576 x 2048, 32 rows 30 / 35 / 28, 64 rows 32 / 52 / 36
-    glu       (a workgroup of either takes half as many columns) 8192 x 2048, 64 rows 17 / 15 / 22; 8192 x 4096, 16 rows 20 / 17 / 33; 16384 x
-              4096, 16 rows 37 / 33 / 39, 32 rows 36 / 39 / 41; 32768 x 4096, 4 rows 66 / 54 / 65, 64 rows 69 / 95 / 72; 10240 x 5632, 1 row 28 / 33 / 52"""
-    if M > 64 or K > 6144 or (N * K > 1 << 28 and (M > 4 or end == "glu")):
+    plain     up to 16 rows: 2048 x 2048, 1 row 8.5 / 4.0 / 7.4; 4096 x 4096, 16 rows 16.4 / 8.3 / 14.6; 7168 x 4096, 16 rows 16.3 / 13.7 / 16.5;
+              16384 x 1024, 4 rows 10.3 / 9.9 / 8.4; 16384 x 4096, 8 rows 34.7 / 24.8 / 29.2; 128256 x 4096, 4 rows 193 / 164 / 180; 4096 x
+              11008, 4 rows 39 / 18.7 / 35; 8192 x 16384, 16 rows 62 / 56 / 63
+              up to 32: 4096 x 4096 14.0 / 9.2 / 15.9; 8192 x 2048 14.4 / 10.4 / 11.1; 11312 x 4096 23.2 / 26.1 / 21.0; 32768 x 4096 69.7 / 68 /
+              52.4; 4096 x 11008 32 / 25.6 / 41; 6144 x 5632 20.4 / 23.5 / 23.7
+              up to 64: 4096 x 2048 12.3 / 8.2 / 12; 10240 x 4096 29.4 / 31 / 24.7; 16384 x 2048 19.7 / 26 / 19.3; 24576 x 2048 28 / 37 / 31; 32768
+              x 4096 66 / 90 / 58; 6144 x 4096 18.7 / 23 / 21.8
+    act       8192 x 4096, 64 rows 26.1 / 24.8 / 25.3; 32768 x 2048, 64 rows 50 / 51 / 39; 24576 x 5632, 64 rows 74 / 110 / 70
+    glu       (a workgroup of either takes half as many columns) 8192 x 2048, 64 rows 17 / 13 / 19; 16384 x 4096, 16 rows 37 / 27 / 36, 32 rows
+              37 / 30 / 35; 24576 x 4096, 24 rows 52 / 41 / 43, 64 rows 53 / 58 / 46; 32768 x 4096, 8 rows 66 / 47 / 60, 16384 x 2048, 24 rows
+              20 / 17 / 20; 32768 x 1024, 4 rows 20 / 18 / 14
+    Between the lines the library is up to 5 % slower, and up to 25 % for units of 25 and more rows against 8 K to 16 K features."""
+    if M > 64 or K > 16384 or (N * K > 1 << 28 and (M > 4 or end == "glu")):
         return None
     if end == "glu":
         if K > 4096:
             return None
-        if M <= 4 and N * K <= 1 << 27 and (N < 32768 or K > 1024):
-            return "own"
-        if N >= 24576 and (K <= 2048 or M <= 16 or N >= 32768):
+        if N >= 32768 and (K <= 1024 or M > 8):
             return "shared"
-        small = N <= 8192 or (N <= 16384 and K <= 2048)
-        if M <= 8 or (M <= 16 and (N <= 12288 or small)) or (M <= 24 and small) or (K <= 2048 and N * K <= 1 << 24):
+        if M <= 16 or (M <= 32 and K > 2048) or N <= 8192 and (M <= 32 or K <= 2048) or (M <= 24 and N <= 16384):
             return "own"
-        return None
+        return "shared" if N >= 24576 else None
+    if K > 6144:  # whole lines for each of a workgroup's waves
+        return "own" if K % 256 == 0 and (M <= 8 or (M <= 16 and N <= 4096) or (M <= 32 and 2048 < N <= 4096)) else None
     if K > 4096:
-        return "own" if M <= 2 or (M <= 4 and (end or N <= 4096 or 8192 <= N <= 32768)) else None
-    if M <= 4:
-        return "shared" if N >= 32768 and K <= 1024 else "own"
-    if (M <= 16 and N * K <= 1 << 24) or (M <= 32 and N * K <= 1 << 24 and N < 8192) or (N * K <= 1 << 22 and K <= 2048):
+        if M <= 2 or (M <= 4 and (end or N <= 4096 or 8192 <= N <= 32768)) or (M <= 32 and 2048 <= N <= 4096):
+            return "own"
+        return "shared" if N >= 10240 and (M <= 16 or end) else None
+    if M <= 8:
+        return "shared" if N >= 131072 or (N >= 10240 and K <= 1024) else "own"
+    if M <= 16:
+        return "own" if N * K < 1 << 25 and (N < 10240 or K > 1024) else "shared" if N >= 10240 else None
+    if M <= 32:
+        if N * K <= 1 << 24 and (N < 8192 or K > 1024):
+            return "own"
+        return "shared" if N >= 10240 or (N >= 8192 and K <= 3072) else None
+    if N * K <= 1 << 23 or (N * K < 1 << 24 and K <= 2048):
         return "own"
-    if N < 8192 or (N < 10240 and K > 3072):
-        return None
-    if M <= 16 or (N <= 16384 and (M <= 32 or end or K <= 1024)) or (
-            M <= 32 and ((K <= 1024 and N * K <= 1 << 26) or (end and (K <= 2048 or N >= 32768)))):
-        return "shared"
-    return None
+    return "shared" if 10240 <= N <= 16384 or (N >= 28672 and (end or K >= 2048)) else None
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, end: str = "") -> Optional[str]:

@@ -536,6 +536,21 @@ def test_few_rows_forms(M, f, rest, K, shared):
         assert torch.equal(a, hops.glu(y, 0, f, kind)) and torch.equal(q, y[:, 2 * f:])
 
 
+@pytest.mark.parametrize("K", [64, 160, 512, 544, 1088, 8192])  # lines of 64 k: one, two and a half, a wave's last one half, chunks of four and a rest
+@pytest.mark.parametrize("M", [3, 24, 50])
+def test_few_rows_and_experts_in_lines(M, K):
+    """Both forms and the experts' kernel, which read weights in lines of 64 k, against 64 bits; rows and weights end where their
+    allocations do.  fp32 sums, one bf16 rounding: 2^-8 of the value and 1e-6 sqrt(K) of what cancels."""
+    g = _g(77)
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, 88, K, s=K ** -0.5, dt=BF).cuda()
+    z, ext = x.double() @ w.double().t(), hops.native()
+    y = torch.full((3, M, 88), float("nan"), dtype=BF, device="cuda")
+    for shared in (False, True):
+        ext.few_rows(y[int(shared)], None, x, w, -1, 0.0, shared)
+    ext.grouped_gemm(y[2], x, w.view(1, 88, K), torch.tensor([0, M], dtype=torch.int32, device="cuda"), None, 1, 0, False, True, 0.0)
+    assert bool(((y.double() - z).abs() <= 2 ** -8 * z.abs() + 1e-6 * K ** 0.5).all())
+
+
 @pytest.mark.parametrize("M", [1, 257, 600])
 @pytest.mark.parametrize("f,rest,K", [(128, 0, 192), (144, 48, 256), (400, 272, 320), (16, 256, 192)])  # tiles of 128 features and 256 columns
 @pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
