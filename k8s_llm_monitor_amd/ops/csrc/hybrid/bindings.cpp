@@ -25,7 +25,7 @@ int k8sllm_hy_decay_scan(float* o, const void* qkv, long stride, int q_col, int 
                          long z_stride, const float* z_bias, const float* a_log, float inv_tau, int dkind, int per_head,
                          const void* beta, long b_stride, const float* bonus, float* state, const int* cu,
                          const int* ctx, const int* slot, int S, int H, int Gk, int dk, int dv, float q_scale, int unit,
-                         int f32, float* ws, long T, hipStream_t s);
+                         int f32, float* ws, long T, int step, hipStream_t s);
 long k8sllm_hy_decay_scan_ws(long T, int H, int Gk, int dk);
 int k8sllm_hy_router_grouped(int* ids, float* wts, const void* h, long T, int d, const float* wr, const float* corr, int E,
                              int K, int groups, int keep, float scale, int soft, int best2, int renorm, int f32,
@@ -69,7 +69,7 @@ int k8sllm_hy_ssm_scan(float* y, const void* xbc, const void* proj, long p_strid
 int k8sllm_hy_selective_scan(void* out, const void* xc, const void* q, long q_stride, int b_col, int c_col,
                              const void* dt, long dt_stride, const float* dt_bias, const float* a_log, const float* d_skip,
                              const void* z, long z_stride, float* state, const int* cu, const int* ctx, const int* slot,
-                             int S, long T, int C, int N, int f32, float* ws, hipStream_t s);
+                             int S, long T, int C, int N, int f32, float* ws, int step, hipStream_t s);
 long k8sllm_hy_selective_scan_ws(long T, int S, int longest, int C, int N, int mode);
 int k8sllm_hy_join_norm(void* out, float* residual, const void* y0, int t0, const void* y1, int t1, const float* w0,
                         const float* w1, float mix, const float* pw, const float* pb, const float* nw, const float* nb,
@@ -500,7 +500,7 @@ void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, Opt
                                         (long)(T - singles), (int)longest, (int)nh, (int)N, (int)P, (int)nt, cur());
     if (rc != 1) {
       check(rc, "ssm_scan (chunked)");
-      return scan(singles, singles, 1);
+      return scan(singles, singles, 0);
     }
   }
   scan(S, T, mode == 3 ? 0 : mode);
@@ -751,7 +751,8 @@ void decay_scan(Tensor o, Tensor qkv, int64_t q_col, int64_t k_col, int64_t v_co
     check(k8sllm_hy_decay_scan(o.data_ptr<float>(), qkv.data_ptr(), qkv.stride(0), (int)q_col, (int)k_col, (int)v_col, zp, z.stride(0),
                                z_bias.data_ptr<float>(), ap, (float)(1.0 / tau), (int)dkind, per_head, bp, bstride, wp_bonus,
                                state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(), (int)segments,
-                               (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale, unit, f, wp, (long)rows, cur()),
+                               (int)H, (int)Gk, (int)dk, (int)dv, (float)q_scale, unit, f, wp, (long)rows,
+                               mode == 0 && rows <= segments, cur()),
           "decay_scan");
   };
   const int* cu1 = cu.data_ptr<int>() + singles;
@@ -832,7 +833,7 @@ void selective_scan(Tensor out, Tensor xc, Tensor q, int64_t b_col, int64_t c_co
                                  dt.stride(0), dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), d_skip.data_ptr<float>(),
                                  (const char*)proj.data_ptr() + z_col * proj.element_size(), proj.stride(0),
                                  state.data_ptr<float>(), cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(),
-                                 (int)ctx.numel(), T, (int)C, (int)N, f, n_ws > 0 ? ws.data_ptr<float>() : nullptr, cur()),
+                                 (int)ctx.numel(), T, (int)C, (int)N, f, n_ws > 0 ? ws.data_ptr<float>() : nullptr, mode == 0, cur()),
         "selective_scan");
 }
 

@@ -45,24 +45,10 @@ __device__ __forceinline__ float decay_f(float x, int kind, float A, float inv_t
 }
 
 // One token of the recurrence for a lane's 8 key channels; returns the column's read-out (all lanes of the
-// column hold it).  gv: this token's decays (one number for all channels where HD).
-template <int CH, int MODE, bool HD>
-__device__ __forceinline__ float scan_token(float (&S)[8], const float* __restrict__ gp, float gh,
-                                            const float* __restrict__ kp, const float* __restrict__ qp, float v,
-                                            float bt, float kq) {
-  float gv[8];
-  if (HD) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) gv[i] = gh;
-  } else {
-    const float4 g0 = *reinterpret_cast<const float4*>(gp), g1 = *reinterpret_cast<const float4*>(gp + 4);
-    gv[0] = g0.x; gv[1] = g0.y; gv[2] = g0.z; gv[3] = g0.w;
-    gv[4] = g1.x; gv[5] = g1.y; gv[6] = g1.z; gv[7] = g1.w;
-  }
-  const float4 k0 = *reinterpret_cast<const float4*>(kp), k1 = *reinterpret_cast<const float4*>(kp + 4);
-  const float4 q0 = *reinterpret_cast<const float4*>(qp), q1 = *reinterpret_cast<const float4*>(qp + 4);
-  const float kv[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-  const float qv[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+// column hold it).  gv: this token's decays.
+template <int CH, int MODE>
+__device__ __forceinline__ float scan_channels(float (&S)[8], const float (&gv)[8], const float (&kv)[8], const float (&qv)[8], float v,
+                                               float bt, float kq) {
   float pk0 = 0.f, pk1 = 0.f, pq0 = 0.f, pq1 = 0.f;  // two accumulators per sum: half the dependent adds
 #pragma unroll
   for (int i = 0; i < 8; i += 2) {
@@ -85,8 +71,25 @@ __device__ __forceinline__ float scan_token(float (&S)[8], const float* __restri
   const float pq = lanes_sum<CH>(pq0 + pq1);
   const float u = MODE == kDelta ? bt * (v - pk) : v;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) S[i] += kv[i] * u;
+  for (int i = 0; i < 8; ++i) S[i] = fmaf(kv[i], u, S[i]);
   return pq + u * kq;
+}
+
+// The same with decays, key and query in LDS (one decay for all channels, gh, where HD)
+template <int CH, int MODE, bool HD>
+__device__ __forceinline__ float scan_token(float (&S)[8], const float* __restrict__ gp, float gh,
+                                            const float* __restrict__ kp, const float* __restrict__ qp, float v,
+                                            float bt, float kq) {
+  float gv[8], kv[8], qv[8];
+  if (HD) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) gv[i] = gh;
+  } else {
+    load8(gp, gv);
+  }
+  load8(kp, kv);
+  load8(qp, qv);
+  return scan_channels<CH, MODE>(S, gv, kv, qv, v, bt, kq);
 }
 
 template <typename T, int CH, int MODE, bool HD>
@@ -211,6 +214,120 @@ __global__ __launch_bounds__(256) void decay_scan_kernel(float* __restrict__ o, 
         if (n0 + i < dk) sp[i] = S[i];
     }
   }
+}
+
+// Steps of one token a segment (decode): a pass over the states.  A wave's lanes lie over the rows of the state as in decay_scan_kernel, R
+// times over, so that 32 R bytes a lane are on their way before anything waits, and a (segment, head)'s key, query and decays are prepared by few
+// workgroups; every 16 lanes form the norms for themselves.  The same operations in the same order: the same bits.
+// us, decay_scan_kernel / here: delta rule with a decay per head, 32 heads of 128 x 128, 4 segments 8.6 / 7.5, 16 25.8 / 19.8, 64 81 / 58 (4.6 TB/s);
+// 64 heads of 64 x 64 with a bonus, 16 segments 12.6 / 10.2, 64 43 / 33.7; 32 heads, 1 segment 4.3 / 3.7.  Eight rows a lane: 19.8 -> 20.9, 33.7 -> 40.2.
+template <typename T, int CH, int MODE, bool HD, int R, bool ONCE>
+__global__ __launch_bounds__(256) void decay_step_kernel(float* __restrict__ o, const T* __restrict__ qkv, long stride,
+                                                         int q_col, int k_col, int v_col, const T* __restrict__ z,
+                                                         long z_stride, const float* __restrict__ z_bias,
+                                                         const float* __restrict__ a_log, float inv_tau, int dkind,
+                                                         const T* __restrict__ beta, long b_stride,
+                                                         const float* __restrict__ bonus,
+                                                         float* __restrict__ state, const int* __restrict__ cu,
+                                                         const int* __restrict__ ctx, const int* __restrict__ slot,
+                                                         int H, int Gk, int dk, int dv, float q_scale, int unit) {
+  constexpr int PW = 64 / CH, PB = 4 * PW * R;
+  __shared__ __attribute__((aligned(16))) float qs[8 * CH], ks[8 * CH], gs[HD ? 4 : 8 * CH];
+  const int s = blockIdx.x, h = blockIdx.y, sl = slot[s], t0 = cu[s], t1 = cu[s + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, chunk = lane % CH, j16 = lane & 15;
+  const int p0 = blockIdx.z * PB + wave * PW * R + lane / CH, inner = H * dv;  // rows p0 + PW r
+  if (sl < 0) {  // padding rows: defined output, no state
+    if (chunk == 0)
+      for (int t = t0; t < t1; ++t)
+        for (int r = 0; r < R; ++r)
+          if (p0 + PW * r < dv) o[(long)t * inner + (long)h * dv + p0 + PW * r] = 0.f;
+    return;
+  }
+  if (t1 <= t0) return;
+  const int n0 = chunk * 8, nc = min(n0, dk - 8), g = h / (H / Gk);  // channels beyond dk: the last ones again, nothing reads them
+  const bool live = n0 < dk;
+  float* sp = state + ((long)sl * H + h) * dv * dk + nc;
+  float S[R][8];
+  const bool carried = ctx[s] > 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int i = 0; i < 8; i += 4) {
+      const f32v4 v = load_state<ONCE>(sp + (long)min(p0 + PW * r, dv - 1) * dk + i);
+      S[r][i] = v[0]; S[r][i + 1] = v[1]; S[r][i + 2] = v[2]; S[r][i + 3] = v[3];
+    }
+  const float A = a_log != nullptr ? expf(a_log[h]) : 0.f;
+  for (int t = t0; t < t1; ++t) {
+    const T* row = qkv + (long)t * stride;
+    float v[R], gh = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = ldf(row + v_col + (long)h * dv + min(p0 + PW * r, dv - 1));
+    const float bt = MODE == kDelta ? sigmoid_f(ldf(beta + (long)t * b_stride + h)) : 0.f;
+    if (HD) gh = decay_f(ldf(z + (long)t * z_stride + h) + z_bias[h], dkind, A, inv_tau);
+    for (int n = threadIdx.x; n < dk; n += 256) {
+      qs[n] = ldf(row + q_col + (long)g * dk + n);
+      ks[n] = ldf(row + k_col + (long)g * dk + n);
+      if (!HD) gs[n] = decay_f(ldf(z + (long)t * z_stride + (long)h * dk + n) + z_bias[h * dk + n], dkind, A, inv_tau);
+    }
+    if (!carried && t == t0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) S[r][i] = 0.f;
+    }
+    __syncthreads();
+    float sq = 0.f, sk = 0.f;  // 16 lanes a row: unit norms, the query scale and k . q
+    if (unit) {
+      for (int n = j16; n < dk; n += 16) {
+        sq += qs[n] * qs[n];
+        sk += ks[n] * ks[n];
+      }
+      sq = lanes_sum<16>(sq);
+      sk = lanes_sum<16>(sk);
+    }
+    const float mq = unit ? q_scale / sqrtf(sq + 1e-6f) : q_scale;
+    const float mk = unit ? 1.0f / sqrtf(sk + 1e-6f) : 1.f;
+    float kq = 0.f;
+    for (int n = j16; n < dk; n += 16) {
+      const float qv = qs[n] * mq, kv = ks[n] * mk;
+      kq += MODE == kBonus ? qv * kv * bonus[g * dk + n] : qv * kv;
+    }
+    kq = lanes_sum<16>(kq);
+    float gv[8], kv[8], qv[8];
+    if (HD) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) gv[i] = gh;
+    } else {
+      load8(gs + nc, gv);
+    }
+    load8(ks + nc, kv);
+    load8(qs + nc, qv);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      kv[i] = live ? kv[i] * mk : 0.f;
+      qv[i] = live ? qv[i] * mq : 0.f;
+      gv[i] = live ? gv[i] : 0.f;
+    }
+    if (!live && t == t0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) S[r][i] = 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float y = scan_channels<CH, MODE>(S[r], gv, kv, qv, v[r], bt, kq);
+      if (chunk == 0 && p0 + PW * r < dv) o[(long)t * inner + (long)h * dv + p0 + PW * r] = y;
+    }
+    if (t + 1 < t1) __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (live && p0 + PW * r < dv) {
+#pragma unroll
+      for (int i = 0; i < 8; i += 4)
+        store_state<ONCE>(sp + (long)(p0 + PW * r) * dk + i, f32v4{S[r][i], S[r][i + 1], S[r][i + 2], S[r][i + 3]});
+    }
 }
 
 // ---- the two-launch form for prompts
@@ -453,11 +570,26 @@ struct ScanArgs {
   int unit;
   float* ws;
   long rows;
+  int step;
 };
 
 template <typename T, int CH, int MODE, bool HD>
 static void launch_scan_ch(const ScanArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)a.S, (unsigned)a.H, (unsigned)((a.dv + 256 / CH - 1) / (256 / CH)));
+  if (a.step) {
+    // four rows of the state a lane where that still gives each compute unit two workgroups
+    const bool once = 4l * a.S * a.H * a.dk * a.dv > kStateOnceBytes, four = (long)a.S * a.H * ((a.dv + 1024 / CH - 1) / (1024 / CH)) >= 512;
+    const dim3 sg((unsigned)a.S, (unsigned)a.H, (unsigned)(four ? (a.dv + 1024 / CH - 1) / (1024 / CH) : grid.z));
+#define K8SLLM_DSTEP(R, ONCE)                                                                                                \
+  hipLaunchKernelGGL((decay_step_kernel<T, CH, MODE, HD, R, ONCE>), sg, dim3(256), 0, s, a.o, (const T*)a.qkv, a.stride, a.q_col, \
+                     a.k_col, a.v_col, (const T*)a.z, a.z_stride, a.z_bias, a.a_log, a.inv_tau, a.dkind, (const T*)a.beta,     \
+                     a.b_stride, a.bonus, a.state, a.cu, a.ctx, a.slot, a.H, a.Gk, a.dk, a.dv, a.q_scale, a.unit)
+    if (!four) K8SLLM_DSTEP(1, false);
+    else if (once) K8SLLM_DSTEP(4, true);
+    else K8SLLM_DSTEP(4, false);
+#undef K8SLLM_DSTEP
+    return;
+  }
   if (a.ws == nullptr) {
     hipLaunchKernelGGL((decay_scan_kernel<T, CH, MODE, HD>), grid, dim3(256), 0, s, a.o, (const T*)a.qkv, a.stride, a.q_col,
                        a.k_col, a.v_col, (const T*)a.z, a.z_stride, a.z_bias, a.a_log, a.inv_tau, a.dkind,
@@ -504,17 +636,18 @@ long k8sllm_hy_decay_scan_ws(long T, int H, int Gk, int dk) { return T * ((long)
 // beta != nullptr: the delta rule; bonus != nullptr ([H][dk], Gk == H): the bonus form; neither: plain.
 // dkind: 0 exp(-exp(a_log) softplus(x)), 1 sigmoid(x)^(inv_tau), 2 exp(-exp(x)).  per_head: z and z_bias hold
 // one decay logit per head.  ws != nullptr: the two-launch form for prompts, with
-// k8sllm_hy_decay_scan_ws(T, ...) floats of workspace (T = rows of the step)
+// k8sllm_hy_decay_scan_ws(T, ...) floats of workspace (T = rows of the step); step: the step kernel where it applies
 int k8sllm_hy_decay_scan(float* o, const void* qkv, long stride, int q_col, int k_col, int v_col, const void* z,
                          long z_stride, const float* z_bias, const float* a_log, float inv_tau, int dkind, int per_head,
                          const void* beta, long b_stride, const float* bonus, float* state, const int* cu,
                          const int* ctx, const int* slot, int S, int H, int Gk, int dk, int dv, float q_scale, int unit,
-                         int f32, float* ws, long T, hipStream_t s) {
+                         int f32, float* ws, long T, int step, hipStream_t s) {
   if (S <= 0) return 0;
   if (Gk < 1 || H % Gk || dk < 1 || dv < 1 || dkind < 0 || dkind > 2 || (dkind == 0 && a_log == nullptr)) return -1;
   if (bonus != nullptr && (beta != nullptr || Gk != H)) return -1;
   const ScanArgs a = {o, qkv, stride, q_col, k_col, v_col, z, z_stride, z_bias, a_log, inv_tau, dkind, beta, b_stride, bonus,
-                      state, cu, ctx, slot, S, H, Gk, dk, dv, q_scale, unit, ws, T};
+                      state, cu, ctx, slot, S, H, Gk, dk, dv, q_scale, unit, ws, T,
+                      step && ws == nullptr && dk % 8 == 0 && reinterpret_cast<uintptr_t>(state) % 16 == 0};
   const int mode = beta != nullptr ? kDelta : bonus != nullptr ? kBonus : kPlain;
   return f32 ? launch_scan_t<float>(a, mode, per_head, s) : launch_scan_t<bf16_t>(a, mode, per_head, s);
 }

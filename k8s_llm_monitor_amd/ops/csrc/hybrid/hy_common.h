@@ -31,6 +31,16 @@ __device__ __forceinline__ void load8(const float* p, float* f) {
   f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
   f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
 }
+// 4 consecutive elements (8-byte aligned for bf16, 16-byte for fp32)
+__device__ __forceinline__ void load4(const bf16_t* p, float* f) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  f[0] = __uint_as_float(v.x << 16); f[1] = __uint_as_float(v.x & 0xffff0000u);
+  f[2] = __uint_as_float(v.y << 16); f[3] = __uint_as_float(v.y & 0xffff0000u);
+}
+__device__ __forceinline__ void load4(const float* p, float* f) {
+  const float4 a = *reinterpret_cast<const float4*>(p);
+  f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
+}
 __device__ __forceinline__ void store8(bf16_t* p, const float* f) { *reinterpret_cast<uint4*>(p) = pack8(f); }
 __device__ __forceinline__ void store8(float* p, const float* f) {
   *reinterpret_cast<float4*>(p) = make_float4(f[0], f[1], f[2], f[3]);
@@ -39,6 +49,21 @@ __device__ __forceinline__ void store8(float* p, const float* f) {
 __device__ __forceinline__ void load8_any(const void* p, int dt, long i, float* f) {
   if (dt == 2) load8(reinterpret_cast<const float*>(p) + i, f);
   else load8(reinterpret_cast<const bf16_t*>(p) + i, f);
+}
+
+// Four fp32 of a recurrent state; ONCE: non-temporal, where a step's states are more than the caches keep until the next step
+constexpr long kStateOnceBytes = 8l << 20;
+using f32v4 = float __attribute__((ext_vector_type(4)));
+template <bool ONCE>
+__device__ __forceinline__ f32v4 load_state(const float* p) {
+  const f32v4* q = reinterpret_cast<const f32v4*>(p);
+  return ONCE ? __builtin_nontemporal_load(q) : *q;
+}
+template <bool ONCE>
+__device__ __forceinline__ void store_state(float* p, f32v4 v) {
+  f32v4* q = reinterpret_cast<f32v4*>(p);
+  if (ONCE) __builtin_nontemporal_store(v, q);
+  else *q = v;
 }
 
 // Eight 16-bit values of tokens j .. j + 7, zero where not (j < end): what lies behind a sequence's last token in its last page is

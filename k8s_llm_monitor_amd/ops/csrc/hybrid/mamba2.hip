@@ -202,6 +202,13 @@ __global__ __launch_bounds__(256) void conv_state_step_kernel(T* __restrict__ st
   for (int i = 0; i < H; ++i) st[(long)i * C] = keep[i];
 }
 
+// State 4 i + j behind a token.  Which of the two products is rounded before they meet is the choice that a compiler once made, spelled out:
+// a decode step's bits decide near ties of routers behind it.
+template <int NPT>
+__device__ __forceinline__ float next_state(int j, float dA, float S, float dtx, float b) {
+  return NPT == 4 || (NPT < 64 && j == 0) ? fmaf(dA, S, dtx * b) : fmaf(dtx, b, dA * S);
+}
+
 // Workgroup = 4 waves = 64 values of p for one (segment, head); in a wave lanes are (p % 16,
 // chunk = lane / 16): chunk k holds states n in [k * NPT, (k + 1) * NPT) of its p in registers, and
 // the 4 partial sums of y meet through two xor-shuffles.  The inputs of 16 tokens at a time (B, C
@@ -290,10 +297,10 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(float* __restrict__ y, co
 #pragma unroll
       for (int i = 0; i < NPT / 4; ++i) {
         const float4 bv = bp[i], cv = cp[i];
-        S[4 * i + 0] = dA * S[4 * i + 0] + dtx * bv.x;
-        S[4 * i + 1] = dA * S[4 * i + 1] + dtx * bv.y;
-        S[4 * i + 2] = dA * S[4 * i + 2] + dtx * bv.z;
-        S[4 * i + 3] = dA * S[4 * i + 3] + dtx * bv.w;
+        S[4 * i + 0] = next_state<NPT>(0, dA, S[4 * i + 0], dtx, bv.x);
+        S[4 * i + 1] = next_state<NPT>(1, dA, S[4 * i + 1], dtx, bv.y);
+        S[4 * i + 2] = next_state<NPT>(2, dA, S[4 * i + 2], dtx, bv.z);
+        S[4 * i + 3] = next_state<NPT>(3, dA, S[4 * i + 3], dtx, bv.w);
         acc += S[4 * i + 0] * cv.x + S[4 * i + 1] * cv.y + S[4 * i + 2] * cv.z + S[4 * i + 3] * cv.w;
       }
       acc = xor32_sum_f(xor16_sum(acc));
@@ -304,6 +311,101 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(float* __restrict__ y, co
 #pragma unroll
     for (int i = 0; i < NPT; ++i)
       if (n0 + i < N) sp[(long)(n0 + i) * P] = S[i];
+  }
+}
+
+// Steps of one token a segment (decode): a pass over the states.  A workgroup takes 64 values of p of one (segment, head); a thread
+// holds four of them for every sixteenth group of four states, so that rows of the state are read and written 256 bytes at a time, and all of its
+// loads are on their way before anything waits.  Groups' sums meet in LDS in the order of ssm_scan_kernel: the same bits.  That kernel's 4-byte
+// accesses met 64 bytes of a row, behind the staging of tiles of 16 tokens.
+// us, ssm_scan_kernel / here: 64 heads of 64 x 128, 1 segment 9.5 / 4.6, 16 22.6 / 14.5, 64 75.7 / 49.0 (5.5 TB/s), 128 129 / 98;
+// 16 heads of 128 x 128 with a fixed decay, 1 segment 8.4 / 3.6, 32 19.5 / 14.1; 64 of them 40.2 / 26.8.  States above 8 MB of a step are
+// non-temporal: at 34 MB 18.6 / 14.5.
+template <typename T, int NPT, bool ONCE>
+__global__ __launch_bounds__(256) void ssm_step_kernel(float* __restrict__ y, const T* __restrict__ xbc, const T* __restrict__ proj,
+                                                       long p_stride, int dt_col, const float* __restrict__ dt_bias,
+                                                       const float* __restrict__ a_log, const float* __restrict__ d_skip,
+                                                       const float* __restrict__ decay, float* __restrict__ state,
+                                                       const int* __restrict__ cu, const int* __restrict__ ctx,
+                                                       const int* __restrict__ slot, int nh, int P, int N, int G) {
+  constexpr int GPT = NPT <= 16 ? 1 : NPT / 16;  // groups of a thread
+  __shared__ __attribute__((aligned(16))) float part[16 * GPT][68];
+  const int s = blockIdx.x, h = blockIdx.y, sl = slot[s], t0 = cu[s], t1 = cu[s + 1];
+  const int lane = threadIdx.x & 63, tg = threadIdx.x >> 4, p4 = blockIdx.z * 64 + 4 * (threadIdx.x & 15);
+  const int chunk = lane >> 4, pl = (threadIdx.x >> 6) * 16 + (lane & 15), p = blockIdx.z * 64 + pl;  // as in ssm_scan_kernel
+  if (sl < 0) {  // padding rows: defined output, no state
+    if (p < P && lane < 16)
+      for (int t = t0; t < t1; ++t) y[(long)t * nh * P + (long)h * P + p] = 0.f;
+    return;
+  }
+  if (t1 <= t0) return;
+  const int inner = nh * P, C = inner + 2 * G * N, g = h / (nh / G), pc = min(p4, P - 4);
+  float* sp = state + ((long)sl * nh + h) * N * P + pc;
+  int n[GPT];
+#pragma unroll
+  for (int i = 0; i < GPT; ++i) n[i] = min(4 * (tg + 16 * i), N - 4);  // groups behind the last repeat it, and nothing reads them
+  f32v4 S[GPT][4];
+  const bool carried = ctx[s] > 0;
+#pragma unroll
+  for (int i = 0; i < GPT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) S[i][j] = load_state<ONCE>(sp + (long)(n[i] + j) * P);
+  const bool fixed = decay != nullptr;
+  const float A = fixed ? 0.f : expf(a_log[h]), Dh = fixed ? 0.f : d_skip[h], bias = fixed ? 0.f : dt_bias[h];
+  for (int t = t0; t < t1; ++t) {
+    const T* row = xbc + (long)t * C;
+    float x[4], b[GPT][4], c[GPT][4];
+    load4(row + (long)h * P + pc, x);
+#pragma unroll
+    for (int i = 0; i < GPT; ++i) {
+      load4(row + inner + (long)g * N + n[i], b[i]);
+      load4(row + inner + (long)(G + g) * N + n[i], c[i]);
+    }
+    const float xl = ldf(row + (long)h * P + min(p, P - 1));
+    float dt = 1.f, dA;
+    if (fixed) {
+      dA = decay[h];
+    } else {
+      const float raw = ldf(proj + (long)t * p_stride + dt_col + h) + bias;
+      dt = raw > 20.f ? raw : log1pf(expf(raw));
+      dA = expf(-A * dt);
+    }
+    if (t == t0 && !carried) {
+#pragma unroll
+      for (int i = 0; i < GPT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[i][j] = f32v4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < GPT; ++i) {
+      f32v4 sum;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float dtx = dt * x[v];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[i][j][v] = next_state<NPT>(j, dA, S[i][j][v], dtx, b[i][j]);
+        sum[v] = fmaf(S[i][3][v], c[i][3], fmaf(S[i][2][v], c[i][2], fmaf(S[i][0][v], c[i][0], S[i][1][v] * c[i][1])));
+      }
+      *reinterpret_cast<f32v4*>(&part[tg + 16 * i][4 * (threadIdx.x & 15)]) = sum;
+    }
+    __syncthreads();
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < NPT / 4; ++i) {
+      const int q = chunk * (NPT / 4) + i;
+      acc += 4 * q < N ? part[q][pl] : 0.f;
+    }
+    acc = xor32_sum_f(xor16_sum(acc));
+    if (p < P && lane < 16) y[(long)t * inner + (long)h * P + p] = fmaf(Dh, xl, acc);
+    if (t + 1 < t1) __syncthreads();
+  }
+  if (p4 < P) {
+#pragma unroll
+    for (int i = 0; i < GPT; ++i)
+      if (4 * (tg + 16 * i) < N) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) store_state<ONCE>(sp + (long)(n[i] + j) * P, S[i][j]);
+      }
   }
 }
 
@@ -666,7 +768,7 @@ using namespace k8sllm;
 template <typename T>
 static int launch_scan(float* y, const void* xbc, const void* proj, long p_stride, int dt_col, const float* dt_bias,
                        const float* a_log, const float* d_skip, const float* decay, float* state, const int* cu, const int* ctx,
-                       const int* slot, int S, int nh, int P, int N, int G, int wide, hipStream_t s) {
+                       const int* slot, int S, int nh, int P, int N, int G, int wide, int step, hipStream_t s) {
   if (wide && N > 8) {  // long segments: 8 states per lane
     const int vec = N % 8 == 0 && (nh * P) % 8 == 0 && reinterpret_cast<uintptr_t>(xbc) % 16 == 0;
     // the tile form wants 16-byte rows of B and C and 4 values of p at a time; below 33 states half its products would be padding
@@ -697,6 +799,22 @@ static int launch_scan(float* y, const void* xbc, const void* proj, long p_strid
     return (int)hipGetLastError();
   }
   const dim3 grid((unsigned)S, (unsigned)nh, (unsigned)((P + 63) / 64));
+  // one token a segment, rows that the step kernel can read four values at a time
+  if (step && P % 4 == 0 && N % 4 == 0 && N <= 256 && reinterpret_cast<uintptr_t>(state) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(xbc) % (4 * sizeof(T)) == 0) {
+    const bool once = 4l * S * nh * N * P > kStateOnceBytes;
+#define K8SLLM_STEP(NPT)                                                                                                 \
+  hipLaunchKernelGGL((once ? &ssm_step_kernel<T, NPT, true> : &ssm_step_kernel<T, NPT, false>), grid, dim3(256), 0, s, y,  \
+                     (const T*)xbc, (const T*)proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot, nh, \
+                     P, N, G)
+    if (N <= 16) K8SLLM_STEP(4);
+    else if (N <= 32) K8SLLM_STEP(8);
+    else if (N <= 64) K8SLLM_STEP(16);
+    else if (N <= 128) K8SLLM_STEP(32);
+    else K8SLLM_STEP(64);
+#undef K8SLLM_STEP
+    return (int)hipGetLastError();
+  }
 #define K8SLLM_SCAN(NPT)                                                                                              \
   hipLaunchKernelGGL((ssm_scan_kernel<T, NPT>), grid, dim3(256), 0, s, y, (const T*)xbc, (const T*)proj, p_stride,    \
                      dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot, nh, P, N, G)
@@ -750,12 +868,12 @@ int k8sllm_hy_ssm_scan(float* y, const void* xbc, const void* proj, long p_strid
                        const int* slot, int S, long T, int nh, int P, int N, int G, int f32, int mode, hipStream_t s) {
   if (S <= 0) return 0;
   if (G < 1 || nh % G) return -1;
-  // mode 0: by the step's mean segment length (prompts: the thin mapping); 1 / 2: forced (tests)
-  const int wide = mode == 2 || (mode == 0 && T >= 32L * S);
+  // mode 0: by the step's mean segment length (prompts: the thin mapping; one token each: the step kernel); 1 / 2: forced (tests)
+  const int wide = mode == 2 || (mode == 0 && T >= 32L * S), step = mode == 0 && T <= S;
   if (decay == nullptr && (proj == nullptr || dt_bias == nullptr || a_log == nullptr || d_skip == nullptr)) return -1;
   return f32 ? launch_scan<float>(y, xbc, proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot,
-                                  S, nh, P, N, G, wide, s)
+                                  S, nh, P, N, G, wide, step, s)
              : launch_scan<bf16_t>(y, xbc, proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot,
-                                   S, nh, P, N, G, wide, s);
+                                   S, nh, P, N, G, wide, step, s);
 }
 }

@@ -806,7 +806,7 @@ def ssm_scan(xbc: torch.Tensor, proj: Optional[torch.Tensor], dt_col: int, dt_bi
     back at its end.  Returns y [T, nh*P] fp32.
 
     GPU: two lane mappings of the same arithmetic, chosen by the step's mean segment length (``mode`` 1 / 2 forces the
-    decode / the prompt one).
+    decode / the prompt one); steps of one token a segment take a pass over the states, with the decode mapping's bits.
 
     ``decay`` [nh] fp32 (then ``proj``, ``dt_bias``, ``a_log``, ``d_skip`` are not read): the
     recurrence with a fixed decay per head, step size 1 and no skip term,
@@ -897,7 +897,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
 
     GPU: steps of prompts (a mean segment length of 32 rows or more, or a ``longest`` segment of 256) run as two launches - everything
     that does not depend on the state (decays, unit norms, k . q, beta) for all rows at once into a
-    workspace, then the recurrence over it; decode steps run as one launch.  bf16 prompts of the delta rule with one decay
+    workspace, then the recurrence over it; decode steps run as one launch, of one token a segment as a pass over the states.  bf16 prompts of the delta rule with one decay
     per head, and without the delta rule and unit norms of decays per channel (``dk`` a multiple of 32 up to 128, ``dv`` of
     16), go in chunks of 64 tokens on the matrix cores, fp32 operands as three bf16 parts that add up to them, and the first
     ``singles`` segments, running sequences' next tokens, beside them as in a decode step: their bits do not depend on what else
@@ -966,7 +966,7 @@ def selective_scan(xc: torch.Tensor, q: torch.Tensor, b_col: int, c_col: int, dt
     ``xc`` [T, C] (contiguous), ``dt`` [T, C] (a projection), B and C: columns ``b_col`` / ``c_col`` .. of ``q``
     (N each); ``state`` [slots, C, N] fp32 is read at the segment's start (zero where seg_ctx is 0) and
     written back at its end.  ``longest``: rows of the longest segment (0: not known); ``mode``
-    (device only): 0 whole segments or spans of tokens side by side, by the sizes, 1 whole, 2 spans.  Returns out [T, C] in the activation dtype."""
+    (device only): 0 whole segments (of one token each: a pass over the states) or spans of tokens side by side, by the sizes, 1 whole, 2 spans.  Returns out [T, C] in the activation dtype."""
     T, C = xc.shape
     N = a_log.shape[1]
     if not xc.is_cuda:

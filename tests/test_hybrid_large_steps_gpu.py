@@ -551,6 +551,77 @@ def test_few_rows_and_experts_in_lines(M, K):
     assert bool(((y.double() - z).abs() <= 2 ** -8 * z.abs() + 1e-6 * K ** 0.5).all())
 
 
+def _singles(g, n):
+    """Segments, cached tokens and slots of a decode step: a fresh sequence, a padding row and, at last, no token beside two of one sequence."""
+    ctx = torch.randint(1, 900, (n,), generator=g)
+    slot = torch.randperm(n + 2, generator=g)[:n]
+    ctx[0], slot[1] = 0, -1
+    cu = torch.arange(n + 1)
+    cu[n - 2 + 1] = cu[n - 2]
+    return _i32(cu.tolist()).cuda(), _i32(ctx.tolist()).cuda(), _i32(slot.tolist()).cuda()
+
+
+def _same_step(f, state):
+    """The step kernel (mode 0) and the scan (mode 1): the same results and states, whatever a slot held that starts fresh."""
+    state[:] = torch.where(torch.rand(state.shape[0], device="cuda").view(-1, *[1] * (state.dim() - 1)) < 0.2, float("nan"), state)
+    a, b = state.clone(), state.clone()
+    ya, yb = f(a, 0), f(b, 1)
+    torch.testing.assert_close(ya, yb, rtol=0, atol=0, equal_nan=True)
+    torch.testing.assert_close(a, b, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+@pytest.mark.parametrize("n", [3, 66])
+@pytest.mark.parametrize("nh,P,N,G", [(4, 64, 128, 1), (2, 100, 16, 2), (6, 4, 36, 3), (2, 128, 256, 1), (3, 72, 100, 3), (256, 64, 128, 1)])
+def test_one_token_a_segment_ssm(n, nh, P, N, G, dt):
+    """Decode steps of the Mamba-2 recurrence: values and states around the workgroup's 64 and the groups of four, every sum as in the scan."""
+    if nh * n > 1000 and dt == torch.float32:
+        pytest.skip("the largest states once")
+    g = _g(78)
+    cu, ctx, slot = _singles(g, n)
+    C = nh * P + 2 * G * N
+    x, proj, par = _r(g, n, C, dt=dt).cuda(), _r(g, n, nh + 3, dt=dt).cuda(), [_r(g, nh).cuda() for _ in range(3)]
+    state = _r(g, n + 2, nh, N, P).cuda()
+    _same_step(lambda s, mode: hops.ssm_scan(x, proj, 3, *par, s, cu, ctx, slot, nh, P, N, G, mode=mode), state)
+    if G == nh or G == 1:
+        xx = _r(g, n, nh * P + 2 * nh * N, dt=dt).cuda()
+        dec = torch.rand(nh, generator=g).cuda()
+        _same_step(lambda s, mode: hops.linear_attention(xx, dec, s, cu, ctx, slot, nh, N, P, mode=mode), state)
+
+
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+@pytest.mark.parametrize("n,H,Gk,dk,dv", [(3, 4, 2, 128, 128), (40, 16, 16, 64, 64), (24, 40, 20, 128, 128), (5, 2, 1, 96, 20), (30, 32, 32, 8, 300),
+                                          (9, 16, 16, 256, 72), (130, 32, 32, 64, 64)])
+def test_one_token_a_segment_decay(n, H, Gk, dk, dv, dt):
+    """Decode steps of the recurrences with decays, one and four rows of the state a lane: the delta rule with decays per channel and per
+    head, plain, with a bonus; every sum as in the scan."""
+    g = _g(79)
+    cu, ctx, slot = _singles(g, n)
+    cols = 2 * Gk * dk + H * dv
+    x, z, beta = _r(g, n, cols + 8, dt=dt).cuda(), _r(g, n, H * dk, dt=dt).cuda(), _r(g, n, H, dt=dt).cuda()
+    zb, al, state = _r(g, H * dk).cuda(), _r(g, H).cuda(), _r(g, n + 2, H, dv, dk).cuda()
+    args = (x, 0, Gk * dk, 2 * Gk * dk)
+
+    def run(zz, bias, **kw):
+        _same_step(lambda s, mode: hops.decay_scan(*args, zz, bias, s, cu, ctx, slot, H, Gk, dk, dv, dk ** -0.5, mode=mode, **kw), state)
+
+    run(z, zb, a_log=al, beta=beta, unit=True)
+    run(z[:, :H].contiguous(), zb[:H].contiguous(), a_log=al, beta=beta, unit=True)
+    run(z, zb, tau=16.0)
+    if Gk == H:
+        run(z, zb, decay="exp_exp", bonus=_r(g, H, dk).cuda())
+
+
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+@pytest.mark.parametrize("n,C,N", [(3, 70, 16), (24, 1000, 16), (5, 33, 4), (4, 65, 8), (6, 100, 24), (5, 40, 64), (3, 20, 256), (70, 8192, 16)])
+def test_one_token_a_segment_selective(n, C, N, dt):
+    g = _g(80)
+    cu, ctx, slot = _singles(g, n)
+    xc, q, d, proj = (_r(g, n, w, dt=dt).cuda() for w in (C, 2 * N + 5, C, 2 * C))
+    par = (_r(g, C).cuda(), _r(g, C, N).cuda(), _r(g, C).cuda())
+    _same_step(lambda s, mode: hops.selective_scan(xc, q, 5, 5 + N, d, *par, proj, C, s, cu, ctx, slot, mode=mode), _r(g, n + 2, C, N).cuda())
+
+
 @pytest.mark.parametrize("M", [1, 257, 600])
 @pytest.mark.parametrize("f,rest,K", [(128, 0, 192), (144, 48, 256), (400, 272, 320), (16, 256, 192)])  # tiles of 128 features and 256 columns
 @pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
