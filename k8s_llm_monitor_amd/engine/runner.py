@@ -212,7 +212,7 @@ class ModelRunner:
             seen[w] = first, n, list(accumulate(n))
         sizes = dict(ids=T, pos=T, slots=T, cu=len(seqs) + 1, qs=nq, st=nq, lidx=nl, temp=R, topk=R, topp=R,
                      gcu=hy + 1 if hy else 0, gctx=hy, gslot=hy,
-                     cst=len(seqs) if paged else 0, bt=len(seqs) * W, dbt=nd * Wd, dlen=nd,
+                     cst=len(seqs) if paged else 0, cend=len(seqs) if hy else 0, bt=len(seqs) * W, dbt=nd * Wd, dlen=nd,
                      mcu=len(seqs) + 2 if kA else 0, mqs=nq if kA else 0, mst=nq if kA else 0,
                      mlidx=len(seqs) if kA else 0)
         for w, (_, _, ends) in seen.items():
@@ -254,6 +254,7 @@ class ModelRunner:
             v["gctx"][:nd] = [q.num_tokens - 1 for q in decode]
             v["gctx"][nd:] = starts
             v["gslot"][:] = [getattr(q, "state_slot", -1) for q in rows]
+            v["cend"][:] = np.asarray(starts, dtype=np.int32) + np.asarray(lens, dtype=np.int32)
         v["temp"].view(np.float32)[:] = [s.params.temperature for s in rows]
         v["topk"][:] = [s.params.top_k for s in rows]
         v["topp"].view(np.float32)[:] = [s.params.top_p for s in rows]
@@ -297,6 +298,9 @@ class ModelRunner:
         if hy:
             meta.seg_cu, meta.seg_ctx, meta.seg_slot = dv["gcu"], dv["gctx"], dv["gslot"]
             meta.seg_max = max([1] * (nd > 0) + lens)
+            if logit_rows is None:
+                meta.ends = dv["cend"]
+                meta.logits_span = (T - 1, T) if R == 1 else None
             if seen:
                 meta.chunk_rows = cu
                 meta.page_lists = {w: PageList(dv[f"pgl{w}"], dv[f"pgb{w}"].view(len(seqs), W), ends, max(n))

@@ -111,6 +111,27 @@ class _Params:
         return t.to(torch.bfloat16).to(self.device, dt).contiguous()  # values a bf16 checkpoint could hold
 
 
+def _take(rows, *ts: torch.Tensor) -> tuple:
+    """These rows (a tensor of them or a slice) of each; None: all.  Rows of 16-bit projections stay a multiple of 16 bytes apart, as the
+    kernels' accesses want them."""
+    def some(t: torch.Tensor) -> torch.Tensor:
+        if isinstance(rows, slice):
+            return t[rows]
+        r = t.index_select(0, rows)
+        return F.pad(r, (0, -r.shape[1] % 8))[:, :r.shape[1]] if r.dim() == 2 and r.shape[1] % 8 else r
+
+    return ts if rows is None else tuple(some(t) for t in ts)
+
+
+def _attend_ends(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, meta: AttnMeta, *args, gate: Optional[torch.Tensor] = None,
+                 **kw) -> torch.Tensor:
+    """Windowed attention of a prefill step's decode rows and each chunk's last row (``q``, in that order) as decode rows."""
+    nd = meta.num_decode
+    parts = [hops.window_attention_decode(q[a:b], kc, vc, bt, n, *args, gate=gate[a:b] if gate is not None else None, **kw)
+             for a, b, bt, n in ((0, nd, meta.dec_block_tables, meta.dec_seq_lens), (nd, q.shape[0], meta.block_tables, meta.ends)) if b > a]
+    return parts[0] if len(parts) == 1 else torch.cat(parts)
+
+
 class WindowAttention:
     """Grouped-query attention with a whole-projection RMSNorm of q and of k, no positional
     rotation, a sliding window of ``mask.size`` keys (0 / absent: unbounded) and a softmax sink."""
@@ -144,7 +165,7 @@ class WindowAttention:
         """(bytes per page, bytes per state slot)."""
         return BLOCK * self.G * (self.dk + self.dv) * esize, 0
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> torch.Tensor:
         H, G, dk, dv = self.H, self.G, self.dk, self.dv
         qkv = F.linear(h, self.wqkv)
         kc, vc = cache["k"], cache["v"]
@@ -152,6 +173,8 @@ class WindowAttention:
         args = (H, G, dk, dv, self.scale, self.window, self.sink)
         if not meta.is_prefill:
             o = hops.window_attention_decode(qkv, kc, vc, meta.block_tables, meta.seq_lens, *args, vec=bool(self.fast))
+        elif rows is not None and meta.ends is not None:
+            o = _attend_ends(*_take(rows, qkv), kc, vc, meta, *args, vec=bool(self.fast))
         else:
             nd = meta.num_decode
             # mfma 2: the register kernel.  The staged one (201 -> 88 us at 4 x 2048 rows, 16 heads) rounds the weights against
@@ -163,6 +186,7 @@ class WindowAttention:
                 od = hops.window_attention_decode(qkv[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
                                                   vec=bool(self.fast))
                 o = torch.cat([od, o])
+            (o,) = _take(rows, o)
         return F.linear(o, self.wo)
 
 
@@ -200,12 +224,13 @@ class Mamba2Mixer:
     def cache_bytes(self, esize: int) -> tuple:
         return 0, (self.taps - 1) * self.C * esize + self.nh * self.N * self.P * 4
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> torch.Tensor:
         proj = F.linear(h, self.w_in)
         seg = (meta.seg_cu, meta.seg_ctx, meta.seg_slot)
         xbc = hops.conv_silu(proj, self.inner, self.C, self.conv_w, self.conv_b, cache["conv"], *seg)
         y = hops.ssm_scan(xbc, proj, self.inner + self.C, self.dt_bias, self.a_log, self.d_skip, cache["ssm"], *seg,
                           self.nh, self.P, self.N, self.G)
+        y, proj = _take(rows, y, proj)
         g = hops.gated_group_norm(y, proj, 0, self.norm_w, self.eps, self.ng, h.dtype)
         return F.linear(g, self.wo)
 
@@ -306,53 +331,55 @@ class LatentAttention:
     def cache_bytes(self, esize: int) -> tuple:
         return (0 if self.kv_from is not None else BLOCK * (self.pitch + self.R) * esize), 0
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> torch.Tensor:
         H, dn, dr, dv, Q, R = self.H, self.dn, self.dr, self.dv, self.Q, self.R
-        T = h.shape[0]
+        own = self.kv_from is None
+        pos = meta.positions
+        ends = rows is not None and meta.ends is not None
+        if ends and not own:  # nothing of the other rows goes to pages
+            h, pos = _take(rows, h, pos)
         proj = down = hops.linear(h, self.w_down)
-        if self.n_tail:
-            self.tail_out = (proj, self.n_in)
+        kc, vc = cache["k"], cache["v"]
         if proj.shape[1] > self.n_down:
             down = proj[:, :self.n_down]
-        gate = proj[:, self.n_down:self.n_in] if self.has_gate else None
-        kc, vc = cache["k"], cache["v"]
-        own = self.kv_from is None
-        hops.latent_prep(down, Q, R, dr, self.qn, self.kn, self.eps, meta.positions, self.freq,
+        hops.latent_prep(down, Q, R, dr, self.qn, self.kn, self.eps, pos, self.freq,
                          kc if own else None, vc if own else None, meta.slot_mapping if own else None, pairs=self.pairs)
+        if ends and own:
+            proj, pos = _take(rows, proj, pos)
+            down = proj[:, :self.n_down]
+        gate = proj[:, self.n_down:self.n_in] if self.has_gate else None
         q = hops.linear(down[:, :Q], self.w_uq)
-        ex = self._expand_ok(h, meta)
+        T = q.shape[0]
+        ex = not ends and self._expand_ok(h, meta)
         nd = meta.num_decode if meta.is_prefill else T  # single-token rows in front
         parts = []
         if nd or not ex:
             n = nd if ex else T
-            parts.append(self._forward_latent(q[:n], meta, kc, vc, gate[:n] if gate is not None else None, not ex))
+            # (first row, end, pages, whose positions they see) of attention over the latent pages
+            runs = [(0, T, meta.block_tables, dict(seq_lens=meta.seq_lens))] if not meta.is_prefill else [
+                (0, nd, meta.dec_block_tables, dict(seq_lens=meta.dec_seq_lens)),
+                (nd, n, meta.block_tables, dict(seq_lens=meta.ends) if ends else dict(cu=meta.cu_seqlens, ctx=meta.ctx_start))]
+            parts.append(self._forward_latent(q[:n], pos, kc, vc, gate, [r for r in runs if r[1] > r[0]]))
         if ex:
             parts.append(self._forward_expanded(q[nd:], meta, kc, gate[nd:] if gate is not None else None))
-        return hops.linear(parts[0] if len(parts) == 1 else torch.cat(parts), self.wo)
+        o = parts[0] if len(parts) == 1 else torch.cat(parts)
+        if rows is not None and not ends:
+            o, proj = _take(rows, o, proj)
+        if self.n_tail:
+            self.tail_out = (proj, self.n_in)
+        return hops.linear(o, self.wo)
 
-    def _forward_latent(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
-                        chunks: bool) -> torch.Tensor:
-        """Attention over the latent pages: the step's single-token rows and, with ``chunks``, its prompt rows."""
+    def _forward_latent(self, q: torch.Tensor, pos: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
+                        runs: list) -> torch.Tensor:
+        """Attention over the latent pages: rows ``q``, in ``runs`` of (first row, end, their pages, what they see of them)."""
         H, dn, dr, dv, R = self.H, self.dn, self.dr, self.dv, self.R
         T = q.shape[0]
         # the per-head key expansion moved to the query: q_lat[h] = q_unrotated[h] @ W_uk[h]  ([H, T, R])
         q_lat = torch.bmm(q.view(T, H, dn + dr)[:, :, :dn].transpose(0, 1), self.w_uk.view(H, dn, R))
-        qa = hops.latent_queries(q, q_lat, H, dn, dr, meta.positions, self.freq, self.pitch, pairs=self.pairs)
-        args = (H, self.scale, self.window, self.sinks)
-        kw = dict(fast=self.fast, sink=self.sink)
-        if not meta.is_prefill:
-            o = hops.latent_attention(qa, kc, vc, meta.block_tables, *args, seq_lens=meta.seq_lens, gate=gate, **kw)
-        else:
-            nd = meta.num_decode
-            gc, gd = (gate[nd:], gate[:nd]) if gate is not None else (None, None)
-            parts = []
-            if nd:
-                parts.append(hops.latent_attention(qa[:nd], kc, vc, meta.dec_block_tables, *args, seq_lens=meta.dec_seq_lens,
-                                                   gate=gd, **kw))
-            if chunks:
-                parts.append(hops.latent_attention(qa[nd:], kc, vc, meta.block_tables, *args, cu=meta.cu_seqlens,
-                                                   ctx=meta.ctx_start, gate=gc, **kw))
-            o = parts[0] if len(parts) == 1 else torch.cat(parts)
+        qa = hops.latent_queries(q, q_lat, H, dn, dr, pos, self.freq, self.pitch, pairs=self.pairs)
+        parts = [hops.latent_attention(qa[a:b], kc, vc, tables, H, self.scale, self.window, self.sinks, fast=self.fast, sink=self.sink,
+                                       gate=gate[a:b] if gate is not None else None, **seen) for a, b, tables, seen in runs]
+        o = parts[0] if len(parts) == 1 else torch.cat(parts)
         # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T, written head by head
         # into the rows the out-projection reads
         v = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
@@ -485,12 +512,11 @@ class RotaryAttention:
     def cache_bytes(self, esize: int) -> tuple:
         return BLOCK * self.G * (self.dk + self.dv) * esize, 0
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None,
+                rows=None) -> torch.Tensor:
         H, G, dk, dv = self.H, self.G, self.dk, self.dv
         if proj is None:
             proj = hops.linear(h, self.w_in)
-        if self.n_tail:
-            self.tail_out = (proj, self.n_in)
         kc, vc = cache["k"], cache["v"]
         hops.rotary_cache(proj, H, G, dk, dv, meta.positions, self.freq, self.pairs, self.temp, kc, vc, meta.slot_mapping,
                           norm=self.norm, qw=self.qn, kw=self.kn, eps=self.eps, v_from_k=self.v_from_k)
@@ -500,6 +526,9 @@ class RotaryAttention:
         if not meta.is_prefill:
             o = hops.window_attention_decode(proj, kc, vc, meta.block_tables, meta.seq_lens, *args, vec=bool(self.fast),
                                              gate=proj if hg else None, **kw)
+        elif rows is not None and meta.ends is not None:
+            (proj,) = _take(rows, proj)
+            o = _attend_ends(proj, kc, vc, meta, *args, vec=bool(self.fast), gate=proj if hg else None, **kw)
         else:
             nd = meta.num_decode
             o = hops.window_attention_prefill(proj[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
@@ -508,6 +537,9 @@ class RotaryAttention:
                 od = hops.window_attention_decode(proj[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
                                                   vec=bool(self.fast), gate=proj[:nd] if hg else None, **kw)
                 o = torch.cat([od, o])
+            o, proj = _take(rows, o, proj)
+        if self.n_tail:
+            self.tail_out = (proj, self.n_in)
         if self.has_gate and not hg:
             o = hops.sigmoid_gate(o, proj, self.g_col)
         return hops.linear(o, self.wo)
@@ -567,13 +599,14 @@ class LightningMixer:
     def cache_bytes(self, esize: int) -> tuple:
         return 0, self.H * self.dk * self.dv * 4
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> torch.Tensor:
         proj = hops.linear(h, self.w_in)
-        if self.n_tail:
-            self.tail_out = (proj, self.n_in)
         vkq = hops.activation_cols(proj, 0, self.n_act, "silu")
         o = hops.linear_attention(vkq, self.decay, cache["state"], meta.seg_cu, meta.seg_ctx, meta.seg_slot,
                                   self.H, self.dk, self.dv, longest=meta.seg_max, singles=meta.num_decode)
+        o, proj = _take(rows, o, proj)
+        if self.n_tail:
+            self.tail_out = (proj, self.n_in)
         g = hops.gated_group_norm(o, proj, self.n_act, self.norm_w, self.eps, 1, h.dtype, after=True)
         return hops.linear(g, self.wo)
 
@@ -645,7 +678,8 @@ class GatedDeltaMixer:
     def cache_bytes(self, esize: int) -> tuple:
         return 0, (self.taps - 1) * self.C * esize + self.H * self.dk * self.dv * 4
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None,
+                rows=None) -> torch.Tensor:
         H, Gk, dk, dv = self.H, self.Gk, self.dk, self.dv
         if proj is None:
             proj = hops.linear(h, self.w_in)
@@ -655,6 +689,7 @@ class GatedDeltaMixer:
         o = hops.decay_scan(qkv, 0, Gk * dk, 2 * Gk * dk, z, self.dt_bias, cache["state"], *seg, H, Gk, dk, dv,
                             dk ** -0.5, a_log=self.a_log, beta=proj, beta_col=self.b_col, unit=True, z_col=z_col,
                             longest=meta.seg_max, singles=meta.num_decode)
+        o, proj = _take(rows, o, proj)
         if self.low_rank_gate:
             gate = hops.linear(proj[:, self.g_col:self.g_col + self.rg], self.wg2)
             g = hops.gated_group_norm(o, gate, 0, self.norm_all, self.eps, H, h.dtype, after=True)
@@ -708,13 +743,15 @@ class GatedLinearMixer:
     def cache_bytes(self, esize: int) -> tuple:
         return 0, self.H * self.dk * self.dv * 4
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, proj: Optional[torch.Tensor] = None,
+                rows=None) -> torch.Tensor:
         H, dk, dv = self.H, self.dk, self.dv
         if proj is None:
             proj = hops.linear(h, self.w_in)
         z = hops.linear(proj[:, self.a_col:self.a_col + self.ra], self.wa2)
         o = hops.decay_scan(proj, 0, H * dk, 2 * H * dk, z, self.a_bias, cache["state"], meta.seg_cu, meta.seg_ctx,
                             meta.seg_slot, H, H, dk, dv, dk ** -0.5, tau=self.tau, longest=meta.seg_max, singles=meta.num_decode)
+        o, proj = _take(rows, o, proj)
         g = hops.gated_group_norm(o, proj, self.g_col, self.norm_all, self.eps, H, h.dtype, after=True, gate="silu")
         return hops.linear(g, self.wo)
 
@@ -759,7 +796,7 @@ class Mamba1Mixer:
     def cache_bytes(self, esize: int) -> tuple:
         return 0, (self.taps - 1) * self.inner * esize + self.inner * self.N * 4
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> torch.Tensor:
         C, N, r = self.inner, self.N, self.rank
         seg = (meta.seg_cu, meta.seg_ctx, meta.seg_slot)
         proj = hops.linear(h, self.w_in)
@@ -768,7 +805,7 @@ class Mamba1Mixer:
         dt = hops.linear(q[:, :r], self.w_dt)
         y = hops.selective_scan(x, q, r, r + N, dt, self.dt_bias, self.a_log, self.d_skip, proj, C, cache["state"], *seg,
                                 meta.seg_max)
-        return hops.linear(y, self.wo)
+        return hops.linear(*_take(rows, y), self.wo)
 
     def export(self, p: str) -> dict:
         return {p + "in": self.w_in, p + "conv": self.conv_w, p + "conv.b": self.conv_b, p + "x": self.w_x, p + "dt": self.w_dt,
@@ -813,7 +850,7 @@ class WkvMixer:
     def cache_bytes(self, esize: int) -> tuple:
         return 0, 4 * (self.d + self.H * self.dk * self.dk)
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> torch.Tensor:
         T, n, H, dk = h.shape[0], self.n, self.H, self.dk
         seg = (meta.seg_cu, meta.seg_ctx, meta.seg_slot)
         dtype = self.wo.dtype
@@ -823,6 +860,7 @@ class WkvMixer:
         z = hops.linear(hops.linear_act(mix[:, 4], self.w1, "tanh"), self.w2)
         o = hops.decay_scan(rkvg, 0, n, 2 * n, z, self.w0, cache["state"], *seg, H, H, dk, dk, 1.0, decay="exp_exp", bonus=self.u,
                             longest=meta.seg_max, singles=meta.num_decode)
+        o, rkvg = _take(rows, o, rkvg)
         g = hops.gated_group_norm(o, rkvg, 3 * n, self.norm_w, self.eps, H, dtype, after=True, gate="silu")
         return hops.linear(g, self.wo)
 
@@ -895,9 +933,9 @@ class SideBySide:
         a, b = (x.cache_bytes(esize) for x in self.subs)
         return a[0] + b[0], a[1] + b[1]
 
-    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict) -> tuple:
+    def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> tuple:
         proj = hops.linear(h, self.w_in)
-        yl, yr = (x.forward(h, meta, cache[side], proj=proj[:, a:b])
+        yl, yr = (x.forward(h, meta, cache[side], proj=proj[:, a:b], rows=rows)
                   for x, side, (a, b) in zip(self.subs, ("left", "right"), self.cols))
         if self.out_w is not None:
             return yl, yr
@@ -1340,6 +1378,7 @@ class HybridLM:
         x0 = hops.embed_pos(ids, meta.positions, self.embed, self.pos, meta.dec_src, meta.dec_prev)
         x = x0.clone() if c.loop and c.loop[2] > 1 else x0
         pending: tuple = ()
+        want = self._wanted(meta, ids.numel())
         for r, (li, t, first) in enumerate(self.runs):
             adds, vec = pending, None
             if first:
@@ -1347,12 +1386,14 @@ class HybridLM:
                 if t > 0:
                     adds = adds + (x0,)
             h = hops.add_norm(x, adds, vec, self.norms[li], c.norm_eps, True, self.dtype)
-            ym = self.mixers[li].forward(h, meta, caches[r])
+            rows = want if r + 1 == len(self.runs) else None
+            ym = self.mixers[li].forward(h, meta, caches[r], rows=rows)
+            x, h = _take(rows, x, h)
             ff = self.ffns[li]
             pending = (ym, ff.forward(h)) if ff is not None else (ym,)
             if self.layer_probe is not None:
                 self.layer_probe.append(x + sum(a.float() for a in pending))
-        if meta.logits_idx is not None:
+        if meta.logits_idx is not None and want is None:
             idx = meta.logits_idx
             x = x.index_select(0, idx)
             pending = tuple(a.index_select(0, idx) for a in pending)
@@ -1384,6 +1425,7 @@ class HybridLM:
         if self.summed:
             return self._forward_summed(ids, x, meta, caches)
         pending: tuple = ()
+        want = None if self.depth_avg else self._wanted(meta, T)
         for r, (li, t, first) in enumerate(self.runs):
             if first and self.loop_step is not None:
                 x += self.loop_step[t]
@@ -1392,7 +1434,9 @@ class HybridLM:
                                     caches[r]["shift"], *seg, self.dtype, multi=meta.is_prefill)
             else:
                 h = hops.add_norm(x, pending, None, self.norms[li], c.norm_eps, self.one_plus, self.dtype)
-            pending = (self.mixers[li].forward(h, meta, caches[self.kv_run[r]]),)
+            rows = want if r + 1 == L else None
+            pending = (self.mixers[li].forward(h, meta, caches[self.kv_run[r]], rows=rows),)
+            (x,) = _take(rows, x)
             ff = self.ffns[li]
             if ff is not None:
                 h2 = hops.add_norm(x, pending, None, self.norms2[li], c.norm_eps, self.one_plus, self.dtype)
@@ -1402,7 +1446,7 @@ class HybridLM:
                 pending = ()
             if self.layer_probe is not None:
                 self.layer_probe.append(x + sum(a.float() for a in pending))
-        if meta.logits_idx is not None:
+        if meta.logits_idx is not None and want is None:
             idx = meta.logits_idx
             x = x.index_select(0, idx)
             pending = tuple(a.index_select(0, idx) for a in pending)
@@ -1418,13 +1462,16 @@ class HybridLM:
         eps, op, ctr, sd = c.norm_eps, self.one_plus, self.center, self.side_dim
         pend: tuple = ()  # (branch result, weight) pairs not yet in the stream
         normed = None  # (y, weight vector) of a branch that joins through its own RMS norm
+        want = None if sd else self._wanted(meta, ids.numel())
         for r, (li, t, first) in enumerate(self.runs):
             if first and self.loop_step is not None:
                 hops.sum_norm(x, pend, normed, None, eps, False, False, torch.float32)  # the stream, complete
                 pend, normed = (), None
                 x += self.loop_step[t]
             h = hops.sum_norm(x, pend, normed, self.norms[li], eps, ctr, op, self.dtype)
-            y = self.mixers[li].forward(h, meta, caches[self.kv_run[r]])
+            rows = want if r + 1 == len(self.runs) else None
+            y = self.mixers[li].forward(h, meta, caches[self.kv_run[r]], rows=rows)
+            (x,) = _take(rows, x)
             pend, normed = (y if isinstance(y, tuple) else ((y, 1.0),)), None
             ff = self.ffns[li]
             if ff is not None:
@@ -1442,7 +1489,7 @@ class HybridLM:
                     yf = normed[0].float()
                     full = full + yf * torch.rsqrt(yf.pow(2).mean(-1, keepdim=True) + eps) * normed[1]
                 self.layer_probe.append(full)
-        if meta.logits_idx is not None:
+        if meta.logits_idx is not None and want is None:
             idx = meta.logits_idx
             x = x.index_select(0, idx)
             pend = tuple((a.index_select(0, idx), w) for a, w in pend)
@@ -1461,10 +1508,13 @@ class HybridLM:
         def join(stream, pre, dtype):
             return hops.join_norm(stream, pend[0], pend[1], pre, eps, dtype, **pend[2])
 
+        want = self._wanted(meta, x.shape[0])
         for r, (li, _, _) in enumerate(self.runs):
             mx, ff = self.mixers[li], self.ffns[li]
             h = join(x, (self.norms[li], self.bias1[li]), torch.float32 if getattr(mx, "h_fp32", False) else self.dtype)
-            y = mx.forward(h, meta, caches[self.kv_run[r]])
+            rows = want if r + 1 == len(self.runs) else None
+            y = mx.forward(h, meta, caches[self.kv_run[r]], rows=rows)
+            (x,) = _take(rows, x)
             pend = (y, self.post1[li], dict(branch_w=mx.out_w, mix=mx.mix)) if isinstance(y, tuple) else ((y,), self.post1[li], {})
             if ff is not None:
                 pend = ((ff.forward(join(x, (self.norms2[li], self.bias2[li]), self.dtype)),), self.post2[li], {})
@@ -1472,7 +1522,7 @@ class HybridLM:
                 full = x.clone()
                 join(full, None, self.dtype)
                 self.layer_probe.append(full)
-        if meta.logits_idx is not None:
+        if meta.logits_idx is not None and want is None:
             idx = meta.logits_idx
             x = x.index_select(0, idx)
             pend = (tuple(a.index_select(0, idx) for a in pend[0]), *pend[1:])
@@ -1488,22 +1538,40 @@ class HybridLM:
         def step(hc, w):  # the pending result into the streams; the next sublayer's input
             return hops.stream_norm(xs, y, write, hc[0] if hc is not None else None, w, eps, self.dtype, S)
 
+        want = self._wanted(meta, x.shape[0])
         for r, (li, t, first) in enumerate(self.runs):
             if first and self.loop_step is not None:
                 raise ValueError("loop vectors are not built for several residual streams")
+            rows = want if r + 1 == len(self.runs) else None
             for hc, w, sub in ((self.hc1[li], self.norms[li], self.mixers[li]), (self.hc2[li], self.norms2[li], self.ffns[li])):
                 if sub is None:
                     continue
                 h, xs = step(hc, w)
-                y = sub.forward(h, meta, caches[self.kv_run[r]]) if sub is self.mixers[li] else sub.forward(h)
+                if sub is self.mixers[li]:
+                    y = sub.forward(h, meta, caches[self.kv_run[r]], rows=rows)
+                    (xs,) = _take(rows, xs)
+                else:
+                    y = sub.forward(h)
                 write = (hc[1], hc[2])
             if self.layer_probe is not None:  # the sum of the streams with the pending result
                 full = torch.einsum("nsd,st->nd", xs.expand(-1, S, -1), write[0]) + write[1].sum() * y.float()
                 self.layer_probe.append(full)
-        if meta.logits_idx is not None:
+        if meta.logits_idx is not None and want is None:
             idx = meta.logits_idx
             xs, y = xs.index_select(0, idx), y.index_select(0, idx)
         return self._logits(step(None, self.final_norm)[0])
+
+    def _wanted(self, meta: AttnMeta, T: int):
+        """The rows whose results a prefill step returns, if they are few: what the last layer makes of the others once its pages and
+        states are written reaches neither logits nor caches, so it goes on with these from its mixer's result on.  A slice where they
+        lie together, else a tensor for steps whose kernels take longer than the launches that pick rows (width 1024, us, all rows /
+        these: 2 x 350 tokens 1064 / 1074, 3 x 700 1090 / 1023; in fp32 3 x 331 beside 5 1170 / 1129).  None: all rows."""
+        idx = meta.logits_idx
+        if idx is None or not meta.is_prefill or self.layer_probe is not None or not 0 < 2 * idx.numel() <= T:
+            return None
+        if meta.logits_span is not None:
+            return slice(*meta.logits_span)
+        return idx if T * self.cfg.d_model * self.dtype.itemsize >= 1 << 21 else None
 
     def _logits(self, hf: torch.Tensor) -> torch.Tensor:
         c = self.cfg
@@ -1521,6 +1589,7 @@ class HybridLM:
         c = self.cfg
         eps, op, mult = c.norm_eps, self.one_plus, c.residual_mult
         pend = None  # (y, projection holding the gate logits, their first column, bias)
+        want = self._wanted(meta, x.shape[0])
         for r, (li, t, first) in enumerate(self.runs):
             if first and self.loop_step is not None:
                 if pend is not None:
@@ -1530,7 +1599,11 @@ class HybridLM:
             h = hops.add_norm(x, (), None, w1, eps, op, self.dtype) if pend is None else \
                 hops.gated_add_norm(x, pend[0], pend[1], pend[2], pend[3], mult, w1, eps, op, self.dtype)
             mx = self.mixers[li]
-            y = mx.forward(h, meta, caches[self.kv_run[r]])
+            rows = want if r + 1 == len(self.runs) else None
+            y = mx.forward(h, meta, caches[self.kv_run[r]], rows=rows)
+            (x,) = _take(rows, x)
+            if self.rg1[li]["w"] is not None:
+                (h,) = _take(rows, h)
             pend = (y, *self._gate_of(mx, self.rg1[li], h), self.rg1[li]["b"])
             ff = self.ffns[li]
             if ff is not None:
@@ -1541,7 +1614,7 @@ class HybridLM:
                 d = x.shape[1]
                 g = pend[1][:, pend[2]:pend[2] + d].float() + pend[3].float()
                 self.layer_probe.append(x + mult * pend[0].float() * torch.sigmoid(g))
-        if meta.logits_idx is not None:
+        if meta.logits_idx is not None and want is None:
             idx, d = meta.logits_idx, x.shape[1]
             x = x.index_select(0, idx)
             if pend is not None:

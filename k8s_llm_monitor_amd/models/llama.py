@@ -93,6 +93,10 @@ class AttnMeta:
     seg_max: int = 0  # rows of the longest segment (0: not known)
     # prefill: every chunk of this step starts at position 0 (whole prompts, nothing cached before)
     all_fresh: bool = False
+    # layer-list prefill: ``logits_idx`` is the decode rows, then every chunk's last row, which sees this many positions [S] int32
+    # (None: other rows)
+    ends: Optional[torch.Tensor] = None
+    logits_span: Optional[tuple] = None  # ``logits_idx`` as (first row, end) where the rows lie together
     # layer-list prefill, latent attention's expanded form: a PageList for each attention window of those layers (0: none),
     # and cu_seqlens on the host
     page_lists: Optional[dict] = None
@@ -687,16 +691,20 @@ class CausalLM:
         n = len(self.layers)
         x = ops.rms_norm(residual, self.layers[0]["attn_norm"], eps)
         ss = None
+        # behind the last layer's attention only the rows whose logits the step returns are read: the same tile kernels on these
+        few = meta.logits_idx is not None and 0 < 2 * meta.logits_idx.numel() <= x.shape[0]
         for i, L in enumerate(self.layers):
             kv = kv_caches[i] if kv_caches is not None else None
             o = self._attn_core(L, x, meta, kv, rowscale=(ss, eps) if ss is not None else None)
+            if i + 1 == n and few:
+                o, residual = o[meta.logits_idx], residual[meta.logits_idx].contiguous()
             x, ss = ops.gemm_tile_resid(o, L["wo"], residual, L["mlp_norm"])
             act = ops.prefill_linear(x, L["w13"], swiglu=self._swg, rowscale=(ss, eps))
             if i + 1 < n:
                 x, ss = ops.gemm_tile_resid(act, L["w2"], residual, self.layers[i + 1]["attn_norm"])
             else:
                 y = ops.prefill_linear(act, L["w2"])
-                if meta.logits_idx is not None:
+                if meta.logits_idx is not None and not few:
                     y = y[meta.logits_idx]
                     residual = residual[meta.logits_idx].contiguous()
                 x = ops.fused_add_rms_norm(y.contiguous(), residual, self.final_norm, eps)

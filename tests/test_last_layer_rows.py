@@ -1,0 +1,102 @@
+"""A prefill step that returns few rows' logits goes on with these rows alone behind its last mixer: logits, pages and states against a step
+that returns every row's."""
+import dataclasses
+
+import pytest
+import torch
+
+from k8s_llm_monitor_amd.engine.block_manager import BlockManager
+from k8s_llm_monitor_amd.engine.runner import ModelRunner, RunnerConfig
+from k8s_llm_monitor_amd.engine.sequence import SamplingParams, Sequence
+from k8s_llm_monitor_amd.models import HybridLM, build_model, get_config
+
+PRESETS = ["dunesun-tiny", "kisutar-tiny", "bitonex-tiny", "levovik-tiny", "dopivik-tiny", "zifisun-tiny"]
+
+
+@pytest.fixture(autouse=True)
+def _small_steps(monkeypatch):
+    """Steps of these sizes too pick rows that do not lie together."""
+    real = HybridLM._wanted
+
+    def wanted(self, meta, T):
+        w = real(self, meta, T)
+        few = meta.is_prefill and meta.logits_idx is not None and 0 < 2 * meta.logits_idx.numel() <= T
+        return meta.logits_idx if w is None and few else w
+
+    monkeypatch.setattr(HybridLM, "_wanted", wanted)
+
+
+def _step(model, every, cuts):
+    """Logits of the last rows and the caches after one prompt of 9 tokens, then prompts of 37, 5 and 50 in portions, the last of them beside
+    its running sequence."""
+    runner = ModelRunner(model, RunnerConfig(max_num_seqs=4, max_model_len=128, num_blocks=40, keep_logits=True, use_graphs=False))
+    manager = BlockManager(40, watermark=0.0, prefix_caching=False, state_slots=getattr(runner, "num_state_slots", 0))
+    g = torch.Generator().manual_seed(5)
+    ids = [torch.randint(3, model.cfg.vocab_size, (n,), generator=g).tolist() for n in (37, 5, 50, 9)]
+    seqs = [Sequence(prompt_ids=t, params=SamplingParams(temperature=0.0, ignore_eos=True)) for t in ids]
+    out = []
+    for q in seqs:
+        assert manager.allocate(q)
+
+    def go(pro, dec):
+        with torch.no_grad():
+            rows = [[0] for _ in dec] + [list(range(q.chunk)) for q in pro]
+            h = runner.prefill_launch(pro, dec, logit_rows=rows if every else None)
+        z = h.logits if every else runner.last_logits
+        last = torch.tensor([len(r) for r in rows]).cumsum(0) - 1
+        out.append((z[last.to(z.device)] if every else z).float().cpu())
+
+    run = seqs[3]
+    run.num_computed, run.chunk = 0, len(ids[3]) - 1
+    go([run], [])
+    run.prompt_ids, run.output_ids = ids[3][:-1], ids[3][-1:]
+    run.num_computed, run.chunk, run.prefilled = len(ids[3]) - 1, 1, True
+    for a, b in zip(cuts, cuts[1:]):
+        pro = [q for q in seqs[:3] if len(q.prompt_ids) > int(len(q.prompt_ids) * a)]
+        for q in pro:
+            q.num_computed = int(len(q.prompt_ids) * a)
+            q.chunk = int(len(q.prompt_ids) * b) - q.num_computed
+        go(pro, [run] if b == 1 else [])
+
+    def flat(c):
+        return [t for v in c.values() for t in (flat(v) if isinstance(v, dict) else [v])]
+
+    return out, [t.float().cpu() for c in runner.kv for t in (flat(c) if isinstance(c, dict) else c)]
+
+
+def _compare(model, tol):
+    for cuts in ((0, 1), (0, 0.4, 1)):
+        (a, ca), (b, cb) = _step(model, False, cuts), _step(model, True, cuts)
+        for x, y in zip(a, b):
+            assert x.shape == y.shape and float((x - y).norm() / y.norm()) < tol
+        for x, y in zip(ca, cb):  # what the last mixer wrote does not depend on whose logits are wanted
+            torch.testing.assert_close(x, y, rtol=0, atol=0)
+
+
+def _models(name, device, dtype):
+    cfg = get_config(name)
+    for k in range(1, len(cfg.layers) + 1):  # every layer as the last one
+        yield HybridLM(dataclasses.replace(cfg, name=f"{name}-{k}", layers=cfg.layers[:k], loop=None), device=device, dtype=dtype, seed=3)
+
+
+@pytest.mark.parametrize("name", PRESETS)
+def test_last_layer_on_wanted_rows(name):
+    for m in _models(name, "cpu", torch.float32):
+        _compare(m, 1e-4)  # fp32 sums of other shapes
+
+
+def test_last_layer_on_wanted_rows_llama():
+    _compare(build_model(get_config("llama-tiny"), device="cpu", dtype=torch.float32, seed=3), 1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 3e-2)])  # bf16: one layer's roundings, each 2^-9
+@pytest.mark.parametrize("name", PRESETS)
+def test_gpu_last_layer_on_wanted_rows(name, dtype, tol):
+    for m in _models(name, "cuda:0", dtype):
+        _compare(m, tol)
+
+
+@pytest.mark.gpu
+def test_gpu_last_layer_on_wanted_rows_llama():
+    _compare(build_model(get_config("llama-tiny-d128"), device="cuda:0", dtype=torch.bfloat16, seed=3), 1e-2)
