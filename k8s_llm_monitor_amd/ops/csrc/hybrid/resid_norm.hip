@@ -20,6 +20,8 @@
 //   gated_lookup      out = gelu_tanh(gate) * table[id][col : col + n]
 #include "hy_common.h"
 
+#include <algorithm>
+
 namespace k8sllm {
 
 template <typename T>
@@ -27,12 +29,24 @@ __global__ __launch_bounds__(256) void embed_pos_kernel(float* __restrict__ out,
                                                         const int* __restrict__ positions, const T* __restrict__ emb,
                                                         const T* __restrict__ pos, const int* __restrict__ src,
                                                         const int* __restrict__ prev, int d, int vocab, int max_pos,
-                                                        float scale) {
+                                                        float scale, int vec) {
   const long t = blockIdx.x;
   int id = ids[t];
   if (src != nullptr && src[t] >= 0) id = prev[src[t]];
   id = min(max(id, 0), vocab - 1);
   const T* e = emb + (long)id * d;
+  if (vec) {  // 8 columns per thread and trip: 8000 rows of 2048, bf16, 20.1 -> 17.9 us, 24 of 4096 4.6 -> 3.5
+    const T* q = pos != nullptr ? pos + (long)min(max(positions[t], 0), max_pos - 1) * d : nullptr;
+    for (int c = threadIdx.x * 8; c < d; c += 2048) {
+      float x[8], a[8];
+      load8(e + c, x);
+      if (q != nullptr) load8(q + c, a);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = x[i] * scale + (q != nullptr ? a[i] : 0.f);
+      store8(out + t * d + c, x);
+    }
+    return;
+  }
   const T* p = nullptr;
   if (pos != nullptr) p = pos + (long)min(max(positions[t], 0), max_pos - 1) * d;
   for (int c = threadIdx.x; c < d; c += 256) out[t * d + c] = ldf(e + c) * scale + (p != nullptr ? ldf(p + c) : 0.f);
@@ -764,7 +778,7 @@ __global__ __launch_bounds__(256) void token_mix_kernel(T* __restrict__ out, con
   float* st = sl >= 0 ? state + (long)sl * d : nullptr;
   const float* last = h + (long)(cu[s + 1] - 1) * d;
   T* o = out + row * n * d;
-  for (int c = threadIdx.x * V; c < d; c += 256 * V) {
+  for (int c = (blockIdx.y * 256 + threadIdx.x) * V; c < d; c += 256 * V * gridDim.y) {
     float x[V], p[V], m[V];
     ldv<V>(hr + c, x);
     if (!first) {
@@ -816,12 +830,13 @@ int k8sllm_hy_embed_pos(float* out, const int* ids, const int* positions, const 
                         const int* src, const int* prev, long T, int d, int vocab, int max_pos, float scale, int f32,
                         hipStream_t s) {
   if (T <= 0) return 0;
+  const int vec = d % 8 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(emb) | reinterpret_cast<uintptr_t>(pos)) & 15) == 0;
   if (f32)
     hipLaunchKernelGGL(embed_pos_kernel<float>, dim3(T), dim3(256), 0, s, out, ids, positions, (const float*)emb,
-                       (const float*)pos, src, prev, d, vocab, max_pos, scale);
+                       (const float*)pos, src, prev, d, vocab, max_pos, scale, vec);
   else
     hipLaunchKernelGGL(embed_pos_kernel<bf16_t>, dim3(T), dim3(256), 0, s, out, ids, positions, (const bf16_t*)emb,
-                       (const bf16_t*)pos, src, prev, d, vocab, max_pos, scale);
+                       (const bf16_t*)pos, src, prev, d, vocab, max_pos, scale, vec);
   return (int)hipGetLastError();
 }
 
@@ -1046,8 +1061,10 @@ int k8sllm_hy_join_norm(void* out, float* residual, const void* y0, int t0, cons
 int k8sllm_hy_token_mix(void* out, const float* h, const float* mu, int n, float* state, const int* cu, const int* ctx,
                         const int* slot, int S, long rows, int d, int f32, hipStream_t s) {
   if (rows <= 0 || S <= 0) return 0;
+  // the few rows of a decode step: a row over as many workgroups as its columns take one trip in (24 rows of 4096, five mixes, 8.1 -> 4.9 us; 200 9.9 -> 7.0)
+  const unsigned parts = rows >= 256 ? 1 : (unsigned)std::max(1, std::min(16, d / 1024));
 #define K8SLLM_TM(T_, V)                                                                                              \
-  hipLaunchKernelGGL((token_mix_kernel<T_, V>), dim3((unsigned)rows), dim3(256), 0, s, (T_*)out, h, mu, n, state, cu, ctx, \
+  hipLaunchKernelGGL((token_mix_kernel<T_, V>), dim3((unsigned)rows, parts), dim3(256), 0, s, (T_*)out, h, mu, n, state, cu, ctx, \
                      slot, S, d)
   if (f32) {
     if (d % 4 == 0) K8SLLM_TM(float, 4); else K8SLLM_TM(float, 1);

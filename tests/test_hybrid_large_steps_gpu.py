@@ -622,6 +622,39 @@ def test_one_token_a_segment_selective(n, C, N, dt):
     _same_step(lambda s, mode: hops.selective_scan(xc, q, 5, 5 + N, d, *par, proj, C, s, cu, ctx, slot, mode=mode), _r(g, n + 2, C, N).cuda())
 
 
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+@pytest.mark.parametrize("n,C,bias", [(3, 8, True), (24, 2056, False), (66, 4352, True)])
+def test_one_token_a_segment_conv(n, C, bias, dt):
+    """The decode steps' convolution with its history, against the launches of steps with a longer segment (here of five rows behind
+    the others): the same bits in rows and slots; a fresh sequence, a padding row, no row beside two of one sequence."""
+    g = _g(81)
+    cu, ctx, slot = _singles(g, n)
+    proj, w, b = _r(g, n + 5, C + 24, dt=dt).cuda(), _r(g, C, 4).cuda(), _r(g, C).cuda() if bias else None
+    a = _r(g, n + 3, 3, C, dt=dt).cuda()
+    b2 = a.clone()
+    got = hops.conv_silu(proj[:n], 16, C, w, b, a, cu, ctx, slot)
+
+    def more(t, v):
+        return torch.cat([t, torch.tensor([v], dtype=torch.int32, device="cuda")])
+
+    want = hops.conv_silu(proj, 16, C, w, b, b2, more(cu, n + 5), more(ctx, 0), more(slot, n + 2))
+    a[n + 2] = b2[n + 2]
+    assert torch.equal(got, want[:n]) and torch.equal(a, b2)
+
+
+@pytest.mark.parametrize("n,d", [(1, 1024), (30, 4096), (7, 2052), (255, 3000), (256, 2048)])
+def test_token_mix_of_few_rows(n, d):
+    """Rows over one or several workgroups: fp32 products of the torch form (a difference, a product and a sum: 3e-7 of values up to 10)."""
+    g = _g(82)
+    cu, ctx, slot = _i32(list(range(n + 1))), torch.randint(0, 3, (n,), generator=g).int(), torch.randperm(n, generator=g).int()
+    h, mu, st = _r(g, n, d), _r(g, 5, d), _r(g, n, d)
+    sg = st.clone().cuda()
+    want = hops.token_mix(h, mu, st, cu, ctx, slot, torch.float32)
+    got = hops.token_mix(h.cuda(), mu.cuda(), sg, cu.cuda(), ctx.cuda(), slot.cuda(), torch.float32)
+    torch.testing.assert_close(got.cpu(), want, rtol=1e-6, atol=3e-6)
+    assert torch.equal(sg.cpu(), st)
+
+
 @pytest.mark.parametrize("M", [1, 257, 600])
 @pytest.mark.parametrize("f,rest,K", [(128, 0, 192), (144, 48, 256), (400, 272, 320), (16, 256, 192)])  # tiles of 128 features and 256 columns
 @pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "relu"])
