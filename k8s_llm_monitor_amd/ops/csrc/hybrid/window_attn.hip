@@ -16,6 +16,7 @@
 #include <utility>
 
 #include "stream_rows.h"
+#include "value_pages.h"
 
 namespace k8sllm {
 
@@ -38,9 +39,15 @@ __global__ __launch_bounds__(256) void qk_norm_cache_kernel(T* __restrict__ qkv,
                                                             const float* __restrict__ qw,
                                                             const float* __restrict__ kw, float eps, int nq, int nk,
                                                             int nv, T* __restrict__ k_cache, T* __restrict__ v_cache,
-                                                            const int* __restrict__ slots, int bs) {
+                                                            const int* __restrict__ slots, int bs, long rows, int runs) {
   __shared__ float red[4];
-  const long t = blockIdx.x;
+  if constexpr (sizeof(T) == 2) {
+    if (blockIdx.x < runs) {  // the first workgroups write the values
+      write_value_runs(qkv + nq + nk, stride, rows, blockIdx.x, nv, v_cache, slots);
+      return;
+    }
+  }
+  const long t = blockIdx.x - runs;
   T* row = qkv + t * stride;
   const long slot = (slots != nullptr && k_cache != nullptr) ? slots[t] : -1;
   float sq = 0.f, sk = 0.f;
@@ -94,7 +101,7 @@ __global__ __launch_bounds__(256) void qk_norm_cache_kernel(T* __restrict__ qkv,
     if (slot >= 0) k_cache[slot * nk + c] = row[nq + c];
   }
   }
-  if (slot >= 0)
+  if (slot >= 0 && !runs)
     for (int c = threadIdx.x; c < nv; c += 256) v_cache[((slot / bs) * nv + c) * bs + slot % bs] = row[nq + nk + c];
 }
 
@@ -947,9 +954,12 @@ int k8sllm_hy_window_f32(void* out, const void* qkv, long q_stride, const void* 
 int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float* kw, float eps, long T, int nq,
                             int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s) {
   if (T <= 0) return 0;
+  const int runs =
+      !f32 && k_cache != nullptr && value_runs_ok(qkv, stride, nq + nk, nv, v_cache, slots, T, bs) ? value_groups(T, nv) : 0;
+  const unsigned grid = (unsigned)(T + runs);
 #define K8SLLM_QK(T_, NV)                                                                                             \
-  hipLaunchKernelGGL((qk_norm_cache_kernel<T_, NV>), dim3(T), dim3(256), 0, s, (T_*)qkv, stride, qw, kw, eps, nq, nk, nv, \
-                     (T_*)k_cache, (T_*)v_cache, slots, bs)
+  hipLaunchKernelGGL((qk_norm_cache_kernel<T_, NV>), dim3(grid), dim3(256), 0, s, (T_*)qkv, stride, qw, kw, eps, nq, nk, nv, \
+                     (T_*)k_cache, (T_*)v_cache, slots, bs, T, runs)
 #define K8SLLM_QKT(T_)                                          \
   if (nq <= 2048 && nk <= 2048) K8SLLM_QK(T_, 8);               \
   else if (nq <= 4096 && nk <= 4096) K8SLLM_QK(T_, 16);         \

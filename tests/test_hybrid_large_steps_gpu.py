@@ -1228,3 +1228,55 @@ def test_grouped_tiles_of_rows_at_any_address(at):
     if at != 8:
         with pytest.raises(RuntimeError, match="alignment"):
             ops.native().gemm_tile_rows(want, x, w, off, idx, K, False, 0)
+
+
+@pytest.mark.parametrize("T,Hq,G,dk,dv,nf,extra,pairs,dt", [
+    (255, 4, 2, 64, 64, 32, 8, False, BF),        # the last size whose values go row by row
+    (256, 4, 2, 64, 72, 24, 8, True, BF),         # entries that pass; values not a multiple of a group's columns
+    (1023, 3, 1, 128, 640, 64, 0, False, BF),     # two groups of value columns
+    (1025, 3, 1, 128, 40, 64, 16, True, BF),      # several rows a workgroup, the last with one
+    (1030, 2, 2, 48, 32, 8, 0, False, BF),
+    (300, 2, 1, 36, 34, 18, 2, False, BF),        # neither eight neighbours nor 16-byte rows
+    (270, 2, 1, 36, 33, 18, 0, True, BF),         # odd rows: values row by row
+    (1040, 2, 1, 2048, 16, 1024, 0, False, BF),   # more frequencies than a workgroup holds
+    (1025, 2, 2, 64, 64, 32, 0, True, torch.float32),
+])
+def test_values_to_pages_in_runs(T, Hq, G, dk, dv, nf, extra, pairs, dt):
+    """rotary_cache and qk_norm_cache of large steps: decode rows, then sequences that begin and end inside pages, rows that are not
+    written, pages in any order.  Values are copies: equal to the bit; turned and normed entries as the fp32 form up to one rounding."""
+    g = _g(90)
+    nv, bs = G * dv, 16
+    lens = [1, 1, 1, 37, 5, T - 45]
+    starts = [15, 0, 7, 11, 16, 3]
+    nb = sum((a + n + 15) // 16 for a, n in zip(starts, lens)) + 2
+    pages, slots, at = torch.randperm(nb, generator=g), [], 0
+    for a, n in zip(starts, lens):
+        p = torch.arange(a, a + n)
+        slots.append(pages[at + p // 16] * 16 + p % 16)
+        at += (a + n + 15) // 16
+    slots = torch.cat(slots).to(torch.int32)
+    slots[[20, 60, T - 1]] = -1
+    pos = torch.randint(0, 4000, (T,), generator=g, dtype=torch.int32)
+    freq = hops.rotary_freq(1e4, nf)
+    temp = torch.rand(Hq, generator=g) + 0.5
+    x = _r(g, T, (Hq + G) * dk + nv + extra, dt=dt)
+    tol = dict(rtol=2 ** -7, atol=2 ** -7) if dt == BF else dict(rtol=1e-5, atol=1e-5)  # one rounding; some units of fp32
+
+    def run(device, norm):
+        y = (x[:, :(Hq + G) * dk + nv] if norm else x).to(device, copy=True).contiguous()
+        kc = torch.zeros(nb, bs, G * dk, dtype=dt, device=device)
+        vc = torch.zeros(nb, G, dv, bs, dtype=dt, device=device)
+        s = slots.to(device)
+        if norm:
+            w = torch.linspace(0.5, 1.5, Hq * dk, device=device)
+            hops.qk_norm_cache(y, w, w[:G * dk].contiguous(), 1e-5, Hq, G, dk, dv, kc, vc, s)
+        else:
+            hops.rotary_cache(y, Hq, G, dk, dv, pos.to(device), freq.to(device), pairs, temp.to(device), kc, vc, s)
+        return y.cpu(), kc.cpu(), vc.cpu()
+
+    for norm in (False, True):
+        want, got = run("cpu", norm), run("cuda", norm)
+        assert torch.equal(got[2], want[2])
+        assert torch.equal(got[0][:, (Hq + G) * dk:], want[0][:, (Hq + G) * dk:])
+        torch.testing.assert_close(got[0].float(), want[0].float(), **tol)
+        torch.testing.assert_close(got[1].float(), want[1].float(), **tol)
