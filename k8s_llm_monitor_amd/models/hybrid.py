@@ -981,12 +981,13 @@ class RoutedFFN:
             wr = torch.cat([wr, p.get(prefix + "shared.sg", (1, d), s, small=True)])
         self.wr = wr.contiguous()
 
-    def forward(self, h: torch.Tensor) -> torch.Tensor:
-        ids, wts, gate = hops.moe_router(h, self.wr, self.bias, self.E, self.K)
+    def forward(self, h: torch.Tensor, routed: Optional[tuple] = None, join: bool = False):
+        """``routed``: h's router results, if the norm's launch gave them; ``join``: the sum is left to the next norm (ops.hybrid.ExpertSum)."""
+        ids, wts, gate = routed or hops.moe_router(h, self.wr, self.bias, self.E, self.K)
         shared = None
         if self.fs:
             shared = F.linear(hops.swiglu(F.linear(h, self.ws13)), self.ws2)
-        return hops.moe_experts(h, ids, wts, self.w13, self.w2, shared, gate, il=self.il)
+        return hops.moe_experts(h, ids, wts, self.w13, self.w2, shared, gate, il=self.il, join=join)
 
 
 def _softplus(z: float) -> float:
@@ -1385,18 +1386,25 @@ class HybridLM:
                 vec = self.loop_step[t]
                 if t > 0:
                     adds = adds + (x0,)
-            h = hops.add_norm(x, adds, vec, self.norms[li], c.norm_eps, True, self.dtype)
             rows = want if r + 1 == len(self.runs) else None
+            ff = self.ffns[li]
+            routed = None
+            if isinstance(ff, RoutedFFN) and rows is None and hops.route_with_norm(*x.shape, ff.wr.shape[0]):
+                h, routed = hops.add_norm(x, adds, vec, self.norms[li], c.norm_eps, True, self.dtype, route=(ff.wr, ff.bias, ff.E, ff.K))
+            else:
+                h = hops.add_norm(x, adds, vec, self.norms[li], c.norm_eps, True, self.dtype)
             ym = self.mixers[li].forward(h, meta, caches[r], rows=rows)
             x, h = _take(rows, x, h)
-            ff = self.ffns[li]
-            pending = (ym, ff.forward(h)) if ff is not None else (ym,)
+            if isinstance(ff, RoutedFFN):
+                pending = (ym, ff.forward(h, routed, join=self.layer_probe is None))
+            else:
+                pending = (ym, ff.forward(h)) if ff is not None else (ym,)
             if self.layer_probe is not None:
                 self.layer_probe.append(x + sum(a.float() for a in pending))
         if meta.logits_idx is not None and want is None:
             idx = meta.logits_idx
             x = x.index_select(0, idx)
-            pending = tuple(a.index_select(0, idx) for a in pending)
+            pending = tuple((a.rows() if isinstance(a, hops.ExpertSum) else a).index_select(0, idx) for a in pending)
         hf = hops.add_norm(x, pending, None, self.final_norm, c.norm_eps, True, self.dtype)
         return self._logits(hf)
 

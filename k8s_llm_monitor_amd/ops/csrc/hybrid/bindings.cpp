@@ -31,7 +31,9 @@ int k8sllm_hy_router_grouped(int* ids, float* wts, const void* h, long T, int d,
                              int K, int groups, int keep, float scale, int soft, int best2, int renorm, int f32,
                              hipStream_t s);
 int k8sllm_hy_add_norm(void* out, float* residual, const void* a0, int t0, const void* a1, int t1, const void* a2,
-                       int t2, const float* vec, const float* w, long rows, int d, float eps, int one_plus, int f32,
+                       int t2, const float* vec, const float* w, long rows, int d, float eps, int one_plus, const void* ys,
+                       const int* inv, const float* wts, const void* shared, const float* gate, int K, int* r_ids, float* r_wts,
+                       float* r_gate, const float* wr, const float* bias, int rE, int rK, int rows_w, int over_all, int f32,
                        hipStream_t s);
 int k8sllm_hy_gated_group_norm(void* out, const float* y, const void* z, long z_stride, const float* w, long rows,
                                int n, int groups, float eps, int after, int f32, hipStream_t s);
@@ -180,23 +182,78 @@ void embed_pos(Tensor out, Tensor ids, Tensor positions, Tensor emb, OptT pos, O
         "embed_pos");
 }
 
-void add_norm(Tensor out, Tensor residual, OptT a0, OptT a1, OptT a2, OptT vec, Tensor w, double eps, bool one_plus) {
+// ys, inv, wts (, shared (, gate)): addend `at` is the sum of each row's experts (moe_combine).  r_ids, r_wts (, r_gate), wr (, bias):
+// the normed rows' router (moe_router) in the same launch.
+void add_norm_experts(Tensor out, Tensor residual, OptT a0, OptT a1, OptT a2, OptT vec, Tensor w, double eps, bool one_plus, int64_t at,
+                      OptT ys, OptT inv, OptT wts, OptT shared, OptT gate, OptT r_ids, OptT r_wts, OptT r_gate, OptT wr, OptT bias,
+                      int64_t E, int64_t K, bool over_all) {
   const int f = act(out, "out");
   f32c(residual, "residual");
   f32c(w, "w");
   TORCH_CHECK(residual.dim() == 2 && out.is_contiguous() && out.numel() == residual.numel(), "add_norm: out shape");
   const int64_t rows = residual.size(0), d = residual.size(1);
   TORCH_CHECK(w.numel() == d, "add_norm: w [d]");
-  const int t0 = any_dt(a0, rows * d, "addend 0"), t1 = any_dt(a1, rows * d, "addend 1"), t2 = any_dt(a2, rows * d, "addend 2");
+  int t[3] = {any_dt(a0, rows * d, "addend 0"), any_dt(a1, rows * d, "addend 1"), any_dt(a2, rows * d, "addend 2")};
   if (vec.has_value()) {
     f32c(*vec, "vec");
     TORCH_CHECK(vec->numel() == d, "add_norm: vec [d]");
   }
-  check(k8sllm_hy_add_norm(out.data_ptr(), residual.data_ptr<float>(), t0 ? a0->data_ptr() : nullptr, t0,
-                           t1 ? a1->data_ptr() : nullptr, t1, t2 ? a2->data_ptr() : nullptr, t2,
-                           vec.has_value() ? vec->data_ptr<float>() : nullptr, w.data_ptr<float>(), rows, (int)d, (float)eps,
-                           one_plus, f, cur()),
+  const void* sh = nullptr;
+  const float* gp = nullptr;
+  int64_t Ks = 0;
+  if (ys.has_value()) {
+    TORCH_CHECK(at >= 0 && at < 3 && t[at] == 0 && inv.has_value() && wts.has_value() && d % 8 == 0, "add_norm: the experts' sum");
+    same(*ys, f, "ys");
+    i32c(*inv, "inv_idx");
+    f32c(*wts, "wts");
+    Ks = wts->numel() / std::max<int64_t>(rows, 1);
+    TORCH_CHECK(ys->dim() == 2 && ys->is_contiguous() && ys->size(1) == d && ys->size(0) == rows * Ks && inv->numel() == rows * Ks &&
+                    wts->numel() == rows * Ks,
+                "add_norm: the experts' rows");
+    if (shared.has_value()) {
+      same(*shared, f, "shared");
+      TORCH_CHECK(shared->is_contiguous() && shared->numel() == rows * d, "shared [T, d]");
+      sh = shared->data_ptr();
+      if (gate.has_value()) {
+        f32c(*gate, "gate");
+        TORCH_CHECK(gate->numel() == rows, "gate [T]");
+        gp = gate->data_ptr<float>();
+      }
+    }
+    t[at] = 3;
+  }
+  float* rg = nullptr;
+  if (r_ids.has_value()) {
+    TORCH_CHECK(r_wts.has_value() && wr.has_value() && d % 8 == 0 && d > 0, "add_norm: router");
+    i32c(*r_ids, "ids");
+    f32c(*r_wts, "wts");
+    f32c(*wr, "router weight");
+    TORCH_CHECK(wr->dim() == 2 && wr->size(1) == d && (wr->size(0) == E || wr->size(0) == E + 1) && wr->size(0) <= 9, "router rows");
+    TORCH_CHECK(K >= 1 && K <= E && r_ids->numel() == rows * K && r_wts->numel() == rows * K, "router: outputs");
+    if (bias.has_value()) {
+      f32c(*bias, "router bias");
+      TORCH_CHECK(bias->numel() >= E, "router bias [E]");
+    }
+    if (r_gate.has_value()) {
+      f32c(*r_gate, "gate");
+      TORCH_CHECK(r_gate->numel() == rows && wr->size(0) == E + 1, "gate [T] needs the extra router row");
+      rg = r_gate->data_ptr<float>();
+    }
+  }
+  const bool ro = r_ids.has_value(), jo = ys.has_value();
+  check(k8sllm_hy_add_norm(out.data_ptr(), residual.data_ptr<float>(), a0.has_value() ? a0->data_ptr() : nullptr, t[0],
+                           a1.has_value() ? a1->data_ptr() : nullptr, t[1], a2.has_value() ? a2->data_ptr() : nullptr, t[2],
+                           vec.has_value() ? vec->data_ptr<float>() : nullptr, w.data_ptr<float>(), rows, (int)d, (float)eps, one_plus,
+                           jo ? ys->data_ptr() : nullptr, jo ? inv->data_ptr<int>() : nullptr, jo ? wts->data_ptr<float>() : nullptr, sh,
+                           gp, (int)Ks, ro ? r_ids->data_ptr<int>() : nullptr, ro ? r_wts->data_ptr<float>() : nullptr, rg,
+                           ro ? wr->data_ptr<float>() : nullptr, ro && bias.has_value() ? bias->data_ptr<float>() : nullptr, (int)E, (int)K,
+                           ro ? (int)wr->size(0) : 0, over_all, f, cur()),
         "add_norm");
+}
+
+void add_norm(Tensor out, Tensor residual, OptT a0, OptT a1, OptT a2, OptT vec, Tensor w, double eps, bool one_plus) {
+  const OptT none;
+  add_norm_experts(out, residual, a0, a1, a2, vec, w, eps, one_plus, 0, none, none, none, none, none, none, none, none, none, none, 0, 0, false);
 }
 
 // after 0: norm(y * silu(z)) * w;  1: norm(y) * w * sigmoid(z);  2: norm(y) * w * silu(z)
@@ -1177,6 +1234,7 @@ bool latent_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, OptT
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_pos", &embed_pos);
   m.def("add_norm", &add_norm);
+  m.def("add_norm_experts", &add_norm_experts);
   m.def("gated_group_norm", &gated_group_norm);
   m.def("swiglu", &swiglu);
   m.def("gated_add_norm", &gated_add_norm);

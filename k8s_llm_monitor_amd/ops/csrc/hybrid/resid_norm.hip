@@ -18,7 +18,7 @@
 //                     RMS-normed ones;  out = LN(residual) * nw + nb
 //   token_mix         out[t][j] = h[t] + (h[t-1] - h[t]) * mu[j], the row before a segment from the sequence's slot
 //   gated_lookup      out = gelu_tanh(gate) * table[id][col : col + n]
-#include "hy_common.h"
+#include "router.h"
 
 #include <algorithm>
 
@@ -52,35 +52,74 @@ __global__ __launch_bounds__(256) void embed_pos_kernel(float* __restrict__ out,
   for (int c = threadIdx.x; c < d; c += 256) out[t * d + c] = ldf(e + c) * scale + (p != nullptr ? ldf(p + c) : 0.f);
 }
 
-template <typename T>
+// An addend that is the weighted sum of a token's experts (moe_combine's, without the identity experts), formed where it is added: its fp32 rows
+// are neither written nor read, and a launch goes.
+struct ExpertSum {
+  const void* ys;
+  const int* inv;
+  const float* wts;
+  const void* shared;
+  const float* gate;
+  int K;
+};
+// The router of the normed rows
+struct Route {
+  int* ids;
+  float* wts;
+  float* gate;
+  const float* wr;
+  const float* bias;
+  int E, K, rows_w, over_all;
+};
+
+// t0, t1, t2: an addend's type, 0 none, 1 bf16, 2 fp32, 3 (JOIN) the experts' sum.  A thread keeps its first eight columns in registers between sum
+// and norm.  NR > 0: the router's at most NR weight rows with their logits here too, in the order of hy_router_kernel's sums (from the rounded
+// row); the weights, 64 KB a row from L2 at 8 x 2048, are on their way while the row is summed.
+// A bf16 branch and two experts, us, moe_combine and norm / one launch: 8192 rows of 2048 73 / 55, 200 7.0 / 4.8, 1 5.2 / 4.4; with the router of 8
+// behind them / in it too: 64 rows of 2048 8.1 / 6.7, 255 10.0 / 8.4, 64 of 4096 10.8 / 9.2, 200 of 1024 (fp32) 8.8 / 7.3.
+template <typename T, bool JOIN, int NR>
 __global__ __launch_bounds__(256) void add_norm_kernel(T* __restrict__ out, float* __restrict__ residual,
                                                        const void* a0, int t0, const void* a1, int t1, const void* a2,
                                                        int t2, const float* __restrict__ vec,
-                                                       const float* __restrict__ w, int d, float eps, int one_plus) {
+                                                       const float* __restrict__ w, int d, float eps, int one_plus, ExpertSum ex,
+                                                       Route ro) {
   __shared__ float red[4];
   const long row = blockIdx.x;
   float* r = residual + row * d;
   float ss = 0.f;
   if ((d & 7) == 0) {  // 8 columns per thread and trip, 16 / 32-byte accesses
-    for (int c = threadIdx.x * 8; c < d; c += 2048) {
-      float x[8], a[8];
+    auto addend = [&](const void* p, int t, int c, float (&x)[8]) {
+      float a[8];
+      if (JOIN && t == 3) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[i] = 0.f;
+        float v[8];
+#pragma unroll 2
+        for (int k = 0; k < ex.K; ++k) {
+          const float wk = ex.wts[row * ex.K + k];
+          load8(reinterpret_cast<const T*>(ex.ys) + (long)ex.inv[row * ex.K + k] * d + c, v);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) a[i] = fmaf(wk, v[i], a[i]);
+        }
+        if (ex.shared != nullptr) {
+          const float gs = ex.gate != nullptr ? ex.gate[row] : 1.f;
+          load8(reinterpret_cast<const T*>(ex.shared) + row * d + c, v);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) a[i] = fmaf(gs, v[i], a[i]);
+        }
+      } else {
+        load8_any(p, t, row * d + c, a);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] += a[i];
+    };
+    auto sum = [&](int c, float (&x)[8]) {
       load8(r + c, x);
-      if (t0) {
-        load8_any(a0, t0, row * d + c, a);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] += a[i];
-      }
-      if (t1) {
-        load8_any(a1, t1, row * d + c, a);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] += a[i];
-      }
-      if (t2) {
-        load8_any(a2, t2, row * d + c, a);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] += a[i];
-      }
+      if (t0) addend(a0, t0, c, x);
+      if (t1) addend(a1, t1, c, x);
+      if (t2) addend(a2, t2, c, x);
       if (vec != nullptr) {
+        float a[8];
         load8(vec + c, a);
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] += a[i];
@@ -88,16 +127,70 @@ __global__ __launch_bounds__(256) void add_norm_kernel(T* __restrict__ out, floa
       store8(r + c, x);
 #pragma unroll
       for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
+    };
+    const int c0 = threadIdx.x * 8, cc = min(c0, d - 8);
+    float x0[8], g0[8], rw[NR > 0 ? NR : 1][8], acc[NR > 0 ? NR : 1];
+    load8(w + cc, g0);
+#pragma unroll
+    for (int e = 0; e < NR; ++e) {  // rows past rows_w read the last one
+      load8(ro.wr + (long)min(e, ro.rows_w - 1) * d + cc, rw[e]);
+      acc[e] = 0.f;
+    }
+    if (c0 < d) sum(c0, x0);
+    for (int c = c0 + 2048; c < d; c += 2048) {
+      float x[8];
+      sum(c, x);
     }
     ss = block_sum<256>(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float)d + eps);
-    for (int c = threadIdx.x * 8; c < d; c += 2048) {  // each thread re-reads what it wrote
-      float x[8], g[8];
-      load8(r + c, x);
-      load8(w + c, g);
+    auto norm = [&](int c, float (&x)[8], const float (&g)[8]) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] *= inv * (one_plus ? 1.f + g[i] : g[i]);
       store8(out + row * d + c, x);
+    };
+    auto logits = [&](const float (&x)[8], int e, const float (&v)[8]) {
+      T h[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) stf(h + i, x[i]);
+      float a = fmaf(ldf(h), v[0], ldf(h + 1) * v[1]);
+#pragma unroll
+      for (int i = 2; i < 8; ++i) a = fmaf(ldf(h + i), v[i], a);
+      acc[e] += a;
+    };
+    if (c0 < d) {
+      norm(c0, x0, g0);
+#pragma unroll
+      for (int e = 0; e < NR; ++e) logits(x0, e, rw[e]);
+    }
+    for (int c = c0 + 2048; c < d; c += 2048) {  // each thread re-reads what it wrote
+      float x[8], g[8];
+      load8(r + c, x);
+      load8(w + c, g);
+      norm(c, x, g);
+#pragma unroll
+      for (int e = 0; e < NR; ++e) {
+        float v[8];
+        load8(ro.wr + (long)min(e, ro.rows_w - 1) * d + c, v);
+        logits(x, e, v);
+      }
+    }
+    if constexpr (NR > 0) {
+      __shared__ float part[4][NR], lg[NR];
+      __shared__ int sel[kMaxK];
+      const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = threadIdx.x;
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        const float v = wave_sum(acc[j]);
+        if (lane == 0) part[wave][j] = v;
+      }
+      __syncthreads();
+      if (wave > 0) return;
+      if (e < ro.rows_w) {
+        const float a = part[0][e] + part[1][e] + part[2][e] + part[3][e];
+        lg[e] = (e < ro.E && ro.bias != nullptr) ? a + ro.bias[e] : a;
+      }
+      __builtin_amdgcn_wave_barrier();  // a wave's LDS instructions execute in issue order
+      router_choose(lg, sel, ro.ids, ro.wts, ro.gate, row, ro.E, ro.K, ro.over_all);
     }
     return;
   }
@@ -840,16 +933,31 @@ int k8sllm_hy_embed_pos(float* out, const int* ids, const int* positions, const 
   return (int)hipGetLastError();
 }
 
+// An addend of type 3 is the experts' sum (ys ..); r_ids: with the router of the normed rows.  Both want d % 8 == 0, the router at most 9 rows.
 int k8sllm_hy_add_norm(void* out, float* residual, const void* a0, int t0, const void* a1, int t1, const void* a2,
-                       int t2, const float* vec, const float* w, long rows, int d, float eps, int one_plus, int f32,
+                       int t2, const float* vec, const float* w, long rows, int d, float eps, int one_plus, const void* ys,
+                       const int* inv, const float* wts, const void* shared, const float* gate, int K, int* r_ids, float* r_wts,
+                       float* r_gate, const float* wr, const float* bias, int rE, int rK, int rows_w, int over_all, int f32,
                        hipStream_t s) {
   if (rows <= 0) return 0;
-  if (f32)
-    hipLaunchKernelGGL(add_norm_kernel<float>, dim3(rows), dim3(256), 0, s, (float*)out, residual, a0, t0, a1, t1, a2,
-                       t2, vec, w, d, eps, one_plus);
-  else
-    hipLaunchKernelGGL(add_norm_kernel<bf16_t>, dim3(rows), dim3(256), 0, s, (bf16_t*)out, residual, a0, t0, a1, t1,
-                       a2, t2, vec, w, d, eps, one_plus);
+  const bool join = t0 == 3 || t1 == 3 || t2 == 3;
+  if ((join || r_ids != nullptr) && d % 8 != 0) return -1;
+  if (r_ids != nullptr && (d < 8 || rows_w > 9 || rK < 1 || rK > rE || rK > kMaxK || rows_w < rE || rows_w > rE + 1)) return -1;
+  const ExpertSum ex{ys, inv, wts, shared, gate, K};
+  const Route ro{r_ids, r_wts, r_gate, wr, bias, rE, rK, rows_w, over_all};
+#define K8SLLM_AN(T_, J, NR)                                                                                               \
+  hipLaunchKernelGGL((add_norm_kernel<T_, J, NR>), dim3(rows), dim3(256), 0, s, (T_*)out, residual, a0, t0, a1, t1, a2, t2, vec, w, d, \
+                     eps, one_plus, ex, ro)
+#define K8SLLM_ANR(T_, J)                         \
+  if (r_ids == nullptr) K8SLLM_AN(T_, J, 0);      \
+  else if (rows_w <= 8) K8SLLM_AN(T_, J, 8);      \
+  else K8SLLM_AN(T_, J, 9)
+#define K8SLLM_ANJ(T_) \
+  if (join) { K8SLLM_ANR(T_, true); } else { K8SLLM_ANR(T_, false); }
+  if (f32) { K8SLLM_ANJ(float) } else { K8SLLM_ANJ(bf16_t) }
+#undef K8SLLM_ANJ
+#undef K8SLLM_ANR
+#undef K8SLLM_AN
   return (int)hipGetLastError();
 }
 

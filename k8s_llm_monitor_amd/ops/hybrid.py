@@ -29,7 +29,7 @@ from __future__ import annotations
 
 import importlib
 import math
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 import torch.nn.functional as F
@@ -89,12 +89,31 @@ def embed_pos(ids: torch.Tensor, positions: torch.Tensor, embed: torch.Tensor, p
     return out
 
 
+class ExpertSum(NamedTuple):
+    """What moe_experts(join=True) returns on the GPU: the chosen experts' rows, not yet summed.  add_norm takes it as an addend;
+    ``rows()`` is the sum itself (fp32 [T, d])."""
+    ys: torch.Tensor
+    inv: torch.Tensor
+    wts: torch.Tensor
+    shared: Optional[torch.Tensor]
+    gate: Optional[torch.Tensor]
+
+    def rows(self) -> torch.Tensor:
+        out = torch.empty(self.wts.shape[0], self.ys.shape[1], dtype=torch.float32, device=self.ys.device)
+        native().moe_combine(out, self.ys, self.inv, self.wts, self.shared, self.gate, None, None, 0)
+        return out
+
+
 def add_norm(residual: torch.Tensor, addends: tuple, vec: Optional[torch.Tensor], w: torch.Tensor, eps: float,
-             one_plus: bool, out_dtype: torch.dtype) -> torch.Tensor:
+             one_plus: bool, out_dtype: torch.dtype, route: Optional[tuple] = None):
     """``residual`` (fp32 [T, d], updated in place) += sum of ``addends`` ([T, d] each, any float
     dtype, at most three) + ``vec`` ([d], broadcast over the rows); returns the RMSNorm of the new
     residual times ``w`` (``one_plus``: times ``1 + w``) in ``out_dtype``.  The sum and the norm
-    are fp32."""
+    are fp32.  An addend may be an ExpertSum of rows of ``out_dtype`` (``d`` a multiple of 8).  ``route`` (wr, bias, E, K): returns
+    (rows, moe_router's results for them), in one launch for the steps that ``route_with_norm`` names."""
+    if route is not None and not (residual.is_cuda and route_with_norm(*residual.shape, route[0].shape[0])):
+        h = add_norm(residual, addends, vec, w, eps, one_plus, out_dtype)
+        return h, moe_router(h, *route)
     if not residual.is_cuda:
         for a in addends:
             residual += a.float()
@@ -106,8 +125,26 @@ def add_norm(residual: torch.Tensor, addends: tuple, vec: Optional[torch.Tensor]
     assert len(addends) <= 3
     out = torch.empty(residual.shape, dtype=out_dtype, device=residual.device)
     a = list(addends) + [None] * (3 - len(addends))
-    native().add_norm(out, residual, a[0], a[1], a[2], vec, w, float(eps), bool(one_plus))
-    return out
+    at = next((i for i, x in enumerate(a) if isinstance(x, ExpertSum)), -1)
+    if at < 0 and route is None:
+        native().add_norm(out, residual, a[0], a[1], a[2], vec, w, float(eps), bool(one_plus))
+        return out
+    ex: tuple = (None,) * 5
+    if at >= 0:
+        ex, a[at] = a[at], None
+    wr, bias, E, K = route or (None, None, 0, 0)
+    routed: tuple = (None, None, None)
+    if route is not None:
+        T, dev = residual.shape[0], residual.device
+        routed = (torch.empty(T, K, dtype=torch.int32, device=dev), torch.empty(T, K, dtype=torch.float32, device=dev),
+                  torch.empty(T, dtype=torch.float32, device=dev) if wr.shape[0] == E + 1 else None)
+    native().add_norm_experts(out, residual, a[0], a[1], a[2], vec, w, float(eps), bool(one_plus), at, *ex, *routed, wr, bias, E, K, False)
+    return out if route is None else (out, routed)
+
+
+def route_with_norm(T: int, d: int, rows_w: int) -> bool:
+    """Steps whose router runs in the norm's launch: few rows, for a row reads all router weights (hy_router_walk_kernel keeps them for many)."""
+    return T < 256 and d % 8 == 0 and d > 0 and rows_w <= 9
 
 
 def sum_norm(residual: torch.Tensor, addends: tuple, normed: Optional[tuple], w: Optional[torch.Tensor], eps: float,
@@ -1080,7 +1117,7 @@ TILE_MIN_ROWS = 1024
 def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
                 shared: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None, il: bool = False,
                 mfma: bool = True, act: str = "swiglu", limit: float = 0.0, tile: bool = False,
-                identity: int = 0) -> torch.Tensor:
+                identity: int = 0, join: bool = False):
     """Sum over each token's chosen experts of ``wts * down_e(silu(gate_e h) * up_e h)`` with
     ``w13`` [E, 2*ff, d] (gate rows then up rows; ``il``: interleaved per 128 rows as [64 gate |
     64 up], ops.interleave_gate_up) and ``w2`` [E, d, ff], plus ``gate * shared`` (the shared
@@ -1088,7 +1125,7 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
     experts ``down_e(gelu(up_e h))`` with ``w13`` [E, ff, d]; "relu_sq": the same with the squared ReLU.
     ``identity``: ids E .. E + identity - 1 are experts whose output is h itself.  ``act`` "clamped_swish": gated experts whose
     unit is ``g * sigmoid(1.702 g) * (u + 1)`` with g = min(gate_e h, limit), u = clamp(up_e h, -limit,
-    limit).  fp32 [T, d].
+    limit).  fp32 [T, d]; ``join``: on the GPU, where add_norm can form the sum, an ExpertSum.
 
     GPU: the (token, slot) pairs are counting-sorted by expert on the device and both projections
     run as ONE grouped launch each over the sorted rows (SwiGLU in the first epilogue); no host
@@ -1151,6 +1188,8 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torc
         ext.grouped_gemm(a, h, w13, offsets, sorted_idx, K, code, il, mfma, float(limit))
         ys = torch.empty(n, d, dtype=h.dtype, device=h.device)
         ext.grouped_gemm(ys, a, w2, offsets, None, 1, 0, False, mfma, 0.0)
+    if join and not identity and d % 8 == 0:
+        return ExpertSum(ys, inv_idx, wts, shared, gate)
     out = torch.empty(T, d, dtype=torch.float32, device=h.device)
     ext.moe_combine(out, ys, inv_idx, wts, shared, gate, ids if identity else None, h if identity else None, E)
     return out

@@ -1280,3 +1280,39 @@ def test_values_to_pages_in_runs(T, Hq, G, dk, dv, nf, extra, pairs, dt):
         assert torch.equal(got[0][:, (Hq + G) * dk:], want[0][:, (Hq + G) * dk:])
         torch.testing.assert_close(got[0].float(), want[0].float(), **tol)
         torch.testing.assert_close(got[1].float(), want[1].float(), **tol)
+
+
+@pytest.mark.parametrize("T,d,E,K,at,shared,dt", [
+    (1, 8, 3, 1, 0, False, BF), (3, 264, 8, 2, 1, True, BF), (64, 2048, 8, 2, 1, False, BF), (255, 2056, 7, 5, 2, True, BF),
+    (256, 4104, 8, 8, 1, True, BF), (300, 1024, 5, 3, 1, False, BF), (37, 1000, 8, 2, 1, True, torch.float32), (64, 4096, 9, 2, 0, False, torch.float32),
+    (5, 24, 12, 2, 1, True, BF),  # more weight rows than the norm's launch takes
+])
+def test_experts_sum_and_router_with_the_norm(T, d, E, K, at, shared, dt):
+    """add_norm that forms the experts' sum and routes its rows, against the launches it replaces: the same bits; and against the fp32 form
+    (a bf16 row's rounding)."""
+    g = _g(91)
+    x = _r(g, T, d)
+    ys, wts = _r(g, T * K, d, dt=dt), torch.rand(T, K, generator=g)
+    sh, gate = (_r(g, T, d, dt=dt), torch.rand(T, generator=g)) if shared else (None, None)
+    inv = torch.randperm(T * K, generator=g).to(torch.int32)
+    adds = [_r(g, T, d, dt=dt), _r(g, T, d)]
+    w, vec = torch.rand(d, generator=g), _r(g, d)
+    wr, bias = _r(g, E + int(shared), d, s=d ** -0.5), _r(g, E)
+    dev = lambda t: t.cuda() if t is not None else None
+    ex = hops.ExpertSum(*map(dev, (ys, inv, wts, sh, gate)))
+    route = (wr.cuda(), bias.cuda(), E, K)
+    cadds = [a.cuda() for a in adds]
+    x1, x2, x3 = (x.cuda() for _ in range(3))
+    h1 = hops.add_norm(x1, tuple(cadds[:at] + [ex.rows()] + cadds[at:]), vec.cuda(), w.cuda(), 1e-5, True, dt)
+    r1 = hops.moe_router(h1, *route)
+    fused = tuple(cadds[:at] + [ex] + cadds[at:])
+    h2, r2 = hops.add_norm(x2, fused, vec.cuda(), w.cuda(), 1e-5, True, dt, route=route)
+    h3 = hops.add_norm(x3, fused, vec.cuda(), w.cuda(), 1e-5, True, dt)
+    for a, b in ((x1, x2), (x1, x3), (h1, h2), (h1, h3), *((a, b) for a, b in zip(r1, r2) if a is not None)):
+        assert torch.equal(a, b)
+    s = (wts.unsqueeze(-1) * ys.float()[inv.long()].view(T, K, d)).sum(1)
+    if shared:
+        s += gate.unsqueeze(-1) * sh.float()
+    want = hops.add_norm(x, tuple(adds[:at] + [s] + adds[at:]), vec, w, 1e-5, True, dt)
+    tol = 2 ** -7 if dt == BF else 1e-5
+    torch.testing.assert_close(h2.cpu().float(), want.float(), rtol=tol, atol=tol)
