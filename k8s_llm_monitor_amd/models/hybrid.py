@@ -372,19 +372,14 @@ class LatentAttention:
     def _forward_latent(self, q: torch.Tensor, pos: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
                         runs: list) -> torch.Tensor:
         """Attention over the latent pages: rows ``q``, in ``runs`` of (first row, end, their pages, what they see of them)."""
-        H, dn, dr, dv, R = self.H, self.dn, self.dr, self.dv, self.R
-        T = q.shape[0]
+        H, dn, dr = self.H, self.dn, self.dr
         # the per-head key expansion moved to the query: q_lat[h] = q_unrotated[h] @ W_uk[h]  ([H, T, R])
-        q_lat = torch.bmm(q.view(T, H, dn + dr)[:, :, :dn].transpose(0, 1), self.w_uk.view(H, dn, R))
-        qa = hops.latent_queries(q, q_lat, H, dn, dr, pos, self.freq, self.pitch, pairs=self.pairs)
+        qa = hops.latent_head_queries(q, self.w_uk, H, dn, dr, pos, self.freq, self.pitch, pairs=self.pairs)
         parts = [hops.latent_attention(qa[a:b], kc, vc, tables, H, self.scale, self.window, self.sinks, fast=self.fast, sink=self.sink,
                                        gate=gate[a:b] if gate is not None else None, **seen) for a, b, tables, seen in runs]
         o = parts[0] if len(parts) == 1 else torch.cat(parts)
-        # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T, written head by head
-        # into the rows the out-projection reads
-        v = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
-        torch.bmm(o.view(T, H, R).transpose(0, 1), self.w_uv.view(H, dv, R).transpose(1, 2), out=v.transpose(0, 1))
-        return v.view(T, H * dv)
+        # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T
+        return hops.latent_head_values(o, self.w_uv, H)
 
     def _expand_ok(self, h: torch.Tensor, meta: AttnMeta) -> bool:
         rows = h.shape[0] - meta.num_decode

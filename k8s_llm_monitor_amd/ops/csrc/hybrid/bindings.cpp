@@ -109,6 +109,9 @@ int k8sllm_hy_activation(void* out, const void* x, long n, int kind, float a, fl
 int k8sllm_hy_latent_prep(void* proj, long stride, long T, int Q, int R, int dr, const float* qw, const float* kw,
                           float eps, const int* positions, const float* freq, int nf, int pairs, void* k_cache,
                           int kw_pitch, void* v_cache, const int* slots, int bs, int f32, hipStream_t s);
+int k8sllm_hy_latent_head_queries(void* out, const void* q, long q_stride, const void* wk, long T, int H, int dn, int dr, int R, int w,
+                                  const int* positions, const float* freq, int nf, int pairs, hipStream_t s);
+int k8sllm_hy_latent_head_values(void* v, const void* o, const void* wv, long T, int H, int dv, int R, hipStream_t s);
 int k8sllm_hy_latent_queries(void* out, const void* q, long q_stride, const void* q_lat, long T, int H, int dn, int dr,
                              int R, int w, const int* positions, const float* freq, int nf, int pairs, int f32,
                              hipStream_t s);
@@ -1190,6 +1193,39 @@ void latent_queries(Tensor out, Tensor q, Tensor q_lat, int64_t H, int64_t dn, i
         "latent_queries");
 }
 
+// q_lat = q W per head and latent_queries of it, in one launch (bf16); wk [H * dn, R]
+void latent_head_queries(Tensor out, Tensor q, Tensor wk, int64_t H, int64_t dn, int64_t dr, Tensor positions, Tensor freq, bool pairs) {
+  same(q, 0, "q");
+  same(out, 0, "out");
+  same(wk, 0, "w_uk");
+  f32c(freq, "freq");
+  i32c(positions, "positions");
+  const int64_t T = q.size(0);
+  TORCH_CHECK(H >= 1 && q.dim() == 2 && q.stride(1) == 1 && q.size(1) == H * (dn + dr), "q [T, H * (dim + rot)]");
+  TORCH_CHECK(wk.dim() == 2 && wk.is_contiguous() && wk.size(0) == H * dn, "w_uk [H * dim, R]");
+  const int64_t R = wk.size(1);
+  TORCH_CHECK(out.dim() == 2 && out.is_contiguous() && out.size(0) == T && out.size(1) % H == 0 && out.size(1) / H >= R + dr &&
+                  positions.numel() >= T && 2 * freq.numel() <= dr,
+              "latent_head_queries: out [T, H * pitch] / positions / freq");
+  check(k8sllm_hy_latent_head_queries(out.data_ptr(), q.data_ptr(), q.stride(0), wk.data_ptr(), T, (int)H, (int)dn, (int)dr, (int)R,
+                                      (int)(out.size(1) / H), positions.data_ptr<int>(), freq.data_ptr<float>(), (int)freq.numel(), pairs,
+                                      cur()),
+        "latent_head_queries");
+}
+
+// v[t][h] = W[h] o[t][h] (bf16); wv [H * dv, R]
+void latent_head_values(Tensor v, Tensor o, Tensor wv, int64_t H) {
+  same(v, 0, "v");
+  same(o, 0, "o");
+  same(wv, 0, "w_uv");
+  const int64_t T = o.size(0);
+  TORCH_CHECK(H >= 1 && wv.dim() == 2 && wv.is_contiguous() && wv.size(0) % H == 0, "w_uv [H * vdim, R]");
+  const int64_t dv = wv.size(0) / H, R = wv.size(1);
+  TORCH_CHECK(o.dim() == 2 && o.is_contiguous() && o.size(1) == H * R && v.is_contiguous() && v.numel() == T * H * dv,
+              "latent_head_values: o [T, H * R], v [T, H * vdim]");
+  check(k8sllm_hy_latent_head_values(v.data_ptr(), o.data_ptr(), wv.data_ptr(), T, (int)H, (int)dv, (int)R, cur()), "latent_head_values");
+}
+
 // The matrix-core latent attention; false: these sizes or dtype are not the kernel's, nothing was
 // launched.  cu / ctx given: prompt chunks (block_tables per segment); else one row per sequence.
 bool latent_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, OptT cu, OptT ctx, OptT seq_lens,
@@ -1260,6 +1296,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("activation", &activation);
   m.def("latent_prep", &latent_prep);
   m.def("latent_queries", &latent_queries);
+  m.def("latent_head_queries", &latent_head_queries);
+  m.def("latent_head_values", &latent_head_values);
   m.def("latent_attention", &latent_attention);
   m.def("sum_norm", &sum_norm);
   m.def("gated_lookup", &gated_lookup);

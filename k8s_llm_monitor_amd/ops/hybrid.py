@@ -710,6 +710,43 @@ def latent_queries(q: torch.Tensor, q_lat: torch.Tensor, H: int, dim: int, rot_d
     return out
 
 
+# Up to these rows the per-head products of latent attention are latent_heads.hip's.  Us, library (with the rows put together) / own: queries,
+# 8 heads of 96 + 32 over 256, 1 row 11.6 / 4.2, 64 13.5 / 4.7, 2048 23 / 10.7; 32 of 128 + 64 over 512, 64 rows 45 / 7.5, 2048 101 / 94.  Values,
+# 8 of 128 over 256, 1 row 7.3 / 4.5, 256 9.7 / 5.9, 512 5.6 / 7.6; 32 of 128 over 512, 64 rows 9.4 / 8.5, 128 10.5 / 11.1, 256 14.3 / 19.4: there by
+# their multiplications too.
+HEAD_QUERY_ROWS, HEAD_VALUE_ROWS, HEAD_VALUE_WORK = 2048, 256, 1 << 28
+
+
+def _head_rows(most: int, *ts: torch.Tensor) -> bool:
+    return (ts[0].is_cuda and ts[0].shape[0] <= most and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in ts)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)))
+
+
+def latent_head_queries(q: torch.Tensor, w_uk: torch.Tensor, H: int, dim: int, rot_dim: int, positions: torch.Tensor,
+                        freq: torch.Tensor, pitch: int = 0, pairs: bool = False) -> torch.Tensor:
+    """latent_queries of the unrotated parts times each head's key expansion ``w_uk`` [H * dim, R]."""
+    T, R = q.shape[0], w_uk.shape[1]
+    pitch = pitch or R + rot_dim
+    if _head_rows(HEAD_QUERY_ROWS, q, w_uk) and not (dim % 8 or rot_dim % 8 or R % 8 or pitch % 8 or q.stride(0) % 8):
+        out = torch.empty(T, H * pitch, dtype=q.dtype, device=q.device)
+        native().latent_head_queries(out, q, w_uk, int(H), int(dim), int(rot_dim), positions, freq, bool(pairs))
+        return out
+    q_lat = torch.bmm(q.view(T, H, dim + rot_dim)[:, :, :dim].transpose(0, 1), w_uk.view(H, dim, R))
+    return latent_queries(q, q_lat, H, dim, rot_dim, positions, freq, pitch, pairs)
+
+
+def latent_head_values(o: torch.Tensor, w_uv: torch.Tensor, H: int) -> torch.Tensor:
+    """Per head ``W_uv[h] o[t][h]``: [T, H * R] and ``w_uv`` [H * vdim, R] -> [T, H * vdim]."""
+    T, R = o.shape[0], w_uv.shape[1]
+    dv = w_uv.shape[0] // H
+    v = torch.empty(T, H, dv, dtype=o.dtype, device=o.device)
+    if _head_rows(HEAD_VALUE_ROWS, o, w_uv) and R % 8 == 0 and T * H * dv * R < HEAD_VALUE_WORK:
+        native().latent_head_values(v, o, w_uv, int(H))
+    else:  # written head by head into the rows that the out-projection reads
+        torch.bmm(o.view(T, H, R).transpose(0, 1), w_uv.view(H, dv, R).transpose(1, 2), out=v.transpose(0, 1))
+    return v.view(T, H * dv)
+
+
 def rotate_heads(x: torch.Tensor, heads: int, dim: int, positions: torch.Tensor, freq: torch.Tensor, pairs: bool,
                  rot_off: int = 0) -> None:
     """In place on rows [T, heads * dim]: entries ``rot_off .. rot_off + 2 len(freq)`` of every head turn by the

@@ -1316,3 +1316,29 @@ def test_experts_sum_and_router_with_the_norm(T, d, E, K, at, shared, dt):
     want = hops.add_norm(x, tuple(adds[:at] + [s] + adds[at:]), vec, w, 1e-5, True, dt)
     tol = 2 ** -7 if dt == BF else 1e-5
     torch.testing.assert_close(h2.cpu().float(), want.float(), rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("T,H,dn,dr,dv,R,pitch,nf,pairs,sliced", [
+    (1, 8, 96, 32, 128, 256, 288, 16, False, False), (16, 3, 8, 8, 16, 8, 16, 4, True, False), (17, 5, 40, 8, 24, 72, 96, 2, False, False),
+    (33, 2, 128, 64, 40, 136, 224, 32, True, False), (70, 4, 64, 32, 65, 128, 160, 0, False, False), (2048, 1, 32, 8, 16, 128, 160, 4, True, False),
+    (2049, 1, 32, 8, 16, 128, 160, 4, False, False), (256, 2, 24, 8, 7, 264, 288, 4, False, False), (257, 2, 24, 8, 7, 264, 288, 4, False, False),
+    (9, 2, 20, 6, 12, 36, 42, 3, True, False),  # not in 16-byte pieces
+    (5, 2, 32, 32, 32, 64, 96, 16, False, True),  # rows inside wider ones (two heads of 64)
+])
+def test_latent_heads(T, H, dn, dr, dv, R, pitch, nf, pairs, sliced):
+    """Per-head products around latent attention at and around tiles of 16 rows and 128 columns and the sizes that leave them.  fp32 sums of
+    bf16 products, one rounding: 2^-8 of the value; the turned part the same; copies and zeros equal."""
+    g = _g(92)
+    q = _r(g, T, H * (dn + dr) * (2 if sliced else 1), dt=BF)
+    wk, wv, o = _r(g, H * dn, R, s=R ** -0.5, dt=BF), _r(g, H * dv, R, s=R ** -0.5, dt=BF), _r(g, T, H * R, dt=BF)
+    pos, freq = torch.randint(0, 4000, (T,), generator=g, dtype=torch.int32), hops.rotary_freq(1e4, nf)
+    cut = lambda t: t[:, :H * (dn + dr)]
+    lat = torch.bmm(cut(q).reshape(T, H, dn + dr)[:, :, :dn].transpose(0, 1).float().contiguous(), wk.view(H, dn, R).float()).to(BF)
+    want = hops.latent_queries(cut(q).contiguous(), lat, H, dn, dr, pos, freq, pitch, pairs).view(T, H, pitch)
+    gq = cut(q.cuda())
+    got = hops.latent_head_queries(gq, wk.cuda(), H, dn, dr, pos.cuda(), freq.cuda(), pitch, pairs).cpu().view(T, H, pitch)
+    torch.testing.assert_close(got.float(), want.float(), rtol=2 ** -7, atol=2 ** -7)
+    assert torch.equal(got[..., R + 2 * nf:], want[..., R + 2 * nf:])
+    v = torch.bmm(o.view(T, H, R).transpose(0, 1).float().contiguous(), wv.view(H, dv, R).transpose(1, 2).float().contiguous())
+    got = hops.latent_head_values(o.cuda(), wv.cuda(), H).cpu().view(T, H, dv)
+    torch.testing.assert_close(got.float(), v.transpose(0, 1), rtol=2 ** -7, atol=2 ** -7)
