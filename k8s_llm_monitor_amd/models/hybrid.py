@@ -126,10 +126,12 @@ def _take(rows, *ts: torch.Tensor) -> tuple:
 def _attend_ends(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, meta: AttnMeta, *args, gate: Optional[torch.Tensor] = None,
                  **kw) -> torch.Tensor:
     """Windowed attention of a prefill step's decode rows and each chunk's last row (``q``, in that order) as decode rows."""
-    nd = meta.num_decode
-    parts = [hops.window_attention_decode(q[a:b], kc, vc, bt, n, *args, gate=gate[a:b] if gate is not None else None, **kw)
-             for a, b, bt, n in ((0, nd, meta.dec_block_tables, meta.dec_seq_lens), (nd, q.shape[0], meta.block_tables, meta.ends)) if b > a]
-    return parts[0] if len(parts) == 1 else torch.cat(parts)
+    nd, (H, _, _, dv) = meta.num_decode, args[:4]
+    out = torch.empty(q.shape[0], H * dv, dtype=q.dtype, device=q.device)
+    for a, b, bt, n in ((0, nd, meta.dec_block_tables, meta.dec_seq_lens), (nd, q.shape[0], meta.block_tables, meta.ends)):
+        if b > a:
+            hops.window_attention_decode(q[a:b], kc, vc, bt, n, *args, gate=gate[a:b] if gate is not None else None, out=out[a:b], **kw)
+    return out
 
 
 class WindowAttention:
@@ -180,12 +182,12 @@ class WindowAttention:
             # mfma 2: the register kernel.  The staged one (201 -> 88 us at 4 x 2048 rows, 16 heads) rounds the weights against
             # another running maximum, and this design's routers - the softmax over the two best of near-equal logits - turn such
             # differences into other experts: recurrent states behind them moved by more than their root mean square.
-            o = hops.window_attention_prefill(qkv[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
-                                              *args, mfma=2 if self.fast == 1 else self.fast)
+            o = torch.empty(qkv.shape[0], H * dv, dtype=qkv.dtype, device=qkv.device)
+            hops.window_attention_prefill(qkv[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
+                                          *args, mfma=2 if self.fast == 1 else self.fast, out=o[nd:])
             if nd:  # a mixed step: the single decode tokens in front go through the decode kernel
-                od = hops.window_attention_decode(qkv[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
-                                                  vec=bool(self.fast))
-                o = torch.cat([od, o])
+                hops.window_attention_decode(qkv[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
+                                             vec=bool(self.fast), out=o[:nd])
             (o,) = _take(rows, o)
         return F.linear(o, self.wo)
 
@@ -352,17 +354,16 @@ class LatentAttention:
         T = q.shape[0]
         ex = not ends and self._expand_ok(h, meta)
         nd = meta.num_decode if meta.is_prefill else T  # single-token rows in front
-        parts = []
+        o = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
         if nd or not ex:
             n = nd if ex else T
             # (first row, end, pages, whose positions they see) of attention over the latent pages
             runs = [(0, T, meta.block_tables, dict(seq_lens=meta.seq_lens))] if not meta.is_prefill else [
                 (0, nd, meta.dec_block_tables, dict(seq_lens=meta.dec_seq_lens)),
                 (nd, n, meta.block_tables, dict(seq_lens=meta.ends) if ends else dict(cu=meta.cu_seqlens, ctx=meta.ctx_start))]
-            parts.append(self._forward_latent(q[:n], pos, kc, vc, gate, [r for r in runs if r[1] > r[0]]))
+            self._forward_latent(q[:n], pos, kc, vc, gate, [r for r in runs if r[1] > r[0]], o[:n])
         if ex:
-            parts.append(self._forward_expanded(q[nd:], meta, kc, gate[nd:] if gate is not None else None))
-        o = parts[0] if len(parts) == 1 else torch.cat(parts)
+            self._forward_expanded(q[nd:], meta, kc, gate[nd:] if gate is not None else None, o[nd:])
         if rows is not None and not ends:
             o, proj = _take(rows, o, proj)
         if self.n_tail:
@@ -370,8 +371,8 @@ class LatentAttention:
         return hops.linear(o, self.wo)
 
     def _forward_latent(self, q: torch.Tensor, pos: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
-                        runs: list) -> torch.Tensor:
-        """Attention over the latent pages: rows ``q``, in ``runs`` of (first row, end, their pages, what they see of them)."""
+                        runs: list, out: torch.Tensor) -> None:
+        """Attention over the latent pages: rows ``q``, in ``runs`` of (first row, end, their pages, what they see of them), into ``out``."""
         H, dn, dr = self.H, self.dn, self.dr
         # the per-head key expansion moved to the query: q_lat[h] = q_unrotated[h] @ W_uk[h]  ([H, T, R])
         qa = hops.latent_head_queries(q, self.w_uk, H, dn, dr, pos, self.freq, self.pitch, pairs=self.pairs)
@@ -379,7 +380,7 @@ class LatentAttention:
                                        gate=gate[a:b] if gate is not None else None, **seen) for a, b, tables, seen in runs]
         o = parts[0] if len(parts) == 1 else torch.cat(parts)
         # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T
-        return hops.latent_head_values(o, self.w_uv, H)
+        hops.latent_head_values(o, self.w_uv, H, out)
 
     def _expand_ok(self, h: torch.Tensor, meta: AttnMeta) -> bool:
         rows = h.shape[0] - meta.num_decode
@@ -401,27 +402,26 @@ class LatentAttention:
                 cuts.append(i)
         return list(zip(cuts, cuts[1:] + [len(seen.ends)]))
 
-    def _forward_expanded(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def _forward_expanded(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, gate: Optional[torch.Tensor], out: torch.Tensor) -> None:
         """Prompt rows: per-head keys and values of every position they see in temporary pages, windowed
-        attention's matrix-core kernel over them.  ``q`` [rows, H * (dim + rot_dim)] still unturned."""
+        attention's matrix-core kernel over them, into ``out``.  ``q`` [rows, H * (dim + rot_dim)] still unturned."""
         H, dn, dr, dv = self.H, self.dn, self.dr, self.dv
         nd = meta.num_decode
         seen = meta.page_lists[self.window]
         hops.rotate_heads(q, H, dn + dr, meta.positions[nd:], self.freq, self.pairs, dn)
 
-        def attend(pages, q, cu, ctx, tables, gate):
+        def attend(pages, q, cu, ctx, tables, gate, out):
             kt, vt = hops.latent_expand(kc, pages, self.w_uk, self.w_uv, H, self.R, dr)
-            return hops.window_attention_prefill(q, kt, vt, cu, ctx, tables, H, H, dn + dr, dv, self.scale, self.window, self.sink,
-                                                 mfma=self.fast, sinks=self.sinks, gate=gate)
+            hops.window_attention_prefill(q, kt, vt, cu, ctx, tables, H, H, dn + dr, dv, self.scale, self.window, self.sink,
+                                          mfma=self.fast, sinks=self.sinks, gate=gate, out=out)
 
         if seen.ends[-1] <= self.most_pages:
-            return attend(seen.pages, q, meta.cu_seqlens, meta.ctx_start, seen.tables, gate)
-        out = []
+            attend(seen.pages, q, meta.cu_seqlens, meta.ctx_start, seen.tables, gate, out)
+            return
         for a, b in self._expand_groups(seen):  # (one group's pages are given back before the next one's are made)
             r, p = meta.chunk_rows[a:b + 1:b - a].tolist(), ([0] + seen.ends)[a:b + 1:b - a]
-            out.append(attend(seen.pages[p[0]:p[1]], q[r[0]:r[1]], meta.cu_seqlens[a:b + 1] - r[0], meta.ctx_start[a:b],
-                              seen.tables[a:b] - p[0], gate[r[0]:r[1]] if gate is not None else None))
-        return torch.cat(out)
+            attend(seen.pages[p[0]:p[1]], q[r[0]:r[1]], meta.cu_seqlens[a:b + 1] - r[0], meta.ctx_start[a:b],
+                   seen.tables[a:b] - p[0], gate[r[0]:r[1]] if gate is not None else None, out[r[0]:r[1]])
 
 
 class RotaryAttention:
@@ -516,8 +516,8 @@ class RotaryAttention:
         hops.rotary_cache(proj, H, G, dk, dv, meta.positions, self.freq, self.pairs, self.temp, kc, vc, meta.slot_mapping,
                           norm=self.norm, qw=self.qn, kw=self.kn, eps=self.eps, v_from_k=self.v_from_k)
         args = (H, G, dk, dv, self.scale, self.window, self.sink)
-        kw = dict(sinks=self.sinks, chunked=self.chunked, cap=self.cap, keep=self.keep, g_col=self.g_col)
-        hg = self.gate_heads
+        kw = dict(sinks=self.sinks, chunked=self.chunked, cap=self.cap, keep=self.keep, g_col=self.g_col, by_value=not self.gate_heads)
+        hg = self.has_gate
         if not meta.is_prefill:
             o = hops.window_attention_decode(proj, kc, vc, meta.block_tables, meta.seq_lens, *args, vec=bool(self.fast),
                                              gate=proj if hg else None, **kw)
@@ -526,17 +526,15 @@ class RotaryAttention:
             o = _attend_ends(proj, kc, vc, meta, *args, vec=bool(self.fast), gate=proj if hg else None, **kw)
         else:
             nd = meta.num_decode
-            o = hops.window_attention_prefill(proj[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
-                                              *args, mfma=self.fast, gate=proj[nd:] if hg else None, **kw)
+            o = torch.empty(proj.shape[0], H * dv, dtype=proj.dtype, device=proj.device)
+            hops.window_attention_prefill(proj[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
+                                          *args, mfma=self.fast, gate=proj[nd:] if hg else None, out=o[nd:], **kw)
             if nd:
-                od = hops.window_attention_decode(proj[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
-                                                  vec=bool(self.fast), gate=proj[:nd] if hg else None, **kw)
-                o = torch.cat([od, o])
+                hops.window_attention_decode(proj[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
+                                             vec=bool(self.fast), gate=proj[:nd] if hg else None, out=o[:nd], **kw)
             o, proj = _take(rows, o, proj)
         if self.n_tail:
             self.tail_out = (proj, self.n_in)
-        if self.has_gate and not hg:
-            o = hops.sigmoid_gate(o, proj, self.g_col)
         return hops.linear(o, self.wo)
 
     def export(self, p: str) -> dict:

@@ -55,12 +55,13 @@ int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float
 int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                              const int* cu, const int* ctx, const int* block_tables, int bt_stride, int S, long T,
                              int Hq, int G, int dk, int dv, int bs, float scale, int window, int chunked, int keep,
-                             float cap, int sink, const float* sinks, const void* gate, long g_stride, int f32, int mfma,
-                             hipStream_t s);
+                             float cap, int sink, const float* sinks, const void* gate, long g_stride, int* by_value, int f32,
+                             int mfma, hipStream_t s);
 int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                             const int* block_tables, int bt_stride, const int* seq_lens, int B, int Hq, int G, int dk,
                             int dv, int bs, float scale, int window, int chunked, int keep, float cap, int sink,
-                            const float* sinks, const void* gate, long g_stride, int f32, int vec, int heads, hipStream_t s);
+                            const float* sinks, const void* gate, long g_stride, int* by_value, int f32, int vec, int heads,
+                            hipStream_t s);
 int k8sllm_hy_conv_silu(void* out, const void* proj, long stride, int col0, int C, const float* cw, const float* cb,
                         int taps, void* state, const int* cu, const int* ctx, const int* slot, int S, long T, int f32,
                         hipStream_t s);
@@ -387,13 +388,19 @@ struct Gate {
   const void* p = nullptr;
   long stride = 0;
 };
-Gate gate_of(const OptT& gate, int64_t g_col, int64_t rows, int64_t Hq, int f) {
+// n logits a row: one per head, or (by_value, and then a kernel may take it if the rows are in 16-byte pieces) per value
+Gate gate_of(const OptT& gate, int64_t g_col, int64_t rows, int64_t n, int f, int* by_value) {
   Gate g;
   if (!gate.has_value()) return g;
   same(*gate, f, "gate");
-  TORCH_CHECK(gate->dim() == 2 && gate->stride(1) == 1 && gate->size(0) >= rows && g_col >= 0 && g_col + Hq <= gate->size(1),
-              "gate [T, >= g_col + heads]");
-  g.p = (const char*)gate->data_ptr() + g_col * gate->element_size();
+  TORCH_CHECK(gate->dim() == 2 && gate->stride(1) == 1 && gate->size(0) >= rows && g_col >= 0 && g_col + n <= gate->size(1),
+              "gate [T, >= g_col + heads (by value: + heads * vdim)]");
+  const void* p = (const char*)gate->data_ptr() + g_col * gate->element_size();
+  if (*by_value && (f || gate->stride(0) % 8 || reinterpret_cast<uintptr_t>(p) % 16)) {
+    *by_value = 0;  // the caller gates the rows
+    return g;
+  }
+  g.p = p;
   g.stride = gate->stride(0);
   return g;
 }
@@ -423,10 +430,11 @@ void qk_norm_cache(Tensor qkv, Tensor qw, Tensor kw, double eps, int64_t Hq, int
         "qk_norm_cache");
 }
 
-void window_attention_prefill(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_cache, Tensor cu, Tensor ctx,
+// true: the rows are gated (see by_value)
+bool window_attention_prefill(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_cache, Tensor cu, Tensor ctx,
                               Tensor block_tables, int64_t Hq, int64_t G, int64_t dk, int64_t dv, double scale,
                               int64_t window, bool sink, OptT sinks, int64_t mfma, bool chunked, double cap,
-                              int64_t keep, OptT gate, int64_t g_col) {
+                              int64_t keep, OptT gate, int64_t g_col, bool by_value) {
   const int f = act(qkv, "qkv");
   same(out, f, "out");
   pages(k_cache, f, G * dk, "k_cache");
@@ -442,19 +450,21 @@ void window_attention_prefill(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_c
   TORCH_CHECK(cu.numel() == S + 1 && block_tables.size(0) >= S, "cu [S+1], block_tables [S, W]");
   TORCH_CHECK(window >= 0 && G >= 1 && Hq % G == 0 && cap >= 0, "heads / window / cap");
   TORCH_CHECK(keep >= 0 && (keep == 0 || (window > 0 && !chunked)), "kept first positions go with a sliding window");
-  const Gate ga = gate_of(gate, g_col, T, Hq, f);
+  int wide = by_value && gate.has_value();
+  const Gate ga = gate_of(gate, g_col, T, wide ? Hq * dv : Hq, f, &wide);
   check(k8sllm_hy_window_prefill(out.data_ptr(), qkv.data_ptr(), qkv.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                                  cu.data_ptr<int>(), ctx.data_ptr<int>(), block_tables.data_ptr<int>(),
                                  (int)block_tables.stride(0), (int)S, T, (int)Hq, (int)G, (int)dk, (int)dv,
                                  (int)k_cache.size(1), (float)scale, (int)window, chunked, (int)keep, (float)cap, sink,
-                                 sink_ptr(sinks, Hq), ga.p, ga.stride, f, (int)mfma, cur()),
+                                 sink_ptr(sinks, Hq), ga.p, ga.stride, &wide, f, (int)mfma, cur()),
         "window_attention_prefill");
+  return wide != 0;
 }
 
-void window_attention_decode(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_cache, Tensor block_tables,
+bool window_attention_decode(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_cache, Tensor block_tables,
                              Tensor seq_lens, int64_t Hq, int64_t G, int64_t dk, int64_t dv, double scale,
                              int64_t window, bool sink, OptT sinks, bool vec, bool chunked, double cap, int64_t keep,
-                             OptT gate, int64_t g_col, int64_t heads) {
+                             OptT gate, int64_t g_col, int64_t heads, bool by_value) {
   const int f = act(qkv, "qkv");
   same(out, f, "out");
   pages(k_cache, f, G * dk, "k_cache");
@@ -469,13 +479,15 @@ void window_attention_decode(Tensor out, Tensor qkv, Tensor k_cache, Tensor v_ca
   TORCH_CHECK(seq_lens.numel() >= B && block_tables.size(0) >= B, "seq_lens [B], block_tables [B, W]");
   TORCH_CHECK(window >= 0 && G >= 1 && Hq % G == 0 && cap >= 0, "heads / window / cap");
   TORCH_CHECK(keep >= 0 && (keep == 0 || (window > 0 && !chunked)), "kept first positions go with a sliding window");
-  const Gate ga = gate_of(gate, g_col, B, Hq, f);
+  int wide = by_value && gate.has_value();
+  const Gate ga = gate_of(gate, g_col, B, wide ? Hq * dv : Hq, f, &wide);
   check(k8sllm_hy_window_decode(out.data_ptr(), qkv.data_ptr(), qkv.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                                 block_tables.data_ptr<int>(), (int)block_tables.stride(0), seq_lens.data_ptr<int>(),
                                 (int)B, (int)Hq, (int)G, (int)dk, (int)dv, (int)k_cache.size(1), (float)scale,
                                 (int)window, chunked, (int)keep, (float)cap, sink, sink_ptr(sinks, Hq), ga.p, ga.stride,
-                                f, vec, (int)heads, cur()),
+                                &wide, f, vec, (int)heads, cur()),
         "window_attention_decode");
+  return wide != 0;
 }
 
 void segs(const Tensor& cu, const Tensor& ctx, const Tensor& slot) {
@@ -1255,7 +1267,8 @@ bool latent_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, OptT
     TORCH_CHECK(slp != nullptr && seq_lens->numel() >= T && block_tables.size(0) >= T, "seq_lens [T], block_tables [T, W]");
   }
   TORCH_CHECK(window >= 0 && H >= 1, "heads / window");
-  const Gate ga = gate_of(gate, g_col, T, H, 0);
+  int by_head = 0;
+  const Gate ga = gate_of(gate, g_col, T, H, 0, &by_head);
   const int rc = k8sllm_hy_latent_attention(out.data_ptr(), q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                                             cup, ctxp, slp, block_tables.data_ptr<int>(), (int)block_tables.stride(0), (int)S, T,
                                             (int)H, (int)dkp, (int)dv, (int)k_cache.size(1), (float)scale, (int)window,

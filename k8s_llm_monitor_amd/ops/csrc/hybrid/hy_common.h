@@ -101,6 +101,15 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
 __device__ __forceinline__ float silu_f(float z) { return z / (1.f + __expf(-z)); }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
 
+// four rounded values times the sigmoids of their logits, rounded again
+__device__ __forceinline__ uint2 gate_rounded(uint2 x, uint2 z) {
+  auto half = [](uint32_t a, uint32_t b) {
+    return pack2(__uint_as_float(a << 16) * sigmoid_f(__uint_as_float(b << 16)),
+                 __uint_as_float(a & 0xffff0000u) * sigmoid_f(__uint_as_float(b & 0xffff0000u)));
+  };
+  return make_uint2(half(x.x, z.x), half(x.y, z.y));
+}
+
 // Where row tile ``tile`` of ROWS rows lies among experts whose rows are offsets[e] .. offsets[e + 1] - 1: expert e, its rows r0 .. r1 - 1 and the
 // tile's number in it; false behind the last.  Up to 64 experts one after another, from the scalar cache; more of them 64 at a time, a
 // lane each (the sum over 64 takes about 1 us, of a load that waits behind the weights': 2 rows beside 128 experts 46 -> 13 us, 64 rows

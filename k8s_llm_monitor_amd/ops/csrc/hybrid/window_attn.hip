@@ -9,7 +9,8 @@
 // from position 0 of the sequence).  keep > 0 (window form): the first ``keep`` positions of the sequence stay
 // visible to every later row besides its window.  cap > 0: a score s (after the scale) becomes cap * tanh(s / cap).
 // gate (optional, rows g_stride apart, one logit per query head): a head's output is multiplied by
-// sigmoid(gate[row][head]) before its one rounding.
+// sigmoid(gate[row][head]) before its one rounding.  by_value (the bf16 kernels for head sizes of 64 and 128): one logit per value, and the rounded
+// output is multiplied by its sigmoid and rounded, as sigmoid_gate does in a pass of its own (7830 rows of 2048 20 us, 3749 12, one row 4).
 // The sink is one more softmax term with no value and a fixed score - 0, or a learned unscaled logit
 // per query head (sinks[h]): the running maximum starts at that score and the running denominator at 1.  Scores, weights and the output accumulation are fp32.
 #include <type_traits>
@@ -477,7 +478,7 @@ __global__ __launch_bounds__(64 * NW, PER_CU * NW / 4) void window_decode_row_ke
                                                                 const int* __restrict__ block_tables, int bt_stride,
                                                                 const int* __restrict__ seq_lens, int Hq, int G, float scale, int window, int chunked, int keep,
                                                                 float cap, int sink, const float* __restrict__ sinks,
-                                                                const bf16_t* __restrict__ gate, long g_stride) {
+                                                                const bf16_t* __restrict__ gate, long g_stride, int by_value) {
   constexpr int bs = 16;
   __shared__ float ml_s[NW][R][2];
   constexpr int dk = 64 * DKC, dv = 64 * VC;
@@ -658,8 +659,9 @@ __global__ __launch_bounds__(64 * NW, PER_CU * NW / 4) void window_decode_row_ke
       L += ml_s[w][r][1] * f;
       val += reinterpret_cast<const float*>(k_s[w])[r * dv + dcol] * f;
     }
-    const float gt = gate != nullptr ? sigmoid_f(bf2f(gate[(long)b * g_stride + h0 + r])) : 1.f;
-    o[c] = f2bf(L > 0.f ? val / L * gt : 0.f);
+    const float gt = gate != nullptr && !by_value ? sigmoid_f(bf2f(gate[(long)b * g_stride + h0 + r])) : 1.f;
+    const bf16_t x = f2bf(L > 0.f ? val / L * gt : 0.f);
+    o[c] = by_value ? f2bf(bf2f(x) * sigmoid_f(bf2f(gate[(long)b * g_stride + (long)h0 * dv + c]))) : x;
   }
 }
 
@@ -698,7 +700,7 @@ __global__ __launch_bounds__(WH ? 64 * WH : 64, WH == 0 || QT == 4 ? 1 : 3) void
     const bf16_t* __restrict__ v_cache, const int* __restrict__ cu, const int* __restrict__ ctx,
     const int* __restrict__ block_tables, int bt_stride, int S, int Hq, int G, float scale, int window,
     int chunked, int keep, float cap, int sink, const float* __restrict__ sinks, const bf16_t* __restrict__ gate,
-    long g_stride) {
+    long g_stride, int by_value) {
   // pages hold 16 tokens; scores live in the base-2 domain (scale * log2 e folded in) so that every
   // exponential is one v_exp_f32
   const float sc2 = scale * 1.44269504088896341f;
@@ -924,13 +926,15 @@ __global__ __launch_bounds__(WH ? 64 * WH : 64, WH == 0 || QT == 4 ? 1 : 3) void
     if (CAP == 2) l[t] = xor32_sum_f(xor16_sum(l[t]));
     if (!q_live[t]) continue;  // oacc[t][dt][i] = O[q = 16 t + c16][d = 16 dt + 4 quad + i]
     float inv = l[t] > 0.f ? 1.f / l[t] : 0.f;
-    if (gate != nullptr) inv *= sigmoid_f(bf2f(gate[(long)(row0 + 16 * t + c16) * g_stride + h]));
+    if (gate != nullptr && !by_value) inv *= sigmoid_f(bf2f(gate[(long)(row0 + 16 * t + c16) * g_stride + h]));
+    const bf16_t* gv = by_value ? gate + (long)(row0 + 16 * t + c16) * g_stride + (long)h * DV + 4 * quad : nullptr;
     bf16_t* orow = out + (long)(row0 + 16 * t + c16) * Hq * DV + (long)h * DV;
 #pragma unroll
     for (int dt = 0; dt < DV / 16; ++dt) {
       uint2 w;
       w.x = pack2(oacc[t][dt][0] * inv, oacc[t][dt][1] * inv);
       w.y = pack2(oacc[t][dt][2] * inv, oacc[t][dt][3] * inv);
+      if (by_value) w = gate_rounded(w, *reinterpret_cast<const uint2*>(gv + 16 * dt));
       *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * quad) = w;
     }
   }
@@ -945,7 +949,7 @@ extern "C" {
 int k8sllm_hy_window_flash(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache, const int* cu,
                            const int* ctx, const int* block_tables, int bt_stride, int S, long T, int Hq, int G, int dk, int dv,
                            float scale, int window, int chunked, int keep, float cap, int plain_cap, int sink,
-                           const float* sinks, const void* gate, long g_stride, hipStream_t s);
+                           const float* sinks, const void* gate, long g_stride, int by_value, hipStream_t s);
 int k8sllm_hy_window_f32(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache, const int* cu,
                          const int* ctx, const int* block_tables, int bt_stride, int S, long T, int Hq, int G, int dk, int dv,
                          int bs, float scale, int window, int chunked, int keep, float cap, int sink, const float* sinks,
@@ -973,8 +977,9 @@ int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float
 int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                              const int* cu, const int* ctx, const int* block_tables, int bt_stride, int S, long T,
                              int Hq, int G, int dk, int dv, int bs, float scale, int window, int chunked, int keep,
-                             float cap, int sink, const float* sinks, const void* gate, long g_stride, int f32, int mfma,
-                             hipStream_t s) {
+                             float cap, int sink, const float* sinks, const void* gate, long g_stride, int* by_value_, int f32,
+                             int mfma, hipStream_t s) {
+  const int by_value = *by_value_;
   if (T <= 0 || S <= 0) return 0;
   if (keep < 0 || (keep > 0 && (chunked || window <= 0))) return -1;
   if (dk > kGenDK || dv > 64 * kGenVC || G < 1 || Hq % G) return -1;
@@ -984,7 +989,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
     if (mfma == kFlashForced || (mfma == 1 && (T * Hq >= kFlashPairs || keys >= kFlashKeys))) {
       const int rc = k8sllm_hy_window_flash(out, qkv, q_stride, k_cache, v_cache, cu, ctx, block_tables, bt_stride, S, T, Hq, G,
                                             dk, dv, scale, window, chunked, keep, cap, cap <= kMaxCapPlain && !sink, sink,
-                                            sinks, gate, g_stride, s);
+                                            sinks, gate, g_stride, by_value, s);
       if (rc != 1 || mfma == kFlashForced) return rc;
     }
     // query rows per wave: 32 once the step is large enough to fill the chip that way (two row tiles share every K / V^T
@@ -1002,7 +1007,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
 #define K8SLLM_WPW(DK, DV, QT, CAP, WH)                                                                                \
   hipLaunchKernelGGL((window_prefill_mfma_kernel<DK, DV, QT, CAP, WH>), grid, dim3(WH ? 64 * WH : 64), 0, s, (bf16_t*)out, \
                      (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu, ctx,             \
-                     block_tables, bt_stride, S, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
+                     block_tables, bt_stride, S, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride, by_value)
 #define K8SLLM_WP(DK, DV, QT) \
   if (cap > 0.f && cap <= kMaxCapPlain && !sink) { K8SLLM_WPC(DK, DV, QT, 2); } \
   else if (cap > 0.f) { K8SLLM_WPC(DK, DV, QT, 1); } \
@@ -1023,6 +1028,7 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
     return (int)hipGetLastError();
   }
   if (mfma == kFlashForced) return 1;
+  if (by_value) gate = nullptr, *by_value_ = 0;  // (the caller gates the rows)
   if (f32 && mfma) {  // head sizes of 64 and 128: window_f32.hip, faster at every size measured there
     const int rc = k8sllm_hy_window_f32(out, qkv, q_stride, k_cache, v_cache, cu, ctx, block_tables, bt_stride, S, T, Hq, G, dk, dv,
                                         bs, scale, window, chunked, keep, cap, sink, sinks, gate, g_stride, 0, s);
@@ -1042,7 +1048,9 @@ int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const vo
 int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                             const int* block_tables, int bt_stride, const int* seq_lens, int B, int Hq, int G, int dk,
                             int dv, int bs, float scale, int window, int chunked, int keep, float cap, int sink,
-                            const float* sinks, const void* gate, long g_stride, int f32, int vec, int heads, hipStream_t s) {
+                            const float* sinks, const void* gate, long g_stride, int* by_value_, int f32, int vec, int heads,
+                            hipStream_t s) {
+  const int by_value = *by_value_;
   if (B <= 0) return 0;
   if (keep < 0 || (keep > 0 && (chunked || window <= 0))) return -1;
   if (dk > kGenDK || dv > 64 * kGenVC || G < 1 || Hq % G) return -1;
@@ -1055,7 +1063,7 @@ int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const voi
 #define K8SLLM_WDR(RR, NW, ...)                                                                                        \
   hipLaunchKernelGGL((window_decode_row_kernel<RR, NW, __VA_ARGS__>), dim3(B, Hq / RR), dim3(64 * NW), 0, s, (bf16_t*)out, \
                      (const bf16_t*)qkv, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, \
-                     seq_lens, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
+                     seq_lens, Hq, G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride, by_value)
 #define K8SLLM_WDD(DKC, VC)                                 \
   if (R == 8 && heads == 8) K8SLLM_WDR(8, 4, DKC, VC);      \
   else if (R == 8 && heads == 2) K8SLLM_WDR(2, 4, DKC, VC); \
@@ -1074,6 +1082,9 @@ int k8sllm_hy_window_decode(void* out, const void* qkv, long q_stride, const voi
     }
 #undef K8SLLM_WDD
 #undef K8SLLM_WDR
+  }
+  if (by_value) gate = nullptr, *by_value_ = 0;  // (the caller gates the rows)
+  if (lanes) {
 #define K8SLLM_WD(RR)                                                                                                  \
   hipLaunchKernelGGL((window_decode_vec_kernel<RR, (RR == 8 ? 4 : 8)>), dim3(B, G), dim3(RR == 8 ? 256 : 512), 0, s,     \
                      (bf16_t*)out, (const bf16_t*)qkv,                                                                  \

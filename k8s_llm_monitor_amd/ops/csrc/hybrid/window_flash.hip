@@ -39,7 +39,7 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv, long q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ cu, const int* __restrict__ ctx,
     const int* __restrict__ block_tables, int bt_stride, int S, int Hq, int G, float scale, int window, int chunked,
-    int keep, float cap, int sink, const float* __restrict__ sinks, const bf16_t* __restrict__ gate, long g_stride) {
+    int keep, float cap, int sink, const float* __restrict__ sinks, const bf16_t* __restrict__ gate, long g_stride, int by_value) {
   constexpr int KS = DK / 16, DT = DV / 32, CHK = DK / 8;
   constexpr int WPH = 8 / HW, QR = 32 * WPH;
   constexpr int KB = 64 * DK * 2, TILE = KB + 64 * DV * 2;
@@ -290,7 +290,8 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
   l = xor32_sum_f(l);
   if (myq >= L) return;
   float inv = l > 0.f ? 1.f / l : 0.f;
-  if (gate != nullptr) inv *= sigmoid_f(bf2f(gate[(long)(s0 + myq) * g_stride + h]));
+  const bf16_t* gv = by_value ? gate + (long)(s0 + myq) * g_stride + (long)h * DV + 4 * hh : nullptr;
+  if (gate != nullptr && !by_value) inv *= sigmoid_f(bf2f(gate[(long)(s0 + myq) * g_stride + h]));
   bf16_t* op = out + (long)(s0 + myq) * Hq * DV + (long)h * DV + 4 * hh;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -299,6 +300,7 @@ __global__ __launch_bounds__(512, 2) void window_flash_kernel(
       uint2 v;
       v.x = pack2(o[dt][4 * k] * inv, o[dt][4 * k + 1] * inv);
       v.y = pack2(o[dt][4 * k + 2] * inv, o[dt][4 * k + 3] * inv);
+      if (by_value) v = gate_rounded(v, *reinterpret_cast<const uint2*>(gv + 32 * dt + 8 * k));
       *reinterpret_cast<uint2*>(op + 32 * dt + 8 * k) = v;
     }
 }
@@ -311,7 +313,8 @@ using namespace k8sllm;
 extern "C" int k8sllm_hy_window_flash(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                                       const int* cu, const int* ctx, const int* block_tables, int bt_stride, int S, long T,
                                       int Hq, int G, int dk, int dv, float scale, int window, int chunked, int keep, float cap,
-                                      int plain_cap, int sink, const float* sinks, const void* gate, long g_stride, hipStream_t s) {
+                                      int plain_cap, int sink, const float* sinks, const void* gate, long g_stride, int by_value,
+                                      hipStream_t s) {
   const int R = Hq / G;
   const int hw = R % 8 == 0 ? 8 : R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
   const int qr = 256 / hw;
@@ -324,7 +327,7 @@ extern "C" int k8sllm_hy_window_flash(void* out, const void* qkv, long q_stride,
 #define K8SLLM_WF(DK, DV, HW, CAP)                                                                                     \
   hipLaunchKernelGGL((window_flash_kernel<DK, DV, HW, CAP>), grid, dim3(512), 0, s, (bf16_t*)out, (const bf16_t*)qkv,    \
                      q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu, ctx, block_tables, bt_stride, S, Hq, \
-                     G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride)
+                     G, scale, window, chunked, keep, cap, sink, sinks, (const bf16_t*)gate, g_stride, by_value)
 #define K8SLLM_WFC(DK, DV, HW)                        \
   if (cap > 0.f && plain_cap) K8SLLM_WF(DK, DV, HW, 2); \
   else if (cap > 0.f) K8SLLM_WF(DK, DV, HW, 1);       \

@@ -548,13 +548,15 @@ def window_attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: 
                              ctx: torch.Tensor, block_tables: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int,
                              scale: float, window: int, sink: bool, mfma: int = 1,
                              sinks: Optional[torch.Tensor] = None, chunked: bool = False, cap: float = 0.0, keep: int = 0,
-                             gate: Optional[torch.Tensor] = None, g_col: int = 0) -> torch.Tensor:
+                             gate: Optional[torch.Tensor] = None, g_col: int = 0, by_value: bool = False,
+                             out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Attention of the step's prompt chunks over the paged cache (which already holds their own
     keys): row r of segment s at position p = ctx[s] + r sees positions max(0, p - window + 1) .. p
     (``window`` 0: all of 0 .. p), or with ``chunked`` those of its own chunk of ``window`` positions,
     p - p % window .. p (chunks count from position 0).  ``keep``: with a sliding window, the first ``keep``
     positions of the sequence stay visible too.  ``gate``: rows of a projection [T, *]; head h of a row is
-    multiplied by sigmoid(gate[row, g_col + h]) before it is rounded.  ``cap`` > 0: a score s (after ``scale``) becomes
+    multiplied by sigmoid(gate[row, g_col + h]) before it is rounded; ``by_value``: value d of head h of the rounded row by
+    sigmoid(gate[row, g_col + h * dv + d]), as sigmoid_gate does.  ``out``: the rows to write [T, Hq*dv].  ``cap`` > 0: a score s (after ``scale``) becomes
     ``cap * tanh(s / cap)``.  ``sink``: the softmax denominator has one more term that carries
     no value - exp(0), or exp(sinks[h]) for head h where ``sinks`` [Hq] fp32 is given (a learned,
     unscaled logit).  Scores and weights are fp32.  Returns [T, Hq*dv].  GPU, bf16, head sizes
@@ -563,8 +565,10 @@ def window_attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: 
     that many rows per wave; 256: the staged kernel); fp32, the same sizes: 16 rows per wave on the fp32
     matrix instruction."""
     T = qkv.shape[0]
+    if out is None:
+        out = torch.empty(T, Hq * dv, dtype=qkv.dtype, device=qkv.device)
+    hg = None if by_value else gate
     if not qkv.is_cuda:
-        out = torch.empty(T, Hq * dv, dtype=qkv.dtype)
         bs = k_cache.shape[1]
         cul, ctxl = cu.tolist(), ctx.tolist()
         for s in range(len(ctxl)):
@@ -576,28 +580,31 @@ def window_attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: 
                 p = ctxl[s] + r - cul[s]
                 js = _visible(p, window, chunked, keep)
                 o = _attend(qkv[r, : Hq * dk].float().view(Hq, dk), ks[js], vs[js], scale, sink, sinks, cap)
-                out[r] = _head_gate(o, gate[r] if gate is not None else None, g_col).reshape(-1).to(qkv.dtype)
-        return out
-    out = torch.empty(T, Hq * dv, dtype=qkv.dtype, device=qkv.device)
-    native().window_attention_prefill(out, qkv, k_cache, v_cache, cu, ctx, block_tables, Hq, Hkv, dk, dv, float(scale),
-                                      int(window), bool(sink), sinks, int(mfma), bool(chunked), float(cap), int(keep), gate,
-                                      int(g_col))
-    return out
+                out[r] = _head_gate(o, hg[r] if hg is not None else None, g_col).reshape(-1).to(qkv.dtype)
+        return sigmoid_gate(out, gate[:T], g_col) if by_value and gate is not None else out
+    gated = native().window_attention_prefill(out, qkv, k_cache, v_cache, cu, ctx, block_tables, Hq, Hkv, dk, dv, float(scale),
+                                              int(window), bool(sink), sinks, int(mfma), bool(chunked), float(cap), int(keep), gate,
+                                              int(g_col), bool(by_value))
+    return sigmoid_gate(out, gate[:T], g_col) if by_value and gate is not None and not gated else out
 
 
 def window_attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                             block_tables: torch.Tensor, seq_lens: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int,
                             scale: float, window: int, sink: bool, vec: bool = True,
                             sinks: Optional[torch.Tensor] = None, chunked: bool = False, cap: float = 0.0, keep: int = 0,
-                            gate: Optional[torch.Tensor] = None, g_col: int = 0, heads: int = 0) -> torch.Tensor:
+                            gate: Optional[torch.Tensor] = None, g_col: int = 0, heads: int = 0, by_value: bool = False,
+                            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One query per sequence (its newest token, already in the cache) over the last ``window``
-    cached positions (``chunked``: those of its own chunk; ``cap``, ``keep``, ``gate``: as in
+    cached positions (``chunked``: those of its own chunk; ``cap``, ``keep``, ``gate``, ``by_value``, ``out``: as in
     window_attention_prefill);
     ``seq_lens`` count that token (0: a padding row, output zero).  ``heads``: query heads of a kv
     head that a workgroup takes (GPU, ``vec``, bf16, head sizes of 64 and 128; 0: its choice, others are refused elsewhere)."""
     B = qkv.shape[0]
+    if out is None:
+        out = torch.empty(B, Hq * dv, dtype=qkv.dtype, device=qkv.device)
+    hg = None if by_value else gate
     if not qkv.is_cuda:
-        out = torch.zeros(B, Hq * dv, dtype=qkv.dtype)
+        out.zero_()
         bs = k_cache.shape[1]
         for b, n in enumerate(seq_lens.tolist()):
             if n <= 0:
@@ -607,13 +614,12 @@ def window_attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: t
             ks = k_cache[bt].reshape(-1, Hkv, dk)[js].float()
             vs = v_cache[bt].permute(0, 3, 1, 2).reshape(-1, Hkv, dv)[js].float()
             o = _attend(qkv[b, : Hq * dk].float().view(Hq, dk), ks, vs, scale, sink, sinks, cap)
-            out[b] = _head_gate(o, gate[b] if gate is not None else None, g_col).reshape(-1).to(qkv.dtype)
-        return out
-    out = torch.empty(B, Hq * dv, dtype=qkv.dtype, device=qkv.device)
-    native().window_attention_decode(out, qkv, k_cache, v_cache, block_tables, seq_lens, Hq, Hkv, dk, dv, float(scale),
-                                     int(window), bool(sink), sinks, bool(vec), bool(chunked), float(cap), int(keep), gate,
-                                     int(g_col), int(heads))
-    return out
+            out[b] = _head_gate(o, hg[b] if hg is not None else None, g_col).reshape(-1).to(qkv.dtype)
+        return sigmoid_gate(out, gate[:B], g_col) if by_value and gate is not None else out
+    gated = native().window_attention_decode(out, qkv, k_cache, v_cache, block_tables, seq_lens, Hq, Hkv, dk, dv, float(scale),
+                                             int(window), bool(sink), sinks, bool(vec), bool(chunked), float(cap), int(keep), gate,
+                                             int(g_col), int(heads), bool(by_value))
+    return sigmoid_gate(out, gate[:B], g_col) if by_value and gate is not None and not gated else out
 
 
 # ---------------------------------------------------------------- latent attention
@@ -735,11 +741,11 @@ def latent_head_queries(q: torch.Tensor, w_uk: torch.Tensor, H: int, dim: int, r
     return latent_queries(q, q_lat, H, dim, rot_dim, positions, freq, pitch, pairs)
 
 
-def latent_head_values(o: torch.Tensor, w_uv: torch.Tensor, H: int) -> torch.Tensor:
-    """Per head ``W_uv[h] o[t][h]``: [T, H * R] and ``w_uv`` [H * vdim, R] -> [T, H * vdim]."""
+def latent_head_values(o: torch.Tensor, w_uv: torch.Tensor, H: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Per head ``W_uv[h] o[t][h]``: [T, H * R] and ``w_uv`` [H * vdim, R] -> [T, H * vdim] (``out``: its rows)."""
     T, R = o.shape[0], w_uv.shape[1]
     dv = w_uv.shape[0] // H
-    v = torch.empty(T, H, dv, dtype=o.dtype, device=o.device)
+    v = (torch.empty(T, H * dv, dtype=o.dtype, device=o.device) if out is None else out).view(T, H, dv)
     if _head_rows(HEAD_VALUE_ROWS, o, w_uv) and R % 8 == 0 and T * H * dv * R < HEAD_VALUE_WORK:
         native().latent_head_values(v, o, w_uv, int(H))
     else:  # written head by head into the rows that the out-projection reads

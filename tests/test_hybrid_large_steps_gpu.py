@@ -1342,3 +1342,31 @@ def test_latent_heads(T, H, dn, dr, dv, R, pitch, nf, pairs, sliced):
     v = torch.bmm(o.view(T, H, R).transpose(0, 1).float().contiguous(), wv.view(H, dv, R).transpose(1, 2).float().contiguous())
     got = hops.latent_head_values(o.cuda(), wv.cuda(), H).cpu().view(T, H, dv)
     torch.testing.assert_close(got.float(), v.transpose(0, 1), rtol=2 ** -7, atol=2 ** -7)
+
+
+@pytest.mark.parametrize("mfma,vec,dk,dv,Hq,G,off,dt", [
+    (256, True, 128, 128, 8, 2, 8, BF), (256, True, 64, 128, 3, 3, 0, BF), (2, True, 128, 64, 4, 1, 16, BF), (2, True, 64, 64, 2, 2, 8, BF),
+    (1, True, 128, 128, 4, 1, 4, BF),  # logits not in 16-byte pieces: gated in a pass of its own, as the kernels below do
+    (0, False, 128, 128, 4, 2, 8, BF), (1, True, 48, 40, 4, 2, 8, BF), (1, True, 64, 64, 4, 2, 0, torch.float32),
+])
+def test_gate_by_value(mfma, vec, dk, dv, Hq, G, off, dt):
+    """The output gate in the attention kernels, rows written into a given buffer: the bits of the ungated rows and sigmoid_gate, for chunks
+    around a tile's end and decode rows beside a padding row."""
+    g = _g(93)
+    new, ctx = [65, 1, 130], [0, 40, 17]
+    lens = [c + n for c, n in zip(ctx, new)]
+    kc, vc, bt = _paged(g, dt, lens, Hq, G, dk, dv, nb=sum((n + 15) // 16 for n in lens) + 3)
+    T = sum(new)
+    qkv, z = _r(g, T, Hq * dk + 8, dt=dt).cuda(), _r(g, T, Hq * dv + 24, s=2.0, dt=dt).cuda()
+    dev = [x.cuda() for x in (kc, vc, _i32([0, 65, 66, 196]), _i32(ctx), bt)]
+    a = (Hq, G, dk, dv, dk ** -0.5, 50, True)
+    want = hops.sigmoid_gate(hops.window_attention_prefill(qkv, *dev, *a, mfma=mfma), z, off)
+    rows = torch.full((T + 2, Hq * dv), 7.0, dtype=dt, device="cuda")
+    got = hops.window_attention_prefill(qkv, *dev, *a, mfma=mfma, gate=z, g_col=off, by_value=True, out=rows[1:-1])
+    assert torch.equal(got, want) and torch.equal(rows[1:-1], want) and bool((rows[[0, -1]] == 7).all())
+    n = _i32(lens[:2] + [0]).cuda()
+    want = hops.sigmoid_gate(hops.window_attention_decode(qkv[:3], dev[0], dev[1], bt.cuda(), n, *a, vec=vec), z[:3], off)
+    got = hops.window_attention_decode(qkv[:3], dev[0], dev[1], bt.cuda(), n, *a, vec=vec, gate=z, g_col=off, by_value=True, out=rows[1:4])
+    assert torch.equal(got, want) and bool((rows[0] == 7).all())
+    cpu = hops.window_attention_decode(*(x.cpu() for x in (qkv[:3], dev[0], dev[1], bt, n)), *a, gate=z.cpu(), g_col=off, by_value=True)
+    torch.testing.assert_close(got.cpu().float(), cpu.float(), rtol=2e-2, atol=2e-2)
