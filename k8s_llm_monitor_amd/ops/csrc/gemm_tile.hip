@@ -69,11 +69,25 @@ __device__ __forceinline__ void vm_wait_n() {
 __device__ __forceinline__ void lgkm_wait0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 }  // namespace
 
+// Tiles run in rounds of one a CU, and a last round of few tiles takes most of a full one's time (30 to 45 us of K = 2048 alone on the chip, a full
+// round's 55 to 60).  Up to 64 tiles beyond whole rounds go as four strips of 64 rows each, one a CU, of about half a tile's time; from 65 on
+// the strips would need two rounds, which was no faster (72 tiles of K 1024 35 / 42 us, 128 of K 2048 43.9 / 43.6, 112 behind a round 119 / 126).
+// us, whole tiles / strips: 780 tiles of K 2048 (gated unit) 224 / 214; 258 of K 4096 172 / 157; grouped, 8 experts, 1072 294 / 279 and 536
+// 148 / 140; 320 of K 4096 in 4 experts 204 / 170; 36 of K 1024 28 / 21.
+// Grouped, the count of tiles is known on the device only: each workgroup sums it over the experts, up to kStripExperts of them.
+constexpr int kTileCus = 256, kStripTiles = 64, kStripExperts = 32;
+template <int EPI, int SCH, bool RS>
+constexpr bool tile_strips() {
+  return SCH == 1 && !RS && EPI != TILE_EPI_ROPE && EPI != TILE_EPI_RESID;
+}
+// workgroups that strips of up to this many tiles add
+static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * 32 - tiles; }
+
 template <int EPI, bool GROUPED, int SCH, bool RS = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                          int E, int M, int N, int K, long w_es, int n_mt, int n_nt,
-                                                         TileEpi ep, int wpk) {
+                                                         TileEpi ep, int wpk, int strips) {
   constexpr int HS = 32768;  // one half-slot: 256 rows x 128 B
   __shared__ __attribute__((aligned(16))) char smem[5 * HS];
   const int lane = threadIdx.x & 63;
@@ -81,12 +95,30 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   const int wm = wave >> 1, wn = wave & 1;
 
   // ---- logical tile: bijective XCD remap, then groups of 8 m-tiles ----
-  const int nwg = n_mt * n_nt;
-  const int bid = blockIdx.x, xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
-  const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
+  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>();
+  int mts = n_mt;
+  if (GROUPED && STRIPS && strips) {  // the tiles that there are
+    mts = 0;
+    for (int x = 0; x < E; ++x) mts += (offsets[x + 1] - offsets[x] + 255) >> 8;
+  }
+  int nwg = mts * n_nt, lid, strip = -1;
+  const int bid = blockIdx.x, xcd = bid & 7;
+  const int over = STRIPS && strips ? nwg % kTileCus : 0;  // tiles beyond whole rounds
+  if (over > 0 && over <= kStripTiles && bid >= nwg - over) {
+    const int i = bid - (nwg - over);  // a tile's four strips on one XCD
+    strip = (i >> 3) & 3;
+    lid = (i >> 5) * 8 + (i & 7);
+    if (lid >= over) return;
+    lid += nwg - over;
+  } else {
+    if (GROUPED && bid >= nwg) return;
+    if (over <= kStripTiles) nwg -= over;
+    const int q8 = nwg >> 3, r8 = nwg & 7;
+    lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
+  }
   constexpr int GM = 8;
   const int grp = lid / (GM * n_nt), first_m = grp * GM;
-  const int gsz = min(n_mt - first_m, GM);
+  const int gsz = min(mts - first_m, GM);
   const int in_g = lid - grp * GM * n_nt;
   const int mt = first_m + in_g % gsz, nt = in_g / gsz;
 
@@ -111,6 +143,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   } else {
     row0 = mt * 256;
     mrows = min(256, M - row0);
+  }
+  if (STRIPS && strip >= 0) {
+    row0 += 64 * strip;
+    mrows = min(64, mrows - 64 * strip);
+    if (mrows <= 0) return;
   }
   // GLU: the unit's tiles first, 128 features each, then the rest's
   constexpr bool GLU = tile_epi_glu(EPI);
@@ -197,7 +234,55 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   // chunk cc), issued during the last k-tile's second half so they land behind its MFMAs
   u32x4 resq[EPI == TILE_EPI_RESID ? 16 : 1];
 
-  if constexpr (SCH == 1) {
+  if (STRIPS && strip >= 0) {
+    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  The same instructions in the same
+    // order of k as a whole tile's, so the same bits.
+    constexpr int SS = 8192 + HS;
+    auto fill = [&](int kt) {
+      char* dst = smem + (kt & 3) * SS + wave * 1024;
+      const int k = min(kt, nk - 1);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(dst + p * 4096), 16, soff[0][p], k * 128, 0, 0);
+#pragma unroll
+      for (int p = 0; p < 8; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(dst + 8192 + p * 4096), 16, soff[1][p], k * kstrB, 0, 0);
+    };
+    auto read = [&](int t, int ks, bf16x8 (&a)[8], bf16x8 (&b)[8]) {
+      const char* at = smem + (t & 3) * SS;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) b[j] = *reinterpret_cast<const bf16x8*>(at + 8192 + (8 * wn + j) * 2048 + rdB[ks]);
+#pragma unroll
+      for (int g = 0; g < 2; ++g) a[g] = *reinterpret_cast<const bf16x8*>(at + (2 * wm + g) * 2048 + rd[ks]);
+    };
+    auto mul = [&](const bf16x8 (&a)[8], const bf16x8 (&b)[8]) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[g], acc[g][j], 0, 0, 0);
+    };
+    fill(0);
+    fill(1);
+    fill(2);
+    fill(3);
+    vm_wait_n<30>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0, fa0, fb0);
+    for (int t = 0; t < nk; ++t) {
+      read(t, 1, fa1, fb1);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(fa0, fb0);
+      lgkm_wait0();
+      vm_wait_n<20>();  // k-tile t + 1 is in; the two behind it are on their way
+      __builtin_amdgcn_s_barrier();  // everyone's pieces of it, and everyone has read k-tile t
+      asm volatile("" ::: "memory");
+      read(t + 1, 0, fa0, fb0);
+      fill(t + 4);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(fa1, fb1);
+    }
+    vm_wait_n<0>();
+  } else if constexpr (SCH == 1) {
     // Ring addressing: the half-slot byte offsets of the current tile live in SGPRs and rotate
     // by one conditional subtract per tile, and each sub-step forms ONE A and ONE B fragment base
     // VGPR (every block read is that base + an immediate).
@@ -392,11 +477,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   // the accumulator layout directly, which is what bounds a store tail (T21). ----
   lgkm_wait0();
   __builtin_amdgcn_s_barrier();  // every wave is done with the ring (its last DMAs retired above)
-  auto finish = [&](auto gated) {  // gated: a unit's tile
+  auto finish = [&](auto gated, auto blocks) {  // gated: a unit's tile; blocks: of 16 rows, a wave's
   constexpr bool SWG = decltype(gated)::value;
+  constexpr int RB = decltype(blocks)::value;
   constexpr int OUTW = SWG ? 64 : 128;  // output columns of this wave's quarter
   constexpr int RS_ = OUTW * 2 + 16;                       // LDS row stride (16-B pad: 2-way writes)
-  char* stage = smem + wave * (128 * RS_);
+  char* stage = smem + wave * (16 * RB * RS_);
   const int ml = lane & 15, nq = 4 * (lane >> 4);
   const int rr = lane >> 4, cc = lane & 15;
   uint4 nwv{};
@@ -413,7 +499,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     for (int i = 0; i < 8; ++i) sc[i] = inv_s[wm * 128 + i * 16 + ml];
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < RB; ++i) {
     __builtin_amdgcn_sched_barrier(0);  // one row block's accumulators at a time (no hoisted AGPR reads)
     char* srow = stage + (i * 16 + ml) * RS_ + nq * 2;
     if constexpr (EPI == TILE_EPI_SWIGLU || (GLU && SWG)) {
@@ -545,23 +631,33 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   // branch-free masked stores: a buffer descriptor over this m-tile's rows drops every store past
   // row mrows (out of range), and a lane whose columns are past N gets an out-of-range offset
   const __amdgpu_buffer_rsrc_t yr = rsrc(out + (long)row0 * ldy, (long)mrows * ldy * 2);
-  const uint32_t yo = cc2 * 8 < ncols ? (uint32_t)(((wm * 128 + rr2) * ldy + col0 + cc2 * 8) * 2) : 0x80000000u;
+  const uint32_t yo = cc2 * 8 < ncols ? (uint32_t)(((wm * 16 * RB + rr2) * ldy + col0 + cc2 * 8) * 2) : 0x80000000u;
+  constexpr int NB = 16 * RB / RPI < 8 ? 16 * RB / RPI : 8;
 #pragma unroll
-  for (int b = 0; b < 128 / RPI; b += 8) {  // 8 row groups per batch: reads issued back to back
-    u32x4 v[8];
+  for (int b = 0; b < 16 * RB / RPI; b += NB) {  // 8 row groups per batch: reads issued back to back
+    u32x4 v[NB];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const u32x4*>(stage + ((b + u) * RPI + rr2) * RS_ + cc2 * 16);
+    for (int u = 0; u < NB; ++u) v[u] = *reinterpret_cast<const u32x4*>(stage + ((b + u) * RPI + rr2) * RS_ + cc2 * 16);
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < NB; ++u)
       __builtin_amdgcn_raw_buffer_store_b128(v[u], yr, yo + (uint32_t)((b + u) * RPI * ldy * 2), 0, 0);
   }
   };
-  if constexpr (GLU) {
-    if (unit) finish(std::true_type{});
-    else finish(std::false_type{});
-  } else {
-    finish(std::bool_constant<EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8>{});
+  auto end = [&](auto blocks) {
+    if constexpr (GLU) {
+      if (unit) finish(std::true_type{}, blocks);
+      else finish(std::false_type{}, blocks);
+    } else {
+      finish(std::bool_constant<EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8>{}, blocks);
+    }
+  };
+  if constexpr (STRIPS) {
+    if (strip >= 0) {
+      end(std::integral_constant<int, 2>{});
+      return;
+    }
   }
+  end(std::integral_constant<int, 8>{});
 }
 
 }  // namespace k8sllm
@@ -609,10 +705,13 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   const int n_mt = (M + 255) / 256 + (grouped ? E : 0), n_nt = (N + 255) / 256;
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
-  const dim3 grid((unsigned)nwg);
+  const bool cut = algo == 1 && !rs && epi != TILE_EPI_ROPE && epi != TILE_EPI_RESID && E <= kStripExperts;
+  const long over = nwg % kTileCus;
+  const int strips = cut && (grouped || (over > 0 && over <= kStripTiles));
+  const dim3 grid((unsigned)(nwg + (!strips ? 0 : grouped ? 4 * kStripTiles : strip_groups(over))));
 #define K8_TILE_LAUNCH(EPI_, G_, SCH_, RS_)                                                                          \
   hipLaunchKernelGGL((gemm_w4_kernel<EPI_, G_, SCH_, RS_>), grid, dim3(256), 0, s, (const bf16_t*)X,                \
-                     (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk)
+                     (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk, strips)
 #define K8_TILE_SCH(SCH_)                                                                                            \
   if (grouped) {                                                                                                     \
     if (epi == TILE_EPI_SWIGLU) K8_TILE_LAUNCH(TILE_EPI_SWIGLU, true, SCH_, false);                                  \
@@ -653,9 +752,12 @@ extern "C" int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void
   const int n_mt = (M + 255) / 256, n_nt = glu ? (f + 127) / 128 + (N - 2 * f + 255) / 256 : (N + 255) / 256;
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
+  const long over = nwg % kTileCus;
+  const int strips = over > 0 && over <= kStripTiles;
+  const long groups = nwg + (strips ? strip_groups(over) : 0);
 #define K8_TILE_UNIT(EPI_)                                                                                             \
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false>), dim3((unsigned)nwg), dim3(256), 0, s, (const bf16_t*)X,    \
-                     (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0)
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false>), dim3((unsigned)groups), dim3(256), 0, s, (const bf16_t*)X, \
+                     (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0, strips)
   if (epi == TILE_EPI_GELU_GLU) K8_TILE_UNIT(TILE_EPI_GELU_GLU);
   else if (epi == TILE_EPI_SILU_GLU) K8_TILE_UNIT(TILE_EPI_SILU_GLU);
   else if (epi == TILE_EPI_RELU_GLU) K8_TILE_UNIT(TILE_EPI_RELU_GLU);

@@ -182,3 +182,28 @@ def test_gemm_tile_swiglu8_matches_fp32_and_decode_layout(M, rowscale):
         we = torch.stack([ops.pack_skinny(w8), ops.pack_skinny(w8.flip(1).contiguous())]).contiguous()
         yg = ops.gemm_tile(x, we, off, swiglu=8)
         assert torch.equal(yg[: counts[0]], y[: counts[0]])
+
+
+@pytest.mark.parametrize("m_tiles,n_tiles,last,K,swiglu", [
+    (1, 1, 1, 192, False), (5, 13, 64, 192, True), (8, 8, 65, 256, True), (9, 8, 129, 256, False), (13, 20, 200, 192, True),
+    (16, 20, 256, 192, False), (16, 21, 3, 192, False), (17, 15, 193, 640, True),
+])
+def test_gemm_tile_last_round(m_tiles, n_tiles, last, K, swiglu):
+    """Tiles beyond whole rounds of 256 as strips of 64 rows (up to 64 of them), dense, grouped (with an empty expert and short ones) and
+    ended by a gated unit: the bits of the schedule that has whole tiles only."""
+    g = torch.Generator().manual_seed(5)
+    M, N = 256 * (m_tiles - 1) + last, 256 * n_tiles
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(2, N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    assert torch.equal(ops.gemm_tile(x, w[0], swiglu=swiglu, algo=1), ops.gemm_tile(x, w[0], swiglu=swiglu, algo=0))
+    w3 = torch.cat([w, w[:1]])
+    for cut in (M // 3, M - M // 5, M):
+        off = torch.tensor([0, cut, cut, M], dtype=torch.int32, device="cuda")
+        assert torch.equal(ops.gemm_tile(x, w3, off, swiglu=swiglu, algo=1), ops.gemm_tile(x, w3, off, swiglu=swiglu, algo=0))
+    f = N // 2 - 64  # the unit's last tile is short; 128 more columns stand behind it
+    y, y2 = torch.empty(M, f, dtype=torch.bfloat16, device="cuda"), torch.empty(M, 128, dtype=torch.bfloat16, device="cuda")
+    ops.native().gemm_tile_unit(y, y2, x, w[1], 6)  # SiLU
+    z = ops.gemm_tile(x, w[1], algo=0)
+    up, gate = z[:, f:2 * f].float(), z[:, :f].float()
+    torch.testing.assert_close(y.float(), torch.nn.functional.silu(gate) * up, rtol=2 ** -7, atol=2 ** -7)
+    assert torch.equal(y2, z[:, 2 * f:])
