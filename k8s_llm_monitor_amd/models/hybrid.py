@@ -183,8 +183,9 @@ class WindowAttention:
             # another running maximum, and this design's routers - the softmax over the two best of near-equal logits - turn such
             # differences into other experts: recurrent states behind them moved by more than their root mean square.
             o = torch.empty(qkv.shape[0], H * dv, dtype=qkv.dtype, device=qkv.device)
-            hops.window_attention_prefill(qkv[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
-                                          *args, mfma=2 if self.fast == 1 else self.fast, out=o[nd:])
+            q, po = (qkv[nd:], o[nd:]) if nd else (qkv, o)
+            hops.window_attention_prefill(q, kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
+                                          *args, mfma=2 if self.fast == 1 else self.fast, out=po)
             if nd:  # a mixed step: the single decode tokens in front go through the decode kernel
                 hops.window_attention_decode(qkv[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
                                              vec=bool(self.fast), out=o[:nd])
@@ -363,7 +364,7 @@ class LatentAttention:
                 (nd, n, meta.block_tables, dict(seq_lens=meta.ends) if ends else dict(cu=meta.cu_seqlens, ctx=meta.ctx_start))]
             self._forward_latent(q[:n], pos, kc, vc, gate, [r for r in runs if r[1] > r[0]], o[:n])
         if ex:
-            self._forward_expanded(q[nd:], meta, kc, gate[nd:] if gate is not None else None, o[nd:])
+            self._forward_expanded(*((t if t is None or not nd else t[nd:]) for t in (q, gate, o)), meta, kc)
         if rows is not None and not ends:
             o, proj = _take(rows, o, proj)
         if self.n_tail:
@@ -402,7 +403,7 @@ class LatentAttention:
                 cuts.append(i)
         return list(zip(cuts, cuts[1:] + [len(seen.ends)]))
 
-    def _forward_expanded(self, q: torch.Tensor, meta: AttnMeta, kc: torch.Tensor, gate: Optional[torch.Tensor], out: torch.Tensor) -> None:
+    def _forward_expanded(self, q: torch.Tensor, gate: Optional[torch.Tensor], out: torch.Tensor, meta: AttnMeta, kc: torch.Tensor) -> None:
         """Prompt rows: per-head keys and values of every position they see in temporary pages, windowed
         attention's matrix-core kernel over them, into ``out``.  ``q`` [rows, H * (dim + rot_dim)] still unturned."""
         H, dn, dr, dv = self.H, self.dn, self.dr, self.dv
@@ -527,8 +528,9 @@ class RotaryAttention:
         else:
             nd = meta.num_decode
             o = torch.empty(proj.shape[0], H * dv, dtype=proj.dtype, device=proj.device)
-            hops.window_attention_prefill(proj[nd:], kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
-                                          *args, mfma=self.fast, gate=proj[nd:] if hg else None, out=o[nd:], **kw)
+            q, po = (proj[nd:], o[nd:]) if nd else (proj, o)
+            hops.window_attention_prefill(q, kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
+                                          *args, mfma=self.fast, gate=q if hg else None, out=po, **kw)
             if nd:
                 hops.window_attention_decode(proj[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
                                              vec=bool(self.fast), gate=proj[:nd] if hg else None, out=o[:nd], **kw)
@@ -1369,10 +1371,12 @@ class HybridLM:
         c = self.cfg
         if self.sequential:
             return self._forward_sequential(ids, meta, caches)
-        x0 = hops.embed_pos(ids, meta.positions, self.embed, self.pos, meta.dec_src, meta.dec_prev)
-        x = x0.clone() if c.loop and c.loop[2] > 1 else x0
+        T, embed = ids.numel(), (ids, meta.positions, self.embed, self.pos, meta.dec_src, meta.dec_prev)
+        again = bool(c.loop and c.loop[2] > 1)  # the embeddings join the stream once more
+        x0 = hops.embed_pos(*embed) if again else None
+        x = x0.clone() if again else None
         pending: tuple = ()
-        want = self._wanted(meta, ids.numel())
+        want = self._wanted(meta, T)
         for r, (li, t, first) in enumerate(self.runs):
             adds, vec = pending, None
             if first:
@@ -1381,11 +1385,15 @@ class HybridLM:
                     adds = adds + (x0,)
             rows = want if r + 1 == len(self.runs) else None
             ff = self.ffns[li]
-            routed = None
-            if isinstance(ff, RoutedFFN) and rows is None and hops.route_with_norm(*x.shape, ff.wr.shape[0]):
-                h, routed = hops.add_norm(x, adds, vec, self.norms[li], c.norm_eps, True, self.dtype, route=(ff.wr, ff.bias, ff.E, ff.K))
+            route = (ff.wr, ff.bias, ff.E, ff.K) if isinstance(ff, RoutedFFN) and rows is None and hops.route_with_norm(
+                T, c.d_model, ff.wr.shape[0]) else None
+            if x is None:
+                x, h = hops.embed_norm(*embed, 1.0, vec, self.norms[li], c.norm_eps, True, route=route)
             else:
-                h = hops.add_norm(x, adds, vec, self.norms[li], c.norm_eps, True, self.dtype)
+                h = hops.add_norm(x, adds, vec, self.norms[li], c.norm_eps, True, self.dtype, route=route)
+            routed = None
+            if route is not None:
+                h, routed = h
             ym = self.mixers[li].forward(h, meta, caches[r], rows=rows)
             x, h = _take(rows, x, h)
             if isinstance(ff, RoutedFFN):
@@ -1415,12 +1423,14 @@ class HybridLM:
             stack[1].copy_(stack[0])
             x = stack[1]
         else:
+            if self.gated and not self.S and self.loop_step is None:
+                return self._forward_gated(None, meta, caches, ids)
             x = hops.embed_pos(ids, meta.positions, self.embed, self.pos, meta.dec_src, meta.dec_prev,
                                scale=c.embed_scale)
         if self.S:
             return self._forward_streams(x, meta, caches)
         if self.gated:
-            return self._forward_gated(x, meta, caches)
+            return self._forward_gated(x, meta, caches, ids)
         if self.post_norm:
             return self._forward_post_norm(x, meta, caches)
         if self.summed:
@@ -1584,21 +1594,25 @@ class HybridLM:
             return sub.tail_out
         return F.linear(h, g["w"]), 0
 
-    def _forward_gated(self, x: torch.Tensor, meta: AttnMeta, caches: list) -> torch.Tensor:
+    def _forward_gated(self, x: Optional[torch.Tensor], meta: AttnMeta, caches: list, ids: torch.Tensor) -> torch.Tensor:
         """Sequential blocks with a gated residual: every sublayer's result y joins the stream as
-        ``x += m * y * sigmoid(gate + b)``, folded into the launch of the norm that follows it."""
+        ``x += m * y * sigmoid(gate + b)``, folded into the launch of the norm that follows it.  ``x`` None: the embeddings of ``ids``."""
         c = self.cfg
         eps, op, mult = c.norm_eps, self.one_plus, c.residual_mult
         pend = None  # (y, projection holding the gate logits, their first column, bias)
-        want = self._wanted(meta, x.shape[0])
+        want = self._wanted(meta, ids.numel())
         for r, (li, t, first) in enumerate(self.runs):
             if first and self.loop_step is not None:
                 if pend is not None:
                     raise ValueError("looped layers with a gated residual are not built")
                 x += self.loop_step[t]
             w1 = self.norms[li]
-            h = hops.add_norm(x, (), None, w1, eps, op, self.dtype) if pend is None else \
-                hops.gated_add_norm(x, pend[0], pend[1], pend[2], pend[3], mult, w1, eps, op, self.dtype)
+            if x is None:
+                x, h = hops.embed_norm(ids, meta.positions, self.embed, self.pos, meta.dec_src, meta.dec_prev, c.embed_scale, None, w1, eps, op)
+            elif pend is None:
+                h = hops.add_norm(x, (), None, w1, eps, op, self.dtype)
+            else:
+                h = hops.gated_add_norm(x, pend[0], pend[1], pend[2], pend[3], mult, w1, eps, op, self.dtype)
             mx = self.mixers[li]
             rows = want if r + 1 == len(self.runs) else None
             y = mx.forward(h, meta, caches[self.kv_run[r]], rows=rows)

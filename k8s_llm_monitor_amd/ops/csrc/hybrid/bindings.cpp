@@ -32,9 +32,10 @@ int k8sllm_hy_router_grouped(int* ids, float* wts, const void* h, long T, int d,
                              hipStream_t s);
 int k8sllm_hy_add_norm(void* out, float* residual, const void* a0, int t0, const void* a1, int t1, const void* a2,
                        int t2, const float* vec, const float* w, long rows, int d, float eps, int one_plus, const void* ys,
-                       const int* inv, const float* wts, const void* shared, const float* gate, int K, int* r_ids, float* r_wts,
-                       float* r_gate, const float* wr, const float* bias, int rE, int rK, int rows_w, int over_all, int f32,
-                       hipStream_t s);
+                       const int* inv, const float* wts, const void* shared, const float* gate, int K, const int* ids,
+                       const int* positions, const void* emb, const void* pos, const int* src, const int* prev, int vocab, int max_pos,
+                       float scale, int* r_ids, float* r_wts, float* r_gate, const float* wr, const float* bias, int rE, int rK, int rows_w,
+                       int over_all, int f32, hipStream_t s);
 int k8sllm_hy_gated_group_norm(void* out, const float* y, const void* z, long z_stride, const float* w, long rows,
                                int n, int groups, float eps, int after, int f32, hipStream_t s);
 int k8sllm_hy_gated_add_norm(void* out, float* residual, const void* y, int yt, const void* gate, long g_stride,
@@ -161,29 +162,83 @@ int any_dt(const OptT& t, int64_t numel, const char* n) {  // 0 none, 1 bf16, 2 
   return f ? 2 : 1;
 }
 
-void embed_pos(Tensor out, Tensor ids, Tensor positions, Tensor emb, OptT pos, OptT src, OptT prev, double scale) {
-  const int f = act(emb, "embed");
-  f32c(out, "out");
+struct Embed {
+  const int *ids = nullptr, *positions = nullptr, *src = nullptr, *prev = nullptr;
+  const void *emb = nullptr, *pos = nullptr;
+  int vocab = 1, max_pos = 1;
+};
+Embed embed_of(const Tensor& ids, const Tensor& positions, const Tensor& emb, const OptT& pos, const OptT& src, const OptT& prev, int f) {
+  same(emb, f, "embed");
   i32c(ids, "ids");
   i32c(positions, "positions");
   TORCH_CHECK(emb.dim() == 2 && emb.is_contiguous(), "embed [V, d]");
   const int64_t T = ids.numel(), d = emb.size(1);
-  TORCH_CHECK(out.numel() == T * d && positions.numel() >= T, "embed_pos: sizes");
-  int maxp = 1;
+  TORCH_CHECK(positions.numel() >= T, "embed_pos: sizes");
+  Embed e;
   if (pos.has_value()) {
     same(*pos, f, "pos");
     TORCH_CHECK(pos->dim() == 2 && pos->is_contiguous() && pos->size(1) == d, "pos [P, d]");
-    maxp = (int)pos->size(0);
+    e.max_pos = (int)pos->size(0);
+    e.pos = pos->data_ptr();
   }
-  const int* sp = iptr(src, "src");
-  const int* pp = iptr(prev, "prev");
-  TORCH_CHECK((sp == nullptr) == (pp == nullptr), "src and prev come together");
-  if (sp) {
+  e.src = iptr(src, "src");
+  e.prev = iptr(prev, "prev");
+  TORCH_CHECK((e.src == nullptr) == (e.prev == nullptr), "src and prev come together");
+  if (e.src) {
     TORCH_CHECK(src->numel() >= T && prev->numel() >= 1, "src / prev sizes");
   }
-  check(k8sllm_hy_embed_pos(out.data_ptr<float>(), ids.data_ptr<int>(), positions.data_ptr<int>(), emb.data_ptr(),
-                            pos.has_value() ? pos->data_ptr() : nullptr, sp, pp, T, (int)d, (int)emb.size(0), maxp, (float)scale, f, cur()),
+  e.ids = ids.data_ptr<int>();
+  e.positions = positions.data_ptr<int>();
+  e.emb = emb.data_ptr();
+  e.vocab = (int)emb.size(0);
+  return e;
+}
+
+void embed_pos(Tensor out, Tensor ids, Tensor positions, Tensor emb, OptT pos, OptT src, OptT prev, double scale) {
+  const int f = act(emb, "embed");
+  f32c(out, "out");
+  const Embed e = embed_of(ids, positions, emb, pos, src, prev, f);
+  const int64_t T = ids.numel(), d = emb.size(1);
+  TORCH_CHECK(out.numel() == T * d, "embed_pos: sizes");
+  check(k8sllm_hy_embed_pos(out.data_ptr<float>(), e.ids, e.positions, e.emb, e.pos, e.src, e.prev, T, (int)d, e.vocab, e.max_pos,
+                            (float)scale, f, cur()),
         "embed_pos");
+}
+
+// The router whose results the normed rows' launch writes
+struct Route {
+  int* ids = nullptr;
+  float *wts = nullptr, *gate = nullptr;
+  const float *wr = nullptr, *bias = nullptr;
+  int E = 0, K = 0, rows = 0;
+};
+Route route_of(const OptT& ids, const OptT& wts, const OptT& gate, const OptT& wr, const OptT& bias, int64_t E, int64_t K, int64_t rows,
+               int64_t d) {
+  Route r;
+  if (!ids.has_value()) return r;
+  TORCH_CHECK(wts.has_value() && wr.has_value() && d % 8 == 0 && d > 0, "add_norm: router");
+  i32c(*ids, "ids");
+  f32c(*wts, "wts");
+  f32c(*wr, "router weight");
+  TORCH_CHECK(wr->dim() == 2 && wr->size(1) == d && (wr->size(0) == E || wr->size(0) == E + 1) && wr->size(0) <= 9, "router rows");
+  TORCH_CHECK(K >= 1 && K <= E && ids->numel() == rows * K && wts->numel() == rows * K, "router: outputs");
+  if (bias.has_value()) {
+    f32c(*bias, "router bias");
+    TORCH_CHECK(bias->numel() >= E, "router bias [E]");
+    r.bias = bias->data_ptr<float>();
+  }
+  if (gate.has_value()) {
+    f32c(*gate, "gate");
+    TORCH_CHECK(gate->numel() == rows && wr->size(0) == E + 1, "gate [T] needs the extra router row");
+    r.gate = gate->data_ptr<float>();
+  }
+  r.ids = ids->data_ptr<int>();
+  r.wts = wts->data_ptr<float>();
+  r.wr = wr->data_ptr<float>();
+  r.E = (int)E;
+  r.K = (int)K;
+  r.rows = (int)wr->size(0);
+  return r;
 }
 
 // ys, inv, wts (, shared (, gate)): addend `at` is the sum of each row's experts (moe_combine).  r_ids, r_wts (, r_gate), wr (, bias):
@@ -226,33 +281,40 @@ void add_norm_experts(Tensor out, Tensor residual, OptT a0, OptT a1, OptT a2, Op
     }
     t[at] = 3;
   }
-  float* rg = nullptr;
-  if (r_ids.has_value()) {
-    TORCH_CHECK(r_wts.has_value() && wr.has_value() && d % 8 == 0 && d > 0, "add_norm: router");
-    i32c(*r_ids, "ids");
-    f32c(*r_wts, "wts");
-    f32c(*wr, "router weight");
-    TORCH_CHECK(wr->dim() == 2 && wr->size(1) == d && (wr->size(0) == E || wr->size(0) == E + 1) && wr->size(0) <= 9, "router rows");
-    TORCH_CHECK(K >= 1 && K <= E && r_ids->numel() == rows * K && r_wts->numel() == rows * K, "router: outputs");
-    if (bias.has_value()) {
-      f32c(*bias, "router bias");
-      TORCH_CHECK(bias->numel() >= E, "router bias [E]");
-    }
-    if (r_gate.has_value()) {
-      f32c(*r_gate, "gate");
-      TORCH_CHECK(r_gate->numel() == rows && wr->size(0) == E + 1, "gate [T] needs the extra router row");
-      rg = r_gate->data_ptr<float>();
-    }
-  }
-  const bool ro = r_ids.has_value(), jo = ys.has_value();
+  const Route ro = route_of(r_ids, r_wts, r_gate, wr, bias, E, K, rows, d);
+  const bool jo = ys.has_value();
   check(k8sllm_hy_add_norm(out.data_ptr(), residual.data_ptr<float>(), a0.has_value() ? a0->data_ptr() : nullptr, t[0],
                            a1.has_value() ? a1->data_ptr() : nullptr, t[1], a2.has_value() ? a2->data_ptr() : nullptr, t[2],
                            vec.has_value() ? vec->data_ptr<float>() : nullptr, w.data_ptr<float>(), rows, (int)d, (float)eps, one_plus,
                            jo ? ys->data_ptr() : nullptr, jo ? inv->data_ptr<int>() : nullptr, jo ? wts->data_ptr<float>() : nullptr, sh,
-                           gp, (int)Ks, ro ? r_ids->data_ptr<int>() : nullptr, ro ? r_wts->data_ptr<float>() : nullptr, rg,
-                           ro ? wr->data_ptr<float>() : nullptr, ro && bias.has_value() ? bias->data_ptr<float>() : nullptr, (int)E, (int)K,
-                           ro ? (int)wr->size(0) : 0, over_all, f, cur()),
+                           gp, (int)Ks, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1, 1.f, ro.ids, ro.wts, ro.gate, ro.wr,
+                           ro.bias, ro.E, ro.K, ro.rows, over_all, f, cur()),
         "add_norm");
+}
+
+// embed_pos into `residual`, + vec, normed; with the rows' router (r_ids ..)
+void embed_norm(Tensor out, Tensor residual, Tensor ids, Tensor positions, Tensor emb, OptT pos, OptT src, OptT prev, double scale, OptT vec,
+                Tensor w, double eps, bool one_plus, OptT r_ids, OptT r_wts, OptT r_gate, OptT wr, OptT bias, int64_t E, int64_t K) {
+  const int f = act(out, "out");
+  f32c(residual, "residual");
+  f32c(w, "w");
+  const Embed e = embed_of(ids, positions, emb, pos, src, prev, f);
+  const int64_t rows = ids.numel(), d = emb.size(1);
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  TORCH_CHECK(d % 8 == 0 && aligned(e.emb) && aligned(e.pos), "embed_norm: rows in 16-byte pieces");
+  TORCH_CHECK(residual.dim() == 2 && residual.size(0) == rows && residual.size(1) == d && out.is_contiguous() && out.numel() == rows * d &&
+                  w.numel() == d,
+              "embed_norm: sizes");
+  if (vec.has_value()) {
+    f32c(*vec, "vec");
+    TORCH_CHECK(vec->numel() == d, "embed_norm: vec [d]");
+  }
+  const Route ro = route_of(r_ids, r_wts, r_gate, wr, bias, E, K, rows, d);
+  check(k8sllm_hy_add_norm(out.data_ptr(), residual.data_ptr<float>(), nullptr, 0, nullptr, 0, nullptr, 0,
+                           vec.has_value() ? vec->data_ptr<float>() : nullptr, w.data_ptr<float>(), rows, (int)d, (float)eps, one_plus, nullptr,
+                           nullptr, nullptr, nullptr, nullptr, 0, e.ids, e.positions, e.emb, e.pos, e.src, e.prev, e.vocab, e.max_pos,
+                           (float)scale, ro.ids, ro.wts, ro.gate, ro.wr, ro.bias, ro.E, ro.K, ro.rows, false, f, cur()),
+        "embed_norm");
 }
 
 void add_norm(Tensor out, Tensor residual, OptT a0, OptT a1, OptT a2, OptT vec, Tensor w, double eps, bool one_plus) {
@@ -1284,6 +1346,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_pos", &embed_pos);
   m.def("add_norm", &add_norm);
   m.def("add_norm_experts", &add_norm_experts);
+  m.def("embed_norm", &embed_norm);
   m.def("gated_group_norm", &gated_group_norm);
   m.def("swiglu", &swiglu);
   m.def("gated_add_norm", &gated_add_norm);

@@ -62,6 +62,18 @@ struct ExpertSum {
   const float* gate;
   int K;
 };
+// The rows' embeddings (embed_pos's) as the residual that the sum starts from: a launch and a pass over the fp32 rows less (8192 rows of 2048, in a
+// step, 26 + 28 us before; the step takes 20 less)
+struct Embed {
+  const int* ids;
+  const int* positions;
+  const void* emb;
+  const void* pos;
+  const int* src;
+  const int* prev;
+  int vocab, max_pos;
+  float scale;
+};
 // The router of the normed rows
 struct Route {
   int* ids;
@@ -72,17 +84,17 @@ struct Route {
   int E, K, rows_w, over_all;
 };
 
-// t0, t1, t2: an addend's type, 0 none, 1 bf16, 2 fp32, 3 (JOIN) the experts' sum.  A thread keeps its first eight columns in registers between sum
+// FROM: the residual 0 read, 1 read, and an addend of type 3 is the experts' sum, 2 the embeddings.  t0, t1, t2: an addend's type, 0 none, 1 bf16, 2 fp32.  A thread keeps its first eight columns in registers between sum
 // and norm.  NR > 0: the router's at most NR weight rows with their logits here too, in the order of hy_router_kernel's sums (from the rounded
 // row); the weights, 64 KB a row from L2 at 8 x 2048, are on their way while the row is summed.
 // A bf16 branch and two experts, us, moe_combine and norm / one launch: 8192 rows of 2048 73 / 55, 200 7.0 / 4.8, 1 5.2 / 4.4; with the router of 8
 // behind them / in it too: 64 rows of 2048 8.1 / 6.7, 255 10.0 / 8.4, 64 of 4096 10.8 / 9.2, 200 of 1024 (fp32) 8.8 / 7.3.
-template <typename T, bool JOIN, int NR>
+template <typename T, int FROM, int NR>
 __global__ __launch_bounds__(256) void add_norm_kernel(T* __restrict__ out, float* __restrict__ residual,
                                                        const void* a0, int t0, const void* a1, int t1, const void* a2,
                                                        int t2, const float* __restrict__ vec,
                                                        const float* __restrict__ w, int d, float eps, int one_plus, ExpertSum ex,
-                                                       Route ro) {
+                                                       Embed em, Route ro) {
   __shared__ float red[4];
   const long row = blockIdx.x;
   float* r = residual + row * d;
@@ -90,7 +102,7 @@ __global__ __launch_bounds__(256) void add_norm_kernel(T* __restrict__ out, floa
   if ((d & 7) == 0) {  // 8 columns per thread and trip, 16 / 32-byte accesses
     auto addend = [&](const void* p, int t, int c, float (&x)[8]) {
       float a[8];
-      if (JOIN && t == 3) {
+      if (FROM == 1 && t == 3) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) a[i] = 0.f;
         float v[8];
@@ -113,8 +125,23 @@ __global__ __launch_bounds__(256) void add_norm_kernel(T* __restrict__ out, floa
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] += a[i];
     };
+    const T *er = nullptr, *pr = nullptr;  // the token's embedding, its position's
+    if (FROM == 2) {
+      int id = em.ids[row];
+      if (em.src != nullptr && em.src[row] >= 0) id = em.prev[em.src[row]];
+      er = reinterpret_cast<const T*>(em.emb) + (long)min(max(id, 0), em.vocab - 1) * d;
+      if (em.pos != nullptr) pr = reinterpret_cast<const T*>(em.pos) + (long)min(max(em.positions[row], 0), em.max_pos - 1) * d;
+    }
     auto sum = [&](int c, float (&x)[8]) {
-      load8(r + c, x);
+      if (FROM == 2) {
+        float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        load8(er + c, x);
+        if (pr != nullptr) load8(pr + c, a);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = fmaf(x[i], em.scale, a[i]);
+      } else {
+        load8(r + c, x);
+      }
       if (t0) addend(a0, t0, c, x);
       if (t1) addend(a1, t1, c, x);
       if (t2) addend(a2, t2, c, x);
@@ -933,27 +960,31 @@ int k8sllm_hy_embed_pos(float* out, const int* ids, const int* positions, const 
   return (int)hipGetLastError();
 }
 
-// An addend of type 3 is the experts' sum (ys ..); r_ids: with the router of the normed rows.  Both want d % 8 == 0, the router at most 9 rows.
+// An addend of type 3 is the experts' sum (ys ..); emb: the residual is written, embed_pos's rows (no addends); r_ids: with the router of the normed
+// rows.  All want d % 8 == 0, the router at most 9 rows.
 int k8sllm_hy_add_norm(void* out, float* residual, const void* a0, int t0, const void* a1, int t1, const void* a2,
                        int t2, const float* vec, const float* w, long rows, int d, float eps, int one_plus, const void* ys,
-                       const int* inv, const float* wts, const void* shared, const float* gate, int K, int* r_ids, float* r_wts,
-                       float* r_gate, const float* wr, const float* bias, int rE, int rK, int rows_w, int over_all, int f32,
-                       hipStream_t s) {
+                       const int* inv, const float* wts, const void* shared, const float* gate, int K, const int* ids,
+                       const int* positions, const void* emb, const void* pos, const int* src, const int* prev, int vocab, int max_pos,
+                       float scale, int* r_ids, float* r_wts, float* r_gate, const float* wr, const float* bias, int rE, int rK, int rows_w,
+                       int over_all, int f32, hipStream_t s) {
   if (rows <= 0) return 0;
   const bool join = t0 == 3 || t1 == 3 || t2 == 3;
-  if ((join || r_ids != nullptr) && d % 8 != 0) return -1;
+  if ((join || emb != nullptr || r_ids != nullptr) && d % 8 != 0) return -1;
+  if (emb != nullptr && (t0 || t1 || t2)) return -1;
   if (r_ids != nullptr && (d < 8 || rows_w > 9 || rK < 1 || rK > rE || rK > kMaxK || rows_w < rE || rows_w > rE + 1)) return -1;
   const ExpertSum ex{ys, inv, wts, shared, gate, K};
   const Route ro{r_ids, r_wts, r_gate, wr, bias, rE, rK, rows_w, over_all};
+  const Embed em{ids, positions, emb, pos, src, prev, vocab, max_pos, scale};
 #define K8SLLM_AN(T_, J, NR)                                                                                               \
   hipLaunchKernelGGL((add_norm_kernel<T_, J, NR>), dim3(rows), dim3(256), 0, s, (T_*)out, residual, a0, t0, a1, t1, a2, t2, vec, w, d, \
-                     eps, one_plus, ex, ro)
+                     eps, one_plus, ex, em, ro)
 #define K8SLLM_ANR(T_, J)                         \
   if (r_ids == nullptr) K8SLLM_AN(T_, J, 0);      \
   else if (rows_w <= 8) K8SLLM_AN(T_, J, 8);      \
   else K8SLLM_AN(T_, J, 9)
 #define K8SLLM_ANJ(T_) \
-  if (join) { K8SLLM_ANR(T_, true); } else { K8SLLM_ANR(T_, false); }
+  if (emb != nullptr) { K8SLLM_ANR(T_, 2); } else if (join) { K8SLLM_ANR(T_, 1); } else { K8SLLM_ANR(T_, 0); }
   if (f32) { K8SLLM_ANJ(float) } else { K8SLLM_ANJ(bf16_t) }
 #undef K8SLLM_ANJ
 #undef K8SLLM_ANR

@@ -133,13 +133,35 @@ def add_norm(residual: torch.Tensor, addends: tuple, vec: Optional[torch.Tensor]
     if at >= 0:
         ex, a[at] = a[at], None
     wr, bias, E, K = route or (None, None, 0, 0)
-    routed: tuple = (None, None, None)
-    if route is not None:
-        T, dev = residual.shape[0], residual.device
-        routed = (torch.empty(T, K, dtype=torch.int32, device=dev), torch.empty(T, K, dtype=torch.float32, device=dev),
-                  torch.empty(T, dtype=torch.float32, device=dev) if wr.shape[0] == E + 1 else None)
+    routed = _route_out(residual, route)
     native().add_norm_experts(out, residual, a[0], a[1], a[2], vec, w, float(eps), bool(one_plus), at, *ex, *routed, wr, bias, E, K, False)
     return out if route is None else (out, routed)
+
+
+def _route_out(residual: torch.Tensor, route: Optional[tuple]) -> tuple:
+    if route is None:
+        return None, None, None
+    (wr, _, E, K), T, dev = route, residual.shape[0], residual.device
+    return (torch.empty(T, K, dtype=torch.int32, device=dev), torch.empty(T, K, dtype=torch.float32, device=dev),
+            torch.empty(T, dtype=torch.float32, device=dev) if wr.shape[0] == E + 1 else None)
+
+
+def embed_norm(ids: torch.Tensor, positions: torch.Tensor, embed: torch.Tensor, pos: Optional[torch.Tensor], src: Optional[torch.Tensor],
+               prev: Optional[torch.Tensor], scale: float, vec: Optional[torch.Tensor], w: torch.Tensor, eps: float, one_plus: bool,
+               route: Optional[tuple] = None) -> tuple:
+    """(embed_pos's rows + ``vec``, add_norm's result for them - with ``route`` a pair, as there), in one launch on the GPU where
+    rows are in 16-byte pieces; ``embed``'s dtype is the result's."""
+    d = embed.shape[1]
+    one = route is None or (embed.is_cuda and route_with_norm(ids.numel(), d, route[0].shape[0]))
+    if not (embed.is_cuda and one and d % 8 == 0 and embed.data_ptr() % 16 == 0 and (pos is None or pos.data_ptr() % 16 == 0)):
+        x = embed_pos(ids, positions, embed, pos, src, prev, scale=scale)
+        return x, add_norm(x, (), vec, w, eps, one_plus, embed.dtype, route=route)
+    x = torch.empty(ids.numel(), d, dtype=torch.float32, device=embed.device)
+    out = torch.empty(x.shape, dtype=embed.dtype, device=embed.device)
+    wr, bias, E, K = route or (None, None, 0, 0)
+    routed = _route_out(x, route)
+    native().embed_norm(out, x, ids, positions, embed, pos, src, prev, float(scale), vec, w, float(eps), bool(one_plus), *routed, wr, bias, E, K)
+    return x, (out if route is None else (out, routed))
 
 
 def route_with_norm(T: int, d: int, rows_w: int) -> bool:
@@ -1284,6 +1306,8 @@ def _rows_form(M: int, N: int, K: int, end: str = "") -> Optional[str]:
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, end: str = "") -> Optional[str]:
+    if x.shape[0] > 64:  # (_rows_form has none; before the other checks, 1.5 us a product of a prompt step)
+        return None
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):  # the library's product has a backward
         return None
     if not (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2

@@ -1370,3 +1370,26 @@ def test_gate_by_value(mfma, vec, dk, dv, Hq, G, off, dt):
     assert torch.equal(got, want) and bool((rows[0] == 7).all())
     cpu = hops.window_attention_decode(*(x.cpu() for x in (qkv[:3], dev[0], dev[1], bt, n)), *a, gate=z.cpu(), g_col=off, by_value=True)
     torch.testing.assert_close(got.cpu().float(), cpu.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("T,d,E,pos,prev,shift,dt", [
+    (1, 8, 0, True, True, False, BF), (64, 2048, 8, True, False, True, BF), (255, 2056, 7, False, True, True, BF), (256, 264, 8, True, False, False, BF),
+    (300, 4104, 0, False, False, False, BF), (37, 1000, 8, True, True, True, torch.float32),
+    (5, 20, 4, True, False, True, BF),  # rows not in 16-byte pieces
+])
+def test_embedding_with_the_norm(T, d, E, pos, prev, shift, dt):
+    """embed_norm against embed_pos, add_norm and moe_router: the same bits, tokens and positions outside the tables included."""
+    g = _g(94)
+    emb, pt = _r(g, 50, d, dt=dt).cuda(), _r(g, 40, d, dt=dt).cuda() if pos else None
+    ids, p = (torch.randint(-2, 55, (T,), generator=g, dtype=torch.int32).cuda() for _ in range(2))
+    src = (torch.arange(T, dtype=torch.int32) % 5 - 1).cuda() if prev else None
+    pv = torch.randint(0, 50, (4,), generator=g, dtype=torch.int32).cuda() if prev else None
+    vec, w = _r(g, d).cuda() if shift else None, torch.rand(d, generator=g).cuda()
+    route = (_r(g, E + 1, d, s=d ** -0.5).cuda(), _r(g, E).cuda(), E, 2) if E else None
+    x = hops.embed_pos(ids, p, emb, pt, src, pv, scale=1.7)
+    h = hops.add_norm(x, (), vec, w, 1e-5, True, dt)
+    gx, gh = hops.embed_norm(ids, p, emb, pt, src, pv, 1.7, vec, w, 1e-5, True, route)
+    if E:
+        gh, r = gh
+        assert all(torch.equal(a, b) for a, b in zip(r, hops.moe_router(h, *route)))
+    assert torch.equal(gx, x) and torch.equal(gh, h)
