@@ -180,6 +180,99 @@ __global__ __launch_bounds__(1024) void moe_align_small_kernel(const int* __rest
   }
 }
 
+// Up to 8 NG experts and kAlignChunkItems items: a workgroup places 1024 of them.  It counts all items and those in front of its own, packed eight bits
+// an expert in a thread (hence the limit: at most 63 times four items a thread), sixteen in a wave's sum; ranks among its own come from ballots, as above.  The
+// counting is done over by every workgroup, 64 KB of ids at 16384 items, and costs less than one workgroup's placing.  us, one workgroup's counters
+// (below) / this: 2000 items of 8 experts 10.1 / 6.9, 16384 19.1 / 7.4, 131072 124 / 17; 16384 of 16 27 / 10.7; 1030 of one 4.9 / 6.1, so from
+// three experts on.
+constexpr long kAlignChunkItems = 63 * 4096;
+template <int NG>
+__global__ __launch_bounds__(1024) void moe_align_chunks_kernel(const int* __restrict__ ids, int n, int E, int* __restrict__ offsets,
+                                                                int* __restrict__ sorted_idx, int* __restrict__ inv_idx) {
+  constexpr int NE = 8 * NG;
+  __shared__ int cnt[16][2][NE];  // a wave's items, and those in front of this workgroup's
+  __shared__ int own[16][NE];
+  __shared__ int start[NE];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c0 = blockIdx.x * 1024;
+  const int e = c0 + t < n ? ids[c0 + t] : -1;
+  uint64_t all[NG] = {}, front[NG] = {};
+  for (int i = 4 * t; i < n; i += 4096) {
+    int v[4];
+    if (i + 4 <= n) {
+      const int4 q = *reinterpret_cast<const int4*>(ids + i);
+      v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = i + k < n ? ids[i + k] : -1;
+    }
+    uint64_t add[NG] = {};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int g = 0; g < NG; ++g) add[g] += v[k] >> 3 == g ? 1ull << (8 * (v[k] & 7)) : 0ull;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      all[g] += add[g];
+      front[g] += i < c0 ? add[g] : 0ull;
+    }
+  }
+  int rank = 0, mine = 0;
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    const unsigned long long mask = __ballot(e == i);
+    if (e == i) rank = __popcll(mask & ((1ull << lane) - 1));
+    if (lane == i) mine = __popcll(mask);
+  }
+  if (lane < NE) own[wave][lane] = mine;
+  auto sum = [&](const uint64_t (&x)[NG], int* out) {  // over the wave, sixteen bits an expert
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {  // even experts, odd ones
+        uint32_t w[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          w[p] = (uint32_t)(x[g] >> (32 * p + 8 * h)) & 0x00ff00ffu;
+#pragma unroll
+          for (int o = 1; o < 64; o <<= 1) w[p] += __shfl_xor(w[p], o, 64);
+          if (lane == 0) {
+            out[8 * g + 4 * p + h] = w[p] & 0xffff;
+            out[8 * g + 4 * p + h + 2] = w[p] >> 16;
+          }
+        }
+      }
+  };
+  sum(all, cnt[wave][0]);
+  sum(front, cnt[wave][1]);
+  __syncthreads();
+  if (t < 64) {
+    int tot = 0, f = 0;
+    if (t < NE)
+#pragma unroll
+      for (int w = 0; w < 16; ++w) {
+        tot += cnt[w][0][t];
+        f += cnt[w][1][t];
+      }
+    int x = tot;
+#pragma unroll
+    for (int o = 1; o < NE; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (t < NE) start[t] = x - tot + f;
+    if (blockIdx.x == 0 && t < E) offsets[t] = x - tot;
+    if (blockIdx.x == 0 && t == E - 1) offsets[E] = x;
+  }
+  __syncthreads();
+  if (e >= 0) {
+    int pos = start[e] + rank;
+#pragma unroll
+    for (int w = 0; w < 15; ++w) pos += w < wave ? own[w][e] : 0;
+    sorted_idx[pos] = c0 + t;
+    inv_idx[c0 + t] = pos;
+  }
+}
+
 // NT threads x ME experts of per-thread counters fill the 64 KiB of LDS: 1024 x 16 (Mixtral),
 // 256 x 64, 64 x 256.
 template <int NT, int ME>
@@ -293,6 +386,9 @@ int k8sllm_moe_align(const int* topk_ids, long n, int E, int* expert_offsets, in
   if (n > 0 && n <= 1024 && E <= 64)
     hipLaunchKernelGGL(moe_align_small_kernel, dim3(1), dim3((unsigned)((n + 63) / 64 * 64)), 0, s, topk_ids, (int)n, E, expert_offsets,
                        sorted_idx, inv_idx);
+  else if (E >= 3 && E <= 16 && n > 0 && n <= kAlignChunkItems)
+    hipLaunchKernelGGL((E <= 8 ? &moe_align_chunks_kernel<1> : &moe_align_chunks_kernel<2>), dim3((unsigned)((n + 1023) / 1024)), dim3(1024), 0,
+                       s, topk_ids, (int)n, E, expert_offsets, sorted_idx, inv_idx);
   else if (E <= kMaxE)
     hipLaunchKernelGGL((moe_align_kernel<kAT, kMaxE>), dim3(1), dim3(kAT), 0, s, topk_ids, n, E, expert_offsets,
                        sorted_idx, inv_idx);

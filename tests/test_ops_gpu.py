@@ -687,3 +687,15 @@ def test_rope_and_cache_prefill_block_runs(d):
     _close(qkv, q2.to(DEV), atol=2e-2, rtol=1e-2, what="rope qkv")
     _close(kc, kc0.to(DEV), atol=2e-2, rtol=1e-2, what="k_cache")
     assert torch.equal(vc.cpu(), vc0), "v_cache"
+
+
+@pytest.mark.parametrize("n,E,skew", [(1025, 3, False), (2048, 8, False), (4099, 9, True), (16387, 16, False), (16384, 8, True), (258048, 5, True),
+                                      (258049, 5, True), (3000, 2, False)])
+def test_moe_align_chunks(n, E, skew):
+    """Items over several workgroups, the last one short; nearly all of one expert; the largest count and the one that leaves it."""
+    g = torch.Generator().manual_seed(n)
+    ids = torch.randint(0, E, (n, 1), generator=g, dtype=torch.int32)
+    if skew:
+        ids[torch.rand(n, generator=g) < 0.97] = E - 1
+    for a, b in zip(ops.moe_align(ids.to(DEV), E), ref.moe_align(ids, E)):
+        assert torch.equal(a.cpu(), b)
