@@ -751,13 +751,10 @@ using namespace k8sllm;
 // 8192, 128 rows 100 / 31; 28672 x 4096 (SWIGLU8) 80 rows 90 / 69; 8192 x 2048, 65 rows 33 / 25, 256 34.6 / 34.9, 512 38 / 43 (left whole).  Strips of 64 rows, split, were slower but for 1024
 // columns, and 256 tiles at once slower than 200.  With RESID an 8 B Llama's prompt of 1500 tokens takes 23.4 / 20.9 ms, one of 1900 (128 tiles and
 // more, whole) 27.4 / 26.8.
-// From 1024 rows on only RESID, which a tensor-parallel rank has not: its overlapped prefill takes a step's rows in two parts of at least 1024, whose
-// results are to be the undivided step's to the bit, and parts of K add up in another order.
-constexpr long kSplitRows = 1024;
 static int tile_splits(long M, long N, long K, int epi) {
   const long nk = K >> 6, tiles = (M + 255) / 256 * ((N + 255) / 256);
   const bool rope = epi == TILE_EPI_ROPE, resid = epi == TILE_EPI_RESID, unit = epi == TILE_EPI_SWIGLU || epi == TILE_EPI_SWIGLU8;
-  if (!(epi == TILE_EPI_BF16 || rope || unit || resid) || (M >= kSplitRows && !resid) || tiles > 120 || N % (epi == TILE_EPI_BF16 ? 8 : 128)) return 1;
+  if (!(epi == TILE_EPI_BF16 || rope || unit || resid) || tiles > 120 || N % (epi == TILE_EPI_BF16 ? 8 : 128)) return 1;
   float best = nk * (resid ? 1.1f : tiles <= kStripTiles && !rope ? 0.87f : 1.25f);
   int S = 1;
   for (int n = 2; n <= 16 && n * tiles <= 240; ++n) {
