@@ -673,10 +673,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 }
 
 // The end of a product whose K was split: the sums over the splits in their order, rounded, then what the tile's epilogue EPI does with them (BF16,
-// ROPE, SWIGLU, SWIGLU8, RESID).  A thread takes eight columns, or the eight and those that they meet; RESID: sixteen lanes 128 columns.
+// ROPE, SWIGLU, SWIGLU8).  A thread takes eight columns, or the eight and those that they meet.
 template <int EPI>
 __global__ __launch_bounds__(256) void reduce_tiles_kernel(bf16_t* __restrict__ Y, const float* __restrict__ part_sums, int S, int M, int N,
-                                                           TileEpi ep) {
+                                                           const int* __restrict__ positions, const float* __restrict__ cos_sin, int rope_heads) {
   constexpr bool UNIT = EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8, PAIRS = UNIT || EPI == TILE_EPI_ROPE;
   const long i = (long)blockIdx.x * 256 + threadIdx.x, mn = (long)M * N;
   const int per = PAIRS ? N / 16 : N / 8;
@@ -708,8 +708,8 @@ __global__ __launch_bounds__(256) void reduce_tiles_kernel(bf16_t* __restrict__ 
       *reinterpret_cast<uint4*>(Y + row * (N >> 1) + e * 8) = pack8(o1);
       return;
     }
-    if ((e >> 3) < ep.rope_heads) {
-      const float* cs = ep.cos_sin + (long)ep.positions[row] * 128 + (e & 7) * 8;
+    if ((e >> 3) < rope_heads) {
+      const float* cs = cos_sin + (long)positions[row] * 128 + (e & 7) * 8;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         o1[k] = x1[k] * cs[k] - x2[k] * cs[64 + k];
@@ -720,23 +720,6 @@ __global__ __launch_bounds__(256) void reduce_tiles_kernel(bf16_t* __restrict__ 
     }
     *reinterpret_cast<uint4*>(Y + row * N + c + 64) = hi;
   }
-  if constexpr (EPI == TILE_EPI_RESID) {  // (N % 128 == 0: a row's lanes are whole groups of sixteen)
-    float y[8], rv[8], wf[8], h[8], hw[8], ss = 0.f;
-    unpack8(lo, y);
-    unpack8(*reinterpret_cast<const uint4*>(ep.resid + row * N + c), rv);
-    unpack8(*reinterpret_cast<const uint4*>(ep.norm_w + c), wf);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      h[k] = bf2f(f2bf(y[k] + rv[k]));
-      ss += h[k] * h[k];
-      hw[k] = h[k] * wf[k];
-    }
-    *reinterpret_cast<uint4*>(ep.resid + row * N + c) = pack8(h);
-    *reinterpret_cast<uint4*>(ep.hw + row * N + c) = pack8(hw);
-    ss = row16_sum(ss);
-    if ((e & 15) == 0) ep.ss_out[row * (N >> 7) + (e >> 4)] = ss;
-    return;
-  }
   *reinterpret_cast<uint4*>(Y + row * N + c) = lo;
 }
 
@@ -745,17 +728,16 @@ __global__ __launch_bounds__(256) void reduce_tiles_kernel(bf16_t* __restrict__ 
 using namespace k8sllm;
 
 // How many parts K of a dense product of few tiles is cut into (1: none): a prompt step of some hundred rows has 16 to 100 tiles, each a chain of K / 64
-// k-tiles.  By an estimate of both, in us: a k-tile takes 1.25 with up to 200 tiles on the chip (RESID, whole: 1.1), 1.45 with more, 0.87 as a strip; the parts' sums pass
+// k-tiles.  By an estimate of both, in us: a k-tile takes 1.25 with up to 200 tiles on the chip, 1.45 with more, 0.87 as a strip; the parts' sums pass
 // memory twice and a launch more.  Measured, whole / split (packed weights): 4096 x 4096, 65 rows 56 / 26, 256 56 / 35, 512 57 / 42, 768 58 / 47; 4096 x
 // 14336, 65 rows 168 / 40, 256 166 / 55, 512 170 / 73, 1000 182 / 109; 6144 x 4096 (ROPE) 65 rows 78 / 31, 512 82 / 49, 1000 87 / 68; 1024 x
 // 8192, 128 rows 100 / 31; 28672 x 4096 (SWIGLU8) 80 rows 90 / 69; 8192 x 2048, 65 rows 33 / 25, 256 34.6 / 34.9, 512 38 / 43 (left whole).  Strips of 64 rows, split, were slower but for 1024
-// columns, and 256 tiles at once slower than 200.  With RESID an 8 B Llama's prompt of 1500 tokens takes 23.4 / 20.9 ms, one of 1900 (128 tiles and
-// more, whole) 27.4 / 26.8.
+// columns, and 256 tiles at once slower than 200.
 static int tile_splits(long M, long N, long K, int epi) {
   const long nk = K >> 6, tiles = (M + 255) / 256 * ((N + 255) / 256);
-  const bool rope = epi == TILE_EPI_ROPE, resid = epi == TILE_EPI_RESID, unit = epi == TILE_EPI_SWIGLU || epi == TILE_EPI_SWIGLU8;
-  if (!(epi == TILE_EPI_BF16 || rope || unit || resid) || tiles > 120 || N % (epi == TILE_EPI_BF16 ? 8 : 128)) return 1;
-  float best = nk * (resid ? 1.1f : tiles <= kStripTiles && !rope ? 0.87f : 1.25f);
+  const bool rope = epi == TILE_EPI_ROPE, unit = epi == TILE_EPI_SWIGLU || epi == TILE_EPI_SWIGLU8;
+  if (!(epi == TILE_EPI_BF16 || rope || unit) || tiles > 120 || N % (epi == TILE_EPI_BF16 ? 8 : 128)) return 1;
+  float best = nk * (tiles <= kStripTiles && !rope ? 0.87f : 1.25f);
   int S = 1;
   for (int n = 2; n <= 16 && n * tiles <= 240; ++n) {
     const long per = (nk + n - 1) / n;
@@ -819,13 +801,12 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
     if (S < 2 || algo != 1 || grouped || rs) return -1;
     hipLaunchKernelGGL((gemm_w4_kernel<TILE_EPI_BF16, false, 1, false, true>), dim3((unsigned)nwg, (unsigned)S), dim3(256), 0, s, (const bf16_t*)X,
                        (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk, 0, ws, per);
-    const dim3 groups((unsigned)(((long)M * (N / (epi == TILE_EPI_BF16 || epi == TILE_EPI_RESID ? 8 : 16)) + 255) / 256));
+    const dim3 groups((unsigned)(((long)M * (N / (epi == TILE_EPI_BF16 ? 8 : 16)) + 255) / 256));
 #define K8_TILE_REDUCE(EPI_) \
-  hipLaunchKernelGGL(reduce_tiles_kernel<EPI_>, groups, dim3(256), 0, s, (bf16_t*)Y, ws, S, M, N, ep)
+  hipLaunchKernelGGL(reduce_tiles_kernel<EPI_>, groups, dim3(256), 0, s, (bf16_t*)Y, ws, S, M, N, rope_pos, rope_cs, rope_heads)
     if (epi == TILE_EPI_ROPE) K8_TILE_REDUCE(TILE_EPI_ROPE);
     else if (epi == TILE_EPI_SWIGLU) K8_TILE_REDUCE(TILE_EPI_SWIGLU);
     else if (epi == TILE_EPI_SWIGLU8) K8_TILE_REDUCE(TILE_EPI_SWIGLU8);
-    else if (epi == TILE_EPI_RESID) K8_TILE_REDUCE(TILE_EPI_RESID);
     else K8_TILE_REDUCE(TILE_EPI_BF16);
 #undef K8_TILE_REDUCE
     return (int)hipGetLastError();
