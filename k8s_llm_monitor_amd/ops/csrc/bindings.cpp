@@ -47,8 +47,7 @@ int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void* Y2, int M
 int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, int N, int K, const int* offsets, int E, long w_es,
                      int epi, int algo, const int* rope_pos, const float* rope_cs, int rope_heads,
                      const float* rs_part, int rs_np, float rs_eps, void* resid, void* hw, const void* norm_w,
-                     float* ss_out, int wpk, const int* src, int src_div, long src_rows, float* ws, hipStream_t s);
-long k8sllm_gemm_tile_ws(long M, long N, long K, int epi, int algo);
+                     float* ss_out, int wpk, const int* src, int src_div, long src_rows, hipStream_t s);
 int k8sllm_moe_grouped_gemm(const void* X, const void* W, void* Y, const int* offsets, int E, long rows, int N, int K,
                             long w_es, int epi, hipStream_t s);
 int k8sllm_gemm_skinny(const void* A, long lda, const void* Wp, float* partial, void* Y, long ldy, int M, int N, int K,
@@ -495,15 +494,11 @@ void gemm_tile(torch::Tensor y, torch::Tensor x, torch::Tensor w, c10::optional<
   }
   TORCH_CHECK(swiglu == 0 || swiglu == 1 || swiglu == 8, "gemm_tile: swiglu 0, 1 or 8");
   const int epi = rsd ? 3 : rp ? 2 : (swiglu == 8 ? 4 : swiglu ? 1 : 0);
-  // few tiles: K in parts, their sums in a workspace (stream-ordered caching allocator, graph-pool safe)
-  torch::Tensor ws;
-  const long nws = grouped || rsp || M <= 0 ? 0 : k8sllm_gemm_tile_ws(M, N, K, epi, (int)algo);
-  if (nws) ws = torch::empty({nws}, x.options().dtype(torch::kFloat32));
   check(k8sllm_gemm_tile(x.data_ptr(), w.data_ptr(), rsd ? resid->data_ptr() : y.data_ptr(), M, N, K, op, E,
                          (long)N * K, epi, (int)algo, rp, rc, (int)rope_heads, rsp, rs_np, (float)rs_eps,
                          rsd ? resid->data_ptr() : nullptr, rsd ? hw->data_ptr() : nullptr,
                          rsd ? norm_w->data_ptr() : nullptr, rsd ? ss_out->data_ptr<float>() : nullptr, wpk ? 1 : 0,
-                         nullptr, 1, 0, nws ? ws.data_ptr<float>() : nullptr, cur()),
+                         nullptr, 1, 0, cur()),
         "gemm_tile");
 }
 
@@ -522,7 +517,7 @@ void gemm_tile_rows(torch::Tensor y, torch::Tensor x, torch::Tensor w, torch::Te
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "gemm_tile_rows: alignment of x");
   check(k8sllm_gemm_tile(x.data_ptr(), w.data_ptr(), y.data_ptr(), (int)M, N, K, offsets.data_ptr<int>(), E, (long)N * K, swiglu ? 1 : 0,
                          (int)algo, nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, 0, rows.data_ptr<int>(),
-                         (int)div, x.size(0), nullptr, cur()),
+                         (int)div, x.size(0), cur()),
         "gemm_tile_rows");
 }
 

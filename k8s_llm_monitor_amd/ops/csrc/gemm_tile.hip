@@ -83,12 +83,11 @@ constexpr bool tile_strips() {
 // workgroups that strips of up to this many tiles add
 static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * 32 - tiles; }
 
-// SPLIT: blockIdx.y takes `per` k-tiles and writes its fp32 sums to part [blockIdx.y][M][N], for reduce_tiles_kernel to end.
-template <int EPI, bool GROUPED, int SCH, bool RS = false, bool SPLIT = false>
+template <int EPI, bool GROUPED, int SCH, bool RS = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                          int E, int M, int N, int K, long w_es, int n_mt, int n_nt,
-                                                         TileEpi ep, int wpk, int strips, float* __restrict__ part_sums, int per) {
+                                                         TileEpi ep, int wpk, int strips) {
   constexpr int HS = 32768;  // one half-slot: 256 rows x 128 B
   __shared__ __attribute__((aligned(16))) char smem[5 * HS];
   const int lane = threadIdx.x & 63;
@@ -96,7 +95,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   const int wm = wave >> 1, wn = wave & 1;
 
   // ---- logical tile: bijective XCD remap, then groups of 8 m-tiles ----
-  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>() && !SPLIT;
+  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>();
   int mts = n_mt;
   if (GROUPED && STRIPS && strips) {  // the tiles that there are
     mts = 0;
@@ -192,7 +191,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
                                          sorts ? ep.src_bytes : (long)mrows * K * 2);
   const __amdgpu_buffer_rsrc_t wr = GLU ? rsrc(Wt, (long)N * K * 2)
                                         : rsrc(reinterpret_cast<const char*>(Wt) + (long)n0 * K * 2, (long)nrows * K * 2);
-  const int kb = SPLIT ? blockIdx.y * per : 0, nk = SPLIT ? min(per, (K >> 6) - kb) : K >> 6;
+  const int nk = K >> 6;
 
   // piece p of half-tile (operand o, k-tile kt) into half-slot `slot`; k-tiles past the end re-read
   // the last one (identical bytes into a slot no live fragment read uses), so every sub-step
@@ -200,9 +199,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   auto piece = [&](int o, int p, int kt, int slot) {
     char* dst = smem + slot * HS + (p * 4 + wave) * 1024;
     if (o)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)dst, 16, soff[1][p], (kb + min(kt, nk - 1)) * kstrB, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)dst, 16, soff[1][p], min(kt, nk - 1) * kstrB, 0, 0);
     else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)dst, 16, soff[0][p], (kb + min(kt, nk - 1)) * 128, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)dst, 16, soff[0][p], min(kt, nk - 1) * 128, 0, 0);
   };
   auto issue_half = [&](int o, int kt) {
 #pragma unroll
@@ -241,7 +240,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     constexpr int SS = 8192 + HS;
     auto fill = [&](int kt) {
       char* dst = smem + (kt & 3) * SS + wave * 1024;
-      const int k = kb + min(kt, nk - 1);
+      const int k = min(kt, nk - 1);
 #pragma unroll
       for (int p = 0; p < 2; ++p) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(dst + p * 4096), 16, soff[0][p], k * 128, 0, 0);
 #pragma unroll
@@ -294,7 +293,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     };
     auto pc = [&](int o, int p, int kt, uint32_t slot_bytes) {
       char* dst = smem + slot_bytes + (p * 4 + wave) * 1024;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(o ? wr : xr, (lds_void_t*)dst, 16, soff[o][p], (kb + min(kt, nk - 1)) * (o ? kstrB : 128),
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(o ? wr : xr, (lds_void_t*)dst, 16, soff[o][p], min(kt, nk - 1) * (o ? kstrB : 128),
                                                0, 0);
     };
     // PM (the ring tail, peeled): 0 = B_{t+2} and A_{t+3} refills; 1 = B_{t+2} only (A_{t+3} is
@@ -476,17 +475,6 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   // writes its quarter as bf16 rows (8-B ds_write per 4 columns), then reads back whole rows and
   // stores 16 B per lane, 256 contiguous bytes per row - half the store instructions of writing
   // the accumulator layout directly, which is what bounds a store tail (T21). ----
-  if constexpr (SPLIT) {
-    float* const dst = part_sums + (long)blockIdx.y * M * N + (long)row0 * N + n0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int row = wm * 128 + i * 16 + (lane & 15), col = wn * 128 + j * 16 + 4 * (lane >> 4);
-        if (row < mrows && col < nrows) *reinterpret_cast<f32x4*>(dst + (long)row * N + col) = acc[i][j];
-      }
-    return;
-  }
   lgkm_wait0();
   __builtin_amdgcn_s_barrier();  // every wave is done with the ring (its last DMAs retired above)
   auto finish = [&](auto gated, auto blocks) {  // gated: a unit's tile; blocks: of 16 rows, a wave's
@@ -672,87 +660,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   end(std::integral_constant<int, 8>{});
 }
 
-// The end of a product whose K was split: the sums over the splits in their order, rounded, then what the tile's epilogue EPI does with them (BF16,
-// ROPE, SWIGLU, SWIGLU8).  A thread takes eight columns, or the eight and those that they meet.
-template <int EPI>
-__global__ __launch_bounds__(256) void reduce_tiles_kernel(bf16_t* __restrict__ Y, const float* __restrict__ part_sums, int S, int M, int N,
-                                                           const int* __restrict__ positions, const float* __restrict__ cos_sin, int rope_heads) {
-  constexpr bool UNIT = EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8, PAIRS = UNIT || EPI == TILE_EPI_ROPE;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x, mn = (long)M * N;
-  const int per = PAIRS ? N / 16 : N / 8;
-  const long row = i / per;
-  if (row >= M) return;
-  const int e = (int)(i - row * per), c = !PAIRS ? e * 8 : EPI == TILE_EPI_SWIGLU8 ? e * 16 : (e >> 3) * 128 + (e & 7) * 8;
-  auto sum = [&](int col) {
-    const float* p = part_sums + row * N + col;
-    float v[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = 0.f;
-#pragma unroll 4
-    for (int z = 0; z < S; ++z) {
-      const float4 a = *reinterpret_cast<const float4*>(p + z * mn), b = *reinterpret_cast<const float4*>(p + z * mn + 4);
-      v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
-      v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
-    }
-    return pack8(v);
-  };
-  uint4 lo = sum(c);
-  if constexpr (PAIRS) {
-    uint4 hi = sum(c + (EPI == TILE_EPI_SWIGLU8 ? 8 : 64));
-    float x1[8], x2[8], o1[8], o2[8];
-    unpack8(lo, x1);
-    unpack8(hi, x2);
-    if constexpr (UNIT) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) o1[k] = x1[k] * x2[k] / (1.f + __expf(-x1[k]));
-      *reinterpret_cast<uint4*>(Y + row * (N >> 1) + e * 8) = pack8(o1);
-      return;
-    }
-    if ((e >> 3) < rope_heads) {
-      const float* cs = cos_sin + (long)positions[row] * 128 + (e & 7) * 8;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        o1[k] = x1[k] * cs[k] - x2[k] * cs[64 + k];
-        o2[k] = x2[k] * cs[k] + x1[k] * cs[64 + k];
-      }
-      lo = pack8(o1);
-      hi = pack8(o2);
-    }
-    *reinterpret_cast<uint4*>(Y + row * N + c + 64) = hi;
-  }
-  *reinterpret_cast<uint4*>(Y + row * N + c) = lo;
-}
-
 }  // namespace k8sllm
 
 using namespace k8sllm;
-
-// How many parts K of a dense product of few tiles is cut into (1: none): a prompt step of some hundred rows has 16 to 100 tiles, each a chain of K / 64
-// k-tiles.  By an estimate of both, in us: a k-tile takes 1.25 with up to 200 tiles on the chip, 1.45 with more, 0.87 as a strip; the parts' sums pass
-// memory twice and a launch more.  Measured, whole / split (packed weights): 4096 x 4096, 65 rows 56 / 26, 256 56 / 35, 512 57 / 42, 768 58 / 47; 4096 x
-// 14336, 65 rows 168 / 40, 256 166 / 55, 512 170 / 73, 1000 182 / 109; 6144 x 4096 (ROPE) 65 rows 78 / 31, 512 82 / 49, 1000 87 / 68; 1024 x
-// 8192, 128 rows 100 / 31; 28672 x 4096 (SWIGLU8) 80 rows 90 / 69; 8192 x 2048, 65 rows 33 / 25, 256 34.6 / 34.9, 512 38 / 43 (left whole).  Strips of 64 rows, split, were slower but for 1024
-// columns, and 256 tiles at once slower than 200.
-static int tile_splits(long M, long N, long K, int epi) {
-  const long nk = K >> 6, tiles = (M + 255) / 256 * ((N + 255) / 256);
-  const bool rope = epi == TILE_EPI_ROPE, unit = epi == TILE_EPI_SWIGLU || epi == TILE_EPI_SWIGLU8;
-  if (!(epi == TILE_EPI_BF16 || rope || unit) || tiles > 120 || N % (epi == TILE_EPI_BF16 ? 8 : 128)) return 1;
-  float best = nk * (tiles <= kStripTiles && !rope ? 0.87f : 1.25f);
-  int S = 1;
-  for (int n = 2; n <= 16 && n * tiles <= 240; ++n) {
-    const long per = (nk + n - 1) / n;
-    if (per < 8 || nk - per * (n - 1) < 4) continue;
-    const float us = per * (n * tiles > 200 ? 1.45f : 1.25f) + 8.f + 2.5e-7f * M * N * (8 * n + 2);
-    if (us < best) best = us, S = n;
-  }
-  return S;
-}
-
-// floats of workspace for a dense product's splits; 0: none
-extern "C" long k8sllm_gemm_tile_ws(long M, long N, long K, int epi, int algo) {
-  const int S = algo == 1 ? tile_splits(M, N, K, epi) : 1;
-  return S > 1 ? S * M * N : 0;
-}
 
 // Dense (offsets == nullptr): Y [M][N] (SwiGLU: [M][N / 2]) = X [M][K] . W[N][K]^T.
 // Grouped: W [E][N][K] with expert stride w_es elements; M = total expert-sorted rows (the grid
@@ -765,8 +675,7 @@ extern "C" long k8sllm_gemm_tile_ws(long M, long N, long K, int epi, int algo) {
 extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, int N, int K, const int* offsets, int E,
                                 long w_es, int epi, int algo, const int* rope_pos, const float* rope_cs,
                                 int rope_heads, const float* rs_part, int rs_np, float rs_eps, void* resid, void* hw,
-                                const void* norm_w, float* ss_out, int wpk, const int* src, int src_div, long src_rows, float* ws,
-                                hipStream_t s) {
+                                const void* norm_w, float* ss_out, int wpk, const int* src, int src_div, long src_rows, hipStream_t s) {
   if (M <= 0) return 0;
   const bool grouped = offsets != nullptr;
   if (src != nullptr && (!grouped || src_div < 1 || src_rows < 1)) return -1;
@@ -796,28 +705,13 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   const int n_mt = (M + 255) / 256 + (grouped ? E : 0), n_nt = (N + 255) / 256;
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
-  if (ws != nullptr) {
-    const int S = tile_splits(M, N, K, epi), per = ((K >> 6) + S - 1) / S;
-    if (S < 2 || algo != 1 || grouped || rs) return -1;
-    hipLaunchKernelGGL((gemm_w4_kernel<TILE_EPI_BF16, false, 1, false, true>), dim3((unsigned)nwg, (unsigned)S), dim3(256), 0, s, (const bf16_t*)X,
-                       (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk, 0, ws, per);
-    const dim3 groups((unsigned)(((long)M * (N / (epi == TILE_EPI_BF16 ? 8 : 16)) + 255) / 256));
-#define K8_TILE_REDUCE(EPI_) \
-  hipLaunchKernelGGL(reduce_tiles_kernel<EPI_>, groups, dim3(256), 0, s, (bf16_t*)Y, ws, S, M, N, rope_pos, rope_cs, rope_heads)
-    if (epi == TILE_EPI_ROPE) K8_TILE_REDUCE(TILE_EPI_ROPE);
-    else if (epi == TILE_EPI_SWIGLU) K8_TILE_REDUCE(TILE_EPI_SWIGLU);
-    else if (epi == TILE_EPI_SWIGLU8) K8_TILE_REDUCE(TILE_EPI_SWIGLU8);
-    else K8_TILE_REDUCE(TILE_EPI_BF16);
-#undef K8_TILE_REDUCE
-    return (int)hipGetLastError();
-  }
   const bool cut = algo == 1 && !rs && epi != TILE_EPI_ROPE && epi != TILE_EPI_RESID && E <= kStripExperts;
   const long over = nwg % kTileCus;
   const int strips = cut && (grouped || (over > 0 && over <= kStripTiles));
   const dim3 grid((unsigned)(nwg + (!strips ? 0 : grouped ? 4 * kStripTiles : strip_groups(over))));
 #define K8_TILE_LAUNCH(EPI_, G_, SCH_, RS_)                                                                          \
   hipLaunchKernelGGL((gemm_w4_kernel<EPI_, G_, SCH_, RS_>), grid, dim3(256), 0, s, (const bf16_t*)X,                \
-                     (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk, strips, (float*)nullptr, 0)
+                     (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk, strips)
 #define K8_TILE_SCH(SCH_)                                                                                            \
   if (grouped) {                                                                                                     \
     if (epi == TILE_EPI_SWIGLU) K8_TILE_LAUNCH(TILE_EPI_SWIGLU, true, SCH_, false);                                  \
@@ -863,7 +757,7 @@ extern "C" int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void
   const long groups = nwg + (strips ? strip_groups(over) : 0);
 #define K8_TILE_UNIT(EPI_)                                                                                             \
   hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false>), dim3((unsigned)groups), dim3(256), 0, s, (const bf16_t*)X, \
-                     (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0, strips, (float*)nullptr, 0)
+                     (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0, strips)
   if (epi == TILE_EPI_GELU_GLU) K8_TILE_UNIT(TILE_EPI_GELU_GLU);
   else if (epi == TILE_EPI_SILU_GLU) K8_TILE_UNIT(TILE_EPI_SILU_GLU);
   else if (epi == TILE_EPI_RELU_GLU) K8_TILE_UNIT(TILE_EPI_RELU_GLU);

@@ -207,31 +207,3 @@ def test_gemm_tile_last_round(m_tiles, n_tiles, last, K, swiglu):
     up, gate = z[:, f:2 * f].float(), z[:, :f].float()
     torch.testing.assert_close(y.float(), torch.nn.functional.silu(gate) * up, rtol=2 ** -7, atol=2 ** -7)
     assert torch.equal(y2, z[:, 2 * f:])
-
-
-@pytest.mark.parametrize("M,N,K,packed", [
-    (65, 4096, 4096, True), (1, 256, 1088, False), (43, 6144, 4096, True), (257, 1024, 8192, False), (300, 2064, 2112, True), (512, 512, 16384, False),
-    (1000, 4096, 14336, True), (80, 28672, 4096, True),
-])
-def test_gemm_tile_split_k(M, N, K, packed):
-    """Few tiles with K in parts (the last one short, too): plain, turned, gated in both pairings.  Against the schedule that is never split and the
-    fp32 product: another order of fp32 sums, so a rounding of the result to bf16 may differ (2^-8 of it)."""
-    g = torch.Generator().manual_seed(6)
-    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
-    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
-    wd = ops.pack_skinny(w) if packed else w
-    tol = dict(rtol=2 ** -7, atol=2 ** -7)
-    y = ops.gemm_tile(x, wd, algo=1)
-    torch.testing.assert_close(y.float(), ops.gemm_tile(x, wd, algo=0).float(), **tol)
-    torch.testing.assert_close(y.float(), x.float() @ w.float().t(), **tol)
-    if N % 128 == 0:
-        pos = torch.randint(0, 300, (M,), generator=g, dtype=torch.int32).cuda()
-        cs = torch.randn(300, 128, generator=g).cuda()
-        rope = (pos, cs, max(N // 128 - 2, 0))
-        torch.testing.assert_close(ops.gemm_tile(x, wd, algo=1, rope=rope).float(), ops.gemm_tile(x, wd, algo=0, rope=rope).float(), rtol=2 ** -6, atol=2 ** -5)
-    # gate and up are rounded before they meet: each may be its neighbour, up to 2^-7 of it, which SiLU takes to at most 1.1 + |z| exp(-|z|) times as
-    # much of its value where |z| is small and to (1 + |z|) times below zero; the unit's result is rounded too.  Four such steps:
-    unit = dict(rtol=2 ** -5, atol=2 ** -7)
-    if N % 256 == 0:
-        for kind in (True, 8):
-            torch.testing.assert_close(ops.gemm_tile(x, wd, swiglu=kind, algo=1).float(), ops.gemm_tile(x, wd, swiglu=kind, algo=0).float(), **unit)
