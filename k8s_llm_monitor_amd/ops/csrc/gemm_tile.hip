@@ -83,7 +83,8 @@ constexpr bool tile_strips() {
 // workgroups that strips of up to this many tiles add
 static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * 32 - tiles; }
 
-template <int EPI, bool GROUPED, int SCH, bool RS = false>
+// NARROW: every workgroup a strip of 64 rows x 128 columns, for products of few tiles (narrow_strips).
+template <int EPI, bool GROUPED, int SCH, bool RS = false, bool NARROW = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                          int E, int M, int N, int K, long w_es, int n_mt, int n_nt,
@@ -92,10 +93,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   __shared__ __attribute__((aligned(16))) char smem[5 * HS];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = NARROW ? wave : wave >> 1, wn = NARROW ? 0 : wave & 1;
 
   // ---- logical tile: bijective XCD remap, then groups of 8 m-tiles ----
-  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>();
+  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>() && !NARROW;
   int mts = n_mt;
   if (GROUPED && STRIPS && strips) {  // the tiles that there are
     mts = 0;
@@ -116,11 +117,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int q8 = nwg >> 3, r8 = nwg & 7;
     lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
   }
+  constexpr int TM = NARROW ? 64 : 256, TN = NARROW ? 128 : 256;
   constexpr int GM = 8;
   const int grp = lid / (GM * n_nt), first_m = grp * GM;
   const int gsz = min(mts - first_m, GM);
   const int in_g = lid - grp * GM * n_nt;
-  const int mt = first_m + in_g % gsz, nt = in_g / gsz;
+  // NARROW: n_mt strips of rows by n_nt of columns, a column's strips on one XCD
+  const int mt = NARROW ? (bid >> 3) % n_mt : first_m + in_g % gsz, nt = NARROW ? (bid >> 3) / n_mt * 8 + xcd : in_g / gsz;
+  if (NARROW && nt >= n_nt) return;
 
   int row0, mrows;
   const bf16_t* Wt = W;
@@ -141,8 +145,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     if (e < 0) return;  // uniform: past the last expert's tiles
     Wt = W + (long)e * w_es;
   } else {
-    row0 = mt * 256;
-    mrows = min(256, M - row0);
+    row0 = mt * TM;
+    mrows = min(TM, M - row0);
   }
   if (STRIPS && strip >= 0) {
     row0 += 64 * strip;
@@ -153,8 +157,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   constexpr bool GLU = tile_epi_glu(EPI);
   const int n_unit = GLU ? (ep.f + 127) >> 7 : 0;
   const bool unit = GLU && nt < n_unit;
-  const int n0 = GLU ? (unit ? nt * 128 : 2 * ep.f + (nt - n_unit) * 256) : nt * 256;
-  const int nrows = unit ? 2 * min(128, ep.f - n0) : min(256, N - n0);
+  const int n0 = GLU ? (unit ? nt * 128 : 2 * ep.f + (nt - n_unit) * 256) : nt * TN;
+  const int nrows = unit ? 2 * min(128, ep.f - n0) : min(TN, N - n0);
 
   // ---- DMA of one half-tile (256 rows x 128 B = 32 pieces of 1 KiB): piece p (0..7) of this
   // wave covers rows (p * 4 + wave) * 8 .. + 7; lane -> row + (lane >> 3), physical chunk lane & 7 ----
@@ -234,55 +238,55 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   // chunk cc), issued during the last k-tile's second half so they land behind its MFMAs
   u32x4 resq[EPI == TILE_EPI_RESID ? 16 : 1];
 
-  if (STRIPS && strip >= 0) {
-    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  The same instructions in the same
-    // order of k as a whole tile's, so the same bits.
-    constexpr int SS = 8192 + HS;
-    auto fill = [&](int kt) {
-      char* dst = smem + (kt & 3) * SS + wave * 1024;
+  if (NARROW || (STRIPS && strip >= 0)) {
+    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  NARROW, 64 x 128: 16 x 128, six of 8 + 16.
+    // The same instructions in the same order of k as a whole tile's, so the same bits.
+    constexpr int RB = NARROW ? 1 : 2, BP = NARROW ? 4 : 8, SS = 8192 + BP * 4096, SLOTS = 5 * HS / SS;
+    auto next = [&](int slot) { return slot + SS == SLOTS * SS ? 0 : slot + SS; };
+    auto fill = [&](int kt, int slot) {
+      char* dst = smem + slot + wave * 1024;
       const int k = min(kt, nk - 1);
 #pragma unroll
       for (int p = 0; p < 2; ++p) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(dst + p * 4096), 16, soff[0][p], k * 128, 0, 0);
 #pragma unroll
-      for (int p = 0; p < 8; ++p)
+      for (int p = 0; p < BP; ++p)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(dst + 8192 + p * 4096), 16, soff[1][p], k * kstrB, 0, 0);
     };
-    auto read = [&](int t, int ks, bf16x8 (&a)[8], bf16x8 (&b)[8]) {
-      const char* at = smem + (t & 3) * SS;
+    auto read = [&](int slot, int ks, bf16x8 (&a)[8], bf16x8 (&b)[8]) {
+      const char* at = smem + slot;
 #pragma unroll
       for (int j = 0; j < 8; ++j) b[j] = *reinterpret_cast<const bf16x8*>(at + 8192 + (8 * wn + j) * 2048 + rdB[ks]);
 #pragma unroll
-      for (int g = 0; g < 2; ++g) a[g] = *reinterpret_cast<const bf16x8*>(at + (2 * wm + g) * 2048 + rd[ks]);
+      for (int g = 0; g < RB; ++g) a[g] = *reinterpret_cast<const bf16x8*>(at + (RB * wm + g) * 2048 + rd[ks]);
     };
     auto mul = [&](const bf16x8 (&a)[8], const bf16x8 (&b)[8]) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
+      for (int g = 0; g < RB; ++g)
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[g], acc[g][j], 0, 0, 0);
     };
-    fill(0);
-    fill(1);
-    fill(2);
-    fill(3);
-    vm_wait_n<30>();
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) fill(i, i * SS);
+    vm_wait_n<(SLOTS - 1) * (2 + BP)>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read(0, 0, fa0, fb0);
-    for (int t = 0; t < nk; ++t) {
-      read(t, 1, fa1, fb1);
+    for (int t = 0, at = 0; t < nk; ++t) {
+      read(at, 1, fa1, fb1);
       __builtin_amdgcn_sched_barrier(0);
       mul(fa0, fb0);
       lgkm_wait0();
-      vm_wait_n<20>();  // k-tile t + 1 is in; the two behind it are on their way
+      vm_wait_n<(SLOTS - 2) * (2 + BP)>();  // k-tile t + 1 is in; those behind it are on their way
       __builtin_amdgcn_s_barrier();  // everyone's pieces of it, and everyone has read k-tile t
       asm volatile("" ::: "memory");
-      read(t + 1, 0, fa0, fb0);
-      fill(t + 4);
+      read(next(at), 0, fa0, fb0);
+      fill(t + SLOTS, at);
       __builtin_amdgcn_sched_barrier(0);
       mul(fa1, fb1);
+      at = next(at);
     }
     vm_wait_n<0>();
-  } else if constexpr (SCH == 1) {
+  } else if constexpr (SCH == 1 && !NARROW) {
     // Ring addressing: the half-slot byte offsets of the current tile live in SGPRs and rotate
     // by one conditional subtract per tile, and each sub-step forms ONE A and ONE B fragment base
     // VGPR (every block read is that base + an immediate).
@@ -415,7 +419,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       }
       sub(P1{}, P3{}, fa1, fb1, fa0, fb0, S2, S3, S0, S1, t);
     }
-  } else {
+  } else if constexpr (!NARROW) {
     // One 32-deep sub-step: 64 MFMAs from (ca, cb), each carrying at most one other instruction in
     // its shadow.  The 8 DMA pieces of the sub-step ride MFMAs 4, 12, ..., 60 - evenly spread: an
     // LDS-DMA instruction holds its wave's issue for tens of cycles (MI355X_MICROARCH.md, LDS-DMA
@@ -595,8 +599,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       const int c = lane & 7, rsub = lane >> 3;
       bf16_t* ybase = Y + (long)row0 * N + n0 + wn * 128;
 #pragma unroll 4
-      for (int pass = 0; pass < 16; ++pass) {
-        const int r = pass * 8 + rsub, grow = wm * 128 + r;
+      for (int pass = 0; pass < 2 * RB; ++pass) {
+        const int r = pass * 8 + rsub, grow = wm * 16 * RB + r;
         if (grow >= mrows) continue;
         const uint4 a = *reinterpret_cast<const uint4*>(stage + r * RS_ + c * 16);
         const uint4 b = *reinterpret_cast<const uint4*>(stage + r * RS_ + (c + 8) * 16);
@@ -651,18 +655,33 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       finish(std::bool_constant<EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8>{}, blocks);
     }
   };
+  if constexpr (NARROW) {
+    end(std::integral_constant<int, 1>{});
+    return;
+  }
   if constexpr (STRIPS) {
     if (strip >= 0) {
       end(std::integral_constant<int, 2>{});
       return;
     }
   }
-  end(std::integral_constant<int, 8>{});
+  if constexpr (!NARROW) end(std::integral_constant<int, 8>{});
 }
 
 }  // namespace k8sllm
 
 using namespace k8sllm;
+
+// Whether a dense product's tiles are few enough that strips of 64 x 128 are faster: they are four to eight times as many, and a k-tile of one takes
+// about a third of a tile's (0.4 us; a tile's 1.25, 0.8 for the few that go as strips of 256 columns).  us, tiles / these, packed weights: 4096 x 4096,
+// 80 rows 56 / 35, 300 56 / 36, 600 (two rounds, left) 59; 4096 x 14336, 80 rows 168 / 98, 400 167 / 105; 6144 x 4096 with RoPE, 80 rows 78 / 36, 300
+// 81 / 39, 600 83 / 72; 28672 x 4096 with SwiGLU, 80 rows 90 / 74, 200 (left) 93; 1024 x 8192, any up to 1000 rows 100 / 60.
+static bool narrow_strips(long M, long N, long K, int epi) {
+  const long nk = K >> 6, tiles = (M + 255) / 256 * ((N + 255) / 256), strips = (M + 63) / 64 * ((N + 127) / 128);
+  if (tiles > kTileCus || N % 128 != 0) return false;
+  const float whole = nk * (tiles <= kStripTiles && epi != TILE_EPI_ROPE ? 0.8f : 1.25f);
+  return (strips + kTileCus - 1) / kTileCus * (nk * 0.4f + 6.f) < whole;
+}
 
 // Dense (offsets == nullptr): Y [M][N] (SwiGLU: [M][N / 2]) = X [M][K] . W[N][K]^T.
 // Grouped: W [E][N][K] with expert stride w_es elements; M = total expert-sorted rows (the grid
@@ -705,6 +724,18 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   const int n_mt = (M + 255) / 256 + (grouped ? E : 0), n_nt = (N + 255) / 256;
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
+  if (!grouped && algo == 1 && !rs && epi != TILE_EPI_RESID && narrow_strips(M, N, K, epi)) {
+    const int rows = (M + 63) / 64, cols = N / 128;
+#define K8_TILE_NARROW(EPI_)                                                                                               \
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false, true>), dim3((unsigned)((cols + 7) / 8 * 8 * rows)), dim3(256), 0, s, \
+                     (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, rows, cols, ep, wpk, 0)
+    if (epi == TILE_EPI_SWIGLU) K8_TILE_NARROW(TILE_EPI_SWIGLU);
+    else if (epi == TILE_EPI_SWIGLU8) K8_TILE_NARROW(TILE_EPI_SWIGLU8);
+    else if (epi == TILE_EPI_ROPE) K8_TILE_NARROW(TILE_EPI_ROPE);
+    else K8_TILE_NARROW(TILE_EPI_BF16);
+#undef K8_TILE_NARROW
+    return (int)hipGetLastError();
+  }
   const bool cut = algo == 1 && !rs && epi != TILE_EPI_ROPE && epi != TILE_EPI_RESID && E <= kStripExperts;
   const long over = nwg % kTileCus;
   const int strips = cut && (grouped || (over > 0 && over <= kStripTiles));
