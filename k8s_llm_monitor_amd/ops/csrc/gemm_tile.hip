@@ -83,8 +83,8 @@ constexpr bool tile_strips() {
 // workgroups that strips of up to this many tiles add
 static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * 32 - tiles; }
 
-// NARROW: every workgroup a strip of 64 rows x 128 columns, for products of few tiles (narrow_strips).
-template <int EPI, bool GROUPED, int SCH, bool RS = false, bool NARROW = false>
+// NARROW: every workgroup a strip of 64 rows x 128 (or 64) columns, for products of few tiles (narrow_strips).
+template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                          int E, int M, int N, int K, long w_es, int n_mt, int n_nt,
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int q8 = nwg >> 3, r8 = nwg & 7;
     lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
   }
-  constexpr int TM = NARROW ? 64 : 256, TN = NARROW ? 128 : 256;
+  constexpr int TM = NARROW ? 64 : 256, TN = NARROW ? NARROW : 256;
   constexpr int GM = 8;
   const int grp = lid / (GM * n_nt), first_m = grp * GM;
   const int gsz = min(mts - first_m, GM);
@@ -239,9 +239,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   u32x4 resq[EPI == TILE_EPI_RESID ? 16 : 1];
 
   if (NARROW || (STRIPS && strip >= 0)) {
-    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  NARROW, 64 x 128: 16 x 128, six of 8 + 16.
+    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  NARROW, 64 x 128 (64): 16 x 128 (64), six (ten) of 8 + 16 (8).
     // The same instructions in the same order of k as a whole tile's, so the same bits.
-    constexpr int RB = NARROW ? 1 : 2, BP = NARROW ? 4 : 8, SS = 8192 + BP * 4096, SLOTS = 5 * HS / SS;
+    constexpr int RB = NARROW ? 1 : 2, BP = NARROW ? NARROW / 32 : 8, NJ = NARROW ? NARROW / 16 : 8, SS = 8192 + BP * 4096, SLOTS = 5 * HS / SS;
     auto next = [&](int slot) { return slot + SS == SLOTS * SS ? 0 : slot + SS; };
     auto fill = [&](int kt, int slot) {
       char* dst = smem + slot + wave * 1024;
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     auto read = [&](int slot, int ks, bf16x8 (&a)[8], bf16x8 (&b)[8]) {
       const char* at = smem + slot;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) b[j] = *reinterpret_cast<const bf16x8*>(at + 8192 + (8 * wn + j) * 2048 + rdB[ks]);
+      for (int j = 0; j < NJ; ++j) b[j] = *reinterpret_cast<const bf16x8*>(at + 8192 + (8 * wn + j) * 2048 + rdB[ks]);
 #pragma unroll
       for (int g = 0; g < RB; ++g) a[g] = *reinterpret_cast<const bf16x8*>(at + (RB * wm + g) * 2048 + rd[ks]);
     };
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 #pragma unroll
       for (int g = 0; g < RB; ++g)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[g], acc[g][j], 0, 0, 0);
+        for (int j = 0; j < NJ; ++j) acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[g], acc[g][j], 0, 0, 0);
     };
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) fill(i, i * SS);
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   auto finish = [&](auto gated, auto blocks) {  // gated: a unit's tile; blocks: of 16 rows, a wave's
   constexpr bool SWG = decltype(gated)::value;
   constexpr int RB = decltype(blocks)::value;
-  constexpr int OUTW = SWG ? 64 : 128;  // output columns of this wave's quarter
+  constexpr int OUTW = SWG || NARROW == 64 ? 64 : 128;  // output columns of this wave's quarter
   constexpr int RS_ = OUTW * 2 + 16;                       // LDS row stride (16-B pad: 2-way writes)
   char* stage = smem + wave * (16 * RB * RS_);
   const int ml = lane & 15, nq = 4 * (lane >> 4);
@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < OUTW / 16; ++j) {
         f32x4 v = acc[i][j] * sc[i];
         if constexpr (EPI == TILE_EPI_RELU_SQ) {
 #pragma unroll
@@ -672,15 +672,16 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 
 using namespace k8sllm;
 
-// Whether a dense product's tiles are few enough that strips of 64 x 128 are faster: they are four to eight times as many, and a k-tile of one takes
-// about a third of a tile's (0.4 us; a tile's 1.25, 0.8 for the few that go as strips of 256 columns).  us, tiles / these, packed weights: 4096 x 4096,
-// 80 rows 56 / 35, 300 56 / 36, 600 (two rounds, left) 59; 4096 x 14336, 80 rows 168 / 98, 400 167 / 105; 6144 x 4096 with RoPE, 80 rows 78 / 36, 300
-// 81 / 39, 600 83 / 72; 28672 x 4096 with SwiGLU, 80 rows 90 / 74, 200 (left) 93; 1024 x 8192, any up to 1000 rows 100 / 60.
-static bool narrow_strips(long M, long N, long K, int epi) {
-  const long nk = K >> 6, tiles = (M + 255) / 256 * ((N + 255) / 256), strips = (M + 63) / 64 * ((N + 127) / 128);
-  if (tiles > kTileCus || N % 128 != 0) return false;
+// The columns of the strips of 64 rows that a dense product of few tiles goes in, 0: tiles.  A strip of 128 columns takes 0.4 us a k-tile, one of 64 (plain
+// products, where they are one round) 0.25; a tile takes 1.25, 0.8 where few go as strips of 256 columns.  us, tiles / 128 / 64 columns, packed weights:
+// 4096 x 4096, 80 rows 56 / 35 / 23, 300 56 / 36 (320 of 64 would be two rounds), 600 59 (left); 4096 x 14336, 80 rows 168 / 98 / 58, 400 167 / 105; 1024 x
+// 8192, 300 rows 100 / 59 / 35; 6144 x 4096 with RoPE, 80 rows 78 / 36, 300 81 / 38, 600 83 / 71; 28672 x 4096 with SwiGLU, 80 rows 90 / 73, 200 (left) 90.
+static int narrow_strips(long M, long N, long K, int epi) {
+  const long nk = K >> 6, rows = (M + 63) / 64, tiles = (M + 255) / 256 * ((N + 255) / 256);
+  if (tiles > kTileCus) return 0;
   const float whole = nk * (tiles <= kStripTiles && epi != TILE_EPI_ROPE ? 0.8f : 1.25f);
-  return (strips + kTileCus - 1) / kTileCus * (nk * 0.4f + 6.f) < whole;
+  if (epi == TILE_EPI_BF16 && N % 64 == 0 && rows * (N / 64) <= kTileCus && nk * 0.3f + 6.f < whole) return 64;
+  return N % 128 == 0 && (rows * (N / 128) + kTileCus - 1) / kTileCus * (nk * 0.4f + 6.f) < whole ? 128 : 0;
 }
 
 // Dense (offsets == nullptr): Y [M][N] (SwiGLU: [M][N / 2]) = X [M][K] . W[N][K]^T.
@@ -724,15 +725,17 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   const int n_mt = (M + 255) / 256 + (grouped ? E : 0), n_nt = (N + 255) / 256;
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
-  if (!grouped && algo == 1 && !rs && epi != TILE_EPI_RESID && narrow_strips(M, N, K, epi)) {
-    const int rows = (M + 63) / 64, cols = N / 128;
-#define K8_TILE_NARROW(EPI_)                                                                                               \
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false, true>), dim3((unsigned)((cols + 7) / 8 * 8 * rows)), dim3(256), 0, s, \
+  const int narrow = !grouped && algo == 1 && !rs && epi != TILE_EPI_RESID ? narrow_strips(M, N, K, epi) : 0;
+  if (narrow) {
+    const int rows = (M + 63) / 64, cols = N / narrow;
+#define K8_TILE_NARROW(EPI_, C)                                                                                               \
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false, C>), dim3((unsigned)((cols + 7) / 8 * 8 * rows)), dim3(256), 0, s, \
                      (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, rows, cols, ep, wpk, 0)
-    if (epi == TILE_EPI_SWIGLU) K8_TILE_NARROW(TILE_EPI_SWIGLU);
-    else if (epi == TILE_EPI_SWIGLU8) K8_TILE_NARROW(TILE_EPI_SWIGLU8);
-    else if (epi == TILE_EPI_ROPE) K8_TILE_NARROW(TILE_EPI_ROPE);
-    else K8_TILE_NARROW(TILE_EPI_BF16);
+    if (epi == TILE_EPI_SWIGLU) K8_TILE_NARROW(TILE_EPI_SWIGLU, 128);
+    else if (epi == TILE_EPI_SWIGLU8) K8_TILE_NARROW(TILE_EPI_SWIGLU8, 128);
+    else if (epi == TILE_EPI_ROPE) K8_TILE_NARROW(TILE_EPI_ROPE, 128);
+    else if (narrow == 64) K8_TILE_NARROW(TILE_EPI_BF16, 64);
+    else K8_TILE_NARROW(TILE_EPI_BF16, 128);
 #undef K8_TILE_NARROW
     return (int)hipGetLastError();
   }
