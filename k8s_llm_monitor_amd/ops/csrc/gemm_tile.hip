@@ -83,8 +83,8 @@ constexpr bool tile_strips() {
 // workgroups that strips of up to this many tiles add
 static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * 32 - tiles; }
 
-// NARROW: every workgroup a strip of 64 rows x 128 (or 64) columns, for products of few tiles (narrow_strips).
-template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0>
+// NARROW: every workgroup a strip of 64 (or 128, TALL) rows x 128 (or 64) columns, for products of few tiles (narrow_strips).
+template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0, bool TALL = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                          int E, int M, int N, int K, long w_es, int n_mt, int n_nt,
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int q8 = nwg >> 3, r8 = nwg & 7;
     lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
   }
-  constexpr int TM = NARROW ? 64 : 256, TN = NARROW ? NARROW : 256;
+  constexpr int TM = !NARROW ? 256 : TALL ? 128 : 64, TN = NARROW ? NARROW : 256;
   constexpr int GM = 8;
   const int grp = lid / (GM * n_nt), first_m = grp * GM;
   const int gsz = min(mts - first_m, GM);
@@ -239,23 +239,25 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   u32x4 resq[EPI == TILE_EPI_RESID ? 16 : 1];
 
   if (NARROW || (STRIPS && strip >= 0)) {
-    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  NARROW, 64 x 128 (64): 16 x 128 (64), six (ten) of 8 + 16 (8).
+    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  NARROW, 64 x 128 (64): 16 x 128 (64), six (ten) of 8 + 16 (8); 128 x 128:
+    // 32 x 128, five of 16 + 16.
     // The same instructions in the same order of k as a whole tile's, so the same bits.
-    constexpr int RB = NARROW ? 1 : 2, BP = NARROW ? NARROW / 32 : 8, NJ = NARROW ? NARROW / 16 : 8, SS = 8192 + BP * 4096, SLOTS = 5 * HS / SS;
+    constexpr int RB = NARROW && !TALL ? 1 : 2, AP = TALL ? 4 : 2, BP = NARROW ? NARROW / 32 : 8, NJ = NARROW ? NARROW / 16 : 8;
+    constexpr int SA = AP * 4096, SS = SA + BP * 4096, SLOTS = 5 * HS / SS;
     auto next = [&](int slot) { return slot + SS == SLOTS * SS ? 0 : slot + SS; };
     auto fill = [&](int kt, int slot) {
       char* dst = smem + slot + wave * 1024;
       const int k = min(kt, nk - 1);
 #pragma unroll
-      for (int p = 0; p < 2; ++p) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(dst + p * 4096), 16, soff[0][p], k * 128, 0, 0);
+      for (int p = 0; p < AP; ++p) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(dst + p * 4096), 16, soff[0][p], k * 128, 0, 0);
 #pragma unroll
       for (int p = 0; p < BP; ++p)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(dst + 8192 + p * 4096), 16, soff[1][p], k * kstrB, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(dst + SA + p * 4096), 16, soff[1][p], k * kstrB, 0, 0);
     };
     auto read = [&](int slot, int ks, bf16x8 (&a)[8], bf16x8 (&b)[8]) {
       const char* at = smem + slot;
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) b[j] = *reinterpret_cast<const bf16x8*>(at + 8192 + (8 * wn + j) * 2048 + rdB[ks]);
+      for (int j = 0; j < NJ; ++j) b[j] = *reinterpret_cast<const bf16x8*>(at + SA + (8 * wn + j) * 2048 + rdB[ks]);
 #pragma unroll
       for (int g = 0; g < RB; ++g) a[g] = *reinterpret_cast<const bf16x8*>(at + (RB * wm + g) * 2048 + rd[ks]);
     };
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     };
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) fill(i, i * SS);
-    vm_wait_n<(SLOTS - 1) * (2 + BP)>();
+    vm_wait_n<(SLOTS - 1) * (AP + BP)>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read(0, 0, fa0, fb0);
@@ -276,7 +278,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       __builtin_amdgcn_sched_barrier(0);
       mul(fa0, fb0);
       lgkm_wait0();
-      vm_wait_n<(SLOTS - 2) * (2 + BP)>();  // k-tile t + 1 is in; those behind it are on their way
+      vm_wait_n<(SLOTS - 2) * (AP + BP)>();  // k-tile t + 1 is in; those behind it are on their way
       __builtin_amdgcn_s_barrier();  // everyone's pieces of it, and everyone has read k-tile t
       asm volatile("" ::: "memory");
       read(next(at), 0, fa0, fb0);
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     }
   };
   if constexpr (NARROW) {
-    end(std::integral_constant<int, 1>{});
+    end(std::integral_constant<int, TALL ? 2 : 1>{});
     return;
   }
   if constexpr (STRIPS) {
@@ -672,16 +674,29 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 
 using namespace k8sllm;
 
-// The columns of the strips of 64 rows that a dense product of few tiles goes in, 0: tiles.  A strip of 128 columns takes 0.4 us a k-tile, one of 64 (plain
-// products, where they are one round) 0.25; a tile takes 1.25, 0.8 where few go as strips of 256 columns.  us, tiles / 128 / 64 columns, packed weights:
-// 4096 x 4096, 80 rows 56 / 35 / 23, 300 56 / 36 (320 of 64 would be two rounds), 600 59 (left); 4096 x 14336, 80 rows 168 / 98 / 58, 400 167 / 105; 1024 x
-// 8192, 300 rows 100 / 59 / 35; 6144 x 4096 with RoPE, 80 rows 78 / 36, 300 81 / 38, 600 83 / 71; 28672 x 4096 with SwiGLU, 80 rows 90 / 73, 200 (left) 90.
-static int narrow_strips(long M, long N, long K, int epi) {
-  const long nk = K >> 6, rows = (M + 63) / 64, tiles = (M + 255) / 256 * ((N + 255) / 256);
-  if (tiles > kTileCus) return 0;
-  const float whole = nk * (tiles <= kStripTiles && epi != TILE_EPI_ROPE ? 0.8f : 1.25f);
-  if (epi == TILE_EPI_BF16 && N % 64 == 0 && rows * (N / 64) <= kTileCus && nk * 0.3f + 6.f < whole) return 64;
-  return N % 128 == 0 && (rows * (N / 128) + kTileCus - 1) / kTileCus * (nk * 0.4f + 6.f) < whole ? 128 : 0;
+// The strips that a dense product of few tiles goes in: the least of rounds x (k-tiles x rate + 6 us for its start and end).  Rates, us a k-tile with the
+// chip full: 64 x 64 0.26 (plain products), 64 x 128 0.42, 128 x 128 0.72; a tile 1.25, 0.8 where few go as strips of 256 columns.  us, tiles / 128 x 128 /
+// 64 x 128 / 64 x 64, packed weights: 4096 x 4096, 80 rows 56 / - / 35 / 23, 300 56 / - / 35, 600 59 / 54; 4096 x 14336, 80 rows 168 / - / 98 / 58, 400 167 /
+// - / 104, 600 178 / 161; 6144 x 4096 with RoPE, 80 rows 78 / - / 36, 300 81 / - / 38, 400 - / 57 / 67, 600 83 / 58 / 71, 800 84 / 102 (two rounds); 28672 x
+// 4096 with SwiGLU, 80 rows 90 / 62 / 75 (two rounds), 200 90 / 107 (two rounds).
+struct Strips {
+  int rows = 0, cols = 0;  // 0: tiles
+};
+static Strips narrow_strips(long M, long N, long K, int epi) {
+  const long nk = K >> 6, tiles = (M + 255) / 256 * ((N + 255) / 256);
+  Strips best;
+  if (tiles > kTileCus) return best;
+  float us = nk * (tiles <= kStripTiles && epi != TILE_EPI_ROPE ? 0.8f : 1.25f) + 6.f;
+  auto take = [&](int rows, int cols, float ktile) {
+    if (N % cols) return;
+    const long n = (M + rows - 1) / rows * (N / cols);
+    const float t = (n + kTileCus - 1) / kTileCus * (nk * ktile + 6.f);
+    if (t < us) us = t, best = Strips{rows, cols};
+  };
+  if (epi == TILE_EPI_BF16) take(64, 64, 0.26f);
+  take(64, 128, 0.42f);
+  take(128, 128, 0.72f);
+  return best;
 }
 
 // Dense (offsets == nullptr): Y [M][N] (SwiGLU: [M][N / 2]) = X [M][K] . W[N][K]^T.
@@ -725,17 +740,21 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   const int n_mt = (M + 255) / 256 + (grouped ? E : 0), n_nt = (N + 255) / 256;
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
-  const int narrow = !grouped && algo == 1 && !rs && epi != TILE_EPI_RESID ? narrow_strips(M, N, K, epi) : 0;
-  if (narrow) {
-    const int rows = (M + 63) / 64, cols = N / narrow;
-#define K8_TILE_NARROW(EPI_, C)                                                                                               \
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false, C>), dim3((unsigned)((cols + 7) / 8 * 8 * rows)), dim3(256), 0, s, \
+  const Strips narrow = !grouped && algo == 1 && !rs && epi != TILE_EPI_RESID ? narrow_strips(M, N, K, epi) : Strips{};
+  if (narrow.rows) {
+    const int rows = (M + narrow.rows - 1) / narrow.rows, cols = N / narrow.cols;
+#define K8_TILE_NARROW(EPI_, C, T)                                                                                               \
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false, C, T>), dim3((unsigned)((cols + 7) / 8 * 8 * rows)), dim3(256), 0, s, \
                      (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, rows, cols, ep, wpk, 0)
-    if (epi == TILE_EPI_SWIGLU) K8_TILE_NARROW(TILE_EPI_SWIGLU, 128);
-    else if (epi == TILE_EPI_SWIGLU8) K8_TILE_NARROW(TILE_EPI_SWIGLU8, 128);
-    else if (epi == TILE_EPI_ROPE) K8_TILE_NARROW(TILE_EPI_ROPE, 128);
-    else if (narrow == 64) K8_TILE_NARROW(TILE_EPI_BF16, 64);
-    else K8_TILE_NARROW(TILE_EPI_BF16, 128);
+#define K8_TILE_NARROW_T(T)                                                    \
+  if (epi == TILE_EPI_SWIGLU) K8_TILE_NARROW(TILE_EPI_SWIGLU, 128, T);         \
+  else if (epi == TILE_EPI_SWIGLU8) K8_TILE_NARROW(TILE_EPI_SWIGLU8, 128, T);  \
+  else if (epi == TILE_EPI_ROPE) K8_TILE_NARROW(TILE_EPI_ROPE, 128, T);        \
+  else K8_TILE_NARROW(TILE_EPI_BF16, 128, T)
+    if (narrow.cols == 64) K8_TILE_NARROW(TILE_EPI_BF16, 64, false);
+    else if (narrow.rows == 128) { K8_TILE_NARROW_T(true); }
+    else { K8_TILE_NARROW_T(false); }
+#undef K8_TILE_NARROW_T
 #undef K8_TILE_NARROW
     return (int)hipGetLastError();
   }
