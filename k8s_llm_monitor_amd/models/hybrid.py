@@ -112,13 +112,14 @@ class _Params:
 
 
 def _take(rows, *ts: torch.Tensor) -> tuple:
-    """These rows (a tensor of them or a slice) of each; None: all.  Rows of 16-bit projections stay a multiple of 16 bytes apart, as the
-    kernels' accesses want them."""
+    """These rows (a tensor of them or a slice) of each; None: all.  Rows of a whole tensor come contiguous, as the norms' kernels want
+    residuals and fp32 results; those of columns of wider rows stay a multiple of 8 values apart, as wide accesses want projections."""
     def some(t: torch.Tensor) -> torch.Tensor:
         if isinstance(rows, slice):
             return t[rows]
         r = t.index_select(0, rows)
-        return F.pad(r, (0, -r.shape[1] % 8))[:, :r.shape[1]] if r.dim() == 2 and r.shape[1] % 8 else r
+        n = r.shape[-1]
+        return F.pad(r, (0, -n % 8))[:, :n] if n % 8 and r.dim() == 2 and not t.is_contiguous() else r
 
     return ts if rows is None else tuple(some(t) for t in ts)
 

@@ -9,6 +9,7 @@ from k8s_llm_monitor_amd.engine.block_manager import BlockManager
 from k8s_llm_monitor_amd.engine.runner import ModelRunner, RunnerConfig
 from k8s_llm_monitor_amd.engine.sequence import SamplingParams, Sequence
 from k8s_llm_monitor_amd.models import HybridLM, build_model, get_config
+from k8s_llm_monitor_amd.models.hybrid import _take
 
 PRESETS = ["dunesun-tiny", "kisutar-tiny", "bitonex-tiny", "levovik-tiny", "dopivik-tiny", "zifisun-tiny"]
 
@@ -73,10 +74,37 @@ def _compare(model, tol):
             torch.testing.assert_close(x, y, rtol=0, atol=0)
 
 
-def _models(name, device, dtype):
-    cfg = get_config(name)
+def _models(name, device, dtype, make=get_config):
+    cfg = make(name)
     for k in range(1, len(cfg.layers) + 1):  # every layer as the last one
         yield HybridLM(dataclasses.replace(cfg, name=f"{name}-{k}", layers=cfg.layers[:k], loop=None), device=device, dtype=dtype, seed=3)
+
+
+def _odd(name):
+    """The preset with a width and mixer results that are not a multiple of 8 columns."""
+    cfg, new = get_config(name), []
+    for s in cfg.layers:
+        m = dict(s.mixer)
+        for k in ("vdim", "right.vdim"):
+            if k in m and s.kind != "latent_attention":
+                m[k] = m[k] // 2 | 1
+        if s.kind == "wkv":
+            m["dim"] = 14
+        new.append(dataclasses.replace(s, mixer=tuple(sorted(m.items()))))
+    return dataclasses.replace(cfg, d_model=cfg.d_model + 12, layers=tuple(new))
+
+
+def test_take_keeps_whole_rows():
+    """Rows of whole tensors come whole, whatever their width: the kernels want residuals, normed rows and fp32 results contiguous.  Columns of
+    wider rows stay a multiple of 8 values apart."""
+    idx = torch.tensor([2, 5])
+    for x in (torch.randn(7, 100), torch.randn(7, 45), torch.randn(7, 90).bfloat16(), torch.randn(7, 3, 10)):
+        (y,) = _take(idx, x)
+        assert y.is_contiguous() and torch.equal(y, x[idx])
+    wide = torch.randn(7, 64)
+    for a, b in ((0, 20), (8, 45), (16, 32)):
+        (y,) = _take(idx, wide[:, a:b])
+        assert torch.equal(y, wide[idx, a:b]) and y.stride() == (-(a - b) + (a - b) % 8, 1)
 
 
 @pytest.mark.parametrize("name", PRESETS)
@@ -95,6 +123,13 @@ def test_last_layer_on_wanted_rows_llama():
 def test_gpu_last_layer_on_wanted_rows(name, dtype, tol):
     for m in _models(name, "cuda:0", dtype):
         _compare(m, tol)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["dunesun-tiny", "bitonex-tiny", "levovik-tiny", "dopivik-tiny"])
+def test_gpu_last_layer_on_wanted_rows_odd_widths(name):
+    for m in _models(name, "cuda:0", torch.float32, _odd):
+        _compare(m, 1e-4)
 
 
 @pytest.mark.gpu
