@@ -968,7 +968,7 @@ int k8sllm_hy_add_norm(void* out, float* residual, const void* a0, int t0, const
                        const int* positions, const void* emb, const void* pos, const int* src, const int* prev, int vocab, int max_pos,
                        float scale, int* r_ids, float* r_wts, float* r_gate, const float* wr, const float* bias, int rE, int rK, int rows_w,
                        int over_all, int f32, hipStream_t s) {
-  if (rows <= 0) return 0;
+  if (rows <= 0 || d <= 0) return 0;  // (of width 0 there is nothing to write, and a lane behind the last column reads the last eight)
   const bool join = t0 == 3 || t1 == 3 || t2 == 3;
   if ((join || emb != nullptr || r_ids != nullptr) && d % 8 != 0) return -1;
   if (emb != nullptr && (t0 || t1 || t2)) return -1;

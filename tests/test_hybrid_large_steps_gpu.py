@@ -1393,3 +1393,14 @@ def test_embedding_with_the_norm(T, d, E, pos, prev, shift, dt):
         gh, r = gh
         assert all(torch.equal(a, b) for a, b in zip(r, hops.moe_router(h, *route)))
     assert torch.equal(gx, x) and torch.equal(gh, h)
+
+
+@pytest.mark.parametrize("T", [1, 3, 300])
+def test_add_norm_of_width_0(T):
+    """Nothing is read or written."""
+    x, w = torch.empty(T, 0, device="cuda"), torch.empty(0, device="cuda")
+    for dt in (BF, torch.float32):
+        assert hops.add_norm(x, (), w, w, 1e-5, True, dt).shape == (T, 0)
+        x2, h = hops.embed_norm(_i32([0] * T).cuda(), _i32([0] * T).cuda(), torch.empty(4, 0, dtype=dt, device="cuda"), None, None, None, 1.0, None,
+                                w, 1e-5, True)
+        assert x2.shape == h.shape == (T, 0)
