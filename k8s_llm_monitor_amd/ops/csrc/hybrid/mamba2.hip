@@ -861,8 +861,8 @@ static int launch_scan(float* y, const void* xbc, const void* proj, long p_strid
     return (int)hipGetLastError();
   }
   const dim3 grid((unsigned)S, (unsigned)nh, (unsigned)((P + 63) / 64));
-  // one token a segment, rows that the step kernel can read four values at a time
-  if (step && P % 4 == 0 && N % 4 == 0 && N <= 256 && reinterpret_cast<uintptr_t>(state) % 16 == 0 &&
+  // one token a segment, rows that the step kernel can read four values at a time (some: groups behind the last repeat it)
+  if (step && P % 4 == 0 && N % 4 == 0 && N > 0 && N <= 256 && reinterpret_cast<uintptr_t>(state) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(xbc) % (4 * sizeof(T)) == 0) {
     const bool once = 4l * S * nh * N * P > kStateOnceBytes;
 #define K8SLLM_STEP(NPT)                                                                                                 \

@@ -1404,3 +1404,20 @@ def test_add_norm_of_width_0(T):
         x2, h = hops.embed_norm(_i32([0] * T).cuda(), _i32([0] * T).cuda(), torch.empty(4, 0, dtype=dt, device="cuda"), None, None, None, 1.0, None,
                                 w, 1e-5, True)
         assert x2.shape == h.shape == (T, 0)
+
+
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+@pytest.mark.parametrize("fixed", [False, True])
+def test_one_token_a_segment_without_states(fixed, dt):
+    """A recurrence of no states is its skip term (with a fixed decay: zero)."""
+    g = _g(97)
+    n, nh, P = 5, 2, 64
+    x, z = _r(g, n, nh * P, dt=dt), _r(g, n, nh, dt=dt)
+    dtb, al, dk = (_r(g, nh) for _ in range(3))
+    seg = (_i32(list(range(n + 1))), _i32([3] * n), _i32([0, 1, -1, 2, 3]))
+    a = (x, None if fixed else z, 0, *((None,) * 3 if fixed else (dtb, al, dk)), torch.zeros(4, nh, 0, P), *seg)
+    d = torch.rand(nh, generator=g).cuda() if fixed else None
+    got = hops.ssm_scan(*(t.cuda() if isinstance(t, torch.Tensor) else t for t in a), nh, P, 0, 1, decay=d)
+    want = x.float().view(n, nh, P) * (0.0 if fixed else dk[:, None])
+    want[2] = 0.0  # a padding row
+    torch.testing.assert_close(got.cpu(), want.view(n, nh * P), rtol=1e-6, atol=0)  # one product
