@@ -210,11 +210,16 @@ class ModelRunner:
             first = [max(0, c - w + 1) // BLOCK_SIZE if w else 0 for c in starts]
             n = [(c + n + BLOCK_SIZE - 1) // BLOCK_SIZE - a for c, n, a in zip(starts, lens, first)]
             seen[w] = first, n, list(accumulate(n))
-        sizes = dict(ids=T, pos=T, slots=T, cu=len(seqs) + 1, qs=nq, st=nq, lidx=nl, temp=R, topk=R, topp=R,
-                     gcu=hy + 1 if hy else 0, gctx=hy, gslot=hy,
-                     cst=len(seqs) if paged else 0, cend=len(seqs) if hy else 0, bt=len(seqs) * W, dbt=nd * Wd, dlen=nd,
-                     mcu=len(seqs) + 2 if kA else 0, mqs=nq if kA else 0, mst=nq if kA else 0,
-                     mlidx=len(seqs) if kA else 0)
+        # (only what this step has: every entry costs the host a slice of each copy)
+        sizes = dict(ids=T, pos=T, slots=T, cu=len(seqs) + 1, qs=nq, st=nq, lidx=nl, temp=R, topk=R, topp=R)
+        if hy:
+            sizes.update(gcu=hy + 1, gctx=hy, gslot=hy, cend=len(seqs))
+        if paged:
+            sizes.update(cst=len(seqs), bt=len(seqs) * W)
+        if nd:
+            sizes.update(dbt=nd * Wd, dlen=nd)
+        if kA:
+            sizes.update(mcu=len(seqs) + 2, mqs=nq, mst=nq, mlidx=len(seqs))
         for w, (_, _, ends) in seen.items():
             sizes[f"pgl{w}"], sizes[f"pgb{w}"] = ends[-1], len(seqs) * W
         off, o = {}, 0
@@ -254,7 +259,7 @@ class ModelRunner:
             v["gctx"][:nd] = [q.num_tokens - 1 for q in decode]
             v["gctx"][nd:] = starts
             v["gslot"][:] = [getattr(q, "state_slot", -1) for q in rows]
-            v["cend"][:] = np.asarray(starts, dtype=np.int32) + np.asarray(lens, dtype=np.int32)
+            v["cend"][:] = [c + n for c, n in zip(starts, lens)]
         v["temp"].view(np.float32)[:] = [s.params.temperature for s in rows]
         v["topk"][:] = [s.params.top_k for s in rows]
         v["topp"].view(np.float32)[:] = [s.params.top_p for s in rows]

@@ -114,6 +114,9 @@ class _Params:
 def _take(rows, *ts: torch.Tensor) -> tuple:
     """These rows (a tensor of them or a slice) of each; None: all.  Rows of a whole tensor come contiguous, as the norms' kernels want
     residuals and fp32 results; those of columns of wider rows stay a multiple of 8 values apart, as wide accesses want projections."""
+    if rows is None:
+        return ts
+
     def some(t: torch.Tensor) -> torch.Tensor:
         if isinstance(rows, slice):
             return t[rows]
@@ -121,7 +124,7 @@ def _take(rows, *ts: torch.Tensor) -> tuple:
         n = r.shape[-1]
         return F.pad(r, (0, -n % 8))[:, :n] if n % 8 and r.dim() == 2 and not t.is_contiguous() else r
 
-    return ts if rows is None else tuple(some(t) for t in ts)
+    return tuple(some(t) for t in ts)
 
 
 def _attend_ends(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, meta: AttnMeta, *args, gate: Optional[torch.Tensor] = None,
@@ -179,18 +182,19 @@ class WindowAttention:
         elif rows is not None and meta.ends is not None:
             o = _attend_ends(*_take(rows, qkv), kc, vc, meta, *args, vec=bool(self.fast))
         else:
-            nd = meta.num_decode
+            nd, q, o, po = meta.num_decode, qkv, None, None
+            if nd:  # a mixed step: the single decode tokens in front go through the decode kernel
+                o = torch.empty(qkv.shape[0], H * dv, dtype=qkv.dtype, device=qkv.device)
+                q, po = qkv[nd:], o[nd:]
             # mfma 2: the register kernel.  The staged one (201 -> 88 us at 4 x 2048 rows, 16 heads) rounds the weights against
             # another running maximum, and this design's routers - the softmax over the two best of near-equal logits - turn such
             # differences into other experts: recurrent states behind them moved by more than their root mean square.
-            o = torch.empty(qkv.shape[0], H * dv, dtype=qkv.dtype, device=qkv.device)
-            q, po = (qkv[nd:], o[nd:]) if nd else (qkv, o)
-            hops.window_attention_prefill(q, kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
-                                          *args, mfma=2 if self.fast == 1 else self.fast, out=po)
-            if nd:  # a mixed step: the single decode tokens in front go through the decode kernel
+            po = hops.window_attention_prefill(q, kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
+                                               *args, mfma=2 if self.fast == 1 else self.fast, out=po)
+            if nd:
                 hops.window_attention_decode(qkv[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
                                              vec=bool(self.fast), out=o[:nd])
-            (o,) = _take(rows, o)
+            (o,) = _take(rows, o if nd else po)
         return F.linear(o, self.wo)
 
 
@@ -358,12 +362,14 @@ class LatentAttention:
         nd = meta.num_decode if meta.is_prefill else T  # single-token rows in front
         o = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
         if nd or not ex:
-            n = nd if ex else T
-            # (first row, end, pages, whose positions they see) of attention over the latent pages
-            runs = [(0, T, meta.block_tables, dict(seq_lens=meta.seq_lens))] if not meta.is_prefill else [
-                (0, nd, meta.dec_block_tables, dict(seq_lens=meta.dec_seq_lens)),
-                (nd, n, meta.block_tables, dict(seq_lens=meta.ends) if ends else dict(cu=meta.cu_seqlens, ctx=meta.ctx_start))]
-            self._forward_latent(q[:n], pos, kc, vc, gate, [r for r in runs if r[1] > r[0]], o[:n])
+            # (end, pages, whose positions they see) of the runs of rows that attend over the latent pages
+            runs = []
+            if nd:
+                runs.append((nd, meta.dec_block_tables, dict(seq_lens=meta.dec_seq_lens)) if meta.is_prefill else
+                            (T, meta.block_tables, dict(seq_lens=meta.seq_lens)))
+            if nd < T and not ex:
+                runs.append((T, meta.block_tables, dict(seq_lens=meta.ends) if ends else dict(cu=meta.cu_seqlens, ctx=meta.ctx_start)))
+            self._forward_latent(*((q[:nd], pos, kc, vc, gate, runs, o[:nd]) if ex else (q, pos, kc, vc, gate, runs, o)))
         if ex:
             self._forward_expanded(*((t if t is None or not nd else t[nd:]) for t in (q, gate, o)), meta, kc)
         if rows is not None and not ends:
@@ -374,13 +380,20 @@ class LatentAttention:
 
     def _forward_latent(self, q: torch.Tensor, pos: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, gate: Optional[torch.Tensor],
                         runs: list, out: torch.Tensor) -> None:
-        """Attention over the latent pages: rows ``q``, in ``runs`` of (first row, end, their pages, what they see of them), into ``out``."""
+        """Attention over the latent pages: rows ``q``, in ``runs`` of (end, their pages, what they see of them), into ``out``."""
         H, dn, dr = self.H, self.dn, self.dr
         # the per-head key expansion moved to the query: q_lat[h] = q_unrotated[h] @ W_uk[h]  ([H, T, R])
         qa = hops.latent_head_queries(q, self.w_uk, H, dn, dr, pos, self.freq, self.pitch, pairs=self.pairs)
-        parts = [hops.latent_attention(qa[a:b], kc, vc, tables, H, self.scale, self.window, self.sinks, fast=self.fast, sink=self.sink,
-                                       gate=gate[a:b] if gate is not None else None, **seen) for a, b, tables, seen in runs]
-        o = parts[0] if len(parts) == 1 else torch.cat(parts)
+        args, kw = (H, self.scale, self.window, self.sinks), dict(fast=self.fast, sink=self.sink)
+        if len(runs) == 1 and (gate is None or gate.shape[0] == q.shape[0]):
+            _, tables, seen = runs[0]
+            o = hops.latent_attention(qa, kc, vc, tables, *args, gate=gate, **kw, **seen)
+        else:
+            parts, a = [], 0
+            for b, tables, seen in runs:
+                parts.append(hops.latent_attention(qa[a:b], kc, vc, tables, *args, gate=gate[a:b] if gate is not None else None, **kw, **seen))
+                a = b
+            o = parts[0] if len(parts) == 1 else torch.cat(parts)
         # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T
         hops.latent_head_values(o, self.w_uv, H, out)
 
@@ -527,15 +540,17 @@ class RotaryAttention:
             (proj,) = _take(rows, proj)
             o = _attend_ends(proj, kc, vc, meta, *args, vec=bool(self.fast), gate=proj if hg else None, **kw)
         else:
-            nd = meta.num_decode
-            o = torch.empty(proj.shape[0], H * dv, dtype=proj.dtype, device=proj.device)
-            q, po = (proj[nd:], o[nd:]) if nd else (proj, o)
-            hops.window_attention_prefill(q, kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
-                                          *args, mfma=self.fast, gate=q if hg else None, out=po, **kw)
+            nd, q, o, po = meta.num_decode, proj, None, None
             if nd:
-                hops.window_attention_decode(proj[:nd], kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
-                                             vec=bool(self.fast), gate=proj[:nd] if hg else None, out=o[:nd], **kw)
-            o, proj = _take(rows, o, proj)
+                o = torch.empty(proj.shape[0], H * dv, dtype=proj.dtype, device=proj.device)
+                q, po = proj[nd:], o[nd:]
+            po = hops.window_attention_prefill(q, kc, vc, meta.cu_seqlens, meta.ctx_start, meta.block_tables,
+                                               *args, mfma=self.fast, gate=q if hg else None, out=po, **kw)
+            if nd:
+                q = proj[:nd]
+                hops.window_attention_decode(q, kc, vc, meta.dec_block_tables, meta.dec_seq_lens, *args,
+                                             vec=bool(self.fast), gate=q if hg else None, out=o[:nd], **kw)
+            o, proj = _take(rows, o if nd else po, proj)
         if self.n_tail:
             self.tail_out = (proj, self.n_in)
         return hops.linear(o, self.wo)

@@ -443,6 +443,10 @@ def sigmoid_gate(x: torch.Tensor, proj: torch.Tensor, col: int) -> torch.Tensor:
     return x
 
 
+def _gate_values(x: torch.Tensor, gate: torch.Tensor, col: int) -> torch.Tensor:
+    return sigmoid_gate(x, gate if gate.shape[0] == x.shape[0] else gate[:x.shape[0]], col)
+
+
 def softcap(logits: torch.Tensor, cap: float) -> torch.Tensor:
     """In place on fp32 logits: ``cap * tanh(logits / cap)``."""
     if not logits.is_cuda:
@@ -603,11 +607,11 @@ def window_attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: 
                 js = _visible(p, window, chunked, keep)
                 o = _attend(qkv[r, : Hq * dk].float().view(Hq, dk), ks[js], vs[js], scale, sink, sinks, cap)
                 out[r] = _head_gate(o, hg[r] if hg is not None else None, g_col).reshape(-1).to(qkv.dtype)
-        return sigmoid_gate(out, gate[:T], g_col) if by_value and gate is not None else out
+        return _gate_values(out, gate, g_col) if by_value and gate is not None else out
     gated = native().window_attention_prefill(out, qkv, k_cache, v_cache, cu, ctx, block_tables, Hq, Hkv, dk, dv, float(scale),
                                               int(window), bool(sink), sinks, int(mfma), bool(chunked), float(cap), int(keep), gate,
                                               int(g_col), bool(by_value))
-    return sigmoid_gate(out, gate[:T], g_col) if by_value and gate is not None and not gated else out
+    return _gate_values(out, gate, g_col) if by_value and gate is not None and not gated else out
 
 
 def window_attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -637,11 +641,11 @@ def window_attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: t
             vs = v_cache[bt].permute(0, 3, 1, 2).reshape(-1, Hkv, dv)[js].float()
             o = _attend(qkv[b, : Hq * dk].float().view(Hq, dk), ks, vs, scale, sink, sinks, cap)
             out[b] = _head_gate(o, hg[b] if hg is not None else None, g_col).reshape(-1).to(qkv.dtype)
-        return sigmoid_gate(out, gate[:B], g_col) if by_value and gate is not None else out
+        return _gate_values(out, gate, g_col) if by_value and gate is not None else out
     gated = native().window_attention_decode(out, qkv, k_cache, v_cache, block_tables, seq_lens, Hq, Hkv, dk, dv, float(scale),
                                              int(window), bool(sink), sinks, bool(vec), bool(chunked), float(cap), int(keep), gate,
                                              int(g_col), int(heads), bool(by_value))
-    return sigmoid_gate(out, gate[:B], g_col) if by_value and gate is not None and not gated else out
+    return _gate_values(out, gate, g_col) if by_value and gate is not None and not gated else out
 
 
 # ---------------------------------------------------------------- latent attention
@@ -746,7 +750,8 @@ HEAD_QUERY_ROWS, HEAD_VALUE_ROWS, HEAD_VALUE_WORK = 2048, 256, 1 << 28
 
 
 def _head_rows(most: int, *ts: torch.Tensor) -> bool:
-    return (ts[0].is_cuda and ts[0].shape[0] <= most and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in ts)
+    return (ts[0].dtype == torch.bfloat16 and ts[0].is_cuda and ts[0].shape[0] <= most
+            and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in ts)
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)))
 
 
