@@ -98,11 +98,11 @@ __global__ __launch_bounds__(256) void few_rows_own_kernel(RowsOut o, const bf16
   }
 }
 
-template <int KIND, int MT>
+template <int KIND, int MT, bool ONCE>
 __global__ __launch_bounds__(256) void few_rows_shared_kernel(RowsOut o, const bf16_t* __restrict__ X, long x_stride,
                                                               const bf16_t* __restrict__ W, int Kd) {
   constexpr int NW = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1;
-  using S = SharedRows<MT, NS, NW, true>;
+  using S = SharedRows<MT, NS, NW, ONCE>;
   __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
   int n[NS];
   const bool pair = rows_tiles<KIND>(blockIdx.x * NW + (threadIdx.x >> 6), o.f, n);
@@ -143,12 +143,15 @@ int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const vo
   if (gated ? f <= 0 || f % 16 || N < 2 * f || yg == nullptr : f != 0) return -1;
   const RowsOut o{y, (bf16_t*)yg, M, N, f, f32, cap};
   const unsigned tiles = (unsigned)(gated ? f / 16 + (N - 2 * f + 31) / 32 : (N + 15) / 16);
-  const bool once = 2l * N * Kd > kOnceBytes;  // (the shared form's calls are larger)
+  // (shared, 16 rows, 10240 x 384, us, non-temporal / as usual: 15 such weights in turn, which the memory-side cache holds, 5.3 / 4.5; 100 of them, from
+  // memory, 5.0 / 5.3; 12288 x 320 4.8 / 4.3, 4.5 / 4.75)
+  const bool once = 2l * N * Kd > kOnceBytes;
 #define K8SLLM_FRX(KERNEL, GRID) \
   hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, (const bf16_t*)w, Kd)
-#define K8SLLM_FR(KIND, MT)                                                        \
-  if (shared) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT>), (tiles + 3) / 4);     \
-  else if (once) K8SLLM_FRX((few_rows_own_kernel<KIND, MT, true>), tiles);         \
+#define K8SLLM_FR(KIND, MT)                                                                    \
+  if (shared && once) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT, true>), (tiles + 3) / 4);   \
+  else if (shared) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT, false>), (tiles + 3) / 4);     \
+  else if (once) K8SLLM_FRX((few_rows_own_kernel<KIND, MT, true>), tiles);                     \
   else K8SLLM_FRX((few_rows_own_kernel<KIND, MT, false>), tiles)
 #define K8SLLM_FRM(KIND)              \
   if (M <= 16) { K8SLLM_FR(KIND, 1); } \

@@ -551,6 +551,24 @@ def test_few_rows_and_experts_in_lines(M, K):
     assert bool(((y.double() - z).abs() <= 2 ** -8 * z.abs() + 1e-6 * K ** 0.5).all())
 
 
+@pytest.mark.parametrize("M", [5, 30, 64])
+@pytest.mark.parametrize("shared", [False, True])
+def test_few_rows_of_weights_read_once(M, shared):
+    """Weights of more than 8 MB, which are loaded non-temporal, and the same in halves, which are not: the same bits, and near 64 bits as above."""
+    g = _g(98)
+    N, K = 10304, 448
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
+    assert 2 * w.numel() > 8 << 20 > w.numel()
+    y = torch.full((2, M, N), float("nan"), dtype=BF, device="cuda")
+    hops.native().few_rows(y[0], None, x, w, -1, 0.0, shared)
+    for a in (0, N // 2):
+        h = torch.empty(M, N // 2, dtype=BF, device="cuda")
+        hops.native().few_rows(h, None, x, w[a:a + N // 2], -1, 0.0, shared)
+        y[1, :, a:a + N // 2] = h
+    z = x.double() @ w.double().t()
+    assert torch.equal(y[0], y[1]) and bool(((y[0].double() - z).abs() <= 2 ** -8 * z.abs() + 1e-6 * K ** 0.5).all())
+
+
 def _singles(g, n):
     """Segments, cached tokens and slots of a decode step: a fresh sequence, a padding row and, at last, no token beside two of one sequence."""
     ctx = torch.randint(1, 900, (n,), generator=g)
