@@ -577,14 +577,16 @@ template <typename T, int CH, int MODE, bool HD>
 static void launch_scan_ch(const ScanArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)a.S, (unsigned)a.H, (unsigned)((a.dv + 256 / CH - 1) / (256 / CH)));
   if (a.step) {
-    // four rows of the state a lane where that still gives each compute unit two workgroups
+    // four rows of the state a lane where that still gives each compute unit two workgroups; one row, states of 8 to 16 MB, us, as usual / non-temporal:
+    // delta rule, 32 heads of 128 x 128, 5 segments, 12 layers in turn 8.4 / 7.5, 80 of them, from memory, 8.8 / 6.9; 7 segments 10.4 / 9.9, 11.2 / 9.5
     const bool once = 4l * a.S * a.H * a.dk * a.dv > kStateOnceBytes, four = (long)a.S * a.H * ((a.dv + 1024 / CH - 1) / (1024 / CH)) >= 512;
     const dim3 sg((unsigned)a.S, (unsigned)a.H, (unsigned)(four ? (a.dv + 1024 / CH - 1) / (1024 / CH) : grid.z));
 #define K8SLLM_DSTEP(R, ONCE)                                                                                                \
   hipLaunchKernelGGL((decay_step_kernel<T, CH, MODE, HD, R, ONCE>), sg, dim3(256), 0, s, a.o, (const T*)a.qkv, a.stride, a.q_col, \
                      a.k_col, a.v_col, (const T*)a.z, a.z_stride, a.z_bias, a.a_log, a.inv_tau, a.dkind, (const T*)a.beta,     \
                      a.b_stride, a.bonus, a.state, a.cu, a.ctx, a.slot, a.H, a.Gk, a.dk, a.dv, a.q_scale, a.unit)
-    if (!four) K8SLLM_DSTEP(1, false);
+    if (!four && once) K8SLLM_DSTEP(1, true);
+    else if (!four) K8SLLM_DSTEP(1, false);
     else if (once) K8SLLM_DSTEP(4, true);
     else K8SLLM_DSTEP(4, false);
 #undef K8SLLM_DSTEP

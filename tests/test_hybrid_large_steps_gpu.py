@@ -609,7 +609,7 @@ def test_one_token_a_segment_ssm(n, nh, P, N, G, dt):
 
 @pytest.mark.parametrize("dt", [BF, torch.float32])
 @pytest.mark.parametrize("n,H,Gk,dk,dv", [(3, 4, 2, 128, 128), (40, 16, 16, 64, 64), (24, 40, 20, 128, 128), (5, 2, 1, 96, 20), (30, 32, 32, 8, 300),
-                                          (9, 16, 16, 256, 72), (130, 32, 32, 64, 64)])
+                                          (9, 16, 16, 256, 72), (130, 32, 32, 64, 64), (6, 32, 16, 128, 128)])
 def test_one_token_a_segment_decay(n, H, Gk, dk, dv, dt):
     """Decode steps of the recurrences with decays, one and four rows of the state a lane: the delta rule with decays per channel and per
     head, plain, with a bonus; every sum as in the scan."""
