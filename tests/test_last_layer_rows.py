@@ -5,6 +5,7 @@ import dataclasses
 import pytest
 import torch
 
+from k8s_llm_monitor_amd import ops
 from k8s_llm_monitor_amd.engine.block_manager import BlockManager
 from k8s_llm_monitor_amd.engine.runner import ModelRunner, RunnerConfig
 from k8s_llm_monitor_amd.engine.sequence import SamplingParams, Sequence
@@ -27,13 +28,13 @@ def _small_steps(monkeypatch):
     monkeypatch.setattr(HybridLM, "_wanted", wanted)
 
 
-def _step(model, every, cuts):
-    """Logits of the last rows and the caches after one prompt of 9 tokens, then prompts of 37, 5 and 50 in portions, the last of them beside
+def _step(model, every, cuts, lens=(37, 5, 50, 9), blocks=40):
+    """Logits of the last rows and the caches after one prompt (the last of ``lens``), then the others in portions, the last of them beside
     its running sequence."""
-    runner = ModelRunner(model, RunnerConfig(max_num_seqs=4, max_model_len=128, num_blocks=40, keep_logits=True, use_graphs=False))
-    manager = BlockManager(40, watermark=0.0, prefix_caching=False, state_slots=getattr(runner, "num_state_slots", 0))
+    runner = ModelRunner(model, RunnerConfig(max_num_seqs=4, max_model_len=blocks * 16 // 5, num_blocks=blocks, keep_logits=True, use_graphs=False))
+    manager = BlockManager(blocks, watermark=0.0, prefix_caching=False, state_slots=getattr(runner, "num_state_slots", 0))
     g = torch.Generator().manual_seed(5)
-    ids = [torch.randint(3, model.cfg.vocab_size, (n,), generator=g).tolist() for n in (37, 5, 50, 9)]
+    ids = [torch.randint(3, model.cfg.vocab_size, (n,), generator=g).tolist() for n in lens]
     seqs = [Sequence(prompt_ids=t, params=SamplingParams(temperature=0.0, ignore_eos=True)) for t in ids]
     out = []
     for q in seqs:
@@ -65,9 +66,9 @@ def _step(model, every, cuts):
     return out, [t.float().cpu() for c in runner.kv for t in (flat(c) if isinstance(c, dict) else c)]
 
 
-def _compare(model, tol):
+def _compare(model, tol, *sizes):
     for cuts in ((0, 1), (0, 0.4, 1)):
-        (a, ca), (b, cb) = _step(model, False, cuts), _step(model, True, cuts)
+        (a, ca), (b, cb) = _step(model, False, cuts, *sizes), _step(model, True, cuts, *sizes)
         for x, y in zip(a, b):
             assert x.shape == y.shape and float((x - y).norm() / y.norm()) < tol
         for x, y in zip(ca, cb):  # what the last mixer wrote does not depend on whose logits are wanted
@@ -113,7 +114,8 @@ def test_last_layer_on_wanted_rows(name):
         _compare(m, 1e-4)  # fp32 sums of other shapes
 
 
-def test_last_layer_on_wanted_rows_llama():
+def test_wanted_rows_llama_of_small_steps():
+    """Below 1024 rows (and on the CPU) Llama takes every row to the final norm."""
     _compare(build_model(get_config("llama-tiny"), device="cpu", dtype=torch.float32, seed=3), 1e-4)
 
 
@@ -133,5 +135,24 @@ def test_gpu_last_layer_on_wanted_rows_odd_widths(name):
 
 
 @pytest.mark.gpu
-def test_gpu_last_layer_on_wanted_rows_llama():
+def test_gpu_wanted_rows_llama_of_small_steps():
     _compare(build_model(get_config("llama-tiny-d128"), device="cuda:0", dtype=torch.bfloat16, seed=3), 1e-2)
+
+
+@pytest.mark.gpu
+def test_gpu_last_layer_on_wanted_rows_llama(monkeypatch):
+    """Steps of 1024 rows and more, several prompts and a running sequence's token: behind the last attention only the wanted rows go on,
+    through the same tile kernels, which give a row the same bits whatever rows lie beside it."""
+    rows, real = [], ops.gemm_tile_resid
+    monkeypatch.setattr(ops, "gemm_tile_resid", lambda x, *a, **k: rows.append(x.shape[0]) or real(x, *a, **k))
+    model = build_model(get_config("llama-tiny-d128"), device="cuda:0", dtype=torch.bfloat16, seed=3)
+    n, lens = len(model.layers), (1300, 1111, 1500, 1200)
+    _compare(model, 1e-2, lens, 500)
+    per = 2 * n - 1  # out-projections and all but the last down-projection
+    steps = [rows[i:i + per] for i in range(0, len(rows), per)]
+    few, total = [1, 4, 1, 3, 4], [1199, 3912, 1199, 1564, 2348]  # of one cut, and of a cut at 0.4 (its rows all in such steps)
+    cut = [int(0.4 * t) for t in lens[:3]]
+    assert total[3] == sum(cut) and total[4] == sum(lens[:3]) + 1 - sum(cut)
+    want = [[t] * (per - 1) + [k] for t, k in zip(total, few)]
+    every = [[t] * per for t in total]
+    assert steps == want[:2] + every[:2] + want[2:] + every[2:]
