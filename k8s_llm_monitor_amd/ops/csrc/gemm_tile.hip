@@ -678,7 +678,9 @@ using namespace k8sllm;
 // chip full: 64 x 64 0.26 (plain products), 64 x 128 0.42, 128 x 128 0.72; a tile 1.25, 0.8 where few go as strips of 256 columns.  us, tiles / 128 x 128 /
 // 64 x 128 / 64 x 64, packed weights: 4096 x 4096, 80 rows 56 / - / 35 / 23, 300 56 / - / 35, 600 59 / 54; 4096 x 14336, 80 rows 168 / - / 98 / 58, 400 167 /
 // - / 104, 600 178 / 161; 6144 x 4096 with RoPE, 80 rows 78 / - / 36, 300 81 / - / 38, 400 - / 57 / 67, 600 83 / 58 / 71, 800 84 / 102 (two rounds); 28672 x
-// 4096 with SwiGLU, 80 rows 90 / 62 / 75 (two rounds), 200 90 / 107 (two rounds).
+// 4096 with SwiGLU, 80 rows 90 / 62 / 75 (two rounds), 200 90 / 107 (two rounds).  Rounds are an XCD's: it has whole columns' strips and 32 CUs, so 12
+// columns of 18 strips are two rounds on four of them (1536 x 4096, 2300 rows, us, tile / 128 x 128 52 / 92; 512 x 8192, 5700 rows 97 / 179; of 2280 points
+// of 64 to 5700 rows 39 are then more than 2 % above the least form).
 struct Strips {
   int rows = 0, cols = 0;  // 0: tiles
 };
@@ -689,8 +691,8 @@ static Strips narrow_strips(long M, long N, long K, int epi) {
   float us = nk * (tiles <= kStripTiles && epi != TILE_EPI_ROPE ? 0.8f : 1.25f) + 6.f;
   auto take = [&](int rows, int cols, float ktile) {
     if (N % cols) return;
-    const long n = (M + rows - 1) / rows * (N / cols);
-    const float t = (n + kTileCus - 1) / kTileCus * (nk * ktile + 6.f);
+    const long n = (M + rows - 1) / rows * ((N / cols + 7) / 8);
+    const float t = (n + kTileCus / 8 - 1) / (kTileCus / 8) * (nk * ktile + 6.f);
     if (t < us) us = t, best = Strips{rows, cols};
   };
   if (epi == TILE_EPI_BF16) take(64, 64, 0.26f);

@@ -213,6 +213,7 @@ def test_gemm_tile_last_round(m_tiles, n_tiles, last, K, swiglu):
     (1, 128, 192, False), (65, 4096, 4096, True), (43, 6144, 4096, True), (257, 1024, 8192, False), (512, 512, 1088, False), (80, 28672, 4096, True),
     (600, 6144, 2112, True), (1000, 1024, 4096, False), (70, 320, 512, False), (260, 4096, 2048, True),  # (64 columns: one round of strips, and more)
     (385, 6144, 192, False), (400, 6144, 1088, True), (113, 28672, 320, True), (1000, 4096, 1024, True), (128, 16640, 2048, False),  # (128 rows)
+    (2300, 1536, 192, True), (2300, 1408, 192, False), (1300, 2304, 320, True), (4000, 768, 192, False),  # (columns over the XCDs: two rounds, and one)
 ])
 def test_gemm_tile_narrow_strips(M, N, K, packed):
     """Products of few tiles as strips of 64 x 128, 64 x 64 or 128 x 128: plain, turned, gated in both pairings.  The bits of the schedule that has whole tiles
