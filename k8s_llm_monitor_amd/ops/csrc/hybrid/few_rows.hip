@@ -145,7 +145,7 @@ int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const vo
   const unsigned tiles = (unsigned)(gated ? f / 16 + (N - 2 * f + 31) / 32 : (N + 15) / 16);
   // (shared, 16 rows, 10240 x 384, us, non-temporal / as usual: 15 such weights in turn, which the memory-side cache holds, 5.3 / 4.5; 100 of them, from
   // memory, 5.0 / 5.3; 12288 x 320 4.8 / 4.3, 4.5 / 4.75)
-  const bool once = 2l * N * Kd > kOnceBytes;
+  const bool once = read_once(2l * N * Kd, w, Kd);
 #define K8SLLM_FRX(KERNEL, GRID) \
   hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, (const bf16_t*)w, Kd)
 #define K8SLLM_FR(KIND, MT)                                                                    \

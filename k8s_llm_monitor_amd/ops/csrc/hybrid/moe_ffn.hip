@@ -703,7 +703,7 @@ int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* off
     // Weights that several row tiles read stay in the caches, as those of small calls do (kOnceBytes, stream_rows.h); others are non-temporal (gated /
     // plain us, as usual / non-temporal: 8 experts, 4096 x 3584, 128 rows 87 / 47, 80 / 43; 800 rows 123 / 77, 130 / 79; 2000 rows 242 / 158,
     // 263 / 164).
-    const bool once = rows <= 64l * E && 2 * std::min<long>(rows, E) * (act == 1 || act == 3 ? 2 * N : N) * Kd > kOnceBytes;
+    const bool once = rows <= 64l * E && read_once(2 * std::min<long>(rows, E) * (gated ? 2 * N : N) * Kd, W, Kd);
     const int nw = mt == 4 || (!gated && std::min<long>(rows, E) * ((N + 63) / 64) >= 256) ? 4 : 2;
     const unsigned tiles = (unsigned)(rows / (16 * mt) + E), gz = (tiles + 65534) / 65535;  // (a grid's y ends at 65535)
     const dim3 g((unsigned)((N + 16 * nw - 1) / (16 * nw)), (tiles + gz - 1) / gz, gz);

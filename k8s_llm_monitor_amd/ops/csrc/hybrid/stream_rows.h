@@ -51,7 +51,13 @@ __device__ __forceinline__ int line_frag() {  // of a line's first 32 k; the oth
 }
 // Where this lane finds its chunks of a line's two loads, at k = 0.  K ends inside a line if it is an odd number of 32: the chunks behind
 // it, and lines behind the last, are read from the row's last chunk, and nothing multiplies them.
+// Rows that do not begin at a cache line (an odd number of 32 k) too: two loads meet each of their lines, and what the first brought has gone
+// before the second (4704 k, 1968 columns, 3 rows 7.5 / 7.15, 15 of them in turn 8.8 / 6.6; 928 k, 19776 columns, 1 row 9.9 / 9.7, 11.4 / 10.5; 4128 k,
+// 4096 columns, 1 row 8.1 / 8.3, 9.9 / 9.3).
 constexpr long kOnceBytes = 8l << 20;
+inline bool read_once(long bytes, const void* w, int kd) {
+  return bytes > kOnceBytes && kd % 64 == 0 && reinterpret_cast<uintptr_t>(w) % 128 == 0;
+}
 struct LineSrc {
   const bf16_t* p[2];
   __device__ __forceinline__ int within(int i, int k, int kd) const { return min(k, kd - 8 - line_k(i)); }

@@ -551,12 +551,13 @@ def test_few_rows_and_experts_in_lines(M, K):
     assert bool(((y.double() - z).abs() <= 2 ** -8 * z.abs() + 1e-6 * K ** 0.5).all())
 
 
-@pytest.mark.parametrize("M", [5, 30, 64])
+@pytest.mark.parametrize("M,K", [(5, 448), (30, 448), (64, 448), (30, 480)])
 @pytest.mark.parametrize("shared", [False, True])
-def test_few_rows_of_weights_read_once(M, shared):
-    """Weights of more than 8 MB, which are loaded non-temporal, and the same in halves, which are not: the same bits, and near 64 bits as above."""
+def test_few_rows_of_weights_read_once(M, K, shared):
+    """Weights of more than 8 MB, which are loaded non-temporal where their rows begin at cache lines, and the same in halves, which are not: the
+    same bits, and near 64 bits as above."""
     g = _g(98)
-    N, K = 10304, 448
+    N = 10304
     x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
     assert 2 * w.numel() > 8 << 20 > w.numel()
     y = torch.full((2, M, N), float("nan"), dtype=BF, device="cuda")
