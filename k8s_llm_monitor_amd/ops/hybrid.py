@@ -1275,39 +1275,46 @@ def _rows_form(M: int, N: int, K: int, end: str = "") -> Optional[str]:
               up to 32: 4096 x 4096 14.0 / 9.2 / 15.9; 8192 x 2048 14.4 / 10.4 / 11.1; 11312 x 4096 23.2 / 26.1 / 21.0; 32768 x 4096 69.7 / 68 /
               52.4; 4096 x 11008 32 / 25.6 / 41; 6144 x 5632 20.4 / 23.5 / 23.7
               up to 64: 4096 x 2048 12.3 / 8.2 / 12; 10240 x 4096 29.4 / 31 / 24.7; 16384 x 2048 19.7 / 26 / 19.3; 24576 x 2048 28 / 37 / 31; 32768
-              x 4096 66 / 90 / 58; 6144 x 4096 18.7 / 23 / 21.8
+              x 4096 66 / 90 / 58; 6144 x 4096 18.7 / 23 / 21.8; of few k and many columns 28672 x 256, 48 rows 10.8 / 13.1 / 9.1; 37632 x 256 11.8 /
+              17.1 / 13.8; 54944 x 2496, 56 rows 52 / 91 / 69
     act       8192 x 4096, 64 rows 26.1 / 24.8 / 25.3; 32768 x 2048, 64 rows 50 / 51 / 39; 24576 x 5632, 64 rows 74 / 110 / 70
     glu       (a workgroup of either takes half as many columns) 8192 x 2048, 64 rows 17 / 13 / 19; 16384 x 4096, 16 rows 37 / 27 / 36, 32 rows
               37 / 30 / 35; 24576 x 4096, 24 rows 52 / 41 / 43, 64 rows 53 / 58 / 46; 32768 x 4096, 8 rows 66 / 47 / 60, 16384 x 2048, 24 rows
-              20 / 17 / 20; 32768 x 1024, 4 rows 20 / 18 / 14
-    Between the lines the library is up to 5 % slower, and up to 25 % for units of 25 and more rows against 8 K to 16 K features."""
+              20 / 17 / 20; 32768 x 1024, 4 rows 20 / 18 / 14; of few k 29952 x 64, 16 rows 8.7 / 9.2 / 4.8; 13248 x 256, 48 rows 11.1 / 8.5 / 7.8;
+              23824 x 160, 48 rows 16 / 10.4 / 8.0
+    Over 7000 products of 1 to 64 rows, 256 to 60000 columns and 64 to 16384 k from memory a call takes 1.07 times the least of the three in the
+    mean, a unit 1.08."""
     if M > 64 or K > 16384 or (N * K > 1 << 28 and (M > 4 or end == "glu")):
         return None
     if end == "glu":
         if K > 4096:
             return None
-        if N >= 32768 and (K <= 1024 or M > 8):
+        if N >= 24576 and (K <= 1024 or M > 8):
             return "shared"
-        if M <= 16 or (M <= 32 and K > 2048) or N <= 8192 and (M <= 32 or K <= 2048) or (M <= 24 and N <= 16384):
-            return "own"
-        return "shared" if N >= 24576 else None
+        if M > 16 and N > 8192 and K <= 1024:
+            return "shared" if N > 16384 or (M <= 32 and K <= 512) else "own"
+        return "own" if M <= 16 or (M <= 32 and K > 2048) or N <= 8192 and (M <= 32 or K <= 2048) or (M <= 24 and N <= 16384) else None
     if K > 6144:  # whole lines for each of a workgroup's waves
         return "own" if K % 256 == 0 and (M <= 8 or (M <= 16 and N <= 4096) or (M <= 32 and 2048 < N <= 4096)) else None
     if K > 4096:
         if M <= 2 or (M <= 4 and (end or N <= 4096 or 8192 <= N <= 32768)) or (M <= 32 and 2048 <= N <= 4096):
             return "own"
-        return "shared" if N >= 10240 and (M <= 16 or end) else None
+        return "shared" if N >= 10240 and (M <= 16 or (end and (M <= 32 or N <= 45056))) else None
     if M <= 8:
         return "shared" if N >= 131072 or (N >= 10240 and K <= 1024) else "own"
     if M <= 16:
         return "own" if N * K < 1 << 25 and (N < 10240 or K > 1024) else "shared" if N >= 10240 else None
     if M <= 32:
-        if N * K <= 1 << 24 and (N < 8192 or K > 1024):
+        if N * K <= 1 << 24 and N <= 8192:
             return "own"
         return "shared" if N >= 10240 or (N >= 8192 and K <= 3072) else None
+    if N > 16384 and K <= 512:
+        return "shared" if end or N <= (45056 if K > 256 else 32768) else None
     if N * K <= 1 << 23 or (N * K < 1 << 24 and K <= 2048):
         return "own"
-    return "shared" if 10240 <= N <= 16384 or (N >= 28672 and (end or K >= 2048)) else None
+    if N > 32768 and not (end and (N <= 45056 or K <= 2048)):
+        return None
+    return "shared" if 10240 <= N <= 16384 or (N >= 28672 and (end or K >= 2048)) or (end and 8192 <= N < 10240 and K <= 3072) else None
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, end: str = "") -> Optional[str]:

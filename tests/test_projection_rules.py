@@ -26,3 +26,14 @@ def test_tile_gemm_with_a_unit(M, N, K, f, takes):
 ])
 def test_projections_of_few_rows(end, M, N, K, form):
     assert hops._rows_form(M, N, K, end) == form
+
+
+@pytest.mark.parametrize("end,M,N,K,form", [
+    ("", 33, 56832, 256, None), ("", 48, 28672, 256, "shared"), ("", 64, 16384, 512, "own"), ("", 56, 54944, 2496, None), ("", 64, 32768, 4096, "shared"),
+    ("", 28, 10368, 1056, "shared"), ("", 28, 8192, 2048, "own"), ("act", 48, 35136, 256, "shared"), ("act", 56, 52000, 2688, None),
+    ("act", 56, 45056, 2688, "shared"), ("act", 33, 9920, 2048, "shared"), ("act", 56, 51072, 5056, None), ("act", 56, 45056, 5056, "shared"),
+    ("glu", 16, 29952, 64, "shared"), ("glu", 8, 28672, 1024, "shared"), ("glu", 8, 28672, 1056, "own"), ("glu", 48, 13248, 256, "own"),
+    ("glu", 48, 23824, 160, "shared"), ("glu", 28, 11840, 192, "shared"), ("glu", 28, 11840, 1024, "own"), ("glu", 28, 24576, 4096, "shared"),
+])
+def test_projections_of_few_rows_and_small_k(end, M, N, K, form):
+    assert hops._rows_form(M, N, K, end) == form
