@@ -175,7 +175,7 @@ class WindowAttention:
         H, G, dk, dv = self.H, self.G, self.dk, self.dv
         qkv = F.linear(h, self.wqkv)
         kc, vc = cache["k"], cache["v"]
-        hops.qk_norm_cache(qkv, self.qn, self.kn, self.eps, H, G, dk, dv, kc, vc, meta.slot_mapping)
+        hops.qk_norm_cache(qkv, self.qn, self.kn, self.eps, H, G, dk, dv, kc, vc, meta.slot_mapping, singles=not meta.is_prefill)
         args = (H, G, dk, dv, self.scale, self.window, self.sink)
         if not meta.is_prefill:
             o = hops.window_attention_decode(qkv, kc, vc, meta.block_tables, meta.seq_lens, *args, vec=bool(self.fast))
@@ -529,7 +529,7 @@ class RotaryAttention:
             proj = hops.linear(h, self.w_in)
         kc, vc = cache["k"], cache["v"]
         hops.rotary_cache(proj, H, G, dk, dv, meta.positions, self.freq, self.pairs, self.temp, kc, vc, meta.slot_mapping,
-                          norm=self.norm, qw=self.qn, kw=self.kn, eps=self.eps, v_from_k=self.v_from_k)
+                          norm=self.norm, qw=self.qn, kw=self.kn, eps=self.eps, v_from_k=self.v_from_k, singles=not meta.is_prefill)
         args = (H, G, dk, dv, self.scale, self.window, self.sink)
         kw = dict(sinks=self.sinks, chunked=self.chunked, cap=self.cap, keep=self.keep, g_col=self.g_col, by_value=not self.gate_heads)
         hg = self.has_gate

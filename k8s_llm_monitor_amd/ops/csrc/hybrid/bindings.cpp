@@ -49,10 +49,10 @@ int k8sllm_hy_sigmoid_gate(void* x, const void* z, long z_stride, long rows, int
 int k8sllm_hy_softcap(float* x, long n, float cap, hipStream_t s);
 int k8sllm_hy_rotary_cache(void* qkv, long stride, long T, int Hq, int G, int dk, int dv, const int* positions,
                            const float* freq, int nf, int pairs, const float* q_scale,
-                           void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s);
+                           void* k_cache, void* v_cache, const int* slots, int bs, int singles, int f32, hipStream_t s);
 int k8sllm_hy_swiglu(void* out, const void* gu, long rows, int f, int f32, hipStream_t s);
 int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float* kw, float eps, long T, int nq,
-                            int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s);
+                            int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int singles, int f32, hipStream_t s);
 int k8sllm_hy_window_prefill(void* out, const void* qkv, long q_stride, const void* k_cache, const void* v_cache,
                              const int* cu, const int* ctx, const int* block_tables, int bt_stride, int S, long T,
                              int Hq, int G, int dk, int dv, int bs, float scale, int window, int chunked, int keep,
@@ -468,7 +468,7 @@ Gate gate_of(const OptT& gate, int64_t g_col, int64_t rows, int64_t n, int f, in
 }
 
 void qk_norm_cache(Tensor qkv, Tensor qw, Tensor kw, double eps, int64_t Hq, int64_t G, int64_t dk, int64_t dv,
-                   OptT k_cache, OptT v_cache, OptT slots) {
+                   OptT k_cache, OptT v_cache, OptT slots, bool singles) {
   const int f = act(qkv, "qkv");
   f32c(qw, "qw");
   f32c(kw, "kw");
@@ -488,7 +488,7 @@ void qk_norm_cache(Tensor qkv, Tensor qw, Tensor kw, double eps, int64_t Hq, int
   }
   check(k8sllm_hy_qk_norm_cache(qkv.data_ptr(), qkv.stride(0), qw.data_ptr<float>(), kw.data_ptr<float>(), (float)eps,
                                 qkv.size(0), (int)nq, (int)nk, (int)nv, kc, vc, sp,
-                                k_cache.has_value() ? (int)k_cache->size(1) : 16, f, cur()),
+                                k_cache.has_value() ? (int)k_cache->size(1) : 16, singles, f, cur()),
         "qk_norm_cache");
 }
 
@@ -644,7 +644,7 @@ void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, Opt
 // entries of every q / k head (pairs: entry 2i with 2i + 1, else i with i + len(freq)), q heads times
 // q_scale [Hq] (optional), k and v to the pages.
 void rotary_cache(Tensor qkv, int64_t Hq, int64_t G, int64_t dk, int64_t dv, Tensor positions, Tensor freq, bool pairs,
-                  OptT q_scale, OptT k_cache, OptT v_cache, OptT slots) {
+                  OptT q_scale, OptT k_cache, OptT v_cache, OptT slots, bool singles) {
   const int f = act(qkv, "qkv");
   f32c(freq, "freq");
   i32c(positions, "positions");
@@ -671,7 +671,7 @@ void rotary_cache(Tensor qkv, int64_t Hq, int64_t G, int64_t dk, int64_t dv, Ten
   }
   check(k8sllm_hy_rotary_cache(qkv.data_ptr(), qkv.stride(0), T, (int)Hq, (int)G, (int)dk, (int)dv, positions.data_ptr<int>(),
                                freq.data_ptr<float>(), (int)freq.numel(), pairs, qs, kc, vc, sp,
-                               k_cache.has_value() ? (int)k_cache->size(1) : 16, f, cur()),
+                               k_cache.has_value() ? (int)k_cache->size(1) : 16, singles, f, cur()),
         "rotary_cache");
 }
 

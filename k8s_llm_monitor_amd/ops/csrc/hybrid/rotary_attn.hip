@@ -247,15 +247,15 @@ extern "C" {
 
 int k8sllm_hy_rotary_cache(void* qkv, long stride, long T, int Hq, int G, int dk, int dv, const int* positions,
                            const float* freq, int nf, int pairs, const float* q_scale,
-                           void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s) {
+                           void* k_cache, void* v_cache, const int* slots, int bs, int singles, int f32, hipStream_t s) {
   if (T <= 0) return 0;
   if (nf < 0 || 2 * nf > dk || Hq < 1 || G < 1) return -1;
-  const int runs = !f32 && k_cache != nullptr && value_runs_ok(qkv, stride, (Hq + G) * dk, G * dv, v_cache, slots, T, bs)
+  const int runs = !singles && !f32 && k_cache != nullptr && value_runs_ok(qkv, stride, (Hq + G) * dk, G * dv, v_cache, slots, T, bs)
                        ? value_groups(T, G * dv)
                        : 0;
   const bool wide = nf % 8 == 0 && dk % 8 == 0 && stride % 8 == 0 &&
                     ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(k_cache)) & 15) == 0;
-  const int R = wide && T >= kTurnRows && nf > 0 ? std::max(1, std::min(4, 256 / nf)) : 1;
+  const int R = wide && T >= kTurnRows && nf > 0 && (runs || k_cache == nullptr) ? std::max(1, std::min(4, 256 / nf)) : 1;
   const unsigned grid = (unsigned)((T + R - 1) / R + runs);
 #define K8SLLM_TURN(T_, W) \
   hipLaunchKernelGGL((rotary_cache_kernel<T_, W>), dim3(grid), dim3(256), 0, s, (T_*)qkv, stride, Hq, G, dk, dv, positions, \

@@ -4,6 +4,7 @@
 // lines over the wave and writes a whole page's two values as 64 bytes, a part of a page's in 2-byte stores of its own.
 // rotary_cache, 7830 rows of 2048 + 512 + 512 columns, 7168 apart, bf16: 51 -> 36 us together with its turning (25 of them without pages;
 // the 112 MB take 20 at a copy's rate); qk_norm_cache, 8192 rows of 2048 + 512 + 512: 33 -> 26 (22 without pages).
+// Not for rows of which each is another sequence's: runs of one row wait for the workgroup's others (294 rows of 16 + 2 heads of 64 4.0 us by rows, 7.7).
 #pragma once
 #include "hy_common.h"
 

@@ -956,10 +956,11 @@ int k8sllm_hy_window_f32(void* out, const void* qkv, long q_stride, const void* 
                          const void* gate, long g_stride, int decode, hipStream_t s);
 
 int k8sllm_hy_qk_norm_cache(void* qkv, long stride, const float* qw, const float* kw, float eps, long T, int nq,
-                            int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int f32, hipStream_t s) {
+                            int nk, int nv, void* k_cache, void* v_cache, const int* slots, int bs, int singles, int f32,
+                            hipStream_t s) {
   if (T <= 0) return 0;
   const int runs =
-      !f32 && k_cache != nullptr && value_runs_ok(qkv, stride, nq + nk, nv, v_cache, slots, T, bs) ? value_groups(T, nv) : 0;
+      !singles && !f32 && k_cache != nullptr && value_runs_ok(qkv, stride, nq + nk, nv, v_cache, slots, T, bs) ? value_groups(T, nv) : 0;
   const unsigned grid = (unsigned)(T + runs);
 #define K8SLLM_QK(T_, NV)                                                                                             \
   hipLaunchKernelGGL((qk_norm_cache_kernel<T_, NV>), dim3(grid), dim3(256), 0, s, (T_*)qkv, stride, qw, kw, eps, nq, nk, nv, \

@@ -459,11 +459,11 @@ def softcap(logits: torch.Tensor, cap: float) -> torch.Tensor:
 
 def qk_norm_cache(qkv: torch.Tensor, qw: torch.Tensor, kw: torch.Tensor, eps: float, Hq: int, Hkv: int, dk: int,
                   dv: int, k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor],
-                  slot_mapping: Optional[torch.Tensor]) -> None:
+                  slot_mapping: Optional[torch.Tensor], singles: bool = False) -> None:
     """In place on the fused rows [T, Hq*dk | Hkv*dk | Hkv*dv]: q and k are each divided by the
     root mean square of their WHOLE projection (all heads together, fp32) and multiplied by
     ``qw`` / ``kw``; the normed k and v go to the paged cache at ``slot_mapping`` (< 0: not
-    written)."""
+    written).  ``singles``: as in rotary_cache."""
     nq, nk = Hq * dk, Hkv * dk
     if not qkv.is_cuda:
         q, k = qkv[:, :nq].float(), qkv[:, nq:nq + nk].float()
@@ -478,14 +478,14 @@ def qk_norm_cache(qkv: torch.Tensor, qw: torch.Tensor, kw: torch.Tensor, eps: fl
             bs = k_cache.shape[1]
             v_cache.view(-1, Hkv * dv, bs)[s // bs, :, s % bs] = qkv[ok, nq + nk:]
         return
-    native().qk_norm_cache(qkv, qw, kw, float(eps), Hq, Hkv, dk, dv, k_cache, v_cache, slot_mapping)
+    native().qk_norm_cache(qkv, qw, kw, float(eps), Hq, Hkv, dk, dv, k_cache, v_cache, slot_mapping, bool(singles))
 
 
 def rotary_cache(qkv: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int, positions: torch.Tensor, freq: torch.Tensor,
                  pairs: bool, q_scale: Optional[torch.Tensor], k_cache: Optional[torch.Tensor],
                  v_cache: Optional[torch.Tensor], slot_mapping: Optional[torch.Tensor], norm: int = 0,
                  qw: Optional[torch.Tensor] = None, kw: Optional[torch.Tensor] = None,
-                 eps: float = 0.0, v_from_k: bool = False) -> None:
+                 eps: float = 0.0, v_from_k: bool = False, singles: bool = False) -> None:
     """In place on the fused rows [T, Hq*dk | Hkv*dk | Hkv*dv | ...]: the first ``2 len(freq)`` entries
     of every query and key head turn by the angle ``position * freq[i]`` (fp32; ``pairs``: entry 2i
     with 2i + 1, else entry i with i + len(freq); rotary_freq); the rest of a head passes.  ``q_scale``
@@ -496,7 +496,8 @@ def rotary_cache(qkv: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int, positio
     ``norm``: every query and key head is also RMS-normed over its ``dk`` entries (fp32, ``eps`` inside
     the root) - 1: BEFORE the turn, times ``qw`` / ``kw`` ([dk] fp32, shared by the heads); 2: AFTER the
     turn, no weight.  ``v_from_k``: there are no value columns; the values are the keys as projected
-    (before norm and turn), ``dv == dk``."""
+    (before norm and turn), ``dv == dk``.  ``singles``: every row is another sequence's (GPU: values are then not written by
+    runs of slots)."""
     nq, nk, nv = Hq * dk, Hkv * dk, Hkv * dv
     if not qkv.is_cuda:
         T = qkv.shape[0]
@@ -530,7 +531,7 @@ def rotary_cache(qkv: torch.Tensor, Hq: int, Hkv: int, dk: int, dv: int, positio
         native().rotary_norm_cache(qkv, Hq, Hkv, dk, dv, positions, freq, bool(pairs), int(norm), qw, kw, float(eps), q_scale,
                                    k_cache, v_cache, slot_mapping, bool(v_from_k))
         return
-    native().rotary_cache(qkv, Hq, Hkv, dk, dv, positions, freq, bool(pairs), q_scale, k_cache, v_cache, slot_mapping)
+    native().rotary_cache(qkv, Hq, Hkv, dk, dv, positions, freq, bool(pairs), q_scale, k_cache, v_cache, slot_mapping, bool(singles))
 
 
 def _attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float, sink: bool,

@@ -1440,3 +1440,36 @@ def test_one_token_a_segment_without_states(fixed, dt):
     want = x.float().view(n, nh, P) * (0.0 if fixed else dk[:, None])
     want[2] = 0.0  # a padding row
     torch.testing.assert_close(got.cpu(), want.view(n, nh * P), rtol=1e-6, atol=0)  # one product
+
+
+@pytest.mark.parametrize("T,H,singles", [
+    (3, 2, True), (256, 4, True), (1025, 2, True),   # up to 512 turning pairs a row
+    (511, 13, False), (512, 13, False), (300, 14, False),  # those without and with runs of values; more pairs
+    (300, 14, True), (1030, 20, True),
+])
+def test_values_of_rows_by_themselves(T, H, singles):
+    """Rows whose slots do not follow one another, as a large decode step's, with a few pairs that happen to, inside a page and over two: the values
+    of every row, once.  Copies: equal to the bit."""
+    g, G, dk = _g(91), 3, 64
+    nb = (T + 15) // 16 + 8
+    slots = torch.randperm(nb * 16, generator=g)[:T].to(torch.int32)
+    left = torch.ones(nb * 16, dtype=torch.bool)
+    left[slots.long()] = False
+    for a in (0, 15, 16, T - 3) if T > 16 else ():  # pairs in the first and last rows, over a workgroup's last row
+        p = int((left[:-1] & left[1:]).nonzero()[a % 3])
+        slots[a], slots[a + 1] = p, p + 1
+        left[p:p + 2] = False
+    x = _r(g, T, (H + 2 * G) * dk, dt=BF)
+    freq, pos, w = hops.rotary_freq(1e4, 64), torch.arange(T, dtype=torch.int32), torch.ones(H * dk)
+    for norm in (False, True):
+        out = []
+        for dev in ("cpu", "cuda"):
+            y, kc, vc = x.to(dev, copy=True), torch.zeros(nb, 16, G * dk, dtype=BF, device=dev), torch.zeros(nb, G, dk, 16, dtype=BF, device=dev)
+            if norm:
+                hops.qk_norm_cache(y, w.to(dev), torch.ones(G * dk, device=dev), 1e-5, H, G, dk, dk, kc, vc, slots.to(dev), singles=singles)
+            else:
+                hops.rotary_cache(y, H, G, dk, dk, pos.to(dev), freq.to(dev), False, None, kc, vc, slots.to(dev), singles=singles)
+            out.append((y.cpu(), kc.cpu(), vc.cpu()))
+        assert torch.equal(out[0][2], out[1][2])
+        for a, b in zip(out[0][:2], out[1][:2]):  # turned and normed entries up to one rounding
+            torch.testing.assert_close(a.float(), b.float(), rtol=2 ** -7, atol=2 ** -7)
