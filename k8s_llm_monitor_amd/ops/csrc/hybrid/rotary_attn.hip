@@ -22,6 +22,9 @@ namespace k8sllm {
 
 constexpr int kMaxHeadDim = 1024;
 constexpr long kTurnRows = 1024;  // from here a workgroup takes up to four rows (7830 rows: 28 us by one, 24.6); fewer would leave CUs idle
+constexpr long kFewPairs = 512;  // up to so many turning pairs a row are few (rotary_cache_few_kernel)
+// From so many rows of few pairs values go by runs, with the staged form: 269 rows of 4 + 4 heads of 128 4.2 us by rows, 5.2 by runs; 561 of 8 + 8 6.9, 4.8
+constexpr long kFewRunRows = 512;
 constexpr int kTurns = 512;  // sines and cosines a workgroup of rotary_cache holds at a time
 
 // The norm-only form (norm == 1, nothing turns, head dims of 8 LPH entries): LPH neighbouring lanes hold a head,
@@ -122,6 +125,57 @@ __global__ __launch_bounds__(256) void rotary_norm_cache_kernel(T* __restrict__ 
   }
   __syncthreads();  // the value copy below reads nothing the loop wrote, but keeps the workgroup together
   if (!v_from_k && slot >= 0)
+    for (int c = threadIdx.x; c < nv; c += 256) v_cache[((slot / bs) * nv + c) * bs + slot % bs] = row[nq + nk + c];
+}
+
+// Rows of few turning pairs: a workgroup a row, each pair with sines and cosines of its own, so nothing is staged and no barrier waits.  The same
+// products.  us, staged (below) / here: 1 row of 2 + 2 heads of 32 pairs 3.1 / 2.3, of 8 + 4 of 64 2.8 / 3.0; 64 rows of 8 + 2 of 16 3.9 / 3.0; 220 of 2 + 2
+// of 16 4.0 / 3.3.
+template <typename T>
+__global__ __launch_bounds__(256) void rotary_cache_few_kernel(T* __restrict__ qkv, long stride, int Hq, int G, int dk, int dv,
+                                                               const int* __restrict__ positions, const float* __restrict__ freq, int nf,
+                                                               int pairs, const float* __restrict__ q_scale, T* __restrict__ k_cache,
+                                                               T* __restrict__ v_cache, const int* __restrict__ slots, int bs) {
+  const long t = blockIdx.x;
+  T* row = qkv + t * stride;
+  const int nq = Hq * dk, nk = G * dk, nv = G * dv;
+  const float pos = (float)positions[t];
+  const long slot = (slots != nullptr && k_cache != nullptr) ? slots[t] : -1;
+  T* kp = slot >= 0 ? k_cache + slot * (long)nk : nullptr;
+  const int rest = dk - 2 * nf;  // entries of a head that do not turn
+  for (int e = threadIdx.x; e < (Hq + G) * nf; e += 256) {
+    const int h = e / nf, i = e - h * nf;
+    const int a = pairs ? 2 * i : i, b = pairs ? 2 * i + 1 : i + nf;
+    T* hd = row + (long)h * dk;
+    float sn, cs;
+    sincosf(pos * freq[i], &sn, &cs);
+    const float u = ldf(hd + a), v = ldf(hd + b);
+    float x = fmaf(u, cs, -(v * sn)), y = fmaf(v, cs, u * sn);
+    if (h < Hq && q_scale != nullptr) {
+      x *= q_scale[h];
+      y *= q_scale[h];
+    }
+    stf(hd + a, x);
+    stf(hd + b, y);
+    if (h >= Hq && kp != nullptr) {
+      kp[(h - Hq) * dk + a] = hd[a];
+      kp[(h - Hq) * dk + b] = hd[b];
+    }
+  }
+  if (rest > 0) {
+    if (q_scale != nullptr)
+      for (int e = threadIdx.x; e < Hq * rest; e += 256) {
+        const int h = e / rest, c = e - h * rest + 2 * nf;
+        T* p = row + (long)h * dk + c;
+        stf(p, ldf(p) * q_scale[h]);
+      }
+    if (kp != nullptr)
+      for (int e = threadIdx.x; e < G * rest; e += 256) {
+        const int g = e / rest, c = e - g * rest + 2 * nf;
+        kp[g * dk + c] = row[nq + g * dk + c];
+      }
+  }
+  if (slot >= 0)
     for (int c = threadIdx.x; c < nv; c += 256) v_cache[((slot / bs) * nv + c) * bs + slot % bs] = row[nq + nk + c];
 }
 
@@ -250,9 +304,20 @@ int k8sllm_hy_rotary_cache(void* qkv, long stride, long T, int Hq, int G, int dk
                            void* k_cache, void* v_cache, const int* slots, int bs, int singles, int f32, hipStream_t s) {
   if (T <= 0) return 0;
   if (nf < 0 || 2 * nf > dk || Hq < 1 || G < 1) return -1;
-  const int runs = !singles && !f32 && k_cache != nullptr && value_runs_ok(qkv, stride, (Hq + G) * dk, G * dv, v_cache, slots, T, bs)
+  const bool few = (long)(Hq + G) * nf <= kFewPairs;
+  const int runs = !singles && !f32 && k_cache != nullptr && (!few || T >= kFewRunRows) && value_runs_ok(qkv, stride, (Hq + G) * dk, G * dv, v_cache, slots, T, bs)
                        ? value_groups(T, G * dv)
                        : 0;
+  // (fp32 rows with pages, from kTurnRows on, too: 3397 rows of 40 heads of 128 60 us, by four rows a workgroup 74)
+  if (runs == 0 && (few || (f32 && T >= kTurnRows && k_cache != nullptr))) {
+    if (f32)
+      hipLaunchKernelGGL(rotary_cache_few_kernel<float>, dim3((unsigned)T), dim3(256), 0, s, (float*)qkv, stride, Hq, G, dk, dv, positions, freq, nf,
+                         pairs, q_scale, (float*)k_cache, (float*)v_cache, slots, bs);
+    else
+      hipLaunchKernelGGL(rotary_cache_few_kernel<bf16_t>, dim3((unsigned)T), dim3(256), 0, s, (bf16_t*)qkv, stride, Hq, G, dk, dv, positions, freq,
+                         nf, pairs, q_scale, (bf16_t*)k_cache, (bf16_t*)v_cache, slots, bs);
+    return (int)hipGetLastError();
+  }
   const bool wide = nf % 8 == 0 && dk % 8 == 0 && stride % 8 == 0 &&
                     ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(k_cache)) & 15) == 0;
   const int R = wide && T >= kTurnRows && nf > 0 && (runs || k_cache == nullptr) ? std::max(1, std::min(4, 256 / nf)) : 1;
