@@ -74,6 +74,7 @@ __device__ __forceinline__ void lgkm_wait0() { asm volatile("s_waitcnt lgkmcnt(0
 // the strips would need two rounds, which was no faster (72 tiles of K 1024 35 / 42 us, 128 of K 2048 43.9 / 43.6, 112 behind a round 119 / 126).
 // us, whole tiles / strips: 780 tiles of K 2048 (gated unit) 224 / 214; 258 of K 4096 172 / 157; grouped, 8 experts, 1072 294 / 279 and 536
 // 148 / 140; 320 of K 4096 in 4 experts 204 / 170; 36 of K 1024 28 / 21.
+// Products without such tiles have a kernel without strips (CUT false): 6000 x 12288 x 1408, squared ReLU, 188.5 us with both in one, 186.6 without.
 // Grouped, the count of tiles is known on the device only: each workgroup sums it over the experts, up to kStripExperts of them.
 constexpr int kTileCus = 256, kStripTiles = 64, kStripExperts = 32;
 template <int EPI, int SCH, bool RS>
@@ -84,7 +85,7 @@ constexpr bool tile_strips() {
 static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * 32 - tiles; }
 
 // NARROW: every workgroup a strip of 64 (or 128, TALL) rows x 128 (or 64) columns, for products of few tiles (narrow_strips).
-template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0, bool TALL = false>
+template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0, bool TALL = false, bool CUT = true>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                          int E, int M, int N, int K, long w_es, int n_mt, int n_nt,
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   const int wm = NARROW ? wave : wave >> 1, wn = NARROW ? 0 : wave & 1;
 
   // ---- logical tile: bijective XCD remap, then groups of 8 m-tiles ----
-  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>() && !NARROW;
+  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>() && !NARROW && CUT;
   int mts = n_mt;
   if (GROUPED && STRIPS && strips) {  // the tiles that there are
     mts = 0;
@@ -765,7 +766,9 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   const int strips = cut && (grouped || (over > 0 && over <= kStripTiles));
   const dim3 grid((unsigned)(nwg + (!strips ? 0 : grouped ? 4 * kStripTiles : strip_groups(over))));
 #define K8_TILE_LAUNCH(EPI_, G_, SCH_, RS_)                                                                          \
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, G_, SCH_, RS_>), grid, dim3(256), 0, s, (const bf16_t*)X,                \
+  hipLaunchKernelGGL((strips ? &gemm_w4_kernel<EPI_, G_, SCH_, RS_>                                                  \
+                             : &gemm_w4_kernel<EPI_, G_, SCH_, RS_, 0, false, !tile_strips<EPI_, SCH_, RS_>()>),     \
+                     grid, dim3(256), 0, s, (const bf16_t*)X,                                                        \
                      (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk, strips)
 #define K8_TILE_SCH(SCH_)                                                                                            \
   if (grouped) {                                                                                                     \
@@ -811,7 +814,7 @@ extern "C" int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void
   const int strips = over > 0 && over <= kStripTiles;
   const long groups = nwg + (strips ? strip_groups(over) : 0);
 #define K8_TILE_UNIT(EPI_)                                                                                             \
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false>), dim3((unsigned)groups), dim3(256), 0, s, (const bf16_t*)X, \
+  hipLaunchKernelGGL((strips ? &gemm_w4_kernel<EPI_, false, 1, false> : &gemm_w4_kernel<EPI_, false, 1, false, 0, false, false>), dim3((unsigned)groups), dim3(256), 0, s, (const bf16_t*)X, \
                      (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0, strips)
   if (epi == TILE_EPI_GELU_GLU) K8_TILE_UNIT(TILE_EPI_GELU_GLU);
   else if (epi == TILE_EPI_SILU_GLU) K8_TILE_UNIT(TILE_EPI_SILU_GLU);
