@@ -385,17 +385,16 @@ class LatentAttention:
         # the per-head key expansion moved to the query: q_lat[h] = q_unrotated[h] @ W_uk[h]  ([H, T, R])
         qa = hops.latent_head_queries(q, self.w_uk, H, dn, dr, pos, self.freq, self.pitch, pairs=self.pairs)
         args, kw = (H, self.scale, self.window, self.sinks), dict(fast=self.fast, sink=self.sink)
-        if len(runs) == 1 and (gate is None or gate.shape[0] == q.shape[0]):
-            _, tables, seen = runs[0]
-            o = hops.latent_attention(qa, kc, vc, tables, *args, gate=gate, **kw, **seen)
-        else:
-            parts, a = [], 0
-            for b, tables, seen in runs:
-                parts.append(hops.latent_attention(qa[a:b], kc, vc, tables, *args, gate=gate[a:b] if gate is not None else None, **kw, **seen))
-                a = b
-            o = parts[0] if len(parts) == 1 else torch.cat(parts)
+        left, a = [], 0  # runs of more rows than one of which a workgroup each fills the chip
+        for b, tables, seen in runs:
+            gt = gate[a:b] if gate is not None else None
+            if not hops.latent_attention_values(qa[a:b], kc, vc, tables, *args, self.w_uv, out[a:b], gate=gt, **kw, **seen):
+                left.append((a, b, hops.latent_attention(qa[a:b], kc, vc, tables, *args, gate=gt, **kw, **seen)))
+            a = b
         # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T
-        hops.latent_head_values(o, self.w_uv, H, out)
+        if left:
+            o = left[0][2] if len(left) == 1 else torch.cat([x[2] for x in left])
+            hops.latent_head_values(o, self.w_uv, H, out[left[0][0]:left[-1][1]])
 
     def _expand_ok(self, h: torch.Tensor, meta: AttnMeta) -> bool:
         rows = h.shape[0] - meta.num_decode

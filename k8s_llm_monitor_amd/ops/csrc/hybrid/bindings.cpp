@@ -121,6 +121,13 @@ int k8sllm_hy_latent_attention(void* out, const void* q, long q_stride, const vo
                                const int* cu, const int* ctx, const int* seq_lens, const int* block_tables,
                                int bt_stride, int S, long T, int H, int dkp, int dv, int bs, float scale, int window,
                                const float* sinks, const void* gate, long g_stride, int split, hipStream_t s);
+int k8sllm_hy_latent_parts(long T, int H, int pages, int window);
+int k8sllm_hy_latent_attention_parts(float* o, void* ml, const void* q, long q_stride, const void* k_cache, const void* v_cache,
+                                     const int* cu, const int* ctx, const int* seq_lens, const int* block_tables, int bt_stride,
+                                     int S, long T, int H, int dkp, int dv, int bs, float scale, int window, const float* sinks,
+                                     int np, hipStream_t s);
+int k8sllm_hy_latent_part_values(void* v, const float* o, const void* ml, int np, const void* wv, long T, int H, int dv, int R,
+                                 const void* gate, long g_stride, hipStream_t s);
 int k8sllm_hy_latent_expand(void* kt, void* vt, const void* k_cache, int pitch, const int* page_list, int npages, const void* wk,
                             const void* wv, int H, int R, int dn, int dr, int dv, hipStream_t s);
 int k8sllm_hy_rotate_heads(void* x, long stride, long T, int heads, int D, const int* positions, const float* freq, int nf,
@@ -1300,43 +1307,86 @@ void latent_head_values(Tensor v, Tensor o, Tensor wv, int64_t H) {
   check(k8sllm_hy_latent_head_values(v.data_ptr(), o.data_ptr(), wv.data_ptr(), T, (int)H, (int)dv, (int)R, cur()), "latent_head_values");
 }
 
-// The matrix-core latent attention; false: these sizes or dtype are not the kernel's, nothing was
-// launched.  cu / ctx given: prompt chunks (block_tables per segment); else one row per sequence.
+// What the matrix-core latent attention reads: q [T, H * key pitch]; cu / ctx given: prompt chunks (block_tables per segment); else one
+// row per sequence at its newest token.
+struct LatentArgs {
+  const int *cu = nullptr, *ctx = nullptr, *seq_lens = nullptr;
+  int64_t S = 0, T, dkp, dv;
+};
+LatentArgs latent_args(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const OptT& cu, const OptT& ctx, const OptT& seq_lens,
+                       const Tensor& block_tables, int64_t H, int64_t window) {
+  TORCH_CHECK(k_cache.dim() == 3 && v_cache.dim() == 4, "pages");
+  LatentArgs a;
+  a.dkp = k_cache.size(2);
+  a.dv = v_cache.size(2);
+  a.T = q.size(0);
+  pages(k_cache, 0, a.dkp, "k_cache");
+  vpages(v_cache, k_cache, 0, 1, a.dv);
+  TORCH_CHECK(q.dim() == 2 && q.stride(1) == 1 && q.size(1) == H * a.dkp, "q [T, H * key pitch]");
+  TORCH_CHECK(block_tables.is_cuda() && block_tables.scalar_type() == torch::kInt32 && block_tables.dim() == 2 &&
+                  block_tables.stride(1) == 1,
+              "block_tables [S, W] int32");
+  if (cu.has_value()) {
+    TORCH_CHECK(ctx.has_value(), "cu and ctx come together");
+    a.cu = iptr(cu, "cu");
+    a.ctx = iptr(ctx, "ctx");
+    a.S = ctx->numel();
+    TORCH_CHECK(cu->numel() == a.S + 1 && block_tables.size(0) >= a.S, "cu [S+1], block_tables [S, W]");
+  } else {
+    a.seq_lens = iptr(seq_lens, "seq_lens");
+    TORCH_CHECK(a.seq_lens != nullptr && seq_lens->numel() >= a.T && block_tables.size(0) >= a.T, "seq_lens [T], block_tables [T, W]");
+  }
+  TORCH_CHECK(window >= 0 && H >= 1, "heads / window");
+  return a;
+}
+
+// The matrix-core latent attention; false: these sizes or dtype are not the kernel's, nothing was launched.
 bool latent_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, OptT cu, OptT ctx, OptT seq_lens,
                       Tensor block_tables, int64_t H, double scale, int64_t window, OptT sinks, int64_t split, OptT gate,
                       int64_t g_col) {
   if (act(q, "q") != 0) return false;
   same(out, 0, "out");
-  TORCH_CHECK(k_cache.dim() == 3 && v_cache.dim() == 4, "pages");
-  const int64_t dkp = k_cache.size(2), dv = v_cache.size(2), T = q.size(0);
-  pages(k_cache, 0, dkp, "k_cache");
-  vpages(v_cache, k_cache, 0, 1, dv);
-  TORCH_CHECK(q.dim() == 2 && q.stride(1) == 1 && q.size(1) == H * dkp, "q [T, H * key pitch]");
-  TORCH_CHECK(out.is_contiguous() && out.numel() == T * H * dv, "out [T, H * dv]");
-  TORCH_CHECK(block_tables.is_cuda() && block_tables.scalar_type() == torch::kInt32 && block_tables.dim() == 2 &&
-                  block_tables.stride(1) == 1,
-              "block_tables [S, W] int32");
-  const int *cup = nullptr, *ctxp = nullptr, *slp = nullptr;
-  int64_t S = 0;
-  if (cu.has_value()) {
-    TORCH_CHECK(ctx.has_value(), "cu and ctx come together");
-    cup = iptr(cu, "cu");
-    ctxp = iptr(ctx, "ctx");
-    S = ctx->numel();
-    TORCH_CHECK(cu->numel() == S + 1 && block_tables.size(0) >= S, "cu [S+1], block_tables [S, W]");
-  } else {
-    slp = iptr(seq_lens, "seq_lens");
-    TORCH_CHECK(slp != nullptr && seq_lens->numel() >= T && block_tables.size(0) >= T, "seq_lens [T], block_tables [T, W]");
-  }
-  TORCH_CHECK(window >= 0 && H >= 1, "heads / window");
+  const LatentArgs a = latent_args(q, k_cache, v_cache, cu, ctx, seq_lens, block_tables, H, window);
+  TORCH_CHECK(out.is_contiguous() && out.numel() == a.T * H * a.dv, "out [T, H * dv]");
   int by_head = 0;
-  const Gate ga = gate_of(gate, g_col, T, H, 0, &by_head);
+  const Gate ga = gate_of(gate, g_col, a.T, H, 0, &by_head);
   const int rc = k8sllm_hy_latent_attention(out.data_ptr(), q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
-                                            cup, ctxp, slp, block_tables.data_ptr<int>(), (int)block_tables.stride(0), (int)S, T,
-                                            (int)H, (int)dkp, (int)dv, (int)k_cache.size(1), (float)scale, (int)window,
-                                            sink_ptr(sinks, H), ga.p, ga.stride, (int)split, cur());
+                                            a.cu, a.ctx, a.seq_lens, block_tables.data_ptr<int>(), (int)block_tables.stride(0),
+                                            (int)a.S, a.T, (int)H, (int)a.dkp, (int)a.dv, (int)k_cache.size(1), (float)scale,
+                                            (int)window, sink_ptr(sinks, H), ga.p, ga.stride, (int)split, cur());
   if (rc == 1) return false;
   check(rc, "latent_attention");
+  return true;
+}
+
+// Latent attention of few rows, their windows in parts (0: as many as pay), and the value expansion wv [H * vdim, R] behind it: v [T, H * vdim].
+// false: not these sizes, or one part; nothing was launched.
+bool latent_attention_values(Tensor v, Tensor q, Tensor k_cache, Tensor v_cache, OptT cu, OptT ctx, OptT seq_lens, Tensor block_tables,
+                             int64_t H, double scale, int64_t window, OptT sinks, OptT gate, int64_t g_col, Tensor wv, int64_t np) {
+  if (act(q, "q") != 0) return false;
+  same(v, 0, "v");
+  same(wv, 0, "w_uv");
+  const LatentArgs a = latent_args(q, k_cache, v_cache, cu, ctx, seq_lens, block_tables, H, window);
+  TORCH_CHECK(wv.dim() == 2 && wv.is_contiguous() && wv.size(0) % H == 0 && wv.size(1) == a.dv, "w_uv [H * vdim, R]");
+  const int64_t vdim = wv.size(0) / H;
+  TORCH_CHECK(v.is_contiguous() && v.numel() == a.T * H * vdim, "v [T, H * vdim]");
+  TORCH_CHECK(np >= 0 && np <= 64, "parts");
+  int by_head = 0;
+  const Gate ga = gate_of(gate, g_col, a.T, H, 0, &by_head);
+  if (np == 0) np = k8sllm_hy_latent_parts(a.T, (int)H, (int)block_tables.size(1), (int)window);
+  if (np < 2 || a.T == 0 || a.dv > 256 || a.dv % 16 || a.dkp > 320 || a.dkp % 32 || q.stride(0) % 8 || k_cache.size(1) != 16 ||
+      reinterpret_cast<uintptr_t>(wv.data_ptr()) % 16)
+    return false;
+  const auto f32 = torch::TensorOptions().device(q.device()).dtype(torch::kFloat32);
+  const Tensor o = torch::empty({np, a.T, H, a.dv}, f32), ml = torch::empty({np, a.T, H, 2}, f32);
+  check(k8sllm_hy_latent_attention_parts(o.data_ptr<float>(), ml.data_ptr(), q.data_ptr(), q.stride(0), k_cache.data_ptr(),
+                                         v_cache.data_ptr(), a.cu, a.ctx, a.seq_lens, block_tables.data_ptr<int>(),
+                                         (int)block_tables.stride(0), (int)a.S, a.T, (int)H, (int)a.dkp, (int)a.dv,
+                                         (int)k_cache.size(1), (float)scale, (int)window, sink_ptr(sinks, H), (int)np, cur()),
+        "latent_attention_parts");
+  check(k8sllm_hy_latent_part_values(v.data_ptr(), o.data_ptr<float>(), ml.data_ptr(), (int)np, wv.data_ptr(), a.T, (int)H, (int)vdim,
+                                     (int)a.dv, ga.p, ga.stride, cur()),
+        "latent_part_values");
   return true;
 }
 
@@ -1375,6 +1425,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("latent_head_queries", &latent_head_queries);
   m.def("latent_head_values", &latent_head_values);
   m.def("latent_attention", &latent_attention);
+  m.def("latent_attention_values", &latent_attention_values);
   m.def("sum_norm", &sum_norm);
   m.def("gated_lookup", &gated_lookup);
   m.def("rotary_norm_cache", &rotary_norm_cache);

@@ -9,7 +9,7 @@
 // Rotation: entries i and i + nf of the first 2 * nf entries (nf frequencies, freq[i] given in fp32)
 // turn by the angle position * freq[i] - or, pairs == 1, entries 2i and 2i + 1; angles, sine and cosine
 // are fp32.
-#include "hy_common.h"
+#include "latent_parts.h"
 
 namespace k8sllm {
 
@@ -146,13 +146,17 @@ struct PageIds {
   }
 };
 
-template <int KS_MAX, int DT_MAX, int NW, int QT>
+// PART: few rows leave the chip idle, so gridDim.z workgroups take a row's window, tiles in turn as the waves do, one part of neighbouring tiles
+// each; part z leaves its maximum, denominator and unnormed output (fp32) in ``parts`` and latent_part_values merges them.
+template <int KS_MAX, int DT_MAX, int NW, int QT, bool PART = false>
 __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ cu, const int* __restrict__ ctx,
     const int* __restrict__ seq_lens, const int* __restrict__ block_tables, int bt_stride, int S, int H, int dkp,
-    int dv, float scale, int window, const float* __restrict__ sinks, const bf16_t* __restrict__ gate, long g_stride) {
+    int dv, float scale, int window, const float* __restrict__ sinks, const bf16_t* __restrict__ gate, long g_stride,
+    LatentParts parts = {}) {
   static_assert(NW == 1 || QT == 1, "the window is split over waves only for single tokens");
+  static_assert(!PART || (NW > 1 && QT == 1), "");
   constexpr int OP = DT_MAX * 16 + 4;  // LDS row pitch of the merge buffer (floats)
   __shared__ __attribute__((aligned(16))) float o_s[NW][NW > 1 ? 16 * OP : 4];
   __shared__ float m_s[NW > 1 ? NW : 1][16];
@@ -162,7 +166,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
   // eighth of the (token group, head group) list, so that the windows its waves read overlap in ITS L2
   const int nwg = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
   const int xcd = lin & 7, glin = xcd * (nwg >> 3) + min(xcd, nwg & 7) + (lin >> 3);  // XCD x: workgroups x, x + 8, ..
-  const int hg = glin % (int)gridDim.y, bx = glin / (int)gridDim.y;
+  const int hg = PART ? (int)blockIdx.y : glin % (int)gridDim.y, bx = PART ? (int)blockIdx.x : glin / (int)gridDim.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, quad = lane >> 4;
   // this workgroup's tokens: QT consecutive rows of one segment (token groups are numbered segment
   // by segment), or one sequence's newest token
@@ -191,6 +195,19 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
   }
   const int nh = min(16, H - hg * 16);
   bf16_t* obase = out + ((long)row0 * H + hg * 16) * dv;
+  const long part0 = PART ? ((long)blockIdx.z * gridDim.x + row0) * H + hg * 16 : 0;  // this part of the row's first head
+  // token t of the group sits at position p0 + t and sees keys lo_t .. p0 + t
+  const int lo = window > 0 ? max(0, p0 - window + 1) : 0, hi = p0 + nt;
+  int tile0 = lo >> 4, tile1 = (hi + 15) >> 4;  // its 16-key tiles
+  if (PART && p0 >= 0) {
+    const int n = tile1 - tile0, per = (n + min((int)gridDim.z, (n + NW - 1) / NW) - 1) / min((int)gridDim.z, (n + NW - 1) / NW);
+    tile0 += blockIdx.z * per;
+    tile1 = min(tile1, tile0 + per);
+  }
+  if (PART && (p0 < 0 || tile0 >= tile1)) {  // nothing left for this part
+    if ((int)threadIdx.x < nh) parts.ml[part0 + threadIdx.x] = make_float2(-INFINITY, 0.f);
+    return;
+  }
   if (p0 < 0) {  // padding row of a decode bucket
     for (int c = threadIdx.x; c < nh * dv; c += 64 * NW) obase[c] = 0;
     return;
@@ -198,8 +215,6 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
   const int nks = dkp >> 5, ndt = dv >> 4;
   const int head = hg * 16 + min(c16, nh - 1);
   const int* bt = block_tables + (long)s * bt_stride;
-  // token t of the group sits at position p0 + t and sees keys lo_t .. p0 + t
-  const int lo = window > 0 ? max(0, p0 - window + 1) : 0, hi = p0 + nt;
   bf16x8 qf[QT][KS_MAX];
   f32x4 oacc[QT][DT_MAX];
   float m[QT], l[QT];
@@ -213,7 +228,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
     for (int dt = 0; dt < DT_MAX; ++dt) oacc[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     m[t] = -INFINITY;
     l[t] = 0.f;
-    if (wave == 0) {
+    if (wave == 0 && (!PART || blockIdx.z == 0)) {
       m[t] = sinks != nullptr ? sinks[head] * 1.44269504088896341f : 0.f;
       l[t] = 1.f;
     }
@@ -221,9 +236,9 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
   const bf16_t* kbase = k_cache + 8 * quad;
   const bf16_t* vbase = v_cache + (long)c16 * 16 + 4 * quad;
   const long vpage = (long)dv * 16;
-  const int jfirst = (lo & ~15) + 16 * wave;
+  const int jfirst = 16 * (tile0 + wave), jend = PART ? 16 * tile1 : hi;
   PageIds pages;
-  pages.init(bt, lo >> 4, (hi - 1) >> 4);
+  pages.init(bt, tile0, tile1 - 1);
   bf16x8 kf_n[KS_MAX];
   s16x4 vf_n[DT_MAX];
   auto issue = [&](int j0) {
@@ -239,7 +254,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
   };
   // no register double buffer: with fewer registers two waves fit a SIMD and hide each other's loads
   // better than one wave hides its own (measured both ways)
-  for (int j0 = jfirst; j0 < hi; j0 += 16 * NW) {
+  for (int j0 = jfirst; j0 < jend; j0 += 16 * NW) {
     bf16x8 kf[KS_MAX];
     s16x4 vf[DT_MAX];
     issue(j0);
@@ -342,12 +357,17 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
     const int hh = c / dv, dd = c - hh * dv;
     float M = -INFINITY, L = 0.f, o = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, m_s[w][hh]);  // wave 0's is finite (the sink)
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, m_s[w][hh]);  // wave 0's is finite (the sink, or a part's first tile)
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float f = m_s[w][hh] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_s[w][hh] - M);
       L = fmaf(l_s[w][hh], f, L);
       o = fmaf(o_s[w][hh * OP + dd], f, o);
+    }
+    if (PART) {
+      parts.o[part0 * dv + c] = o;
+      if (dd == 0) parts.ml[part0 + hh] = make_float2(M, L);
+      continue;
     }
     const float gt = gate != nullptr ? sigmoid_f(bf2f(gate[(long)row0 * g_stride + hg * 16 + hh])) : 1.f;
     obase[c] = f2bf(L > 0.f ? o / L * gt : 0.f);
@@ -631,7 +651,7 @@ int k8sllm_hy_latent_attention(void* out, const void* q, long q_stride, const vo
 #define K8SLLM_LA(KS, DT, NW, QT)                                                                                      \
   hipLaunchKernelGGL((latent_attn_mfma_kernel<KS, DT, NW, QT>), grid, dim3(64 * NW), 0, s, (bf16_t*)out,                \
                      (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu, ctx, seq_lens,     \
-                     block_tables, bt_stride, S, H, dkp, dv, scale, window, sinks, (const bf16_t*)gate, g_stride)
+                     block_tables, bt_stride, S, H, dkp, dv, scale, window, sinks, (const bf16_t*)gate, g_stride, LatentParts{})
 #define K8SLLM_LAS(KS, DT)                                            \
   if (nw == 8) K8SLLM_LA(KS, DT, 8, 1);                               \
   else if (nw == 4) K8SLLM_LA(KS, DT, 4, 1);                          \
@@ -641,6 +661,37 @@ int k8sllm_hy_latent_attention(void* out, const void* q, long q_stride, const vo
   else { K8SLLM_LAS(10, 16); }
 #undef K8SLLM_LAS
 #undef K8SLLM_LA
+  return (int)hipGetLastError();
+}
+
+// How many parts a row's window is cut into, for T rows over tables of ``pages`` pages; 1: none.  A workgroup of eight waves takes 4 us for each
+// eight tiles (its loads of 16 key rows ask for 16 lines at a time), one a CU, so few rows are cut until half of the chip is busy, a tile a
+// wave at least; behind that parts cost more in the merge than they save (1.2 us for each four, and their outputs' way through memory).  us with
+// the values behind it, whole / this many parts, 8 heads, 128 + 32 wide: 1 row of 333 keys 10.0 / 9.4, of 1500 21.0 / 11.7, of 4800
+// 50 / 14.6; 16 rows of 1500 22.0 / 14.4, 64 of 1500 25.4 / 18.5, of 4800 61 / 35; 16 heads, 256 + 32: 1 of 1500 35.8 / 15.2, 2 of 4800 95 / 20, 32 of
+// 1500 39.3 / 22.3, 64 of 1500 39.9 / 30.6; 128 of 1500 43.8 / 47.7 in two.  Short windows of many rows lose: 64 rows of 333 keys 18.0 / 20.4.
+int k8sllm_hy_latent_parts(long T, int H, int pages, int window) {
+  const long wgs = T * ((H + 15) / 16);
+  const int tiles = window > 0 ? min(pages, window / 16 + 2) : pages;
+  if (wgs <= 0 || wgs > 64 || tiles < (wgs < 16 ? 16 : 40)) return 1;
+  return (int)min(min(max(128 / wgs, 3l), 16l), (long)((tiles + 7) / 8));
+}
+
+// The same attention, its rows' windows in np parts (latent_part_values then merges them); sizes as above, 1: not these.
+int k8sllm_hy_latent_attention_parts(float* o, void* ml, const void* q, long q_stride, const void* k_cache, const void* v_cache,
+                                     const int* cu, const int* ctx, const int* seq_lens, const int* block_tables, int bt_stride,
+                                     int S, long T, int H, int dkp, int dv, int bs, float scale, int window, const float* sinks,
+                                     int np, hipStream_t s) {
+  if (T <= 0) return 0;
+  if (bs != 16 || dkp % 32 || dv % 16 || dkp > 320 || dv > 256 || q_stride % 8 || np < 1 || np > 65535) return 1;
+  const dim3 grid((unsigned)T, (unsigned)((H + 15) / 16), (unsigned)np);
+#define K8SLLM_LP(KS, DT)                                                                                                       \
+  hipLaunchKernelGGL((latent_attn_mfma_kernel<KS, DT, 8, 1, true>), grid, dim3(512), 0, s, (bf16_t*)nullptr, (const bf16_t*)q,    \
+                     q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu, ctx, seq_lens, block_tables, bt_stride, S, H, \
+                     dkp, dv, scale, window, sinks, (const bf16_t*)nullptr, 0L, LatentParts{o, (float2*)ml})
+  if (dkp <= 128 && dv <= 128) K8SLLM_LP(4, 8);
+  else K8SLLM_LP(10, 16);
+#undef K8SLLM_LP
   return (int)hipGetLastError();
 }
 }

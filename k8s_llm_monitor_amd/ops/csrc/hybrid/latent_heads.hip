@@ -3,7 +3,7 @@
 // so a wave takes the smallest tile that its matrix instruction fills, with its weights' loads in flight together, and the grid is as wide as that
 // gives.  The library's batched products with the launch that put the rows together / these, us: queries of 8 heads of 96 + 32
 // over 256, 1 row 11.6 / 4.2, 64 13.5 / 4.7, 512 14.1 / 5.8; 16 heads, 64 rows 18.9 / 4.4; values of 8 heads of 128, 1 row 7.3 / 4.5, 64 5.9 / 4.9.
-#include "hy_common.h"
+#include "latent_parts.h"
 
 namespace k8sllm {
 
@@ -104,6 +104,88 @@ __global__ __launch_bounds__(64) void latent_head_values_kernel(bf16_t* __restri
     if (n0 + 4 * quad + i < dv) stf(out + i, acc[i]);
 }
 
+// The same of rows whose attention lies in np parts: their merge, times the sigmoid of the row and head's gate, rounded, is the products' operand.
+// Each of a head's dv / 16 workgroups merges its rows again, which costs less than a launch of its own (1.6 us and a round of loads).
+// Four waves take the parts in turn, then a quarter of R each: nothing waits for a part's maximum before its output is on its way.
+__global__ __launch_bounds__(256) void latent_part_values_kernel(bf16_t* __restrict__ v, LatentParts parts, int np,
+                                                                 const bf16_t* __restrict__ wv, int T, int H, int dv, int R,
+                                                                 const bf16_t* __restrict__ gate, long g_stride) {
+  constexpr int KC = 8, NW = 4, KW = KC / NW;  // pieces of 32 k: R <= 256
+  __shared__ __attribute__((aligned(16))) float4 o_s[NW][2 * KC][64];
+  __shared__ float2 ml_s[NW][64];
+  __shared__ hf32x4 red[NW][64];
+  const int h = blockIdx.y, t0 = 16 * blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
+  const int n0 = 16 * blockIdx.x;
+  const bf16_t* wr = wv + ((long)h * dv + min(n0 + col, dv - 1)) * R;
+  const long th = (long)min(t0 + col, T - 1) * H + h, step = (long)T * H;
+  uint4 a[KW];
+#pragma unroll
+  for (int c = 0; c < KW; ++c) {
+    const int k = 32 * (KW * wave + c) + 8 * quad;
+    a[c] = k < R ? *reinterpret_cast<const uint4*>(wr + k) : make_uint4(0, 0, 0, 0);
+  }
+  float M = -INFINITY, L = 0.f, o[KC][8] = {};
+  for (int z = wave; z < np; z += NW) {
+    const float2 ml = parts.ml[z * step + th];
+    const float* p = parts.o + (z * step + th) * R + 8 * quad;
+    float x[KC][8];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) load8(p + (32 * c + 8 * quad < R ? 32 * c : -8 * quad), x[c]);
+    const bool empty = ml.x == -INFINITY;  // its output is not written
+    const float m = fmaxf(M, ml.x), f0 = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - m), f1 = empty ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
+    M = m;
+    L = fmaf(ml.y, f1, L * f0);
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[c][j] = fmaf(empty ? 0.f : x[c][j], f1, o[c][j] * f0);
+  }
+#pragma unroll
+  for (int c = 0; c < KC; ++c) {
+    o_s[wave][2 * c][lane] = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
+    o_s[wave][2 * c + 1][lane] = make_float4(o[c][4], o[c][5], o[c][6], o[c][7]);
+  }
+  ml_s[wave][lane] = make_float2(M, L);
+  __syncthreads();
+  float f[NW];
+  M = -INFINITY;
+  L = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_s[w][lane].x);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const float2 ml = ml_s[w][lane];
+    f[w] = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - M);
+    L = fmaf(ml.y, f[w], L);
+  }
+  float inv = L > 0.f ? 1.f / L : 0.f;
+  if (gate != nullptr) inv *= sigmoid_f(bf2f(gate[(long)min(t0 + col, T - 1) * g_stride + h]));
+  hf32x4 acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < KW; ++c) {
+    float x[8] = {};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float4 u = o_s[w][2 * (KW * wave + c)][lane], s = o_s[w][2 * (KW * wave + c) + 1][lane];
+      const float y[8] = {u.x, u.y, u.z, u.w, s.x, s.y, s.z, s.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = fmaf(y[j], f[w], x[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = 32 * (KW * wave + c) + 8 * quad < R ? x[j] * inv : 0.f;
+    acc = tile_product(a[c], pack8(x), acc);
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave || t0 + col >= T) return;
+#pragma unroll
+  for (int w = 1; w < NW; ++w) acc += red[w][lane];
+  bf16_t* out = v + ((long)(t0 + col) * H + h) * dv + n0 + 4 * quad;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (n0 + 4 * quad + i < dv) stf(out + i, acc[i]);
+}
+
 }  // namespace k8sllm
 
 using namespace k8sllm;
@@ -128,6 +210,16 @@ int k8sllm_hy_latent_head_values(void* v, const void* o, const void* wv, long T,
   if (R < 8 || R % 8 || T > (1 << 19) || H > 65535 || ((reinterpret_cast<uintptr_t>(o) | reinterpret_cast<uintptr_t>(wv)) & 15)) return -1;
   hipLaunchKernelGGL(latent_head_values_kernel, dim3((unsigned)((dv + 15) / 16), (unsigned)H, (unsigned)((T + 15) / 16)), dim3(64), 0, s,
                      (bf16_t*)v, (const bf16_t*)o, (const bf16_t*)wv, (int)T, H, dv, R);
+  return (int)hipGetLastError();
+}
+
+int k8sllm_hy_latent_part_values(void* v, const float* o, const void* ml, int np, const void* wv, long T, int H, int dv, int R,
+                                 const void* gate, long g_stride, hipStream_t s) {
+  if (T <= 0 || H <= 0 || dv <= 0) return 0;
+  if (R < 16 || R % 16 || R > 256 || T > (1 << 19) || H > 65535 || np < 1 || (reinterpret_cast<uintptr_t>(wv) & 15)) return -1;
+  hipLaunchKernelGGL(latent_part_values_kernel, dim3((unsigned)((dv + 15) / 16), (unsigned)H, (unsigned)((T + 15) / 16)), dim3(256), 0, s,
+                     (bf16_t*)v, LatentParts{(float*)o, (float2*)ml}, np, (const bf16_t*)wv, (int)T, H, dv, R, (const bf16_t*)gate,
+                     g_stride);
   return (int)hipGetLastError();
 }
 }

@@ -863,6 +863,19 @@ def latent_attention(qa: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     return window_attention_decode(qa, k_cache, v_cache, block_tables, seq_lens, *args, vec=bool(fast), **kw)
 
 
+def latent_attention_values(qa: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor, H: int,
+                            scale: float, window: int, sinks: Optional[torch.Tensor], w_uv: torch.Tensor, out: torch.Tensor,
+                            cu: Optional[torch.Tensor] = None, ctx: Optional[torch.Tensor] = None,
+                            seq_lens: Optional[torch.Tensor] = None, fast: int = 1, sink: bool = True,
+                            gate: Optional[torch.Tensor] = None, g_col: int = 0, parts: int = 0) -> bool:
+    """``latent_attention`` and ``latent_head_values`` into ``out`` of rows too few to fill the chip, each row's window cut into ``parts``
+    (0: as many as pay) whose merge is the value expansion's prologue.  False: nothing was done, these are not such rows."""
+    if not (fast and _head_rows(HEAD_VALUE_ROWS, qa, w_uv) and out.is_contiguous()):
+        return False
+    return native().latent_attention_values(out, qa, k_cache, v_cache, cu, ctx, seq_lens, block_tables, int(H), float(scale), int(window),
+                                            sinks if sink else _no_sink(H, qa.device), gate, int(g_col), w_uv, int(parts))
+
+
 # ---------------------------------------------------------------- Mamba-2
 
 def conv_silu(proj: torch.Tensor, col0: int, C: int, conv_w: torch.Tensor, conv_b: Optional[torch.Tensor],

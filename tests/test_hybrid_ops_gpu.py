@@ -446,3 +446,32 @@ def test_gelu_experts_on_the_tile_gemm():
     want = H.moe_experts(h, ids, wts, w1, w2, None, None, act="gelu")
     got = H.moe_experts(h.cuda(), ids.cuda(), wts.cuda(), w1.cuda(), w2.cuda(), None, None, act="gelu")
     torch.testing.assert_close(got.cpu(), want, **_tol(dt))
+
+
+@pytest.mark.parametrize("Hq,pitch,R,dv", [(8, 160, 128, 128), (16, 288, 256, 128), (20, 64, 48, 40), (1, 32, 32, 16)])
+@pytest.mark.parametrize("window,parts", [(0, 0), (0, 2), (0, 7), (0, 64), (200, 3), (24, 2)])
+def test_latent_attention_in_parts(Hq, pitch, R, dv, window, parts):
+    """Few rows whose windows are cut into parts (more and fewer than there are tiles, a padding row, partial head groups, a chunk's rows, a
+    gate), merged in the value expansion, against fp32.  Each of value, weight and result is rounded once to bf16 (2^-9)."""
+    dt, g = torch.bfloat16, _g(23)
+    lens = [350, 9, 1, 0, 129, 1100]  # the fourth is a padding row
+    kc, vc, bt = _paged(g, dt, [max(n, 1) for n in lens], Hq, 1, pitch, R, nb=120)
+    sinks, wv, gate = _r(g, Hq, s=1.5), _r(g, Hq * dv, R, s=R ** -0.5, dt=dt), _r(g, 6, Hq + 3, dt=dt)
+    qa = _r(g, 6, Hq * pitch, s=0.25, dt=dt)
+    chunk = dict(cu=_i32([0, 4, 6]), ctx=_i32([346, 1098]))  # rows 346 .. 349 of the first sequence, 1098 and 1099 of the last
+    for seen, tables in ((dict(seq_lens=_i32(lens)), bt), (chunk, bt[[0, 5]])):
+        for gt in (None, gate):
+            full = lambda v: H.latent_attention(qa.float(), kc.float(), v, tables, Hq, 0.2, window, sinks, gate=gt.float() if gt is not None else None,  # noqa: E731
+                                                g_col=3 if gt is not None else 0, **seen).view(6, Hq, R)
+            w = wv.float().view(Hq, dv, R)
+            o, oa = full(vc.float()), full(vc.float().abs())
+            want, most = torch.einsum("thr,hdr->thd", o, w), torch.einsum("thr,hdr->thd", o.abs() + oa, w.abs())
+            out = torch.full((6, Hq * dv), 7.0, dtype=dt, device="cuda")
+            took = H.latent_attention_values(qa.cuda(), kc.cuda(), vc.cuda(), tables.cuda(), Hq, 0.2, window, sinks.cuda(), wv.cuda(), out,
+                                             gate=gt.cuda() if gt is not None else None, g_col=3 if gt is not None else 0, parts=parts,
+                                             **{k: v.cuda() for k, v in seen.items()})
+            assert took
+            err = (out.cpu().float().view(6, Hq, dv) - want).abs()
+            assert bool((err <= 2.0 ** -9 * 1.1 * (want.abs() + most) + 1e-5).all()), (err - 2.0 ** -9 * (want.abs() + most)).max()
+            if "seq_lens" in seen:
+                assert float(out[3].abs().max()) == 0.0
