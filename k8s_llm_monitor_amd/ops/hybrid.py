@@ -1344,14 +1344,35 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, end: str = "") -> Optional[str]:
     return _rows_form(x.shape[0], w.shape[0], w.shape[1], end)
 
 
+def _tile_plain(M: int, N: int, K: int) -> bool:
+    """Whether the tile GEMM takes a large product with nothing behind it: where N is no multiple of its 256 columns and K small, the BLAS
+    library's kernels fall to 350 (K up to 512), 600 (1024) and 800 TFLOP/s (2048, N below 4096), and the tile GEMM's rounds of 256 tiles, estimated
+    here, take less than that.  Elsewhere the library is 5 to 14 % ahead.  us, library / tile GEMM: 6403 x 5648 x 1024 122 / 89, 4800 rows 97 / 64;
+    7830 x 3104 x 2048 129 / 100; 8000 x 1568 x 1024 40 / 32.  Over 400 products of 1024 to 9000 rows, 1024 to 12000 columns and 256 to 2048 k
+    (N no multiple of 256) the 181 that it takes are 1.31 times faster in the mean, the worst 0.98; of multiples of 256 it would lose as many as it wins."""
+    if M < 1024 or not 1024 <= N < 1 << 19 or N % 256 == 0 or N % 16 or K % 64 or not 192 <= K <= 2048 or (K > 1024 and N >= 4096):
+        return False  # (the tile GEMM's offsets into the weights are 31 bits)
+    rounds, over = divmod(-(-M // 256) * -(-N // 256), 256)
+    last = 0.0 if over == 0 else (0.62 if rounds else 0.85) if over <= 64 else 0.82 + 0.18 * over / 256  # strips, or a round that is not full
+    us = (rounds + last) * (9 + 1.45 * K / 64)
+    return us * (350 if K <= 512 else 600 if K <= 1024 else 800) < 2e-6 * M * N * K
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x`` [T, K] times ``w`` [N, K] transposed.  The BLAS library's product, but for the few rows of a decode step in bf16 on the
-    device, K a multiple of 32 and rows 16-byte aligned, where a call takes what it takes to get enough loads in flight
-    (few_rows.hip, by the rule of ``_rows_form``)."""
+    """``x`` [T, K] times ``w`` [N, K] transposed.  The BLAS library's product, but for bf16 on the device with rows 16-byte aligned: the
+    few rows of a decode step, K a multiple of 32, where a call takes what it takes to get enough loads in flight
+    (few_rows.hip, by the rule of ``_rows_form``), and large products by the rule of ``_tile_plain``."""
     form = _few_rows(x, w)
     if form is not None:
         y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
         native().few_rows(y, None, x, w, -1, 0.0, form == "shared")
+        return y
+    if x.shape[0] >= 1024 and _tile_operands(x, w) and _tile_plain(x.shape[0], w.shape[0], w.shape[1]) and not (
+            torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+        from .. import ops
+
+        y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        ops.native().gemm_tile(y, x, w, None, 0, 1)
         return y
     return F.linear(x, w)
 
@@ -1373,10 +1394,14 @@ def _tile_form(M: int, N: int, K: int, f: int) -> bool:
             and 256 * N * 2 < 1 << 31)
 
 
+def _tile_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.is_contiguous()
+            and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
 def _tile_unit(x: torch.Tensor, w: torch.Tensor, f: int) -> bool:
     """Whether ``gemm_tile_unit`` takes these operands, by the rule of ``_tile_form``."""
-    return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and w.is_contiguous()
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _tile_form(x.shape[0], w.shape[0], w.shape[1], f))
+    return _tile_operands(x, w) and _tile_form(x.shape[0], w.shape[0], w.shape[1], f)
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, kind: str) -> torch.Tensor:

@@ -452,7 +452,7 @@ def test_gelu_experts_on_the_tile_gemm():
 @pytest.mark.parametrize("window,parts", [(0, 0), (0, 2), (0, 7), (0, 64), (200, 3), (24, 2)])
 def test_latent_attention_in_parts(Hq, pitch, R, dv, window, parts):
     """Few rows whose windows are cut into parts (more and fewer than there are tiles, a padding row, partial head groups, a chunk's rows, a
-    gate), merged in the value expansion, against fp32.  Each of value, weight and result is rounded once to bf16 (2^-9)."""
+    gate), merged in the value expansion, against fp32.  Weights, values and result are rounded once each to bf16 (2^-8)."""
     dt, g = torch.bfloat16, _g(23)
     lens = [350, 9, 1, 0, 129, 1100]  # the fourth is a padding row
     kc, vc, bt = _paged(g, dt, [max(n, 1) for n in lens], Hq, 1, pitch, R, nb=120)
@@ -472,6 +472,6 @@ def test_latent_attention_in_parts(Hq, pitch, R, dv, window, parts):
                                              **{k: v.cuda() for k, v in seen.items()})
             assert took
             err = (out.cpu().float().view(6, Hq, dv) - want).abs()
-            assert bool((err <= 2.0 ** -9 * 1.1 * (want.abs() + most) + 1e-5).all()), (err - 2.0 ** -9 * (want.abs() + most)).max()
+            assert bool((err <= 2.0 ** -8 * (want.abs() + most) + 1e-5).all()), (err - 2.0 ** -8 * (want.abs() + most)).max()
             if "seq_lens" in seen:
                 assert float(out[3].abs().max()) == 0.0

@@ -37,3 +37,31 @@ def test_projections_of_few_rows(end, M, N, K, form):
 ])
 def test_projections_of_few_rows_and_small_k(end, M, N, K, form):
     assert hops._rows_form(M, N, K, end) == form
+
+
+@pytest.mark.parametrize("M,N,K,takes", [
+    (6403, 5648, 1024, True), (1024, 5648, 1024, False), (7830, 3104, 2048, True), (5400, 3104, 2048, False), (8000, 11296, 2048, False),
+    (7830, 5632, 1024, False), (7830, 5640, 1024, False), (7830, 5648, 1056, False), (7830, 5648, 128, False), (8000, 1040, 192, False), (8000, 1040, 512, True),
+    (1023, 60016, 1024, False), (1024, 60016, 1024, True), (1024, 1 << 19 | 16, 1024, False), (8000, 4080, 2048, True), (8000, 4112, 2048, False),
+])
+def test_tile_gemm_of_plain_products(M, N, K, takes):
+    assert hops._tile_plain(M, N, K) is takes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2304, 5648, 1024), (7937, 3104, 2048), (2048, 8000, 192), (2049, 5680, 512)])
+def test_plain_product_on_the_tile_gemm(M, N, K):
+    """Column counts that end inside a tile, row counts that end behind one and in front of one, few k-tiles.  A sum of K products of bf16 in fp32
+    is within K 2^-24 of the sum of their absolute values, and is rounded once (2^-8)."""
+    import torch
+
+    assert hops._tile_plain(M, N, K)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w = (torch.randn(r, K, generator=g, device="cuda").to(torch.bfloat16) for r in (M, N))
+    want, most = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert bool(((hops.linear(x, w).double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * most).all())
+    xg = x.clone().requires_grad_()  # the library's product has a backward
+    hops.linear(xg, w).sum().backward()
+    assert xg.grad is not None
+    wide = torch.cat([x, x], 1)[:, :K]  # rows of another stride
+    assert torch.equal(hops.linear(wide, w), torch.nn.functional.linear(wide, w))
