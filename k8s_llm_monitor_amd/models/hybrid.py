@@ -281,6 +281,7 @@ class LatentAttention:
     rows are expanded whatever they take, as each projection of the step holds them too.)"""
 
     kind = "latent_attention"
+    first_product = True  # of the input rows, only a projection reads them
     EXPAND_MIN_ROWS = 64
     EXPAND_KEYS = 32
     EXPAND_BYTES = 1 << 30
@@ -465,6 +466,7 @@ class RotaryAttention:
     input projection computed by the caller (this mixer's columns of a wider GEMM)."""
 
     kind = "rotary_attention"
+    first_product = True
 
     def __init__(self, spec: LayerSpec, d: int, eps: float, p: _Params, prefix: str, traits: Optional[dict] = None,
                  tail: Optional[torch.Tensor] = None, opts: Optional[dict] = None):
@@ -576,6 +578,7 @@ class LightningMixer:
     ``tail``: extra rows for the input projection (see LatentAttention)."""
 
     kind = "lightning"
+    first_product = True
     stateful = True
 
     def __init__(self, spec: LayerSpec, d: int, eps: float, p: _Params, prefix: str, traits: Optional[dict] = None,
@@ -1036,6 +1039,8 @@ class GatedDenseFFN:
     """``down(act(gate h) * (up h))`` with ``act`` the tanh GELU (or ``relu``, ``silu``): gate and up (and
     ``tail``: extra rows whose outputs forward leaves in ``tail_out``) in one projection, the gated unit
     in one launch."""
+
+    first_product = True
 
     def __init__(self, spec: DenseSpec, d: int, p: _Params, prefix: str, tail: Optional[torch.Tensor] = None,
                  act: str = "gelu_tanh"):
@@ -1609,6 +1614,11 @@ class HybridLM:
             return sub.tail_out
         return F.linear(h, g["w"]), 0
 
+    @staticmethod
+    def _gated_rows(sub, g: dict, *args):
+        """A sublayer's input rows; not made yet where its first product is all that reads them and can make them."""
+        return (hops.gated_rows if g["w"] is None and getattr(sub, "first_product", False) else hops.gated_add_norm)(*args)
+
     def _forward_gated(self, x: Optional[torch.Tensor], meta: AttnMeta, caches: list, ids: torch.Tensor) -> torch.Tensor:
         """Sequential blocks with a gated residual: every sublayer's result y joins the stream as
         ``x += m * y * sigmoid(gate + b)``, folded into the launch of the norm that follows it.  ``x`` None: the embeddings of ``ids``."""
@@ -1621,24 +1631,27 @@ class HybridLM:
                 if pend is not None:
                     raise ValueError("looped layers with a gated residual are not built")
                 x += self.loop_step[t]
-            w1 = self.norms[li]
+            w1, mx = self.norms[li], self.mixers[li]
+            rows = want if r + 1 == len(self.runs) else None
             if x is None:
                 x, h = hops.embed_norm(ids, meta.positions, self.embed, self.pos, meta.dec_src, meta.dec_prev, c.embed_scale, None, w1, eps, op)
             elif pend is None:
                 h = hops.add_norm(x, (), None, w1, eps, op, self.dtype)
             else:
-                h = hops.gated_add_norm(x, pend[0], pend[1], pend[2], pend[3], mult, w1, eps, op, self.dtype)
-            mx = self.mixers[li]
-            rows = want if r + 1 == len(self.runs) else None
+                h = self._gated_rows(mx if rows is None else None, self.rg1[li], x, *pend, mult, w1, eps, op, self.dtype)
             y = mx.forward(h, meta, caches[self.kv_run[r]], rows=rows)
+            if isinstance(h, hops.GatedRows):
+                x = h.residual
             (x,) = _take(rows, x)
             if self.rg1[li]["w"] is not None:
                 (h,) = _take(rows, h)
             pend = (y, *self._gate_of(mx, self.rg1[li], h), self.rg1[li]["b"])
             ff = self.ffns[li]
             if ff is not None:
-                h2 = hops.gated_add_norm(x, pend[0], pend[1], pend[2], pend[3], mult, self.norms2[li], eps, op, self.dtype)
+                h2 = self._gated_rows(ff, self.rg2[li], x, *pend, mult, self.norms2[li], eps, op, self.dtype)
                 y = ff.forward(h2)
+                if isinstance(h2, hops.GatedRows):
+                    x = h2.residual
                 pend = (y, *self._gate_of(ff, self.rg2[li], h2), self.rg2[li]["b"])
             if self.layer_probe is not None:
                 d = x.shape[1]

@@ -96,6 +96,9 @@ int k8sllm_hy_router(int* ids, float* wts, float* gate, const void* h, long T, i
                      const float* bias, int E, int K, int rows_w, int over_all, int f32, hipStream_t s);
 int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const void* w, int M, int N, int Kd, int f, int kind, int f32,
                        float cap, int shared, hipStream_t s);
+int k8sllm_hy_few_rows_gated(void* y, void* yg, const float* x, float* xn, const void* add, const void* gate, long g_stride,
+                             const float* bias, float mult, const float* nw, float eps, int one_plus, const void* w, int M, int N, int Kd,
+                             int f, int kind, hipStream_t s);
 int k8sllm_hy_grouped_gemm(void* Y, const void* A, const void* W, const int* offsets, const int* sorted_idx, int div,
                            int E, long rows, int N, int Kd, long w_es, int act, int il, int f32, int mfma, float limit,
                            hipStream_t s);
@@ -1087,6 +1090,45 @@ void few_rows(Tensor y, OptT yg, Tensor x, Tensor w, int64_t kind, double cap, b
         "few_rows");
 }
 
+// few_rows of the rows that gated_add_norm makes of residual, add and the gate in proj's columns: xn gets the new residual
+void few_rows_gated(Tensor y, OptT yg, Tensor residual, Tensor xn, Tensor add, Tensor proj, int64_t g_col, Tensor bias, double mult, Tensor nw,
+                    double eps, bool one_plus, Tensor w, int64_t kind) {
+  f32c(residual, "residual");
+  f32c(xn, "new residual");
+  f32c(nw, "norm weight");
+  f32c(bias, "gate bias");
+  same(add, 0, "add");
+  same(proj, 0, "proj");
+  same(w, 0, "w");
+  same(y, 0, "y");
+  int64_t f = 0;
+  void* yp = nullptr;
+  TORCH_CHECK(residual.dim() == 2 && xn.sizes() == residual.sizes() && add.sizes() == residual.sizes() && add.is_contiguous(),
+              "few_rows_gated: residual, new residual, add [M, K]");
+  const int64_t M = residual.size(0), K = residual.size(1);
+  TORCH_CHECK(xn.data_ptr() != residual.data_ptr(), "few_rows_gated: the new residual needs a buffer of its own");
+  TORCH_CHECK(yg.has_value() == (kind >= 0), "few_rows_gated: a gated unit's output");
+  if (yg.has_value()) {
+    same(*yg, 0, "yg");
+    TORCH_CHECK(yg->dim() == 2 && yg->is_contiguous() && yg->size(0) == M, "few_rows_gated: yg [M, f]");
+    f = yg->size(1);
+    yp = yg->data_ptr();
+  }
+  TORCH_CHECK(w.dim() == 2 && w.is_contiguous() && w.size(1) == K && y.dim() == 2 && y.is_contiguous() && y.size(0) == M &&
+                  2 * f + y.size(1) == w.size(0) && nw.numel() == K && bias.numel() == K,
+              "few_rows_gated: layouts");
+  TORCH_CHECK(proj.dim() == 2 && proj.stride(1) == 1 && proj.size(0) == M && g_col >= 0 && g_col + K <= proj.size(1), "few_rows_gated: gate columns");
+  const char* gate = (const char*)proj.data_ptr() + 2 * g_col;
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(w.data_ptr()) | reinterpret_cast<uintptr_t>(add.data_ptr()) |
+               reinterpret_cast<uintptr_t>(residual.data_ptr()) | reinterpret_cast<uintptr_t>(xn.data_ptr()) |
+               reinterpret_cast<uintptr_t>(nw.data_ptr()) | reinterpret_cast<uintptr_t>(bias.data_ptr())) % 16 == 0,
+              "few_rows_gated: alignment");
+  check(k8sllm_hy_few_rows_gated(y.data_ptr(), yp, residual.data_ptr<float>(), xn.data_ptr<float>(), add.data_ptr(), gate, proj.stride(0),
+                                 bias.data_ptr<float>(), (float)mult, nw.data_ptr<float>(), (float)eps, one_plus, w.data_ptr(), (int)M,
+                                 (int)w.size(0), (int)K, (int)f, (int)kind, cur()),
+        "few_rows_gated");
+}
+
 // y [rows, N] = W[e] a over expert-sorted rows; sorted_idx given: a's row of sorted row r is sorted_idx[r] / div
 // act_code: 0 none, 1 SwiGLU (w = [gate rows ; up rows]), 2 erf GELU
 // 3 the clamped gated unit (w = [gate rows ; up rows], limit), 4 squared ReLU
@@ -1415,6 +1457,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_router", &moe_router);
   m.def("moe_align", &moe_align);
   m.def("few_rows", &few_rows);
+  m.def("few_rows_gated", &few_rows_gated);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("moe_combine", &moe_combine);
   m.def("norm_shift", &norm_shift);

@@ -4,6 +4,7 @@
 //   own     a workgroup takes 16 columns, its four waves a quarter of K each with their own copies of the rows; the waves' sums meet in
 //           LDS in the order of K.  As many workgroups as there are column tiles.
 //   shared  a workgroup takes 64 columns and all of K, its four waves share the rows.
+#include "split_bf16.h"
 #include "stream_rows.h"
 
 namespace k8sllm {
@@ -128,6 +129,112 @@ __global__ __launch_bounds__(256) void few_rows_shared_kernel(RowsOut o, const b
     }
 }
 
+// Rows that are made here: the gated residual's sum and its norm (gated_add_norm_kernel, the same sums in the same order) are every workgroup's
+// prologue, behind the first loads of its weights, so the norm is no launch of its own.  Workgroup 0 writes the new residual, to a buffer of its own
+// (the others still read the old one).  What it costs is one round of loads, some 200 instructions a row and two barriers in each workgroup, against a
+// launch: few rows only.  us, norm and product / this, weights from memory: 1 row 3584 x 1024 5.9 / 4.4, 7168 x 2048 9.3 / 7.4, gated unit of 5632 + 2048
+// columns x 2048 15.3 / 11.3; 2 rows 3584 x 1024 5.9 / 4.6, 7168 x 2048 9.2 / 8.8; 4 rows 3584 x 1024 6.2 / 5.6, unit of 2816 + 1024 7.8 / 7.5, 7168 x
+// 2048 9.8 / 11.5; 1 row of 4096 columns 14336 x 4096 24.3 / 29.8.
+struct GatedRows {
+  const float* x;  // [M][Kd], and the new one
+  float* xn;
+  const bf16_t *y, *gate;  // [M][Kd]; rows g_stride apart
+  long g_stride;
+  const float *bias, *w;
+  float mult, eps;
+  int one_plus;
+};
+
+// KIND as above.  M <= MR rows of Kd <= 2048 / RP columns: RP rows at a time, each by 4 / RP waves.  As few_rows_own_kernel: 16 columns a workgroup,
+// its waves a quarter of K each.
+template <int KIND, int MR, int RP, bool ONCE>
+__global__ __launch_bounds__(256) void few_rows_gated_kernel(RowsOut o, GatedRows g, const bf16_t* __restrict__ W, int Kd) {
+  constexpr int NWV = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1, D = 4, P = MR / RP, RW = NWV / RP;
+  using S = HeldRows<NS, D, ONCE>;
+  __shared__ __attribute__((aligned(1024))) char smem[NWV * S::BYTES];
+  __shared__ __attribute__((aligned(16))) bf16_t xs[MR * (2048 / RP + 32)];
+  __shared__ float red[MR][RW];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), pitch = Kd + 32;
+  const int half = wave / RW, at = 8 * (threadIdx.x - 64 * RW * half), c = min(at, Kd - 8);  // a thread past the row's end adds nothing
+  float x[P][8], b[8], nw[8];
+  uint4 y[P], gt[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const long row = min(RP * p + half, o.M - 1);
+    load8(g.x + row * Kd + c, x[p]);
+    y[p] = *reinterpret_cast<const uint4*>(g.y + row * Kd + c);
+    gt[p] = *reinterpret_cast<const uint4*>(g.gate + row * g.g_stride + c);
+  }
+  load8(g.bias + c, b);
+  load8(g.w + c, nw);
+  int n[NS];
+  const bool pair = rows_tiles<KIND>(blockIdx.x, o.f, n);
+  const int per = ((Kd + 63) / 64 + NWV - 1) / NWV * 64, k0 = min(wave * per, Kd);  // a wave's k begin at a line
+  const int kd = min(per, Kd - k0);
+  LineSrc w[NS];
+#pragma unroll
+  for (int t = 0; t < NS; ++t) w[t] = line_src([&](int r) { return W + (long)min(n[t] + r, o.N - 1) * Kd + k0; });
+  char* ring = smem + wave * S::BYTES;
+  S::begin(ring, w, kd);
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int r = RP * p + half;
+    float ss = 0.f, a[8], z[8];
+    unpack8(y[p], a);
+    unpack8(gt[p], z);
+    if (at < Kd) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[p][i] += g.mult * a[i] * sigmoid_f(z[i] + b[i]);
+        ss += x[p][i] * x[p][i];
+      }
+      if (blockIdx.x == 0 && r < o.M) store8(g.xn + (long)r * Kd + c, x[p]);
+    }
+    ss = wave_sum(ss);
+    if (lane == 0) red[r][wave - RW * half] = ss;
+  }
+  lds_barrier();
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int r = RP * p + half;
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < RW; ++i) t += red[r][i];
+    const float inv = 1.0f / sqrtf(t / (float)Kd + g.eps);
+    if (at < Kd) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[p][i] *= inv * (g.one_plus ? 1.f + nw[i] : nw[i]);
+      *reinterpret_cast<uint4*>(xs + r * pitch + c) = pack8(x[p]);
+    }
+  }
+  lds_barrier();
+  f32x4 acc[NS] = {};
+  S::run(ring, w, xs + min(lane & 15, MR - 1) * pitch + k0 + 8 * (lane >> 4), kd, acc);
+  __syncthreads();  // the rings have been read
+  f32x4* sums = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+  for (int t = 0; t < NS; ++t) sums[(wave * NS + t) * 64 + lane] = acc[t];
+  __syncthreads();
+  // element i of lane l: row 4 (l / 16) + i, column l % 16: the rows are lanes 0 to 15's
+  const int l = threadIdx.x & 15, t = threadIdx.x >> 4;
+  if (t >= (pair ? 1 : NS)) return;
+  auto sum = [&](int q) {
+    f32x4 v = sums[q * 64 + l];
+#pragma unroll
+    for (int k = 1; k < NWV; ++k) v += sums[(k * NS + q) * 64 + l];
+    return v;
+  };
+  const f32x4 v = sum(t);
+  if (pair) {
+    const f32x4 u = sum(NS - 1);
+#pragma unroll
+    for (int j = 0; j < MR; ++j) rows_store_unit<KIND>(o, j, n[0] + l, v[j], u[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < MR; ++j) rows_store<KIND>(o, j, n[NS > 1 ? t : 0] + l, v[j]);
+  }
+}
+
 }  // namespace k8sllm
 
 using namespace k8sllm;
@@ -167,6 +274,39 @@ int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const vo
 #undef K8SLLM_FRM
 #undef K8SLLM_FR
 #undef K8SLLM_FRX
+  return (int)hipGetLastError();
+}
+
+// The same of rows made in the prologue (see GatedRows): x, y, xn [M][Kd] contiguous, 16-byte aligned, as are gate's rows, bias and w.
+int k8sllm_hy_few_rows_gated(void* y, void* yg, const float* x, float* xn, const void* add, const void* gate, long g_stride,
+                             const float* bias, float mult, const float* nw, float eps, int one_plus, const void* w, int M, int N, int Kd,
+                             int f, int kind, hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  const bool gated = kind >= 0;
+  if (M > 4 || Kd > (M > 2 ? 1024 : 2048) || Kd < 32 || Kd % 32 || g_stride % 8) return -1;
+  if (gated ? f <= 0 || f % 16 || N < 2 * f || yg == nullptr : f != 0) return -1;
+  const RowsOut o{y, (bf16_t*)yg, M, N, f, 0, 0.f};
+  const GatedRows g{x, xn, (const bf16_t*)add, (const bf16_t*)gate, g_stride, bias, nw, mult, eps, one_plus};
+  const unsigned tiles = (unsigned)(gated ? f / 16 + (N - 2 * f + 31) / 32 : (N + 15) / 16);
+  const bool once = read_once(2l * N * Kd, w, Kd);
+#define K8SLLM_FGX(KIND, MR, RP, ONCE) \
+  hipLaunchKernelGGL((few_rows_gated_kernel<KIND, MR, RP, ONCE>), dim3(tiles), dim3(256), 0, s, o, g, (const bf16_t*)w, Kd)
+#define K8SLLM_FGO(KIND, MR, RP)                 \
+  if (once) { K8SLLM_FGX(KIND, MR, RP, true); } \
+  else { K8SLLM_FGX(KIND, MR, RP, false); }
+#define K8SLLM_FG(KIND)                                   \
+  if (M == 1) { K8SLLM_FGO(KIND, 1, 1) }                  \
+  else if (Kd > 1024) { K8SLLM_FGO(KIND, 2, 1) }          \
+  else if (M == 2) { K8SLLM_FGO(KIND, 2, 2) }             \
+  else { K8SLLM_FGO(KIND, 4, 2) }
+  if (kind == -1) { K8SLLM_FG(-1) }
+  else if (kind == 1) { K8SLLM_FG(1) }
+  else if (kind == 3) { K8SLLM_FG(3) }
+  else if (kind == 4) { K8SLLM_FG(4) }
+  else return -1;
+#undef K8SLLM_FG
+#undef K8SLLM_FGO
+#undef K8SLLM_FGX
   return (int)hipGetLastError();
 }
 }

@@ -223,4 +223,68 @@ struct OwnRows {
   }
 };
 
+// The same with rows that lie in LDS whole (up to 16 of them, row r's k at xs + r * pitch; rows past the last read the last): only weights are
+// streamed.  begin() sends the first D lines on their way, run() takes them all.
+template <int NS, int D, bool ONCE>
+struct HeldRows {
+  static constexpr int BYTES = D * NS * 2048;
+
+  static __device__ __forceinline__ void issue(char* lds, const LineSrc (&w)[NS], int slot, int l, int kd) {
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int k = w[t].within(j, 64 * l, kd);
+        if constexpr (ONCE) w[t].once(lds + (slot * NS + t) * 2048, j, k);
+        else w[t].load(lds + (slot * NS + t) * 2048, j, k);
+      }
+  }
+  static __device__ __forceinline__ void begin(char* lds, const LineSrc (&w)[NS], int kd) {
+    if (kd <= 0) return;
+#pragma unroll
+    for (int d = 0; d < D; ++d) issue(lds, w, d, d, kd);
+  }
+  // x: this lane's row, at the first k of its chunk (lane / 16) of this part
+  static __device__ __forceinline__ void run(char* lds, const LineSrc (&w)[NS], const bf16_t* x, int kd, f32x4 (&acc)[NS]) {
+    if (kd <= 0) return;
+    const int rd = line_frag(), nl = (kd + 63) / 64;
+    int slot = 0;
+    auto consume = [&](int l) {
+      bf16x8 b[2][NS], a[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        a[j] = *reinterpret_cast<const bf16x8*>(x + min(64 * l + 32 * j, kd - 32));
+#pragma unroll
+        for (int t = 0; t < NS; ++t) b[j][t] = *reinterpret_cast<const bf16x8*>(lds + (slot * NS + t) * 2048 + (rd ^ (64 * j)));
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot may be refilled
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (j == 0 || 64 * l + 32 < kd) {
+#pragma unroll
+          for (int t = 0; t < NS; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], b[j][t], acc[t], 0, 0, 0);
+        }
+    };
+    int l = 0;
+    for (; l + D < nl; ++l) {
+      loads_left<2 * (D - 1) * NS>();
+      consume(l);
+      issue(lds, w, slot, l + D, kd);
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    auto rest = [&](auto self, auto dc) {
+      constexpr int d = decltype(dc)::value;
+      if constexpr (d < D) {
+        loads_left<2 * (D - 1 - d) * NS>();
+        if (l + d < nl) {
+          consume(l + d);
+          slot = slot + 1 == D ? 0 : slot + 1;
+        }
+        self(self, std::integral_constant<int, d + 1>{});
+      }
+    };
+    rest(rest, std::integral_constant<int, 0>{});
+  }
+};
+
 }  // namespace k8sllm

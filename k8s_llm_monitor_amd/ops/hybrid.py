@@ -315,6 +315,69 @@ def gated_add_norm(residual: torch.Tensor, y: torch.Tensor, proj: torch.Tensor, 
     return out
 
 
+class GatedRows:
+    """The rows that ``gated_add_norm`` would make, not made yet: the first ``linear`` or ``linear_glu`` of them has the sum and the norm as its
+    prologue (few_rows.hip) where there are few enough; anything else makes them first.  ``residual`` is the new residual behind that."""
+
+    def __init__(self, residual, y, proj, g_col, bias, mult, w, eps, one_plus, dtype):
+        self.args = (residual, y, proj, g_col, bias, mult, w, eps, one_plus)
+        self.dtype, self.shape, self.is_cuda, self.rows = dtype, residual.shape, True, None
+
+    @staticmethod
+    def take(residual: torch.Tensor, y: torch.Tensor, proj: torch.Tensor, g_col: int, *rest) -> bool:
+        """Whether the prologue is this sum's and norm's: bf16 on the device, everything in 16-byte pieces, no gradients."""
+        M, d = residual.shape
+        return (residual.is_cuda and 0 < M <= (4 if d <= 1024 else 2) and d <= 2048 and d % 32 == 0 and y.dtype == proj.dtype == torch.bfloat16
+                and residual.dtype == torch.float32 and residual.is_contiguous() and y.is_contiguous() and y.shape == residual.shape
+                and proj.dim() == 2 and proj.stride(1) == 1 and proj.stride(0) % 8 == 0 and g_col % 8 == 0
+                and all(t.data_ptr() % 16 == 0 for t in (residual, y, proj, rest[0], rest[2]))
+                and not (torch.is_grad_enabled() and any(t.requires_grad for t in (residual, y, proj, rest[0], rest[2]))))
+
+    @property
+    def residual(self) -> torch.Tensor:
+        if self.rows is None and not self.done:
+            self.tensor()
+        return self.new
+
+    done, new = False, None
+
+    def tensor(self) -> torch.Tensor:
+        """The rows as a tensor (the residual is updated in place if no product has made a new one)."""
+        if self.rows is None:
+            if self.done:
+                self.rows = add_norm(self.new, (), None, self.args[6], self.args[7], self.args[8], self.dtype)
+            else:
+                self.rows, self.new = gated_add_norm(*self.args, self.dtype), self.args[0]
+        return self.rows
+
+    def product(self, w: torch.Tensor, f: int = 0, kind: str = "") -> Optional[tuple]:
+        """(unit or None, product of the other rows of w) with the rows made on the way; None: this product is not the prologue's."""
+        x, y, proj, g_col, bias, mult, nw, eps, one_plus = self.args
+        M = x.shape[0]
+        if (self.done or self.rows is not None or w.dtype != torch.bfloat16 or w.dim() != 2 or not w.is_contiguous() or w.data_ptr() % 16
+                or w.shape[1] != x.shape[1] or (torch.is_grad_enabled() and w.requires_grad)
+                or _rows_form(M, w.shape[0], w.shape[1], "glu" if f else "") is None or w.shape[0] > GATED_COLUMNS):
+            return None
+        a = torch.empty(M, f, dtype=self.dtype, device=x.device) if f else None
+        z = torch.empty(M, w.shape[0] - 2 * f, dtype=self.dtype, device=x.device)
+        self.new, self.done = torch.empty_like(x), True
+        native().few_rows_gated(z, a, x, self.new, y, proj, int(g_col), bias, float(mult), nw, float(eps), bool(one_plus), w,
+                                ACTS[kind] if f else -1)
+        return a, z
+
+
+GATED_COLUMNS = 16384
+
+
+def gated_rows(residual: torch.Tensor, y: torch.Tensor, proj: torch.Tensor, g_col: int, bias: torch.Tensor, mult: float, w: torch.Tensor,
+               eps: float, one_plus: bool, out_dtype: torch.dtype):
+    """``gated_add_norm``, or the GatedRows of it where a product can make them."""
+    args = (residual, y, proj, g_col, bias, mult, w, eps, one_plus)
+    if out_dtype == torch.bfloat16 and GatedRows.take(*args):
+        return GatedRows(*args, out_dtype)
+    return gated_add_norm(*args, out_dtype)
+
+
 def norm_shift(residual: torch.Tensor, addends: tuple, w: torch.Tensor, eps: float, one_plus: bool,
                mu: torch.Tensor, state: torch.Tensor, seg_cu: torch.Tensor, seg_ctx: torch.Tensor,
                seg_slot: torch.Tensor, out_dtype: torch.dtype, advance: bool = True,
@@ -1362,6 +1425,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x`` [T, K] times ``w`` [N, K] transposed.  The BLAS library's product, but for bf16 on the device with rows 16-byte aligned: the
     few rows of a decode step, K a multiple of 32, where a call takes what it takes to get enough loads in flight
     (few_rows.hip, by the rule of ``_rows_form``), and large products by the rule of ``_tile_plain``."""
+    if isinstance(x, GatedRows):
+        made = x.product(w)
+        if made is not None:
+            return made[1]
+        x = x.tensor()
     form = _few_rows(x, w)
     if form is not None:
         y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
@@ -1425,6 +1493,11 @@ def linear_glu(x: torch.Tensor, w: torch.Tensor, f: int, kind: str) -> tuple:
     """The gated unit ``act(gate x) * (up x)`` [T, f] of ``w``'s rows [f gate | f up | the rest], and a projection with the column
     at which the rest's outputs begin in it.  ``linear`` and ``glu``, in one launch for the rows that few_rows.hip takes and for large
     steps (by the rule of ``_tile_form``)."""
+    if isinstance(x, GatedRows):
+        made = x.product(w, f, kind) if f > 0 and f % 16 == 0 and kind in GLU_ENDS else None
+        if made is not None:
+            return (*made, 0)
+        x = x.tensor()
     if f > 0 and kind in GLU_ENDS and _tile_unit(x, w, f):
         from .. import ops
 
