@@ -614,9 +614,8 @@ class LightningMixer:
 
     def forward(self, h: torch.Tensor, meta: AttnMeta, cache: dict, rows=None) -> torch.Tensor:
         proj = hops.linear(h, self.w_in)
-        vkq = hops.activation_cols(proj, 0, self.n_act, "silu")
-        o = hops.linear_attention(vkq, self.decay, cache["state"], meta.seg_cu, meta.seg_ctx, meta.seg_slot,
-                                  self.H, self.dk, self.dv, longest=meta.seg_max, singles=meta.num_decode)
+        o = hops.linear_attention(proj, self.decay, cache["state"], meta.seg_cu, meta.seg_ctx, meta.seg_slot,
+                                  self.H, self.dk, self.dv, longest=meta.seg_max, singles=meta.num_decode, silu=True)
         o, proj = _take(rows, o, proj)
         if self.n_tail:
             self.tail_out = (proj, self.n_in)

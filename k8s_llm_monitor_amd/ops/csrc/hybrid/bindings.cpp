@@ -70,6 +70,8 @@ int k8sllm_hy_ssm_scan(float* y, const void* xbc, const void* proj, long p_strid
                        const float* a_log, const float* d_skip, const float* decay, float* state, const int* cu,
                        const int* ctx, const int* slot, int S, long T, int nh, int P, int N, int G, int f32, int mode,
                        hipStream_t s);
+int k8sllm_hy_linear_step(float* y, const void* proj, long x_stride, const float* decay, float* state, const int* cu, const int* ctx,
+                          const int* slot, int S, int H, int dk, int dv, int f32, hipStream_t s);
 int k8sllm_hy_selective_scan(void* out, const void* xc, const void* q, long q_stride, int b_col, int c_col,
                              const void* dt, long dt_stride, const float* dt_bias, const float* a_log, const float* d_skip,
                              const void* z, long z_stride, float* state, const int* cu, const int* ctx, const int* slot,
@@ -648,6 +650,27 @@ void ssm_scan(Tensor y, Tensor xbc, OptT proj, int64_t dt_col, OptT dt_bias, Opt
     }
   }
   scan(S, T, mode == 3 ? 0 : mode);
+}
+
+// Linear attention of one token a segment, v, k and q read through SiLU from the projection's first columns; false: not these sizes, nothing was launched
+bool linear_step(Tensor y, Tensor proj, Tensor decay, Tensor state, Tensor cu, Tensor ctx, Tensor slot, int64_t H, int64_t dk, int64_t dv) {
+  const int f = act(proj, "proj");
+  f32c(y, "y");
+  f32c(state, "state");
+  f32c(decay, "decay");
+  segs(cu, ctx, slot);
+  const int64_t T = proj.size(0), S = ctx.numel();
+  TORCH_CHECK(proj.dim() == 2 && proj.stride(1) == 1 && proj.size(1) >= H * (2 * dk + dv), "proj [T, H*dv | H*dk | H*dk | ...]");
+  TORCH_CHECK(y.numel() == T * H * dv && decay.numel() == H && state.dim() == 4 && state.size(1) == H && state.size(2) == dk &&
+                  state.size(3) == dv,
+              "linear_step: y [T, H*dv], decay [H], state [slots, H, dk, dv]");
+  if (T > S) return false;
+  const int rc = k8sllm_hy_linear_step(y.data_ptr<float>(), proj.data_ptr(), proj.stride(0), decay.data_ptr<float>(), state.data_ptr<float>(),
+                                       cu.data_ptr<int>(), ctx.data_ptr<int>(), slot.data_ptr<int>(), (int)S, (int)H, (int)dk, (int)dv, f,
+                                       cur());
+  if (rc == 1) return false;
+  check(rc, "linear_step");
+  return true;
 }
 
 // In place on the fused rows [T, Hq*dk | G*dk | G*dv | ...]: rotary positions on the first 2 * len(freq)
@@ -1454,6 +1477,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("window_attention_decode", &window_attention_decode);
   m.def("conv_silu", &conv_silu);
   m.def("ssm_scan", &ssm_scan);
+  m.def("linear_step", &linear_step);
   m.def("moe_router", &moe_router);
   m.def("moe_align", &moe_align);
   m.def("few_rows", &few_rows);

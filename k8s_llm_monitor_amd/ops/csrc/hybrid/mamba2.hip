@@ -382,14 +382,16 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(float* __restrict__ y, co
 // accesses met 64 bytes of a row, behind the staging of tiles of 16 tokens.
 // us, ssm_scan_kernel / here: 64 heads of 64 x 128, 1 segment 9.5 / 4.6, 16 22.6 / 14.5, 64 75.7 / 49.0 (5.5 TB/s), 128 129 / 98;
 // 16 heads of 128 x 128 with a fixed decay, 1 segment 8.4 / 3.6, 32 19.5 / 14.1; 64 of them 40.2 / 26.8.  States above 8 MB of a step are
-// non-temporal: at 34 MB 18.6 / 14.5.
+// non-temporal: at 34 MB 18.6 / 14.5.  silu: rows of a projection, read through SiLU and rounded as its own launch leaves them (us, both
+// launches / this: 8 heads of 128 x 128, 1 sequence 5.4 / 4.2, 64 13.2 / 11.1; 32 heads, 16 sequences 12.7 / 11.0).
 template <typename T, int NPT, bool ONCE>
 __global__ __launch_bounds__(256) void ssm_step_kernel(float* __restrict__ y, const T* __restrict__ xbc, const T* __restrict__ proj,
                                                        long p_stride, int dt_col, const float* __restrict__ dt_bias,
                                                        const float* __restrict__ a_log, const float* __restrict__ d_skip,
                                                        const float* __restrict__ decay, float* __restrict__ state,
                                                        const int* __restrict__ cu, const int* __restrict__ ctx,
-                                                       const int* __restrict__ slot, int nh, int P, int N, int G) {
+                                                       const int* __restrict__ slot, int nh, int P, int N, int G, long x_stride,
+                                                       int silu) {
   constexpr int GPT = NPT <= 16 ? 1 : NPT / 16;  // groups of a thread
   __shared__ __attribute__((aligned(16))) float part[16 * GPT][68];
   const int s = blockIdx.x, h = blockIdx.y, sl = slot[s], t0 = cu[s], t1 = cu[s + 1];
@@ -401,7 +403,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(float* __restrict__ y, co
     return;
   }
   if (t1 <= t0) return;
-  const int inner = nh * P, C = inner + 2 * G * N, g = h / (nh / G), pc = min(p4, P - 4);
+  const int inner = nh * P, g = h / (nh / G), pc = min(p4, P - 4);
   float* sp = state + ((long)sl * nh + h) * N * P + pc;
   int n[GPT];
 #pragma unroll
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(float* __restrict__ y, co
   const bool fixed = decay != nullptr;
   const float A = fixed ? 0.f : expf(a_log[h]), Dh = fixed ? 0.f : d_skip[h], bias = fixed ? 0.f : dt_bias[h];
   for (int t = t0; t < t1; ++t) {
-    const T* row = xbc + (long)t * C;
+    const T* row = xbc + (long)t * x_stride;
     float x[4], b[GPT][4], c[GPT][4];
     load4(row + (long)h * P + pc, x);
 #pragma unroll
@@ -424,6 +426,22 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(float* __restrict__ y, co
       load4(row + inner + (long)(G + g) * N + n[i], c[i]);
     }
     const float xl = ldf(row + (long)h * P + min(p, P - 1));
+    if (silu) {
+      auto unit = [](float (&v)[4]) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          T r;
+          stf(&r, act_f<3>(v[k], 0.f, 0.f));
+          v[k] = ldf(&r);
+        }
+      };
+      unit(x);
+#pragma unroll
+      for (int i = 0; i < GPT; ++i) {
+        unit(b[i]);
+        unit(c[i]);
+      }
+    }
     float dt = 1.f, dA;
     if (fixed) {
       dA = decay[h];
@@ -827,6 +845,31 @@ __global__ __launch_bounds__(256, 2) void ssm_scan_tile_kernel(float* __restrict
 
 using namespace k8sllm;
 
+// one token a segment, rows that the step kernel can read four values at a time (some: groups behind the last repeat it)
+template <typename T>
+static bool step_sizes(const void* xbc, const float* state, int P, int N) {
+  return P % 4 == 0 && N % 4 == 0 && N > 0 && N <= 256 && reinterpret_cast<uintptr_t>(state) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(xbc) % (4 * sizeof(T)) == 0;
+}
+template <typename T>
+static int launch_step(float* y, const void* xbc, long x_stride, int silu, const void* proj, long p_stride, int dt_col, const float* dt_bias,
+                       const float* a_log, const float* d_skip, const float* decay, float* state, const int* cu, const int* ctx,
+                       const int* slot, int S, int nh, int P, int N, int G, hipStream_t s) {
+  const dim3 grid((unsigned)S, (unsigned)nh, (unsigned)((P + 63) / 64));
+  const bool once = 4l * S * nh * N * P > kStateOnceBytes;
+#define K8SLLM_STEP(NPT)                                                                                                 \
+  hipLaunchKernelGGL((once ? &ssm_step_kernel<T, NPT, true> : &ssm_step_kernel<T, NPT, false>), grid, dim3(256), 0, s, y,  \
+                     (const T*)xbc, (const T*)proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot, nh, \
+                     P, N, G, x_stride, silu)
+  if (N <= 16) K8SLLM_STEP(4);
+  else if (N <= 32) K8SLLM_STEP(8);
+  else if (N <= 64) K8SLLM_STEP(16);
+  else if (N <= 128) K8SLLM_STEP(32);
+  else K8SLLM_STEP(64);
+#undef K8SLLM_STEP
+  return (int)hipGetLastError();
+}
+
 template <typename T>
 static int launch_scan(float* y, const void* xbc, const void* proj, long p_stride, int dt_col, const float* dt_bias,
                        const float* a_log, const float* d_skip, const float* decay, float* state, const int* cu, const int* ctx,
@@ -861,22 +904,9 @@ static int launch_scan(float* y, const void* xbc, const void* proj, long p_strid
     return (int)hipGetLastError();
   }
   const dim3 grid((unsigned)S, (unsigned)nh, (unsigned)((P + 63) / 64));
-  // one token a segment, rows that the step kernel can read four values at a time (some: groups behind the last repeat it)
-  if (step && P % 4 == 0 && N % 4 == 0 && N > 0 && N <= 256 && reinterpret_cast<uintptr_t>(state) % 16 == 0 &&
-      reinterpret_cast<uintptr_t>(xbc) % (4 * sizeof(T)) == 0) {
-    const bool once = 4l * S * nh * N * P > kStateOnceBytes;
-#define K8SLLM_STEP(NPT)                                                                                                 \
-  hipLaunchKernelGGL((once ? &ssm_step_kernel<T, NPT, true> : &ssm_step_kernel<T, NPT, false>), grid, dim3(256), 0, s, y,  \
-                     (const T*)xbc, (const T*)proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot, nh, \
-                     P, N, G)
-    if (N <= 16) K8SLLM_STEP(4);
-    else if (N <= 32) K8SLLM_STEP(8);
-    else if (N <= 64) K8SLLM_STEP(16);
-    else if (N <= 128) K8SLLM_STEP(32);
-    else K8SLLM_STEP(64);
-#undef K8SLLM_STEP
-    return (int)hipGetLastError();
-  }
+  if (step && step_sizes<T>(xbc, state, P, N))
+    return launch_step<T>(y, xbc, nh * P + 2l * G * N, 0, proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot, S, nh,
+                          P, N, G, s);
 #define K8SLLM_SCAN(NPT)                                                                                              \
   hipLaunchKernelGGL((ssm_scan_kernel<T, NPT>), grid, dim3(256), 0, s, y, (const T*)xbc, (const T*)proj, p_stride,    \
                      dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot, nh, P, N, G)
@@ -942,5 +972,14 @@ int k8sllm_hy_ssm_scan(float* y, const void* xbc, const void* proj, long p_strid
                                   S, nh, P, N, G, wide, step, s)
              : launch_scan<bf16_t>(y, xbc, proj, p_stride, dt_col, dt_bias, a_log, d_skip, decay, state, cu, ctx, slot,
                                    S, nh, P, N, G, wide, step, s);
+}
+
+// Linear attention of one token a segment (T <= S), v, k and q the SiLU of a projection's first columns, rows x_stride apart.  1: not these sizes.
+int k8sllm_hy_linear_step(float* y, const void* proj, long x_stride, const float* decay, float* state, const int* cu, const int* ctx,
+                          const int* slot, int S, int H, int dk, int dv, int f32, hipStream_t s) {
+  if (S <= 0) return 0;
+  if (x_stride % 4 || !(f32 ? step_sizes<float>(proj, state, dv, dk) : step_sizes<bf16_t>(proj, state, dv, dk))) return 1;
+  return f32 ? launch_step<float>(y, proj, x_stride, 1, nullptr, 0, 0, nullptr, nullptr, nullptr, decay, state, cu, ctx, slot, S, H, dv, dk, H, s)
+             : launch_step<bf16_t>(y, proj, x_stride, 1, nullptr, 0, 0, nullptr, nullptr, nullptr, decay, state, cu, ctx, slot, S, H, dv, dk, H, s);
 }
 }

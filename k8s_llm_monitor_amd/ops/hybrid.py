@@ -1031,12 +1031,13 @@ def ssm_scan(xbc: torch.Tensor, proj: Optional[torch.Tensor], dt_col: int, dt_bi
 
 def linear_attention(vkq: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, seg_cu: torch.Tensor,
                      seg_ctx: torch.Tensor, seg_slot: torch.Tensor, H: int, dk: int, dv: int, mode: int = 0,
-                     col_tiles: int = 0, longest: int = 0, singles: int = 0) -> torch.Tensor:
+                     col_tiles: int = 0, longest: int = 0, singles: int = 0, silu: bool = False) -> torch.Tensor:
     """Linear attention with a fixed decay per head, as a recurrence over each segment:
 
         S_t = decay[h] S_(t-1) + k_t v_t^T;   o_t = S_t^T q_t
 
-    ``vkq`` [T, H*dv | H*dk | H*dk] holds v, k, q head by head (contiguous); ``state`` [slots, H, dk,
+    ``vkq`` [T, H*dv | H*dk | H*dk] holds v, k, q head by head (contiguous; ``silu``: they are the SiLU of a wider projection's first
+    columns, which steps of one token a segment form where they read them); ``state`` [slots, H, dk,
     dv] fp32 is read at a segment's start (zero where seg_ctx is 0) and written back at its end.
     Returns o [T, H*dv] fp32.  State, products and sums are fp32.
 
@@ -1047,6 +1048,13 @@ def linear_attention(vkq: torch.Tensor, decay: torch.Tensor, state: torch.Tensor
     segment's first row on.  The first ``singles`` segments, running sequences' next tokens, stay on the scan of a decode step
     beside them.  Else the sequential scan (``ssm_scan`` with the decay
     table; ``mode`` 1 / 2 force its decode / prompt lane mapping)."""
+    if silu:
+        T = vkq.shape[0]
+        if vkq.is_cuda and mode == 0 and T <= seg_ctx.numel():
+            y = torch.empty(T, H * dv, dtype=torch.float32, device=vkq.device)
+            if native().linear_step(y, vkq, decay, state, seg_cu, seg_ctx, seg_slot, int(H), int(dk), int(dv)):
+                return y
+        vkq = activation_cols(vkq, 0, H * (2 * dk + dv), "silu")
     return ssm_scan(vkq, None, 0, None, None, None, state, seg_cu, seg_ctx, seg_slot, H, dv, dk, H, mode, decay=decay,
                     col_tiles=col_tiles, longest=longest, singles=singles)
 

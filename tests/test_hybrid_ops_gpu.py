@@ -511,3 +511,29 @@ def test_products_of_gated_rows(M, d, N, f, kind):
         k = bad.get("rows", 1)
         r = H.gated_rows(x_want.repeat(k, 1), bad.get("y", y).repeat(k, 1), proj.repeat(k, 1), bad.get("g_col", 16), *args[3:], dt)
         assert isinstance(r, torch.Tensor)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("S,heads,dk,dv,wide", [(1, 8, 128, 128, 2048), (5, 3, 36, 20, 40), (33, 2, 64, 132, 0)])
+def test_linear_attention_step_through_silu(dt, S, heads, dk, dv, wide):
+    """Steps of one token a segment read a projection through SiLU: the bits of the activation's own launch and the step behind it, padding and fresh
+    sequences among them; other widths and steps of more tokens take that launch."""
+    g = _g(37)
+    n = heads * (2 * dk + dv)
+    proj, state = _r(g, S, n + wide, dt=dt).cuda(), _r(g, S + 1, heads, dk, dv).cuda()
+    dec = (torch.rand(heads, generator=g) * 0.5 + 0.5).cuda()
+    cu, ctx, slot = _i32(list(range(S + 1))).cuda(), _i32([7 * (i != 2) for i in range(S)]).cuda(), _i32([i if i != 1 else -1 for i in range(S)]).cuda()
+    s1, s2 = state.clone(), state.clone()
+    want = _lin(_silu_cols(proj, n), dec, s1, cu, ctx, slot, heads, dk, dv)
+    got = _lin(proj, dec, s2, cu, ctx, slot, heads, dk, dv, silu=True)
+    assert torch.equal(got, want) and torch.equal(s1, s2) and not torch.equal(s1, state)
+    cu2, two = _i32([0, 2] + list(range(3, S + 2))).cuda(), torch.cat([proj[:1], proj])
+    assert torch.equal(_lin(two, dec, s1, cu2, ctx, slot, heads, dk, dv, silu=True), _lin(_silu_cols(two, n), dec, s2, cu2, ctx, slot, heads, dk, dv))
+
+
+def _silu_cols(proj, n):
+    return H.activation_cols(proj, 0, n, "silu")
+
+
+def _lin(*a, **k):
+    return H.linear_attention(*a, **k)
