@@ -53,11 +53,13 @@ __device__ __forceinline__ bool rows_tiles(int j, int f, int (&n)[KIND >= 0 && K
   }
 }
 
-template <int KIND, int MT, bool ONCE>
+// ONCE, TURN: the weights non-temporal, and from a k of the workgroup's own on (a kernel of its own: the address of a line that is not
+// turned costs a small product 0.15 us otherwise)
+template <int KIND, int MT, bool ONCE, bool TURN = false>
 __global__ __launch_bounds__(256) void few_rows_own_kernel(RowsOut o, const bf16_t* __restrict__ X, long x_stride,
                                                            const bf16_t* __restrict__ W, int Kd) {
   constexpr int NWV = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1, D = MT <= 2 ? 4 : 2, NT = MT * NS;
-  using S = OwnRows<MT, NS, D, ONCE>;
+  using S = OwnRows<MT, NS, D, ONCE, TURN>;
   static_assert(NT <= S::BYTES / 1024, "");
   __shared__ __attribute__((aligned(1024))) char smem[NWV * S::BYTES];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -70,7 +72,7 @@ __global__ __launch_bounds__(256) void few_rows_own_kernel(RowsOut o, const bf16
 #pragma unroll
   for (int m = 0; m < MT; ++m) src[NS + m] = line_src([&](int r) { return X + (long)min(16 * m + r, o.M - 1) * x_stride + k0; });
   f32x4 acc[MT][NS] = {};
-  S::run(smem + wave * S::BYTES, src, min(per, Kd - k0), acc);
+  S::run(smem + wave * S::BYTES, src, min(per, Kd - k0), acc, TURN ? 4 * first_piece(blockIdx.x, per / 256) : 0);
   __syncthreads();  // the rings have been read
   f32x4* red = reinterpret_cast<f32x4*>(smem);
 #pragma unroll
@@ -99,11 +101,11 @@ __global__ __launch_bounds__(256) void few_rows_own_kernel(RowsOut o, const bf16
   }
 }
 
-template <int KIND, int MT, bool ONCE>
+template <int KIND, int MT, bool ONCE, bool TURN = false>
 __global__ __launch_bounds__(256) void few_rows_shared_kernel(RowsOut o, const bf16_t* __restrict__ X, long x_stride,
                                                               const bf16_t* __restrict__ W, int Kd) {
   constexpr int NW = 4, NS = KIND >= 0 && KIND < 16 ? 2 : 1;
-  using S = SharedRows<MT, NS, NW, ONCE>;
+  using S = SharedRows<MT, NS, NW, ONCE, TURN>;
   __shared__ __attribute__((aligned(1024))) char smem[S::BYTES];
   int n[NS];
   const bool pair = rows_tiles<KIND>(blockIdx.x * NW + (threadIdx.x >> 6), o.f, n);
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(256) void few_rows_shared_kernel(RowsOut o, const b
   f32x4 acc[MT][NS] = {};
   S::run(smem, [&](int m) {
     return line_src([&](int r) { return X + (long)min(16 * m + r, o.M - 1) * x_stride; });
-  }, w, Kd, acc);
+  }, w, Kd, acc, TURN ? first_piece(blockIdx.x, Kd / 256) : 0);
   const int c = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int m = 0; m < MT; ++m)
@@ -253,12 +255,16 @@ int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const vo
   // (shared, 16 rows, 10240 x 384, us, non-temporal / as usual: 15 such weights in turn, which the memory-side cache holds, 5.3 / 4.5; 100 of them, from
   // memory, 5.0 / 5.3; 12288 x 320 4.8 / 4.3, 4.5 / 4.75)
   const bool once = read_once(2l * N * Kd, w, Kd);
+  // workgroups begin at k of their own (first_piece) where a wave's rows, or its quarters of them, are whole periods of the channels
+  const bool turn = once && Kd % (shared ? kTurnBytes / 2 : 2 * kTurnBytes) == 0;
 #define K8SLLM_FRX(KERNEL, GRID) \
   hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, (const bf16_t*)w, Kd)
-#define K8SLLM_FR(KIND, MT)                                                                    \
-  if (shared && once) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT, true>), (tiles + 3) / 4);   \
-  else if (shared) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT, false>), (tiles + 3) / 4);     \
-  else if (once) K8SLLM_FRX((few_rows_own_kernel<KIND, MT, true>), tiles);                     \
+#define K8SLLM_FR(KIND, MT)                                                                                \
+  if (shared && turn) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT, true, true>), (tiles + 3) / 4);         \
+  else if (shared && once) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT, true>), (tiles + 3) / 4);          \
+  else if (shared) K8SLLM_FRX((few_rows_shared_kernel<KIND, MT, false>), (tiles + 3) / 4);                 \
+  else if (turn) K8SLLM_FRX((few_rows_own_kernel<KIND, MT, true, true>), tiles);                           \
+  else if (once) K8SLLM_FRX((few_rows_own_kernel<KIND, MT, true>), tiles);                                 \
   else K8SLLM_FRX((few_rows_own_kernel<KIND, MT, false>), tiles)
 #define K8SLLM_FRM(KIND)              \
   if (M <= 16) { K8SLLM_FR(KIND, 1); } \

@@ -64,6 +64,12 @@ struct LineSrc {
   __device__ __forceinline__ void load(char* lds, int i, int k) const { load_piece(lds + 1024 * i, p[i] + k); }
   __device__ __forceinline__ void once(char* lds, int i, int k) const { load_piece_once(lds + 1024 * i, p[i] + k); }
 };
+// Where workgroup b begins among n pieces of its rows, so that those that run side by side are not at the same k: with rows of weights whole
+// periods of the channels apart (4 KB), every workgroup's lines of one k lie in the same channels of its XCD's L2 and of memory.  us, all from k = 0 /
+// so: shared form, 24 rows 16384 x 4096 26.8 / 22.8, x 8192 54 / 45, 32000 x 4096 47 / 43, 64 rows 54 / 49; own form, 1 row 4096 x 16384 26.0 / 22.1,
+// 8192 x 16384 50 / 42; 16384 x 4160, which needs it not, 23.3.  The order of the fp32 sums follows it: what must keep its sums' order begins at 0.
+constexpr int kTurnBytes = 4096;
+__device__ __forceinline__ int first_piece(int b, int n) { return ((b >> 3) + (b & 7)) % n; }
 // row(r): where row r (of 16) begins
 template <class R>
 __device__ __forceinline__ LineSrc line_src(R row) {
@@ -73,7 +79,7 @@ __device__ __forceinline__ LineSrc line_src(R row) {
 // NW waves of one workgroup share 16 MT rows, which come in chunks of 4 lines to a ring of two; each wave streams its own NS
 // weight tiles through a private ring, 4 lines ahead.  Every output is one chain of products in the order of k.  ONCE: the
 // weights' loads are non-temporal.
-template <int MT, int NS, int NW, bool ONCE>
+template <int MT, int NS, int NW, bool ONCE, bool TURN = false>
 struct SharedRows {
   static constexpr int D = 4;  // lines of a chunk, and of the weights' ring
   static constexpr int SLOT = D * MT * 2048, RING = D * NS * 2048, BYTES = 2 * SLOT + NW * RING;
@@ -81,9 +87,12 @@ struct SharedRows {
   static constexpr int P = NW / MT, PER = 2 * D / P, HALVES = P == 1 ? 2 : 1, EVERY = P > 2 ? P / 2 : 1;
   static_assert(NW % MT == 0 && P <= 4, "");
 
-  // x(m): this lane's sources in row tile m of the rows; w[t]: in weight tile t; kd: a multiple of 32
+  // x(m): this lane's sources in row tile m of the rows; w[t]: in weight tile t; kd: a multiple of 32; TURN: of whole
+  // chunks, of which c0 is the first to be taken (first_piece)
   template <class X>
-  static __device__ __forceinline__ void run(char* lds, X x, const LineSrc (&w)[NS], int kd, f32x4 (&acc)[MT][NS]) {
+  static __device__ __forceinline__ void run(char* lds, X x, const LineSrc (&w)[NS], int kd, f32x4 (&acc)[MT][NS], int c0 = 0) {
+    const int nc = kd / (64 * D);
+    auto at = [&](int c) { return !TURN ? c : c + c0 >= nc ? c + c0 - nc : c + c0; };
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rd = line_frag(), nl = (kd + 63) / 64;
     const int m0 = wave % MT, h0 = (wave / MT) & (P > 1 ? 1 : 0), u0 = P > 2 ? wave / MT / 2 : 0;
     const LineSrc xs = x(m0);
@@ -94,12 +103,13 @@ struct SharedRows {
 #pragma unroll
         for (int j = 0; j < HALVES; ++j) {
           const int u = u0 + i * EVERY, h = HALVES == 1 ? h0 : j;
-          const int k = 64 * (c * D + u);
+          const int k = 64 * (at(c) * D + u);
           load_piece(lds + (c & 1) * SLOT + (u * MT + m0) * 2048 + 1024 * h,
                      (h ? xs.p[1] : xs.p[0]) + (decltype(whole)::value ? k : xs.within(h, k, kd)));
         }
     };
-    auto refill = [&](int u, int l, auto whole) {
+    auto refill = [&](int u, int c, auto whole) {
+      const int l = at(c) * D + u;
 #pragma unroll
       for (int t = 0; t < NS; ++t)
 #pragma unroll
@@ -132,7 +142,7 @@ struct SharedRows {
                 a[j][m] = *reinterpret_cast<const bf16x8*>(lds + (c & 1) * SLOT + (u * MT + m) * 2048 + (rd ^ (64 * j)));
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            if (WHOLE || (c + 1) * D + u < nl) refill(u, (c + 1) * D + u, whole);
+            if (WHOLE || (c + 1) * D + u < nl) refill(u, c + 1, whole);
 #pragma unroll
             for (int j = 0; j < 2; ++j)
               if (j == 0 || WHOLE || 64 * (c * D + u) + 32 < kd) {
@@ -150,7 +160,7 @@ struct SharedRows {
     };
     stage(0, std::false_type{});
 #pragma unroll
-    for (int u = 0; u < D; ++u) refill(u, u, std::false_type{});
+    for (int u = 0; u < D; ++u) refill(u, 0, std::false_type{});
     int c = 0;
     for (; 64 * (c + 2) * D <= kd; ++c) chunk(c, std::true_type{});
     for (; c * D < nl; ++c) chunk(c, std::false_type{});
@@ -158,15 +168,18 @@ struct SharedRows {
 };
 
 // One wave streams 16 MT rows and NS weight tiles, its own part of K, through a private ring D lines deep: no barrier.
-template <int MT, int NS, int D, bool ONCE>
+template <int MT, int NS, int D, bool ONCE, bool TURN = false>
 struct OwnRows {
   static constexpr int L = MT + NS, BYTES = D * L * 2048;
 
-  // src: this lane's sources, weight tiles first; kd: k of this part, a multiple of 32
-  static __device__ __forceinline__ void run(char* lds, const LineSrc (&src)[L], int kd, f32x4 (&acc)[MT][NS]) {
+  // src: this lane's sources, weight tiles first; kd: k of this part, a multiple of 32; TURN: of whole lines, of
+  // which l0 is the first to be taken (first_piece)
+  static __device__ __forceinline__ void run(char* lds, const LineSrc (&src)[L], int kd, f32x4 (&acc)[MT][NS], int l0 = 0) {
     if (kd <= 0) return;
     const int rd = line_frag(), nl = (kd + 63) / 64;
-    auto issue = [&](int slot, int l, auto whole) {
+    auto at = [&](int l) { return !TURN || l >= nl ? l : l + l0 >= nl ? l + l0 - nl : l + l0; };
+    auto issue = [&](int slot, int line, auto whole) {
+      const int l = at(line);
 #pragma unroll
       for (int i = 0; i < L; ++i)
 #pragma unroll

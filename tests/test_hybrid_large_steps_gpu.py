@@ -738,6 +738,19 @@ def test_gradients_of_few_rows_products(M):
             assert not f(xg, wg).requires_grad
 
 
+@pytest.mark.parametrize("M", [1, 24, 64])
+@pytest.mark.parametrize("N,K,shared", [(2056, 2048, True), (1544, 4096, True), (520, 8192, False), (264, 16384, False), (1100, 16384, True)])
+def test_few_rows_from_a_k_of_their_own(M, N, K, shared):
+    """Weights above 8 MB with rows of whole 4 KB: each workgroup begins at another k.  Against 64 bits, fp32 sums of K products and one rounding; the
+    columns' workgroups are more than the pieces of K and end inside a tile."""
+    g = _g(75)
+    x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
+    y = torch.empty(M, N, dtype=BF, device="cuda")
+    hops.native().few_rows(y, None, x, w, -1, 0.0, shared)
+    want = x.double() @ w.double().t()
+    assert bool(((y.double() - want).abs() <= 2 ** -8 * want.abs() + 1e-6 * K ** 0.5).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(4, 72, 6144), (5, 72, 6144), (2, 72, 6176), (3, 4096, 4128), (3, 4104, 4128), (16, 8200, 1056), (17, 8184, 1056),
                                    (32, 72, 4096), (33, 72, 4096), (33, 2048, 2048), (33, 2064, 2048), (64, 1024, 96), (65, 1024, 96),
                                    (16, 8192, 4096), (16, 10240, 4096), (64, 16384, 64), (64, 16400, 64)])
