@@ -71,6 +71,24 @@ __device__ __forceinline__ ChunkAt chunk_at(const int* __restrict__ cu, int S, i
   return {-1, 0, 0, 0, 0};
 }
 
+// Which segment the r-th group of workgroups takes, where one workgroup a compute unit is `round` groups: the longest ones first, one a unit, then
+// the shortest first, which come beside them (workgroups go to the units in turn), and so on.  A chain of tokens beside another takes up to twice as
+// long, so that a step of prompts of different lengths took as long as its two longest ones on one unit: 13 prompts of 45 to 901 tokens, us, in the
+// step's order / so: selective scan of 2048 channels 144 / 126, delta rule of 8 heads 72 / 58, wkv of 16 50 / 43.  More than 64 segments: from
+// the last one on (a step's prompts come after its running sequences).
+__device__ __forceinline__ int segment_in_turn(const int* __restrict__ cu, int S, int r, int round) {
+  if (S <= 1 || S > 64) return S - 1 - r;
+  const int k = r / round;
+  if (k & 1) r = min((k + 1) * round, S) - 1 - (r - k * round);
+  const int lane = threadIdx.x & 63, n = lane < S ? cu[lane + 1] - cu[lane] : -1;
+  int rank = 0;
+  for (int j = 0; j < S; ++j) {
+    const int m = __builtin_amdgcn_readlane(n, j);
+    rank += m > n || (m == n && j < lane);
+  }
+  return __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(lane < S && rank == r)));
+}
+
 __device__ __forceinline__ int first_chunk(const int* __restrict__ cu, int s) {
   const int lane = threadIdx.x & 63;
   int total = 0;

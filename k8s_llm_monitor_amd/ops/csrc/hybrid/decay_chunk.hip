@@ -285,10 +285,11 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
   __shared__ __attribute__((aligned(16))) int first[2][NV];  // chunk_seg.h: rows from which a column is no number
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
   if (pair >= (MODE == kWhole ? S_ : n_span) * H) return;
-  // from the last segment on: a step's prompts come after its running sequences, and their chains take longest
   const int h = pair % H, dvb = zb * NV, sp_i = n_span - 1 - pair / H;
-  ChunkAt at = {S_ - 1 - pair / H, 0, 0, 0, 1};
-  if (MODE != kWhole) {
+  ChunkAt at = {0, 0, 0, 0, 1};
+  if (MODE == kWhole) {
+    at.seg = segment_in_turn(cu, S_, pair / H, max(1, 256 / (H * nz)));
+  } else {
     at = chunk_at(cu, S_, sp_i, span * kChunk);
     if (at.seg < 0 || (MODE == kSpanEnds && (at.k == at.count - 1 || slot[at.seg] < 0))) return;
   }

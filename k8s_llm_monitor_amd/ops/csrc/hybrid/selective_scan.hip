@@ -52,8 +52,13 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   __shared__ __attribute__((aligned(16))) float Cs[TB][NS];
   __shared__ float dts[TB][PB], us[TB][PB];
   __shared__ float ys[TB][PB + 64 / LPC];  // padded: the lanes of a channel write neighbouring rows to different banks
-  ChunkAt at = {(int)blockIdx.x, 0, 0, 0, 1};
-  if (MODE != kWhole) {
+  ChunkAt at = {0, 0, 0, 0, 1};
+  int by = blockIdx.y;  // which channels
+  if (MODE == kWhole) {
+    const int i = blockIdx.x + gridDim.x * blockIdx.y, groups = gridDim.y;
+    by = i % groups;
+    at.seg = segment_in_turn(cu, n_seg, i / groups, max(1, 256 / groups));
+  } else {
     at = chunk_at(cu, n_seg, blockIdx.x, span);
     if (at.seg < 0 || (MODE == kSpanEnds && (at.k == at.count - 1 || slot[at.seg] < 0))) return;
   }
@@ -61,7 +66,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   const int sl = slot[s];
   const int t0 = MODE == kWhole ? cu[s] : at.row, t1 = MODE == kWhole ? cu[s + 1] : at.row + at.n;
   const int pc = threadIdx.x % PB, tt0 = threadIdx.x / PB;  // staging: channel pc, tokens tt0 + LPC u
-  const int cs = blockIdx.y * PB + pc;
+  const int cs = by * PB + pc;
   const bool slive = cs < C;
   if (sl < 0) {  // padding rows: defined output, no state
     if (slive)
@@ -71,7 +76,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   if (t1 <= t0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int chunk = lane % LPC, pl = wave * (64 / LPC) + lane / LPC;
-  const int c = blockIdx.y * PB + pl, n0 = chunk * NPL;
+  const int c = by * PB + pl, n0 = chunk * NPL;
   const bool live = c < C;
   const bool vec = (N & 3) == 0 && n0 + NPL <= N;
   const bool carried = ctx[s] > 0 && (MODE == kWhole || at.count == 1 || (MODE == kSpanEnds && at.k == 0));

@@ -738,6 +738,33 @@ def test_gradients_of_few_rows_products(M):
             assert not f(xg, wg).requires_grad
 
 
+@pytest.mark.parametrize("lens", [[130, 0, 64, 5, 5, 257, 1], [70] * 5, [9 * (i % 8) for i in range(64)], [9 * (i % 8) for i in range(65)], [300]])
+def test_segments_in_turn(lens):
+    """Prompts of all lengths (equal and empty ones, a table of 64 entries and one more), which the scans take longest and shortest in turn: each is
+    taken once.  A prompt alone in its step has the same bits."""
+    g = _g(79)
+    S, H, d, C, N = len(lens), 5, 64, 640, 16
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    ctx, slot, T = _i32([0] * S).cuda(), _i32(list(range(S))).cuda(), sum(lens)
+    vkq, dec = _r(g, T, 3 * H * d, dt=BF).cuda(), torch.rand(H, generator=g).cuda()
+    x, q, dt, z = (_r(g, T, n, s=0.3, dt=BF).cuda() for n in (C, 2 * N, C, C))
+    bias, a_log, D = _r(g, C, s=0.3).cuda(), _r(g, C, N, s=0.3).cuda(), _r(g, C).cuda()
+
+    def run(a, b, s0, s1):
+        seg = ((cu[s0:s1 + 1] - cu[s0]).contiguous(), ctx[s0:s1], slot[s0:s1])
+        st1, st2 = torch.zeros(S, H, d, d, device="cuda"), torch.zeros(S, C, N, device="cuda")
+        o1 = hops.linear_attention(vkq[a:b], dec, st1, *seg, H, d, d, mode=3, col_tiles=1)
+        o2 = hops.selective_scan(x[a:b], q[a:b], 0, N, dt[a:b], bias, a_log, D, z[a:b], 0, st2, *seg, mode=1)
+        return o1, o2, st1[s0:s1], st2[s0:s1]
+
+    whole = run(0, T, 0, S)
+    for s, n in enumerate(lens):
+        if n and (s < 8 or s > S - 3):
+            a = int(cu[s])
+            for got, want in zip(run(a, a + n, s, s + 1), whole):
+                assert torch.equal(got, want[a:a + n] if got.shape[0] == n and want.shape[0] == T else want[s:s + 1])
+
+
 @pytest.mark.parametrize("M", [1, 24, 64])
 @pytest.mark.parametrize("N,K,shared", [(2056, 2048, True), (1544, 4096, True), (520, 8192, False), (264, 16384, False), (1100, 16384, True)])
 def test_few_rows_from_a_k_of_their_own(M, N, K, shared):
