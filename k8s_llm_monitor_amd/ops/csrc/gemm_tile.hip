@@ -70,10 +70,13 @@ __device__ __forceinline__ void lgkm_wait0() { asm volatile("s_waitcnt lgkmcnt(0
 }  // namespace
 
 // Tiles run in rounds of one a CU, and a last round of few tiles takes most of a full one's time (30 to 45 us of K = 2048 alone on the chip, a full
-// round's 55 to 60).  Up to 64 tiles beyond whole rounds go as four strips of 64 rows each, one a CU, of about half a tile's time; from 65 on
-// the strips would need two rounds, which was no faster (72 tiles of K 1024 35 / 42 us, 128 of K 2048 43.9 / 43.6, 112 behind a round 119 / 126).
-// us, whole tiles / strips: 780 tiles of K 2048 (gated unit) 224 / 214; 258 of K 4096 172 / 157; grouped, 8 experts, 1072 294 / 279 and 536
-// 148 / 140; 320 of K 4096 in 4 experts 204 / 170; 36 of K 1024 28 / 21.
+// round's 50 to 55).  Up to 64 tiles beyond whole rounds go as four strips of 64 rows each, one a CU, and up to 32 as eight of 64 rows x 128 columns: a chain of
+// k-tiles of 0.8 and 0.4 us.  us, 32 tiles of K 2048 alone, four / eight: 28.6 / 18.2; behind rounds, of K 1024, 32 tiles 45.1 / 39.4.  From 65 on four strips a tile
+// would need two rounds, which was no faster (72 tiles of K 1024 35 / 42 us, 112 behind a round 119 / 126); two strips of 128 rows each were slower (128
+// behind a round, K 2048 90.3 / 95.6, 4096 160 / 175).
+// A strip has accumulators and fragments of its own: with the tile's, hipcc spilled (10 us of 241 in the grouped product below) or moved accumulators in the tile's loop.
+// us, whole tiles / strips: 780 tiles of K 2048 (gated unit) 224 / 183; 258 of K 4096 172 / 157; grouped, 8 experts, K 2048, 1072 294 / 229 and 536
+// 148 / 121; 320 of K 4096 in 4 experts 204 / 170.
 // Products without such tiles have a kernel without strips (CUT false): 6000 x 12288 x 1408, squared ReLU, 188.5 us with both in one, 186.6 without.
 // Grouped, the count of tiles is known on the device only: each workgroup sums it over the experts, up to kStripExperts of them.
 constexpr int kTileCus = 256, kStripTiles = 64, kStripExperts = 32;
@@ -81,8 +84,9 @@ template <int EPI, int SCH, bool RS>
 constexpr bool tile_strips() {
   return SCH == 1 && !RS && EPI != TILE_EPI_ROPE && EPI != TILE_EPI_RESID;
 }
+constexpr int kFineTiles = 32;  // up to this many such tiles go as eight strips of 64 rows x 128 columns each
 // workgroups that strips of up to this many tiles add
-static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * 32 - tiles; }
+static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * (tiles <= kFineTiles ? 64 : 32) - tiles; }
 
 // NARROW: every workgroup a strip of 64 (or 128, TALL) rows x 128 (or 64) columns, for products of few tiles (narrow_strips).
 template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0, bool TALL = false, bool CUT = true>
@@ -103,13 +107,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     mts = 0;
     for (int x = 0; x < E; ++x) mts += (offsets[x + 1] - offsets[x] + 255) >> 8;
   }
-  int nwg = mts * n_nt, lid, strip = -1;
+  int nwg = mts * n_nt, lid, strip = -1, half = 0;
   const int bid = blockIdx.x, xcd = bid & 7;
   const int over = STRIPS && strips ? nwg % kTileCus : 0;  // tiles beyond whole rounds
   if (over > 0 && over <= kStripTiles && bid >= nwg - over) {
-    const int i = bid - (nwg - over);  // a tile's four strips on one XCD
+    const int i = bid - (nwg - over);  // a tile's strips on one XCD
     strip = (i >> 3) & 3;
-    lid = (i >> 5) * 8 + (i & 7);
+    half = over <= kFineTiles ? (i >> 5) & 1 : 0;
+    lid = (i >> (over <= kFineTiles ? 6 : 5)) * 8 + (i & 7);
     if (lid >= over) return;
     lid += nwg - over;
   } else {
@@ -158,8 +163,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   constexpr bool GLU = tile_epi_glu(EPI);
   const int n_unit = GLU ? (ep.f + 127) >> 7 : 0;
   const bool unit = GLU && nt < n_unit;
-  const int n0 = GLU ? (unit ? nt * 128 : 2 * ep.f + (nt - n_unit) * 256) : nt * TN;
-  const int nrows = unit ? 2 * min(128, ep.f - n0) : min(TN, N - n0);
+  const bool fine = STRIPS && strip >= 0 && over <= kFineTiles;
+  const int n0 = (GLU ? (unit ? nt * 128 : 2 * ep.f + (nt - n_unit) * 256) : nt * TN) + half * (unit ? 64 : 128);
+  const int nrows = unit ? 2 * min(fine ? 64 : 128, ep.f - n0) : min(fine ? 128 : TN, N - n0);
+  if (STRIPS && nrows <= 0) return;
 
   // ---- DMA of one half-tile (256 rows x 128 B = 32 pieces of 1 KiB): piece p (0..7) of this
   // wave covers rows (p * 4 + wave) * 8 .. + 7; lane -> row + (lane >> 3), physical chunk lane & 7 ----
@@ -227,24 +234,204 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   };
 
   float rs_inv = 1.f;  // RS: 1 / rms of this thread's row (threadIdx.x of the tile)
-  f32x4 acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  bf16x8 fa0[8], fb0[8], fa1[8], fb1[8];
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   // RESID: this lane's first 16 residual chunks (rows rr + 4b of the wave's 128, 16 B at column
   // chunk cc), issued during the last k-tile's second half so they land behind its MFMAs
   u32x4 resq[EPI == TILE_EPI_RESID ? 16 : 1];
 
-  if (NARROW || (STRIPS && strip >= 0)) {
-    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  NARROW, 64 x 128 (64): 16 x 128 (64), six (ten) of 8 + 16 (8); 128 x 128:
+  // ---- epilogue: acc[i][j][r] = Y[m][n], m = wm*128 + i*16 + (lane & 15),
+  // n = wn*128 + j*16 + 4 (lane >> 4) + r.  Staged through LDS (the ring is idle now): each wave
+  // writes its quarter as bf16 rows (8-B ds_write per 4 columns), then reads back whole rows and
+  // stores 16 B per lane, 256 contiguous bytes per row - half the store instructions of writing
+  // the accumulator layout directly, which is what bounds a store tail (T21). ----
+  auto finish = [&](auto& acc, auto gated, auto blocks, int wm, int wn) {  // gated: a unit's tile; blocks: of 16 rows, a wave's
+  constexpr bool SWG = decltype(gated)::value;
+  constexpr int RB = decltype(blocks)::value;
+  constexpr int OUTW = SWG || NARROW == 64 ? 64 : 128;  // output columns of this wave's quarter
+  constexpr int RS_ = OUTW * 2 + 16;                       // LDS row stride (16-B pad: 2-way writes)
+  char* stage = smem + wave * (16 * RB * RS_);
+  const int ml = lane & 15, nq = 4 * (lane >> 4);
+  const int rr = lane >> 4, cc = lane & 15;
+  uint4 nwv{};
+  if constexpr (EPI == TILE_EPI_RESID) nwv = *reinterpret_cast<const uint4*>(ep.norm_w + n0 + wn * 128 + cc * 8);
+  // RS: each thread's row scale through LDS (after the staging area) to the lanes holding the row
+  float sc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sc[i] = 1.f;
+  if constexpr (RS) {
+    float* inv_s = reinterpret_cast<float*>(smem + 4 * 128 * (128 * 2 + 16));
+    inv_s[threadIdx.x] = rs_inv;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sc[i] = inv_s[wm * 128 + i * 16 + ml];
+  }
+#pragma unroll
+  for (int i = 0; i < RB; ++i) {
+    __builtin_amdgcn_sched_barrier(0);  // one row block's accumulators at a time (no hoisted AGPR reads)
+    char* srow = stage + (i * 16 + ml) * RS_ + nq * 2;
+    if constexpr (EPI == TILE_EPI_SWIGLU || (GLU && SWG)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float gt = bf2f(f2bf(acc[i][j][r] * sc[i])), up = bf2f(f2bf(acc[i][j + 4][r] * sc[i]));
+          o[r] = GLU ? tile_unit<EPI>(gt, up) : gt * up / (1.f + __expf(-gt));
+        }
+        *reinterpret_cast<uint2*>(srow + j * 32) = uint2{pack2(o[0], o[1]), pack2(o[2], o[3])};
+      }
+    } else if constexpr (EPI == TILE_EPI_SWIGLU8) {
+      // [8 gate | 8 up] per 16-column n-tile j: gate column 4 q + r (q = 0, 1: lanes 0-31) pairs
+      // with up column 8 + 4 q + r in lane + 32.  One v_permlane32_swap per register puts (gate,
+      // up) in both lane halves; lanes 0-31 finish r = 0, 1 and lanes 32-63 r = 2, 3 of feature
+      // 8 j + 4 q + r (4 bytes each).
+      const int hi = lane >> 5, qq = (lane >> 4) & 1;
+      char* srow8 = stage + (i * 16 + ml) * RS_ + (8 * qq + 4 * hi);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float g[4], u[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t v = __float_as_uint(acc[i][j][r] * sc[i]);
+          const auto pr = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+          g[r] = __uint_as_float(pr[0]);
+          u[r] = __uint_as_float(pr[1]);
+        }
+        float o[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const float gt = bf2f(f2bf(hi ? g[2 + k] : g[k])), up = bf2f(f2bf(hi ? u[2 + k] : u[k]));
+          o[k] = gt * up / (1.f + __expf(-gt));
+        }
+        *reinterpret_cast<uint32_t*>(srow8 + j * 16) = pack2(o[0], o[1]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < OUTW / 16; ++j) {
+        f32x4 v = acc[i][j] * sc[i];
+        if constexpr (EPI == TILE_EPI_RELU_SQ) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float z = bf2f(f2bf(v[r]));
+            v[r] = z > 0.f ? z * z : 0.f;
+          }
+        }
+        *reinterpret_cast<uint2*>(srow + j * 32) = uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
+      }
+    }
+  }
+  lgkm_wait0();
+  if constexpr (EPI == TILE_EPI_RESID) {
+    // lane (rr, cc): row rr + 4b, columns cc*8 .. +7 of the wave's quarter; N % 128 == 0 (host)
+    const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
+    const __amdgpu_buffer_rsrc_t rhw = rsrc(ep.hw + (long)row0 * N, (long)mrows * N * 2);
+    const uint32_t ro = (uint32_t)(((wm * 128 + rr) * N + n0 + wn * 128 + cc * 8) * 2);
+    float wf[8];
+    unpack8(nwv, wf);
+    const int ss_np = N >> 7, ssc = (n0 + wn * 128) >> 7;
+#pragma unroll
+    for (int b = 0; b < 32; ++b) {
+      const int r = rr + 4 * b;
+      const uint4 yv = *reinterpret_cast<const uint4*>(stage + r * RS_ + cc * 16);
+      float y[8], rv[8], h[8], hw[8];
+      unpack8(yv, y);
+      const u32x4 rb = resq[b & 15];
+      if (b < 16) resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * (b + 16) * N * 2), 0, 0);
+      unpack8(uint4{rb[0], rb[1], rb[2], rb[3]}, rv);
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        h[e] = bf2f(f2bf(y[e] + rv[e]));
+        ss += h[e] * h[e];
+        hw[e] = h[e] * wf[e];
+      }
+      const uint4 hq = pack8(h), wq = pack8(hw);
+      const uint32_t off = ro + (uint32_t)(4 * b * N * 2);
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4{hq.x, hq.y, hq.z, hq.w}, rres, off, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4{wq.x, wq.y, wq.z, wq.w}, rhw, off, 0, 0);
+      ss = row16_sum(ss);
+      const int grow = wm * 128 + r;
+      if (cc == 0 && grow < mrows) ep.ss_out[(long)(row0 + grow) * ss_np + ssc] = ss;
+    }
+    return;
+  }
+  if constexpr (EPI == TILE_EPI_ROPE) {
+    const int head = (n0 + wn * 128) >> 7;
+    if (head < ep.rope_heads && nrows - wn * 128 >= 128) {
+      // one lane per (row, chunk pair c, c + 8): 8 rows per pass, 16 passes over the quarter's rows
+      const int c = lane & 7, rsub = lane >> 3;
+      bf16_t* ybase = Y + (long)row0 * N + n0 + wn * 128;
+#pragma unroll 4
+      for (int pass = 0; pass < 2 * RB; ++pass) {
+        const int r = pass * 8 + rsub, grow = wm * 16 * RB + r;
+        if (grow >= mrows) continue;
+        const uint4 a = *reinterpret_cast<const uint4*>(stage + r * RS_ + c * 16);
+        const uint4 b = *reinterpret_cast<const uint4*>(stage + r * RS_ + (c + 8) * 16);
+        const float* cs = ep.cos_sin + (long)ep.positions[row0 + grow] * 128;
+        const float4 c0 = *reinterpret_cast<const float4*>(cs + c * 8), c1 = *reinterpret_cast<const float4*>(cs + c * 8 + 4);
+        const float4 s0 = *reinterpret_cast<const float4*>(cs + 64 + c * 8),
+                     s1 = *reinterpret_cast<const float4*>(cs + 64 + c * 8 + 4);
+        const float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        const float ss[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+        float x1[8], x2[8], o1[8], o2[8];
+        unpack8(a, x1);
+        unpack8(b, x2);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          o1[j] = x1[j] * cc[j] - x2[j] * ss[j];
+          o2[j] = x2[j] * cc[j] + x1[j] * ss[j];
+        }
+        bf16_t* yr = ybase + (long)grow * N;
+        *reinterpret_cast<uint4*>(yr + c * 8) = pack8(o1);
+        *reinterpret_cast<uint4*>(yr + 64 + c * 8) = pack8(o2);
+      }
+      return;
+    }
+  }
+  constexpr int CPR = OUTW / 8;  // 16-B chunks per row
+  constexpr int RPI = 64 / CPR;  // rows per wave instruction
+  const int ldy = GLU ? (SWG ? ep.f : N - 2 * ep.f) : SWG ? (N >> 1) : N;
+  const int col0 = GLU ? (SWG ? n0 + wn * 64 : n0 - 2 * ep.f + wn * 128) : SWG ? ((n0 + wn * 128) >> 1) : n0 + wn * 128;
+  const int ncols = SWG ? (nrows >> 1) - wn * 64 : nrows - wn * 128;
+  bf16_t* const out = GLU && !SWG ? ep.y2 : Y;
+  const int rr2 = lane / CPR, cc2 = lane % CPR;
+  // branch-free masked stores: a buffer descriptor over this m-tile's rows drops every store past
+  // row mrows (out of range), and a lane whose columns are past N gets an out-of-range offset
+  const __amdgpu_buffer_rsrc_t yr = rsrc(out + (long)row0 * ldy, (long)mrows * ldy * 2);
+  const uint32_t yo = cc2 * 8 < ncols ? (uint32_t)(((wm * 16 * RB + rr2) * ldy + col0 + cc2 * 8) * 2) : 0x80000000u;
+  constexpr int NB = 16 * RB / RPI < 8 ? 16 * RB / RPI : 8;
+#pragma unroll
+  for (int b = 0; b < 16 * RB / RPI; b += NB) {  // 8 row groups per batch: reads issued back to back
+    u32x4 v[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) v[u] = *reinterpret_cast<const u32x4*>(stage + ((b + u) * RPI + rr2) * RS_ + cc2 * 16);
+#pragma unroll
+    for (int u = 0; u < NB; ++u)
+      __builtin_amdgcn_raw_buffer_store_b128(v[u], yr, yo + (uint32_t)((b + u) * RPI * ldy * 2), 0, 0);
+  }
+  };
+  auto end = [&](auto& acc, auto blocks, int wm, int wn) {
+    if constexpr (GLU) {
+      if (unit) finish(acc, std::true_type{}, blocks, wm, wn);
+      else finish(acc, std::false_type{}, blocks, wm, wn);
+    } else {
+      finish(acc, std::bool_constant<EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8>{}, blocks, wm, wn);
+    }
+  };
+  // a strip, of 64 (TALL: 128) rows x COLS columns; wm, wn: the wave's place in it
+  auto strip_of = [&](auto cols, int wm, int wn) {
+    constexpr int COLS = decltype(cols)::value;
+    // 64 x 256: the waves' quarters are 32 x 128, the ring four k-tiles of 8 + 32 KiB, one barrier a k-tile.  64 x 128 (64): 16 x 128 (64), six (ten) of 8 + 16 (8); 128 x 128:
     // 32 x 128, five of 16 + 16.
     // The same instructions in the same order of k as a whole tile's, so the same bits.
-    constexpr int RB = NARROW && !TALL ? 1 : 2, AP = TALL ? 4 : 2, BP = NARROW ? NARROW / 32 : 8, NJ = NARROW ? NARROW / 16 : 8;
+    constexpr int RB = COLS < 256 && !TALL ? 1 : 2, AP = TALL ? 4 : 2, BP = COLS / 32, NJ = COLS < 128 ? COLS / 16 : 8;
     constexpr int SA = AP * 4096, SS = SA + BP * 4096, SLOTS = 5 * HS / SS;
+    f32x4 acc[RB][NJ];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 fa0[RB], fb0[NJ], fa1[RB], fb1[NJ];
     auto next = [&](int slot) { return slot + SS == SLOTS * SS ? 0 : slot + SS; };
     auto fill = [&](int kt, int slot) {
       char* dst = smem + slot + wave * 1024;
@@ -255,14 +442,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       for (int p = 0; p < BP; ++p)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(dst + SA + p * 4096), 16, soff[1][p], k * kstrB, 0, 0);
     };
-    auto read = [&](int slot, int ks, bf16x8 (&a)[8], bf16x8 (&b)[8]) {
+    auto read = [&](int slot, int ks, bf16x8 (&a)[RB], bf16x8 (&b)[NJ]) {
       const char* at = smem + slot;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) b[j] = *reinterpret_cast<const bf16x8*>(at + SA + (8 * wn + j) * 2048 + rdB[ks]);
 #pragma unroll
       for (int g = 0; g < RB; ++g) a[g] = *reinterpret_cast<const bf16x8*>(at + (RB * wm + g) * 2048 + rd[ks]);
     };
-    auto mul = [&](const bf16x8 (&a)[8], const bf16x8 (&b)[8]) {
+    auto mul = [&](const bf16x8 (&a)[RB], const bf16x8 (&b)[NJ]) {
 #pragma unroll
       for (int g = 0; g < RB; ++g)
 #pragma unroll
@@ -289,7 +476,29 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       at = next(at);
     }
     vm_wait_n<0>();
-  } else if constexpr (SCH == 1 && !NARROW) {
+    lgkm_wait0();
+    __builtin_amdgcn_s_barrier();  // every wave is done with the ring
+    end(acc, std::integral_constant<int, RB>{}, wm, wn);
+  };
+  if constexpr (NARROW) {
+    strip_of(std::integral_constant<int, NARROW>{}, wm, wn);
+    return;
+  }
+  if constexpr (STRIPS) {  // (accumulators of their own: with the tile's, its loop moves them to and fro)
+    if (strip >= 0) {
+      if (fine) strip_of(std::integral_constant<int, 128>{}, wave, 0);
+      else strip_of(std::integral_constant<int, 256>{}, wm, wn);
+      return;
+    }
+  }
+  f32x4 acc[8][8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  bf16x8 fa0[8], fb0[8], fa1[8], fb1[8];
+  if constexpr (SCH == 1 && !NARROW) {
     // Ring addressing: the half-slot byte offsets of the current tile live in SGPRs and rotate
     // by one conditional subtract per tile, and each sub-step forms ONE A and ONE B fragment base
     // VGPR (every block read is that base + an immediate).
@@ -477,198 +686,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     vm_wait_n<0>();
   }
 
-  // ---- epilogue: acc[i][j][r] = Y[m][n], m = wm*128 + i*16 + (lane & 15),
-  // n = wn*128 + j*16 + 4 (lane >> 4) + r.  Staged through LDS (the ring is idle now): each wave
-  // writes its quarter as bf16 rows (8-B ds_write per 4 columns), then reads back whole rows and
-  // stores 16 B per lane, 256 contiguous bytes per row - half the store instructions of writing
-  // the accumulator layout directly, which is what bounds a store tail (T21). ----
   lgkm_wait0();
   __builtin_amdgcn_s_barrier();  // every wave is done with the ring (its last DMAs retired above)
-  auto finish = [&](auto gated, auto blocks) {  // gated: a unit's tile; blocks: of 16 rows, a wave's
-  constexpr bool SWG = decltype(gated)::value;
-  constexpr int RB = decltype(blocks)::value;
-  constexpr int OUTW = SWG || NARROW == 64 ? 64 : 128;  // output columns of this wave's quarter
-  constexpr int RS_ = OUTW * 2 + 16;                       // LDS row stride (16-B pad: 2-way writes)
-  char* stage = smem + wave * (16 * RB * RS_);
-  const int ml = lane & 15, nq = 4 * (lane >> 4);
-  const int rr = lane >> 4, cc = lane & 15;
-  uint4 nwv{};
-  if constexpr (EPI == TILE_EPI_RESID) nwv = *reinterpret_cast<const uint4*>(ep.norm_w + n0 + wn * 128 + cc * 8);
-  // RS: each thread's row scale through LDS (after the staging area) to the lanes holding the row
-  float sc[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) sc[i] = 1.f;
-  if constexpr (RS) {
-    float* inv_s = reinterpret_cast<float*>(smem + 4 * 128 * (128 * 2 + 16));
-    inv_s[threadIdx.x] = rs_inv;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sc[i] = inv_s[wm * 128 + i * 16 + ml];
-  }
-#pragma unroll
-  for (int i = 0; i < RB; ++i) {
-    __builtin_amdgcn_sched_barrier(0);  // one row block's accumulators at a time (no hoisted AGPR reads)
-    char* srow = stage + (i * 16 + ml) * RS_ + nq * 2;
-    if constexpr (EPI == TILE_EPI_SWIGLU || (GLU && SWG)) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float gt = bf2f(f2bf(acc[i][j][r] * sc[i])), up = bf2f(f2bf(acc[i][j + 4][r] * sc[i]));
-          o[r] = GLU ? tile_unit<EPI>(gt, up) : gt * up / (1.f + __expf(-gt));
-        }
-        *reinterpret_cast<uint2*>(srow + j * 32) = uint2{pack2(o[0], o[1]), pack2(o[2], o[3])};
-      }
-    } else if constexpr (EPI == TILE_EPI_SWIGLU8) {
-      // [8 gate | 8 up] per 16-column n-tile j: gate column 4 q + r (q = 0, 1: lanes 0-31) pairs
-      // with up column 8 + 4 q + r in lane + 32.  One v_permlane32_swap per register puts (gate,
-      // up) in both lane halves; lanes 0-31 finish r = 0, 1 and lanes 32-63 r = 2, 3 of feature
-      // 8 j + 4 q + r (4 bytes each).
-      const int hi = lane >> 5, qq = (lane >> 4) & 1;
-      char* srow8 = stage + (i * 16 + ml) * RS_ + (8 * qq + 4 * hi);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float g[4], u[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t v = __float_as_uint(acc[i][j][r] * sc[i]);
-          const auto pr = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-          g[r] = __uint_as_float(pr[0]);
-          u[r] = __uint_as_float(pr[1]);
-        }
-        float o[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const float gt = bf2f(f2bf(hi ? g[2 + k] : g[k])), up = bf2f(f2bf(hi ? u[2 + k] : u[k]));
-          o[k] = gt * up / (1.f + __expf(-gt));
-        }
-        *reinterpret_cast<uint32_t*>(srow8 + j * 16) = pack2(o[0], o[1]);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < OUTW / 16; ++j) {
-        f32x4 v = acc[i][j] * sc[i];
-        if constexpr (EPI == TILE_EPI_RELU_SQ) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float z = bf2f(f2bf(v[r]));
-            v[r] = z > 0.f ? z * z : 0.f;
-          }
-        }
-        *reinterpret_cast<uint2*>(srow + j * 32) = uint2{pack2(v[0], v[1]), pack2(v[2], v[3])};
-      }
-    }
-  }
-  lgkm_wait0();
-  if constexpr (EPI == TILE_EPI_RESID) {
-    // lane (rr, cc): row rr + 4b, columns cc*8 .. +7 of the wave's quarter; N % 128 == 0 (host)
-    const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
-    const __amdgpu_buffer_rsrc_t rhw = rsrc(ep.hw + (long)row0 * N, (long)mrows * N * 2);
-    const uint32_t ro = (uint32_t)(((wm * 128 + rr) * N + n0 + wn * 128 + cc * 8) * 2);
-    float wf[8];
-    unpack8(nwv, wf);
-    const int ss_np = N >> 7, ssc = (n0 + wn * 128) >> 7;
-#pragma unroll
-    for (int b = 0; b < 32; ++b) {
-      const int r = rr + 4 * b;
-      const uint4 yv = *reinterpret_cast<const uint4*>(stage + r * RS_ + cc * 16);
-      float y[8], rv[8], h[8], hw[8];
-      unpack8(yv, y);
-      const u32x4 rb = resq[b & 15];
-      if (b < 16) resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * (b + 16) * N * 2), 0, 0);
-      unpack8(uint4{rb[0], rb[1], rb[2], rb[3]}, rv);
-      float ss = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        h[e] = bf2f(f2bf(y[e] + rv[e]));
-        ss += h[e] * h[e];
-        hw[e] = h[e] * wf[e];
-      }
-      const uint4 hq = pack8(h), wq = pack8(hw);
-      const uint32_t off = ro + (uint32_t)(4 * b * N * 2);
-      __builtin_amdgcn_raw_buffer_store_b128(u32x4{hq.x, hq.y, hq.z, hq.w}, rres, off, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(u32x4{wq.x, wq.y, wq.z, wq.w}, rhw, off, 0, 0);
-      ss = row16_sum(ss);
-      const int grow = wm * 128 + r;
-      if (cc == 0 && grow < mrows) ep.ss_out[(long)(row0 + grow) * ss_np + ssc] = ss;
-    }
-    return;
-  }
-  if constexpr (EPI == TILE_EPI_ROPE) {
-    const int head = (n0 + wn * 128) >> 7;
-    if (head < ep.rope_heads && nrows - wn * 128 >= 128) {
-      // one lane per (row, chunk pair c, c + 8): 8 rows per pass, 16 passes over the quarter's rows
-      const int c = lane & 7, rsub = lane >> 3;
-      bf16_t* ybase = Y + (long)row0 * N + n0 + wn * 128;
-#pragma unroll 4
-      for (int pass = 0; pass < 2 * RB; ++pass) {
-        const int r = pass * 8 + rsub, grow = wm * 16 * RB + r;
-        if (grow >= mrows) continue;
-        const uint4 a = *reinterpret_cast<const uint4*>(stage + r * RS_ + c * 16);
-        const uint4 b = *reinterpret_cast<const uint4*>(stage + r * RS_ + (c + 8) * 16);
-        const float* cs = ep.cos_sin + (long)ep.positions[row0 + grow] * 128;
-        const float4 c0 = *reinterpret_cast<const float4*>(cs + c * 8), c1 = *reinterpret_cast<const float4*>(cs + c * 8 + 4);
-        const float4 s0 = *reinterpret_cast<const float4*>(cs + 64 + c * 8),
-                     s1 = *reinterpret_cast<const float4*>(cs + 64 + c * 8 + 4);
-        const float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-        const float ss[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-        float x1[8], x2[8], o1[8], o2[8];
-        unpack8(a, x1);
-        unpack8(b, x2);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          o1[j] = x1[j] * cc[j] - x2[j] * ss[j];
-          o2[j] = x2[j] * cc[j] + x1[j] * ss[j];
-        }
-        bf16_t* yr = ybase + (long)grow * N;
-        *reinterpret_cast<uint4*>(yr + c * 8) = pack8(o1);
-        *reinterpret_cast<uint4*>(yr + 64 + c * 8) = pack8(o2);
-      }
-      return;
-    }
-  }
-  constexpr int CPR = OUTW / 8;  // 16-B chunks per row
-  constexpr int RPI = 64 / CPR;  // rows per wave instruction
-  const int ldy = GLU ? (SWG ? ep.f : N - 2 * ep.f) : SWG ? (N >> 1) : N;
-  const int col0 = GLU ? (SWG ? n0 + wn * 64 : n0 - 2 * ep.f + wn * 128) : SWG ? ((n0 + wn * 128) >> 1) : n0 + wn * 128;
-  const int ncols = SWG ? (nrows >> 1) - wn * 64 : nrows - wn * 128;
-  bf16_t* const out = GLU && !SWG ? ep.y2 : Y;
-  const int rr2 = lane / CPR, cc2 = lane % CPR;
-  // branch-free masked stores: a buffer descriptor over this m-tile's rows drops every store past
-  // row mrows (out of range), and a lane whose columns are past N gets an out-of-range offset
-  const __amdgpu_buffer_rsrc_t yr = rsrc(out + (long)row0 * ldy, (long)mrows * ldy * 2);
-  const uint32_t yo = cc2 * 8 < ncols ? (uint32_t)(((wm * 16 * RB + rr2) * ldy + col0 + cc2 * 8) * 2) : 0x80000000u;
-  constexpr int NB = 16 * RB / RPI < 8 ? 16 * RB / RPI : 8;
-#pragma unroll
-  for (int b = 0; b < 16 * RB / RPI; b += NB) {  // 8 row groups per batch: reads issued back to back
-    u32x4 v[NB];
-#pragma unroll
-    for (int u = 0; u < NB; ++u) v[u] = *reinterpret_cast<const u32x4*>(stage + ((b + u) * RPI + rr2) * RS_ + cc2 * 16);
-#pragma unroll
-    for (int u = 0; u < NB; ++u)
-      __builtin_amdgcn_raw_buffer_store_b128(v[u], yr, yo + (uint32_t)((b + u) * RPI * ldy * 2), 0, 0);
-  }
-  };
-  auto end = [&](auto blocks) {
-    if constexpr (GLU) {
-      if (unit) finish(std::true_type{}, blocks);
-      else finish(std::false_type{}, blocks);
-    } else {
-      finish(std::bool_constant<EPI == TILE_EPI_SWIGLU || EPI == TILE_EPI_SWIGLU8>{}, blocks);
-    }
-  };
-  if constexpr (NARROW) {
-    end(std::integral_constant<int, TALL ? 2 : 1>{});
-    return;
-  }
-  if constexpr (STRIPS) {
-    if (strip >= 0) {
-      end(std::integral_constant<int, 2>{});
-      return;
-    }
-  }
-  if constexpr (!NARROW) end(std::integral_constant<int, 8>{});
+  if constexpr (!NARROW) end(acc, std::integral_constant<int, 8>{}, wm, wn);
 }
 
 }  // namespace k8sllm

@@ -209,6 +209,26 @@ def test_gemm_tile_last_round(m_tiles, n_tiles, last, K, swiglu):
     assert torch.equal(y2, z[:, 2 * f:])
 
 
+@pytest.mark.parametrize("M,N,K,f", [  # 32 and 33 tiles, one behind a round, none of the second half's columns, a unit's half without features
+    (1000, 2048, 256, 960), (1000, 2128, 192, 1056), (4097, 4096, 192, 1984), (300, 128, 640, 48), (300, 400, 192, 80), (8100, 2064, 256, 1000 // 16 * 16),
+])
+def test_gemm_tile_last_round_in_fine_strips(M, N, K, f):
+    """Up to 32 tiles beyond whole rounds of 256 as strips of 64 rows x 128 columns: the bits of whole tiles, weights packed or not; a gated unit with other
+    columns behind it."""
+    g = torch.Generator().manual_seed(6)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    z = ops.gemm_tile(x, w, algo=0)
+    off = torch.tensor([0, M], dtype=torch.int32, device="cuda")  # (dense products of few tiles have strips of their own)
+    assert torch.equal(ops.gemm_tile(x, w[None], off, algo=1), z)
+    assert torch.equal(ops.gemm_tile(x, w, algo=1), z)
+    assert torch.equal(ops.gemm_tile(x, ops.pack_skinny(w)[None], off, algo=1), z)
+    y, y2 = torch.empty(M, f, dtype=torch.bfloat16, device="cuda"), torch.empty(M, N - 2 * f, dtype=torch.bfloat16, device="cuda")
+    ops.native().gemm_tile_unit(y, y2, x, w, 7)  # ReLU: exact but for the product's rounding
+    assert torch.equal(y, (z[:, :f].float().clamp(min=0) * z[:, f:2 * f].float()).to(torch.bfloat16))
+    assert torch.equal(y2, z[:, 2 * f:])
+
+
 @pytest.mark.parametrize("M,N,K,packed", [
     (1, 128, 192, False), (65, 4096, 4096, True), (43, 6144, 4096, True), (257, 1024, 8192, False), (512, 512, 1088, False), (80, 28672, 4096, True),
     (600, 6144, 2112, True), (1000, 1024, 4096, False), (70, 320, 512, False), (260, 4096, 2048, True),  # (64 columns: one round of strips, and more)
