@@ -89,7 +89,8 @@ constexpr int kFineTiles = 32;  // up to this many such tiles go as eight strips
 static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * (tiles <= kFineTiles ? 64 : 32) - tiles; }
 
 // NARROW: every workgroup a strip of 64 (or 128, TALL) rows x 128 (or 64) columns, for products of few tiles (narrow_strips).
-template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0, bool TALL = false, bool CUT = true>
+// MB: row blocks of 16 a wave, half of a tile's (8; 7 where tiles of 224 rows are fewer rounds, row_blocks).
+template <int EPI, bool GROUPED, int SCH, bool RS = false, int NARROW = 0, bool TALL = false, bool CUT = true, int MB = 8>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                          int E, int M, int N, int K, long w_es, int n_mt, int n_nt,
@@ -123,7 +124,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int q8 = nwg >> 3, r8 = nwg & 7;
     lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
   }
-  constexpr int TM = !NARROW ? 256 : TALL ? 128 : 64, TN = NARROW ? NARROW : 256;
+  static_assert(MB == 8 || (!GROUPED && SCH == 1 && !RS && !NARROW && EPI != TILE_EPI_RESID && EPI != TILE_EPI_ROPE));
+  constexpr int TM = !NARROW ? 32 * MB : TALL ? 128 : 64, TN = NARROW ? NARROW : 256;
   constexpr int GM = 8;
   const int grp = lid / (GM * n_nt), first_m = grp * GM;
   const int gsz = min(mts - first_m, GM);
@@ -217,7 +219,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   };
   auto issue_half = [&](int o, int kt) {
 #pragma unroll
-    for (int p = 0; p < 8; ++p) piece(o, p, kt, (2 * kt + o) % 5);
+    for (int p = 0; p < (o ? 8 : MB); ++p) piece(o, p, kt, (2 * kt + o) % 5);
   };
 
   // fragment read: lane row lane & 15 of a 16-row block, 16-B chunk 4 ks + (lane >> 4)
@@ -230,7 +232,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) rdB[ks] = wpk ? ks * 1024 + lane * 16 : rd[ks];
   auto frag = [&](int slot, int ks, int o, int blk) -> bf16x8 {
-    return *reinterpret_cast<const bf16x8*>(smem + slot * HS + ((o ? wn : wm) * 8 + blk) * 2048 + (o ? rdB[ks] : rd[ks]));
+    return *reinterpret_cast<const bf16x8*>(smem + slot * HS + ((o ? wn * 8 : wm * MB) + blk) * 2048 + (o ? rdB[ks] : rd[ks]));
   };
 
   float rs_inv = 1.f;  // RS: 1 / rms of this thread's row (threadIdx.x of the tile)
@@ -399,9 +401,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   // row mrows (out of range), and a lane whose columns are past N gets an out-of-range offset
   const __amdgpu_buffer_rsrc_t yr = rsrc(out + (long)row0 * ldy, (long)mrows * ldy * 2);
   const uint32_t yo = cc2 * 8 < ncols ? (uint32_t)(((wm * 16 * RB + rr2) * ldy + col0 + cc2 * 8) * 2) : 0x80000000u;
-  constexpr int NB = 16 * RB / RPI < 8 ? 16 * RB / RPI : 8;
+  constexpr int NB = RB == 7 ? 7 : 16 * RB / RPI < 8 ? 16 * RB / RPI : 8;
 #pragma unroll
-  for (int b = 0; b < 16 * RB / RPI; b += NB) {  // 8 row groups per batch: reads issued back to back
+  for (int b = 0; b < 16 * RB / RPI; b += NB) {  // 8 (7) row groups per batch: reads issued back to back
     u32x4 v[NB];
 #pragma unroll
     for (int u = 0; u < NB; ++u) v[u] = *reinterpret_cast<const u32x4*>(stage + ((b + u) * RPI + rr2) * RS_ + cc2 * 16);
@@ -491,18 +493,18 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       return;
     }
   }
-  f32x4 acc[8][8];
+  f32x4 acc[MB][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  bf16x8 fa0[8], fb0[8], fa1[8], fb1[8];
+  bf16x8 fa0[MB], fb0[8], fa1[MB], fb1[8];
   if constexpr (SCH == 1 && !NARROW) {
     // Ring addressing: the half-slot byte offsets of the current tile live in SGPRs and rotate
     // by one conditional subtract per tile, and each sub-step forms ONE A and ONE B fragment base
     // VGPR (every block read is that base + an immediate).
-    const uint32_t fbA0 = (uint32_t)(rd[0] + wm * 16384), fbA1 = (uint32_t)(rd[1] + wm * 16384);
+    const uint32_t fbA0 = (uint32_t)(rd[0] + wm * MB * 2048), fbA1 = (uint32_t)(rd[1] + wm * MB * 2048);
     const uint32_t fbB0 = (uint32_t)(rdB[0] + wn * 16384), fbB1 = (uint32_t)(rdB[1] + wn * 16384);
     auto rd16 = [&](uint32_t base, int blk) -> bf16x8 {
       return *reinterpret_cast<const bf16x8*>(smem + base + blk * 2048);
@@ -516,29 +518,30 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     // past the end); 2 = no refill; 3 = no refill and, in (t, 1), no reads of tile t+1 (there is
     // none).  The tail issues no dummy pieces (a re-read of the last k-tile kept the counts fixed:
     // 40 of every tile's 1064 pieces per wave, ~4 % of the DMA issue at K = 4096).
-    auto sub = [&](auto ph, auto pm, bf16x8 (&ca)[8], bf16x8 (&cb)[8], bf16x8 (&na)[8], bf16x8 (&nb)[8],
+    auto sub = [&](auto ph, auto pm, bf16x8 (&ca)[MB], bf16x8 (&cb)[8], bf16x8 (&na)[MB], bf16x8 (&nb)[8],
                    uint32_t sa, uint32_t sb, uint32_t da, uint32_t db, int t) {
       constexpr int PH = decltype(ph)::value, PM = decltype(pm)::value;
+      constexpr int GAP = MB == 8 ? 6 : 5;  // products between two of (t, 0)'s pieces
       constexpr bool READS = !(PH == 1 && PM == 3);
       // sa / sb: half-slot bytes of the fragments read here; da / db: B_{t+2}'s / A_{t+3}'s targets
       const uint32_t ba = sa + (PH == 0 ? fbA1 : fbA0), bb = sb + (PH == 0 ? fbB1 : fbB0);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int g = 0; g < 8; ++g) {
+      for (int g = 0; g < MB; ++g) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int n = g * 8 + j;
           acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cb[j], ca[g], acc[g][j], 0, 0, 0);
           if (n < 8) {
             if constexpr (READS) nb[n] = rd16(bb, n);
-          } else if (n < 16) {
+          } else if (n < 8 + MB) {
             if constexpr (READS) na[n - 8] = rd16(ba, n - 8);
           } else if (PH == 0 && PM <= 1 && n == 19) {  // frees tile t's half-slots for the refills
             lgkm_wait0();
             __builtin_amdgcn_s_barrier();
-          } else if (PH == 0 && PM <= 1 && n >= 22 && (n - 22) % 6 == 0 && (n - 22) / 6 < 7) {
-            pc(1, (n - 22) / 6, t + 2, da);
-          } else if (PH == 1 && PM <= 1 && n >= 19 && (n - 19) % 5 == 0 && (n - 19) / 5 < 9) {
+          } else if (PH == 0 && PM <= 1 && n >= 22 && (n - 22) % GAP == 0 && (n - 22) / GAP < 7) {
+            pc(1, (n - 22) / GAP, t + 2, da);
+          } else if (PH == 1 && PM <= 1 && n >= 19 && (n - 19) % 5 == 0 && (n - 19) / 5 < 1 + MB) {
             const int i = 7 + (n - 19) / 5;
             if (i < 8)
               pc(1, i, t + 2, da);
@@ -566,7 +569,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     issue_half(0, 1);
     issue_half(1, 1);
     issue_half(0, 2);
-    vm_wait_n<24>();
+    vm_wait_n<8 + 2 * MB>();
     __builtin_amdgcn_s_barrier();
     if constexpr (RS) {
       float sum = 0.f;
@@ -577,7 +580,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     }
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
-      fa0[g] = frag(0, 0, 0, g);
+      if (g < MB) fa0[g] = frag(0, 0, 0, g);
       fb0[g] = frag(1, 0, 1, g);
     }
     // half-slot bytes of tile t: S0 = (2t % 5) HS (A_t), S1 = ((2t + 1) % 5) HS (B_t), S2 / S3 =
@@ -590,12 +593,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       S2 = s4;
       S3 = s0;
     };
-    // vmcnt at the mid-tile wait: B_{t+1} must have landed; younger are A_{t+2} (8) + B_{t+2}'s
-    // first 7 pieces (15) in the steady state and at t = nk - 3, nothing from t = nk - 2 on
+    // vmcnt at the mid-tile wait: B_{t+1} must have landed; younger are A_{t+2} (MB) + B_{t+2}'s
+    // first 7 pieces in the steady state and at t = nk - 3, nothing from t = nk - 2 on
     for (int t = 0; t < nk - 3; ++t) {
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the previous sub-step's reads, explicitly
       sub(P0{}, P0{}, fa0, fb0, fa1, fb1, S0, S1, S0, S1, t);
-      vm_wait_n<15>();
+      vm_wait_n<7 + MB>();
       __builtin_amdgcn_s_barrier();
       sub(P1{}, P0{}, fa1, fb1, fa0, fb0, S2, S3, S0, S1, t);
       rotate();
@@ -604,7 +607,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       const int t = nk - 3;
       __builtin_amdgcn_s_waitcnt(0xc07f);
       sub(P0{}, P1{}, fa0, fb0, fa1, fb1, S0, S1, S0, S1, t);
-      vm_wait_n<15>();
+      vm_wait_n<7 + MB>();
       __builtin_amdgcn_s_barrier();
       sub(P1{}, P1{}, fa1, fb1, fa0, fb0, S2, S3, S0, S1, t);
       rotate();
@@ -688,7 +691,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 
   lgkm_wait0();
   __builtin_amdgcn_s_barrier();  // every wave is done with the ring (its last DMAs retired above)
-  if constexpr (!NARROW) end(acc, std::integral_constant<int, 8>{}, wm, wn);
+  if constexpr (!NARROW) end(acc, std::integral_constant<int, MB>{}, wm, wn);
 }
 
 }  // namespace k8sllm
@@ -720,6 +723,16 @@ static Strips narrow_strips(long M, long N, long K, int epi) {
   take(64, 128, 0.42f);
   take(128, 128, 0.72f);
   return best;
+}
+
+// Row blocks a wave of a dense product's tiles: 7 (tiles of 224 rows) where their rounds take less than those of 256 rows.
+static int row_blocks(long M, long n_nt, long K) {
+  auto us = [&](int blocks) {
+    const long n = (M + 32 * blocks - 1) / (32 * blocks) * n_nt, over = n % kTileCus;
+    const float last = over == 0 ? 0.f : over <= kFineTiles ? 0.35f : over <= kStripTiles ? 0.5f : 1.f;
+    return ((float)(n / kTileCus) + last) * (8.f + (blocks == 8 ? 1.45f : 1.31f) * (K >> 6));
+  };
+  return us(7) < 0.98f * us(8) ? 7 : 8;
 }
 
 // Dense (offsets == nullptr): Y [M][N] (SwiGLU: [M][N / 2]) = X [M][K] . W[N][K]^T.
@@ -827,19 +840,27 @@ extern "C" int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void
   if (N <= 0 || N % 16 || K % 64 || K < 192 || (glu ? f <= 0 || f % 16 || N < 2 * f : f != 0)) return -1;
   if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31) || 256L * N * 2 >= (1L << 31)) return -3;
   const TileEpi ep{nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, f, (bf16_t*)Y2, nullptr, 1, 0};
-  const int n_mt = (M + 255) / 256, n_nt = glu ? (f + 127) / 128 + (N - 2 * f + 255) / 256 : (N + 255) / 256;
+  const int n_nt = glu ? (f + 127) / 128 + (N - 2 * f + 255) / 256 : (N + 255) / 256, mb = row_blocks(M, n_nt, K), n_mt = (M + 32 * mb - 1) / (32 * mb);
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
   const long over = nwg % kTileCus;
   const int strips = over > 0 && over <= kStripTiles;
   const long groups = nwg + (strips ? strip_groups(over) : 0);
-#define K8_TILE_UNIT(EPI_)                                                                                             \
-  hipLaunchKernelGGL((strips ? &gemm_w4_kernel<EPI_, false, 1, false> : &gemm_w4_kernel<EPI_, false, 1, false, 0, false, false>), dim3((unsigned)groups), dim3(256), 0, s, (const bf16_t*)X, \
-                     (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0, strips)
+#define K8_TILE_UNIT_OF(EPI_, CUT_, MB_)                                                                                          \
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI_, false, 1, false, 0, false, CUT_, MB_>), dim3((unsigned)groups), dim3(256), 0, s,       \
+                     (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, (const int*)nullptr, 1, M, N, K, 0L, n_mt, n_nt, ep, 0, strips)
+#define K8_TILE_UNIT(EPI_)                                                              \
+  do {                                                                                  \
+    if (mb == 8 && strips) K8_TILE_UNIT_OF(EPI_, true, 8);                              \
+    else if (mb == 8) K8_TILE_UNIT_OF(EPI_, false, 8);                                  \
+    else if (strips) K8_TILE_UNIT_OF(EPI_, true, 7);                                    \
+    else K8_TILE_UNIT_OF(EPI_, false, 7);                                               \
+  } while (0)
   if (epi == TILE_EPI_GELU_GLU) K8_TILE_UNIT(TILE_EPI_GELU_GLU);
   else if (epi == TILE_EPI_SILU_GLU) K8_TILE_UNIT(TILE_EPI_SILU_GLU);
   else if (epi == TILE_EPI_RELU_GLU) K8_TILE_UNIT(TILE_EPI_RELU_GLU);
   else K8_TILE_UNIT(TILE_EPI_RELU_SQ);
 #undef K8_TILE_UNIT
+#undef K8_TILE_UNIT_OF
   return (int)hipGetLastError();
 }

@@ -229,6 +229,24 @@ def test_gemm_tile_last_round_in_fine_strips(M, N, K, f):
     assert torch.equal(y2, z[:, 2 * f:])
 
 
+@pytest.mark.parametrize("M,N,K,f", [  # tiles of 224 rows: one, two and 32 strips' tiles behind rounds, none; the last tile of 1, 33 and 224 rows; three k-tiles
+    (224 * 28 + 1, 4096, 192, 1984), (224 * 14 + 33, 4096, 256, 2048), (6403, 4096, 320, 2000), (7830, 13312, 192, 5632), (224 * 16, 8192 - 128, 640, 3072),
+])
+def test_gemm_tile_units_of_224_rows(M, N, K, f):
+    """Units and squared ReLU on tiles of 224 rows where those are fewer rounds: the bits of the other schedule's whole tiles."""
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    z = ops.gemm_tile(x, w, algo=0)
+    y, y2 = torch.empty(M, f, dtype=torch.bfloat16, device="cuda"), torch.empty(M, N - 2 * f, dtype=torch.bfloat16, device="cuda")
+    ops.native().gemm_tile_unit(y, y2, x, w, 7)  # ReLU: exact but for the product's rounding
+    assert torch.equal(y, (z[:, :f].float().clamp(min=0) * z[:, f:2 * f].float()).to(torch.bfloat16))
+    assert torch.equal(y2, z[:, 2 * f:])
+    q = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    ops.native().gemm_tile_unit(q, None, x, w, 8)
+    assert torch.equal(q, (z.float().clamp(min=0) ** 2).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("M,N,K,packed", [
     (1, 128, 192, False), (65, 4096, 4096, True), (43, 6144, 4096, True), (257, 1024, 8192, False), (512, 512, 1088, False), (80, 28672, 4096, True),
     (600, 6144, 2112, True), (1000, 1024, 4096, False), (70, 320, 512, False), (260, 4096, 2048, True),  # (64 columns: one round of strips, and more)
