@@ -428,11 +428,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     // The same instructions in the same order of k as a whole tile's, so the same bits.
     constexpr int RB = COLS < 256 && !TALL ? 1 : 2, AP = TALL ? 4 : 2, BP = COLS / 32, NJ = COLS < 128 ? COLS / 16 : 8;
     constexpr int SA = AP * 4096, SS = SA + BP * 4096, SLOTS = 5 * HS / SS;
-    f32x4 acc[RB][NJ];
+    f32x4 acc[RB][NJ];  // each its own zero: of one value for all, hipcc moved them all on, in every k-tile (36 moves beside 16 products in 64 x 128)
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NJ; ++j) {
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(acc[i][j]));
+      }
     bf16x8 fa0[RB], fb0[NJ], fa1[RB], fb1[NJ];
     auto next = [&](int slot) { return slot + SS == SLOTS * SS ? 0 : slot + SS; };
     auto fill = [&](int kt, int slot) {
@@ -699,7 +702,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 using namespace k8sllm;
 
 // The strips that a dense product of few tiles goes in: the least of rounds x (k-tiles x rate + 6 us for its start and end).  Rates, us a k-tile with the
-// chip full: 64 x 64 0.26 (plain products), 64 x 128 0.42, 128 x 128 0.72; a tile 1.25, 0.8 where few go as strips of 256 columns.  us, tiles / 128 x 128 /
+// chip full: 64 x 64 0.26 (plain products), 64 x 128 0.42, 128 x 128 0.72; a tile 1.25, 0.8 where few go as strips of 256 columns.  (Of before the strips'
+// accumulators stayed where they are; now 0.22, 0.35 and 0.55: 4096 x 14336, 400 rows 94 / 81, 600 rows 150 / 120; 6144 x 4096, 144 rows 29 / 26, 600 rows
+// 47 / 39; with SwiGLU 28672 x 4096, 80 rows 51 / 45.  By those the choice would be the same but for 4096 x 14336 from 1025 rows.)  us, tiles / 128 x 128 /
 // 64 x 128 / 64 x 64, packed weights: 4096 x 4096, 80 rows 56 / - / 35 / 23, 300 56 / - / 35, 600 59 / 54; 4096 x 14336, 80 rows 168 / - / 98 / 58, 400 167 /
 // - / 104, 600 178 / 161; 6144 x 4096 with RoPE, 80 rows 78 / - / 36, 300 81 / - / 38, 400 - / 57 / 67, 600 83 / 58 / 71, 800 84 / 102 (two rounds); 28672 x
 // 4096 with SwiGLU, 80 rows 90 / 62 / 75 (two rounds), 200 90 / 107 (two rounds).  Rounds are an XCD's: it has whole columns' strips and 32 CUs, so 12
@@ -725,7 +730,9 @@ static Strips narrow_strips(long M, long N, long K, int epi) {
   return best;
 }
 
-// Row blocks a wave of a dense product's tiles: 7 (tiles of 224 rows) where their rounds take less than those of 256 rows.
+// Row blocks a wave of a dense product's tiles: 7 (tiles of 224 rows) where their rounds take less than those of 256 rows, by a tile's time of 8 us and 1.45
+// (1.31) a k-tile and a last round's part of it: 0.35 as fine strips, 0.5 as four a tile.  us, 256 / 224 rows: units of 6403 x 4096 x 1024 (1.6 rounds / 1.8) 57 / 53.5,
+// 3137 x 6656 x 1024 58.5 / 52.7, 1822 x 11264 x 2048 94 / 85.5, 1374 x 26112 x 4096 256 / 239; of 45 none is slower.
 static int row_blocks(long M, long n_nt, long K) {
   auto us = [&](int blocks) {
     const long n = (M + 32 * blocks - 1) / (32 * blocks) * n_nt, over = n % kTileCus;
