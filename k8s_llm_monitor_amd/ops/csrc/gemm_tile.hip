@@ -77,13 +77,12 @@ __device__ __forceinline__ void lgkm_wait0() { asm volatile("s_waitcnt lgkmcnt(0
 // A strip has accumulators and fragments of its own: with the tile's, hipcc spilled (10 us of 241 in the grouped product below) or moved accumulators in the tile's loop.
 // us, whole tiles / strips: 780 tiles of K 2048 (gated unit) 224 / 183; 258 of K 4096 172 / 157; grouped, 8 experts, K 2048, 1072 294 / 229 and 536
 // 148 / 121; 320 of K 4096 in 4 experts 204 / 170.
+// So do residual, rotation and row scale, a strip's own at its end; with tiles of 224 rows (row_blocks), us before / after: residual, 4096 columns of K 14336,
+// 520 rows 228 / 145, 1200 rows 226 / 203, 4300 rows 554 / 397, 5000 rows 554 / 471; of K 4096, 1024 rows 78 / 50, 4300 rows 174 / 127; 6144 x 4096 with RoPE, 3000 rows
+// 179 / 129; SwiGLU 28672 x 4096, 1200 rows 271 / 247, 1636 rows 366 / 324; of 72 such products of 520 to 16000 rows none is slower by more than 0.5 %.
 // Products without such tiles have a kernel without strips (CUT false): 6000 x 12288 x 1408, squared ReLU, 188.5 us with both in one, 186.6 without.
 // Grouped, the count of tiles is known on the device only: each workgroup sums it over the experts, up to kStripExperts of them.
 constexpr int kTileCus = 256, kStripTiles = 64, kStripExperts = 32;
-template <int EPI, int SCH, bool RS>
-constexpr bool tile_strips() {
-  return SCH == 1 && !RS && EPI != TILE_EPI_ROPE && EPI != TILE_EPI_RESID;
-}
 constexpr int kFineTiles = 32;  // up to this many such tiles go as eight strips of 64 rows x 128 columns each
 // workgroups that strips of up to this many tiles add
 static inline long strip_groups(long tiles) { return (tiles + 7) / 8 * (tiles <= kFineTiles ? 64 : 32) - tiles; }
@@ -102,7 +101,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   const int wm = NARROW ? wave : wave >> 1, wn = NARROW ? 0 : wave & 1;
 
   // ---- logical tile: bijective XCD remap, then groups of 8 m-tiles ----
-  constexpr bool STRIPS = tile_strips<EPI, SCH, RS>() && !NARROW && CUT;
+  constexpr bool STRIPS = SCH == 1 && !NARROW && CUT;
   int mts = n_mt;
   if (GROUPED && STRIPS && strips) {  // the tiles that there are
     mts = 0;
@@ -124,7 +123,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int q8 = nwg >> 3, r8 = nwg & 7;
     lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
   }
-  static_assert(MB == 8 || (!GROUPED && SCH == 1 && !RS && !NARROW && EPI != TILE_EPI_RESID && EPI != TILE_EPI_ROPE));
+  static_assert(MB == 8 || (!GROUPED && SCH == 1 && !NARROW));
   constexpr int TM = !NARROW ? 32 * MB : TALL ? 128 : 64, TN = NARROW ? NARROW : 256;
   constexpr int GM = 8;
   const int grp = lid / (GM * n_nt), first_m = grp * GM;
@@ -257,15 +256,15 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   uint4 nwv{};
   if constexpr (EPI == TILE_EPI_RESID) nwv = *reinterpret_cast<const uint4*>(ep.norm_w + n0 + wn * 128 + cc * 8);
   // RS: each thread's row scale through LDS (after the staging area) to the lanes holding the row
-  float sc[8];
+  float sc[RB];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) sc[i] = 1.f;
+  for (int i = 0; i < RB; ++i) sc[i] = 1.f;
   if constexpr (RS) {
     float* inv_s = reinterpret_cast<float*>(smem + 4 * 128 * (128 * 2 + 16));
     inv_s[threadIdx.x] = rs_inv;
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sc[i] = inv_s[wm * 128 + i * 16 + ml];
+    for (int i = 0; i < RB; ++i) sc[i] = inv_s[wm * 16 * RB + i * 16 + ml];
   }
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
@@ -327,18 +326,18 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     // lane (rr, cc): row rr + 4b, columns cc*8 .. +7 of the wave's quarter; N % 128 == 0 (host)
     const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
     const __amdgpu_buffer_rsrc_t rhw = rsrc(ep.hw + (long)row0 * N, (long)mrows * N * 2);
-    const uint32_t ro = (uint32_t)(((wm * 128 + rr) * N + n0 + wn * 128 + cc * 8) * 2);
+    const uint32_t ro = (uint32_t)(((wm * 16 * RB + rr) * N + n0 + wn * 128 + cc * 8) * 2);
     float wf[8];
     unpack8(nwv, wf);
     const int ss_np = N >> 7, ssc = (n0 + wn * 128) >> 7;
 #pragma unroll
-    for (int b = 0; b < 32; ++b) {
+    for (int b = 0; b < 4 * RB; ++b) {
       const int r = rr + 4 * b;
       const uint4 yv = *reinterpret_cast<const uint4*>(stage + r * RS_ + cc * 16);
       float y[8], rv[8], h[8], hw[8];
       unpack8(yv, y);
       const u32x4 rb = resq[b & 15];
-      if (b < 16) resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * (b + 16) * N * 2), 0, 0);
+      if (b + 16 < 4 * RB) resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * (b + 16) * N * 2), 0, 0);
       unpack8(uint4{rb[0], rb[1], rb[2], rb[3]}, rv);
       float ss = 0.f;
 #pragma unroll
@@ -352,7 +351,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       __builtin_amdgcn_raw_buffer_store_b128(u32x4{hq.x, hq.y, hq.z, hq.w}, rres, off, 0, 0);
       __builtin_amdgcn_raw_buffer_store_b128(u32x4{wq.x, wq.y, wq.z, wq.w}, rhw, off, 0, 0);
       ss = row16_sum(ss);
-      const int grow = wm * 128 + r;
+      const int grow = wm * 16 * RB + r;
       if (cc == 0 && grow < mrows) ep.ss_out[(long)(row0 + grow) * ss_np + ssc] = ss;
     }
     return;
@@ -460,6 +459,15 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[g], acc[g][j], 0, 0, 0);
     };
+    if constexpr (RS) {  // in a tile's order
+      const float* rp = ep.rs_part + (long)(row0 + min((int)threadIdx.x, mrows - 1)) * ep.rs_np;
+      float sum = 0.f;
+      for (int j = 0; j < ep.rs_np; j += 4) {
+        const f32x4 q = *reinterpret_cast<const f32x4*>(rp + j);
+        sum += (q[0] + q[1]) + (q[2] + q[3]);
+      }
+      rs_inv = rsqrtf(sum / (float)K + ep.rs_eps);
+    }
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) fill(i, i * SS);
     vm_wait_n<(SLOTS - 1) * (AP + BP)>();
@@ -479,6 +487,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       __builtin_amdgcn_sched_barrier(0);
       mul(fa1, fb1);
       at = next(at);
+    }
+    if constexpr (EPI == TILE_EPI_RESID) {
+      const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
+      const uint32_t ro = (uint32_t)(((wm * 16 * RB + (lane >> 4)) * N + n0 + wn * 128 + (lane & 15) * 8) * 2);
+#pragma unroll
+      for (int b = 0; b < 4 * RB; ++b) resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * b * N * 2), 0, 0);
     }
     vm_wait_n<0>();
     lgkm_wait0();
@@ -630,7 +644,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       sub(P0{}, P3{}, fa0, fb0, fa1, fb1, S0, S1, S0, S1, t);
       if constexpr (EPI == TILE_EPI_RESID) {
         const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
-        const uint32_t ro = (uint32_t)(((wm * 128 + (lane >> 4)) * N + n0 + wn * 128 + (lane & 15) * 8) * 2);
+        const uint32_t ro = (uint32_t)(((wm * 16 * MB + (lane >> 4)) * N + n0 + wn * 128 + (lane & 15) * 8) * 2);
 #pragma unroll
         for (int b = 0; b < 16; ++b)
           resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * b * N * 2), 0, 0);
@@ -780,9 +794,8 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   // 32-bit DMA offsets (X: relative to the tile's first row; W: within one expert / n-tile)
   if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31)) return -3;
   if (epi == TILE_EPI_RESID && 256L * N * 2 >= (1L << 31)) return -3;
-  const int n_mt = (M + 255) / 256 + (grouped ? E : 0), n_nt = (N + 255) / 256;
-  const long nwg = (long)n_mt * n_nt;
-  if (nwg > (1L << 30)) return -2;
+  const int n_nt = (N + 255) / 256;
+  if (((M + 255) / 256 + (grouped ? E : 0)) * (long)n_nt > (1L << 30)) return -2;
   const Strips narrow = !grouped && algo == 1 && !rs && epi != TILE_EPI_RESID ? narrow_strips(M, N, K, epi) : Strips{};
   if (narrow.rows) {
     const int rows = (M + narrow.rows - 1) / narrow.rows, cols = N / narrow.cols;
@@ -801,15 +814,25 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
 #undef K8_TILE_NARROW
     return (int)hipGetLastError();
   }
-  const bool cut = algo == 1 && !rs && epi != TILE_EPI_ROPE && epi != TILE_EPI_RESID && E <= kStripExperts;
+  const bool cut = algo == 1 && (!grouped || E <= kStripExperts);
+  // (interleaved per 128 rows, gate and up are not on the path that serves dense models)
+  const int mb = algo == 1 && !grouped && epi != TILE_EPI_SWIGLU ? row_blocks(M, n_nt, K) : 8;
+  const int n_mt = grouped ? (M + 255) / 256 + E : (M + 32 * mb - 1) / (32 * mb);
+  const long nwg = (long)n_mt * n_nt;
   const long over = nwg % kTileCus;
   const int strips = cut && (grouped || (over > 0 && over <= kStripTiles));
   const dim3 grid((unsigned)(nwg + (!strips ? 0 : grouped ? 4 * kStripTiles : strip_groups(over))));
-#define K8_TILE_LAUNCH(EPI_, G_, SCH_, RS_)                                                                          \
-  hipLaunchKernelGGL((strips ? &gemm_w4_kernel<EPI_, G_, SCH_, RS_>                                                  \
-                             : &gemm_w4_kernel<EPI_, G_, SCH_, RS_, 0, false, !tile_strips<EPI_, SCH_, RS_>()>),     \
+#define K8_TILE_OF(EPI_, G_, SCH_, RS_, MB_)                                                                          \
+  hipLaunchKernelGGL((strips ? &gemm_w4_kernel<EPI_, G_, SCH_, RS_, 0, false, true, MB_>                              \
+                             : &gemm_w4_kernel<EPI_, G_, SCH_, RS_, 0, false, SCH_ == 0, MB_>),                       \
                      grid, dim3(256), 0, s, (const bf16_t*)X,                                                        \
                      (const bf16_t*)W, (bf16_t*)Y, offsets, E, M, N, K, w_es, n_mt, n_nt, ep, wpk, strips)
+#define K8_TILE_LAUNCH(EPI_, G_, SCH_, RS_)                                                                          \
+  do {                                                                                                               \
+    constexpr int MB7 = G_ || SCH_ == 0 || EPI_ == TILE_EPI_SWIGLU ? 8 : 7;                                          \
+    if (mb == 8) K8_TILE_OF(EPI_, G_, SCH_, RS_, 8);                                                                 \
+    else K8_TILE_OF(EPI_, G_, SCH_, RS_, MB7);                                                                       \
+  } while (0)
 #define K8_TILE_SCH(SCH_)                                                                                            \
   if (grouped) {                                                                                                     \
     if (epi == TILE_EPI_SWIGLU) K8_TILE_LAUNCH(TILE_EPI_SWIGLU, true, SCH_, false);                                  \
@@ -834,6 +857,7 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   }
 #undef K8_TILE_SCH
 #undef K8_TILE_LAUNCH
+#undef K8_TILE_OF
   return (int)hipGetLastError();
 }
 

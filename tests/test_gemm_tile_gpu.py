@@ -247,6 +247,36 @@ def test_gemm_tile_units_of_224_rows(M, N, K, f):
     assert torch.equal(q, (z.float().clamp(min=0) ** 2).to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("M,N,K", [  # behind rounds: 1, 32, 33 and 64 tiles, none; tiles of 224 rows and of 256; a last tile of one row
+    (4097, 4096, 512), (4608, 4096, 512), (3073, 5376, 1024), (5120, 4096, 512), (1636, 28672, 512), (3585, 4096, 512), (700, 6144, 1536), (257, 1024, 512),
+])
+def test_gemm_tile_fused_ends_of_strips(M, N, K):
+    """Residual, rotation and row scale at the end of strips and of tiles of 224 rows: the bits of the plain product on whole tiles, finished here.  (Scales are
+    powers of two, so that they commute with every rounding.)"""
+    g = torch.Generator().manual_seed(8)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    wr = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    w = ops.pack_skinny(wr)
+    z = ops.gemm_tile(x, wr, algo=0)
+    r, nw = torch.randn(M, N, generator=g).to(torch.bfloat16).cuda(), (torch.rand(N, generator=g) + 0.5).to(torch.bfloat16).cuda()
+    h = (z.float() + r.float()).to(torch.bfloat16)
+    hw, ss = ops.gemm_tile_resid(x, w, r, nw)
+    assert torch.equal(r, h)
+    assert torch.equal(hw, (h.float() * nw.float()).to(torch.bfloat16))
+    torch.testing.assert_close(ss, (h.float() ** 2).view(M, N // 128, 128).sum(2), rtol=1e-5, atol=1e-5)  # 128 fp32 terms
+    row = torch.arange(M, device=DEV)
+    scale = (2.0 ** (row % 5 - 2)).float()[:, None]
+    part = torch.zeros(M, K // 128, device=DEV)
+    part[:, 1:2] = K / scale ** 2  # 1 / rms = scale
+    pos, cs = (row % 97).to(torch.int32), torch.rand(97, 128, generator=g).cuda()
+    heads = N // 128 - 3
+    want = ops.gemm_tile(x, wr, algo=0, rope=(pos, cs, heads))
+    assert torch.equal(ops.gemm_tile(x, w, algo=1, rope=(pos, cs, heads)), want)
+    assert torch.equal(ops.gemm_tile(x, w, algo=1, rope=(pos, cs, heads), rowscale=(part, 0.0)), (want.float() * scale).to(torch.bfloat16))
+    big = (x.float() * scale).to(torch.bfloat16)
+    assert torch.equal(ops.gemm_tile(x, w, swiglu=8, algo=1, rowscale=(part, 0.0)), ops.gemm_tile(big, wr, swiglu=8, algo=0))
+
+
 @pytest.mark.parametrize("M,N,K,packed", [
     (1, 128, 192, False), (65, 4096, 4096, True), (43, 6144, 4096, True), (257, 1024, 8192, False), (512, 512, 1088, False), (80, 28672, 4096, True),
     (600, 6144, 2112, True), (1000, 1024, 4096, False), (70, 320, 512, False), (260, 4096, 2048, True),  # (64 columns: one round of strips, and more)
