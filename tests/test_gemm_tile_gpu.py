@@ -277,6 +277,29 @@ def test_gemm_tile_fused_ends_of_strips(M, N, K):
     assert torch.equal(ops.gemm_tile(x, w, swiglu=8, algo=1, rowscale=(part, 0.0)), ops.gemm_tile(big, wr, swiglu=8, algo=0))
 
 
+@pytest.mark.parametrize("M,N,K", [  # tiles of 224 and of 256 rows, alone, behind 64 x 256 strips and in front of 64 x 128 ones
+    (1, 128, 192), (300, 384, 192), (4097, 384, 320), (9000, 384, 192), (4097, 4224, 192), (7937, 4224, 192), (10240, 4224, 192), (4609, 4224, 256),
+    (1025, 28544, 192), (1537, 28544, 192),
+])
+def test_gemm_tile_residual_behind_half_a_tile(M, N, K):
+    """N % 256 == 128: the last tile's second 128 columns are not there.  Every row's residual, weighted row and sums of squares are the plain product's,
+    finished here, and nothing behind the buffers' ends is written."""
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    nw = (torch.rand(N, generator=g) + 0.5).to(torch.bfloat16).cuda()
+    z, r = ops.gemm_tile(x, w, algo=0), torch.randn(M, N, generator=g).to(torch.bfloat16).cuda()
+    h = (z.float() + r.float()).to(torch.bfloat16)
+    bufs = [torch.full((M * n + 512,), 7.0, dtype=dt, device=DEV) for n, dt in ((N, torch.bfloat16), (N, torch.bfloat16), (N // 128, torch.float32))]
+    res, hw, ss = (b[:-512].view(M, -1) for b in bufs)
+    for wt in (w, ops.pack_skinny(w)):
+        res.copy_(r)
+        ops.gemm_tile_resid(x, wt, res, nw, hw, ss)
+        assert torch.equal(res, h) and torch.equal(hw, (h.float() * nw.float()).to(torch.bfloat16))
+        torch.testing.assert_close(ss, (h.float() ** 2).view(M, N // 128, 128).sum(2), rtol=1e-5, atol=1e-5)  # 128 fp32 terms
+        assert all(bool((b[-512:] == 7.0).all()) for b in bufs)
+
+
 @pytest.mark.parametrize("M,N,K,packed", [
     (1, 128, 192, False), (65, 4096, 4096, True), (43, 6144, 4096, True), (257, 1024, 8192, False), (512, 512, 1088, False), (80, 28672, 4096, True),
     (600, 6144, 2112, True), (1000, 1024, 4096, False), (70, 320, 512, False), (260, 4096, 2048, True),  # (64 columns: one round of strips, and more)
