@@ -71,22 +71,44 @@ __device__ __forceinline__ ChunkAt chunk_at(const int* __restrict__ cu, int S, i
   return {-1, 0, 0, 0, 0};
 }
 
-// Which segment the r-th group of workgroups takes, where one workgroup a compute unit is `round` groups: the longest ones first, one a unit, then
-// the shortest first, which come beside them (workgroups go to the units in turn), and so on.  A chain of tokens beside another takes up to twice as
-// long, so that a step of prompts of different lengths took as long as its two longest ones on one unit: 13 prompts of 45 to 901 tokens, us, in the
-// step's order / so: selective scan of 2048 channels 144 / 126, delta rule of 8 heads 72 / 58, wkv of 16 50 / 43.  More than 64 segments: from
-// the last one on (a step's prompts come after its running sequences).
-__device__ __forceinline__ int segment_in_turn(const int* __restrict__ cu, int S, int r, int round) {
-  if (S <= 1 || S > 64) return S - 1 - r;
-  const int k = r / round;
-  if (k & 1) r = min((k + 1) * round, S) - 1 - (r - k * round);
-  const int lane = threadIdx.x & 63, n = lane < S ? cu[lane + 1] - cu[lane] : -1;
-  int rank = 0;
-  for (int j = 0; j < S; ++j) {
-    const int m = __builtin_amdgcn_readlane(n, j);
-    rank += m > n || (m == n && j < lane);
+// Which segment the r-th group of ``per`` workgroups takes.  The longest ones first, one workgroup a unit, then those that come beside them from the
+// shortest on, and so on: workgroups go to the units in turn, and a chain of tokens beside another takes up to twice as long, so that a step of
+// prompts of different lengths took as long as its two longest ones on one unit.  us, in the step's order / so: 13 prompts of 45 to 901 tokens, selective
+// scan of 2048 channels 150 / 123, delta rule of 8 heads 110 / 104, linear attention of 16 85 / 75, wkv of 16 87 / 84; 32 such prompts, linear attention of
+// 8 108 / 87.  No more workgroups than units, more than ``most`` of them or more than 64 segments: from the last one on (a step's prompts come after its
+// running sequences).  Short segments behind one another pay for the choice (64 of 5 to 94 tokens, delta rule of 8 heads 93 / 104, linear attention of 16
+// 59 / 67), and over many rounds they even out by themselves (64 of 45 to 901 tokens, delta rule of 16 heads 811 / 812), so the chunks' scans make none
+// beyond four rounds; the selective scan, whose tokens take longest, does (64 of 5 to 94 tokens, 4096 channels 103 / 69, of 45 to 901 880 / 535).  Equal
+// lengths cost nothing or 1 us (64 of 64 tokens, linear attention of 8 heads 31.0 / 31.4; 16 of 500 42 / 42).
+// The lanes hold the whole table, so that nothing is loaded behind the choice; the r-th longest is found from the highest bit of the lengths on.
+struct SegAt {
+  int seg, slot, t0, t1;  // its rows: t0 .. t1 - 1
+};
+__device__ __forceinline__ SegAt segment_in_turn(const int* __restrict__ cu, const int* __restrict__ slot, int S, int r, int per,
+                                                 int most = 1024) {
+  if (S * per <= 256 || S * per > most || S > 64) {
+    const int s = S - 1 - r;
+    return {s, slot[s], cu[s], cu[s + 1]};
   }
-  return __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(lane < S && rank == r)));
+  const int round = max(1, 256 / per);
+  const int lane = threadIdx.x & 63, i = min(lane, S - 1), c = cu[i], n = cu[i + 1] - c, sl = slot[i], k = r / round;
+  if (k & 1) r = min((k + 1) * round, S) - 1 - (r - k * round);
+  // those that may be the r-th longest (of equal ones in the step's order)
+  unsigned long long left = S == 64 ? ~0ull : (1ull << S) - 1;
+  if (__ballot(n != __builtin_amdgcn_readfirstlane(n)) != 0)
+    for (int bit = __ballot(n >> 12) ? 30 : 11; bit >= 0 && (left & (left - 1)); --bit) {
+      const unsigned long long on = left & __ballot((n >> bit) & 1);
+      const int more = __popcll(on);
+      if (r < more) {
+        left = on;
+      } else {
+        r -= more;
+        left &= ~on;
+      }
+    }
+  const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(left >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)left, 0));
+  const int s = __builtin_ctzll(__ballot(before == r) & left), t0 = __builtin_amdgcn_readlane(c, s);
+  return {s, __builtin_amdgcn_readlane(sl, s), t0, t0 + __builtin_amdgcn_readlane(n, s)};
 }
 
 __device__ __forceinline__ int first_chunk(const int* __restrict__ cu, int s) {

@@ -287,14 +287,17 @@ __global__ __launch_bounds__(512, 2) void decay_chunk_scan_kernel(float* __restr
   if (pair >= (MODE == kWhole ? S_ : n_span) * H) return;
   const int h = pair % H, dvb = zb * NV, sp_i = n_span - 1 - pair / H;
   ChunkAt at = {0, 0, 0, 0, 1};
+  SegAt own;
   if (MODE == kWhole) {
-    at.seg = segment_in_turn(cu, S_, pair / H, max(1, 256 / (H * nz)));
+    own = segment_in_turn(cu, slot, S_, pair / H, H * nz);
+    at.seg = own.seg;
   } else {
     at = chunk_at(cu, S_, sp_i, span * kChunk);
-    if (at.seg < 0 || (MODE == kSpanEnds && (at.k == at.count - 1 || slot[at.seg] < 0))) return;
+    if (at.seg < 0) return;
+    own = {at.seg, slot[at.seg], at.row, at.row + at.n};
+    if (MODE == kSpanEnds && (at.k == at.count - 1 || own.slot < 0)) return;
   }
-  const int s = at.seg;
-  const int sl = slot[s], t0 = MODE == kWhole ? cu[s] : at.row, t1 = MODE == kWhole ? cu[s + 1] : at.row + at.n;
+  const int s = own.seg, sl = own.slot, t0 = own.t0, t1 = own.t1;
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const bool outs = wave < 4;  // wave-uniform

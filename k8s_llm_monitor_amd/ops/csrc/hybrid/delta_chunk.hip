@@ -291,8 +291,8 @@ __global__ __launch_bounds__(512, 2) void delta_scan_kernel(float* __restrict__ 
   // all column blocks of a (segment, head) pair on one XCD: its L2 then serves their common operands
   const int nz = dv / NV, pair = (blockIdx.x & 7) + 8 * (blockIdx.x / (8 * nz)), zb = (blockIdx.x >> 3) % nz;
   if (pair >= S_ * H) return;
-  const int s = segment_in_turn(cu, S_, pair / H, max(1, 256 / (H * nz))), h = pair % H, dvb = zb * NV, g = h / (H / Gk);
-  const int sl = slot[s], t0 = cu[s], t1 = cu[s + 1];
+  const SegAt at = segment_in_turn(cu, slot, S_, pair / H, H * nz);
+  const int s = at.seg, sl = at.slot, t0 = at.t0, t1 = at.t1, h = pair % H, dvb = zb * NV, g = h / (H / Gk);
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const bool outs = wave < 4;  // wave-uniform

@@ -53,18 +53,22 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   __shared__ float dts[TB][PB], us[TB][PB];
   __shared__ float ys[TB][PB + 64 / LPC];  // padded: the lanes of a channel write neighbouring rows to different banks
   ChunkAt at = {0, 0, 0, 0, 1};
+  SegAt own;
   int by = blockIdx.y;  // which channels
   if (MODE == kWhole) {
-    const int i = blockIdx.x + gridDim.x * blockIdx.y, groups = gridDim.y;
-    by = i % groups;
-    at.seg = segment_in_turn(cu, n_seg, i / groups, max(1, 256 / groups));
+    // (segments side by side within a round: an XCD has few of them, whose tokens its L2 then holds for all channels)
+    const int i = blockIdx.x + gridDim.x * blockIdx.y, groups = gridDim.y, round = min(max(1, 256 / groups), n_seg);
+    const int k = i / (round * groups), j = i - k * round * groups, m = min(round, n_seg - k * round);
+    by = j / m;
+    own = segment_in_turn(cu, slot, n_seg, k * round + j - by * m, groups, 1 << 30);
+    at.seg = own.seg;
   } else {
     at = chunk_at(cu, n_seg, blockIdx.x, span);
-    if (at.seg < 0 || (MODE == kSpanEnds && (at.k == at.count - 1 || slot[at.seg] < 0))) return;
+    if (at.seg < 0) return;
+    own = {at.seg, slot[at.seg], at.row, at.row + at.n};
+    if (MODE == kSpanEnds && (at.k == at.count - 1 || own.slot < 0)) return;
   }
-  const int s = at.seg;
-  const int sl = slot[s];
-  const int t0 = MODE == kWhole ? cu[s] : at.row, t1 = MODE == kWhole ? cu[s + 1] : at.row + at.n;
+  const int s = own.seg, sl = own.slot, t0 = own.t0, t1 = own.t1;
   const int pc = threadIdx.x % PB, tt0 = threadIdx.x / PB;  // staging: channel pc, tokens tt0 + LPC u
   const int cs = by * PB + pc;
   const bool slive = cs < C;

@@ -765,6 +765,40 @@ def test_segments_in_turn(lens):
                 assert torch.equal(got, want[a:a + n] if got.shape[0] == n and want.shape[0] == T else want[s:s + 1])
 
 
+@pytest.mark.parametrize("lens", [[130, 0, 64, 5, 5, 257, 1, 90, 65, 3, 700], [70] * 12, [9 * (i % 8) for i in range(42)], [(i * 37) % 150 for i in range(43)],
+                                  [4200 if i == 5 else (i * 53) % 120 for i in range(20)]])
+def test_segments_in_turn_over_rounds(lens):
+    """More workgroups (24 a segment) than units, up to four rounds of them and one segment more: linear attention, the delta rule, decays per channel with
+    a bonus and, of 20 workgroups a segment, the selective scan.  A prompt alone in its step, which no choice is made for, has the same bits."""
+    g = _g(80)
+    S, H, dk, dv, C, N = len(lens), 24, 32, 16, 1280, 16
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    ctx, slot, T = _i32([0] * S).cuda(), _i32([i if i != 4 else -1 for i in range(S)]).cuda(), sum(lens)  # the fifth is padding
+    qkv, z, beta = _r(g, T, H * (2 * dk + dv), dt=BF).cuda(), _r(g, T, H * dk, dt=BF).cuda(), _r(g, T, H, dt=BF).cuda()
+    dec, zb, al, u = torch.rand(H, generator=g).cuda(), _r(g, H * dk).cuda(), _r(g, H).cuda(), _r(g, H, dk).cuda()
+    x, q, dt, gate = (_r(g, T, n, s=0.3, dt=BF).cuda() for n in (C, 2 * N, C, C))
+    bias, a_log, D = _r(g, C, s=0.3).cuda(), _r(g, C, N, s=0.3).cuda(), _r(g, C).cuda()
+
+    def run(s0, s1):
+        a, b = int(cu[s0]), int(cu[s1])
+        seg, at = ((cu[s0:s1 + 1] - cu[s0]).contiguous(), ctx[s0:s1], slot[s0:s1]), (0, H * dk, 2 * H * dk)
+        st = [torch.zeros(S, H, *n, device="cuda") for n in ((dk, dv), (dv, dk), (dv, dk))] + [torch.zeros(S, C, N, device="cuda")]
+        out = [hops.linear_attention(qkv[a:b], dec, st[0], *seg, H, dk, dv, mode=3),
+               hops.decay_scan(qkv[a:b], *at, z[a:b, :H].contiguous(), zb[:H].contiguous(), st[1], *seg, H, H, dk, dv, dk ** -0.5, a_log=al, beta=beta[a:b],
+                               unit=True, mode=3),
+               hops.decay_scan(qkv[a:b], *at, z[a:b], zb, st[2], *seg, H, H, dk, dv, 1.0, decay="exp_exp", bonus=u, mode=3),
+               hops.selective_scan(x[a:b], q[a:b], 0, N, dt[a:b], bias, a_log, D, gate[a:b], 0, st[3], *seg, mode=1)]
+        return out, [t[s0:s1] for t in st]
+
+    whole, states = run(0, S)
+    for s, n in enumerate(lens):
+        if n and (s < 8 or s > S - 3):
+            a = int(cu[s])
+            out, st = run(s, s + 1)
+            for got, want in zip(out + st, [w[a:a + n] for w in whole] + [w[s:s + 1] for w in states]):
+                assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M", [1, 24, 64])
 @pytest.mark.parametrize("N,K,shared", [(2056, 2048, True), (1544, 4096, True), (520, 8192, False), (264, 16384, False), (1100, 16384, True)])
 def test_few_rows_from_a_k_of_their_own(M, N, K, shared):
