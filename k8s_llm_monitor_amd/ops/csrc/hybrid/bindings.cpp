@@ -126,13 +126,12 @@ int k8sllm_hy_latent_attention(void* out, const void* q, long q_stride, const vo
                                const int* cu, const int* ctx, const int* seq_lens, const int* block_tables,
                                int bt_stride, int S, long T, int H, int dkp, int dv, int bs, float scale, int window,
                                const float* sinks, const void* gate, long g_stride, int split, hipStream_t s);
-int k8sllm_hy_latent_parts(long T, int H, int pages, int window);
-int k8sllm_hy_latent_attention_parts(float* o, void* ml, const void* q, long q_stride, const void* k_cache, const void* v_cache,
-                                     const int* cu, const int* ctx, const int* seq_lens, const int* block_tables, int bt_stride,
-                                     int S, long T, int H, int dkp, int dv, int bs, float scale, int window, const float* sinks,
-                                     int np, hipStream_t s);
-int k8sllm_hy_latent_part_values(void* v, const float* o, const void* ml, int np, const void* wv, long T, int H, int dv, int R,
-                                 const void* gate, long g_stride, hipStream_t s);
+int k8sllm_hy_latent_attention_parts(void* out, float* o, void* ml, int* n, int least, const void* q, long q_stride, const void* k_cache,
+                                     const void* v_cache, const int* cu, const int* ctx, const int* seq_lens, const int* block_tables,
+                                     int bt_stride, int S, long T, int H, int dkp, int dv, int bs, float scale, int window,
+                                     const float* sinks, const void* gate, long g_stride, int np, hipStream_t s);
+int k8sllm_hy_latent_part_values(void* v, const void* one, const float* o, const void* ml, const int* n, int most, const void* wv, long T, int H,
+                                 int dv, int R, const void* gate, long g_stride, hipStream_t s);
 int k8sllm_hy_latent_expand(void* kt, void* vt, const void* k_cache, int pitch, const int* page_list, int npages, const void* wk,
                             const void* wv, int H, int R, int dn, int dr, int dv, hipStream_t s);
 int k8sllm_hy_rotate_heads(void* x, long stride, long T, int heads, int D, const int* positions, const float* freq, int nf,
@@ -1424,10 +1423,10 @@ bool latent_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, OptT
   return true;
 }
 
-// Latent attention of few rows, their windows in parts (0: as many as pay), and the value expansion wv [H * vdim, R] behind it: v [T, H * vdim].
-// false: not these sizes, or one part; nothing was launched.
+// Latent attention of few rows, their windows in up to np parts (one where they are of fewer than ``least`` tiles), and the value expansion
+// wv [H * vdim, R] behind it: v [T, H * vdim].  false: not these sizes; nothing was launched.
 bool latent_attention_values(Tensor v, Tensor q, Tensor k_cache, Tensor v_cache, OptT cu, OptT ctx, OptT seq_lens, Tensor block_tables,
-                             int64_t H, double scale, int64_t window, OptT sinks, OptT gate, int64_t g_col, Tensor wv, int64_t np) {
+                             int64_t H, double scale, int64_t window, OptT sinks, OptT gate, int64_t g_col, Tensor wv, int64_t np, int64_t least) {
   if (act(q, "q") != 0) return false;
   same(v, 0, "v");
   same(wv, 0, "w_uv");
@@ -1435,22 +1434,25 @@ bool latent_attention_values(Tensor v, Tensor q, Tensor k_cache, Tensor v_cache,
   TORCH_CHECK(wv.dim() == 2 && wv.is_contiguous() && wv.size(0) % H == 0 && wv.size(1) == a.dv, "w_uv [H * vdim, R]");
   const int64_t vdim = wv.size(0) / H;
   TORCH_CHECK(v.is_contiguous() && v.numel() == a.T * H * vdim, "v [T, H * vdim]");
-  TORCH_CHECK(np >= 0 && np <= 64, "parts");
+  TORCH_CHECK(np >= 1 && np <= 64 && least >= 1 && least < 1 << 30, "parts");
   int by_head = 0;
   const Gate ga = gate_of(gate, g_col, a.T, H, 0, &by_head);
-  if (np == 0) np = k8sllm_hy_latent_parts(a.T, (int)H, (int)block_tables.size(1), (int)window);
-  if (np < 2 || a.T == 0 || a.dv > 256 || a.dv % 16 || a.dkp > 320 || a.dkp % 32 || q.stride(0) % 8 || k_cache.size(1) != 16 ||
+  if (a.T == 0 || a.dv > 256 || a.dv % 16 || a.dkp > 320 || a.dkp % 32 || q.stride(0) % 8 || k_cache.size(1) != 16 ||
       reinterpret_cast<uintptr_t>(wv.data_ptr()) % 16)
     return false;
-  const auto f32 = torch::TensorOptions().device(q.device()).dtype(torch::kFloat32);
-  const Tensor o = torch::empty({np, a.T, H, a.dv}, f32), ml = torch::empty({np, a.T, H, 2}, f32);
-  check(k8sllm_hy_latent_attention_parts(o.data_ptr<float>(), ml.data_ptr(), q.data_ptr(), q.stride(0), k_cache.data_ptr(),
-                                         v_cache.data_ptr(), a.cu, a.ctx, a.seq_lens, block_tables.data_ptr<int>(),
-                                         (int)block_tables.stride(0), (int)a.S, a.T, (int)H, (int)a.dkp, (int)a.dv,
-                                         (int)k_cache.size(1), (float)scale, (int)window, sink_ptr(sinks, H), (int)np, cur()),
+  // one buffer: the parts' outputs, rows of one part, the parts' maxima and denominators, how many each row has
+  const int64_t rows = a.T * H, fo = np * rows * a.dv, fm = 2 * np * rows, fb = rows * a.dv / 2;
+  const Tensor ws = torch::empty({fo + fm + fb + a.T}, torch::TensorOptions().device(q.device()).dtype(torch::kFloat32));
+  float* o = ws.data_ptr<float>();
+  void* one = o + fo;
+  float* ml = o + fo + fb;
+  int* n = reinterpret_cast<int*>(ml + fm);
+  check(k8sllm_hy_latent_attention_parts(one, o, ml, n, (int)least, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), a.cu,
+                                         a.ctx, a.seq_lens, block_tables.data_ptr<int>(), (int)block_tables.stride(0), (int)a.S, a.T, (int)H,
+                                         (int)a.dkp, (int)a.dv, (int)k_cache.size(1), (float)scale, (int)window, sink_ptr(sinks, H), ga.p,
+                                         ga.stride, (int)np, cur()),
         "latent_attention_parts");
-  check(k8sllm_hy_latent_part_values(v.data_ptr(), o.data_ptr<float>(), ml.data_ptr(), (int)np, wv.data_ptr(), a.T, (int)H, (int)vdim,
-                                     (int)a.dv, ga.p, ga.stride, cur()),
+  check(k8sllm_hy_latent_part_values(v.data_ptr(), one, o, ml, n, (int)np, wv.data_ptr(), a.T, (int)H, (int)vdim, (int)a.dv, ga.p, ga.stride, cur()),
         "latent_part_values");
   return true;
 }

@@ -146,8 +146,9 @@ struct PageIds {
   }
 };
 
-// PART: few rows leave the chip idle, so gridDim.z workgroups take a row's window, tiles in turn as the waves do, one part of neighbouring tiles
-// each; part z leaves its maximum, denominator and unnormed output (fp32) in ``parts`` and latent_part_values merges them.
+// PART: few rows leave the chip idle, so up to gridDim.z workgroups take a row's window, tiles in turn as the waves do, one part of neighbouring tiles
+// each; part z leaves its maximum, denominator and unnormed output (fp32) in ``parts`` and latent_part_values merges them.  How many parts a row has
+// follows from its own tiles and gridDim.z, not from how wide the table is; one is what a launch without parts makes of it.
 template <int KS_MAX, int DT_MAX, int NW, int QT, bool PART = false>
 __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache,
@@ -199,14 +200,20 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
   // token t of the group sits at position p0 + t and sees keys lo_t .. p0 + t
   const int lo = window > 0 ? max(0, p0 - window + 1) : 0, hi = p0 + nt;
   int tile0 = lo >> 4, tile1 = (hi + 15) >> 4;  // its 16-key tiles
-  if (PART && p0 >= 0) {
-    const int n = tile1 - tile0, per = (n + min((int)gridDim.z, (n + NW - 1) / NW) - 1) / min((int)gridDim.z, (n + NW - 1) / NW);
+  bool part = false;
+  if (PART) {
+    const int n = p0 < 0 ? 0 : tile1 - tile0;
+    int per = max(n, 1), np = 1;
+    if (n >= parts.least) {  // (least >= 1)
+      np = min((int)gridDim.z, (n + NW - 1) / NW);
+      per = (n + np - 1) / np;
+      np = (n + per - 1) / per;
+    }
+    if ((int)blockIdx.z >= np) return;
+    if (blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) parts.n[row0] = np;
+    part = np > 1;
     tile0 += blockIdx.z * per;
     tile1 = min(tile1, tile0 + per);
-  }
-  if (PART && (p0 < 0 || tile0 >= tile1)) {  // nothing left for this part
-    if ((int)threadIdx.x < nh) parts.ml[part0 + threadIdx.x] = make_float2(-INFINITY, 0.f);
-    return;
   }
   if (p0 < 0) {  // padding row of a decode bucket
     for (int c = threadIdx.x; c < nh * dv; c += 64 * NW) obase[c] = 0;
@@ -364,7 +371,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(
       L = fmaf(l_s[w][hh], f, L);
       o = fmaf(o_s[w][hh * OP + dd], f, o);
     }
-    if (PART) {
+    if (PART && part) {
       parts.o[part0 * dv + c] = o;
       if (dd == 0) parts.ml[part0 + hh] = make_float2(M, L);
       continue;
@@ -664,31 +671,18 @@ int k8sllm_hy_latent_attention(void* out, const void* q, long q_stride, const vo
   return (int)hipGetLastError();
 }
 
-// How many parts a row's window is cut into, for T rows over tables of ``pages`` pages; 1: none.  A workgroup of eight waves takes 4 us for each
-// eight tiles (its loads of 16 key rows ask for 16 lines at a time), one a CU, so few rows are cut until half of the chip is busy, a tile a
-// wave at least; behind that parts cost more in the merge than they save (1.2 us for each four, and their outputs' way through memory).  us with
-// the values behind it, whole / this many parts, 8 heads, 128 + 32 wide: 1 row of 333 keys 10.0 / 9.4, of 1500 21.0 / 11.7, of 4800
-// 50 / 14.6; 16 rows of 1500 22.0 / 14.4, 64 of 1500 25.4 / 18.5, of 4800 61 / 35; 16 heads, 256 + 32: 1 of 1500 35.8 / 15.2, 2 of 4800 95 / 20, 32 of
-// 1500 39.3 / 22.3, 64 of 1500 39.9 / 30.6; 128 of 1500 43.8 / 47.7 in two.  Short windows of many rows lose: 64 rows of 333 keys 18.0 / 20.4.
-int k8sllm_hy_latent_parts(long T, int H, int pages, int window) {
-  const long wgs = T * ((H + 15) / 16);
-  const int tiles = window > 0 ? min(pages, window / 16 + 2) : pages;
-  if (wgs <= 0 || wgs > 64 || tiles < (wgs < 16 ? 16 : 40)) return 1;
-  return (int)min(min(max(128 / wgs, 3l), 16l), (long)((tiles + 7) / 8));
-}
-
-// The same attention, its rows' windows in np parts (latent_part_values then merges them); sizes as above, 1: not these.
-int k8sllm_hy_latent_attention_parts(float* o, void* ml, const void* q, long q_stride, const void* k_cache, const void* v_cache,
-                                     const int* cu, const int* ctx, const int* seq_lens, const int* block_tables, int bt_stride,
-                                     int S, long T, int H, int dkp, int dv, int bs, float scale, int window, const float* sinks,
-                                     int np, hipStream_t s) {
+// The same attention, its rows' windows in up to np parts (LatentParts; latent_part_values then merges them); sizes as above, 1: not these.
+int k8sllm_hy_latent_attention_parts(void* out, float* o, void* ml, int* n, int least, const void* q, long q_stride, const void* k_cache,
+                                     const void* v_cache, const int* cu, const int* ctx, const int* seq_lens, const int* block_tables,
+                                     int bt_stride, int S, long T, int H, int dkp, int dv, int bs, float scale, int window,
+                                     const float* sinks, const void* gate, long g_stride, int np, hipStream_t s) {
   if (T <= 0) return 0;
   if (bs != 16 || dkp % 32 || dv % 16 || dkp > 320 || dv > 256 || q_stride % 8 || np < 1 || np > 65535) return 1;
   const dim3 grid((unsigned)T, (unsigned)((H + 15) / 16), (unsigned)np);
 #define K8SLLM_LP(KS, DT)                                                                                                       \
-  hipLaunchKernelGGL((latent_attn_mfma_kernel<KS, DT, 8, 1, true>), grid, dim3(512), 0, s, (bf16_t*)nullptr, (const bf16_t*)q,    \
+  hipLaunchKernelGGL((latent_attn_mfma_kernel<KS, DT, 8, 1, true>), grid, dim3(512), 0, s, (bf16_t*)out, (const bf16_t*)q,        \
                      q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu, ctx, seq_lens, block_tables, bt_stride, S, H, \
-                     dkp, dv, scale, window, sinks, (const bf16_t*)nullptr, 0L, LatentParts{o, (float2*)ml})
+                     dkp, dv, scale, window, sinks, (const bf16_t*)gate, g_stride, LatentParts{o, (float2*)ml, n, least})
   if (dkp <= 128 && dv <= 128) K8SLLM_LP(4, 8);
   else K8SLLM_LP(10, 16);
 #undef K8SLLM_LP

@@ -104,82 +104,107 @@ __global__ __launch_bounds__(64) void latent_head_values_kernel(bf16_t* __restri
     if (n0 + 4 * quad + i < dv) stf(out + i, acc[i]);
 }
 
-// The same of rows whose attention lies in np parts: their merge, times the sigmoid of the row and head's gate, rounded, is the products' operand.
+// The same of rows whose attention lies in parts (LatentParts): their merge, times the sigmoid of the row and head's gate, rounded, is the products' operand.
 // Each of a head's dv / 16 workgroups merges its rows again, which costs less than a launch of its own (1.6 us and a round of loads).
-// Four waves take the parts in turn, then a quarter of R each: nothing waits for a part's maximum before its output is on its way.
-__global__ __launch_bounds__(256) void latent_part_values_kernel(bf16_t* __restrict__ v, LatentParts parts, int np,
+// Four waves take the parts in turn and put a quarter of R each into LDS, and the last one, which has the fewest parts, multiplies: in the order of
+// latent_head_values_kernel, and rows of one part with what is already finished for them, so that a row has the same bits whatever stands beside it.
+// Sixteen rows of one part each need nothing else.  All that may be needed is on its way before it is known what is (a round of loads less: 64 rows of
+// 1500 keys, 16 heads, 32.7 / 31.9 us).
+__global__ __launch_bounds__(256) void latent_part_values_kernel(bf16_t* __restrict__ v, const bf16_t* __restrict__ one, LatentParts parts, int most,
                                                                  const bf16_t* __restrict__ wv, int T, int H, int dv, int R,
                                                                  const bf16_t* __restrict__ gate, long g_stride) {
   constexpr int KC = 8, NW = 4, KW = KC / NW;  // pieces of 32 k: R <= 256
   __shared__ __attribute__((aligned(16))) float4 o_s[NW][2 * KC][64];
   __shared__ float2 ml_s[NW][64];
-  __shared__ hf32x4 red[NW][64];
+  __shared__ uint4 x_s[KC][64];
   const int h = blockIdx.y, t0 = 16 * blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
-  const int n0 = 16 * blockIdx.x;
-  const bf16_t* wr = wv + ((long)h * dv + min(n0 + col, dv - 1)) * R;
-  const long th = (long)min(t0 + col, T - 1) * H + h, step = (long)T * H;
-  uint4 a[KW];
+  const int n0 = 16 * blockIdx.x, t = min(t0 + col, T - 1);
+  const long th = (long)t * H + h, step = (long)T * H;
+  const int np = parts.n[t];
+  uint4 a[KC], b[KC];
+  auto load = [&](uint4 (&x)[KC], const bf16_t* row) {
 #pragma unroll
-  for (int c = 0; c < KW; ++c) {
-    const int k = 32 * (KW * wave + c) + 8 * quad;
-    a[c] = k < R ? *reinterpret_cast<const uint4*>(wr + k) : make_uint4(0, 0, 0, 0);
+    for (int c = 0; c < KC; ++c) {
+      const int k = 32 * c + 8 * quad;
+      x[c] = *reinterpret_cast<const uint4*>(row + (k < R ? k : 0));
+      if (k >= R) x[c] = make_uint4(0, 0, 0, 0);
+    }
+  };
+  const bool last = wave == NW - 1;
+  if (last) {
+    load(a, wv + ((long)h * dv + min(n0 + col, dv - 1)) * R);
+    load(b, one + th * R);
   }
-  float M = -INFINITY, L = 0.f, o[KC][8] = {};
-  for (int z = wave; z < np; z += NW) {
-    const float2 ml = parts.ml[z * step + th];
-    const float* p = parts.o + (z * step + th) * R + 8 * quad;
-    float x[KC][8];
+  float2 ml;
+  float x[KC][8];
+  auto part = [&](int z) {  // (what is not there is in the buffer, and read by nobody)
+    const long at = z < most ? z * step + th : 0;
+    const float* p = parts.o + at * R + 8 * quad;
+    ml = parts.ml[at];
 #pragma unroll
     for (int c = 0; c < KC; ++c) load8(p + (32 * c + 8 * quad < R ? 32 * c : -8 * quad), x[c]);
-    const bool empty = ml.x == -INFINITY;  // its output is not written
-    const float m = fmaxf(M, ml.x), f0 = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - m), f1 = empty ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
-    M = m;
-    L = fmaf(ml.y, f1, L * f0);
+  };
+  part(wave);
+  if (__ballot(np > 1) != 0) {  // the same rows in every wave
+    float M = -INFINITY, L = 0.f, o[KC][8] = {};
+    for (int z = wave; __ballot(np > 1 && z < np) != 0; z += NW) {
+      if (z > wave) part(z);
+      if (np <= 1 || z >= np) continue;
+      const float m = fmaxf(M, ml.x), f0 = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - m), f1 = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
+      M = m;
+      L = fmaf(ml.y, f1, L * f0);
 #pragma unroll
-    for (int c = 0; c < KC; ++c)
+      for (int c = 0; c < KC; ++c)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[c][j] = fmaf(empty ? 0.f : x[c][j], f1, o[c][j] * f0);
-  }
-#pragma unroll
-  for (int c = 0; c < KC; ++c) {
-    o_s[wave][2 * c][lane] = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
-    o_s[wave][2 * c + 1][lane] = make_float4(o[c][4], o[c][5], o[c][6], o[c][7]);
-  }
-  ml_s[wave][lane] = make_float2(M, L);
-  __syncthreads();
-  float f[NW];
-  M = -INFINITY;
-  L = 0.f;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_s[w][lane].x);
-#pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    const float2 ml = ml_s[w][lane];
-    f[w] = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - M);
-    L = fmaf(ml.y, f[w], L);
-  }
-  float inv = L > 0.f ? 1.f / L : 0.f;
-  if (gate != nullptr) inv *= sigmoid_f(bf2f(gate[(long)min(t0 + col, T - 1) * g_stride + h]));
-  hf32x4 acc{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int c = 0; c < KW; ++c) {
-    float x[8] = {};
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float4 u = o_s[w][2 * (KW * wave + c)][lane], s = o_s[w][2 * (KW * wave + c) + 1][lane];
-      const float y[8] = {u.x, u.y, u.z, u.w, s.x, s.y, s.z, s.w};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = fmaf(y[j], f[w], x[j]);
+        for (int j = 0; j < 8; ++j) o[c][j] = fmaf(x[c][j], f1, o[c][j] * f0);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = 32 * (KW * wave + c) + 8 * quad < R ? x[j] * inv : 0.f;
-    acc = tile_product(a[c], pack8(x), acc);
-  }
-  red[wave][lane] = acc;
-  __syncthreads();
-  if (wave || t0 + col >= T) return;
+    for (int c = 0; c < KC; ++c) {
+      o_s[wave][2 * c][lane] = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
+      o_s[wave][2 * c + 1][lane] = make_float4(o[c][4], o[c][5], o[c][6], o[c][7]);
+    }
+    ml_s[wave][lane] = make_float2(M, L);
+    __syncthreads();
+    float f[NW];
+    M = -INFINITY;
+    L = 0.f;
 #pragma unroll
-  for (int w = 1; w < NW; ++w) acc += red[w][lane];
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_s[w][lane].x);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float2 q = ml_s[w][lane];
+      f[w] = q.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(q.x - M);
+      L = fmaf(q.y, f[w], L);
+    }
+    float inv = L > 0.f ? 1.f / L : 0.f;
+    if (gate != nullptr) inv *= sigmoid_f(bf2f(gate[(long)t * g_stride + h]));
+#pragma unroll
+    for (int c = 0; c < KW; ++c) {
+      float y[8] = {};
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float4 u = o_s[w][2 * (KW * wave + c)][lane], s = o_s[w][2 * (KW * wave + c) + 1][lane];
+        const float q[8] = {u.x, u.y, u.z, u.w, s.x, s.y, s.z, s.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[j] = fmaf(q[j], f[w], y[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] *= inv;
+      x_s[KW * wave + c][lane] = pack8(y);
+    }
+    __syncthreads();
+    if (last && np > 1) {
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+        if (32 * c + 8 * quad < R) b[c] = x_s[c][lane];
+    }
+  }
+  if (!last) return;
+  hf32x4 acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < KC; ++c)
+    if (32 * c < R) acc = tile_product(a[c], b[c], acc);
+  if (t0 + col >= T) return;
   bf16_t* out = v + ((long)(t0 + col) * H + h) * dv + n0 + 4 * quad;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -213,13 +238,14 @@ int k8sllm_hy_latent_head_values(void* v, const void* o, const void* wv, long T,
   return (int)hipGetLastError();
 }
 
-int k8sllm_hy_latent_part_values(void* v, const float* o, const void* ml, int np, const void* wv, long T, int H, int dv, int R,
-                                 const void* gate, long g_stride, hipStream_t s) {
+// most: how many parts the buffers hold
+int k8sllm_hy_latent_part_values(void* v, const void* one, const float* o, const void* ml, const int* n, int most, const void* wv, long T, int H,
+                                 int dv, int R, const void* gate, long g_stride, hipStream_t s) {
   if (T <= 0 || H <= 0 || dv <= 0) return 0;
-  if (R < 16 || R % 16 || R > 256 || T > (1 << 19) || H > 65535 || np < 1 || (reinterpret_cast<uintptr_t>(wv) & 15)) return -1;
+  if (R < 16 || R % 16 || R > 256 || T > (1 << 19) || H > 65535 || most < 1 || (reinterpret_cast<uintptr_t>(wv) & 15)) return -1;
   hipLaunchKernelGGL(latent_part_values_kernel, dim3((unsigned)((dv + 15) / 16), (unsigned)H, (unsigned)((T + 15) / 16)), dim3(256), 0, s,
-                     (bf16_t*)v, LatentParts{(float*)o, (float2*)ml}, np, (const bf16_t*)wv, (int)T, H, dv, R, (const bf16_t*)gate,
-                     g_stride);
+                     (bf16_t*)v, (const bf16_t*)one,
+                     LatentParts{(float*)o, (float2*)ml, (int*)n, 0}, most, (const bf16_t*)wv, (int)T, H, dv, R, (const bf16_t*)gate, g_stride);
   return (int)hipGetLastError();
 }
 }

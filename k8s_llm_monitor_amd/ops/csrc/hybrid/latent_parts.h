@@ -4,11 +4,13 @@
 
 namespace k8sllm {
 
-// part z, row t, head h at (z * rows + t) * heads + h: the unnormed output [R] and (largest base-2 logit, denominator); (-inf, 0): an
-// empty part, whose output is not written
+// n[t]: the parts of row t; of more than one, part z's unnormed output [R] and (largest base-2 logit, denominator) of head h are at
+// (z * rows + t) * heads + h; what one part has is finished in ``out`` [rows][heads][R].  Rows of fewer than ``least`` tiles are one part.
 struct LatentParts {
   float* o;
   float2* ml;
+  int* n;
+  int least;
 };
 
 }  // namespace k8sllm

@@ -926,17 +926,37 @@ def latent_attention(qa: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     return window_attention_decode(qa, k_cache, v_cache, block_tables, seq_lens, *args, vec=bool(fast), **kw)
 
 
+def latent_parts(T: int, H: int, R: int, pages: int, window: int) -> tuple:
+    """(parts, tiles from which on a row has them) of latent attention's T rows over tables of ``pages`` pages; one part: as a whole.  A workgroup of
+    eight waves takes 4 us for each eight tiles (its loads of 16 key rows ask for 16 lines at a time), one a CU, so few rows are cut until half of the chip
+    is busy, a tile a wave at least; behind that parts cost more in the merge than they save (1.2 us for each four, and their outputs' way through memory).
+    Tables are as wide as the longest sequence may become, so a row of few tiles is one part by itself.  us with the values behind it, whole / so, tables of
+    512 pages: 8 heads, 128 + 32 wide, 1 row of 20 keys 7.7 / 8.4, 333 10.7 / 10.3, 1500 21.3 / 12.5, 4800 51 / 14.7; 16 rows of 100 8.8 / 9.4, 700 14.1 / 13.6,
+    1500 22.0 / 15.3; 64 of 333 11.3 / 11.9, 1500 26.1 / 20.0, 4800 62 / 36; 16 heads, 256 + 32, 1 of 20 11.8 / 11.7, 1500 36 / 16.0; 32 of 1500 39.9 / 24.2, 64 of
+    333 18.3 / 19.2, 1500 40.4 / 31.8.  (With every row of such a table in 3 to 16 parts, 1 row of 20 keys took 10.6, 64 of 333 12.3 and 21.3.)"""
+    wgs = T * -(-H // 16)
+    if wgs == 0 or wgs > 64:
+        return 1, 1
+    least = 16 if wgs < 16 or (wgs <= 32 and R > 128) else 40  # 333 keys, 16 heads, 256 + 32: 16 rows 17.7 / 15.9, 64 18.5 / 21.3
+    tiles = min(pages, window // 16 + 2) if window > 0 else pages
+    return (min(max(128 // wgs, 3), 16, -(-tiles // 8)) if tiles >= least else 1), least
+
+
 def latent_attention_values(qa: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor, H: int,
                             scale: float, window: int, sinks: Optional[torch.Tensor], w_uv: torch.Tensor, out: torch.Tensor,
                             cu: Optional[torch.Tensor] = None, ctx: Optional[torch.Tensor] = None,
                             seq_lens: Optional[torch.Tensor] = None, fast: int = 1, sink: bool = True,
-                            gate: Optional[torch.Tensor] = None, g_col: int = 0, parts: int = 0) -> bool:
-    """``latent_attention`` and ``latent_head_values`` into ``out`` of rows too few to fill the chip, each row's window cut into ``parts``
-    (0: as many as pay) whose merge is the value expansion's prologue.  False: nothing was done, these are not such rows."""
+                            gate: Optional[torch.Tensor] = None, g_col: int = 0, parts: int = 0, least: int = 1) -> bool:
+    """``latent_attention`` and ``latent_head_values`` into ``out`` of rows too few to fill the chip, the window of a row of ``least`` tiles or more cut
+    into up to ``parts`` (0: as many as pay) whose merge is the value expansion's prologue.  False: nothing was done, these are not such rows."""
+    if parts == 0:
+        parts, least = latent_parts(qa.shape[0], H, w_uv.shape[1], block_tables.shape[1], window)
+        if parts == 1:
+            return False
     if not (fast and _head_rows(HEAD_VALUE_ROWS, qa, w_uv) and out.is_contiguous()):
         return False
     return native().latent_attention_values(out, qa, k_cache, v_cache, cu, ctx, seq_lens, block_tables, int(H), float(scale), int(window),
-                                            sinks if sink else _no_sink(H, qa.device), gate, int(g_col), w_uv, int(parts))
+                                            sinks if sink else _no_sink(H, qa.device), gate, int(g_col), w_uv, int(parts), int(least))
 
 
 # ---------------------------------------------------------------- Mamba-2

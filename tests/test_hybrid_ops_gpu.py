@@ -452,7 +452,8 @@ def test_gelu_experts_on_the_tile_gemm():
 @pytest.mark.parametrize("window,parts", [(0, 0), (0, 2), (0, 7), (0, 64), (200, 3), (24, 2)])
 def test_latent_attention_in_parts(Hq, pitch, R, dv, window, parts):
     """Few rows whose windows are cut into parts (more and fewer than there are tiles, a padding row, partial head groups, a chunk's rows, a
-    gate), merged in the value expansion, against fp32.  Weights, values and result are rounded once each to bf16 (2^-8)."""
+    gate), merged in the value expansion, against fp32.  Weights, the merged output and the result are rounded once each to bf16, which moves a number
+    by up to 2^-8 of it (half of the last of eight bits)."""
     dt, g = torch.bfloat16, _g(23)
     lens = [350, 9, 1, 0, 129, 1100]  # the fourth is a padding row
     kc, vc, bt = _paged(g, dt, [max(n, 1) for n in lens], Hq, 1, pitch, R, nb=120)
@@ -475,6 +476,40 @@ def test_latent_attention_in_parts(Hq, pitch, R, dv, window, parts):
             assert bool((err <= 2.0 ** -8 * (want.abs() + most) + 1e-5).all()), (err - 2.0 ** -8 * (want.abs() + most)).max()
             if "seq_lens" in seen:
                 assert float(out[3].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("Hq,pitch,R,dv", [(8, 160, 128, 128), (16, 288, 256, 128), (20, 64, 48, 40)])
+@pytest.mark.parametrize("T", [6, 21])  # one and two groups of 16 rows; the second has another least count of tiles
+def test_latent_rows_beside_others_and_wide_tables(Hq, pitch, R, dv, T):
+    """A row's bits follow from its own keys and how many rows there are: not from the table's width nor from how many parts its neighbours have; a row of few
+    tiles has those of the launches without parts.  A padding row, rows around the least counts of tiles, windows."""
+    dt, g = torch.bfloat16, _g(41)
+    lens = ([20, 241, 0, 333, 1500, 240, 256, 625, 640, 641, 1] * 2)[:T]
+    kc, vc, bt = _paged(g, dt, [max(n, 1) for n in lens], Hq, 1, pitch, R, nb=640)
+    kc, vc, sinks, wv = kc.cuda(), vc.cuda(), _r(g, Hq, s=1.5).cuda(), _r(g, Hq * dv, R, s=R ** -0.5, dt=dt).cuda()
+    qa, gate = _r(g, T, Hq * pitch, s=0.25, dt=dt).cuda(), _r(g, T, Hq, dt=dt).cuda()
+
+    def whole(sl, tables, window):
+        o = H.latent_attention(qa, kc, vc, tables, Hq, 0.2, window, sinks, seq_lens=sl, gate=gate)
+        return H.latent_head_values(o, wv, Hq)
+
+    def run(n, width, window):
+        sl, tables = _i32(n).cuda(), torch.nn.functional.pad(bt, (0, max(width - bt.shape[1], 0)))[:, :width].contiguous().cuda()
+        out = torch.full((T, Hq * dv), 7.0, dtype=dt, device="cuda")
+        took = H.latent_attention_values(qa, kc, vc, tables, Hq, 0.2, window, sinks, wv, out, seq_lens=sl, gate=gate)
+        assert took == (H.latent_parts(T, Hq, R, width, window)[0] > 1)
+        return out if took else whole(sl, tables, window)
+
+    for window in (0, 700):
+        want, least = run(lens, 94, window), H.latent_parts(T, Hq, R, 94, window)[1]
+        assert torch.equal(run(lens, 512, window), want)
+        ref = whole(_i32(lens).cuda(), bt.cuda(), window)
+        few = [i for i, n in enumerate(lens) if -(-n // 16) - (max(0, n - window) // 16 if window else 0) < least]
+        assert few and torch.equal(want[few], ref[few]) and (len(few) == T or not torch.equal(want, ref))
+    short = [min(n, 200) for n in lens]  # all of one part, in the table that has parts and in one that has not
+    assert torch.equal(run(short, 512, 0), run(short, 13, 0)) and torch.equal(run(short, 512, 0), whole(_i32(short).cuda(), bt.cuda(), 0))
+    mixed = [n if i % 2 else min(n, 100) for i, n in enumerate(lens)]  # other neighbours
+    assert torch.equal(run(mixed, 512, 0)[1::2], run(lens, 512, 0)[1::2])
 
 
 @pytest.mark.parametrize("M,d,N,f,kind", [(1, 1024, 3584, 0, ""), (2, 1024, 1568, 0, ""), (2, 2048, 7184, 0, ""), (4, 992, 33, 0, ""), (3, 32, 16, 0, ""),

@@ -48,6 +48,16 @@ def test_tile_gemm_of_plain_products(M, N, K, takes):
     assert hops._tile_plain(M, N, K) is takes
 
 
+@pytest.mark.parametrize("T,H,R,pages,window,want", [
+    (0, 8, 128, 512, 0, (1, 1)), (1, 8, 128, 15, 0, (1, 16)), (1, 8, 128, 16, 0, (2, 16)), (1, 8, 128, 512, 0, (16, 16)), (8, 16, 256, 512, 0, (16, 16)),
+    (15, 8, 128, 512, 0, (8, 16)), (16, 8, 128, 39, 0, (1, 40)), (16, 8, 128, 40, 0, (5, 40)), (16, 16, 256, 39, 0, (5, 16)), (16, 20, 256, 512, 0, (4, 16)),
+    (17, 20, 256, 512, 0, (3, 40)), (64, 16, 256, 512, 0, (3, 40)), (65, 16, 256, 512, 0, (1, 1)), (33, 20, 256, 512, 0, (1, 1)), (1, 8, 128, 512, 200, (1, 16)),
+    (1, 8, 128, 512, 1024, (9, 16)),
+])
+def test_parts_of_latent_rows(T, H, R, pages, window, want):
+    assert hops.latent_parts(T, H, R, pages, window) == want
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(2304, 5648, 1024), (7937, 3104, 2048), (2048, 8000, 192), (2049, 5680, 512)])
 def test_plain_product_on_the_tile_gemm(M, N, K):
