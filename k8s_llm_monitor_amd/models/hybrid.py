@@ -388,14 +388,16 @@ class LatentAttention:
         args, kw = (H, self.scale, self.window, self.sinks), dict(fast=self.fast, sink=self.sink)
         left, a = [], 0  # runs of more rows than one of which a workgroup each fills the chip
         for b, tables, seen in runs:
-            gt = gate[a:b] if gate is not None else None
-            if not hops.latent_attention_values(qa[a:b], kc, vc, tables, *args, self.w_uv, out[a:b], gate=gt, **kw, **seen):
-                left.append((a, b, hops.latent_attention(qa[a:b], kc, vc, tables, *args, gate=gt, **kw, **seen)))
+            qs, gt, to = (t if t is None or t.shape[0] == b - a else t[a:b] for t in (qa, gate, out))
+            parts, least = hops.latent_parts(b - a, H, self.R, tables.shape[1], self.window)
+            if parts == 1 or not hops.latent_attention_values(qs, kc, vc, tables, *args, self.w_uv, to, gate=gt, parts=parts, least=least, **kw, **seen):
+                left.append((a, to, hops.latent_attention(qs, kc, vc, tables, *args, gate=gt, **kw, **seen)))
             a = b
         # ... and the value expansion to the result: v[h] = o_lat[h] @ W_uv[h]^T
-        if left:
-            o = left[0][2] if len(left) == 1 else torch.cat([x[2] for x in left])
-            hops.latent_head_values(o, self.w_uv, H, out[left[0][0]:left[-1][1]])
+        if len(left) == 1:
+            hops.latent_head_values(left[0][2], self.w_uv, H, left[0][1])
+        elif left:
+            hops.latent_head_values(torch.cat([x[2] for x in left]), self.w_uv, H, out[left[0][0]:a])
 
     def _expand_ok(self, h: torch.Tensor, meta: AttnMeta) -> bool:
         rows = h.shape[0] - meta.num_decode
@@ -1614,9 +1616,9 @@ class HybridLM:
         return F.linear(h, g["w"]), 0
 
     @staticmethod
-    def _gated_rows(sub, g: dict, *args):
-        """A sublayer's input rows; not made yet where its first product is all that reads them and can make them."""
-        return (hops.gated_rows if g["w"] is None and getattr(sub, "first_product", False) else hops.gated_add_norm)(*args)
+    def _gated_rows(sub, g: dict, few: bool, *args):
+        """A sublayer's input rows; not made yet where they are few and its first product is all that reads them and can make them."""
+        return (hops.gated_rows if few and g["w"] is None and getattr(sub, "first_product", False) else hops.gated_add_norm)(*args)
 
     def _forward_gated(self, x: Optional[torch.Tensor], meta: AttnMeta, caches: list, ids: torch.Tensor) -> torch.Tensor:
         """Sequential blocks with a gated residual: every sublayer's result y joins the stream as
@@ -1625,6 +1627,7 @@ class HybridLM:
         eps, op, mult = c.norm_eps, self.one_plus, c.residual_mult
         pend = None  # (y, projection holding the gate logits, their first column, bias)
         want = self._wanted(meta, ids.numel())
+        few = ids.numel() <= hops.GATED_ROWS  # (known here, not once a sublayer: the host's time bounds a short prompt's step)
         for r, (li, t, first) in enumerate(self.runs):
             if first and self.loop_step is not None:
                 if pend is not None:
@@ -1637,7 +1640,7 @@ class HybridLM:
             elif pend is None:
                 h = hops.add_norm(x, (), None, w1, eps, op, self.dtype)
             else:
-                h = self._gated_rows(mx if rows is None else None, self.rg1[li], x, *pend, mult, w1, eps, op, self.dtype)
+                h = self._gated_rows(mx, self.rg1[li], few and rows is None, x, *pend, mult, w1, eps, op, self.dtype)
             y = mx.forward(h, meta, caches[self.kv_run[r]], rows=rows)
             if isinstance(h, hops.GatedRows):
                 x = h.residual
@@ -1647,7 +1650,7 @@ class HybridLM:
             pend = (y, *self._gate_of(mx, self.rg1[li], h), self.rg1[li]["b"])
             ff = self.ffns[li]
             if ff is not None:
-                h2 = self._gated_rows(ff, self.rg2[li], x, *pend, mult, self.norms2[li], eps, op, self.dtype)
+                h2 = self._gated_rows(ff, self.rg2[li], few, x, *pend, mult, self.norms2[li], eps, op, self.dtype)
                 y = ff.forward(h2)
                 if isinstance(h2, hops.GatedRows):
                     x = h2.residual

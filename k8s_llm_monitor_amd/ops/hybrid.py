@@ -327,7 +327,7 @@ class GatedRows:
     def take(residual: torch.Tensor, y: torch.Tensor, proj: torch.Tensor, g_col: int, *rest) -> bool:
         """Whether the prologue is this sum's and norm's: bf16 on the device, everything in 16-byte pieces, no gradients."""
         M, d = residual.shape
-        return (residual.is_cuda and 0 < M <= (4 if d <= 1024 else 2) and d <= 2048 and d % 32 == 0 and y.dtype == proj.dtype == torch.bfloat16
+        return (residual.is_cuda and 0 < M <= (GATED_ROWS if d <= 1024 else 2) and d <= 2048 and d % 32 == 0 and y.dtype == proj.dtype == torch.bfloat16
                 and residual.dtype == torch.float32 and residual.is_contiguous() and y.is_contiguous() and y.shape == residual.shape
                 and proj.dim() == 2 and proj.stride(1) == 1 and proj.stride(0) % 8 == 0 and g_col % 8 == 0
                 and all(t.data_ptr() % 16 == 0 for t in (residual, y, proj, rest[0], rest[2]))
@@ -366,7 +366,7 @@ class GatedRows:
         return a, z
 
 
-GATED_COLUMNS = 16384
+GATED_ROWS, GATED_COLUMNS = 4, 16384  # the most that its prologue takes
 
 
 def gated_rows(residual: torch.Tensor, y: torch.Tensor, proj: torch.Tensor, g_col: int, bias: torch.Tensor, mult: float, w: torch.Tensor,
@@ -1458,16 +1458,18 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         if made is not None:
             return made[1]
         x = x.tensor()
-    form = _few_rows(x, w)
-    if form is not None:
-        y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
-        native().few_rows(y, None, x, w, -1, 0.0, form == "shared")
-        return y
-    if x.shape[0] >= 1024 and _tile_operands(x, w) and _tile_plain(x.shape[0], w.shape[0], w.shape[1]) and not (
+    M = x.shape[0]
+    if M <= 64:  # (rows between the two rules are a prompt's whose step the host's time bounds: they meet no other check)
+        form = _few_rows(x, w)
+        if form is not None:
+            y = torch.empty(M, w.shape[0], dtype=x.dtype, device=x.device)
+            native().few_rows(y, None, x, w, -1, 0.0, form == "shared")
+            return y
+    elif M >= 1024 and _tile_operands(x, w) and _tile_plain(M, w.shape[0], w.shape[1]) and not (
             torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
         from .. import ops
 
-        y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        y = torch.empty(M, w.shape[0], dtype=x.dtype, device=x.device)
         ops.native().gemm_tile(y, x, w, None, 0, 1)
         return y
     return F.linear(x, w)
@@ -1496,8 +1498,8 @@ def _tile_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def _tile_unit(x: torch.Tensor, w: torch.Tensor, f: int) -> bool:
-    """Whether ``gemm_tile_unit`` takes these operands, by the rule of ``_tile_form``."""
-    return _tile_operands(x, w) and _tile_form(x.shape[0], w.shape[0], w.shape[1], f)
+    """Whether ``gemm_tile_unit`` takes these operands, by the rule of ``_tile_form`` (which takes no fewer rows than 0.8 of a tile's)."""
+    return x.shape[0] > 204 and _tile_operands(x, w) and _tile_form(x.shape[0], w.shape[0], w.shape[1], f)
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, kind: str) -> torch.Tensor:

@@ -138,6 +138,19 @@ def test_latent_expanded_form_equals_the_oracle(monkeypatch):
     close(a["c"], want["c"])
 
 
+def test_forms_of_few_rows_are_asked_for_few_rows_only(monkeypatch):
+    """The host's time bounds a short prompt's step: forms that take up to 4 and up to 64 rows are not gone into for more."""
+    rig, calls = rig_for(FULL, 5), []
+    for name in ("gated_rows", "latent_attention_values"):
+        monkeypatch.setattr(hops, name, lambda *a, _f=getattr(hops, name), _n=name, **k: calls.append(_n) or _f(*a, **k))
+    t = toks(72, FULL["vocab"], 6)
+    rig.step([("a", t[:65])])
+    rig.step([("a", t[65:70])])  # (the tables of prompt rows end where they do)
+    assert calls == []
+    rig.step([("a", t[70:71])])
+    assert set(calls) == {"latent_attention_values", "gated_rows"}
+
+
 def test_layer_outputs_match_oracle():
     rig = rig_for(FULL, 5)
     t = toks(19, FULL["vocab"], 3)
