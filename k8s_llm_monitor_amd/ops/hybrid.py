@@ -1465,7 +1465,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             y = torch.empty(M, w.shape[0], dtype=x.dtype, device=x.device)
             native().few_rows(y, None, x, w, -1, 0.0, form == "shared")
             return y
-    elif M >= 1024 and _tile_operands(x, w) and _tile_plain(M, w.shape[0], w.shape[1]) and not (
+    elif M >= 1024 and w.dim() == 2 and _tile_plain(M, w.shape[0], w.shape[1]) and _tile_operands(x, w) and not (
             torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
         from .. import ops
 
@@ -1492,9 +1492,15 @@ def _tile_form(M: int, N: int, K: int, f: int) -> bool:
             and 256 * N * 2 < 1 << 31)
 
 
+def _transformed(*ts: torch.Tensor) -> bool:
+    """Whether something beside the values hangs on a product that only torch's own carries on: a tangent, a function transform (vmap, jvp), a trace."""
+    return (torch._C._are_functorch_transforms_active() or torch.jit.is_tracing()
+            or any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in ts))
+
+
 def _tile_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.is_contiguous()
-            and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and w.is_contiguous() and not _transformed(x, w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
 def _tile_unit(x: torch.Tensor, w: torch.Tensor, f: int) -> bool:

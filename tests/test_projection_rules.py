@@ -75,3 +75,36 @@ def test_plain_product_on_the_tile_gemm(M, N, K):
     assert xg.grad is not None
     wide = torch.cat([x, x], 1)[:, :K]  # rows of another stride
     assert torch.equal(hops.linear(wide, w), torch.nn.functional.linear(wide, w))
+
+
+def test_transforms_and_tangents_are_seen():
+    import torch
+    import torch.autograd.forward_ad as fw
+
+    x, w, seen = torch.randn(3, 4), torch.randn(2, 4), []
+    f = lambda v: seen.append(hops._transformed(v, w)) or v * 2.0  # noqa: E731
+    f(x)
+    torch.func.vmap(f)(x)
+    torch.func.jvp(f, (x,), (x,))
+    with fw.dual_level():
+        f(fw.make_dual(x, x))
+        f(x)
+    torch.jit.trace(f, (x,), check_trace=False)
+    assert seen == [False, True, True, True, False, True]
+
+
+@pytest.mark.gpu
+def test_large_products_keep_tangents():
+    """A product that the tile GEMM takes otherwise: torch's own where a tangent goes through it."""
+    import torch
+    import torch.autograd.forward_ad as fw
+
+    M, N, K = 2304, 5648, 1024
+    assert hops._tile_plain(M, N, K)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x, w, t = (torch.randn(r, K, generator=g, device="cuda").to(torch.bfloat16) for r in (M, N, M))
+    with fw.dual_level():
+        y = fw.unpack_dual(hops.linear(fw.make_dual(x, t), w))
+    assert torch.equal(y.primal, torch.nn.functional.linear(x, w)) and torch.equal(y.tangent, torch.nn.functional.linear(t, w))
+    y, dy = torch.func.jvp(lambda v: hops.linear(v, w), (x,), (t,))
+    assert torch.equal(dy, torch.nn.functional.linear(t, w))
