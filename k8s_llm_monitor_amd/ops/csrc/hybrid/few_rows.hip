@@ -255,8 +255,9 @@ int k8sllm_hy_few_rows(void* y, void* yg, const void* x, long x_stride, const vo
   // (shared, 16 rows, 10240 x 384, us, non-temporal / as usual: 15 such weights in turn, which the memory-side cache holds, 5.3 / 4.5; 100 of them, from
   // memory, 5.0 / 5.3; 12288 x 320 4.8 / 4.3, 4.5 / 4.75)
   const bool once = read_once(2l * N * Kd, w, Kd);
-  // workgroups begin at k of their own (first_piece) where a wave's rows, or its quarters of them, are whole periods of the channels
-  const bool turn = once && Kd % (shared ? kTurnBytes / 2 : 2 * kTurnBytes) == 0;
+  // workgroups begin at k of their own (first_piece) where a wave's rows, or its quarters of them, are whole periods of the channels, and there are
+  // enough of them to meet in one
+  const bool turn = once && (shared ? (tiles + 3) / 4 : tiles) >= kTurnGroups && Kd % (shared ? kTurnBytes / 2 : 2 * kTurnBytes) == 0;
 #define K8SLLM_FRX(KERNEL, GRID) \
   hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(256), 0, s, o, (const bf16_t*)x, x_stride, (const bf16_t*)w, Kd)
 #define K8SLLM_FR(KIND, MT)                                                                                \

@@ -66,9 +66,11 @@ struct LineSrc {
 };
 // Where workgroup b begins among n pieces of its rows, so that those that run side by side are not at the same k: with rows of weights whole
 // periods of the channels apart (4 KB), every workgroup's lines of one k lie in the same channels of its XCD's L2 and of memory.  us, all from k = 0 /
-// so: shared form, 24 rows 16384 x 4096 26.8 / 22.8, x 8192 54 / 45, 32000 x 4096 47 / 43, 64 rows 54 / 49; own form, 1 row 4096 x 16384 26.0 / 22.1,
-// 8192 x 16384 50 / 42; 16384 x 4160, which needs it not, 23.3.  The order of the fp32 sums follows it: what must keep its sums' order begins at 0.
-constexpr int kTurnBytes = 4096;
+// so: shared form, 24 rows 16384 x 4096 28.8 / 24.9, 65536 x 4096 99 / 87, 16 rows 16384 x 6144 43 / 36, 65536 x 10240 227 / 209; of rows of one period
+// 8192 x 2048 11.9 / 11.5, 32000 x 2048 27.4 / 26.5, 64 rows 34.3 / 32.2, 24 rows 10240 x 2048 12.2 / 12.2; own form, 1 row 4096 x 16384 28.3 / 23.8, 4096 x 8192
+// 15.6 / 14.5, 8192 x 8192 27.2 / 26.0; 16384 x 4160, which needs it not, 23.3.  Few workgroups do not meet and lose a little: 1 row 1024 x 16384 14.9 / 15.5,
+// 512 x 16384 14.0 / 14.3.  The order of the fp32 sums follows it: what must keep its sums' order begins at 0.
+constexpr int kTurnBytes = 4096, kTurnGroups = 128;
 __device__ __forceinline__ int first_piece(int b, int n) { return ((b >> 3) + (b & 7)) % n; }
 // row(r): where row r (of 16) begins
 template <class R>

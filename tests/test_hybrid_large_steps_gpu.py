@@ -800,10 +800,11 @@ def test_segments_in_turn_over_rounds(lens):
 
 
 @pytest.mark.parametrize("M", [1, 24, 64])
-@pytest.mark.parametrize("N,K,shared", [(2056, 2048, True), (1544, 4096, True), (520, 8192, False), (264, 16384, False), (1100, 16384, True)])
+@pytest.mark.parametrize("N,K,shared", [(2056, 2048, True), (1544, 4096, True), (520, 8192, False), (264, 16384, False), (1100, 16384, True),  # below 128
+                                        (8136, 2048, True), (8120, 2048, True), (8200, 6144, True), (2040, 8192, False), (2024, 8192, False), (2056, 16384, False)])
 def test_few_rows_from_a_k_of_their_own(M, N, K, shared):
-    """Weights above 8 MB with rows of whole 4 KB: each workgroup begins at another k.  Against 64 bits, fp32 sums of K products and one rounding; the
-    columns' workgroups are more than the pieces of K and end inside a tile."""
+    """Weights above 8 MB with rows of whole 4 KB: each workgroup begins at another k where there are 128 and more.  Against 64 bits, fp32 sums of K products
+    and one rounding; the columns' workgroups are more than the pieces of K and end inside a tile."""
     g = _g(75)
     x, w = _r(g, M, K, dt=BF).cuda(), _r(g, N, K, s=K ** -0.5, dt=BF).cuda()
     y = torch.empty(M, N, dtype=BF, device="cuda")
