@@ -44,6 +44,7 @@ int k8sllm_moe_combine(void* out, const void* expert_out, const int* inv_idx, co
                        int d, hipStream_t s);
 int k8sllm_gather_rows(void* out, const void* x, const int* idx, long n, int d, int div, hipStream_t s);
 int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void* Y2, int M, int N, int K, int f, int epi, hipStream_t s);
+void k8sllm_gemm_tile_form(int M, int N, int K, int f, int epi, int rs, int* out);
 int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, int N, int K, const int* offsets, int E, long w_es,
                      int epi, int algo, const int* rope_pos, const float* rope_cs, int rope_heads,
                      const float* rs_part, int rs_np, float rs_eps, void* resid, void* hw, const void* norm_w,
@@ -989,6 +990,11 @@ PYBIND11_MODULE(_k8sllm_ops, m) {
   m.def("moe_grouped_gemm", &moe_grouped_gemm);
   m.def("gemm_tile_rows", &gemm_tile_rows);
   m.def("gemm_tile_unit", &gemm_tile_unit);
+  m.def("gemm_tile_form", [](int64_t M, int64_t N, int64_t K, int64_t f, int64_t epi, bool rs) {  // (rows, columns, how many) of a dense product's tiles
+    int out[3];
+    k8sllm_gemm_tile_form((int)M, (int)N, (int)K, (int)f, (int)epi, rs, out);
+    return std::make_tuple(out[0], out[1], out[2]);
+  });
   m.def("gemm_tile", &gemm_tile, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("offsets"), py::arg("swiglu"),
         py::arg("algo") = 1, py::arg("rope_pos") = py::none(), py::arg("rope_cs") = py::none(),
         py::arg("rope_heads") = 0, py::arg("rs_part") = py::none(), py::arg("rs_eps") = 1e-5,

@@ -760,6 +760,21 @@ static int row_blocks(long M, long n_nt, long K) {
   return us(7) < 0.98f * us(8) ? 7 : 8;
 }
 
+// What a dense product of schedule 1 runs on.  (Interleaved per 128 rows, gate and up are not on the path that serves dense models.)
+static Strips dense_strips(int M, int N, int K, int epi, bool rs) {
+  return epi > TILE_EPI_SWIGLU8 || epi == TILE_EPI_RESID || rs ? Strips{} : narrow_strips(M, N, K, epi);
+}
+static int col_tiles(int N, int f) { return f > 0 ? (f + 127) / 128 + (N - 2 * f + 255) / 256 : (N + 255) / 256; }
+static int dense_blocks(int M, int n_nt, int K, int epi) { return epi == TILE_EPI_SWIGLU ? 8 : row_blocks(M, n_nt, K); }
+// out: rows and columns of a strip or tile, and how many of them
+extern "C" void k8sllm_gemm_tile_form(int M, int N, int K, int f, int epi, int rs, int* out) {
+  const Strips s = dense_strips(M, N, K, epi, rs != 0);
+  const int n_nt = col_tiles(N, f), rows = s.rows ? s.rows : 32 * dense_blocks(M, n_nt, K, epi);
+  out[0] = rows;
+  out[1] = s.rows ? s.cols : 256;
+  out[2] = (M + rows - 1) / rows * (s.rows ? N / s.cols : n_nt);
+}
+
 // Dense (offsets == nullptr): Y [M][N] (SwiGLU: [M][N / 2]) = X [M][K] . W[N][K]^T.
 // Grouped: W [E][N][K] with expert stride w_es elements; M = total expert-sorted rows (the grid
 // bound: ceil(M / 256) + E m-tiles); expert e's rows are offsets[e] .. offsets[e + 1] - 1.
@@ -798,9 +813,9 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
   // 32-bit DMA offsets (X: relative to the tile's first row; W: within one expert / n-tile)
   if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31)) return -3;
   if (epi == TILE_EPI_RESID && 256L * N * 2 >= (1L << 31)) return -3;
-  const int n_nt = (N + 255) / 256;
+  const int n_nt = col_tiles(N, 0);
   if (((M + 255) / 256 + (grouped ? E : 0)) * (long)n_nt > (1L << 30)) return -2;
-  const Strips narrow = !grouped && algo == 1 && !rs && epi != TILE_EPI_RESID ? narrow_strips(M, N, K, epi) : Strips{};
+  const Strips narrow = !grouped && algo == 1 ? dense_strips(M, N, K, epi, rs) : Strips{};
   if (narrow.rows) {
     const int rows = (M + narrow.rows - 1) / narrow.rows, cols = N / narrow.cols;
 #define K8_TILE_NARROW(EPI_, C, T)                                                                                               \
@@ -819,8 +834,7 @@ extern "C" int k8sllm_gemm_tile(const void* X, const void* W, void* Y, int M, in
     return (int)hipGetLastError();
   }
   const bool cut = algo == 1 && (!grouped || E <= kStripExperts);
-  // (interleaved per 128 rows, gate and up are not on the path that serves dense models)
-  const int mb = algo == 1 && !grouped && epi != TILE_EPI_SWIGLU ? row_blocks(M, n_nt, K) : 8;
+  const int mb = algo == 1 && !grouped ? dense_blocks(M, n_nt, K, epi) : 8;
   const int n_mt = grouped ? (M + 255) / 256 + E : (M + 32 * mb - 1) / (32 * mb);
   const long nwg = (long)n_mt * n_nt;
   const long over = nwg % kTileCus;
@@ -875,7 +889,7 @@ extern "C" int k8sllm_gemm_tile_unit(const void* X, const void* W, void* Y, void
   if (N <= 0 || N % 16 || K % 64 || K < 192 || (glu ? f <= 0 || f % 16 || N < 2 * f : f != 0)) return -1;
   if ((long)N * K * 2 >= (1L << 31) || 256L * K * 2 >= (1L << 31) || 256L * N * 2 >= (1L << 31)) return -3;
   const TileEpi ep{nullptr, nullptr, 0, nullptr, 0, 0.f, nullptr, nullptr, nullptr, nullptr, f, (bf16_t*)Y2, nullptr, 1, 0};
-  const int n_nt = glu ? (f + 127) / 128 + (N - 2 * f + 255) / 256 : (N + 255) / 256, mb = row_blocks(M, n_nt, K), n_mt = (M + 32 * mb - 1) / (32 * mb);
+  const int n_nt = col_tiles(N, f), mb = dense_blocks(M, n_nt, K, epi), n_mt = (M + 32 * mb - 1) / (32 * mb);
   const long nwg = (long)n_mt * n_nt;
   if (nwg > (1L << 30)) return -2;
   const long over = nwg % kTileCus;

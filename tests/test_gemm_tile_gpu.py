@@ -229,11 +229,21 @@ def test_gemm_tile_last_round_in_fine_strips(M, N, K, f):
     assert torch.equal(y2, z[:, 2 * f:])
 
 
-@pytest.mark.parametrize("M,N,K,f", [  # tiles of 224 rows: one, two and 32 strips' tiles behind rounds, none; the last tile of 1, 33 and 224 rows; three k-tiles
-    (224 * 28 + 1, 4096, 192, 1984), (224 * 14 + 33, 4096, 256, 2048), (6403, 4096, 320, 2000), (7830, 13312, 192, 5632), (224 * 16, 8192 - 128, 640, 3072),
+def _form(M, N, K, f=0, epi=0, rowscale=False):
+    """(rows of a tile, tiles, tiles beyond whole rounds of 256) of a dense product, by the launcher's own rule."""
+    rows, cols, n = ops.native().gemm_tile_form(M, N, K, f, epi, rowscale)
+    return (rows, n, n % 256) if cols == 256 else (rows, n, None)
+
+
+@pytest.mark.parametrize("M,N,K,f,form", [  # the last tile of 1, 33, 131, 150 and 224 rows; behind whole rounds 1, 8, 32, 33, 48 and 64 tiles in strips, none, and too many
+    (224 * 28 + 1, 4096, 192, 1984, (224, 493, 237)), (224 * 14 + 33, 4096, 256, 2048, (224, 240, 240)), (6403, 4096, 320, 2000, (224, 493, 237)),
+    (7830, 13312, 192, 5632, (256, 1612, 76)), (224 * 16, 8192 - 128, 640, 3072, (224, 512, 0)), (200, 65792, 192, 128, (224, 257, 1)),
+    (1281, 11264, 192, 5632, (224, 264, 8)), (2561, 6144, 320, 2048, (224, 288, 32)), (2688, 6144, 192, 3072, (224, 288, 32)), (200, 73984, 192, 128, (224, 289, 33)),
+    (1025, 28672, 192, 14336, (224, 560, 48)), (1119, 16384, 256, 8192, (224, 320, 64)), (4097, 4096, 192, 1984, (256, 289, 33)),
 ])
-def test_gemm_tile_units_of_224_rows(M, N, K, f):
-    """Units and squared ReLU on tiles of 224 rows where those are fewer rounds: the bits of the other schedule's whole tiles."""
+def test_gemm_tile_units_of_224_rows(M, N, K, f, form):
+    """Units and squared ReLU on tiles of 224 rows where those are fewer rounds, whole ones beside strips among them: the bits of the other schedule's whole tiles."""
+    assert _form(M, N, K, f, 7) == form
     g = torch.Generator().manual_seed(7)
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
     w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
@@ -247,17 +257,24 @@ def test_gemm_tile_units_of_224_rows(M, N, K, f):
     assert torch.equal(q, (z.float().clamp(min=0) ** 2).to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("M,N,K", [  # behind rounds: 1, 32, 33 and 64 tiles, none; tiles of 224 rows and of 256; a last tile of one row
-    (4097, 4096, 512), (4608, 4096, 512), (3073, 5376, 1024), (5120, 4096, 512), (1636, 28672, 512), (3585, 4096, 512), (700, 6144, 1536), (257, 1024, 512),
+@pytest.mark.parametrize("M,N,K,form", [  # behind whole rounds 1, 16, 17, 32, 33, 48, 59 and 64 tiles, none, too many; a last tile of one row and of all
+    (4097, 4096, 512, (256, 272, 16)), (4608, 4096, 512, (256, 288, 32)), (3073, 5376, 1024, (256, 273, 17)), (5120, 4096, 512, (256, 320, 64)),
+    (1636, 28672, 512, (256, 784, 16)), (3585, 4096, 512, (256, 240, 240)), (700, 6144, 1536, (224, 96, 96)), (257, 1024, 512, (224, 8, 8)),
+    (200, 65792, 512, (224, 257, 1)), (2610, 6144, 512, (224, 288, 32)), (1537, 28672, 512, (224, 784, 16)), (224, 73984, 512, (224, 289, 33)),
+    (1085, 28672, 512, (224, 560, 48)), (3329, 5376, 1024, (224, 315, 59)), (1120, 16384, 512, (224, 320, 64)), (6945, 4096, 512, (224, 512, 0)),
+    (5121, 4096, 512, (224, 368, 112)),
 ])
-def test_gemm_tile_fused_ends_of_strips(M, N, K):
+def test_gemm_tile_fused_ends_of_strips(M, N, K, form):
     """Residual, rotation and row scale at the end of strips and of tiles of 224 rows: the bits of the plain product on whole tiles, finished here.  (Scales are
     powers of two, so that they commute with every rounding.)"""
+    assert _form(M, N, K, epi=3) == form and _form(M, N, K, epi=2, rowscale=True) == form and _form(M, N, K, epi=4, rowscale=True) == form
     g = torch.Generator().manual_seed(8)
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
     wr = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
     w = ops.pack_skinny(wr)
     z = ops.gemm_tile(x, wr, algo=0)
+    if _form(M, N, K) == form:
+        assert torch.equal(ops.gemm_tile(x, w, algo=1), z)
     r, nw = torch.randn(M, N, generator=g).to(torch.bfloat16).cuda(), (torch.rand(N, generator=g) + 0.5).to(torch.bfloat16).cuda()
     h = (z.float() + r.float()).to(torch.bfloat16)
     hw, ss = ops.gemm_tile_resid(x, w, r, nw)
@@ -277,13 +294,15 @@ def test_gemm_tile_fused_ends_of_strips(M, N, K):
     assert torch.equal(ops.gemm_tile(x, w, swiglu=8, algo=1, rowscale=(part, 0.0)), ops.gemm_tile(big, wr, swiglu=8, algo=0))
 
 
-@pytest.mark.parametrize("M,N,K", [  # tiles of 224 and of 256 rows, alone, behind 64 x 256 strips and in front of 64 x 128 ones
-    (1, 128, 192), (300, 384, 192), (4097, 384, 320), (9000, 384, 192), (4097, 4224, 192), (7937, 4224, 192), (10240, 4224, 192), (4609, 4224, 256),
-    (1025, 28544, 192), (1537, 28544, 192),
+@pytest.mark.parametrize("M,N,K,form", [  # tiles of 224 and of 256 rows, alone, in 64 x 256 strips and in 64 x 128 ones, and whole ones beside those
+    (1, 128, 192, (224, 1, 1)), (300, 384, 192, (224, 4, 4)), (4097, 384, 320, (224, 38, 38)), (9000, 384, 192, (224, 82, 82)), (4097, 4224, 192, (256, 289, 33)),
+    (7937, 4224, 192, (256, 544, 32)), (10240, 4224, 192, (256, 680, 168)), (4609, 4224, 256, (224, 357, 101)), (1025, 28544, 192, (224, 560, 48)),
+    (1537, 28544, 192, (224, 784, 16)),
 ])
-def test_gemm_tile_residual_behind_half_a_tile(M, N, K):
+def test_gemm_tile_residual_behind_half_a_tile(M, N, K, form):
     """N % 256 == 128: the last tile's second 128 columns are not there.  Every row's residual, weighted row and sums of squares are the plain product's,
     finished here, and nothing behind the buffers' ends is written."""
+    assert _form(M, N, K, epi=3) == form
     g = torch.Generator().manual_seed(9)
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
     w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
