@@ -516,8 +516,8 @@ def test_latent_rows_beside_others_and_wide_tables(Hq, pitch, R, dv, T):
                                           (1, 2016, 48, 0, ""), (2, 1056, 100, 0, ""), (1, 1024, 6656, 2816, "gelu_tanh"),
                                           (2, 2048, 1072, 512, "silu"), (3, 480, 128, 64, "relu")])
 def test_products_of_gated_rows(M, d, N, f, kind):
-    """The gated residual's sum and norm as a product's prologue: the same residual bit for bit as the launch of its own; the rows' sums of squares
-    may be in another order, which rounds a value of them the other way (2^-8 of it) now and then, and the product is rounded once; what no product takes is made."""
+    """The gated residual's sum and norm as a product's prologue, the same sums in the same order: the residual, and the products of few_rows.hip's own form over
+    the rows that the launch of its own makes, bit for bit; what no product takes is made."""
     g, dt = _g(31), torch.bfloat16
     x, y, proj = _r(g, M, d).cuda(), _r(g, M, d, dt=dt).cuda(), _r(g, M, d + 24, dt=dt).cuda()
     bias, nw = _r(g, d).cuda(), (_r(g, d, s=0.2) + 1).cuda()
@@ -525,19 +525,19 @@ def test_products_of_gated_rows(M, d, N, f, kind):
     args = (y, proj, 16, bias, 0.5, nw, 1e-6, False)
     x_want = x.clone()
     h = H.gated_add_norm(x_want, *args, dt)
-    want = h.double() @ w.double().t()
-    most = 2.0 ** -9 * (h.double().abs() @ w.double().abs().t())
+    want, unit = torch.empty(M, N - 2 * f, dtype=dt, device="cuda"), torch.empty(M, f, dtype=dt, device="cuda") if f else None
+    H.native().few_rows(want, unit, h, w, H.ACTS[kind] if f else -1, 0.0, False)
     rows = H.gated_rows(x, *args, dt)
     assert isinstance(rows, H.GatedRows) and rows.shape == x.shape
     if f:
         a, z, col = H.linear_glu(rows, w, f, kind)
-        gate, up = (t.to(dt).float() for t in (want[:, :f], want[:, f:2 * f]))
-        unit = H._act_torch(gate, kind) * up
-        assert bool(((a.float() - unit).abs() <= 2.0 ** -6 * unit.abs() + 1e-3).all())  # gate and up may each be rounded the other way
-        z, want, most = z[:, col:], want[:, 2 * f:], most[:, 2 * f:]
+        assert torch.equal(a, unit)
+        z = z[:, col:]
     else:
         z = H.linear(rows, w)
-    assert bool(((z.double() - want).abs() <= 2.0 ** -8 * want.abs() + most).all())
+    assert torch.equal(z, want)
+    exact = h.double() @ w[2 * f:].double().t()  # fp32 sums of d products, one rounding
+    assert bool(((z.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + 1e-6 * d ** 0.5).all())
     assert torch.equal(rows.residual, x_want) and rows.residual.data_ptr() != x.data_ptr()
     torch.testing.assert_close(rows.tensor().float(), h.float(), rtol=2.0 ** -7, atol=1e-6)  # made again from the new residual
     made = H.gated_rows(x, *args, dt)
