@@ -254,10 +254,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   const int ml = lane & 15, nq = 4 * (lane >> 4);
   const int rr = lane >> 4, cc = lane & 15;
   uint4 nwv{};
-  if constexpr (EPI == TILE_EPI_RESID) {
-    if (nrows <= wn * 128) return;  // N % 256 == 128: the last tile's second 128 columns are not there (the row behind them is; no barrier follows)
-    nwv = *reinterpret_cast<const uint4*>(ep.norm_w + n0 + wn * 128 + cc * 8);
-  }
+  // RESID, N % 256 == 128: the last tile's second 128 columns are not there (the next row's first are), so its waves have descriptors of no bytes.  (Scalar:
+  // hipcc spilled up to 48 registers around a branch.  The residual's loads in front of this, of the next row there, are left: nothing is made of them, and
+  // masks took 28 registers and more.)
+  const int live = nrows > wn * 128 ? mrows : 0;
+  if constexpr (EPI == TILE_EPI_RESID) nwv = *reinterpret_cast<const uint4*>(ep.norm_w + (live ? n0 + wn * 128 : 0) + cc * 8);
   // RS: each thread's row scale through LDS (after the staging area) to the lanes holding the row
   float sc[RB];
 #pragma unroll
@@ -327,8 +328,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
   lgkm_wait0();
   if constexpr (EPI == TILE_EPI_RESID) {
     // lane (rr, cc): row rr + 4b, columns cc*8 .. +7 of the wave's quarter; N % 128 == 0 (host)
-    const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
-    const __amdgpu_buffer_rsrc_t rhw = rsrc(ep.hw + (long)row0 * N, (long)mrows * N * 2);
+    const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)live * N * 2);
+    const __amdgpu_buffer_rsrc_t rhw = rsrc(ep.hw + (long)row0 * N, (long)live * N * 2);
     const uint32_t ro = (uint32_t)(((wm * 16 * RB + rr) * N + n0 + wn * 128 + cc * 8) * 2);
     float wf[8];
     unpack8(nwv, wf);
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       __builtin_amdgcn_raw_buffer_store_b128(u32x4{wq.x, wq.y, wq.z, wq.w}, rhw, off, 0, 0);
       ss = row16_sum(ss);
       const int grow = wm * 16 * RB + r;
-      if (cc == 0 && grow < mrows) ep.ss_out[(long)(row0 + grow) * ss_np + ssc] = ss;
+      if (cc == 0 && grow < live) ep.ss_out[(long)(row0 + grow) * ss_np + ssc] = ss;
     }
     return;
   }
@@ -493,8 +494,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     }
     if constexpr (EPI == TILE_EPI_RESID) {
       const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
-      // (columns past N: out of range, nothing is read)
-      const uint32_t ro = nrows > wn * 128 ? (uint32_t)(((wm * 16 * RB + (lane >> 4)) * N + n0 + wn * 128 + (lane & 15) * 8) * 2) : 0x80000000u;
+      const uint32_t ro = (uint32_t)(((wm * 16 * RB + (lane >> 4)) * N + n0 + wn * 128 + (lane & 15) * 8) * 2);
 #pragma unroll
       for (int b = 0; b < 4 * RB; ++b) resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * b * N * 2), 0, 0);
     }
@@ -648,7 +648,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
       sub(P0{}, P3{}, fa0, fb0, fa1, fb1, S0, S1, S0, S1, t);
       if constexpr (EPI == TILE_EPI_RESID) {
         const __amdgpu_buffer_rsrc_t rres = rsrc(ep.resid + (long)row0 * N, (long)mrows * N * 2);
-        const uint32_t ro = nrows > wn * 128 ? (uint32_t)(((wm * 16 * MB + (lane >> 4)) * N + n0 + wn * 128 + (lane & 15) * 8) * 2) : 0x80000000u;
+        const uint32_t ro = (uint32_t)(((wm * 16 * MB + (lane >> 4)) * N + n0 + wn * 128 + (lane & 15) * 8) * 2);
 #pragma unroll
         for (int b = 0; b < 16; ++b)
           resq[b] = __builtin_amdgcn_raw_buffer_load_b128(rres, ro + (uint32_t)(4 * b * N * 2), 0, 0);
