@@ -106,14 +106,15 @@ __global__ __launch_bounds__(64) void latent_head_values_kernel(bf16_t* __restri
 
 // The same of rows whose attention lies in parts (LatentParts): their merge, times the sigmoid of the row and head's gate, rounded, is the products' operand.
 // Each of a head's dv / 16 workgroups merges its rows again, which costs less than a launch of its own (1.6 us and a round of loads).
-// Four waves take the parts in turn and put a quarter of R each into LDS, and the last one, which has the fewest parts, multiplies: in the order of
-// latent_head_values_kernel, and rows of one part with what is already finished for them, so that a row has the same bits whatever stands beside it.
-// Sixteen rows of one part each need nothing else.  All that may be needed is on its way before it is known what is (a round of loads less: 64 rows of
-// 1500 keys, 16 heads, 32.7 / 31.9 us).
-__global__ __launch_bounds__(256) void latent_part_values_kernel(bf16_t* __restrict__ v, const bf16_t* __restrict__ one, LatentParts parts, int most,
-                                                                 const bf16_t* __restrict__ wv, int T, int H, int dv, int R,
-                                                                 const bf16_t* __restrict__ gate, long g_stride) {
-  constexpr int KC = 8, NW = 4, KW = KC / NW;  // pieces of 32 k: R <= 256
+// NW waves take the parts in turn and put their pieces of R into LDS, and one more multiplies: in the order of latent_head_values_kernel, and rows of one
+// part with what is already finished for them, so that a row has the same bits whatever stands beside it.  Sixteen rows of one part each need nothing
+// else.  All that may be needed is on its way before it is known what is (a round of loads less: 64 rows of 1500 keys, 16 heads, 32.7 / 31.9 us).  Three
+// waves for three parts: two workgroups of five waves share no unit (64 rows of 700 keys, 16 heads, 26.2 / 24.6).
+template <int NW>
+__global__ __launch_bounds__(64 * (NW + 1)) void latent_part_values_kernel(bf16_t* __restrict__ v, const bf16_t* __restrict__ one, LatentParts parts, int most,
+                                                                           const bf16_t* __restrict__ wv, int T, int H, int dv, int R,
+                                                                           const bf16_t* __restrict__ gate, long g_stride) {
+  constexpr int KC = 8;  // pieces of 32 k: R <= 256
   __shared__ __attribute__((aligned(16))) float4 o_s[NW][2 * KC][64];
   __shared__ float2 ml_s[NW][64];
   __shared__ uint4 x_s[KC][64];
@@ -121,19 +122,37 @@ __global__ __launch_bounds__(256) void latent_part_values_kernel(bf16_t* __restr
   const int n0 = 16 * blockIdx.x, t = min(t0 + col, T - 1);
   const long th = (long)t * H + h, step = (long)T * H;
   const int np = parts.n[t];
-  uint4 a[KC], b[KC];
-  auto load = [&](uint4 (&x)[KC], const bf16_t* row) {
+  if (wave == NW) {
+    uint4 a[KC], b[KC];
+    auto load = [&](uint4 (&x)[KC], const bf16_t* row) {
 #pragma unroll
-    for (int c = 0; c < KC; ++c) {
-      const int k = 32 * c + 8 * quad;
-      x[c] = *reinterpret_cast<const uint4*>(row + (k < R ? k : 0));
-      if (k >= R) x[c] = make_uint4(0, 0, 0, 0);
-    }
-  };
-  const bool last = wave == NW - 1;
-  if (last) {
+      for (int c = 0; c < KC; ++c) {
+        const int k = 32 * c + 8 * quad;
+        x[c] = *reinterpret_cast<const uint4*>(row + (k < R ? k : 0));
+        if (k >= R) x[c] = make_uint4(0, 0, 0, 0);
+      }
+    };
     load(a, wv + ((long)h * dv + min(n0 + col, dv - 1)) * R);
     load(b, one + th * R);
+    if (__ballot(np > 1) != 0) {  // the same rows in every wave
+      __syncthreads();
+      __syncthreads();
+      if (np > 1) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+          if (32 * c + 8 * quad < R) b[c] = x_s[c][lane];
+      }
+    }
+    hf32x4 acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+      if (32 * c < R) acc = tile_product(a[c], b[c], acc);
+    if (t0 + col >= T) return;
+    bf16_t* out = v + ((long)(t0 + col) * H + h) * dv + n0 + 4 * quad;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n0 + 4 * quad + i < dv) stf(out + i, acc[i]);
+    return;
   }
   float2 ml;
   float x[KC][8];
@@ -145,70 +164,56 @@ __global__ __launch_bounds__(256) void latent_part_values_kernel(bf16_t* __restr
     for (int c = 0; c < KC; ++c) load8(p + (32 * c + 8 * quad < R ? 32 * c : -8 * quad), x[c]);
   };
   part(wave);
-  if (__ballot(np > 1) != 0) {  // the same rows in every wave
-    float M = -INFINITY, L = 0.f, o[KC][8] = {};
-    for (int z = wave; __ballot(np > 1 && z < np) != 0; z += NW) {
-      if (z > wave) part(z);
-      if (np <= 1 || z >= np) continue;
-      const float m = fmaxf(M, ml.x), f0 = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - m), f1 = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
-      M = m;
-      L = fmaf(ml.y, f1, L * f0);
+  if (__ballot(np > 1) == 0) return;
+  float M = -INFINITY, L = 0.f, o[KC][8] = {};
+  for (int z = wave; __ballot(np > 1 && z < np) != 0; z += NW) {
+    if (z > wave) part(z);
+    if (np <= 1 || z >= np) continue;
+    const float m = fmaxf(M, ml.x), f0 = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - m), f1 = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
+    M = m;
+    L = fmaf(ml.y, f1, L * f0);
 #pragma unroll
-      for (int c = 0; c < KC; ++c)
+    for (int c = 0; c < KC; ++c)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) o[c][j] = fmaf(x[c][j], f1, o[c][j] * f0);
-    }
+      for (int j = 0; j < 8; ++j) o[c][j] = fmaf(x[c][j], f1, o[c][j] * f0);
+  }
 #pragma unroll
-    for (int c = 0; c < KC; ++c) {
-      o_s[wave][2 * c][lane] = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
-      o_s[wave][2 * c + 1][lane] = make_float4(o[c][4], o[c][5], o[c][6], o[c][7]);
-    }
-    ml_s[wave][lane] = make_float2(M, L);
-    __syncthreads();
-    float f[NW];
-    M = -INFINITY;
-    L = 0.f;
+  for (int c = 0; c < KC; ++c) {
+    o_s[wave][2 * c][lane] = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
+    o_s[wave][2 * c + 1][lane] = make_float4(o[c][4], o[c][5], o[c][6], o[c][7]);
+  }
+  ml_s[wave][lane] = make_float2(M, L);
+  __syncthreads();
+  float f[NW];
+  M = -INFINITY;
+  L = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_s[w][lane].x);
+  for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_s[w][lane].x);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const float2 q = ml_s[w][lane];
+    f[w] = q.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(q.x - M);
+    L = fmaf(q.y, f[w], L);
+  }
+  float inv = L > 0.f ? 1.f / L : 0.f;
+  if (gate != nullptr) inv *= sigmoid_f(bf2f(gate[(long)t * g_stride + h]));
+#pragma unroll
+  for (int i = 0; i < (KC + NW - 1) / NW; ++i) {
+    const int c = NW * i + wave;
+    if (c >= KC) break;
+    float y[8] = {};
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float2 q = ml_s[w][lane];
-      f[w] = q.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(q.x - M);
-      L = fmaf(q.y, f[w], L);
+      const float4 u = o_s[w][2 * c][lane], s = o_s[w][2 * c + 1][lane];
+      const float q[8] = {u.x, u.y, u.z, u.w, s.x, s.y, s.z, s.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] = fmaf(q[j], f[w], y[j]);
     }
-    float inv = L > 0.f ? 1.f / L : 0.f;
-    if (gate != nullptr) inv *= sigmoid_f(bf2f(gate[(long)t * g_stride + h]));
 #pragma unroll
-    for (int c = 0; c < KW; ++c) {
-      float y[8] = {};
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const float4 u = o_s[w][2 * (KW * wave + c)][lane], s = o_s[w][2 * (KW * wave + c) + 1][lane];
-        const float q[8] = {u.x, u.y, u.z, u.w, s.x, s.y, s.z, s.w};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) y[j] = fmaf(q[j], f[w], y[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] *= inv;
-      x_s[KW * wave + c][lane] = pack8(y);
-    }
-    __syncthreads();
-    if (last && np > 1) {
-#pragma unroll
-      for (int c = 0; c < KC; ++c)
-        if (32 * c + 8 * quad < R) b[c] = x_s[c][lane];
-    }
+    for (int j = 0; j < 8; ++j) y[j] *= inv;
+    x_s[c][lane] = pack8(y);
   }
-  if (!last) return;
-  hf32x4 acc{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int c = 0; c < KC; ++c)
-    if (32 * c < R) acc = tile_product(a[c], b[c], acc);
-  if (t0 + col >= T) return;
-  bf16_t* out = v + ((long)(t0 + col) * H + h) * dv + n0 + 4 * quad;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (n0 + 4 * quad + i < dv) stf(out + i, acc[i]);
+  __syncthreads();
 }
 
 }  // namespace k8sllm
@@ -243,9 +248,14 @@ int k8sllm_hy_latent_part_values(void* v, const void* one, const float* o, const
                                  int dv, int R, const void* gate, long g_stride, hipStream_t s) {
   if (T <= 0 || H <= 0 || dv <= 0) return 0;
   if (R < 16 || R % 16 || R > 256 || T > (1 << 19) || H > 65535 || most < 1 || (reinterpret_cast<uintptr_t>(wv) & 15)) return -1;
-  hipLaunchKernelGGL(latent_part_values_kernel, dim3((unsigned)((dv + 15) / 16), (unsigned)H, (unsigned)((T + 15) / 16)), dim3(256), 0, s,
-                     (bf16_t*)v, (const bf16_t*)one,
-                     LatentParts{(float*)o, (float2*)ml, (int*)n, 0}, most, (const bf16_t*)wv, (int)T, H, dv, R, (const bf16_t*)gate, g_stride);
+  const dim3 grid((unsigned)((dv + 15) / 16), (unsigned)H, (unsigned)((T + 15) / 16));
+  const LatentParts p{(float*)o, (float2*)ml, (int*)n, 0};
+  if (most <= 3)
+    hipLaunchKernelGGL(latent_part_values_kernel<3>, grid, dim3(256), 0, s, (bf16_t*)v, (const bf16_t*)one, p, most, (const bf16_t*)wv, (int)T, H, dv, R,
+                       (const bf16_t*)gate, g_stride);
+  else
+    hipLaunchKernelGGL(latent_part_values_kernel<4>, grid, dim3(320), 0, s, (bf16_t*)v, (const bf16_t*)one, p, most, (const bf16_t*)wv, (int)T, H, dv, R,
+                       (const bf16_t*)gate, g_stride);
   return (int)hipGetLastError();
 }
 }

@@ -931,9 +931,9 @@ def latent_parts(T: int, H: int, R: int, pages: int, window: int) -> tuple:
     eight waves takes 4 us for each eight tiles (its loads of 16 key rows ask for 16 lines at a time), one a CU, so few rows are cut until half of the chip
     is busy, a tile a wave at least; behind that parts cost more in the merge than they save (1.2 us for each four, and their outputs' way through memory).
     Tables are as wide as the longest sequence may become, so a row of few tiles is one part by itself.  us with the values behind it, whole / so, tables of
-    512 pages: 8 heads, 128 + 32 wide, 1 row of 20 keys 7.7 / 8.4, 333 10.7 / 10.3, 1500 21.3 / 12.5, 4800 51 / 14.7; 16 rows of 100 8.8 / 9.4, 700 14.1 / 13.6,
-    1500 22.0 / 15.3; 64 of 333 11.3 / 11.9, 1500 26.1 / 20.0, 4800 62 / 36; 16 heads, 256 + 32, 1 of 20 11.8 / 11.7, 1500 36 / 16.0; 32 of 1500 39.9 / 24.2, 64 of
-    333 18.3 / 19.2, 1500 40.4 / 31.8.  (With every row of such a table in 3 to 16 parts, 1 row of 20 keys took 10.6, 64 of 333 12.3 and 21.3.)"""
+    512 pages: 8 heads, 128 + 32 wide, 1 row of 20 keys 7.8 / 7.9, 333 10.6 / 10.2, 1500 21.4 / 12.2, 4800 51 / 14.4; 16 rows of 100 8.8 / 9.0, 700 14.2 / 13.4,
+    1500 22.0 / 15.2; 64 of 333 11.3 / 11.4, 1500 26.1 / 19.9, 4800 62 / 36; 16 heads, 256 + 32, 1 of 20 11.9 / 11.5, 1500 36 / 16.0; 32 of 1500 39.9 / 24.0, 64 of
+    333 18.5 / 18.7, 1500 40.3 / 32.3.  (With every row of such a table in 3 to 16 parts, 1 row of 20 keys took 10.6, 64 of 333 12.3 and 21.3.)"""
     wgs = T * -(-H // 16)
     if wgs == 0 or wgs > 64:
         return 1, 1
