@@ -118,7 +118,8 @@ __global__ __launch_bounds__(64 * (NW + 1)) void latent_part_values_kernel(bf16_
   __shared__ __attribute__((aligned(16))) float4 o_s[NW][2 * KC][64];
   __shared__ float2 ml_s[NW][64];
   __shared__ uint4 x_s[KC][64];
-  const int h = blockIdx.y, t0 = 16 * blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
+  const int h = blockIdx.y, t0 = 16 * blockIdx.z, lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // (scalar: the waves' branches hold barriers)
   const int n0 = 16 * blockIdx.x, t = min(t0 + col, T - 1);
   const long th = (long)t * H + h, step = (long)T * H;
   const int np = parts.n[t];
