@@ -1505,7 +1505,8 @@ def _tile_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def _tile_unit(x: torch.Tensor, w: torch.Tensor, f: int) -> bool:
     """Whether ``gemm_tile_unit`` takes these operands, by the rule of ``_tile_form`` (which takes no fewer rows than 0.8 of a tile's)."""
-    return x.shape[0] > 204 and _tile_operands(x, w) and _tile_form(x.shape[0], w.shape[0], w.shape[1], f)
+    M = x.shape[0]
+    return M > 204 and w.dim() == 2 and _tile_form(M, w.shape[0], w.shape[1], f) and _tile_operands(x, w)
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, kind: str) -> torch.Tensor:
