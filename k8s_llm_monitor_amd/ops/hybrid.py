@@ -839,8 +839,8 @@ def latent_head_values(o: torch.Tensor, w_uv: torch.Tensor, H: int, out: Optiona
     v = (torch.empty(T, H * dv, dtype=o.dtype, device=o.device) if out is None else out).view(T, H, dv)
     if _head_rows(HEAD_VALUE_ROWS, o, w_uv) and R % 8 == 0 and T * H * dv * R < HEAD_VALUE_WORK:
         native().latent_head_values(v, o, w_uv, int(H))
-    else:  # written head by head into the rows that the out-projection reads
-        torch.bmm(o.view(T, H, R).transpose(0, 1), w_uv.view(H, dv, R).transpose(1, 2), out=v.transpose(0, 1))
+    else:  # written head by head into the rows that the out-projection reads (a right operand that is a transposed view has faulted in bf16)
+        torch.bmm(o.view(T, H, R).transpose(0, 1), w_uv.view(H, dv, R).transpose(1, 2).contiguous(), out=v.transpose(0, 1))
     return v.view(T, H * dv)
 
 

@@ -138,6 +138,15 @@ def test_latent_expanded_form_equals_the_oracle(monkeypatch):
     close(a["c"], want["c"])
 
 
+def test_batched_products_have_contiguous_right_operands(monkeypatch):
+    """The library's batched bf16 products have faulted on the device where the right operand was a transposed view."""
+    seen, real = [], torch.bmm
+    monkeypatch.setattr(torch, "bmm", lambda a, b, **k: seen.append(b.is_contiguous()) or real(a, b, **k))
+    rig = rig_for(FULL, 5)
+    rig.step([("a", toks(20, FULL["vocab"], 6))])
+    assert len(seen) >= 4 and all(seen)
+
+
 def test_forms_of_few_rows_are_asked_for_few_rows_only(monkeypatch):
     """The host's time bounds a short prompt's step: forms that take up to 4 and up to 64 rows are not gone into for more."""
     rig, calls = rig_for(FULL, 5), []
