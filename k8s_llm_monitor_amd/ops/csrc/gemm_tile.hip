@@ -719,10 +719,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 
 using namespace k8sllm;
 
-// The strips that a dense product of few tiles goes in: the least of rounds x (k-tiles x rate + 6 us for its start and end).  Rates, us a k-tile with the
-// chip full: 64 x 64 0.26 (plain products), 64 x 128 0.42, 128 x 128 0.72; a tile 1.25, 0.8 where few go as strips of 256 columns.  (Of before the strips'
-// accumulators stayed where they are; now 0.22, 0.35 and 0.55: 4096 x 14336, 400 rows 94 / 81, 600 rows 150 / 120; 6144 x 4096, 144 rows 29 / 26, 600 rows
-// 47 / 39; with SwiGLU 28672 x 4096, 80 rows 51 / 45.  By those the choice would be the same but for 4096 x 14336 from 1025 rows.)  us, tiles / 128 x 128 /
+// The strips that a dense product of few tiles goes in: the least of rounds x (k-tiles x rate + 6 us for its start and end).  The rates, us a k-tile with the
+// chip full, are of strips whose accumulators moved: 64 x 64 0.26 (plain products), 64 x 128 0.42, 128 x 128 0.72; a tile 1.25, 0.8 where few go as strips of
+// 256 columns (not yet with RoPE, then).  They stand because the choice does: by the present ones (0.22, 0.35 and 0.55; 4096 x 14336, 400 rows 94 / 81 us, 600
+// rows 150 / 120; 6144 x 4096, 144 rows 29 / 26, 600 rows 47 / 39; with SwiGLU 28672 x 4096, 80 rows 51 / 45) it would be the same but for 4096 x 14336 from
+// 1025 rows on.  How the kernels compared when it was made, us, tiles / 128 x 128 /
 // 64 x 128 / 64 x 64, packed weights: 4096 x 4096, 80 rows 56 / - / 35 / 23, 300 56 / - / 35, 600 59 / 54; 4096 x 14336, 80 rows 168 / - / 98 / 58, 400 167 /
 // - / 104, 600 178 / 161; 6144 x 4096 with RoPE, 80 rows 78 / - / 36, 300 81 / - / 38, 400 - / 57 / 67, 600 83 / 58 / 71, 800 84 / 102 (two rounds); 28672 x
 // 4096 with SwiGLU, 80 rows 90 / 62 / 75 (two rounds), 200 90 / 107 (two rounds).  Rounds are an XCD's: it has whole columns' strips and 32 CUs, so 12

@@ -1438,9 +1438,10 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, end: str = "") -> Optional[str]:
 def _tile_plain(M: int, N: int, K: int) -> bool:
     """Whether the tile GEMM takes a large product with nothing behind it: where N is no multiple of its 256 columns and K small, the BLAS
     library's kernels fall to 350 (K up to 512), 600 (1024) and 800 TFLOP/s (2048, N below 4096), and the tile GEMM's rounds of 256 tiles, estimated
-    here, take less than that.  Elsewhere the library is 5 to 14 % ahead.  us, library / tile GEMM: 6403 x 5648 x 1024 122 / 89, 4800 rows 97 / 64;
-    7830 x 3104 x 2048 129 / 100; 8000 x 1568 x 1024 40 / 32.  Over 400 products of 1024 to 9000 rows, 1024 to 12000 columns and 256 to 2048 k
-    (N no multiple of 256) the 181 that it takes are 1.31 times faster in the mean, the worst 0.98; of multiples of 256 it would lose as many as it wins."""
+    here, take less than that.  us, library / tile GEMM: 6403 x 5648 x 1024 127 / 82, 4800 rows 100 / 55; 7830 x 3104 x 2048 131 / 86; 8000 x 1568 x 1024 41 /
+    29.  Over 404 products of 1024 to 9000 rows, 1024 to 12000 columns and 256 to 2048 k (N no multiple of 256) the 107 that it takes are 1.36 times faster in the
+    mean, the worst 1.10.  The estimate is of 256-row tiles and slower strips than the kernel has: of the 297 that it leaves 174 would be faster too,
+    100 slower.  (Multiples of 256 were measured with that kernel: as many would lose as win.)"""
     if M < 1024 or not 1024 <= N < 1 << 19 or N % 256 == 0 or N % 16 or K % 64 or not 192 <= K <= 2048 or (K > 1024 and N >= 4096):
         return False  # (the tile GEMM's offsets into the weights are 31 bits)
     rounds, over = divmod(-(-M // 256) * -(-N // 256), 256)
