@@ -1481,13 +1481,13 @@ GLU_ENDS = ("gelu_tanh", "silu", "relu")  # gated units that the projections' ke
 
 
 def _tile_form(M: int, N: int, K: int, f: int) -> bool:
-    """Whether the tile GEMM takes a large product with a unit at its end (a gated one of f features, or f 0): its tiles take 5 % longer
-    than the BLAS library's, which leaves the unit a launch of its own that reads and writes the products once more.  us, library and
-    launch / tile GEMM: 7830 rows, 2 x 5632 + 2048 columns, K 2048 388 + 47 / 355; 3749 rows 236 + 25 / 195; 6403 x 4096 x 1024 (1.6
-    rounds of tiles) 53 + 18 / 58.  At least four fifths of the tiles' area must be products: 53248 columns, K 2048 1 row 48 / 62, 128
-    rows 59 / 64, 300 rows (two row tiles) 97 / 109, 256 rows 74 / 68, 1300 rows (six) 331 / 279."""
+    """Whether the tile GEMM takes a large product with a unit at its end (a gated one of f features, or f 0), which the BLAS library leaves a
+    launch of its own that reads and writes the products once more.  us, library and launch / tile GEMM: 7830 rows, 2 x 5632 + 2048 columns, K
+    2048 377 + 54 / 339; 3749 rows 225 + 23 / 168; 6403 x 4096 x 1024 (1.6 rounds of tiles) 49 + 17 / 53.  At least four fifths of the tiles' area
+    must be products: 53248 columns, K 2048 1 row 52 / 57, 128 rows 61 / 59, 300 rows (two row tiles) 89 / 91, 256 rows 70 / 62, 1300 rows
+    (six) 308 / 235.  Rounds are counted in tiles of 256 rows without strips, as the kernel was when the rule was made; it leaves the library some
+    products that would be faster now: 4300 x 4096 x 1024 55 / 46, 2500 x 8192 x 1024 63 / 50, 2700 x 4096 x 1024 34 / 28."""
     tiles = -(-M // 256) * (-(-f // 128) + -(-(N - 2 * f) // 256))
-    # one tile a compute unit at a time: a last round that is mostly empty takes as long as a full one
     return (tiles >= 200 and tiles >= 0.7 * 256 * -(-tiles // 256) and M * N >= 0.8 * 256 * 256 * tiles
             and K % 64 == 0 and K >= 192 and N % 16 == 0 and f % 16 == 0 and 2 * f <= N and max(N, 256) * max(K, 256) * 2 < 1 << 31
             and 256 * N * 2 < 1 << 31)
